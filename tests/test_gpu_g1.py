@@ -44,6 +44,18 @@ def test_generators_match_oracle_stream(pv, orc):
     assert jac_to_affine(g.host()[0]) == ec_mul(fr_ints(mt_random_vec(np.random.RandomState(321), 1))[0], (G1_X, G1_Y))
 
 
+@pytest.mark.parametrize("n", [1, 65, (1 << 17) - 1, (1 << 17) + 130])
+def test_normalisation_at_the_edges_of_its_lane_counts(pv, orc, n):
+    """one point a lane up to 2^17, four above, infinities among them; a few points tiled, since normalisation takes each alone"""
+    few = oracle_gens(orc, 17, 5)
+    doubled = np.zeros_like(few)
+    orc_check(orc.orc_g1_op(0, few, few, doubled, 5))           # z != 1
+    few = np.concatenate([few, doubled, np.zeros((1, 36), np.uint32)])
+    at = np.arange(n) % 11
+    got = pv.g1_binop(3, pv.g1_from_host(few[at])).host()
+    assert (got == norm(orc, few)[at]).all()
+
+
 def test_elementwise_and_special_cases(pv, orc):
     gens = oracle_gens(orc, 11, 16)
     inf = np.zeros(36, np.uint32)

@@ -128,6 +128,20 @@ def test_batch_inverse(pv, orc, n):
         assert not got[3].any()
 
 
+@pytest.mark.parametrize("n", [511, 513, 1 << 18, (1 << 18) + 1, (1 << 18) + 2047])
+def test_batch_inverse_at_the_edges_of_its_lane_counts(pv, orc, n):
+    """Two values a lane up to 2^18, eight above; values a Euclidean quotient does not fit (1, 2, -1, powers of two) and zeros among them."""
+    S = ch(n, n)
+    beta = ch(7, 1)[0]
+    b = fr_ints(beta.reshape(1, 8))[0]
+    odd = [0, 1, 2, R_MOD - 1, R_MOD - 2, 1 << 64, (1 << 128) + 1, 1 << 254]
+    at = [0, 1, 256, 300, n // 2, n - 1, n - 2, n - 3]
+    S[at] = fr_array([(x - b) % R_MOD for x in odd])
+    exp = np.zeros_like(S)
+    orc_check(orc.orc_lookup_inv(S, n, beta, exp))
+    assert (pv.batch_inv(pv.from_fr(S), beta).host() == exp).all()
+
+
 def test_batch_inverse_at_full_size_inverts(pv):
     """2^24 + 5 values: the products of the workgroups are themselves too many for one step, so the scheme nests twice.
     Checked by what an inverse is: out * (in + beta) == 1 everywhere (0 where in + beta == 0)."""

@@ -12,6 +12,9 @@
 // the top limb clear, the running value never needs an (N+2)-th limb.
 #pragma once
 #include <cstdint>
+#if defined(__x86_64__) && !defined(__HIP_DEVICE_COMPILE__)
+#include <immintrin.h>
+#endif
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
 #define ZK_HD __host__ __device__ __forceinline__
@@ -42,6 +45,15 @@ struct FrK {
         constexpr uint32_t t[8] = {4092763245u, 3382307216u, 2274516003u, 728559051u, 1918122383u, 97719446u, 2673475345u, 122214873u};
         return t[i];
     }
+    ZK_HD static constexpr uint32_t R3(int i) {    // R^3 mod r
+        constexpr uint32_t t[8] = {1134261167u, 3324778503u, 2364565904u, 457051416u, 3350590488u, 1943092337u, 3369808873u, 1848269753u};
+        return t[i];
+    }
+    static constexpr int L30 = 9;                  // limbs of 30 bits (euclid_inverse)
+    ZK_HD static constexpr int32_t P30(int i) {
+        constexpr int32_t t[9] = {1, 1073741820, 1072021487, 795410623, 567805267, 660611110, 399803187, 701811303, 29677};
+        return t[i];
+    }
 };
 struct FpK {
     static constexpr int N = 12;
@@ -56,6 +68,15 @@ struct FpK {
     }
     ZK_HD static constexpr uint32_t R2(int i) {
         constexpr uint32_t t[12] = {473175878u, 4108263220u, 164693233u, 175564454u, 1284880085u, 2380613484u, 2476573632u, 1743489193u, 3038352685u, 2591637125u, 2462770090u, 295210981u};
+        return t[i];
+    }
+    ZK_HD static constexpr uint32_t R3(int i) {
+        constexpr uint32_t t[12] = {3645678048u, 3980962923u, 61320696u, 828343070u, 1633561053u, 2589144362u, 2451445601u, 885018206u, 1701988136u, 621990965u, 2440387917u, 178664544u};
+        return t[i];
+    }
+    static constexpr int L30 = 13;
+    ZK_HD static constexpr int32_t P30(int i) {
+        constexpr int32_t t[13] = {1073719979, 670826495, 356515835, 721420204, 821437470, 55215066, 288093811, 316751073, 752313463, 517541166, 698659258, 982409209, 1704209};
         return t[i];
     }
 };
@@ -106,8 +127,58 @@ ZK_HD uint32_t addc32(uint32_t a, uint32_t b, uint32_t& c) { const uint64_t t = 
 ZK_HD uint32_t subb32(uint32_t a, uint32_t b, uint32_t& c) { const uint64_t t = (uint64_t)a - b - c; c = (uint32_t)(t >> 32) & 1u; return (uint32_t)t; }
 #endif
 
+#if !defined(__HIP_DEVICE_COMPILE__)
+// Host side: the same residues on 64-bit limbs
+#if defined(__x86_64__)
+static inline unsigned char addc64(unsigned char c, uint64_t a, uint64_t b, uint64_t& out) {
+    unsigned long long o;
+    c = _addcarry_u64(c, a, b, &o);
+    out = o;
+    return c;
+}
+static inline unsigned char subb64(unsigned char c, uint64_t a, uint64_t b, uint64_t& out) {
+    unsigned long long o;
+    c = _subborrow_u64(c, a, b, &o);
+    out = o;
+    return c;
+}
+#else
+static inline unsigned char addc64(unsigned char c, uint64_t a, uint64_t b, uint64_t& out) {
+    const unsigned __int128 t = (unsigned __int128)a + b + c;
+    out = (uint64_t)t;
+    return (unsigned char)(t >> 64);
+}
+static inline unsigned char subb64(unsigned char c, uint64_t a, uint64_t b, uint64_t& out) {
+    const unsigned __int128 t = (unsigned __int128)a - b - c;
+    out = (uint64_t)t;
+    return (unsigned char)(t >> 64) & 1;
+}
+#endif
+template <int N> struct Host64 {
+    typedef typename KOf<N>::K K;
+    static constexpr int M = N / 2;
+    static constexpr uint64_t P(int i) { return ((uint64_t)K::P(2 * i + 1) << 32) | K::P(2 * i); }
+    static inline void load(uint64_t* x, const Big<N>& a) { __builtin_memcpy(x, a.v, 4 * N); }
+    static inline Big<N> store(const uint64_t* x) { Big<N> r; __builtin_memcpy(r.v, x, 4 * N); return r; }
+    // x - P if x (with `top` above it) is at least P, else x
+    static inline Big<N> reduced(const uint64_t* x, uint64_t top) {
+        uint64_t d[M], r[M];
+        unsigned char br = 0;
+#pragma GCC unroll 8
+        for (int i = 0; i < M; ++i) br = subb64(br, x[i], P(i), d[i]);
+        const uint64_t keep = (br && !top) ? ~(uint64_t)0 : 0;
+        for (int i = 0; i < M; ++i) r[i] = (x[i] & keep) | (d[i] & ~keep);
+        return store(r);
+    }
+};
+#endif
 // r = a - P if a >= P else a   (a < 2P, carry_in = bit 32N of a)
 template <int N> ZK_HD Big<N> reduce_once(const Big<N>& a, uint32_t carry_in = 0) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+    uint64_t x[N / 2];
+    Host64<N>::load(x, a);
+    return Host64<N>::reduced(x, carry_in);
+#else
     typedef typename KOf<N>::K K;
     Big<N> d;
     uint32_t br = 0;
@@ -118,15 +189,38 @@ template <int N> ZK_HD Big<N> reduce_once(const Big<N>& a, uint32_t carry_in = 0
 #pragma unroll
     for (int i = 0; i < N; ++i) r.v[i] = keep ? a.v[i] : d.v[i];
     return r;
+#endif
 }
 template <int N> ZK_HD Big<N> add(const Big<N>& a, const Big<N>& b) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+    uint64_t x[N / 2], y[N / 2];
+    Host64<N>::load(x, a);
+    Host64<N>::load(y, b);
+    unsigned char c = 0;
+#pragma GCC unroll 8
+    for (int i = 0; i < N / 2; ++i) c = addc64(c, x[i], y[i], x[i]);
+    return Host64<N>::reduced(x, c);
+#else
     Big<N> s;
     uint32_t c = 0;
 #pragma unroll
     for (int i = 0; i < N; ++i) s.v[i] = addc32(a.v[i], b.v[i], c);
     return reduce_once(s, c);
+#endif
 }
 template <int N> ZK_HD Big<N> sub(const Big<N>& a, const Big<N>& b) {
+#if !defined(__HIP_DEVICE_COMPILE__)
+    uint64_t x[N / 2], y[N / 2];
+    Host64<N>::load(x, a);
+    Host64<N>::load(y, b);
+    unsigned char br = 0, c = 0;
+#pragma GCC unroll 8
+    for (int i = 0; i < N / 2; ++i) br = subb64(br, x[i], y[i], x[i]);
+    const uint64_t mask = br ? ~(uint64_t)0 : 0;   // a < b: add P back
+#pragma GCC unroll 8
+    for (int i = 0; i < N / 2; ++i) c = addc64(c, x[i], Host64<N>::P(i) & mask, x[i]);
+    return Host64<N>::store(x);
+#else
     typedef typename KOf<N>::K K;
     Big<N> d;
     uint32_t br = 0;
@@ -137,6 +231,7 @@ template <int N> ZK_HD Big<N> sub(const Big<N>& a, const Big<N>& b) {
 #pragma unroll
     for (int i = 0; i < N; ++i) d.v[i] = addc32(d.v[i], K::P(i) & mask, c);
     return d;
+#endif
 }
 template <int N> ZK_HD Big<N> neg(const Big<N>& a) { return sub(big_zero<N>(), a); }
 template <int N> ZK_HD Big<N> dbl(const Big<N>& a) {
@@ -449,41 +544,49 @@ static inline void wide_mac(WideAcc& w, const Big<8>& a, const Big<8>& b) {
 }
 #endif
 // Montgomery product a*b*R^-1 mod p, canonical.  Inputs < p.
+#if !defined(__HIP_DEVICE_COMPILE__)
+// -p^-1 mod 2^64 from p's low 64 bits (p odd): each step of Newton's iteration doubles the bits that are right
+constexpr uint64_t host_inv64(uint64_t p) {
+    uint64_t x = p;                                     // right to three bits
+    for (int i = 0; i < 5; ++i) x *= 2 - p * x;
+    return 0 - x;
+}
+#endif
 template <int N> ZK_HD Big<N> mont_mul(const Big<N>& a, const Big<N>& b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     return mont_mul_columns(a, b);
 #else
-    typedef typename KOf<N>::K K;
-    uint32_t t[N + 1];
-#pragma unroll
-    for (int i = 0; i <= N; ++i) t[i] = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        uint64_t c = 0;
-#pragma unroll
-        for (int j = 0; j < N; ++j) {
-            c += (uint64_t)a.v[j] * b.v[i] + t[j];
-            t[j] = (uint32_t)c;
-            c >>= 32;
+    // Host side (challenges, round polynomials, claims): operand scanning on 64-bit limbs, a quarter of the multiplications of the
+    // 32-bit form
+    typedef Host64<N> H;
+    constexpr int M = N / 2;
+    constexpr uint64_t INV64 = host_inv64(H::P(0));
+    uint64_t x[M], y[M], t[M + 1] = {};
+    H::load(x, a);
+    H::load(y, b);
+#pragma GCC unroll 8
+    for (int i = 0; i < M; ++i) {
+        unsigned __int128 c = 0;
+#pragma GCC unroll 8
+        for (int j = 0; j < M; ++j) {
+            c += (unsigned __int128)x[j] * y[i] + t[j];
+            t[j] = (uint64_t)c;
+            c >>= 64;
         }
-        c += t[N];
-        t[N] = (uint32_t)c;   // bit 32(N+1) is never set: t < 2p + p*2^32 < 2^(32(N+1))
-        const uint32_t m = t[0] * K::INV;
-        c = ((uint64_t)m * K::P(0) + t[0]) >> 32;
-#pragma unroll
-        for (int j = 1; j < N; ++j) {
-            c += (uint64_t)m * K::P(j) + t[j];
-            t[j - 1] = (uint32_t)c;
-            c >>= 32;
+        t[M] += (uint64_t)c;   // nothing above: t < 2p + p*2^64 < 2^(64(M+1))
+        const uint64_t m = t[0] * INV64;
+        c = ((unsigned __int128)m * H::P(0) + t[0]) >> 64;
+#pragma GCC unroll 8
+        for (int j = 1; j < M; ++j) {
+            c += (unsigned __int128)m * H::P(j) + t[j];
+            t[j - 1] = (uint64_t)c;
+            c >>= 64;
         }
-        c += t[N];
-        t[N - 1] = (uint32_t)c;
-        t[N] = (uint32_t)(c >> 32);
+        c += t[M];
+        t[M - 1] = (uint64_t)c;
+        t[M] = (uint64_t)(c >> 64);
     }
-    Big<N> r;
-#pragma unroll
-    for (int i = 0; i < N; ++i) r.v[i] = t[i];
-    return reduce_once(r, t[N]);
+    return H::reduced(t, t[M]);
 #endif
 }
 #if !defined(__HIP_DEVICE_COMPILE__)
@@ -531,9 +634,8 @@ template <int N> ZK_HD Big<N> mont_inverse_fermat(Big<N> a) {
 }
 // Inverse, Montgomery in / Montgomery out (0 -> 0), by the binary "almost Montgomery inverse": shifts, additions and
 // subtractions on u, v, r, s (about 1.4 * bits steps) produce a^-1 * 2^k, and one or two Montgomery products remove
-// the power of two.  About twenty times less work than the exponentiation for one value; it is what bounds the
-// latency of every batched inversion (one inverse per batch, the other lanes wait for it).
-template <int N> ZK_HD Big<N> mont_inverse(const Big<N>& a) {
+// the power of two.  Serves the rare inputs that mont_inverse gives up on, and as its cross-check.
+template <int N> ZK_HD Big<N> mont_inverse_binary(const Big<N>& a) {
     typedef typename KOf<N>::K K;
     constexpr int BITS = (N == 8) ? 255 : 381;
     if (is_zero(a)) return a;
@@ -599,6 +701,152 @@ template <int N> ZK_HD Big<N> mont_inverse(const Big<N>& a) {
         e -= step;
     }
     return y;
+}
+
+// 1 / a mod p of the number as it stands, a != 0.  It is the serial part of every batched inversion and normalisation (one
+// lane works, its workgroup waits), so what counts is its latency: the binary form's 500-odd (Fr) / 760-odd (Fp) steps over all
+// limbs took 140 / 350 us of one lane.  This is Lehmer's form of the Euclidean algorithm: the quotients are found on double
+// approximations of f and g (53 leading bits; centred quotients take 2.4 bits each), gathered into a 2x2 integer matrix until
+// an entry would pass 2^24, and the matrix is then applied to f, g and to the cofactors d, e on signed limbs of 30 bits --
+// eleven to twelve batches for Fr, about seventeen for Fp, of some ten double-precision steps and one pass of multiply-adds.
+// A quotient that is off by rounding costs progress, never correctness: every matrix has determinant +-1 and is applied
+// exactly, so (f, g) keeps its gcd and f = d a, g = e a (mod p) hold throughout.  Inputs whose quotient does not fit (chance
+// about 2^-29 a step) or that do not finish in the given number of batches take the binary form.
+template <int N> ZK_HD bool euclid_inverse(const Big<N>& a, Big<N>& out) {
+    typedef typename KOf<N>::K K;
+    constexpr int L = K::L30;
+    constexpr int32_t M30 = (1 << 30) - 1;
+    int32_t f[L], g[L], d[L], e[L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+        const int w = (30 * i) >> 5, sh = (30 * i) & 31;
+        uint32_t x = a.v[w] >> sh;
+        if (sh > 2 && w + 1 < N) x |= a.v[w + 1] << (32 - sh);
+        f[i] = K::P30(i);
+        g[i] = (int32_t)(x & (uint32_t)M30);
+        d[i] = 0;
+        e[i] = i == 0 ? 1 : 0;
+    }
+    auto approx = [](const int32_t* x) {
+        double r = (double)x[L - 1];
+#pragma unroll
+        for (int i = L - 2; i >= 0; --i) r = __builtin_fma(r, 1073741824.0, (double)x[i]);
+        return r;
+    };
+    auto is_nil = [](const int32_t* x) {
+        int32_t o = 0;
+#pragma unroll
+        for (int i = 0; i < L; ++i) o |= x[i];
+        return o == 0;
+    };
+    auto quotient = [](double x, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        return __builtin_rint(x * __builtin_amdgcn_rcp(y));
+#else
+        return __builtin_rint(x / y);
+#endif
+    };
+    // [x; y] = [[ux, vx], [uy, vy]] [x; y], exact
+    auto apply = [](int32_t* x, int32_t* y, int32_t ux, int32_t vx, int32_t uy, int32_t vy) {
+        int64_t cx = 0, cy = 0;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int32_t a0 = x[i], b0 = y[i];
+            cx += (int64_t)ux * a0;
+            cy += (int64_t)uy * a0;
+            cx += (int64_t)vx * b0;
+            cy += (int64_t)vy * b0;
+            if (i < L - 1) {
+                x[i] = (int32_t)cx & M30;
+                y[i] = (int32_t)cy & M30;
+                cx >>= 30;
+                cy >>= 30;
+            } else {
+                x[i] = (int32_t)cx;
+                y[i] = (int32_t)cy;
+            }
+        }
+    };
+    constexpr double LIM = 16777216.0, FIRST = 536870912.0;
+    bool done = false;
+    for (int batch = 0; batch < 2 * L + 8 && !done; ++batch) {
+        double x = approx(f), y = approx(g);
+        double ux = 1.0, vx = 0.0, uy = 0.0, vy = 1.0, lim = FIRST;      // the batch's first quotient may be larger: nothing multiplies it yet
+        for (int step = 0; step < 32; ++step) {
+            if (y == 0.0) break;
+            const double q = quotient(x, y);
+            const double nu = __builtin_fma(-q, uy, ux), nv = __builtin_fma(-q, vy, vx);
+            if (!(__builtin_fabs(nu) <= lim && __builtin_fabs(nv) <= lim)) break;
+            x = __builtin_fma(-q, y, x);
+            ux = nu;
+            vx = nv;
+            if (x == 0.0) break;
+            const double q2 = quotient(y, x);
+            const double mu = __builtin_fma(-q2, ux, uy), mv = __builtin_fma(-q2, vx, vy);
+            if (__builtin_fabs(vx) > 1.0) lim = LIM;
+            if (!(__builtin_fabs(mu) <= lim && __builtin_fabs(mv) <= lim)) break;
+            y = __builtin_fma(-q2, x, y);
+            uy = mu;
+            vy = mv;
+            lim = LIM;
+        }
+        const int32_t iux = (int32_t)ux, ivx = (int32_t)vx, iuy = (int32_t)uy, ivy = (int32_t)vy;
+        if (ivx == 0 && iuy == 0) return false;      // no quotient fits
+        apply(f, g, iux, ivx, iuy, ivy);
+        apply(d, e, iux, ivx, iuy, ivy);
+        done = is_nil(f) || is_nil(g);
+    }
+    if (!done) return false;
+    // the other of the two is +-1; its cofactor times that sign is the inverse, up to multiples of p
+    const bool use_e = is_nil(f);
+    bool negative = use_e ? g[L - 1] < 0 : f[L - 1] < 0;
+    int32_t r[L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) r[i] = use_e ? e[i] : d[i];
+    if (r[L - 1] < 0) {                     // |r|, with its sign kept aside
+        negative = !negative;
+        int32_t c = 0;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int32_t t = c - r[i];
+            r[i] = i < L - 1 ? t & M30 : t;
+            c = t >> 30;
+        }
+    }
+    constexpr int TOP = (N == 8) ? 256 : 382;           // |r| below 2^TOP < 3p
+    if (r[L - 1] >> (TOP - 30 * (L - 1))) return false;
+    Big<N> y;
+#pragma unroll
+    for (int w = 0; w < N; ++w) {
+        const int i = (32 * w) / 30, sh = 32 * w - 30 * i;
+        uint32_t v = (uint32_t)r[i] >> sh;
+        if (i + 1 < L) v |= (uint32_t)r[i + 1] << (30 - sh);
+        if (i + 2 < L && 60 - sh < 32) v |= (uint32_t)r[i + 2] << (60 - sh);
+        y.v[w] = v;
+    }
+    y = reduce_once(reduce_once(y));
+    out = negative ? neg(y) : y;
+    return true;
+}
+#if defined(__HIP_DEVICE_COMPILE__)
+static __device__ __attribute__((noinline)) Fr mont_inverse_rare(const Fr a) { return mont_inverse_binary(a); }
+static __device__ __attribute__((noinline)) Fp mont_inverse_rare(const Fp a) { return mont_inverse_binary(a); }
+#else
+template <int N> inline Big<N> mont_inverse_rare(const Big<N>& a) { return mont_inverse_binary(a); }
+#endif
+// 1 / a mod p of the number as it stands (0 -> 0)
+template <int N> ZK_HD Big<N> plain_inverse(const Big<N>& a) {
+    if (is_zero(a)) return a;
+    Big<N> r;
+    if (euclid_inverse(a, r)) return r;
+    return from_mont(from_mont(mont_inverse_rare(a)));      // the binary form returns R^2 / a
+}
+template <int N> ZK_HD Big<N> mont_inverse(const Big<N>& a) {
+    typedef typename KOf<N>::K K;
+    Big<N> r3;
+#pragma unroll
+    for (int i = 0; i < N; ++i) r3.v[i] = K::R3(i);
+    return mont_mul(plain_inverse(a), r3);                   // (aR)^-1 R^3 / R = a^-1 R
 }
 
 // ---- standard-form helpers (tensors hold standard-form residues) ---------------------------------

@@ -119,27 +119,26 @@ __global__ void __launch_bounds__(GT) k_g1_me_step(G1Jac* __restrict__ out, cons
 }
 
 // ---- batch normalisation to z = 1 -------------------------------------------------------------------------
-// Each lane owns CH consecutive points: prefix products of z, one Fermat inversion, back-substitution.
+// Each lane owns CH points, GT apart: prefix products of z, one inversion, back-substitution.
 // Infinity (z == 0) is skipped in the product and written as all-zero limbs.
-static constexpr int CH = 8;
-template <bool AFFINE_OUT> __global__ void __launch_bounds__(GT) k_g1_normalize(void* outv, const G1Jac* in, size_t n) {
-    const size_t base = ((size_t)blockIdx.x * GT + threadIdx.x) * CH;
+template <bool AFFINE_OUT, int CH> __global__ void __launch_bounds__(GT) k_g1_normalize(void* outv, const G1Jac* in, size_t n) {
+    const size_t base = (size_t)blockIdx.x * GT * CH + threadIdx.x;
     if (base >= n) return;
     Fp pre[CH];
     Fp run = big_one_mont<12>();
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
         pre[c] = run;
-        if (base + c < n) {
-            const Fp z = in[base + c].z;
+        if (base + (size_t)c * GT < n) {
+            const Fp z = in[base + (size_t)c * GT].z;
             if (!is_zero(z)) run = fp_mul(run, z);
         }
     }
     Fp inv = mont_inverse(run);
 #pragma unroll
     for (int c = CH - 1; c >= 0; --c) {
-        if (base + c >= n) continue;
-        const G1Jac p = in[base + c];
+        if (base + (size_t)c * GT >= n) continue;
+        const G1Jac p = in[base + (size_t)c * GT];
         Fp ox = big_zero<12>(), oy = big_zero<12>(), oz = big_zero<12>();
         if (!is_zero(p.z)) {
             const Fp zi = fp_mul(inv, pre[c]);
@@ -151,12 +150,19 @@ template <bool AFFINE_OUT> __global__ void __launch_bounds__(GT) k_g1_normalize(
         }
         if (AFFINE_OUT) {
             G1Affine* out = reinterpret_cast<G1Affine*>(outv);
-            out[base + c].x = ox; out[base + c].y = oy;
+            out[base + (size_t)c * GT].x = ox; out[base + (size_t)c * GT].y = oy;
         } else {
             G1Jac* out = reinterpret_cast<G1Jac*>(outv);
-            out[base + c].x = ox; out[base + c].y = oy; out[base + c].z = oz;
+            out[base + (size_t)c * GT].x = ox; out[base + (size_t)c * GT].y = oy; out[base + (size_t)c * GT].z = oz;
         }
     }
+}
+
+// An inversion costs a lane about ten products and a point's own part eight: one point a lane while the launch is two waves a SIMD
+// or less (its time is then about one lane's: 131072 generators took 408 us with eight a lane and the binary inverse), four a lane above.
+template <bool AFFINE_OUT> static void g1_normalize_queue(void* out, const G1Jac* in, size_t n, hipStream_t st) {
+    if (n <= (size_t)1 << 17) hipLaunchKernelGGL((k_g1_normalize<AFFINE_OUT, 1>), dim3(cdiv(n, (size_t)GT)), dim3(GT), 0, st, out, in, n);
+    else hipLaunchKernelGGL((k_g1_normalize<AFFINE_OUT, 4>), dim3(cdiv(n, (size_t)GT * 4)), dim3(GT), 0, st, out, in, n);
 }
 
 // the normalised points once more in the 29-bit-limb form that the bucket kernels add in (infinity stays all-zero)
@@ -1353,10 +1359,10 @@ static int open_prep_build(A29* out, const G1Jac* gens, size_t n, Arena& arena, 
     Scratch& pj = arena.add(sizeof(G1Jac) * half_up);
     Scratch& paff = arena.add(sizeof(G1Affine) * half_up);
     if (aff.rc || pj.rc || paff.rc) return aff.rc ? aff.rc : (pj.rc ? pj.rc : paff.rc);
-    hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(n, CH), GT)), dim3(GT), 0, st, aff.p, gens, n);
+    g1_normalize_queue<true>(aff.p, gens, n, st);
     hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(n, 256)), dim3(256), 0, st, out, aff.as<G1Affine>(), n);
     hipLaunchKernelGGL(k_open_pair_points, dim3(cdiv(half_up, GT)), dim3(GT), 0, st, pj.as<G1Jac>(), aff.as<G1Affine>(), n, half_up, 0);
-    hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(half_up, CH), GT)), dim3(GT), 0, st, paff.p, pj.as<G1Jac>(), half_up);
+    g1_normalize_queue<true>(paff.p, pj.as<G1Jac>(), half_up, st);
     hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(half_up, 256)), dim3(256), 0, st, out + n, paff.as<G1Affine>(), half_up);
     ZK_LAUNCH_CHECK();
     return 0;
@@ -1694,7 +1700,7 @@ int zk_g1_me(uint32_t* out_host, const void* a, size_t n, const uint32_t* u, int
 // canonical form: z = ONE (Montgomery), infinity = all-zero limbs.  out may alias in.
 int zk_g1_normalize(void* out, const void* in, size_t n, void* st) {
     if (n == 0) return 0;
-    hipLaunchKernelGGL(k_g1_normalize<false>, dim3(cdiv(cdiv(n, CH), GT)), dim3(GT), 0, (hipStream_t)st, out, (const G1Jac*)in, n);
+    g1_normalize_queue<false>(out, (const G1Jac*)in, n, (hipStream_t)st);
     ZK_LAUNCH_CHECK();
     return 0;
 }
@@ -1734,7 +1740,7 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     hipLaunchKernelGGL(k_msm_table_bases, dim3(cdiv(ngen, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (const G1Jac*)gens, ngen, c, nwin);
     for (uint32_t logk = 0; logk + 1 < c; ++logk)
         hipLaunchKernelGGL(k_msm_table_fill, dim3(cdiv(((size_t)nwin * ngen) << logk, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (size_t)nwin * ngen, c - 1, logk);
-    hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(tab_n, CH), GT)), dim3(GT), 0, st, taba.p, tabj.as<G1Jac>(), tab_n);
+    g1_normalize_queue<true>(taba.p, tabj.as<G1Jac>(), tab_n, st);
     Scratch tab29(sizeof(A29) * tab_n, st);
     if (tab29.rc) return tab29.rc;
     hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(tab_n, 256)), dim3(256), 0, st, tab29.as<A29>(), taba.as<G1Affine>(), tab_n);
@@ -1780,7 +1786,7 @@ int zk_g1_fixed_base_mul(void* out, const uint32_t* base_host, const void* scala
         hipLaunchKernelGGL(k_msm_table_bases, dim3(1), dim3(GT), 0, st, tabj.as<G1Jac>(), b.as<G1Jac>(), (size_t)1, 8u, FB_WIN);
         for (uint32_t logk = 0; logk < 7; ++logk)
             hipLaunchKernelGGL(k_msm_table_fill, dim3(cdiv((size_t)FB_WIN << logk, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (size_t)FB_WIN, 7u, logk);
-        hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(tab_n, CH), GT)), dim3(GT), 0, st, taba.p, tabj.as<G1Jac>(), tab_n);
+        g1_normalize_queue<true>(taba.p, tabj.as<G1Jac>(), tab_n, st);
         hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(tab_n, 256)), dim3(256), 0, st, (A29*)tab, taba.as<G1Affine>(), tab_n);
         ZK_LAUNCH_CHECK();
         ZK_HIP(hipStreamSynchronize(st));               // later calls may come on other streams
@@ -1816,7 +1822,7 @@ int zk_g1_open_round(void* new_scalars, void* new_gens, uint32_t* sums_host, con
     if (rc) return rc;
     hipLaunchKernelGGL(k_a29_to_jac, dim3(cdiv(new_size, GT)), dim3(GT), 0, st, (G1Jac*)new_gens, n29.as<A29>(), new_size);
     hipLaunchKernelGGL(k_open_horner, dim3(3, 1), dim3(GT), 0, st, pts.as<G1Jac>(), wsum.as<G1Jac>(), 1u, 3u, 0u);
-    hipLaunchKernelGGL(k_g1_normalize<false>, dim3(1), dim3(GT), 0, st, pts.p, pts.as<G1Jac>(), (size_t)3);
+    g1_normalize_queue<false>(pts.p, pts.as<G1Jac>(), (size_t)3, st);
     ZK_LAUNCH_CHECK();
     void* stage = nullptr;
     rc = staging(&stage, sizeof(G1Jac) * 3);
@@ -1872,7 +1878,7 @@ static int open_cross_sums_queue(Arena& arena, const OpenItem* items, int count,
         Scratch& a29 = arena.add(sizeof(A29) * terms);
         Scratch& dg = arena.add((size_t)(MW + 1) * terms);
         if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
-        hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(terms, CH), GT)), dim3(GT), 0, aux, aff.p, (const G1Jac*)items[i].rows, terms);
+        g1_normalize_queue<true>(aff.p, (const G1Jac*)items[i].rows, terms, aux);
         hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(terms, 256)), dim3(256), 0, aux, a29.as<A29>(), aff.as<G1Affine>(), terms);
         base[i] = a29.as<A29>();
         digs[i] = dg.as<int8_t>();
@@ -2110,7 +2116,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     }
     if (!tail_done)
         for (int i = 0; i < count; ++i) hipLaunchKernelGGL(k_open_finish, dim3(1), dim3(GT), 0, st, pts.as<G1Jac>() + npts * i, cg[i], (uint32_t)rounds);
-    hipLaunchKernelGGL(k_g1_normalize<false>, dim3(cdiv(cdiv(npts * count, CH), GT)), dim3(GT), 0, st, pts.p, pts.as<G1Jac>(), npts * count);
+    g1_normalize_queue<false>(pts.p, pts.as<G1Jac>(), npts * count, st);
     ZK_LAUNCH_CHECK();
     for (int i = 0; i < count; ++i) job.final_scalar[i] = cs[i];
     return 0;
@@ -2262,7 +2268,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                 pr->comb3 = nullptr;
             } else {
                 static_assert(COMB_W % 2 == 0, "the doublings alternate between two buffers and must end in the table");
-                hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(n, CH), GT)), dim3(GT), 0, st, aff.p, (const G1Jac*)gens, n);
+                g1_normalize_queue<true>(aff.p, (const G1Jac*)gens, n, st);
                 for (int b = 0; b < JUMP_TABS; ++b) {
                     G1Jac* T = tj.as<G1Jac>() + (size_t)b * COMB_N * no;
                     auto entry = [&](int m) { return T + (size_t)(m - 1) * no; };
@@ -2281,7 +2287,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                         hipLaunchKernelGGL(k_g1_add, dim3(cdiv(no, GT)), dim3(GT), 0, st, entry(m), entry(prev), entry(m ^ prev), no, no, 0);
                     }
                 }
-                hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(ne, CH), GT)), dim3(GT), 0, st, ta.p, tj.as<G1Jac>(), ne);
+                g1_normalize_queue<true>(ta.p, tj.as<G1Jac>(), ne, st);
                 hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(ne, 256)), dim3(256), 0, st, (A29*)pr->comb3, ta.as<G1Affine>(), ne);
                 if (hipGetLastError() != hipSuccess) rc = hip_fail(hipErrorLaunchFailure, "jump table build", __FILE__, __LINE__);
             }
@@ -2322,10 +2328,10 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                     }
                 };
                 G1Jac* T = tj.as<G1Jac>();
-                hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(n, CH), GT)), dim3(GT), 0, st, aff.p, (const G1Jac*)gens, n);
+                g1_normalize_queue<true>(aff.p, (const G1Jac*)gens, n, st);
                 hipLaunchKernelGGL(k_open_pair_points, dim3(cdiv(np, GT)), dim3(GT), 0, st, T, aff.as<G1Affine>(), n, np, 1);
                 fill(T, np);
-                hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(ne, CH), GT)), dim3(GT), 0, st, ta.p, tj.as<G1Jac>(), ne);
+                g1_normalize_queue<true>(ta.p, tj.as<G1Jac>(), ne, st);
                 hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(ne, 256)), dim3(256), 0, st, (A29*)pr->comb, ta.as<G1Affine>(), ne);
                 if (second) {
                     // F from the odd-numbered generators, H from the first round's differences (entry 1 of its table, affine in ta);
@@ -2334,7 +2340,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                     hipLaunchKernelGGL(k_open_pair_diff, dim3(cdiv(nq, GT)), dim3(GT), 0, st, T + ne2, ta.as<G1Affine>(), (size_t)0, (size_t)1, np, nq);
                     fill(T, nq);
                     fill(T + ne2, nq);
-                    hipLaunchKernelGGL(k_g1_normalize<true>, dim3(cdiv(cdiv(2 * ne2, CH), GT)), dim3(GT), 0, st, ta.p, tj.as<G1Jac>(), 2 * ne2);
+                    g1_normalize_queue<true>(ta.p, tj.as<G1Jac>(), 2 * ne2, st);
                     hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(2 * ne2, 256)), dim3(256), 0, st, (A29*)pr->comb2, ta.as<G1Affine>(), 2 * ne2);
                 }
                 if (rc == 0 && hipGetLastError() != hipSuccess) rc = hip_fail(hipErrorLaunchFailure, "comb build", __FILE__, __LINE__);

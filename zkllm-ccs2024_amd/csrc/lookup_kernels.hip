@@ -318,113 +318,45 @@ __global__ void __launch_bounds__(TPB) k_range_table(Fr* __restrict__ table, int
 }
 
 // ---- batch inversion -----------------------------------------------------------------------------------------------
-// out[i] = 1 / (in[i] + beta), 0 where the sum is 0.  A workgroup inverts T * 8 values with one field inversion:
-// every lane multiplies its 8 values up, the T lane products go up a product tree in LDS, the root is inverted, and
-// the inverse comes down the tree (a child's inverse is the parent's inverse times the sibling) and through each
-// lane's values backwards.  About 3.4 multiplications per value.
-// The standard-form inputs are used as they are: x is the Montgomery representation of x/R, every product of the
-// scheme is then a Montgomery representation too, and the two stray factors of R in each result are removed once per
-// workgroup by multiplying the root's inverse by R^-1 (a Montgomery product with R^-1 multiplies by R^-2).
-//
-// One field inversion is a serial computation of about 140 us on one lane, during which the rest of its workgroup
-// waits with its registers held.  Large inputs therefore run in three steps (MODE): BI_UP only multiplies up to the
-// workgroup's root and writes it to roots[workgroup]; the roots -- a few thousand numbers -- are inverted by this same
-// scheme (the corrected inverse of a root is exactly the plain inverse of the number written); BI_DOWN repeats the
-// way up, takes its root's inverse from roots_inv[workgroup] and comes down.  The two large steps then have no serial part.
-enum { BI_FULL = 0, BI_UP = 1, BI_DOWN = 2 };
-static constexpr int BI_T = 512, BI_CH = 8;        // single-step form (small inputs)
-static constexpr int BI_T3 = 256;                  // three-step form
-template <int T, int MODE>
-__global__ void __launch_bounds__(T) k_batch_inv(Fr* __restrict__ out, const Fr* __restrict__ in, const Fr beta, size_t n, Fr* __restrict__ roots, const Fr* __restrict__ roots_inv) {
-    __shared__ uint32_t node[8][2 * T];      // level 0 (lane products) at [0, T), level 1 at [T, T + T/2), ... root at 2T - 2
-    const uint32_t t = threadIdx.x;
-    const size_t base = ((size_t)blockIdx.x * T + t) * BI_CH;
-    const Fr one_m = big_one_mont<8>();
-    Fr x[BI_CH], pre[BI_CH];
+// out[i] = 1 / (in[i] + beta), 0 where the sum is 0.  A lane takes CH values a workgroup apart: it multiplies them up, inverts
+// the product and comes back down, with no exchange between lanes.  plain_inverse costs a lane about ten Montgomery products,
+// so with CH = 8 a value costs (24 + 10) / 8 of them, a quarter more than with a product tree over the workgroup and one
+// inversion for it, and the serial part that such a root has (and three launches at the larger sizes) is gone: 2^16 table entries
+// took 210 us that way.  The inputs are used as they are: Montgomery products of plain numbers carry factors R^-1 that cancel
+// when the product's plain inverse is what comes back down.
+template <int CH>
+__global__ void __launch_bounds__(256) k_batch_inv(Fr* __restrict__ out, const Fr* __restrict__ in, const Fr beta, size_t n) {
+    const size_t base = (size_t)blockIdx.x * 256 * CH + threadIdx.x;
+    if (base >= n) return;
+    Fr x[CH], pre[CH];
     uint32_t nz = 0;
-    Fr tot = one_m;
+    Fr tot = big_one_mont<8>();
 #pragma unroll
-    for (int c = 0; c < BI_CH; ++c) {
+    for (int c = 0; c < CH; ++c) {
+        const size_t i = base + (size_t)c * 256;
         Fr v = big_zero<8>();
-        if (base + c < n) v = add(in[base + c], beta);
+        if (i < n) v = add(in[i], beta);
         const bool nzc = !is_zero(v);
         nz |= (nzc ? 1u : 0u) << c;
-        x[c] = nzc ? v : one_m;
+        x[c] = nzc ? v : big_one_mont<8>();
         pre[c] = tot;
         tot = mont_mul(tot, x[c]);
     }
-    auto put = [&](const Fr& v, uint32_t i) {
+    Fr inv_run = plain_inverse(tot);
 #pragma unroll
-        for (int l = 0; l < 8; ++l) node[l][i] = v.v[l];
-    };
-    auto get = [&](uint32_t i) {
-        Fr v;
-#pragma unroll
-        for (int l = 0; l < 8; ++l) v.v[l] = node[l][i];
-        return v;
-    };
-    put(tot, t);
-    __syncthreads();
-    // up: level L has T >> L nodes starting at off(L) = 2*T - (2*T >> L)
-    uint32_t off = 0;
-    for (uint32_t cnt = T / 2; cnt >= 1; cnt >>= 1) {
-        const uint32_t noff = off + 2 * cnt;
-        if (t < cnt) put(mont_mul(get(off + 2 * t), get(off + 2 * t + 1)), noff + t);
-        __syncthreads();
-        off = noff;
-    }
-    // off is now the root's index
-    if (MODE == BI_UP) {
-        if (t == 0) roots[blockIdx.x] = get(off);
-        return;
-    }
-    if (MODE == BI_DOWN) {
-        if (t == 0) put(roots_inv[blockIdx.x], off);
-    } else if (t < 64) {
-        Fr inv = mont_inverse(get(off));
-        constexpr uint32_t RINV[8] = {4269129792u, 334977897u, 165441631u, 2876230287u, 1333208682u, 1912866698u, 805346647u, 465471123u};   // R^-1 mod r
-        Fr k;
-#pragma unroll
-        for (int l = 0; l < 8; ++l) k.v[l] = RINV[l];
-        inv = mont_mul(inv, k);
-        if (t == 0) put(inv, off);
-    }
-    __syncthreads();
-    // down: the inverse of a node replaces its value; a child reads the parent's inverse and its sibling's value first
-    for (uint32_t cnt = 1; cnt < (uint32_t)T; cnt <<= 1) {
-        const uint32_t coff = off - 2 * cnt;          // children level: 2*cnt nodes
-        Fr inv_c = one_m;
-        if (t < 2 * cnt) inv_c = mont_mul(get(off + (t >> 1)), get(coff + (t ^ 1u)));
-        __syncthreads();
-        if (t < 2 * cnt) put(inv_c, coff + t);
-        __syncthreads();
-        off = coff;
-    }
-    Fr inv_run = get(t);
-#pragma unroll
-    for (int c = BI_CH - 1; c >= 0; --c) {
+    for (int c = CH - 1; c >= 0; --c) {
+        const size_t i = base + (size_t)c * 256;
         const Fr inv_c = mont_mul(inv_run, pre[c]);
         inv_run = mont_mul(inv_run, x[c]);
-        if (base + c < n) out[base + c] = ((nz >> c) & 1u) ? inv_c : big_zero<8>();
+        if (i < n) out[i] = ((nz >> c) & 1u) ? inv_c : big_zero<8>();
     }
 }
-// queues out = 1 / (in + beta) on st; scratch comes from the arena, which must outlive the launches
-static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, Arena& arena, hipStream_t st) {
+// queues out = 1 / (in + beta) on st
+static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, hipStream_t st) {
     if (n == 0) return 0;
-    if (n <= (size_t)2 * BI_T * BI_CH) {
-        hipLaunchKernelGGL((k_batch_inv<BI_T, BI_FULL>), dim3(cdiv(n, (size_t)BI_T * BI_CH)), dim3(BI_T), 0, st, out, in, beta, n, (Fr*)nullptr, (const Fr*)nullptr);
-        ZK_LAUNCH_CHECK();
-        return 0;
-    }
-    const size_t m = cdiv(n, (size_t)BI_T3 * BI_CH);
-    Scratch& roots = arena.add(sizeof(Fr) * 2 * m);
-    if (roots.rc) return roots.rc;
-    Fr* r = roots.as<Fr>();
-    hipLaunchKernelGGL((k_batch_inv<BI_T3, BI_UP>), dim3(m), dim3(BI_T3), 0, st, (Fr*)nullptr, in, beta, n, r, (const Fr*)nullptr);
-    ZK_LAUNCH_CHECK();
-    int rc = batch_inv_queue(r + m, r, big_zero<8>(), m, arena, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL((k_batch_inv<BI_T3, BI_DOWN>), dim3(m), dim3(BI_T3), 0, st, out, in, beta, n, (Fr*)nullptr, (const Fr*)(r + m));
+    // few values a lane while that leaves the chip at two waves a SIMD or less: the launch then takes what one lane takes
+    if (n <= (size_t)1 << 18) hipLaunchKernelGGL(k_batch_inv<2>, dim3(cdiv(n, 512)), dim3(256), 0, st, out, in, beta, n);
+    else hipLaunchKernelGGL(k_batch_inv<8>, dim3(cdiv(n, 2048)), dim3(256), 0, st, out, in, beta, n);
     ZK_LAUNCH_CHECK();
     return 0;
 }
@@ -518,12 +450,7 @@ __device__ __forceinline__ Fr hinted_query(const Fr* __restrict__ S, size_t i, c
 static __device__ __attribute__((noinline)) Fr inv_plus_beta_alone(const Fr sv, const Fr beta) {
     const Fr v = add(sv, beta);
     if (is_zero(v)) return big_zero<8>();
-    // v is the Montgomery form of v/R: its Montgomery inverse is R^2/v, and a Montgomery product with R^-1 leaves 1/v
-    constexpr uint32_t RINV[8] = {4269129792u, 334977897u, 165441631u, 2876230287u, 1333208682u, 1912866698u, 805346647u, 465471123u};
-    Fr k;
-#pragma unroll
-    for (int l = 0; l < 8; ++l) k.v[l] = RINV[l];
-    return mont_mul(mont_inverse(v), k);
+    return plain_inverse(v);
 }
 // *unit (optional): the returned a satisfies a * (sv + beta) == 1 by construction (the hinted entry matched and is invertible)
 __device__ __forceinline__ Fr inv_by_hint(const Fr& sv, size_t i, const HintSrc& h, bool* unit = nullptr) {
@@ -2084,9 +2011,7 @@ int zk_range_table(void* table, int32_t low, uint32_t len, uint32_t table_size, 
 // out[i] = 1 / (in[i] + beta), standard form; 0 where in[i] + beta == 0 (tlookup_inv_kernel tlookup.cu:50-62)
 int zk_fr_batch_inv(void* out, const void* in, const uint32_t* beta, size_t n, void* st) {
     if (n == 0) return 0;
-    Arena tmp((hipStream_t)st);
-    // large inputs use scratch memory that goes back to the allocator when this returns, remembered as last used on `st`
-    return batch_inv_queue((Fr*)out, (const Fr*)in, load_fr(beta), n, tmp, (hipStream_t)st);
+    return batch_inv_queue((Fr*)out, (const Fr*)in, load_fr(beta), n, (hipStream_t)st);
 }
 // E[t] for t < 2^k (Montgomery form) from k standard-form challenges; out holds 2^k elements
 int zk_eq_table(void* out, const uint32_t* u, int k, void* stv) {
@@ -2441,10 +2366,18 @@ static bool eq_prefix_scales(std::vector<Fr>& out, const uint32_t* u_eq, int rou
     std::vector<Fr> c((size_t)rounds);
     const Fr one = big_one_mont<8>();
     if (rounds >= 1) c[0] = one;
+    std::vector<Fr> d((size_t)rounds);
     for (int r = 1; r < rounds; ++r) {
-        const Fr d = sub(one, to_mont(load_fr(u_eq + 8 * (size_t)(k - r))));
-        if (is_zero(d)) return false;
-        c[r] = mont_mul(c[r - 1], mont_inverse(d));
+        d[r] = sub(one, to_mont(load_fr(u_eq + 8 * (size_t)(k - r))));
+        if (is_zero(d[r])) return false;
+        c[r] = mont_mul(c[r - 1], d[r]);
+    }
+    if (rounds >= 2) {          // c[r] = 1 / (d[1] ... d[r]): one inversion, then back down
+        Fr inv = mont_inverse(c[rounds - 1]);
+        for (int r = rounds - 1; r >= 1; --r) {
+            c[r] = inv;
+            inv = mont_mul(inv, d[r]);
+        }
     }
     out.swap(c);
     return true;
@@ -2957,7 +2890,7 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     Scratch& B = job->arena.add(sizeof(Fr) * N);
     Scratch& dp = job->arena.add(sizeof(Fr) * (reduce_grid(N) + 1));
     if (B.rc || dp.rc) return B.rc ? B.rc : dp.rc;
-    rc = batch_inv_queue(B.as<Fr>(), (const Fr*)T, b, N, job->arena, st);
+    rc = batch_inv_queue(B.as<Fr>(), (const Fr*)T, b, N, st);
     const Fr* Aptr = nullptr;
     HintSrc hs;
     if (rc == 0 && hint) {
@@ -2991,7 +2924,7 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     } else if (rc == 0) {
         Scratch& A = job->arena.add(sizeof(Fr) * D);
         rc = A.rc;
-        if (rc == 0) rc = batch_inv_queue(A.as<Fr>(), (const Fr*)S, b, D, job->arena, st);
+        if (rc == 0) rc = batch_inv_queue(A.as<Fr>(), (const Fr*)S, b, D, st);
         Aptr = A.as<Fr>();
     }
     if (rc) return rc;

@@ -77,12 +77,10 @@ Polynomial& Polynomial::operator-=(const Polynomial& o) { *this = *this - o; ret
 Polynomial& Polynomial::operator*=(const Polynomial& o) { *this = *this * o; return *this; }
 
 Fr_t Polynomial::operator()(const Fr_t& x) {
-    Fr_t pw = kOne, res = kZero;
-    for (size_t i = 0; i < coefficients_.size(); ++i) {
-        res = res + coefficients_[i] * pw;
-        pw = pw * x;
-    }
-    return res;
+    const zk::Fr xm = zk::to_mont(F(x));          // one Montgomery product a coefficient
+    zk::Fr res = zk::big_zero<8>();
+    for (size_t i = coefficients_.size(); i-- > 0;) res = zk::add(zk::mont_mul(xm, res), F(coefficients_[i]));
+    return T(res);
 }
 int Polynomial::getDegree() const { return (int)coefficients_.size() - 1; }
 void Polynomial::setCoefficients(int degree, Fr_t* c) { coefficients_.assign(c, c + degree + 1); }

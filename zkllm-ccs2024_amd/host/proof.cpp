@@ -318,8 +318,11 @@ Fr_t multi_hadamard_end(HadamardPending& pd, vector<Polynomial>& proof) {
         std::vector<Fr_t> coefs(sums.begin() + (size_t)r * (K + 1), sums.begin() + (size_t)(r + 1) * (K + 1));
         proof.push_back(Polynomial(coefs));
         zk_record(coefs);
-        Polynomial p = proof.back() * Polynomial::eq(pd.u[k - 1 - r]);
-        if (claim != p(kZero) + p(kOne)) throw std::runtime_error("multi_hadamard_sumchecks: claim != p(0) + p(1)");
+        // eq(u) is 1 - u at 0 and u at 1; the polynomial is its first coefficient at 0 and the sum of all at 1
+        const Fr_t& ur = pd.u[k - 1 - r];
+        Fr_t at_one = coefs[0];
+        for (uint i = 1; i <= K; ++i) at_one = at_one + coefs[i];
+        if (claim != (kOne - ur) * coefs[0] + ur * at_one) throw std::runtime_error("multi_hadamard_sumchecks: claim != p(0) + p(1)");
         claim = proof.back()(pd.v[k - 1 - r]);
     }
     return claim;

@@ -1,10 +1,12 @@
 #include "tlookup.hpp"
 
+#include <cstring>
+
 #include "../../include/zkllm_hip.h"
+#include "../csrc/field.hpp"
 
 #define ZKC(call) zk_check((call), #call)
 
-static const Fr_t kZero{{0, 0, 0, 0, 0, 0, 0, 0}};
 static const Fr_t kOne{{1, 0, 0, 0, 0, 0, 0, 0}};
 // 1/2 mod r (tlookup.cu:179-180)
 static const Fr_t TWO_INV{{2147483649u, 2147483647u, 2147429887u, 2849952257u, 80800770u, 429714436u, 2496577188u, 972477353u}};
@@ -158,46 +160,65 @@ Fr_t tLookup_sumcheck_end(LookupPending& pd) {
     const vector<Fr_t>&u = pd.u, &v = pd.v;
     const uint n1 = ceilLog2(D / N);               // phase-1 rounds
     const uint k = (uint)u.size();
-    Fr_t alpha = pd.alpha;
-    Fr_t alpha_sq = pd.alpha * pd.alpha;
-    Fr_t claim = pd.alpha + alpha_sq;
-    if (k == 0) { zk_record(claim); return claim; }
+    if (k == 0) {
+        const Fr_t claim = pd.alpha + pd.alpha * pd.alpha;
+        zk_record(claim);
+        return claim;
+    }
     Fr_t bm;
     std::vector<Fr_t> sums((size_t)k * 11);
     void* h = pd.handle;
     pd.handle = nullptr;
     ZKC(zk_lookup_prove_end(h, bm.val, sums[0].val));
     pd.keep.clear();
-    Fr_t C = alpha_sq - bm;
-    const Fr_t inv_ratio = Fr_t{{N, 0, 0, 0, 0, 0, 0, 0}} / Fr_t{{D, 0, 0, 0, 0, 0, 0, 0}};
+    // Every product of the rounds has a factor that is known in Montgomery form (alpha, the eq factors, the challenge, N / D), so it
+    // is one Montgomery product and leaves the other factor's standard form; the polynomials are their four coefficients.
+    using zk::Fr;
+    auto load = [](const Fr_t& x) { Fr r; memcpy(r.v, x.val, 32); return r; };
+    auto store = [](const Fr& x) { Fr_t r; memcpy(r.val, x.v, 32); return r; };
+    const Fr one = load(kOne), half_m = zk::to_mont(load(TWO_INV));
+    const Fr inv_ratio_m = zk::to_mont(load(Fr_t{{N, 0, 0, 0, 0, 0, 0, 0}} / Fr_t{{D, 0, 0, 0, 0, 0, 0, 0}}));
+    Fr alpha_m = zk::to_mont(load(pd.alpha));
+    const Fr alpha_sq = zk::mont_mul(alpha_m, load(pd.alpha));
+    Fr alpha_sq_m = zk::to_mont(alpha_sq);
+    Fr claim = zk::add(load(pd.alpha), alpha_sq);
+    Fr C = zk::sub(alpha_sq, load(bm));
+    std::vector<Fr_t> coefs(4);
     for (uint r = 0; r < k; ++r) {
-        const Fr_t* s = &sums[(size_t)r * 11];
+        Fr s[11];
+        memcpy(s, &sums[(size_t)r * 11], sizeof(s));
         const bool phase2 = r >= n1;
-        const Fr_t& ub = u[k - 1 - r];
-        const Fr_t& vr = phase2 ? v[k - 1 - (r - n1)] : v[n1 - 1 - r];
-        Polynomial p;
-        if (!phase2) {
-            Polynomial p0({alpha * s[0], alpha * s[1], alpha * s[2]});
-            Polynomial p1({s[3], s[4]});
-            p0 *= Polynomial::eq(ub);
-            p = p0 + p1 + Polynomial(C * TWO_INV);
-        } else {
-            const Fr_t coef = inv_ratio * alpha_sq;
-            Polynomial p0({alpha * s[0] + coef * s[5], alpha * s[1] + coef * s[6], alpha * s[2] + coef * s[7]});
-            Polynomial p1({s[3], s[4]});
-            Polynomial p2({s[8], s[9], s[10]});
-            p = Polynomial::eq(ub) * p0 + p1 - p2 * Polynomial(inv_ratio);
+        const Fr ub = load(u[k - 1 - r]), vr = load(phase2 ? v[k - 1 - (r - n1)] : v[n1 - 1 - r]);
+        const Fr ub_m = zk::to_mont(ub), vr_m = zk::to_mont(vr);
+        const Fr one_m = zk::big_one_mont<8>();
+        // eq(ub) = e0 + e1 x; p = eq(ub) q + (s3 + s4 x) + the rest
+        const Fr e0 = zk::sub(one_m, ub_m), e1 = zk::sub(zk::dbl(ub_m), one_m);
+        Fr q[3], c[4];
+        for (int i = 0; i < 3; ++i) q[i] = zk::mont_mul(alpha_m, s[i]);
+        if (phase2) {
+            const Fr coef_m = zk::mont_mul(inv_ratio_m, alpha_sq_m);
+            for (int i = 0; i < 3; ++i) q[i] = zk::add(q[i], zk::mont_mul(coef_m, s[5 + i]));
         }
-        zk_record(p.coefficients());
-        if (claim != p(kZero) + p(kOne)) throw std::runtime_error(phase2 ? "tLookup_phase2: claim != p(0) + p(1)" : "tLookup_phase1: claim != p(0) + p(1)");
-        claim = p(vr);
-        const Fr_t e = Polynomial::eq(ub, vr);
-        alpha = alpha * e;
-        if (phase2) alpha_sq = alpha_sq * e;
-        else C = C * TWO_INV;
+        c[0] = zk::add(zk::mont_mul(e0, q[0]), s[3]);
+        c[1] = zk::add(zk::add(zk::mont_mul(e0, q[1]), zk::mont_mul(e1, q[0])), s[4]);
+        c[2] = zk::add(zk::mont_mul(e0, q[2]), zk::mont_mul(e1, q[1]));
+        c[3] = zk::mont_mul(e1, q[2]);
+        if (phase2) for (int i = 0; i < 3; ++i) c[i] = zk::sub(c[i], zk::mont_mul(inv_ratio_m, s[8 + i]));
+        else c[0] = zk::add(c[0], zk::mont_mul(half_m, C));
+        for (int i = 0; i < 4; ++i) coefs[i] = store(c[i]);
+        zk_record(coefs);
+        const Fr at_one = zk::add(zk::add(c[0], c[1]), zk::add(c[2], c[3]));
+        if (!zk::equal(claim, zk::add(c[0], at_one))) throw std::runtime_error(phase2 ? "tLookup_phase2: claim != p(0) + p(1)" : "tLookup_phase1: claim != p(0) + p(1)");
+        claim = c[3];
+        for (int i = 2; i >= 0; --i) claim = zk::add(zk::mont_mul(vr_m, claim), c[i]);
+        const Fr uv = zk::mont_mul(ub_m, vr);
+        const Fr e_m = zk::to_mont(zk::add(zk::sub(zk::dbl(uv), zk::add(ub, vr)), one));        // eq(ub, vr)
+        alpha_m = zk::mont_mul(alpha_m, e_m);
+        if (phase2) alpha_sq_m = zk::mont_mul(alpha_sq_m, e_m);
+        else C = zk::mont_mul(half_m, C);
     }
-    zk_record(claim);
-    return claim;
+    zk_record(store(claim));
+    return store(claim);
 }
 
 Fr_t tLookup_sumcheck(const FrTensor& S0, const FrTensor& T0, const FrTensor& m0, const Fr_t& alpha0, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v) {

@@ -4,7 +4,6 @@
 
 #define ZKC(call) zk_check((call), #call)
 
-static const Fr_t TEMP_ZERO{{0, 0, 0, 0, 0, 0, 0, 0}};
 static const Fr_t TEMP_ONE{{1, 0, 0, 0, 0, 0, 0, 0}};
 
 zkFC::zkFC(uint input_size, uint output_size, const FrTensor& weight)
@@ -151,7 +150,7 @@ vector<Claim> zkFC::prove_end(Pending& p) const {
         Polynomial poly({r[at], r[at + 1], r[at + 2]});
         at += 3;
         zk_record(poly.coefficients());
-        if (claim != poly(TEMP_ZERO) + poly(TEMP_ONE)) throw std::runtime_error("claim != p(0) + p(1)");
+        if (claim != r[at - 3] + r[at - 3] + r[at - 2] + r[at - 1]) throw std::runtime_error("claim != p(0) + p(1)");
         claim = poly(u_input[--k]);
     }
     const Fr_t final_claim = claim, claim_X = r[at], claim_W = r[at + 1];
@@ -180,7 +179,8 @@ Fr_t zkip(const Fr_t& claim0, const FrTensor& a0, const FrTensor& b0, const vect
     auto check_round = [&](Polynomial& p, const Fr_t& chal) {
         proof.push_back(p);
         zk_record(p.coefficients());
-        if (claim != p(TEMP_ZERO) + p(TEMP_ONE)) throw std::runtime_error("claim != p(0) + p(1)");
+        const vector<Fr_t> c = p.coefficients();
+        if (claim != c[0] + c[0] + c[1] + c[2]) throw std::runtime_error("claim != p(0) + p(1)");
         claim = p(chal);
     };
     while (k > 0) {
@@ -239,8 +239,8 @@ Fr_t zkip_stacked(const Fr_t& claim0, const FrTensor& A0, const FrTensor& B0, co
         Polynomial p({c[0], c[1], c[2]});
         proof.push_back(p);
         zk_record(p.coefficients());
-        Polynomial q = Polynomial::eq(uN[kN - 1 - r]) * p;
-        if (claim != q(TEMP_ZERO) + q(TEMP_ONE)) throw std::runtime_error("claim != q(0) + q(1)");
+        const Fr_t& ur = uN[kN - 1 - r];          // eq(u) is 1 - u at 0 and u at 1
+        if (claim != (TEMP_ONE - ur) * c[0] + ur * (c[0] + c[1] + c[2])) throw std::runtime_error("claim != q(0) + q(1)");
         claim = p(vN[kN - 1 - r]);
         keep.emplace_back(n_out * D);
         keep.emplace_back(n_out * D);
