@@ -288,17 +288,18 @@ __global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__
 // The endomorphism and the expansion of T hold for points of the order-r subgroup, which is where the
 // generators live (Commitment::random draws multiples of the group generator, commitment.cu:9-20).
 // All rounds are queued without a host round trip; the proof points come back in one copy, normalised to z = 1.
-static constexpr int MW = 32;        // 8-bit signed windows over a 255-bit scalar
-static constexpr int MT = 128;       // lanes of a bucket workgroup = buckets (digit magnitudes 1..128)
-static constexpr int MSEG = 4096;    // elements per chunk (12-bit list entries)
+static constexpr int MW = 32;        // 8-bit signed windows of a scalar split as k1 + k2 lambda: 16 of each half
+static constexpr int MWH = MW / 2;
+static constexpr int MT = 128;       // buckets of a window (digit magnitudes 1..128)
+static constexpr int MSEG = 4096;    // most elements of a chunk (12-bit list entries)
 static constexpr int MSL = 64;       // lanes of a bucket-accumulation workgroup (one wave): each takes two buckets of its chunk
 static constexpr int MHEAVY = 256;   // a bucket above this many elements of a chunk is summed by the whole workgroup
-struct MsmDesc { const int8_t* digits; const A29* base; uint32_t dstride, count, s_mul, s_off, b_mul, b_off, slot; };   // element i: recoded scalar i*s_mul+s_off of dstride, point base[i*b_mul+b_off]
+struct MsmDesc { const int8_t* digits; const A29* base; uint32_t dstride, count, s_mul, s_off, b_mul, b_off; };   // element i: recoded scalar i*s_mul+s_off of dstride, point base[i*b_mul+b_off]
 static constexpr int OB_MAX = 8;           // openings of equal size that share their rounds' launches
-static constexpr int OB_SUMS = 3 * OB_MAX;
-template <int NMAX> struct MsmDescs { MsmDesc d[NMAX]; };
-static constexpr int TAIL_N = 1024;        // generators at which the remaining rounds are computed in one batch (work grows with it, latency shrinks)
+static constexpr int TABLE_MIN_N = 1024;   // results of a fold below which no fold tables are made for it
+static constexpr int LAST_N = 16384;       // generators of a job (all its openings together) at which the remaining rounds are computed in one batch
 static constexpr int TAIL_LEVELS = 20;     // most rounds the batch takes
+static constexpr int SPAN_MAX_N = 1 << 17; // generators of a job up to which three rounds are taken as a batch of sums beside one fold
 struct GlvK { uint32_t k1[4], k2[4]; };
 
 __device__ __forceinline__ bool aff_is_inf(const G1Affine& p) { return is_zero(p.x) && is_zero(p.y); }   // normalised infinity: all-zero limbs
@@ -354,12 +355,78 @@ static __device__ __attribute__((noinline)) G1Jac g1_mul_glv(const G1Jac& P, con
     return out;
 }
 
-// Signed 8-bit digits of the balanced representative of every scalar, written window-major: D[w*n + i] in [-128, 127]
-// for w < MW, and D[MW*n + i] = 1 when the scalar was replaced by r - s (its point is then subtracted).  Taking the
-// smaller of s and r - s gives small negative values (r - x, as weights are embedded) as few non-zero windows as
-// small positive ones, instead of r's high bytes in every one of them.  A window byte above 127 becomes byte - 256
-// and carries one into the next window; the top window of a value below 2^254 cannot overflow.
+// Signed 8-bit digits of every scalar, written window-major: the scalar is split as +-k1 +-k2 lambda with |k1|, |k2| < 2^127
+// ([lambda](x, y) = (beta x, y), see glv_beta), D[w*n + i] in [-128, 127] is digit w of |k1| for w < MWH and digit w - MWH of |k2|
+// above, and D[MW*n + i] says which halves are subtracted (bit 0: k1, bit 1: k2).  The halves share the points they are summed over;
+// what the split buys is the end of a sum, whose Horner walk over the windows is 120 doublings instead of 248.
+// The smaller of s and r - s is split (weights are embedded as small values of either sign: a value below lambda / 2 is its own k1,
+// and its high windows are empty).  A window byte above 127 becomes byte - 256 and carries one into the next window; the top byte
+// of a half is at most 0x57, so the carry ends there.
 struct RecodeBatch { int8_t* D[OB_MAX]; const Fr* S[OB_MAX]; };      // blockIdx.y names the pair
+// a = round(x / lambda) and k1 = x - a lambda for x < 2^254: the quotient's estimate is the high half of x times 2^256 / lambda, at
+// most one short, and the remainder's comparison with lambda / 2 mends it.  k1 comes as magnitude and sign.
+__device__ __forceinline__ void glv_split_centred(const uint32_t* x, uint32_t (&k1)[4], bool& k1_neg, uint32_t (&a)[4]) {
+    constexpr uint32_t MU[5] = {0xf6cfee30u, 0x63f6e522u, 0xe01faaddu, 0x7c6becf1u, 1u};          // floor(2^256 / lambda)
+    constexpr uint32_t LAM[4] = {0xffffffffu, 0u, 0x0001a402u, 0xac45a401u};
+    uint32_t p[13];
+#pragma unroll
+    for (int i = 0; i < 13; ++i) p[i] = 0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        uint64_t c = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            c += (uint64_t)MU[i] * x[j] + p[i + j];
+            p[i + j] = (uint32_t)c;
+            c >>= 32;
+        }
+        p[i + 8] = (uint32_t)c;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = p[8 + i];
+    // rem = x - a lambda, in [0, 2 lambda): five limbs hold it
+    uint32_t q[5], rem[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) q[i] = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint64_t c = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (i + j > 4) break;
+            c += (uint64_t)a[i] * LAM[j] + q[i + j];
+            q[i + j] = (uint32_t)c;
+            c >>= 32;
+        }
+        if (i == 0) q[4] = (uint32_t)c;
+    }
+    uint32_t br = 0;
+#pragma unroll
+    for (int i = 0; i < 5; ++i) rem[i] = subb32(x[i], q[i], br);
+    // above lambda / 2 (0x5622d200.8000d201.00000000.7fffffff): one more lambda off; twice when the estimate was short
+    constexpr uint32_t HALF[5] = {0x7fffffffu, 0u, 0x8000d201u, 0x5622d200u, 0u};
+    bool negative = false;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        uint32_t lt = 0, b2 = 0, c = 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) (void)subb32(HALF[i], rem[i], lt);
+        const bool more = lt != 0 && !negative;                     // rem > lambda / 2
+#pragma unroll
+        for (int i = 0; i < 5; ++i) rem[i] = subb32(rem[i], more && i < 4 ? LAM[i] : 0u, b2);
+        a[0] = addc32(a[0], more ? 1u : 0u, c);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) a[i] = addc32(a[i], 0u, c);
+        negative = (rem[4] >> 31) != 0;
+    }
+    k1_neg = negative;
+    uint32_t b3 = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t n = subb32(0u, rem[i], b3);
+        k1[i] = negative ? n : rem[i];
+    }
+}
 // the digits of scalar i of n (standard form)
 __device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t n, size_t i, const Fr& sv) {
     Fr ng;
@@ -370,18 +437,26 @@ __device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t 
 #pragma unroll
     for (int l = 0; l < 8; ++l) (void)subb32(ng.v[l], sv.v[l], lt);
     const bool flip = lt != 0;
-    uint32_t carry = 0;
+    uint32_t x[8], k1[4], k2[4];
+    bool neg1;
 #pragma unroll
-    for (int l = 0; l < 8; ++l) {
-        const uint32_t word = flip ? ng.v[l] : sv.v[l];
+    for (int l = 0; l < 8; ++l) x[l] = flip ? ng.v[l] : sv.v[l];
+    glv_split_centred(x, k1, neg1, k2);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            uint32_t raw = ((word >> (8 * q)) & 0xFFu) + carry;
-            carry = raw > 127u ? 1u : 0u;
-            D[(size_t)(4 * l + q) * n + i] = (int8_t)(raw > 127u ? (int)raw - 256 : (int)raw);
+    for (int h = 0; h < 2; ++h) {
+        uint32_t carry = 0;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            const uint32_t word = h ? k2[l] : k1[l];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t raw = ((word >> (8 * q)) & 0xFFu) + carry;
+                carry = raw > 127u ? 1u : 0u;
+                D[(size_t)(h * MWH + 4 * l + q) * n + i] = (int8_t)(raw > 127u ? (int)raw - 256 : (int)raw);
+            }
         }
     }
-    D[(size_t)MW * n + i] = flip ? 1 : 0;
+    D[(size_t)MW * n + i] = (int8_t)((flip != neg1 ? 1 : 0) | (flip ? 2 : 0));
 }
 __global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t n) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -389,39 +464,34 @@ __global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t
     msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i]);
 }
 
-// sum over the NT lanes of a workgroup through the LDS pool (36 x NT words); every lane returns the total
-template <int NT = MT> __device__ __forceinline__ G1Jac msm_block_sum(uint32_t* pool, const G1Jac& v, uint32_t t) {
-    __syncthreads();
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&v);
-#pragma unroll
-        for (int l = 0; l < 36; ++l) pool[l * NT + t] = src[l];
-    }
-    __syncthreads();
+// sum over the NT lanes of a workgroup through the LDS pool (43 x NT words); lane 0 returns the total
+static constexpr int J29_WORDS = 43;
+static_assert(sizeof(J29) == 4 * J29_WORDS, "a point is its coordinates and its flag");
+template <int NT> __device__ __forceinline__ J29 j29_block_sum(uint32_t* pool, const J29& v, uint32_t t) {
+    J29 x = v;
     for (uint32_t sd = NT / 2; sd > 0; sd >>= 1) {
-        if (t < sd) {
-            G1Jac x, y;
-            uint32_t* px = reinterpret_cast<uint32_t*>(&x);
-            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+        __syncthreads();
+        if (t >= sd && t < 2 * sd) {
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
 #pragma unroll
-            for (int l = 0; l < 36; ++l) { px[l] = pool[l * NT + t]; py[l] = pool[l * NT + t + sd]; }
-            x = g1_add(x, y);
-#pragma unroll
-            for (int l = 0; l < 36; ++l) pool[l * NT + t] = px[l];
+            for (int l = 0; l < J29_WORDS; ++l) pool[l * (NT / 2) + t - sd] = src[l];
         }
         __syncthreads();
-    }
-    G1Jac tot;
-    uint32_t* pr = reinterpret_cast<uint32_t*>(&tot);
+        if (t < sd) {
+            J29 y;
+            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
 #pragma unroll
-    for (int l = 0; l < 36; ++l) pr[l] = pool[l * NT];
+            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (NT / 2) + t];
+            x = j29_add(x, y);
+        }
+    }
     __syncthreads();
-    return tot;
+    return x;
 }
 
 // One segment's share of sum over elements of digit_w(s) * base: the segment's MT raw buckets,
 // partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold / k_msm_point reduce them).
-// One wave per workgroup.  Per chunk of MSEG elements:
+// One wave per workgroup.  Per chunk of `chunk` elements (at most MSEG):
 //  1. the bucket sizes are counted (one LDS atomic per element) and the elements are sorted by bucket into one list in
 //     LDS (counting sort: 12-bit position in the chunk + sign);
 //  2. the buckets are ranked by size and lane j takes the j-th largest and the j-th smallest: list lengths of uniform
@@ -430,25 +500,25 @@ template <int NT = MT> __device__ __forceinline__ G1Jac msm_block_sum(uint32_t* 
 //     (67 % with one bucket per lane);
 //  3. a bucket with more than MHEAVY elements (scalars that share a digit: equal values, a common high byte) is left out
 //     of the lists and summed by all lanes together, each over its own share of the chunk.
-template <int NMAX>
-__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(G1Jac* __restrict__ partial, const MsmDescs<NMAX> descs, const MsmDesc* __restrict__ ddescs, uint32_t nseg, uint32_t chunks_per_seg) {
+__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(J29* __restrict__ partial, const MsmDesc* __restrict__ descs, uint32_t nseg, uint32_t chunks_per_seg, uint32_t chunk) {
     __shared__ uint32_t cnt[MT], off[MT], cursor[MT];
     __shared__ uint8_t order[MT];
-    __shared__ uint32_t pool[36 * MSL];            // the sorted list (u16 x MSEG), then the 36 x MSL point tree of the heavy buckets
-    static_assert(36 * MSL * 4 >= MSEG * 2, "pool too small for the list");
+    __shared__ uint32_t pool[J29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the point tree of the heavy buckets
+    static_assert(J29_WORDS * MSL * 4 >= MSEG * 2, "pool too small for the list");
     static_assert(MSEG <= 4096, "12-bit list entries");
     uint16_t* list = reinterpret_cast<uint16_t*>(pool);
-    const MsmDesc d = ddescs ? ddescs[blockIdx.z] : descs.d[blockIdx.z];      // many sums: the descriptors lie in device memory
+    const MsmDesc d = descs[blockIdx.z];
     const A29* __restrict__ A = d.base;
     const uint32_t w = blockIdx.y, seg = blockIdx.x, t = threadIdx.x, zz = blockIdx.z;
     const int8_t* __restrict__ Dw = d.digits + (size_t)w * d.dstride;
     const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
-    G1Jac* __restrict__ out = partial + (((size_t)zz * MW + w) * nseg + seg) * MT;
+    const uint32_t half = w / (uint32_t)MWH;
+    J29* __restrict__ out = partial + (((size_t)zz * MW + w) * nseg + seg) * MT;
     bool first = true;                                  // nothing written to `out` yet (the same for every lane)
     for (uint32_t ch = 0; ch < chunks_per_seg; ++ch) {
-        const uint32_t e0 = (seg * chunks_per_seg + ch) * MSEG;
+        const uint32_t e0 = (seg * chunks_per_seg + ch) * chunk;
         if (e0 >= d.count) break;
-        const uint32_t e1 = (e0 + MSEG < d.count) ? e0 + MSEG : d.count;
+        const uint32_t e1 = (e0 + chunk < d.count) ? e0 + chunk : d.count;
         cnt[t] = 0; cnt[t + MSL] = 0;
         __syncthreads();
         for (uint32_t e = e0 + t; e < e1; e += MSL) {
@@ -481,7 +551,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             const uint32_t mag = (uint32_t)(dg < 0 ? -dg : dg);
             if (cnt[mag - 1] > (uint32_t)MHEAVY) continue;
             const uint32_t pos = atomicAdd(&cursor[mag - 1], 1u);
-            list[pos] = (uint16_t)((e - e0) | (((dg < 0) != (Df[si] != 0)) ? 0x8000u : 0u));
+            list[pos] = (uint16_t)((e - e0) | (((dg < 0) != (((Df[si] >> half) & 1) != 0)) ? 0x8000u : 0u));
         }
         __syncthreads();
         {
@@ -493,9 +563,8 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (uint32_t i = 0;; ++i) {
                 if (i == lenA) {
                     // the end of the first list: its bucket goes out (added to what earlier chunks of this segment left there)
-                    G1Jac v = j29_to_jac(acc29);
-                    if (!first) v = g1_add(out[bA], v);
-                    out[bA] = v;
+                    if (!first) acc29 = j29_add(out[bA], acc29);
+                    out[bA] = acc29;
                     acc29 = j29_infinity();
                     pos = off[bB];
                 }
@@ -506,9 +575,8 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 if (en & 0x8000u) pt.y = fq29_neg(pt.y);
                 acc29 = j29_add_mixed(acc29, pt);
             }
-            G1Jac v = j29_to_jac(acc29);
-            if (!first) v = g1_add(out[bB], v);
-            out[bB] = v;
+            if (!first) acc29 = j29_add(out[bB], acc29);
+            out[bB] = acc29;
         }
         __threadfence_block();
         __syncthreads();
@@ -521,217 +589,61 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 if ((uint32_t)(dg < 0 ? -dg : dg) != b + 1) continue;
                 A29 pt = A[(size_t)e * d.b_mul + d.b_off];
                 if (a29_is_inf(pt)) continue;
-                if ((dg < 0) != (Df[si] != 0)) pt.y = fq29_neg(pt.y);
+                if ((dg < 0) != (((Df[si] >> half) & 1) != 0)) pt.y = fq29_neg(pt.y);
                 h29 = j29_add_mixed(h29, pt);
             }
-            const G1Jac h = msm_block_sum<MSL>(pool, j29_to_jac(h29), t);
-            if (t == 0) out[b] = g1_add(out[b], h);            // its list was empty: the slot holds what earlier chunks left (or infinity)
+            const J29 h = j29_block_sum<MSL>(pool, h29, t);
+            if (t == 0) out[b] = j29_add(out[b], h);            // its list was empty: the slot holds what earlier chunks left (or infinity)
         }
         __threadfence_block();
         __syncthreads();
         first = false;
     }
     if (first) {                                       // a segment past the end of this sum: empty buckets
-        out[t] = g1_infinity();
-        out[t + MSL] = g1_infinity();
+        out[t] = j29_infinity();
+        out[t + MSL] = j29_infinity();
     }
 }
 // raw buckets of up to 8 consecutive segments summed: out[(row * gridDim.y + group) * MT + t], row = sum * MW + w
-__global__ void __launch_bounds__(MT) k_msm_bucket_fold(G1Jac* __restrict__ out, const G1Jac* __restrict__ buckets, uint32_t nseg) {
+__global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, const J29* __restrict__ buckets, uint32_t nseg) {
     const uint32_t t = threadIdx.x, row = blockIdx.x, grp = blockIdx.y;
     const uint32_t s0 = grp * 8, s1 = (s0 + 8 < nseg) ? s0 + 8 : nseg;
-    const G1Jac* b = buckets + (size_t)row * nseg * MT;
-    G1Jac acc = b[(size_t)s0 * MT + t];
-    for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = g1_add(acc, b[(size_t)sg * MT + t]);
+    const J29* b = buckets + (size_t)row * nseg * MT;
+    J29 acc = b[(size_t)s0 * MT + t];
+    for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = j29_add(acc, b[(size_t)sg * MT + t]);
     out[((size_t)row * gridDim.y + grp) * MT + t] = acc;
 }
-// The whole sum from the raw buckets of all its windows, one workgroup per sum: lane t first combines bucket t+1 over the
-// windows, sum_w 2^(8w) B[w][t+1] (one Horner walk of 248 doublings, the segments of a window added on the way), and only
-// then weights it by t+1 -- one weighting and one lane sum per sum instead of one per window, and no Horner pass of a
-// single lane over window sums afterwards.  Raw buckets: buckets[((z MW + w) nseg + seg) MT + t].  wsum != nullptr: the point
-// goes where k_open_horner expects the window sums of sum z, wsum[(z / n_per) item_stride + (z % n_per) MW + w] (the sums of one
-// opening lie together, the openings of a batch item_stride apart): the point as window 0, infinity above; else into
-// pts[descs[z].slot].
-// list != nullptr: sum z is list[z] -- its raw buckets, their segment count and where its window sums go (the sums of
-// several rounds of a job in one launch, behind the last round's bucket accumulation).
-struct PointDesc { const G1Jac* buckets; G1Jac* W; uint32_t nseg, pad; };
-__global__ void __launch_bounds__(MT) k_msm_point(G1Jac* __restrict__ wsum, G1Jac* __restrict__ pts, const MsmDesc* __restrict__ descs, const G1Jac* __restrict__ buckets,
-                                                  uint32_t nseg, uint32_t n_per, uint32_t item_stride, const PointDesc* __restrict__ list) {
-    __shared__ uint32_t pool[36 * MT];
-    const uint32_t t = threadIdx.x, z = blockIdx.x;
-    if (list) { buckets = list[z].buckets; nseg = list[z].nseg; }
-    const size_t zb = list ? 0 : z;
-    // The walk is one lane's chain of 248 doublings: it runs in 29-bit limbs (two thirds of the instructions of the 32-bit
-    // formulas, and the point stays in registers instead of travelling through private memory at every call).
+// The sums of a list from the raw buckets of all their windows, one workgroup per sum: lane t takes bucket (t mod MT) + 1 of one
+// half's windows, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings, the segments of a window added on the way), weights it by
+// its digit, the lanes of the second half apply the endomorphism, and the workgroup's lanes are summed -- one weighting and one
+// lane sum per sum instead of one per window, and no Horner pass of a single lane over window sums afterwards.
+// Raw buckets: buckets[(w nseg + seg) MT + b].  The walk is one lane's chain, so a launch takes what one lane takes whatever the
+// number of sums: all of a job's sums that nothing waits for go into one launch.
+struct PointDesc { const J29* buckets; G1Jac* out; uint32_t nseg, pad; };
+__global__ void __launch_bounds__(2 * MT) k_msm_point(const PointDesc* __restrict__ list) {
+    __shared__ uint32_t pool[J29_WORDS * MT];
+    const uint32_t t = threadIdx.x, half = t / (uint32_t)MT, b = t % (uint32_t)MT;
+    const PointDesc d = list[blockIdx.x];
     J29 r = j29_infinity();
-    for (int w = MW - 1; w >= 0; --w) {
-        if (w != MW - 1)
+    for (int w = MWH - 1; w >= 0; --w) {
+        if (__any(!r.inf))
             for (int k = 0; k < 8; ++k) r = j29_double(r);
-        const G1Jac* b = buckets + (zb * MW + (uint32_t)w) * nseg * MT;
-        for (uint32_t sg = 0; sg < nseg; ++sg) {
-            const G1Jac pt = b[(size_t)sg * MT + t];
-            if (!is_zero(pt.z)) r = j29_add(r, j29_from_jac(pt));
+        const J29* row = d.buckets + (size_t)(half * MWH + (uint32_t)w) * d.nseg * MT;
+        for (uint32_t sg = 0; sg < d.nseg; ++sg) {
+            const J29 pt = row[(size_t)sg * MT + b];
+            if (!pt.inf) r = j29_add(r, pt);
         }
     }
-    J29 q29 = j29_infinity();
+    J29 q = j29_infinity();
     for (int bit = 7; bit >= 0; --bit) {
-        q29 = j29_double(q29);
-        if (((t + 1) >> bit) & 1u) q29 = j29_add(q29, r);
+        q = j29_double(q);
+        if (((b + 1) >> bit) & 1u) q = j29_add(q, r);
     }
-    const G1Jac q = j29_to_jac(q29);
-    const G1Jac tot = msm_block_sum(pool, q, t);
-    if (wsum || list) {
-        G1Jac* __restrict__ W = list ? list[z].W : wsum + (size_t)(z / n_per) * item_stride + (size_t)(z % n_per) * MW;
-        if (t == 0) W[0] = tot;
-        else if (t < (uint32_t)MW) W[t] = g1_infinity();
-    } else if (t == 0) pts[descs[z].slot] = tot;
+    if (half) q.x = fq29_mul(q.x, fq29_from_fp(glv_beta()));
+    q = j29_block_sum<2 * MT>(pool, q, t);
+    if (t == 0) *d.out = j29_to_jac(q);
 }
 
-// ---- the single points of the halving rounds, once per opening ---------------------------------------------------------
-// None of this feeds a fold, so nothing of it sits between two rounds: the rounds only leave their window sums behind
-// (W[(3 * round + j) * MW + w], j = 0, 1, 2 for T, T0, T1), and after the last round
-//  k_open_horner assembles every sum from its windows, sum_w 2^(8w) W[w], one lane per sum, all sums side by side;
-//  k_open_chain  computes T of every round r >= 1 (the reference sums s_i g_i over the folded vectors, commitment.cu:103): unrolling
-//                T_r = u(1-u) T_(r-1) + (1-u)^2 T0_(r-1) + u^2 T1_(r-1)   (u = the challenge of round r-1)
-//                down to round 0 makes T_r a combination of T_0 and the T0, T1 of the rounds before r with coefficients
-//                that are products of the challenges -- all rounds at once, one lane per term.
-// blockIdx.y: the opening of a batch (its points npts apart, its window sums wstride apart)
-__global__ void __launch_bounds__(GT) k_open_horner(G1Jac* __restrict__ pts0, const G1Jac* __restrict__ Wall0, uint32_t halving_rounds, uint32_t npts, uint32_t wstride) {
-    if (threadIdx.x != 0) return;
-    G1Jac* __restrict__ pts = pts0 + (size_t)blockIdx.y * npts;
-    const G1Jac* __restrict__ Wall = Wall0 + (size_t)blockIdx.y * wstride;
-    const uint32_t x = blockIdx.x, round = x / 3, j = x % 3;
-    if (round >= halving_rounds || (round > 0 && j == 0)) return;
-    const G1Jac* W = Wall + (size_t)x * MW;
-    G1Jac r = W[MW - 1];
-    for (int w = MW - 2; w >= 0; --w) {
-        for (int k = 0; k < 8; ++k) r = g1_double(r);
-        r = g1_add(r, W[w]);
-    }
-    pts[x] = r;
-}
-// k = k1 + k2 * lambda, 0 <= k1 < lambda (r = lambda^2 + lambda + 1, so k2 <= lambda + 1): one long division, as glv_split on the host
-__device__ __forceinline__ GlvK glv_split_device(const Fr& k) {
-    const uint64_t lam_hi = 0xac45a4010001a402ull, lam_lo = 0x00000000ffffffffull;
-    uint64_t rh = 0, rl = 0, qh = 0, ql = 0;
-    for (int i = 255; i >= 0; --i) {
-        const bool top = (rh >> 63) != 0;
-        rh = (rh << 1) | (rl >> 63);
-        rl = (rl << 1) | ((k.v[i >> 5] >> (i & 31)) & 1u);
-        qh = (qh << 1) | (ql >> 63);
-        ql <<= 1;
-        if (top || rh > lam_hi || (rh == lam_hi && rl >= lam_lo)) {
-            const uint64_t nl = rl - lam_lo;
-            rh = rh - lam_hi - (rl < lam_lo ? 1u : 0u);
-            rl = nl;
-            ql |= 1u;
-        }
-    }
-    GlvK o;
-    o.k1[0] = (uint32_t)rl; o.k1[1] = (uint32_t)(rl >> 32); o.k1[2] = (uint32_t)rh; o.k1[3] = (uint32_t)(rh >> 32);
-    o.k2[0] = (uint32_t)ql; o.k2[1] = (uint32_t)(ql >> 32); o.k2[2] = (uint32_t)qh; o.k2[3] = (uint32_t)(qh >> 32);
-    return o;
-}
-// [k1]P + [k2]phi(P) with a k of the lane's own: one doubling and at most one addition per bit, whatever the other lanes hold
-static __device__ __attribute__((noinline)) G1Jac g1_mul_glv_lane(const G1Jac& P, const GlvK& k) {
-    G1Jac Q = P;
-    Q.x = fp_mul(P.x, glv_beta());
-    const G1Jac PQ = g1_add(P, Q);
-    G1Jac out = g1_infinity();
-    for (int i = 127; i >= 0; --i) {
-        out = g1_double(out);
-        const uint32_t b = ((k.k1[i >> 5] >> (i & 31)) & 1u) | (((k.k2[i >> 5] >> (i & 31)) & 1u) << 1);
-        if (b) {
-            const G1Jac t = b == 1 ? P : (b == 2 ? Q : PQ);
-            out = g1_add(out, t);
-        }
-    }
-    return out;
-}
-// the same walk in 29-bit limbs.  P stays in registers; beta x (the abscissa of phi(P)) and P + phi(P) wait in LDS, word-
-// interleaved over the workgroup's NT lanes (tab: 57 x NT words), so the walk fits the register file without spilling.
-template <int NT> static __device__ J29 j29_mul_glv_lane(const J29& P, const GlvK& k, int32_t (*tab)[NT]) {
-    const uint32_t t = threadIdx.x;
-    {
-        J29 Q = P;
-        Q.x = fq29_mul(P.x, fq29_from_fp(glv_beta()));
-        const J29 PQ = j29_add(P, Q);
-#pragma unroll
-        for (int l = 0; l < 14; ++l) { tab[l][t] = Q.x.l[l]; tab[14 + l][t] = PQ.x.l[l]; tab[28 + l][t] = PQ.y.l[l]; tab[42 + l][t] = PQ.z.l[l]; }
-        tab[56][t] = (int32_t)PQ.inf;
-    }
-    J29 out = j29_infinity();
-    for (int i = 127; i >= 0; --i) {
-        out = j29_double(out);
-        const uint32_t b = ((k.k1[i >> 5] >> (i & 31)) & 1u) | (((k.k2[i >> 5] >> (i & 31)) & 1u) << 1);
-        if (b) {
-            J29 a = P;
-            if (b == 2) {
-#pragma unroll
-                for (int l = 0; l < 14; ++l) a.x.l[l] = tab[l][t];
-            } else if (b == 3) {
-#pragma unroll
-                for (int l = 0; l < 14; ++l) { a.x.l[l] = tab[14 + l][t]; a.y.l[l] = tab[28 + l][t]; a.z.l[l] = tab[42 + l][t]; }
-                a.inf = (uint32_t)tab[56][t];
-            }
-            out = j29_add(out, a);
-        }
-    }
-    return out;
-}
-// grid: halving_rounds - 1 workgroups; workgroup x computes T of round x + 1 into pts[3 * (x + 1)].  Needs T_0 and all T0, T1.
-// U: the openings' challenges in Montgomery form, opening y's at U + y * ustride
-__global__ void __launch_bounds__(GT) k_open_chain(G1Jac* __restrict__ pts0, const Fr* __restrict__ U, uint32_t halving_rounds, uint32_t npts, uint32_t ustride) {
-    __shared__ uint32_t pool[36 * GT];
-    __shared__ int32_t walk_tab[57][GT];
-    G1Jac* __restrict__ pts = pts0 + (size_t)blockIdx.y * npts;
-    const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
-    const uint32_t r = blockIdx.x + 1, t = threadIdx.x;
-    const Fr one = big_one_mont<8>();
-    G1Jac acc = g1_infinity();
-    if (r < halving_rounds) {
-        for (uint32_t i = t; i < 2 * r + 1; i += GT) {
-            // term i: i == 0 -> T_0 with prod_{j<r} a_j;  i = 1 + 2k + s -> (s ? T1_k : T0_k) with (s ? u_k^2 : (1-u_k)^2) prod_{k<j<r} a_j,  a_j = u_j (1 - u_j)
-            const uint32_t k = i == 0 ? 0u : (i - 1) / 2, s1 = i == 0 ? 0u : (i - 1) & 1u;
-            Fr c = one;
-            for (uint32_t j = (i == 0 ? 0u : k + 1); j < r; ++j) c = mont_mul(c, mont_mul(usu[j], sub(one, usu[j])));
-            if (i != 0) {
-                const Fr f = s1 ? usu[k] : sub(one, usu[k]);
-                c = mont_mul(c, mont_mul(f, f));
-            }
-            const G1Jac P = pts[i == 0 ? 0u : 3 * k + 1 + s1];
-            if (!is_zero(P.z)) acc = g1_add(acc, j29_to_jac(j29_mul_glv_lane<GT>(j29_from_jac(P), glv_split_device(from_mont(c)), walk_tab)));
-        }
-    }
-    // sum over the lanes
-    __syncthreads();
-    {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(&acc);
-#pragma unroll
-        for (int l = 0; l < 36; ++l) pool[l * GT + t] = src[l];
-    }
-    __syncthreads();
-    for (uint32_t sd = GT / 2; sd > 0; sd >>= 1) {
-        if (t < sd) {
-            G1Jac x, y;
-            uint32_t* px = reinterpret_cast<uint32_t*>(&x);
-            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
-#pragma unroll
-            for (int l = 0; l < 36; ++l) { px[l] = pool[l * GT + t]; py[l] = pool[l * GT + t + sd]; }
-            x = g1_add(x, y);
-#pragma unroll
-            for (int l = 0; l < 36; ++l) pool[l * GT + t] = px[l];
-        }
-        __syncthreads();
-    }
-    if (t == 0 && r < halving_rounds) {
-        G1Jac tot;
-        uint32_t* pr = reinterpret_cast<uint32_t*>(&tot);
-#pragma unroll
-        for (int l = 0; l < 36; ++l) pr[l] = pool[l * GT];
-        pts[3 * r] = tot;
-    }
-}
 // Sums of an opening's first rounds from commitments of the opened tensor's rows.  The opened vector is the row fold of a
 // tensor W, s = sum_r e_r W[r] with e_r = prod_j (bit_j(r) ? v_j : 1 - v_j) over the row challenges v, so every sum of the
 // form  sum_j s_(L j + x) g_(L j + y)  equals  sum_r e_r X[r]  with  X[r] = sum_j W[r][L j + x] g_(L j + y),  a point that
@@ -742,97 +654,114 @@ __global__ void __launch_bounds__(GT) k_open_chain(G1Jac* __restrict__ pts0, con
 //   T0_q = sum_j s^(q)_(2j) g^(q)_(2j+1) = sum_{a,b} c(a,b) sum_j s_(2^(q+1) j + a) g_(2^(q+1) j + 2^q + b),   T1_q likewise with the halves exchanged,
 // and T of round 0 is the same combination of the row commitments themselves.  `pts`: [pattern][row] points, pattern 0 the row
 // commitments, then for q = 0 .. cross_rounds - 1 the 4^q patterns (a 2^q + b) of T0_q followed by those of T1_q.
-// Target t of an opening: 0 = T of round 0, 1 + 2q + side = T0_q / T1_q.  The results go where k_open_horner reads the window
-// sums of those points: the point in window 0, infinity above.  They equal the sums over all generators exactly when `pts`
-// are such commitments of the opened tensor -- what the caller states by passing them.
-__host__ __device__ __forceinline__ void cross_target(uint32_t t, uint32_t& q, uint32_t& first_pattern, uint32_t& npat, uint32_t& slot) {
-    if (t == 0) { q = 0; first_pattern = 0; npat = 1; slot = 0; return; }
-    q = (t - 1) >> 1;
-    const uint32_t side = (t - 1) & 1u, four_q = 1u << (2 * q);
-    npat = four_q;
-    first_pattern = 1 + 2 * (four_q - 1) / 3 + side * four_q;
-    slot = (3 * q + 1 + side) * (uint32_t)MW;
+// T of the later rounds r follows from these points as well: unrolling
+//   T_r = u(1-u) T_(r-1) + (1-u)^2 T0_(r-1) + u^2 T1_(r-1)   (u = the challenge of round r-1)
+// down to round 0 makes T_r the sum over all patterns of the rounds before r, with the products of those coefficients.
+// Target t of an opening with `full` rounds: 0 = T of round 0, 1 + 2q + side = T0_q / T1_q, 2 full + r = T_r (1 <= r < full).  The sums equal
+// the sums over all generators exactly when `pts` are such commitments of the opened tensor -- what the caller states by
+// passing them.
+__host__ __device__ __forceinline__ uint32_t cross_patterns(uint32_t rounds) { return 1u + 2u * (((1u << (2 * rounds)) - 1u) / 3u); }
+// first_pattern, npat: the points of target t; first_term: its coefficients' place (in patterns) among the terms; slot: its place in the proof
+__host__ __device__ __forceinline__ void cross_target(uint32_t t, uint32_t full, uint32_t& first_pattern, uint32_t& npat, uint32_t& first_term, uint32_t& slot) {
+    if (t == 0) { first_pattern = first_term = 0; npat = 1; slot = 0; return; }
+    if (t > 2 * full) {
+        const uint32_t r = t - 2 * full;
+        first_pattern = 0;
+        npat = cross_patterns(r);
+        first_term = cross_patterns(full);
+        for (uint32_t j = 1; j < r; ++j) first_term += cross_patterns(j);
+        slot = 3 * r;
+        return;
+    }
+    const uint32_t q = (t - 1) >> 1, side = (t - 1) & 1u;
+    npat = 1u << (2 * q);
+    first_pattern = first_term = cross_patterns(q) + side * npat;
+    slot = 3 * q + 1 + side;
 }
 // These sums are bucket multi-scalar multiplications.  Term g = pattern * nrows + row of an opening, in the order `pts`
 // lays the points out, has the coefficient eq(u_rows, row) * c(pattern) -- c = 1 for the row commitments, the product of the
-// earlier rounds' challenges for a cross pattern -- and a target is the sum over a contiguous range of terms: one bucket sum
-// per target over the normalised points, with the digits of all terms written once, as k_msm_recode writes them
-// (D: (MW + 1) x terms bytes).  A term costs 32 mixed additions (a scalar multiplication of its own would cost a 129-step walk).
+// earlier rounds' challenges for a cross pattern; the terms of T_1, T_2, ... follow, pattern by pattern again -- and a target is
+// the sum over a contiguous range of terms: one bucket sum per target over the normalised points, with the digits of all
+// terms written once, as k_msm_recode writes them (D: (MW + 1) x terms bytes).  A term costs 32 mixed additions (a scalar
+// multiplication of its own would cost a 129-step walk).
 struct CrossDigitItem { int8_t* D; const Fr* u_rows; const Fr* u; uint32_t nrows, k_rows; };
 struct CrossDigitBatch { CrossDigitItem it[OB_MAX]; };
 // grid (ceil(most terms / 256), openings)
-__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t npatterns) {
+__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t full, uint32_t nterm_patterns) {
     const CrossDigitItem& it = cb.it[blockIdx.y];
-    const size_t terms = (size_t)npatterns * it.nrows, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t terms = (size_t)nterm_patterns * it.nrows, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= terms) return;
-    const uint32_t p = (uint32_t)(i / it.nrows), row = (uint32_t)(i - (size_t)p * it.nrows);
+    uint32_t p = (uint32_t)(i / it.nrows), t_round = 0;
+    const uint32_t row = (uint32_t)(i - (size_t)p * it.nrows);
+    if (p >= cross_patterns(full)) {                    // a term of T_r, r = t_round
+        p -= cross_patterns(full);
+        for (t_round = 1; p >= cross_patterns(t_round); ++t_round) p -= cross_patterns(t_round);
+    }
     const Fr one = big_one_mont<8>();
     Fr coef = one;
     for (uint32_t j = 0; j < it.k_rows; ++j) coef = mont_mul(coef, ((row >> j) & 1u) ? it.u_rows[j] : sub(one, it.u_rows[j]));
+    uint32_t k0 = 0;                                    // the T_r expansion multiplies by u (1 - u) of the rounds from here on
     if (p != 0) {
-        uint32_t q = 0, first = 1;                      // the patterns of round q: T0's 4^q, then T1's
-        while (p >= first + (2u << (2 * q))) { first += 2u << (2 * q); ++q; }
-        const uint32_t pl = (p - first) & ((1u << (2 * q)) - 1u), a = pl >> q, b = pl & ((1u << q) - 1u);
+        uint32_t q = 0;                                 // the patterns of round q: T0's 4^q, then T1's
+        while (p >= cross_patterns(q + 1)) ++q;
+        const uint32_t in_q = p - cross_patterns(q), pl = in_q & ((1u << (2 * q)) - 1u), a = pl >> q, b = pl & ((1u << q) - 1u);
         for (uint32_t k = 0; k < q; ++k) {
             const Fr uk = it.u[k], nk = sub(one, uk);
             coef = mont_mul(coef, mont_mul(((a >> k) & 1u) ? uk : nk, ((b >> k) & 1u) ? nk : uk));
         }
+        if (t_round) {
+            const Fr f = (in_q >> (2 * q)) ? it.u[q] : sub(one, it.u[q]);
+            coef = mont_mul(coef, mont_mul(f, f));
+            k0 = q + 1;
+        }
     }
+    for (uint32_t k = k0; k < t_round; ++k) coef = mont_mul(coef, mont_mul(it.u[k], sub(one, it.u[k])));
     msm_recode_store(it.D, terms, i, from_mont(coef));
+}
+// Row commitments without cross patterns give T of round 0 alone; T of the rounds behind it follows from it and from T0, T1 of the rounds
+// before by the same unrolling.  Those points lie in the proof itself: the digits of T_1 .. T_(R-1) as bucket sums over an opening's
+// first 3 R proof points (T, T0, T1 a round; the T of later rounds take no part: zeros).  U: the challenges, opening y's at U + y * ustride
+__global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__ D0, const Fr* __restrict__ U, uint32_t ustride, uint32_t R) {
+    const uint32_t terms = (R - 1) * 3 * R, i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= terms) return;
+    const Fr* __restrict__ u = U + (size_t)blockIdx.y * ustride;
+    const uint32_t r = 1 + i / (3 * R), m = i % (3 * R), k = m / 3, j = m % 3;
+    const Fr one = big_one_mont<8>();
+    Fr c = big_zero<8>();
+    if (m == 0 || (j != 0 && k < r)) {
+        c = one;
+        if (m != 0) {
+            const Fr f = j == 2 ? u[k] : sub(one, u[k]);
+            c = mont_mul(f, f);
+        }
+        for (uint32_t q = m == 0 ? 0u : k + 1; q < r; ++q) c = mont_mul(c, mont_mul(u[q], sub(one, u[q])));
+    }
+    msm_recode_store(D0 + (size_t)blockIdx.y * (MW + 1) * terms, terms, i, from_mont(c));
 }
 // ---- the fold on 29-bit-limb affine points ----------------------------------------------------------------------------------
 // The rounds of an opening keep the generators in ONE form: affine, 29-bit limbs (A29; all-zero limbs = infinity), canonical
 // limbs.  The bucket sums add out of it, the fold reads it and writes the next round's generators in it -- no
 // normalisation or conversion pass between two rounds.
-// 1 / v for every lane of a 64-lane workgroup with one field inversion (product tree in LDS; the root goes through the
-// 32-bit form, where the binary inverse lives).  v must not be 0 mod p (lanes with nothing to invert pass one).
-// lds: 14 x 128 words.
-__device__ __forceinline__ Fq29 block_inv64_29(const Fq29& v, int32_t (*lds)[2 * GT]) {
-    const uint32_t t = threadIdx.x;
-    auto put = [&](const Fq29& x, uint32_t i) {
-#pragma unroll
-        for (int l = 0; l < 14; ++l) lds[l][i] = x.l[l];
-    };
-    auto get = [&](uint32_t i) {
-        Fq29 x;
-#pragma unroll
-        for (int l = 0; l < 14; ++l) x.l[l] = lds[l][i];
-        return x;
-    };
-    __syncthreads();
-    put(v, t);
-    __syncthreads();
-    uint32_t off = 0;
-    for (uint32_t cnt = GT / 2; cnt >= 1; cnt >>= 1) {
-        const uint32_t noff = off + 2 * cnt;
-        if (t < cnt) put(fq29_mul(get(off + 2 * t), get(off + 2 * t + 1)), noff + t);
-        __syncthreads();
-        off = noff;
+// 1 / v, every lane its own: all lanes of a wave execute the inversion's instructions in any case, so a product tree over the
+// lanes around one inversion only adds to them.  v must not be 0 mod p (lanes with nothing to invert pass one).
+__device__ __forceinline__ Fq29 fq29_inverse(const Fq29& v) { return fq29_from_fp(mont_inverse(fq29_to_fp(v))); }
+// w as an affine point with canonical limbs (infinity: all zero)
+__device__ __forceinline__ A29 a29_from_j29(const J29& w) {
+    A29 o;
+    o.x = o.y = fq29_zero();
+    const Fq29 zi = fq29_inverse(w.inf ? fq29_one() : w.z);
+    if (!w.inf) {
+        const Fq29 zi2 = fq29_sqr(zi);
+        o.x = fq29_canon(fq29_mul(w.x, zi2));
+        o.y = fq29_canon(fq29_mul(fq29_mul(w.y, zi2), zi));
     }
-    {
-        const Fq29 root_inv = fq29_from_fp(mont_inverse(fq29_to_fp(get(off))));      // every lane the same value: no divergence
-        __syncthreads();
-        if (t == 0) put(root_inv, off);
-        __syncthreads();
-    }
-    for (uint32_t cnt = 1; cnt < (uint32_t)GT; cnt <<= 1) {
-        const uint32_t coff = off - 2 * cnt;
-        Fq29 c = fq29_one();
-        if (t < 2 * cnt) c = fq29_mul(get(off + (t >> 1)), get(coff + (t ^ 1u)));
-        __syncthreads();
-        if (t < 2 * cnt) put(c, coff + t);
-        __syncthreads();
-        off = coff;
-    }
-    const Fq29 r = get(t);
-    __syncthreads();
-    return r;
+    return o;
 }
 struct FoldItem { Fr* ns; A29* ng; const Fr* s; const A29* g; uint32_t* special; Fr u_mont; JsfK jsf; };
 struct FoldBatch { FoldItem it[OB_MAX]; };          // blockIdx.y names the opening; all of one size
 // Pair g of the round: s' and g' = a1 + [u](a0 - a1), all in 29-bit limbs.  The scalar multiplication walks the joint
 // sparse form of the split challenge over the all-affine table {D, phi(D), D + phi(D), D - phi(D)}, D = a0 - a1, and the
-// result is brought back to affine form in the kernel (a third inversion batched over the 64 lanes).  Pairs whose inputs
+// result is brought back to affine form in the kernel.  Pairs whose inputs
 // are special (a0 at infinity, equal abscissae, an abscissa of zero) are not computed here: their indices go to
 // `special` ([0] = count, then the indices) and k_open_fold_special takes them.
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
@@ -844,10 +773,7 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
     uint32_t* __restrict__ special = fb.it[blockIdx.y].special;
     const Fr u_mont = fb.it[blockIdx.y].u_mont;
     const JsfK& jsf = fb.it[blockIdx.y].jsf;
-    __shared__ int32_t fold_lds[4 * 14 * GT];
-    static_assert(4 * 14 * GT >= 14 * 2 * GT, "the inversion buffer shares the table's space");
-    int32_t (*inv_lds)[2 * GT] = reinterpret_cast<int32_t (*)[2 * GT]>(fold_lds);
-    int32_t (*tab)[14][GT] = reinterpret_cast<int32_t (*)[14][GT]>(fold_lds);
+    __shared__ int32_t tab[4][14][GT];
     const size_t g = (size_t)blockIdx.x * GT + threadIdx.x;
     const bool live = g < new_size;
     const size_t g0 = 2 * g, g1 = 2 * g + 1;
@@ -869,7 +795,7 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
         if (fq29_is_zero_mod_p(den)) { general = true; den = one29; }
     }
     const bool need_sub = live && !general && !inf1;          // D = a0 - a1 needs 1 / (x0 - x1)
-    Fq29 inv = block_inv64_29(den, inv_lds);
+    Fq29 inv = fq29_inverse(den);
     Fq29 xD = a0.x, yD = a0.y;
     if (need_sub) {
         const Fq29 lam = fq29_mul(fq29_add(a0.y, a1.y), inv);          // -a1 = (x1, -y1)
@@ -879,7 +805,7 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
     }
     if (live && !general && fq29_is_zero_mod_p(xD)) general = true;       // x = 0: not in the subgroup; the table below would divide by it
     const bool fast = live && !general;
-    inv = block_inv64_29(fast ? xD : one29, inv_lds);
+    inv = fq29_inverse(fast ? xD : one29);
     J29 w = j29_infinity();
     if (fast) {
         {
@@ -923,17 +849,8 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
         }
         if (!inf1) w = j29_add_mixed(w, a1);
     }
-    // back to affine: 1 / z batched over the lanes (the table in LDS is no longer needed)
-    const bool has_z = fast && !w.inf;
-    const Fq29 zi = block_inv64_29(has_z ? w.z : one29, inv_lds);
+    const A29 o = a29_from_j29(w);
     if (fast) {
-        A29 o;
-        o.x = o.y = fq29_zero();
-        if (has_z) {
-            const Fq29 zi2 = fq29_sqr(zi);
-            o.x = fq29_canon(fq29_mul(w.x, zi2));
-            o.y = fq29_canon(fq29_mul(fq29_mul(w.y, zi2), zi));
-        }
         new_gens[g] = o;
     } else if (general) {
         const uint32_t slot = atomicAdd(&special[0], 1u);
@@ -965,7 +882,6 @@ struct CombBatch { CombItem it[OB_MAX]; };
 template <int NT>
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_open_fold_comb(const CombBatch cb, size_t old_size, size_t new_size) {
-    __shared__ int32_t inv_lds[14][2 * GT];
     Fr* __restrict__ new_scalars = cb.it[blockIdx.y].ns;
     A29* __restrict__ new_gens = cb.it[blockIdx.y].ng;
     const Fr* __restrict__ scalars = cb.it[blockIdx.y].s;
@@ -1012,18 +928,8 @@ k_open_fold_comb(const CombBatch cb, size_t old_size, size_t new_size) {
         }
         if (!inf1) w = j29_add_mixed(w, a1);
     }
-    const bool has_z = fast && !w.inf;
-    const Fq29 zi = block_inv64_29(has_z ? w.z : fq29_one(), inv_lds);
-    if (fast) {
-        A29 o;
-        o.x = o.y = fq29_zero();
-        if (has_z) {
-            const Fq29 zi2 = fq29_sqr(zi);
-            o.x = fq29_canon(fq29_mul(w.x, zi2));
-            o.y = fq29_canon(fq29_mul(fq29_mul(w.y, zi2), zi));
-        }
-        new_gens[g] = o;
-    }
+    const A29 o = a29_from_j29(w);
+    if (fast) new_gens[g] = o;
 }
 // ---- three rounds in one: the generators after the third fold straight from the prepared ones -------------------------------------
 // When T0 and T1 of the first three rounds come from cross commitments of the opened tensor, nothing reads the generators of
@@ -1038,7 +944,6 @@ struct JumpItem { Fr* ns; A29* ng; const Fr* s; const A29* g; const A29* tab; Fr
 struct JumpBatch { JumpItem it[OB_MAX]; };
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_open_fold_jump(const JumpBatch jb, size_t new_size) {
-    __shared__ int32_t inv_lds[14][2 * GT];
     const JumpItem& it = jb.it[blockIdx.y];
     const size_t g = (size_t)blockIdx.x * GT + threadIdx.x;
     const bool live = g < new_size;
@@ -1080,17 +985,87 @@ k_open_fold_jump(const JumpBatch jb, size_t new_size) {
         }
         if (!inf1) w = j29_add_mixed(w, a1);
     }
-    const bool has_z = live && !w.inf;
-    const Fq29 zi = block_inv64_29(has_z ? w.z : fq29_one(), inv_lds);
-    if (live) {
-        A29 o;
-        o.x = o.y = fq29_zero();
-        if (has_z) {
-            const Fq29 zi2 = fq29_sqr(zi);
-            o.x = fq29_canon(fq29_mul(w.x, zi2));
-            o.y = fq29_canon(fq29_mul(fq29_mul(w.y, zi2), zi));
+    const A29 o = a29_from_j29(w);
+    if (live) it.ng[g] = o;
+}
+// ---- three rounds in one without tables ------------------------------------------------------------------------------------------
+// The same combination g^(3)_m = sum_{b<8} c_b g_(8m+b) with nothing prepared: wave b of a workgroup multiplies the b-th generator of
+// 64 results by c_b (one scalar for the wave: the walk of k_open_fold29 over the joint sparse form of the split c_b), and the eight
+// products are added up through LDS.  As much work as three rounds of halving one after the other (8 walks for 7 pairs'), but one
+// walk's latency instead of three: a walk of one wave a SIMD takes 2.4 ms whatever its number of lanes.  65536 generators ... YY.
+struct SpanBatch { A29* ng[OB_MAX]; const A29* g[OB_MAX]; };
+__global__ void __launch_bounds__(8 * GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_open_fold_span(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old_size, size_t new_size) {
+    __shared__ int32_t lds[8][4][14][GT];
+    const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT)), t = threadIdx.x % GT;
+    int32_t (*tab)[14][GT] = lds[b];
+    const JsfK& jsf = jsfs[blockIdx.y * 8 + b];
+    const size_t m = (size_t)blockIdx.x * GT + t;
+    A29 p;
+    p.x = p.y = fq29_zero();
+    if (m < new_size && 8 * m + b < old_size) p = sb.g[blockIdx.y][8 * m + b];
+    const bool inf = a29_is_inf(p), x0 = !inf && fq29_is_zero_mod_p(p.x);
+    J29 w = j29_infinity();
+    {
+        const Fq29 inv = fq29_inverse((inf || x0) ? fq29_one() : p.x), one29 = fq29_one();
+        const Fq29 xQ = fq29_mul(p.x, fq29_from_fp(glv_beta())), xPQ = fq29_mul(p.x, fq29_from_fp(glv_beta2()));
+        const Fq29 lam = fq29_mul(fq29_mul(fq29_from_fp(glv_minus2_over_beta_minus_1()), p.y), inv);   // slope of P + (beta x, -y)
+        const Fq29 xPmQ = fq29_mul(fq29_add(fq29_sqr(lam), xPQ), one29);
+        const Fq29 yPmQ = fq29_mul(fq29_sub(fq29_mul(lam, fq29_sub(p.x, xPmQ)), p.y), one29);
+#pragma unroll
+        for (int l = 0; l < 14; ++l) {
+            tab[0][l][t] = xQ.l[l];
+            tab[1][l][t] = xPQ.l[l];
+            tab[2][l][t] = xPmQ.l[l];
+            tab[3][l][t] = yPmQ.l[l];
         }
-        it.ng[g] = o;
+    }
+    for (int i = (int)jsf.len - 1; i >= 0; --i) {
+        w = j29_double(w);
+        const uint32_t dg = (jsf.dig[i >> 3] >> ((i & 7) * 4)) & 0xFu;    // (d1 + 1) | (d2 + 1) << 2, the same for every lane
+        const int d1 = (int)(dg & 3u) - 1, d2 = (int)(dg >> 2) - 1;
+        if (d1 == 0 && d2 == 0) continue;
+        A29 q;
+        bool negate;
+        int xi = -1;
+        if (d2 == 0) { q = p; negate = d1 < 0; }
+        else {
+            xi = d1 == 0 ? 0 : (d1 == d2 ? 1 : 2);
+#pragma unroll
+            for (int l = 0; l < 14; ++l) q.x.l[l] = tab[xi][l][t];
+            if (xi == 2) {
+#pragma unroll
+                for (int l = 0; l < 14; ++l) q.y.l[l] = tab[3][l][t];
+                negate = d1 < 0;
+            } else {
+                q.y = p.y;
+                negate = xi == 0 ? d2 < 0 : d1 > 0;                          // P + phi(P) = (beta^2 x, -y)
+            }
+        }
+        if (negate) q.y = fq29_neg(q.y);
+        // a point of abscissa zero is its own image under phi (outside the prime-order subgroup): P - phi(P) is infinity
+        if (!inf && !(x0 && xi == 2)) w = j29_add_mixed(w, q);
+    }
+    uint32_t* pool = reinterpret_cast<uint32_t*>(&lds[0][0][0][0]);
+    for (uint32_t sd = 4; sd > 0; sd >>= 1) {
+        __syncthreads();
+        if (b >= sd && b < 2 * sd) {
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(&w);
+#pragma unroll
+            for (int l = 0; l < J29_WORDS; ++l) pool[((b - sd) * J29_WORDS + l) * GT + t] = src[l];
+        }
+        __syncthreads();
+        if (b < sd) {
+            J29 y;
+            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[(b * J29_WORDS + l) * GT + t];
+            w = j29_add(w, y);
+        }
+    }
+    if (b == 0) {
+        const A29 o = a29_from_j29(w);
+        if (m < new_size) sb.ng[blockIdx.y][m] = o;
     }
 }
 // the pairs k_open_fold29 left out, by the general Jacobian route in 32-bit limbs (one lane per pair, an inversion each)
@@ -1131,15 +1106,13 @@ __global__ void __launch_bounds__(GT) k_open_fold_special(const SpecialBatch sb,
         new_gens[g] = o;
     }
 }
-// generator pairs' sums g_2i + g_2i+1 (an odd last element alone) for T of the first round; and the pairs' scalar sums
-// negate: the differences g_2i - g_2i+1 instead (what the first round's comb is built on)
-__global__ void __launch_bounds__(GT) k_open_pair_points(G1Jac* __restrict__ pj, const G1Affine* __restrict__ A, size_t old_size, size_t half_up, int negate) {
+// the generator pairs' differences g_2i - g_2i+1 (an odd last element alone): what the first round's comb is built on
+__global__ void __launch_bounds__(GT) k_open_pair_points(G1Jac* __restrict__ pj, const G1Affine* __restrict__ A, size_t old_size, size_t half_up) {
     const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i >= half_up) return;
     G1Jac p = aff_to_jac(A[2 * i]);
     if (2 * i + 1 < old_size) {
-        G1Affine b = A[2 * i + 1];
-        if (negate) b = g1_neg(b);
+        const G1Affine b = g1_neg(A[2 * i + 1]);
         if (!aff_is_inf(b)) p = g1_add_mixed(p, b);
     }
     pj[i] = p;
@@ -1165,14 +1138,6 @@ __global__ void __launch_bounds__(GT) k_open_span_diff(G1Jac* __restrict__ out, 
     if (!aff_is_inf(last)) p = g1_add_mixed(p, last);
     out[m] = p;
 }
-struct PairBatch { Fr* ps[OB_MAX]; const Fr* s[OB_MAX]; };
-__global__ void __launch_bounds__(256) k_open_pair_scalars(const PairBatch pb, size_t old_size, size_t half_up) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= half_up) return;
-    Fr* __restrict__ ps = pb.ps[blockIdx.y];
-    const Fr* __restrict__ scalars = pb.s[blockIdx.y];
-    ps[i] = (2 * i + 1 < old_size) ? add(scalars[2 * i], scalars[2 * i + 1]) : scalars[2 * i];
-}
 __global__ void __launch_bounds__(GT) k_a29_to_jac(G1Jac* __restrict__ out, const A29* __restrict__ in, size_t n) {
     const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i >= n) return;
@@ -1185,14 +1150,37 @@ __global__ void __launch_bounds__(256) k_a29_canon(A29* __restrict__ a, size_t n
     v.x = fq29_canon(v.x); v.y = fq29_canon(v.y);
     a[i] = v;
 }
-// ---- the last rounds in one batch ---------------------------------------------------------------------------------------
-// Once n0 <= TAIL_N generators are left, every later round's generators are fixed linear combinations of these n0
-// points: g at level j, block i, is sum over k in block i of W_j(k) g_k with W_j(k) = prod_{b<j} (bit_b(k) ? 1-u_b : u_b).
-// So T, T0, T1 of all remaining rounds and the final generator are multi-scalar multiplications over the same n0
-// affine points with coefficients that are plain field arithmetic; they run as one launch instead of a chain of
-// rounds that each wait for a scalar multiplication.
+// ---- rounds in one batch ------------------------------------------------------------------------------------------------
+// Over n0 generators, every later round's generators are fixed linear combinations of these n0 points: g at level j, block i, is
+// sum over k in block i of W_j(k) g_k with W_j(k) = prod_{b<j} (bit_b(k) ? 1-u_b : u_b).  So T, T0, T1 of any number of rounds and the
+// final generator are multi-scalar multiplications over the same n0 affine points with coefficients that are plain field
+// arithmetic; they run as one launch instead of a chain of rounds that each wait for a scalar multiplication.
 // Folded scalars of all levels: level 0 is S itself, level j >= 1 sits at SL + sum_{1<=i<j} n_i, n_i = ceil(n0 / 2^i).
-struct TailPtrs { Fr* SL[OB_MAX]; const Fr* S[OB_MAX]; };      // per opening of a batch (blockIdx.x of k_tail_scalars, blockIdx.y of k_tail_coeffs)
+struct TailPtrs { Fr* SL[OB_MAX]; const Fr* S[OB_MAX]; };      // per opening of a batch (blockIdx.x of k_tail_scalars, blockIdx.y of k_tail_scalars3 and k_tail_coeffs)
+// three levels at once, a lane for every eight scalars
+__global__ void __launch_bounds__(256) k_tail_scalars3(const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0) {
+    const uint32_t g = blockIdx.x * 256 + threadIdx.x, n1 = (n0 + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2;
+    if (g >= n3) return;
+    const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
+    const Fr* __restrict__ S = tp.S[blockIdx.y];
+    Fr* __restrict__ L1 = tp.SL[blockIdx.y];
+    Fr* __restrict__ L2 = L1 + n1;
+    Fr* __restrict__ L3 = L2 + n2;
+    Fr v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = 8 * g + i < n0 ? S[8 * g + i] : big_zero<8>();      // a missing scalar counts as zero: s0 - u s0
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const Fr u = usu[k];
+        const uint32_t nk = k == 0 ? n1 : (k == 1 ? n2 : n3), per = 4u >> k;
+        Fr* __restrict__ L = k == 0 ? L1 : (k == 1 ? L2 : L3);
+#pragma unroll
+        for (int i = 0; i < (4 >> k); ++i) {
+            v[i] = add(v[2 * i], mont_mul(u, sub(v[2 * i + 1], v[2 * i])));
+            if (per * g + i < nk) L[per * g + i] = v[i];
+        }
+    }
+}
 // U: the tail's challenges (Montgomery form), opening y's at U + y * ustride
 // One workgroup per opening (the levels follow each other behind a barrier) of TAIL_SCALAR_T lanes: four waves find room on
 // a compute unit whose SIMDs each hold a point kernel's waves; the sixteen of a 1024-lane workgroup waited milliseconds for it.
@@ -1215,12 +1203,12 @@ __global__ void __launch_bounds__(TAIL_SCALAR_T) k_tail_scalars(const TailPtrs t
     }
 }
 // C[(3j+0)*n0 + k] = s_j[k>>j] W_j(k); C[(3j+1)*n0 + k] = s_j[(k>>j)-1] W_j(k) for odd k>>j; C[(3j+2)*n0 + k] = s_j[(k>>j)+1] W_j(k)
-// for even k>>j with a partner; zero elsewhere.  C[3*levels*n0 + k] = W_levels(k).
-__global__ void __launch_bounds__(256) k_tail_coeffs(Fr* __restrict__ C0, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels) {
+// for even k>>j with a partner; zero elsewhere.  C[3*levels*n0 + k] = W_levels(k) when `final_gen`.
+__global__ void __launch_bounds__(256) k_tail_coeffs(Fr* __restrict__ C0, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels, uint32_t final_gen) {
     const uint32_t k = blockIdx.x * 256 + threadIdx.x;
     if (k >= n0) return;
     const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
-    Fr* __restrict__ C = C0 + (size_t)blockIdx.y * (3 * levels + 1) * n0;
+    Fr* __restrict__ C = C0 + (size_t)blockIdx.y * (3 * levels + final_gen) * n0;
     const Fr* __restrict__ SL = tp.SL[blockIdx.y];
     const Fr* __restrict__ S = tp.S[blockIdx.y];
     const Fr one_m = big_one_mont<8>();
@@ -1241,7 +1229,7 @@ __global__ void __launch_bounds__(256) k_tail_coeffs(Fr* __restrict__ C0, const 
         nxt += ns;
         n = ns;
     }
-    C[(size_t)(3 * levels) * n0 + k] = from_mont(W);
+    if (final_gen) C[(size_t)(3 * levels) * n0 + k] = from_mont(W);
 }
 __global__ void __launch_bounds__(64) k_u32_zero(uint32_t* __restrict__ p, uint32_t n, size_t stride) {      // p[i * stride] = 0, i < n
     for (uint32_t i = threadIdx.x; i < n; i += 64) p[(size_t)i * stride] = 0u;
@@ -1305,6 +1293,25 @@ static const int g_fold_timer_hook = (at_shutdown([] {
     g_fold_timer.ev.clear();
     g_fold_timer.on = false;
 }), 0);
+struct FoldTimed {
+    hipEvent_t t0 = nullptr;
+    hipStream_t st;
+    explicit FoldTimed(hipStream_t st) : st(st) {
+        if (g_fold_timer.on && hipEventCreate(&t0) == hipSuccess) (void)hipEventRecord(t0, st);
+    }
+    void end(int method, double fp_mults, unsigned long long pairs) {
+        hipEvent_t t1 = nullptr;
+        if (!t0 || hipEventCreate(&t1) != hipSuccess) return;
+        (void)hipEventRecord(t1, st);
+        std::lock_guard<std::mutex> lk(g_fold_timer.mu);
+        g_fold_timer.ev.emplace_back(t0, t1);
+        g_fold_timer.fp_mults += fp_mults;
+        g_fold_timer.pairs += pairs;
+        g_fold_timer.method.push_back(method);
+        g_fold_timer.m_mults[method] += fp_mults;
+        g_fold_timer.m_pairs[method] += pairs;
+    }
+};
 // Fp multiplications of one pair of the fold by the formulas' count (two 8-limb products aside)
 static double fold_fp_mults_per_pair(const JsfK& j) {
     int adds = 0;
@@ -1350,38 +1357,22 @@ static JsfK jsf_of(const GlvK& k) {
     return out;
 }
 
-// The generators of an opening in the form its rounds work on: A29 points, and behind them the pair sums
-// g_2i + g_2i+1 that T of the first round is summed over (n + ceil(n/2) points in one array).  Nothing in it depends on
-// what is opened, so a caller that opens against the same generators again keeps it (zk_g1_open_prepare).
+// The generators of an opening in the form its rounds work on: A29 points.  Nothing in it depends on what is opened, so a
+// caller that opens against the same generators again keeps it (zk_g1_open_prepare).
 static int open_prep_build(A29* out, const G1Jac* gens, size_t n, Arena& arena, hipStream_t st) {
-    const size_t half_up = (n + 1) / 2;
     Scratch& aff = arena.add(sizeof(G1Affine) * n);
-    Scratch& pj = arena.add(sizeof(G1Jac) * half_up);
-    Scratch& paff = arena.add(sizeof(G1Affine) * half_up);
-    if (aff.rc || pj.rc || paff.rc) return aff.rc ? aff.rc : (pj.rc ? pj.rc : paff.rc);
+    if (aff.rc) return aff.rc;
     g1_normalize_queue<true>(aff.p, gens, n, st);
     hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(n, 256)), dim3(256), 0, st, out, aff.as<G1Affine>(), n);
-    hipLaunchKernelGGL(k_open_pair_points, dim3(cdiv(half_up, GT)), dim3(GT), 0, st, pj.as<G1Jac>(), aff.as<G1Affine>(), n, half_up, 0);
-    g1_normalize_queue<true>(paff.p, pj.as<G1Jac>(), half_up, st);
-    hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(half_up, 256)), dim3(256), 0, st, out + n, paff.as<G1Affine>(), half_up);
     ZK_LAUNCH_CHECK();
     return 0;
 }
 
-// Queues one round: the scalars' digits and the fold on st, the bucket sums on aux.  gens: the round's generators (A29);
-// with_T (the first round): the pair sums follow them at gens + old_size.  wsum_round: the round's 3 x MW window sums
-// (T, T0, T1); without with_T the first MW are left alone (T of that round then comes from k_open_chain).
-// Round 0 needs T = sum_j s_j g_j over all generators besides T0 and T1.  With the pairs' sums,
-//   sum_i (s_2i + s_2i+1)(g_2i + g_2i+1) = T + T0 + T1,
-// so T costs a bucket sum over half as many points: pair i gets the scalar s_2i + s_2i+1 (mod r: the generators have
-// order r) and the point g_2i + g_2i+1; an odd last element stands alone.  k_open_t_fix takes T0 and T1 off again,
-// window by window.
-__global__ void __launch_bounds__(64) k_open_t_fix(G1Jac* __restrict__ wsum0, uint32_t item_stride) {
-    const uint32_t w = threadIdx.x;
-    if (w >= (uint32_t)MW) return;
-    G1Jac* __restrict__ wsum = wsum0 + (size_t)blockIdx.x * item_stride;
-    wsum[w] = g1_add(g1_add(wsum[w], g1_neg(wsum[MW + w])), g1_neg(wsum[2 * MW + w]));
-}
+// One opening of the batch: its scalars, its challenges (rounds x 8 limbs) and its generators -- Jacobian, or null when
+// `prep` (their prepared form, open_prep_build) is given
+struct OpenItem { const void* scalars; const void* gens; const A29* prep; const uint32_t* u; const A29* comb = nullptr; const A29* comb2 = nullptr;
+                  const void* rows = nullptr; uint32_t nrows = 0; const uint32_t* u_rows = nullptr; int k_rows = 0; int cross_rounds = 0;
+                  const A29* comb3 = nullptr; };
 // One round of `count` openings of equal size (count <= OB_MAX): one launch of each kernel covers all of them.
 // comb: the first round's table; comb2 (second round): the tables of F and H one after the other, u_prev the first round's challenge
 struct RoundItem { Fr* new_scalars; A29* new_gens; const Fr* scalars; const A29* gens; Fr u; const A29* comb = nullptr; const A29* comb2 = nullptr; Fr u_prev = Fr(); };
@@ -1405,101 +1396,127 @@ static CombK comb_of(const GlvK& k) {
         }
     return ck;
 }
-// given: what of this round's sums comes from commitments of the tensor's rows (open_cross_sums_queue) and is not summed here:
-// 0 nothing, 1 T of the first round (no pair sums), 2 T0 and T1 as well (no bucket sums at all: the round is its fold)
-// later (optional): the reductions of this round's raw buckets are appended to it instead of launched (the caller runs them
-// all at once behind its last round); a round whose T comes from the pair sums (k_open_t_fix) reduces at once
-static int open_round_launch(const RoundItem* items, int count, size_t old_size, bool with_T, int given, G1Jac* wsum_round, uint32_t wsum_item_stride, Arena& arena,
-                             hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>* later = nullptr) {
+// c_b = prod_q (bit_q(b) ? 1 - u_q : u_q) over three rounds' challenges (standard form in and out)
+static void fold_span_coefficients(Fr* c, const uint32_t* u) {
+    const Fr one = big_one_mont<8>();
+    for (int b = 0; b < JUMP_SPAN; ++b) {
+        Fr m = one;
+        for (int q = 0; q < JUMP_ROUNDS; ++q) {
+            const Fr um = to_mont(load_fr(u + 8 * (size_t)q));
+            m = mont_mul(m, ((b >> q) & 1) ? sub(one, um) : um);
+        }
+        c[b] = from_mont(m);
+    }
+}
+// Small host arrays of a job (challenges, descriptors) on their way to the device: copied through pinned buffers of 64 KiB that are
+// held until the job ends, into device blocks of the job's arena.
+struct JobUploads {
+    Arena* arena = nullptr;
+    std::vector<void*> pins;
+    std::vector<char*> devs;
+    size_t used = 0;
+    static constexpr size_t CAP = 64 << 10;
+    int put(const void* src, size_t bytes, hipStream_t st, const void** dev) {
+        ZK_ARG(bytes <= CAP, "opening: too many sums");
+        if (pins.empty() || used + bytes > CAP) {
+            Scratch& d = arena->add(CAP);
+            if (d.rc) return d.rc;
+            void* h = nullptr;
+            const int rc = pinned_acquire(&h);
+            if (rc) return rc;
+            pins.push_back(h);
+            devs.push_back(d.as<char>());
+            used = 0;
+        }
+        memcpy((char*)pins.back() + used, src, bytes);
+        ZK_HIP(hipMemcpyAsync(devs.back() + used, (char*)pins.back() + used, bytes, hipMemcpyHostToDevice, st));
+        *dev = devs.back() + used;
+        used = (used + bytes + 255) / 256 * 256;
+        return 0;
+    }
+    ~JobUploads() { for (void* h : pins) pinned_release(h); }
+};
+// `aux` waits for what `st` holds so far
+static int join_streams(hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events) {
+    if (aux == st) return 0;
+    hipEvent_t ev;
+    ZK_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+    events.push_back(ev);
+    ZK_HIP(hipEventRecord(ev, st));
+    ZK_HIP(hipStreamWaitEvent(aux, ev, 0));
+    return 0;
+}
+// The bucket accumulation of some sums of at most count_max elements on st; their reductions, sum z into out[z], are appended to `later`.
+static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1Jac*>& out, size_t count_max, Arena& arena, JobUploads& up, hipStream_t st,
+                             std::vector<PointDesc>& later) {
+    const uint32_t n_msm = (uint32_t)d.size();
+    if (n_msm == 0) return 0;
+    // One chunk per workgroup, and chunks short enough for two workgroups a SIMD where there are few elements: a workgroup's time is its
+    // chunk's elements over 64 lanes.  Very large inputs take more chunks per workgroup to bound the bucket storage.
+    uint32_t chunk = MSEG;
+    while (chunk > 256 && (size_t)n_msm * MW * cdiv(count_max, chunk / 2) <= 2048) chunk /= 2;
+    const uint32_t chunks = count_max ? cdiv(count_max, chunk) : 1u;
+    const uint32_t cps = (chunks + 255u) / 256u;
+    uint32_t ns = (chunks + cps - 1) / cps;
+    const void* dd = nullptr;
+    int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
+    if (rc) return rc;
+    Scratch& partial = arena.add(sizeof(J29) * n_msm * MW * (size_t)ns * MT);
+    if (partial.rc) return partial.rc;
+    hipLaunchKernelGGL(k_msm_seg, dim3(ns, MW, n_msm), dim3(MSL), 0, st, partial.as<J29>(), (const MsmDesc*)dd, ns, cps, chunk);
+    // the segments' raw buckets summed eight at a time (a lane per bucket and window: the reduction, one workgroup per sum, then
+    // walks single buckets)
+    const J29* cur = partial.as<J29>();
+    while (ns > 1) {
+        const uint32_t ng = (ns + 7) / 8;
+        Scratch& nxt = arena.add(sizeof(J29) * n_msm * MW * (size_t)ng * MT);
+        if (nxt.rc) return nxt.rc;
+        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, st, nxt.as<J29>(), cur, ns);
+        cur = nxt.as<J29>();
+        ns = ng;
+    }
+    ZK_LAUNCH_CHECK();
+    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], 1u, 0u});
+    return 0;
+}
+static int points_queue(std::vector<PointDesc>& list, JobUploads& up, hipStream_t st) {
+    if (list.empty()) return 0;
+    const void* dl = nullptr;
+    int rc = up.put(list.data(), sizeof(PointDesc) * list.size(), st, &dl);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_msm_point, dim3((unsigned)list.size()), dim3(2 * MT), 0, st, (const PointDesc*)dl);
+    ZK_LAUNCH_CHECK();
+    list.clear();
+    return 0;
+}
+// One halving round: the scalars' digits and the fold on st, the bucket sums on aux (their reductions are appended to `later`).
+// pts: where the round's T, T0, T1 of opening 0 go; opening i's npts further.
+// given: what of this round's sums comes from commitments of the tensor's rows (open_cross_sums_queue, k_open_unroll_digits) and is not
+// summed here: 0 nothing, 1 T, 2 T0 and T1 as well (no bucket sums at all: the round is its fold)
+// comb_round: 0 the first round (fold table RoundItem::comb, when all items have one), 1 the second (comb2), 2 a later one
+static int open_round_launch(const RoundItem* items, int count, size_t old_size, int comb_round, int given, G1Jac* pts, size_t npts, Arena& arena, JobUploads& up,
+                             hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
     ZK_ARG(old_size < (1ull << 31), "opening: more than 2^31 generators");
     ZK_ARG(count >= 1 && count <= OB_MAX, "opening: bad batch size");
     const size_t new_size = (old_size + 1) / 2;
-    const bool chained = !with_T || given >= 1;
-    if (given < 2) {
     const size_t dig_bytes = (size_t)(MW + 1) * old_size;
-    Scratch& dig = arena.add(dig_bytes * count);
-    if (dig.rc) return dig.rc;
-    {
+    const int8_t* digits = nullptr;
+    if (given < 2) {
+        Scratch& dig = arena.add(dig_bytes * count);
+        if (dig.rc) return dig.rc;
+        digits = dig.as<int8_t>();
         RecodeBatch rb;
         for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>() + dig_bytes * (i < count ? i : 0); rb.S[i] = items[i < count ? i : 0].scalars; }
         hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(old_size, 256), count), dim3(256), 0, st, rb, old_size);
         ZK_LAUNCH_CHECK();
-    }
-    if (aux != st) {
-        hipEvent_t ready;
-        ZK_HIP(hipEventCreateWithFlags(&ready, hipEventDisableTiming));
-        events.push_back(ready);
-        ZK_HIP(hipEventRecord(ready, st));
-        ZK_HIP(hipStreamWaitEvent(aux, ready, 0));
-    }
-    // ---- side chain (aux): bucket sums, window sums; nothing here feeds the next fold ----
-    MsmDescs<OB_SUMS> descs;
-    const uint32_t half = (uint32_t)(old_size / 2);
-    const uint32_t half_up = (uint32_t)new_size;
-    const uint32_t n_per = chained ? 2u : 3u, n_msm = n_per * (uint32_t)count;
-    const uint32_t ds = (uint32_t)old_size;
-    const int8_t* dig2p = nullptr;
-    const size_t dig2_bytes = (size_t)(MW + 1) * half_up;
-    if (!chained) {
-        Scratch& ps = arena.add(sizeof(Fr) * half_up * count);
-        Scratch& dig2 = arena.add(dig2_bytes * count);
-        if (ps.rc || dig2.rc) return ps.rc ? ps.rc : dig2.rc;
-        PairBatch pb;
-        RecodeBatch rb;
-        for (int i = 0; i < OB_MAX; ++i) {
-            const int k = i < count ? i : 0;
-            pb.ps[i] = ps.as<Fr>() + (size_t)half_up * k; pb.s[i] = items[k].scalars;
-            rb.D[i] = dig2.as<int8_t>() + dig2_bytes * k; rb.S[i] = pb.ps[i];
-        }
-        hipLaunchKernelGGL(k_open_pair_scalars, dim3(cdiv(half_up, 256), count), dim3(256), 0, aux, pb, old_size, (size_t)half_up);
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(half_up, 256), count), dim3(256), 0, aux, rb, (size_t)half_up);
-        dig2p = dig2.as<int8_t>();
-    }
-    uint32_t q = 0;
-    for (int i = 0; i < count; ++i) {
-        const int8_t* dg = dig.as<int8_t>() + dig_bytes * i;
-        if (!chained) descs.d[q++] = MsmDesc{dig2p + dig2_bytes * i, items[i].gens, half_up, half_up, 1u, 0u, 1u, (uint32_t)old_size, 0u};
-        descs.d[q++] = MsmDesc{dg, items[i].gens, ds, half, 2u, 0u, 2u, 1u, 1u};
-        descs.d[q++] = MsmDesc{dg, items[i].gens, ds, half, 2u, 1u, 2u, 0u, 2u};
-    }
-    for (; q < (uint32_t)OB_SUMS; ++q) descs.d[q] = MsmDesc{dig.as<int8_t>(), items[0].gens, ds, 0u, 1u, 0u, 1u, 0u, 0u};
-    // One chunk per workgroup: many short workgroups keep every compute unit busy to the end of the launch (with few
-    // long ones, all equally long, whatever does not fit the first turn waits a whole turn); the raw buckets of the
-    // segments are summed afterwards.  Very large inputs take more chunks per workgroup to bound the bucket storage.
-    const size_t count_max = chained ? half : half_up;
-    const uint32_t chunks = count_max ? cdiv(count_max, MSEG) : 1u;
-    const uint32_t cps = (chunks + 255u) / 256u;
-    const uint32_t nseg = (chunks + cps - 1) / cps;
-    Scratch& partial = arena.add(sizeof(G1Jac) * n_msm * MW * (size_t)nseg * MT);
-    if (partial.rc) return partial.rc;
-    G1Jac* wsum = wsum_round + (size_t)(3 - n_per) * MW;
-    hipLaunchKernelGGL(k_msm_seg<OB_SUMS>, dim3(nseg, MW, n_msm), dim3(MSL), 0, aux, partial.as<G1Jac>(), descs, (const MsmDesc*)nullptr, nseg, cps);
-    {
-        // sum the segments' raw buckets eight at a time (a lane per bucket and window: the reduction, one workgroup per sum,
-        // then walks single buckets), then weight and total
-        const G1Jac* cur = partial.as<G1Jac>();
-        uint32_t ns = nseg;
-        while (ns > 1) {
-            const uint32_t ng = (ns + 7) / 8;
-            Scratch& nxt = arena.add(sizeof(G1Jac) * n_msm * MW * (size_t)ng * MT);
-            if (nxt.rc) return nxt.rc;
-            hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, aux, nxt.as<G1Jac>(), cur, ns);
-            cur = nxt.as<G1Jac>();
-            ns = ng;
-        }
-        if (later && chained) {
-            for (uint32_t z = 0; z < n_msm; ++z)
-                later->push_back(PointDesc{cur + (size_t)z * MW * ns * MT, wsum + (size_t)(z / n_per) * wsum_item_stride + (size_t)(z % n_per) * MW, ns, 0u});
-        } else hipLaunchKernelGGL(k_msm_point, dim3(n_msm), dim3(MT), 0, aux, wsum, (G1Jac*)nullptr, (const MsmDesc*)nullptr, cur, ns, n_per, wsum_item_stride, (const PointDesc*)nullptr);
-    }
-    if (!chained) hipLaunchKernelGGL(k_open_t_fix, dim3(count), dim3(64), 0, aux, wsum, wsum_item_stride);
-    ZK_LAUNCH_CHECK();
+        int rc = join_streams(st, aux, events);
+        if (rc) return rc;
     }
     // ---- critical chain (st): the fold ----
     const size_t sp_stride = 1 + new_size;
     Scratch& special = arena.add(sizeof(uint32_t) * sp_stride * count);
     if (special.rc) return special.rc;
-    bool use_comb = with_T, use_comb2 = !with_T;
+    bool use_comb = comb_round == 0, use_comb2 = comb_round == 1;
     for (int i = 0; i < count; ++i) { use_comb = use_comb && items[i].comb != nullptr; use_comb2 = use_comb2 && items[i].comb2 != nullptr; }
     FoldBatch fb;
     CombBatch cbt;
@@ -1534,81 +1551,38 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
         sb.ng[i] = items[k].new_gens; sb.g[i] = items[k].gens; sb.special[i] = sp; sb.ku[i] = ku;
     }
     hipLaunchKernelGGL(k_u32_zero, dim3(1), dim3(64), 0, st, special.as<uint32_t>(), (uint32_t)count, sp_stride);
-    hipEvent_t t0 = nullptr, t1 = nullptr;
-    if (g_fold_timer.on) {
-        ZK_HIP(hipEventCreate(&t0));
-        ZK_HIP(hipEventCreate(&t1));
-        ZK_HIP(hipEventRecord(t0, st));
-    }
+    FoldTimed timed(st);
     if (use_comb) hipLaunchKernelGGL(k_open_fold_comb<1>, dim3(cdiv(new_size, GT), count), dim3(GT), 0, st, cbt, old_size, new_size);
     else if (use_comb2) hipLaunchKernelGGL(k_open_fold_comb<2>, dim3(cdiv(new_size, GT), count), dim3(GT), 0, st, cbt, old_size, new_size);
     else hipLaunchKernelGGL(k_open_fold29, dim3(cdiv(new_size, GT), count), dim3(GT), 0, st, fb, old_size, new_size);
-    if (g_fold_timer.on) {
-        ZK_HIP(hipEventRecord(t1, st));
-        std::lock_guard<std::mutex> lk(g_fold_timer.mu);
-        g_fold_timer.ev.emplace_back(t0, t1);
-        g_fold_timer.fp_mults += fp_mults;
-        g_fold_timer.pairs += new_size * (size_t)count;
-        const int mth = (use_comb || use_comb2) ? 1 : 0;
-        g_fold_timer.method.push_back(mth);
-        g_fold_timer.m_mults[mth] += fp_mults;
-        g_fold_timer.m_pairs[mth] += new_size * (size_t)count;
-    }
+    timed.end((use_comb || use_comb2) ? 1 : 0, fp_mults, new_size * (size_t)count);
     hipLaunchKernelGGL(k_open_fold_special, dim3(16, count), dim3(GT), 0, st, sb, old_size);
     ZK_LAUNCH_CHECK();
+    // ---- side chain (aux): nothing here feeds the next fold ----
+    if (given < 2) {
+        std::vector<MsmDesc> d;
+        std::vector<G1Jac*> out;
+        const uint32_t half = (uint32_t)(old_size / 2), ds = (uint32_t)old_size;
+        for (int i = 0; i < count; ++i) {
+            const int8_t* dg = digits + dig_bytes * i;
+            G1Jac* o = pts + npts * i;
+            if (given == 0) { d.push_back(MsmDesc{dg, items[i].gens, ds, ds, 1u, 0u, 1u, 0u}); out.push_back(o); }
+            d.push_back(MsmDesc{dg, items[i].gens, ds, half, 2u, 0u, 2u, 1u}); out.push_back(o + 1);
+            d.push_back(MsmDesc{dg, items[i].gens, ds, half, 2u, 1u, 2u, 0u}); out.push_back(o + 2);
+        }
+        return bucket_sums_queue(d, out, given == 0 ? old_size : half, arena, up, aux, later);
+    }
     return 0;
 }
 
-// Queues the batch for the last `levels` rounds (rounds r0 .. r0+levels-1 of `rounds`) over n0 <= TAIL_N generators.
-// Writes T, T0, T1 of those rounds and the final generator into pts; *final_scalar points at the folded scalar.
-// Challenges and bucket-sum descriptors of a job travel through one pinned host buffer of 64 KiB (held until the job
-// ends) into one device block: the challenges of all openings (Montgomery form, `rounds` per opening) in its first half, the
-// descriptors of the batched last rounds in its second.
-static constexpr size_t JOB_U_BYTES = 32768, JOB_DESC_BYTES = 32768;
-static int open_tail_launch(const Fr** scalars, const A29* const* gens, int count, size_t n0, int levels, int r0, int rounds, G1Jac* pts, const Fr* U_dev, void* pin_host,
-                            void* desc_dev, Arena& arena, hipStream_t st) {
-    const int n_msm = 3 * levels + 1;
-    const int total = n_msm * count;
-    ZK_ARG(sizeof(MsmDesc) * (size_t)total <= JOB_DESC_BYTES, "opening: too many sums in the batched last rounds");
-    const size_t npts = 3 * (size_t)rounds + 1;
-    const size_t sl_n = n0 + (size_t)levels + 1;
-    Scratch& sl = arena.add(sizeof(Fr) * sl_n * count);
-    const uint32_t nseg = cdiv(n0, MSEG), cps = 1;       // one chunk per workgroup, as in the halving rounds
-    const size_t ncoef = (size_t)n_msm * n0 * count;
-    Scratch& coef = arena.add(sizeof(Fr) * ncoef);
-    Scratch& partial = arena.add(sizeof(G1Jac) * total * MW * (size_t)nseg * MT);
-    Scratch& dig = arena.add((size_t)(MW + 1) * ncoef);
-    if (sl.rc) return sl.rc;
-    if (coef.rc) return coef.rc;
-    if (partial.rc) return partial.rc;
-    if (dig.rc) return dig.rc;
-    ZK_ARG(ncoef < (1ull << 32), "opening: batched last rounds too large");
-    TailPtrs tp;
-    for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; tp.SL[i] = sl.as<Fr>() + sl_n * k; tp.S[i] = scalars[k]; }
-    hipLaunchKernelGGL(k_tail_scalars, dim3(count), dim3(TAIL_SCALAR_T), 0, st, tp, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels);
-    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, 256), count), dim3(256), 0, st, coef.as<Fr>(), tp, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels);
-    {
-        RecodeBatch rb;
-        for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>(); rb.S[i] = coef.as<Fr>(); }
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, 256), 1), dim3(256), 0, st, rb, ncoef);
-    }
-    MsmDesc* hd = reinterpret_cast<MsmDesc*>((char*)pin_host + JOB_U_BYTES);
-    for (int it = 0; it < count; ++it)
-        for (int i = 0; i < n_msm; ++i) {
-            const uint32_t slot = (uint32_t)(npts * it) + (i == 3 * levels ? 3u * (uint32_t)rounds : 3u * (uint32_t)r0 + (uint32_t)i);
-            hd[it * n_msm + i] = MsmDesc{dig.as<int8_t>(), gens[it], (uint32_t)ncoef, (uint32_t)n0, 1u, (uint32_t)(((size_t)it * n_msm + i) * n0), 1u, 0u, slot};
-        }
-    ZK_HIP(hipMemcpyAsync(desc_dev, hd, sizeof(MsmDesc) * (size_t)total, hipMemcpyHostToDevice, st));
-    const MsmDesc* dd = (const MsmDesc*)desc_dev;
-    hipLaunchKernelGGL(k_msm_seg<1>, dim3(nseg, MW, total), dim3(MSL), 0, st, partial.as<G1Jac>(), MsmDescs<1>(), dd, nseg, cps);
-    hipLaunchKernelGGL(k_msm_point, dim3(total), dim3(MT), 0, st, (G1Jac*)nullptr, pts, dd, partial.as<G1Jac>(), nseg, 1u, 0u, (const PointDesc*)nullptr);
-    ZK_LAUNCH_CHECK();
-    // the folded scalar is the single element of the last level
-    size_t off = 0, nn = n0;
-    for (int j = 1; j < levels; ++j) { nn = (nn + 1) / 2; off += nn; }
-    for (int it = 0; it < count; ++it) scalars[it] = sl.as<Fr>() + sl_n * it + off;
-    return 0;
-}
+// `levels` rounds (r0 .. r0 + levels - 1 of `rounds`) in one batch over n0 generators: the scalars of all levels on st, then T, T0, T1 of
+// those rounds as bucket sums with formed coefficients on aux.  last: the batch takes all rounds that are left and the final
+// generator is one more sum; otherwise (three levels) the generators are folded three times at once on st and *gens names the results.
+// *scalars: the folded scalars.  pts: the proof points of opening 0 (npts an opening).  no_t_below: T of rounds below it is not summed here.
+static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, int no_t_below, const OpenItem* items, G1Jac* pts, size_t npts,
+                             const Fr* U_dev, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later);
+// g^(3) of every opening from its generators in one launch (k_open_fold_span); challenges: rounds r0 .. r0 + 2
+static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const OpenItem* items, Arena& arena, JobUploads& up, hipStream_t st);
 
 extern "C" {
 
@@ -1807,28 +1781,28 @@ int zk_g1_open_round(void* new_scalars, void* new_gens, uint32_t* sums_host, con
     const size_t new_size = (old_size + 1) / 2;
     Scratch pts(sizeof(G1Jac) * 3, st);
     if (pts.rc) return pts.rc;
-    Scratch wsum(sizeof(G1Jac) * 3 * MW, st);
-    if (wsum.rc) return wsum.rc;
     Arena arena(st);
-    Scratch& g29 = arena.add(sizeof(A29) * (old_size + new_size));
+    JobUploads up;
+    up.arena = &arena;
+    Scratch& g29 = arena.add(sizeof(A29) * old_size);
     Scratch& n29 = arena.add(sizeof(A29) * new_size);
     if (g29.rc || n29.rc) return g29.rc ? g29.rc : n29.rc;
     int rc = open_prep_build(g29.as<A29>(), (const G1Jac*)gens, old_size, arena, st);
     if (rc) return rc;
-    std::vector<hipEvent_t> evs;
+    std::vector<hipEvent_t> evs;          // one stream: none is made
+    std::vector<PointDesc> later;
     const RoundItem item{(Fr*)new_scalars, n29.as<A29>(), (const Fr*)scalars, g29.as<A29>(), load_fr(u), nullptr};
-    rc = open_round_launch(&item, 1, old_size, true, 0, wsum.as<G1Jac>(), 0u, arena, st, st, evs);
-    (void)evs;
-    if (rc) return rc;
+    rc = open_round_launch(&item, 1, old_size, 0, 0, pts.as<G1Jac>(), 3, arena, up, st, st, evs, later);
+    if (rc == 0) rc = points_queue(later, up, st);
+    if (rc) { (void)hipStreamSynchronize(st); return rc; }
     hipLaunchKernelGGL(k_a29_to_jac, dim3(cdiv(new_size, GT)), dim3(GT), 0, st, (G1Jac*)new_gens, n29.as<A29>(), new_size);
-    hipLaunchKernelGGL(k_open_horner, dim3(3, 1), dim3(GT), 0, st, pts.as<G1Jac>(), wsum.as<G1Jac>(), 1u, 3u, 0u);
     g1_normalize_queue<false>(pts.p, pts.as<G1Jac>(), (size_t)3, st);
     ZK_LAUNCH_CHECK();
     void* stage = nullptr;
     rc = staging(&stage, sizeof(G1Jac) * 3);
     if (rc) return rc;
     ZK_HIP(hipMemcpyAsync(stage, pts.p, sizeof(G1Jac) * 3, hipMemcpyDeviceToHost, st));
-    ZK_HIP(hipStreamSynchronize(st));
+    ZK_HIP(hipStreamSynchronize(st));          // (the uploads' pinned buffers go back when this returns)
     memcpy(sums_host, stage, sizeof(G1Jac) * 3);
     return 0;
 }
@@ -1845,88 +1819,135 @@ struct OpenJob {
     hipEvent_t ready = nullptr;    // only for jobs on a side stream
     hipStream_t aux = nullptr;     // second stream of the job (bucket sums beside the folds); equals st when the job has one stream
     std::vector<hipEvent_t> events;
-    void* pin = nullptr;           // pinned host buffer behind the job's challenges and descriptors
-    void* pin2 = nullptr;          // and behind the list of its rounds' bucket reductions
+    JobUploads up;                 // challenges, descriptors
     uint64_t ticket = 0;           // the launch thread's ticket while it queues the job's kernels
     int queue_rc = 0;              // what queuing returned, and its message
     std::string queue_err;
-    ~OpenJob() { pinned_release(pin); pinned_release(pin2); }
+    OpenJob() { up.arena = &arena; }
 };
-// One opening of the batch: its scalars, its challenges (rounds x 8 limbs) and its generators -- Jacobian, or null when
-// `prep` (their prepared form, open_prep_build) is given
-struct OpenItem { const void* scalars; const void* gens; const A29* prep; const uint32_t* u; const A29* comb = nullptr; const A29* comb2 = nullptr;
-                  const void* rows = nullptr; uint32_t nrows = 0; const uint32_t* u_rows = nullptr; int k_rows = 0; int cross_rounds = 0;
-                  const A29* comb3 = nullptr; };
-// The targets of every opening of a batch (T of round 0, then T0, T1 of the first `full` rounds) as bucket sums over the
-// openings' [pattern][row] points, on aux.  The raw buckets' reductions are appended to `later`: the caller runs them with
-// those of its halving rounds, so the 248 doublings of a reduction are waited for once per job.
-static int open_cross_sums_queue(Arena& arena, const OpenItem* items, int count, int full, G1Jac* wsum, uint32_t wstride, const Fr* const* urow_dev, const Fr* U_dev, int rounds,
-                                 hipStream_t aux, std::vector<PointDesc>& later) {
-    const uint32_t ntargets = 1u + 2u * (uint32_t)full;
-    const uint32_t npatterns = 1u + 2u * (((1u << (2 * full)) - 1u) / 3u);
-    const uint32_t widest = full ? (1u << (2 * (full - 1))) : 1u;           // patterns of the largest target
+// The targets of every opening of a batch (T of round 0; T0, T1 of the first `full` rounds; T of those rounds behind the first) as
+// bucket sums over the openings' [pattern][row] points, on aux.
+static int open_cross_sums_queue(const OpenItem* items, int count, uint32_t full, G1Jac* pts, size_t npts, const Fr* const* urow_dev, const Fr* U_dev, int rounds, Arena& arena,
+                                 JobUploads& up, hipStream_t aux, std::vector<PointDesc>& later) {
+    const uint32_t ntargets = 1u + 2u * full + (full > 1 ? full - 1 : 0u);
+    const uint32_t npatterns = cross_patterns(full);
+    uint32_t nterm_patterns = npatterns;
+    for (uint32_t r = 1; r < full; ++r) nterm_patterns += cross_patterns(r);
     CrossDigitBatch db;
     const A29* base[OB_MAX];
     const int8_t* digs[OB_MAX];
     size_t most_terms = 0, most_count = 0;
     for (int i = 0; i < count; ++i) {
-        const size_t terms = (size_t)npatterns * items[i].nrows;
+        const size_t points = (size_t)npatterns * items[i].nrows, terms = (size_t)nterm_patterns * items[i].nrows;
         ZK_ARG(items[i].nrows >= 1 && terms < (1ull << 31), "zk_g1_open: bad row count");
         most_terms = std::max(most_terms, terms);
-        most_count = std::max(most_count, (size_t)widest * items[i].nrows);
-        Scratch& aff = arena.add(sizeof(G1Affine) * terms);
-        Scratch& a29 = arena.add(sizeof(A29) * terms);
+        Scratch& aff = arena.add(sizeof(G1Affine) * points);
+        Scratch& a29 = arena.add(sizeof(A29) * points);
         Scratch& dg = arena.add((size_t)(MW + 1) * terms);
         if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
-        g1_normalize_queue<true>(aff.p, (const G1Jac*)items[i].rows, terms, aux);
-        hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(terms, 256)), dim3(256), 0, aux, a29.as<A29>(), aff.as<G1Affine>(), terms);
+        g1_normalize_queue<true>(aff.p, (const G1Jac*)items[i].rows, points, aux);
+        hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(points, 256)), dim3(256), 0, aux, a29.as<A29>(), aff.as<G1Affine>(), points);
         base[i] = a29.as<A29>();
         digs[i] = dg.as<int8_t>();
         db.it[i] = CrossDigitItem{dg.as<int8_t>(), urow_dev[i], U_dev + (size_t)i * rounds, items[i].nrows, (uint32_t)items[i].k_rows};
     }
     for (int i = count; i < OB_MAX; ++i) db.it[i] = db.it[0];
-    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, npatterns);
+    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, full, nterm_patterns);
     ZK_LAUNCH_CHECK();
-    const uint32_t chunks = cdiv(most_count, MSEG);
-    const uint32_t cps = (chunks + 255u) / 256u;
-    const uint32_t nseg = (chunks + cps - 1) / cps;
-    const uint32_t n_msm = ntargets * (uint32_t)count;
-    Scratch& partial = arena.add(sizeof(G1Jac) * n_msm * MW * (size_t)nseg * MT);
-    if (partial.rc) return partial.rc;
-    const int per = std::max(1, OB_SUMS / (int)ntargets);                  // openings whose targets fit one launch's descriptors
-    for (int g0 = 0; g0 < count; g0 += per) {
-        const int gc = std::min(per, count - g0);
-        MsmDescs<OB_SUMS> descs;
-        uint32_t z = 0;
-        for (int i = g0; i < g0 + gc; ++i)
-            for (uint32_t t = 0; t < ntargets; ++t) {
-                uint32_t q, p0, npat, slot;
-                cross_target(t, q, p0, npat, slot);
-                const uint32_t terms = npatterns * items[i].nrows, off = p0 * items[i].nrows;
-                descs.d[z++] = MsmDesc{digs[i], base[i], terms, npat * items[i].nrows, 1u, off, 1u, off, 0u};
-            }
-        const uint32_t used = z;
-        for (; z < (uint32_t)OB_SUMS; ++z) descs.d[z] = MsmDesc{digs[0], base[0], 0u, 0u, 1u, 0u, 1u, 0u, 0u};
-        hipLaunchKernelGGL(k_msm_seg<OB_SUMS>, dim3(nseg, MW, used), dim3(MSL), 0, aux, partial.as<G1Jac>() + (size_t)g0 * ntargets * MW * nseg * MT, descs, (const MsmDesc*)nullptr,
-                           nseg, cps);
-    }
-    const G1Jac* cur = partial.as<G1Jac>();
-    uint32_t ns = nseg;
-    while (ns > 1) {
-        const uint32_t ng = (ns + 7) / 8;
-        Scratch& nxt = arena.add(sizeof(G1Jac) * n_msm * MW * (size_t)ng * MT);
-        if (nxt.rc) return nxt.rc;
-        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, aux, nxt.as<G1Jac>(), cur, ns);
-        cur = nxt.as<G1Jac>();
-        ns = ng;
-    }
-    ZK_LAUNCH_CHECK();
+    std::vector<MsmDesc> d;
+    std::vector<G1Jac*> out;
     for (int i = 0; i < count; ++i)
         for (uint32_t t = 0; t < ntargets; ++t) {
-            uint32_t q, p0, npat, slot;
-            cross_target(t, q, p0, npat, slot);
-            later.push_back(PointDesc{cur + ((size_t)i * ntargets + t) * MW * ns * MT, wsum + (size_t)wstride * i + slot, ns, 0u});
+            uint32_t p0, npat, t0, slot;
+            cross_target(t, full, p0, npat, t0, slot);
+            const uint32_t nr = items[i].nrows;
+            most_count = std::max(most_count, (size_t)npat * nr);
+            d.push_back(MsmDesc{digs[i], base[i], nterm_patterns * nr, npat * nr, 1u, t0 * nr, 1u, p0 * nr});
+            out.push_back(pts + npts * i + slot);
         }
+    return bucket_sums_queue(d, out, most_count, arena, up, aux, later);
+}
+static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const OpenItem* items, Arena& arena, JobUploads& up, hipStream_t st) {
+    const size_t ns = (((n0 + 1) / 2 + 1) / 2 + 1) / 2;
+    Scratch& g2 = arena.add(sizeof(A29) * ns * count);
+    if (g2.rc) return g2.rc;
+    std::vector<JsfK> jsf((size_t)count * JUMP_SPAN);
+    SpanBatch sb;
+    double fp_mults = 0;
+    for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; sb.ng[i] = g2.as<A29>() + ns * k; sb.g[i] = gens[k]; }
+    for (int i = 0; i < count; ++i) {
+        Fr c[JUMP_SPAN];
+        fold_span_coefficients(c, items[i].u + 8 * (size_t)r0);
+        for (int b = 0; b < JUMP_SPAN; ++b) {
+            jsf[(size_t)i * JUMP_SPAN + b] = jsf_of(glv_split(c[b]));
+            fp_mults += (fold_fp_mults_per_pair(jsf[(size_t)i * JUMP_SPAN + b]) + 2.0) * (double)ns;      // about what the walk of a pair takes
+        }
+    }
+    const void* dj = nullptr;
+    int rc = up.put(jsf.data(), sizeof(JsfK) * jsf.size(), st, &dj);
+    if (rc) return rc;
+    FoldTimed timed(st);
+    hipLaunchKernelGGL(k_open_fold_span, dim3(cdiv(ns, GT), count), dim3(8 * GT), 0, st, sb, (const JsfK*)dj, n0, ns);
+    ZK_LAUNCH_CHECK();
+    timed.end(0, fp_mults, ns * (size_t)count * (JUMP_SPAN - 1));
+    for (int i = 0; i < count; ++i) gens[i] = g2.as<A29>() + ns * i;
+    return 0;
+}
+static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, int no_t_below, const OpenItem* items, G1Jac* pts, size_t npts,
+                             const Fr* U_dev, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
+    const uint32_t fin = last ? 1u : 0u, n_msm = 3 * (uint32_t)levels + fin;
+    const size_t sl_n = n0 + (size_t)levels + 1;
+    Scratch& sl = arena.add(sizeof(Fr) * sl_n * count);
+    const size_t ncoef = (size_t)n_msm * n0 * count;
+    Scratch& coef = arena.add(sizeof(Fr) * ncoef);
+    Scratch& dig = arena.add((size_t)(MW + 1) * ncoef);
+    if (sl.rc || coef.rc || dig.rc) return sl.rc ? sl.rc : (coef.rc ? coef.rc : dig.rc);
+    ZK_ARG(ncoef < (1ull << 32), "opening: batched rounds too large");
+    TailPtrs tp;
+    for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; tp.SL[i] = sl.as<Fr>() + sl_n * k; tp.S[i] = scalars[k]; }
+    const TailPtrs all = tp;
+    size_t n = n0, off = 0;               // off: where the level just formed starts
+    for (int j = 0; j < levels;) {
+        if (levels - j >= 3 && (n > 2048 || levels == 3)) {
+            hipLaunchKernelGGL(k_tail_scalars3, dim3(cdiv((n + 7) / 8, 256), count), dim3(256), 0, st, tp, U_dev + r0 + j, (uint32_t)rounds, (uint32_t)n);
+            const size_t n1 = (n + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2;
+            for (int i = 0; i < OB_MAX; ++i) { tp.S[i] = tp.SL[i] + n1 + n2; tp.SL[i] += n1 + n2 + n3; }
+            off = (size_t)(tp.S[0] - sl.as<Fr>());
+            n = n3;
+            j += 3;
+        } else {
+            hipLaunchKernelGGL(k_tail_scalars, dim3(count), dim3(TAIL_SCALAR_T), 0, st, tp, U_dev + r0 + j, (uint32_t)rounds, (uint32_t)n, (uint32_t)(levels - j));
+            off = (size_t)(tp.SL[0] - sl.as<Fr>());
+            for (; j < levels; ++j) { n = (n + 1) / 2; if (j + 1 < levels) off += n; }
+        }
+    }
+    ZK_LAUNCH_CHECK();
+    int rc = join_streams(st, aux, events);
+    if (rc) return rc;
+    const A29* before[OB_MAX];
+    for (int i = 0; i < count; ++i) before[i] = gens[i];
+    if (!last) {
+        rc = open_span_fold(gens, count, n0, r0, items, arena, up, st);
+        if (rc) return rc;
+    }
+    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, 256), count), dim3(256), 0, aux, coef.as<Fr>(), all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, fin);
+    {
+        RecodeBatch rb;
+        for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>(); rb.S[i] = coef.as<Fr>(); }
+        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, 256), 1), dim3(256), 0, aux, rb, ncoef);
+    }
+    ZK_LAUNCH_CHECK();
+    std::vector<MsmDesc> d;
+    std::vector<G1Jac*> out;
+    for (int it = 0; it < count; ++it)
+        for (uint32_t i = 0; i < n_msm; ++i) {
+            if (i < 3 * (uint32_t)levels && i % 3 == 0 && r0 + (int)(i / 3) < no_t_below) continue;
+            d.push_back(MsmDesc{dig.as<int8_t>(), before[it], (uint32_t)ncoef, (uint32_t)n0, 1u, (uint32_t)(((size_t)it * n_msm + i) * n0), 1u, 0u});
+            out.push_back(pts + npts * it + (i == 3 * (uint32_t)levels ? 3 * (size_t)rounds : 3 * (size_t)r0 + i));
+        }
+    rc = bucket_sums_queue(d, out, n0, arena, up, aux, later);
+    if (rc) return rc;
+    for (int it = 0; it < count; ++it) scalars[it] = sl.as<Fr>() + sl_n * it + off;
     return 0;
 }
 // rows (optional): commitments of the opened tensor's rows, [pattern][row] as open_cross_sums_queue takes them -- the row
@@ -1942,30 +1963,21 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     job.rounds = rounds;
     job.count = count;
     const size_t npts = 3 * (size_t)rounds + 1;
-    const uint32_t wstride = 3u * MW * (uint32_t)(rounds ? rounds : 1);      // window sums of one opening's halving rounds
     Scratch& pts = job.arena.add(sizeof(G1Jac) * npts * count);
-    Scratch& wsum = job.arena.add(sizeof(G1Jac) * (size_t)wstride * count);
     if (pts.rc) return pts.rc;
-    if (wsum.rc) return wsum.rc;
     job.pts = pts.as<G1Jac>();
-    size_t n_urows = 0;
-    for (int i = 0; i < count; ++i) n_urows += items[i].rows ? (size_t)items[i].k_rows : 0;
-    ZK_ARG(sizeof(Fr) * ((size_t)rounds * count + n_urows) <= JOB_U_BYTES, "zk_g1_open: too many rounds for the batch");
-    Scratch& jdev = job.arena.add(JOB_U_BYTES + JOB_DESC_BYTES);
-    if (jdev.rc) return jdev.rc;
-    {
-        int prc = pinned_acquire(&job.pin);
-        if (prc) return prc;
-        Fr* hu = (Fr*)job.pin;
-        for (int i = 0; i < count; ++i)
-            for (int r = 0; r < rounds; ++r) hu[(size_t)i * rounds + r] = to_mont(load_fr(items[i].u + 8 * r));
-        size_t at = (size_t)rounds * count;           // the row challenges follow
-        for (int i = 0; i < count; ++i)
-            if (items[i].rows)
-                for (int j = 0; j < items[i].k_rows; ++j) hu[at++] = to_mont(load_fr(items[i].u_rows + 8 * j));
-        if (at) ZK_HIP(hipMemcpyAsync(jdev.p, job.pin, sizeof(Fr) * at, hipMemcpyHostToDevice, st));
+    std::vector<Fr> hu;           // the challenges, Montgomery form, `rounds` an opening; the row challenges follow
+    for (int i = 0; i < count; ++i)
+        for (int r = 0; r < rounds; ++r) hu.push_back(to_mont(load_fr(items[i].u + 8 * r)));
+    for (int i = 0; i < count; ++i)
+        if (items[i].rows)
+            for (int j = 0; j < items[i].k_rows; ++j) hu.push_back(to_mont(load_fr(items[i].u_rows + 8 * j)));
+    const void* ud = nullptr;
+    if (!hu.empty()) {
+        int rc = job.up.put(hu.data(), sizeof(Fr) * hu.size(), st, &ud);
+        if (rc) return rc;
     }
-    const Fr* U_dev = jdev.as<Fr>();
+    const Fr* U_dev = (const Fr*)ud;
     const Fr* urow_dev[OB_MAX];
     {
         size_t at = (size_t)rounds * count;
@@ -1977,99 +1989,107 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         cs[i] = (const Fr*)items[i].scalars;
         cg[i] = items[i].prep;
         if (!cg[i]) {
-            Scratch& g29 = job.arena.add(sizeof(A29) * (n + (n + 1) / 2));
+            Scratch& g29 = job.arena.add(sizeof(A29) * n);
             if (g29.rc) return g29.rc;
             int rc = open_prep_build(g29.as<A29>(), (const G1Jac*)items[i].gens, n, job.arena, st);
             if (rc) return rc;
             cg[i] = g29.as<A29>();
         }
     }
+    auto last_batch = [&](size_t size, int r) { return size * (size_t)count <= (size_t)LAST_N && rounds - r <= TAIL_LEVELS; };
     // commitments of the tensors' rows: which sums they replace (all openings of the batch must bring them)
-    bool with_rows = true;
+    bool with_rows = true, comb3 = true;
     int cross_r = 64;
-    for (int i = 0; i < count; ++i) { with_rows = with_rows && items[i].rows != nullptr; cross_r = std::min(cross_r, items[i].cross_rounds); }
-    if (!with_rows) cross_r = 0;
-    int rounds_from_rows = 0;                 // halving rounds that take sums from the row commitments
-    if (with_rows) {
-        int halving = 0;
-        size_t sz = n;
-        for (int r = 0; r < rounds && !(sz <= (size_t)TAIL_N && rounds - r <= TAIL_LEVELS); ++r) { ++halving; sz = (sz + 1) / 2; }
-        rounds_from_rows = std::min(halving, std::max(cross_r, 1));
+    for (int i = 0; i < count; ++i) {
+        with_rows = with_rows && items[i].rows != nullptr;
+        cross_r = std::min(cross_r, items[i].cross_rounds);
+        comb3 = comb3 && items[i].comb3 != nullptr;
     }
+    int halving = 0;
+    {
+        size_t sz = n;
+        for (int r = 0; r < rounds && !last_batch(sz, r); ++r) { ++halving; sz = (sz + 1) / 2; }
+    }
+    // row commitments alone: T of the first round from them, T of the rounds over more than TABLE_MIN_N generators unrolled from it
+    int rows_t = 0;
+    if (with_rows && cross_r == 0)
+        for (size_t sz = n; rows_t < rounds && sz > (size_t)TABLE_MIN_N; sz = (sz + 1) / 2) ++rows_t;
+    if (!with_rows || halving == 0) cross_r = 0;
+    // three rounds as one fold: their sums all come from cross commitments
+    const bool jump = halving > 0 && with_rows && cross_r >= JUMP_ROUNDS && rounds >= JUMP_ROUNDS && !(n & (n - 1)) && n >= (size_t)JUMP_SPAN;
+    if (jump) cross_r = JUMP_ROUNDS;
+    else cross_r = std::min(cross_r, halving);
     std::vector<PointDesc> later;        // bucket reductions that nothing waits for before the end: one launch behind the last round
-    if (rounds_from_rows > 0) {
-        if (aux != st) {          // the challenges travel on st
-            hipEvent_t up;
-            ZK_HIP(hipEventCreateWithFlags(&up, hipEventDisableTiming));
-            job.events.push_back(up);
-            ZK_HIP(hipEventRecord(up, st));
-            ZK_HIP(hipStreamWaitEvent(aux, up, 0));
-        }
-        int rc = open_cross_sums_queue(job.arena, items, count, std::min(rounds_from_rows, cross_r), wsum.as<G1Jac>(), wstride, urow_dev, U_dev, rounds, aux, later);
+    if (rows_t > 1) GLAUNCH(k_g1_fill, npts * count, st, job.pts, g1_infinity(), npts * count);
+    if (cross_r > 0 || rows_t > 0) {
+        int rc = join_streams(st, aux, job.events);          // the challenges travel on st
+        if (rc == 0) rc = open_cross_sums_queue(items, count, (uint32_t)cross_r, job.pts, npts, urow_dev, U_dev, rounds, job.arena, job.up, aux, later);
         if (rc) return rc;
     }
     size_t size = n;
-    int halving_rounds = rounds;
+    int r = 0;
     bool tail_done = false;
-    int r_first = 0;
-    // three rounds as one fold: every opening brings the jump tables and cross commitments for those rounds, and all
-    // three are halving rounds
-    {
-        bool jump = with_rows && cross_r >= JUMP_ROUNDS && rounds_from_rows >= JUMP_ROUNDS && rounds >= JUMP_ROUNDS && !(n & (n - 1));
-        for (int i = 0; i < count; ++i) jump = jump && items[i].comb3 != nullptr;
-        if (jump) {
-            const size_t ns = n >> JUMP_ROUNDS;
+    if (jump) {
+        const size_t ns = n >> JUMP_ROUNDS;
+        if (comb3) {
             Scratch& s2 = job.arena.add(sizeof(Fr) * ns * count);
             Scratch& g2 = job.arena.add(sizeof(A29) * ns * count);
             if (s2.rc) return s2.rc;
             if (g2.rc) return g2.rc;
             JumpBatch jb;
             double fp_mults = 0;
-            const Fr one = big_one_mont<8>();
             for (int i = 0; i < OB_MAX; ++i) {
                 const int k = i < count ? i : 0;
                 JumpItem& f = jb.it[i];
                 f.ns = s2.as<Fr>() + ns * k; f.ng = g2.as<A29>() + ns * k; f.s = cs[k]; f.g = cg[k]; f.tab = items[k].comb3;
-                Fr um[JUMP_ROUNDS];
-                for (int q = 0; q < JUMP_ROUNDS; ++q) um[q] = f.u_mont[q] = to_mont(load_fr(items[k].u + 8 * q));
+                for (int q = 0; q < JUMP_ROUNDS; ++q) f.u_mont[q] = to_mont(load_fr(items[k].u + 8 * q));
+                Fr c[JUMP_SPAN];
+                fold_span_coefficients(c, items[k].u);
                 for (int b = 0; b < JUMP_TABS; ++b) {
-                    Fr c = one;           // c_b = prod_q (bit_q(b) ? 1 - u_q : u_q)
-                    for (int q = 0; q < JUMP_ROUNDS; ++q) c = mont_mul(c, ((b >> q) & 1) ? sub(one, um[q]) : um[q]);
-                    f.ck[b] = comb_of(glv_split(from_mont(c)));
+                    f.ck[b] = comb_of(glv_split(c[b]));
                     if (i < count) fp_mults += (comb_fp_mults_per_pair(f.ck[b]) - 7.0 * COMB_W - 19.0) * (double)ns;
                 }
                 if (i < count) fp_mults += (7.0 * COMB_W + 19.0) * (double)ns;
             }
-            hipEvent_t t0 = nullptr, t1 = nullptr;
-            if (g_fold_timer.on) {
-                ZK_HIP(hipEventCreate(&t0));
-                ZK_HIP(hipEventCreate(&t1));
-                ZK_HIP(hipEventRecord(t0, st));
-            }
+            FoldTimed timed(st);
             hipLaunchKernelGGL(k_open_fold_jump, dim3(cdiv(ns, GT), count), dim3(GT), 0, st, jb, ns);
             ZK_LAUNCH_CHECK();
-            if (g_fold_timer.on) {
-                ZK_HIP(hipEventRecord(t1, st));
-                std::lock_guard<std::mutex> lk(g_fold_timer.mu);
-                g_fold_timer.ev.emplace_back(t0, t1);
-                g_fold_timer.fp_mults += fp_mults;
-                g_fold_timer.pairs += ns * (size_t)count * (JUMP_SPAN - 1);       // pairs the three rounds fold: 4 + 2 + 1 per result
-                g_fold_timer.method.push_back(2);
-                g_fold_timer.m_mults[2] += fp_mults;
-                g_fold_timer.m_pairs[2] += ns * (size_t)count * (JUMP_SPAN - 1);
-            }
+            timed.end(2, fp_mults, ns * (size_t)count * (JUMP_SPAN - 1));       // pairs the three rounds fold: 4 + 2 + 1 per result
             for (int i = 0; i < count; ++i) { cs[i] = s2.as<Fr>() + ns * i; cg[i] = g2.as<A29>() + ns * i; }
-            size = ns;
-            r_first = JUMP_ROUNDS;
-        }
-    }
-    for (int r = r_first; r < rounds; ++r) {
-        if (size <= (size_t)TAIL_N && rounds - r <= TAIL_LEVELS) {
-            int rc = open_tail_launch(cs, cg, count, size, rounds - r, r, rounds, pts.as<G1Jac>(), U_dev, job.pin, (char*)jdev.p + JOB_U_BYTES, job.arena, st);
+        } else {
+            const size_t sl_n = n;          // levels 1 to 3 of the scalars
+            Scratch& sl = job.arena.add(sizeof(Fr) * sl_n * count);
+            if (sl.rc) return sl.rc;
+            TailPtrs tp;
+            for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; tp.SL[i] = sl.as<Fr>() + sl_n * k; tp.S[i] = cs[k]; }
+            hipLaunchKernelGGL(k_tail_scalars3, dim3(cdiv(ns, 256), count), dim3(256), 0, st, tp, U_dev, (uint32_t)rounds, (uint32_t)n);
+            ZK_LAUNCH_CHECK();
+            int rc = open_span_fold(cg, count, n, 0, items, job.arena, job.up, st);
             if (rc) return rc;
-            halving_rounds = r;
+            for (int i = 0; i < count; ++i) cs[i] = sl.as<Fr>() + sl_n * i + n / 2 + n / 4;
+        }
+        size = ns;
+        r = JUMP_ROUNDS;
+    }
+    while (r < rounds) {
+        if (last_batch(size, r)) {
+            std::vector<PointDesc> mine;
+            int rc = open_batch_launch(cs, cg, count, size, rounds - r, true, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, st, job.events, mine);
+            if (rc == 0) rc = points_queue(mine, job.up, st);
+            if (rc) return rc;
             tail_done = true;
             break;
+        }
+        bool comb = r <= 1;
+        for (int i = 0; i < count; ++i) comb = comb && (r == 0 ? items[i].comb : items[i].comb2) != nullptr;
+        // Three rounds as a batch of sums beside one fold where a round's fold would leave the chip half empty and take one walk's
+        // latency (2.4 ms) all the same; above that a round at a time, which sums over fewer points.
+        if (!comb && r >= cross_r && rounds - r >= JUMP_ROUNDS && size * (size_t)count <= (size_t)SPAN_MAX_N) {
+            int rc = open_batch_launch(cs, cg, count, size, JUMP_ROUNDS, false, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, aux, job.events, later);
+            if (rc) return rc;
+            size = (((size + 1) / 2 + 1) / 2 + 1) / 2;
+            r += JUMP_ROUNDS;
+            continue;
         }
         const size_t ns = (size + 1) / 2;
         Scratch& s2 = job.arena.add(sizeof(Fr) * ns * count);
@@ -2082,41 +2102,43 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
             if (r == 0) ri[i].comb = items[i].comb;
             if (r == 1) { ri[i].comb2 = items[i].comb2; ri[i].u_prev = load_fr(items[i].u + 8 * (r - 1)); }
         }
-        const int given = !with_rows ? 0 : (r < cross_r ? 2 : (r == 0 ? 1 : 0));
-        int rc = open_round_launch(ri, count, size, r == 0, given, wsum.as<G1Jac>() + (size_t)3 * MW * r, wstride, job.arena, st, aux, job.events, aux != st ? &later : nullptr);
+        const int given = r < cross_r ? 2 : (r < rows_t ? 1 : 0);
+        int rc = open_round_launch(ri, count, size, std::min(r, 2), given, job.pts + 3 * (size_t)r, npts, job.arena, job.up, st, aux, job.events, later);
         if (rc) return rc;
         for (int i = 0; i < count; ++i) { cs[i] = ri[i].new_scalars; cg[i] = ri[i].new_gens; }
         size = ns;
+        ++r;
     }
-    if (!later.empty()) {
-        ZK_ARG(sizeof(PointDesc) * later.size() <= 65536, "zk_g1_open: too many sums");
-        int prc = pinned_acquire(&job.pin2);
-        if (prc) return prc;
-        memcpy(job.pin2, later.data(), sizeof(PointDesc) * later.size());
-        Scratch& ld = job.arena.add(sizeof(PointDesc) * later.size());
-        if (ld.rc) return ld.rc;
-        ZK_HIP(hipMemcpyAsync(ld.p, job.pin2, sizeof(PointDesc) * later.size(), hipMemcpyHostToDevice, aux));
-        hipLaunchKernelGGL(k_msm_point, dim3((unsigned)later.size()), dim3(MT), 0, aux, (G1Jac*)nullptr, (G1Jac*)nullptr, (const MsmDesc*)nullptr, (const G1Jac*)nullptr, 0u, 1u, 0u,
-                           (const PointDesc*)ld.p);
-        ZK_LAUNCH_CHECK();
+    {
+        int rc = points_queue(later, job.up, aux);
+        if (rc == 0) rc = join_streams(aux, st, job.events);
+        if (rc) return rc;
     }
-    // the single points of the halving rounds, behind the last bucket sums
-    if (halving_rounds > 0) {
-        hipLaunchKernelGGL(k_open_horner, dim3(3 * halving_rounds, count), dim3(GT), 0, aux, pts.as<G1Jac>(), wsum.as<G1Jac>(), (uint32_t)halving_rounds, (uint32_t)npts, wstride);
-        if (halving_rounds > 1)
-            hipLaunchKernelGGL(k_open_chain, dim3(halving_rounds - 1, count), dim3(GT), 0, aux, pts.as<G1Jac>(), U_dev, (uint32_t)halving_rounds, (uint32_t)npts, (uint32_t)rounds);
-        ZK_LAUNCH_CHECK();
-    }
-    if (aux != st) {
-        hipEvent_t done;
-        ZK_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
-        job.events.push_back(done);
-        ZK_HIP(hipEventRecord(done, aux));
-        ZK_HIP(hipStreamWaitEvent(st, done, 0));
+    if (rows_t > 1) {
+        const uint32_t R = (uint32_t)rows_t, np = 3 * R, terms = (R - 1) * np;
+        Scratch& aff = job.arena.add(sizeof(G1Affine) * np);
+        Scratch& a29 = job.arena.add(sizeof(A29) * np * count);
+        Scratch& dg = job.arena.add((size_t)(MW + 1) * terms * count);
+        if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
+        std::vector<MsmDesc> d;
+        std::vector<G1Jac*> out;
+        for (int i = 0; i < count; ++i) {
+            g1_normalize_queue<true>(aff.p, job.pts + npts * i, np, st);
+            hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(np, 256)), dim3(256), 0, st, a29.as<A29>() + (size_t)np * i, aff.as<G1Affine>(), (size_t)np);
+            for (uint32_t q = 1; q < R; ++q) {
+                d.push_back(MsmDesc{dg.as<int8_t>() + (size_t)(MW + 1) * terms * i, a29.as<A29>() + (size_t)np * i, terms, np, 1u, (q - 1) * np, 1u, 0u});
+                out.push_back(job.pts + npts * i + 3 * q);
+            }
+        }
+        hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R);
+        std::vector<PointDesc> mine;
+        int rc = bucket_sums_queue(d, out, np, job.arena, job.up, st, mine);
+        if (rc == 0) rc = points_queue(mine, job.up, st);
+        if (rc) return rc;
     }
     if (!tail_done)
-        for (int i = 0; i < count; ++i) hipLaunchKernelGGL(k_open_finish, dim3(1), dim3(GT), 0, st, pts.as<G1Jac>() + npts * i, cg[i], (uint32_t)rounds);
-    g1_normalize_queue<false>(pts.p, pts.as<G1Jac>(), npts * count, st);
+        for (int i = 0; i < count; ++i) hipLaunchKernelGGL(k_open_finish, dim3(1), dim3(GT), 0, st, job.pts + npts * i, cg[i], (uint32_t)rounds);
+    g1_normalize_queue<false>(pts.p, job.pts, npts * count, st);
     ZK_LAUNCH_CHECK();
     for (int i = 0; i < count; ++i) job.final_scalar[i] = cs[i];
     return 0;
@@ -2140,6 +2162,11 @@ static int open_collect(OpenJob& job, uint32_t* proof_host, uint32_t* final_scal
 // proof_host receives 3*rounds + 1 points: T, T0, T1 of every round, then the folded generator; all normalised to
 // z = 1 (infinity: all-zero limbs).  final_scalar_host: the folded scalar.
 int zk_g1_open(uint32_t* proof_host, uint32_t* final_scalar_host, const void* scalars, const void* gens, size_t n, const uint32_t* u, int rounds, void* stv) {
+    if (n > (size_t)LAST_N) {          // folds and bucket sums beside each other, on two streams
+        void* h = nullptr;
+        int rc = zk_g1_open_begin(&h, scalars, gens, n, u, rounds, stv);
+        return rc ? rc : zk_g1_open_end(h, proof_host, final_scalar_host);
+    }
     OpenJob job;
     const OpenItem item{scalars, gens, nullptr, u};
     int rc = open_queue(job, &item, 1, n, rounds, (hipStream_t)stv, (hipStream_t)stv);
@@ -2203,8 +2230,8 @@ int zk_g1_open_begin(void** handle, const void* scalars, const void* gens, size_
     const OpenItem item{scalars, gens, nullptr, u};
     return open_begin_impl(handle, &item, 1, n, rounds, stv);
 }
-// Generators prepared once for any number of openings against them: their affine 29-bit-limb form and the pair sums of
-// the first round (weight-independent; 1.5 n points of 112 bytes).  The handle is freed with zk_g1_open_prepared_free
+// Generators prepared once for any number of openings against them: their affine 29-bit-limb form
+// (weight-independent; n points of 112 bytes).  The handle is freed with zk_g1_open_prepared_free
 // once no opening that uses it is pending.
 struct OpenPrepared { void* a29 = nullptr; size_t n = 0; void* comb = nullptr; void* comb2 = nullptr; void* comb3 = nullptr; size_t table_bytes = 0; };      // comb3: k_open_fold_jump's tables (instead of the other two)
 static int open_prepare_impl(void** prepared, const void* gens, size_t n, int table_mode, void* stv);
@@ -2215,11 +2242,11 @@ int zk_g1_open_prepare_tables(void** prepared, const void* gens, size_t n, int t
 }
 // bytes of fold tables that zk_g1_open_prepare_tables(.., tables) keeps for n generators (0 where that mode makes none for this n)
 static size_t open_table_bytes(size_t n, int tables) {
-    if (tables >= 3 && !(n & (n - 1)) && (n >> JUMP_ROUNDS) >= (size_t)TAIL_N) return sizeof(A29) * (n >> JUMP_ROUNDS) * COMB_N * JUMP_TABS;
-    if (tables < 1 || n <= (size_t)TAIL_N) return 0;
+    if (tables >= 3 && !(n & (n - 1)) && (n >> JUMP_ROUNDS) >= (size_t)TABLE_MIN_N) return sizeof(A29) * (n >> JUMP_ROUNDS) * COMB_N * JUMP_TABS;
+    if (tables < 1 || n <= (size_t)TABLE_MIN_N) return 0;
     const size_t np = (n + 1) / 2, nq = (np + 1) / 2;
     size_t b = sizeof(A29) * np * COMB_N;
-    if (tables >= 2 && np > (size_t)TAIL_N) b += sizeof(A29) * 2 * nq * COMB_N;
+    if (tables >= 2 && np > (size_t)TABLE_MIN_N) b += sizeof(A29) * 2 * nq * COMB_N;
     return b;
 }
 size_t zk_g1_open_table_bytes(size_t n, int tables) { return open_table_bytes(n, tables < 0 ? 0 : (tables > 3 ? 3 : tables)); }
@@ -2236,7 +2263,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(prepared != nullptr && n >= 1, "zk_g1_open_prepare: null handle or no generators");
     std::unique_ptr<OpenPrepared> pr(new OpenPrepared);
-    int rc = pool_alloc(&pr->a29, sizeof(A29) * (n + (n + 1) / 2), st);
+    int rc = pool_alloc(&pr->a29, sizeof(A29) * n, st);
     if (rc) return rc;
     pr->n = n;
     {
@@ -2254,7 +2281,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
         const int table_rounds = env_rounds >= 0 ? env_rounds : table_mode;
         // mode 3: the seven tables of k_open_fold_jump in place of those two (as large as both together); only for a power of
         // two of generators that leaves more than the batched last rounds take after three folds
-        const bool jump = table_rounds >= 3 && !(n & (n - 1)) && (n >> JUMP_ROUNDS) >= (size_t)TAIL_N;
+        const bool jump = table_rounds >= 3 && !(n & (n - 1)) && (n >> JUMP_ROUNDS) >= (size_t)TABLE_MIN_N;
         if (rc == 0 && jump) {
             const size_t no = n >> JUMP_ROUNDS, ne = no * COMB_N * JUMP_TABS;
             int trc = pool_alloc(&pr->comb3, sizeof(A29) * ne, st);
@@ -2292,10 +2319,10 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                 if (hipGetLastError() != hipSuccess) rc = hip_fail(hipErrorLaunchFailure, "jump table build", __FILE__, __LINE__);
             }
         }
-        if (rc == 0 && n > (size_t)TAIL_N && table_rounds >= 1 && !pr->comb3) {
+        if (rc == 0 && n > (size_t)TABLE_MIN_N && table_rounds >= 1 && !pr->comb3) {
             const size_t np = (n + 1) / 2, ne = np * COMB_N;
             const size_t nq = (np + 1) / 2, ne2 = nq * COMB_N;        // second round: two tables over the pairs of pairs
-            bool second = np > (size_t)TAIL_N && table_rounds >= 2;   // that round is a fold too
+            bool second = np > (size_t)TABLE_MIN_N && table_rounds >= 2;   // that round is a fold too
             int trc = pool_alloc(&pr->comb, sizeof(A29) * ne, st);
             if (trc == 0 && second && pool_alloc(&pr->comb2, sizeof(A29) * 2 * ne2, st) != 0) { pr->comb2 = nullptr; second = false; }
             const size_t nt = second ? std::max(ne, 2 * ne2) : ne;
@@ -2329,7 +2356,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
                 };
                 G1Jac* T = tj.as<G1Jac>();
                 g1_normalize_queue<true>(aff.p, (const G1Jac*)gens, n, st);
-                hipLaunchKernelGGL(k_open_pair_points, dim3(cdiv(np, GT)), dim3(GT), 0, st, T, aff.as<G1Affine>(), n, np, 1);
+                hipLaunchKernelGGL(k_open_pair_points, dim3(cdiv(np, GT)), dim3(GT), 0, st, T, aff.as<G1Affine>(), n, np);
                 fill(T, np);
                 g1_normalize_queue<true>(ta.p, tj.as<G1Jac>(), ne, st);
                 hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(ne, 256)), dim3(256), 0, st, (A29*)pr->comb, ta.as<G1Affine>(), ne);
