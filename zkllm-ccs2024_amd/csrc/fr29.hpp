@@ -30,6 +30,8 @@ ZK_HD Fr29 fr29_const(const int32_t (&t)[9]) {
     return r;
 }
 ZK_HD Fr29 fr29_r() { constexpr int32_t t[9] = {1, 536870904, 529989567, 457704959, 494949691, 201589968, 354471143, 174404527, 7597479}; return fr29_const(t); }
+ZK_HD Fr29 fr29_2_261() { constexpr int32_t t[9] = {536870842, 559, 481694080, 172907520, 250130850, 384216799, 419952827, 139714039, 5047359}; return fr29_const(t); }     // 2^261 mod r
+ZK_HD Fr29 fr29_2_527() { constexpr int32_t t[9] = {238450677, 105123874, 285095421, 524243062, 304996105, 406999561, 483795002, 430521147, 293893}; return fr29_const(t); }     // 2^527 mod r
 ZK_HD Fr29 fr29_2_266() { constexpr int32_t t[9] = {536868651, 18087, 526333248, 216203804, 294598241, 8484555, 89016444, 271483280, 1968430}; return fr29_const(t); }     // 2^266 mod r
 ZK_HD Fr29 fr29_2_271() { constexpr int32_t t[9] = {536798552, 578879, 254716416, 35656607, 98837070, 269398762, 12757061, 312906888, 2209941}; return fr29_const(t); }     // 2^271 mod r
 ZK_HD Fr29 fr29_2_522() { constexpr int32_t t[9] = {175223744, 489824382, 375642521, 475708563, 62229572, 199455800, 136968049, 375395230, 2620817}; return fr29_const(t); }   // 2^522 mod r
@@ -186,8 +188,8 @@ ZK_HD Fr29 fr29_repack(const Big<8>& a) {
     }
     return r;
 }
-// canonical residue of a non-negative value below (PASSES + 1) r, as 8 x 32-bit words
-template <int PASSES = 2> ZK_HD Big<8> fr29_canon_pack(const Fr29& a) {
+// canonical residue of a non-negative value below (PASSES + 1) r
+template <int PASSES = 2> ZK_HD Fr29 fr29_canon(const Fr29& a) {
     Fr29 v = a;
 #pragma unroll
     for (int pass = 0; pass < PASSES; ++pass) {
@@ -202,6 +204,10 @@ template <int PASSES = 2> ZK_HD Big<8> fr29_canon_pack(const Fr29& a) {
         t.l[8] = v.l[8] - fr29_p(8) + c;
         if (t.l[8] >= 0) v = t;
     }
+    return v;
+}
+// a canonical value as 8 x 32-bit words
+ZK_HD Big<8> fr29_pack(const Fr29& v) {
     Big<8> r;
 #pragma unroll
     for (int w = 0; w < 8; ++w) {
@@ -213,6 +219,7 @@ template <int PASSES = 2> ZK_HD Big<8> fr29_canon_pack(const Fr29& a) {
     }
     return r;
 }
+template <int PASSES = 2> ZK_HD Big<8> fr29_canon_pack(const Fr29& a) { return fr29_pack(fr29_canon<PASSES>(a)); }
 
 // A sum of products that is reduced once.  Columns 0..16 take the limb products of every term, column 17 what carries out of
 // them; the operands' limbs are non-negative, so a column grows by less than 9 * 2^58 per term and wide29_carry must run at

@@ -1144,7 +1144,7 @@ static constexpr int TAIL_T = 1024;          // lanes of the single workgroup
 static constexpr int TAIL_HALF = 256;        // largest n_out of the first fused round: one compute unit does all of it
 static constexpr int TAIL_ROUNDS = 16;
 struct TailV { Fr v[TAIL_ROUNDS]; };         // Montgomery form, in round order
-static constexpr int SPLIT_HALF = 32768;     // rounds of at most this many pairs spread each pair over several lanes
+static constexpr int SPLIT_HALF = 32768;     // pairs of a first round up to which queries are inverted ahead of the rounds instead of inside the first one
 
 __device__ __forceinline__ Fr wave_sum(Fr x) {
 #pragma unroll
@@ -1183,132 +1183,191 @@ template <int K> __device__ __forceinline__ void tail_block_sum(Fr (&acc)[K], Fr
     __syncthreads();
 }
 
-// A lookup round splits into four independent tasks per pair, so that short rounds -- where lanes are plentiful and the
-// chain of ~20 dependent field multiplications per pair is what takes the time -- can spread a pair over four lanes:
-//   task 0: sums 0..2 (E-weighted products of A and S + beta)        task 1: sums 5..7 (the same for B and T + beta)
-//   task 2: sums 8..10 (products of m and B), folds of m, A and S     task 3: sums 3..4 (a0, da), folds of B and T
-// Phase 1 has tasks 0 and 3' only (3' = sums 3..4 and the folds of A and S).  acc receives the task's sums (up to 3).
-struct LookupPtrs {
+// ---- several short rounds in one launch -----------------------------------------------------------------------------------------
+// Rounds over short tensors are latency: a launch or a workgroup barrier per round, and within the round the chain of dependent field
+// products of a pair.  A round pairs t with t + n/2 (the top index bit), so the elements that agree in their low bits need nobody
+// else for as many rounds as there are high bits: a workgroup takes c consecutive low indices with all 2^R values of the top R bits
+// (P = c 2^R elements of every tensor, in LDS, 29-bit limbs) and runs R rounds on them, one barrier each.  The challenges are known
+// ahead; each round's sums over the workgroup go to the partial sums of that round, the folded tensors (c elements) to memory.
+// Within a round every product of a pair has a lane of its own, at most two products in a row.  Sixteen lanes (a row of the
+// data-parallel operations) do one thing for sixteen pairs, four waves everything for them --
+//   wave 0: E a0 s0 | E a1 s1 | E da ds                               (s = S + beta; its fourth row idles)
+//   wave 1: E b0 t0 | E b1 t1 | E db dt                               (phase 2)
+//   wave 2: folds of A | S | B | T, and the sums of a0 | a1
+//   wave 3: m0 b0 | m1 b1 | dm db | fold of m                         (phase 2)
+// and the sixteen waves of the workgroup take 64 pairs at a time; a round of fewer leaves the waves of the others out.  The middle
+// coefficients (da s0 + a0 ds and the like) are a1 s1 - a0 s0 - da ds.
+// What binds: instruction issue of the sixteen waves on one compute unit while a round has 64 pairs, the chain of two products
+// below.  These rounds took 17 us each in a workgroup that gave a pair's products to four lanes, 14 us each as launches.
+static constexpr int RM_ROUNDS = 8, RM_P = 1 << RM_ROUNDS, RM_W = 12, RM_ROWS = 16, RM_GROUPS = 4;      // RM_W: words of an element in LDS (rows of sixteen read without conflicts)
+static constexpr size_t RM_MAX_N = (size_t)1 << 17;      // elements from which on a sumcheck's rounds run in such launches
+struct RoundsArgs {
     const Fr *A, *S, *B, *T, *m, *E;
-    Fr *nA, *nS, *nB, *nT, *nm;
-    Fr* nE;      // the next round's eq table (the top variable summed out), written by task 3; may be null
+    Fr *nA, *nS, *nB, *nT, *nm, *nE;      // nA null: nothing is left after these rounds
+    Fr29 beta, v[RM_ROUNDS];              // v: times 2^261
+    uint32_t nlow, log_c, rounds, phase2_from;      // n = nlow << rounds elements; rounds from phase2_from on are phase-2 rounds
+    uint32_t hadamard;                    // the three sums of two tensors A, S alone (beta = 0), with the factor of k_hadamard_round
+    uint32_t fold_e, e_span;              // fold_e: E is this round's table alone and is summed down from round to round; e_span: its first round's is E[t] + E[t + e_span]
+    uint32_t off[RM_ROUNDS];              // where round r's partial sums start
 };
-__device__ __forceinline__ void lookup_task(Fr (&acc)[3], int task, bool phase2, const LookupPtrs& p, const Fr& beta, const Fr& v_mont, size_t t, size_t n_out) {
-    if (task == 0) {
-        const Fr e = p.E[t];
-        const Fr a0 = p.A[t], a1 = p.A[t + n_out], s0r = p.S[t], s1 = p.S[t + n_out];
-        const Fr da = sub(a1, a0), ds = sub(s1, s0r), s0 = add(s0r, beta);
-        acc[0] = add(acc[0], mont_mul(e, mont_mul(a0, s0)));
-        acc[1] = add(acc[1], mont_mul(e, add(mont_mul(da, s0), mont_mul(a0, ds))));
-        acc[2] = add(acc[2], mont_mul(e, mont_mul(da, ds)));
-    } else if (task == 1) {
-        const Fr e = p.E[t];
-        const Fr b0 = p.B[t], b1 = p.B[t + n_out], t0r = p.T[t], t1 = p.T[t + n_out];
-        const Fr db = sub(b1, b0), dt = sub(t1, t0r), t0 = add(t0r, beta);
-        acc[0] = add(acc[0], mont_mul(e, mont_mul(b0, t0)));
-        acc[1] = add(acc[1], mont_mul(e, add(mont_mul(db, t0), mont_mul(b0, dt))));
-        acc[2] = add(acc[2], mont_mul(e, mont_mul(db, dt)));
-    } else if (task == 2) {
-        const Fr b0 = p.B[t], b1 = p.B[t + n_out], m0 = p.m[t], m1 = p.m[t + n_out];
-        const Fr db = sub(b1, b0), dm = sub(m1, m0);
-        acc[0] = add(acc[0], mont_mul(m0, b0));
-        acc[1] = add(acc[1], add(mont_mul(dm, b0), mont_mul(m0, db)));
-        acc[2] = add(acc[2], mont_mul(dm, db));
-        p.nm[t] = add(m0, mont_mul(v_mont, dm));
-        const Fr a0 = p.A[t], s0 = p.S[t];
-        p.nA[t] = add(a0, mont_mul(v_mont, sub(p.A[t + n_out], a0)));
-        p.nS[t] = add(s0, mont_mul(v_mont, sub(p.S[t + n_out], s0)));
-    } else {
-        if (p.nE && t < n_out / 2) p.nE[t] = add(p.E[t], p.E[t + n_out / 2]);
-        const Fr a0 = p.A[t];
-        const Fr da = sub(p.A[t + n_out], a0);
-        acc[0] = add(acc[0], a0);
-        acc[1] = add(acc[1], da);
-        if (phase2) {
-            const Fr b0 = p.B[t], t0 = p.T[t];
-            p.nB[t] = add(b0, mont_mul(v_mont, sub(p.B[t + n_out], b0)));
-            p.nT[t] = add(t0, mont_mul(v_mont, sub(p.T[t + n_out], t0)));
+template <int CTRL> __device__ __forceinline__ uint32_t dpp_plus(uint32_t x) { return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false); }
+__device__ __forceinline__ void fr29_carry_u(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        l[i + 1] += l[i] >> 29;
+        l[i] &= R29M;
+    }
+}
+// limb-wise sums over the rows of sixteen lanes (every lane of the wave active), in each row's last lane; limbs 0..7 below 2^29
+__device__ __forceinline__ void fr29_row_sum(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x112>(dpp_plus<0x111>(l[i]));      // one, then two lanes to the left
+    fr29_carry_u(l);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x118>(dpp_plus<0x114>(l[i]));      // four, eight
+    fr29_carry_u(l);
+}
+__device__ __forceinline__ void rm_put(int32_t* slot, const Fr29& x) {
+    int4* p = reinterpret_cast<int4*>(slot);
+    p[0] = make_int4(x.l[0], x.l[1], x.l[2], x.l[3]);
+    p[1] = make_int4(x.l[4], x.l[5], x.l[6], x.l[7]);
+    slot[8] = x.l[8];
+}
+__device__ __forceinline__ Fr29 rm_get(const int32_t* slot) {
+    const int4* p = reinterpret_cast<const int4*>(slot);
+    const int4 a = p[0], b = p[1];
+    Fr29 x;
+    x.l[0] = a.x; x.l[1] = a.y; x.l[2] = a.z; x.l[3] = a.w;
+    x.l[4] = b.x; x.l[5] = b.y; x.l[6] = b.z; x.l[7] = b.w;
+    x.l[8] = slot[8];
+    return x;
+}
+__device__ __forceinline__ Fr29 fr29_select(bool c, const Fr29& a, const Fr29& b) {
+    Fr29 r;
+#pragma unroll
+    for (int l = 0; l < 9; ++l) r.l[l] = c ? a.l[l] : b.l[l];
+    return r;
+}
+template <bool PHASE2> __global__ void __launch_bounds__(1024)
+k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
+    constexpr int NT = PHASE2 ? 5 : 2;
+    __shared__ int32_t X0[NT][RM_P][RM_W], X1[NT][RM_P / 2][RM_W], XE[RM_P / 2][RM_W];
+    __shared__ uint32_t raw[RM_ROUNDS][RM_GROUPS][RM_ROWS][9];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave & 3u, group = wave >> 2;
+    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u, T = 1024u;
+    const uint32_t nb = gridDim.x, c = 1u << a.log_c;
+    // neighbouring workgroups read neighbouring elements of the same lines: keep them on one die (workgroups go to the eight dies in turn)
+    const uint32_t blk = (nb & 7u) == 0 ? (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    const uint32_t low0 = blk << a.log_c, P = c << a.rounds;
+    {
+        const uint32_t own = PHASE2 && a.phase2_from < a.rounds ? P >> a.phase2_from : 0u;      // elements of B, T, m
+        const Fr* src[5] = {a.A, a.S, a.B, a.T, a.m};
+        // B, T, m enter with the first phase-2 round, which reads the buffer of its parity
+        for (uint32_t i = threadIdx.x; i < (uint32_t)NT * P; i += T) {
+            const uint32_t k = i / P, s = i % P;
+            if (k >= 2 && s >= own) continue;
+            const size_t g = (size_t)(s >> a.log_c) * a.nlow + low0 + (s & (c - 1));
+            const Fr* p = k == 0 ? src[0] : (k == 1 ? src[1] : (k == 2 ? src[2] : (k == 3 ? src[3] : src[4])));
+            rm_put(k >= 2 && (a.phase2_from & 1u) ? X1[k][s] : X0[k][s], fr29_repack(p[g]));
+        }
+        for (uint32_t s = threadIdx.x; s < P / 2; s += T) {
+            const size_t g = (size_t)(s >> a.log_c) * a.nlow + low0 + (s & (c - 1));
+            Fr e = a.E[g];
+            if (a.e_span) e = add(e, a.E[g + a.e_span]);
+            rm_put(XE[s], fr29_repack(e));
+        }
+        for (uint32_t i = threadIdx.x; i < RM_ROUNDS * RM_GROUPS * RM_ROWS * 9; i += T) (&raw[0][0][0][0])[i] = 0u;
+    }
+    __syncthreads();
+    for (uint32_t r = 0; r < a.rounds; ++r) {
+        const bool odd = (r & 1u) != 0, phase2 = PHASE2 && r >= a.phase2_from;
+        const uint32_t half = P >> (r + 1);
+        int32_t* const src = odd ? &X1[0][0][0] : &X0[0][0][0];
+        int32_t* const dst = odd ? &X0[0][0][0] : &X1[0][0][0];
+        const uint32_t ss = (odd ? RM_P / 2 : RM_P) * RM_W, ds = (odd ? RM_P : RM_P / 2) * RM_W;
+        auto rd = [&](uint32_t k, uint32_t slot) { return rm_get(src + k * ss + slot * RM_W); };
+        if (group * 16u < half && (phase2 || !(kind & 1u))) {
+            uint32_t acc[9];
+#pragma unroll
+            for (int l = 0; l < 9; ++l) acc[l] = 0;
+            for (uint32_t t0 = group * 16u; t0 < half; t0 += 16u * RM_GROUPS) {
+                const uint32_t t = t0 + ln;
+                const bool live = t < half;
+                const uint32_t ta = live ? t : 0u, tb = ta + half;
+                Fr29 x;
+                if (kind < 2) {
+                    const uint32_t kx = kind * 2u;
+                    const Fr29 x0 = rd(kx, ta), x1 = rd(kx, tb), y0 = rd(kx + 1, ta), y1 = rd(kx + 1, tb);
+                    x = fr29_select(row == 0, x0, fr29_select(row == 1, x1, fr29_sub_plus_r(x1, x0)));
+                    const Fr29 y = fr29_select(row < 2, fr29_add(fr29_select(row == 0, y0, y1), a.beta), fr29_sub_plus_r(y1, y0));
+                    x = fr29_mul(rm_get(XE[ta]), fr29_mul(x, y));
+                } else if (kind == 2) {
+                    const Fr29 x0 = rd(PHASE2 ? row : (row & 1u), ta), x1 = rd(PHASE2 ? row : (row & 1u), tb);
+                    const Fr29 f = fr29_canon<2>(fr29_add(x0, fr29_mul(a.v[r], fr29_sub_plus_r(x1, x0))));
+                    if (live && row < (phase2 ? 4u : 2u)) rm_put(dst + row * ds + t * RM_W, f);
+                    x = row == 0 ? x0 : rd(0, tb);
+                } else {
+                    const Fr29 m0 = rd(4, ta), m1 = rd(4, tb), b0 = rd(2, ta), b1 = rd(2, tb), dm = fr29_sub_plus_r(m1, m0);
+                    const Fr29 y = fr29_select(row == 0, b0, fr29_select(row == 1, b1, fr29_select(row == 2, fr29_sub_plus_r(b1, b0), a.v[r])));
+                    x = fr29_mul(fr29_select(row == 0, m0, fr29_select(row == 1, m1, dm)), y);
+                    if (live && row == 3) rm_put(dst + 4 * ds + t * RM_W, fr29_canon<2>(fr29_add(m0, x)));
+                }
+                if (live) {
+#pragma unroll
+                    for (int l = 0; l < 9; ++l) acc[l] += (uint32_t)x.l[l];
+                }
+                fr29_carry_u(acc);
+            }
+            fr29_row_sum(acc);
+            if (ln == 15) {
+#pragma unroll
+                for (int l = 0; l < 9; ++l) raw[r][group][kind * 4u + row][l] = acc[l];
+            }
+        }
+        __syncthreads();
+        if (a.fold_e && r + 1 < a.rounds) {
+            for (uint32_t s = threadIdx.x; s < half / 2; s += T) rm_put(XE[s], fr29_canon<1>(fr29_add(rm_get(XE[s]), rm_get(XE[s + half / 2]))));
+            __syncthreads();
+        }
+    }
+    // the sums with the factors the other round kernels leave on them: a product of two elements carries 2^-261 here, another with E = e 2^256
+    // leaves e x y 2^-266; the sums of E's products are e x y 2^-256 there (k_hadamard_round: no factor), of m b 2^-256, of a alone as they are
+    const uint32_t per = a.hadamard ? 3u : (PHASE2 ? 11u : 5u);
+    for (uint32_t i = threadIdx.x; i < per * a.rounds; i += T) {
+        const uint32_t r = i / per, k = i % per;
+        if (!a.hadamard && k >= 5 && r < a.phase2_from) continue;
+        auto sum = [&](uint32_t role, const Fr29& fix) {
+            uint32_t l9[9];
+#pragma unroll
+            for (int l = 0; l < 9; ++l) l9[l] = raw[r][0][role][l] + raw[r][1][role][l] + raw[r][2][role][l] + raw[r][3][role][l];
+            fr29_carry_u(l9);
+            Fr29 x;
+#pragma unroll
+            for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+            return fr29_canon_pack<5>(fr29_mul(x, fix));
+        };
+        Fr o;
+        if (k == 3 || k == 4) {
+            o = sum(8, fr29_2_261());
+            if (k == 4) o = sub(sum(9, fr29_2_261()), o);
         } else {
-            const Fr s0 = p.S[t];
-            p.nA[t] = add(a0, mont_mul(v_mont, da));
-            p.nS[t] = add(s0, mont_mul(v_mont, sub(p.S[t + n_out], s0)));
+            const uint32_t base = k < 3 ? 0u : (k < 8 ? 4u : 12u), which = k < 3 ? k : (k < 8 ? k - 5 : k - 8);
+            const Fr29 fix = k >= 8 ? fr29_2_266() : (a.hadamard ? fr29_2_527() : fr29_2_271());
+            o = sum(base + (which == 0 ? 0u : (which == 2 ? 2u : 1u)), fix);
+            if (which == 1) o = sub(sub(o, sum(base, fix)), sum(base + 2, fix));
         }
+        partials[(size_t)a.off[r] + (size_t)k * nb + blockIdx.x] = o;
     }
-}
-// where a task's sums go in the 11-value layout of a round, and how many it has
-__device__ __forceinline__ int lookup_task_base(int task) { return task == 0 ? 0 : (task == 1 ? 5 : (task == 2 ? 8 : 3)); }
-__device__ __forceinline__ int lookup_task_count(int task) { return task == 3 ? 2 : 3; }
-
-// One round, one task per blockIdx.y (phase 1: y = 0 -> task 0, y = 1 -> task 3; phase 2: y = task).
-// partials[k * gridDim.x + blockIdx.x] for the sums k the task owns.
-template <bool PHASE2> __global__ void __launch_bounds__(TPB)
-k_lookup_round_split(Fr* __restrict__ partials, const LookupPtrs p, const Fr beta, const Fr v_mont, size_t n_out) {
-    const int task = PHASE2 ? (int)blockIdx.y : (blockIdx.y == 0 ? 0 : 3);
-    Fr acc[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) acc[i] = big_zero<8>();
-    for (size_t t = (size_t)blockIdx.x * TPB + threadIdx.x; t < n_out; t += (size_t)gridDim.x * TPB) lookup_task(acc, task, PHASE2, p, beta, v_mont, t, n_out);
-    if (task == 3) {                      // two sums only: row 5 belongs to task 1
-        Fr a2[2] = {acc[0], acc[1]};
-        block_reduce_store<2>(a2, partials + (size_t)3 * gridDim.x);
-    } else {
-        block_reduce_store<3>(acc, partials + (size_t)lookup_task_base(task) * gridDim.x);
-    }
-}
-
-// All remaining rounds of the lookup sumcheck in one workgroup of four 256-lane groups, one per task.  Round r reads
-// buffer set r & 1 and writes the other (round 0 reads the caller's tensors).  sums[r*11 + i] as k_lookup_round orders
-// them (5 used in phase 1).  Rounds from `phase2_from` on are phase-2 rounds.  w: 2 x 6 x n_out0 elements of work space.
-__global__ void __launch_bounds__(TAIL_T)
-k_lookup_tail(Fr* __restrict__ sums, Fr* w, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E,
-              const Fr beta, const TailV vs, uint32_t n_out0, uint32_t rounds, uint32_t phase2_from) {
-    __shared__ uint32_t red[4 * 3 * 4 * 8];       // task x sum x wave x limb
-    const uint32_t grp = threadIdx.x >> 8, lt = threadIdx.x & 255u, wv = lt >> 6, ln = lt & 63u;
-    LookupPtrs p;
-    p.A = A; p.S = S; p.B = B; p.T = T; p.m = m; p.E = E; p.nE = nullptr;
-    const Fr* cE = E;
-    uint32_t n_out = n_out0;
-    for (uint32_t r = 0; r < rounds; ++r) {
-        const bool phase2 = r >= phase2_from;
-        Fr* ws = w + (size_t)(r & 1u) * 6 * n_out0;
-        p.nA = ws; p.nS = ws + n_out0; p.nB = ws + 2 * (size_t)n_out0; p.nT = ws + 3 * (size_t)n_out0; p.nm = ws + 4 * (size_t)n_out0;
-        Fr* nE = ws + 5 * (size_t)n_out0;
-        p.E = cE;
-        const int task = (int)grp;
-        const bool works = phase2 || task == 0 || task == 3;
-        Fr acc[3];
-#pragma unroll
-        for (int i = 0; i < 3; ++i) acc[i] = big_zero<8>();
-        if (works)
-            for (uint32_t t = lt; t < n_out; t += 256) lookup_task(acc, task, phase2, p, beta, vs.v[r], t, n_out);
-        // the halved eq table for the next round, by the lanes that idle in phase 1 (task 1) or finish early (any)
-        const uint32_t nh = n_out >> 1;
-        if (task == 1)
-            for (uint32_t t = lt; t < nh; t += 256) nE[t] = add(cE[t], cE[t + nh]);
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const Fr s = wave_sum(acc[k]);
-            if (ln == 0) {
-#pragma unroll
-                for (int l = 0; l < 8; ++l) red[((grp * 3 + k) * 4 + wv) * 8 + l] = s.v[l];
-            }
+    if (a.nA) {
+        const int32_t* const fin = (a.rounds & 1u) ? &X1[0][0][0] : &X0[0][0][0];
+        const uint32_t fs = ((a.rounds & 1u) ? RM_P / 2 : RM_P) * RM_W, nt = PHASE2 && a.phase2_from < a.rounds ? 5u : 2u;
+        for (uint32_t i = threadIdx.x; i < nt * c; i += T) {
+            const uint32_t k = i >> a.log_c, s = i & (c - 1);
+            Fr* d = k == 0 ? a.nA : (k == 1 ? a.nS : (k == 2 ? a.nB : (k == 3 ? a.nT : a.nm)));
+            d[low0 + s] = fr29_pack(rm_get(fin + k * fs + s * RM_W));
         }
-        __syncthreads();
-        if (wv == 0 && ln < 3 && (int)ln < lookup_task_count(task) && works) {
-            Fr x = big_zero<8>();
-            for (int q = 0; q < 4; ++q) {
-                Fr y;
-#pragma unroll
-                for (int l = 0; l < 8; ++l) y.v[l] = red[((grp * 3 + ln) * 4 + q) * 8 + l];
-                x = add(x, y);
-            }
-            sums[(size_t)r * 11 + lookup_task_base(task) + ln] = x;
-        }
-        p.A = p.nA; p.S = p.nS;
-        if (phase2) { p.B = p.nB; p.T = p.nT; p.m = p.nm; }
-        cE = nE;
-        n_out = nh;
-        __syncthreads();
+        if (a.fold_e)
+            for (uint32_t s = threadIdx.x; s < c; s += T) a.nE[low0 + s] = fr29_pack(rm_get(XE[s]));
     }
 }
 
@@ -2431,6 +2490,61 @@ static bool limbs29() { static const bool on = [] { const char* e = getenv("ZKLL
 // all rounds of the lookup sumcheck; sums land in job.sums
 // A == nullptr with a hint source: 1 / (S + beta) has not been written anywhere; a large first round computes it on
 // the fly, anything else writes it out first.
+// Queues rounds r .. rounds - 1 of a sumcheck over n elements in launches of k_sum_rounds.  hadamard: two tensors A, S; else a lookup whose
+// phase-2 rounds start at round n1.  The rounds' partial sums go behind part_at and are noted in `fin`; eq_prefix: every round reads E's prefix.
+static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& beta, const uint32_t* v, size_t n, int r,
+                        int rounds, int n1, bool eq_prefix, Fr* part_all, size_t& part_at, FinishRounds& fin) {
+    const uint32_t per1 = hadamard ? 3u : 5u;
+    uint32_t e_span = 0;
+    while (r < rounds) {
+        // While there are more workgroups than compute units a launch is throughput, and a round of few pairs a workgroup costs as much as
+        // a full one: three rounds then; all that the workgroup's elements allow, evenly split over the launches, where each has a unit
+        // of its own.
+        const int left = rounds - r;
+        int R = std::min(3, left);
+        if (n <= (size_t)256 * RM_P) {
+            const int launches = (left + RM_ROUNDS - 1) / RM_ROUNDS;
+            R = (left + launches - 1) / launches;
+        }
+        RoundsArgs a;
+        memset(&a, 0, sizeof(a));
+        a.rounds = (uint32_t)R;
+        a.nlow = (uint32_t)(n >> R);
+        while (((size_t)2 << (a.log_c + R)) <= (size_t)RM_P && (2u << a.log_c) <= a.nlow) ++a.log_c;
+        const uint32_t nb = a.nlow >> a.log_c;
+        a.A = A; a.S = S; a.B = B; a.T = T; a.m = m; a.E = E;
+        a.beta = fr29_repack(beta);
+        a.phase2_from = hadamard ? (uint32_t)R : (uint32_t)std::min(std::max(n1 - r, 0), R);
+        a.hadamard = hadamard ? 1u : 0u;
+        a.fold_e = eq_prefix ? 0u : 1u;
+        a.e_span = e_span;
+        const bool phase2 = a.phase2_from < a.rounds;
+        for (int q = 0; q < R; ++q) {
+            a.v[q] = fr29_repack(mont_mul(to_mont(load_fr(v + 8 * (size_t)(r + q))), fr29_pack(fr29_2_261())));
+            const uint32_t k = (uint32_t)q >= a.phase2_from ? 11u : per1;
+            a.off[q] = (uint32_t)part_at;
+            fin.off[r + q] = (uint32_t)part_at; fin.nb[r + q] = nb; fin.k[r + q] = (uint8_t)k;
+            part_at += (size_t)k * nb;
+        }
+        if (r + R < rounds) {
+            const size_t o = a.nlow;
+            Scratch& nx = job.arena.add(sizeof(Fr) * o * 6);
+            if (nx.rc) return nx.rc;
+            a.nA = nx.as<Fr>(); a.nS = a.nA + o; a.nB = a.nS + o; a.nT = a.nB + o; a.nm = a.nT + o; a.nE = a.nm + o;
+        }
+        if (phase2) hipLaunchKernelGGL(k_sum_rounds<true>, dim3(nb), dim3(1024), 0, job.st, part_all, a);
+        else hipLaunchKernelGGL(k_sum_rounds<false>, dim3(nb), dim3(1024), 0, job.st, part_all, a);
+        ZK_LAUNCH_CHECK();
+        A = a.nA; S = a.nS;
+        if (phase2) { B = a.nB; T = a.nT; m = a.nm; }
+        if (!eq_prefix) { E = a.nE; e_span = a.nlow >> 1; }
+        n = a.nlow;
+        r += R;
+    }
+    return 0;
+}
+// partial sums that rounds_queue may need for the rounds of n elements: a workgroup holds 128 pairs of a launch's first round where there are as many
+static size_t rounds_partials(size_t n, int rounds, uint32_t k) { return (size_t)rounds * k * (n / RM_P + 1); }
 static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& b, const uint32_t* v, size_t D, size_t N, int rounds,
                         const HintSrc* hs = nullptr) {
     hipStream_t st = job.st;
@@ -2464,7 +2578,11 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
     size_t part_total = 0;
     {
         size_t c = D;
-        for (int r = 0; r < rounds; ++r) { c >>= 1; part_total += 11 * (size_t)reduce_grid(c); }
+        for (int r = 0; r < rounds; ++r) {
+            c >>= 1;
+            part_total += 11 * (size_t)reduce_grid(c);
+        }
+        part_total += rounds_partials(std::min(D, RM_MAX_N), rounds, 11);
     }
     Scratch& part_all = job.arena.add(sizeof(Fr) * part_total);
     if (sums.rc) return sums.rc;
@@ -2484,16 +2602,10 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         const size_t half = cur >> 1;
         const bool phase2 = r >= n1;
         part.p = part_all.as<Fr>() + part_at;
-        if (half <= (size_t)TAIL_HALF && rounds - r <= TAIL_ROUNDS) {
-            const int rest = rounds - r;
-            Scratch& work = job.arena.add(sizeof(Fr) * 12 * half);
-            if (work.rc) return work.rc;
-            TailV vs;
-            for (int i = 0; i < TAIL_ROUNDS; ++i) vs.v[i] = i < rest ? to_mont(load_fr(v + 8 * (r + i))) : big_zero<8>();
-            hipLaunchKernelGGL(k_lookup_tail, dim3(1), dim3(TAIL_T), 0, st, sums.as<Fr>() + (size_t)r * 11, work.as<Fr>(), cA, cS, cB, cT, cm, cE, b, vs, (uint32_t)half,
-                               (uint32_t)rest, (uint32_t)(phase2 ? 0 : n1 - r));
-            ZK_LAUNCH_CHECK();
-            job.tail_from = r;
+        if (cA && cur <= RM_MAX_N) {
+            int rc = rounds_queue(job, false, cA, cS, cB, cT, cm, cE, b, v, cur, r, rounds, n1, eq_prefix, part_all.as<Fr>(), part_at, fin);
+            if (rc) return rc;
+            fin_rounds = rounds;
             break;
         }
         if (r == 0 && !phase2 && fuse_first && hs->hint_ints && limbs29() && two_rounds_on() && n1 >= 2 && rounds >= 2 && (half >> 1) > (size_t)SPLIT_HALF &&
@@ -2552,7 +2664,7 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         // pairs cost -- so a one-lane-per-pair round with a pair or two per lane pays it per pair.  Those rounds (not the first, whose
         // grid the fused passes choose) take fewer lanes: eight pairs a lane in phase 1, four in phase 2, where the round has them.
         unsigned nb = reduce_grid(half);
-        if (half > (size_t)SPLIT_HALF && !(r == 0 && fuse_first)) nb = round_grid(half, phase2 ? 4 : 8);
+        if (!(r == 0 && fuse_first)) nb = round_grid(half, phase2 ? 4 : 8);
         const Fr vm = to_mont(load_fr(v + 8 * r));
         // the next round's eq table is written by this round's kernel (ping-pong between two buffers of the job)
         Fr* nE = nullptr;
@@ -2566,14 +2678,7 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
             }
             nE = eqbuf[r & 1];
         }
-        if (half <= (size_t)SPLIT_HALF) {
-            // short round: four lanes per pair (two in phase 1), one task per grid row
-            LookupPtrs lp;
-            lp.A = cA; lp.S = cS; lp.B = cB; lp.T = cT; lp.m = cm; lp.E = cE; lp.nE = nE;
-            lp.nA = w; lp.nS = w + half; lp.nB = w + 2 * half; lp.nT = w + 3 * half; lp.nm = w + 4 * half;
-            if (phase2) hipLaunchKernelGGL(k_lookup_round_split<true>, dim3(nb, 4), dim3(TPB), 0, st, part.as<Fr>(), lp, b, vm, half);
-            else hipLaunchKernelGGL(k_lookup_round_split<false>, dim3(nb, 2), dim3(TPB), 0, st, part.as<Fr>(), lp, b, vm, half);
-        } else if (phase2)
+        if (phase2)
             hipLaunchKernelGGL((k_lookup_round<true, false>), dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, w + 2 * half, w + 3 * half, w + 4 * half, cA, cS, cB, cT, cm, cE, b, vm, half, nE,
                                HintSrc());
         else if (r == 0 && fuse_first) {
@@ -2648,6 +2753,7 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
     {
         size_t c = N;
         for (int r = 0; r < rounds; ++r) { c >>= 1; part_total += (size_t)(K + 1) * reduce_grid(c); }
+        part_total += rounds_partials(std::min(N, RM_MAX_N), rounds, (uint32_t)(K + 1));
     }
     Scratch& part_all = job.arena.add(sizeof(Fr) * part_total);
     if (sums.rc) return sums.rc;
@@ -2666,6 +2772,13 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
     for (int r = 0; r < rounds; ++r) {
         const size_t half = n >> 1;
         part.p = part_all.as<Fr>() + part_at;
+        // two tensors: all short rounds in a few launches (a first round over int32 forms is a round of its own)
+        if (K == 2 && n <= RM_MAX_N && !(r == 0 && ints && ints[0] && ints[1] && half > (size_t)TAIL_HALF)) {
+            int rc = rounds_queue(job, true, cur[0], cur[1], nullptr, nullptr, nullptr, cE, big_zero<8>(), v, n, r, rounds, 0, !job.eq_scale.empty(), part_all.as<Fr>(), part_at, fin);
+            if (rc) return rc;
+            fin_rounds = rounds;
+            break;
+        }
         if (half <= (size_t)TAIL_HALF && rounds - r <= TAIL_ROUNDS) {
             const int rest = rounds - r;
             Scratch& work = job.arena.add(sizeof(Fr) * (K + 1) * half);
@@ -2681,7 +2794,7 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
         hipLaunchKernelGGL(k_hadamard_tail<KK>, dim3(1), dim3(TAIL_T), 0, st, so, p, w + (size_t)KK * half, cE, vs, (uint32_t)half, (uint32_t)rest); \
         break;                                                                                                                              \
     }
-            switch (K) { HADS_TAIL(1) HADS_TAIL(2) HADS_TAIL(3) HADS_TAIL(4) }
+            switch (K) { HADS_TAIL(1) HADS_TAIL(3) HADS_TAIL(4) }
 #undef HADS_TAIL
             ZK_LAUNCH_CHECK();
             job.tail_from = r;
