@@ -46,34 +46,68 @@ __device__ __forceinline__ void st_stream(Fr* p, const Fr& x) {
     __builtin_nontemporal_store(b, (u32x4*)p + 1);
 }
 
-// ---- block reduction helper (K sums per thread) -------------------------------------------------------
-template <int K> __device__ __forceinline__ void block_reduce_store(Fr (&acc)[K], Fr* __restrict__ partials) {
-    __shared__ uint32_t red[8][TPB];
+// ---- sums over lanes ----------------------------------------------------------------------------------
+template <int CTRL, int ROWS = 0xF> __device__ __forceinline__ uint32_t dpp_plus(uint32_t x) {
+    return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ void fr29_carry_u(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        l[i + 1] += l[i] >> 29;
+        l[i] &= R29M;
+    }
+}
+// limb-wise sums over the rows of sixteen lanes (every lane of the wave active), in each row's last lane; limbs 0..7 below 2^29
+__device__ __forceinline__ void fr29_row_sum(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x112>(dpp_plus<0x111>(l[i]));      // one, then two lanes to the left
+    fr29_carry_u(l);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x118>(dpp_plus<0x114>(l[i]));      // four, eight
+    fr29_carry_u(l);
+}
+// and over the wave, in its last lane
+__device__ __forceinline__ void fr29_wave_sum(uint32_t (&l)[9]) {
+    fr29_row_sum(l);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x143, 0xC>(dpp_plus<0x142, 0xA>(l[i]));      // row 0 into 1, 2 into 3, then the lower half into the upper
+    fr29_carry_u(l);
+}
+// K sums (the first `keep` of them) over a workgroup's TPB lanes, each lane's values canonical: limb sums by data-parallel adds, no
+// barrier but one (a tree through LDS has eight a sum: 10 us for the five of a lookup round, 4 us this way)
+template <int K> __device__ __forceinline__ void block_reduce_store(Fr (&acc)[K], Fr* __restrict__ partials, uint32_t keep = K) {
+    constexpr int W = TPB / 64;
+    __shared__ uint32_t red[W][K][9];
     const uint32_t t = threadIdx.x;
 #pragma unroll
     for (int k = 0; k < K; ++k) {
+        const Fr29 x = fr29_repack(acc[k]);
+        uint32_t l[9];
 #pragma unroll
-        for (int l = 0; l < 8; ++l) red[l][t] = acc[k].v[l];
-        __syncthreads();
-        for (uint32_t s = TPB / 2; s > 0; s >>= 1) {
-            if (t < s) {
-                Fr x, y;
+        for (int i = 0; i < 9; ++i) l[i] = (uint32_t)x.l[i];
+        fr29_wave_sum(l);
+        if ((t & 63u) == 63u) {
 #pragma unroll
-                for (int l = 0; l < 8; ++l) { x.v[l] = red[l][t]; y.v[l] = red[l][t + s]; }
-                x = add(x, y);
-#pragma unroll
-                for (int l = 0; l < 8; ++l) red[l][t] = x.v[l];
-            }
-            __syncthreads();
+            for (int i = 0; i < 9; ++i) red[t >> 6][k][i] = l[i];
         }
-        if (t == 0) {
-            Fr x;
-#pragma unroll
-            for (int l = 0; l < 8; ++l) x.v[l] = red[l][0];
-            partials[(size_t)k * gridDim.x + blockIdx.x] = x;
-        }
-        __syncthreads();
     }
+    __syncthreads();
+    if (t < keep) {
+        uint32_t l[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            l[i] = red[0][t][i];
+#pragma unroll
+            for (int w = 1; w < W; ++w) l[i] += red[w][t][i];
+        }
+        fr29_carry_u(l);
+        Fr29 x;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) x.l[i] = (int32_t)l[i];
+        // up to 256 r: a product with 2^261 leaves the residue below 5 r
+        partials[(size_t)t * gridDim.x + blockIdx.x] = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));
+    }
+    __syncthreads();
 }
 __global__ void __launch_bounds__(TPB) k_finish(Fr* __restrict__ out, const Fr* __restrict__ partials, uint32_t nb) {
     Fr acc[1] = {big_zero<8>()};
@@ -644,18 +678,28 @@ __device__ __forceinline__ Fr sum9_residue(const uint32_t (&acc)[9]) {
 // as E 2^256: e a0 and e da come out as E a0 / 32 and E da / 32, the three sums of products are kept unreduced (Wide29),
 // reduced once per lane (another 2^-261) and brought to the factor 2^-256 of the other kernel by one product with 2^271.
 // At most 256 pairs per lane (the unreduced sums hold 2^522): the launch site checks.
-__global__ void __launch_bounds__(TPB) k_lookup_round29(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ nS, const Fr* __restrict__ A, const Fr* __restrict__ S,
-                                                        const Fr* __restrict__ E, const Fr beta, const Fr v_mont, size_t n_out, Fr* __restrict__ nE) {
+// A phase-2 round is three such passes side by side (blockIdx.y): 0 as above; 1 over B and T; 2 over m and B with the weight one and
+// beta zero (the sums of the products of m and B; of a pass but the first only its three sums of products are kept).  A lane that
+// did all of a pair would need nine unreduced sums, more registers than there are; B and E are read twice instead.
+struct Round29Ptrs { const Fr *A, *S, *B, *T, *m; Fr *nA, *nS, *nB, *nT, *nm; };
+__global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(2, 2))) k_lookup_round29(Fr* __restrict__ partials, const Round29Ptrs p, const Fr* __restrict__ E, const Fr beta, const Fr v_mont, size_t n_out,
+                                                        Fr* __restrict__ nE) {
+    const uint32_t pass = blockIdx.y;
+    const Fr* __restrict__ A = pass == 0 ? p.A : (pass == 1 ? p.B : p.m);
+    const Fr* __restrict__ S = pass == 0 ? p.S : (pass == 1 ? p.T : p.B);
+    Fr* __restrict__ nA = pass == 0 ? p.nA : (pass == 1 ? p.nB : p.nm);
+    Fr* __restrict__ nS = pass == 0 ? p.nS : p.nT;
     const Fr29 vq = fr29_mul(fr29_repack(v_mont), fr29_2_266());      // v 2^261
-    const Fr29 b29 = fr29_repack(beta);
+    const Fr29 b29 = fr29_repack(pass == 2 ? big_zero<8>() : beta);
     Wide29 w0 = wide29_zero(), w2 = wide29_zero(), wx = wide29_zero();
     uint32_t sa0[9], sa1[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) sa0[i] = sa1[i] = 0;
     uint32_t it = 0;
     for (size_t t = (size_t)blockIdx.x * TPB + threadIdx.x; t < n_out; t += (size_t)gridDim.x * TPB) {
-        const Fr e = E[t];
-        if (nE && t < n_out / 2) nE[t] = add(e, E[t + n_out / 2]);      // the next round's table: the top variable summed out
+        Fr e = big_one_mont<8>();
+        if (pass != 2) e = E[t];
+        if (nE && pass == 0 && t < n_out / 2) nE[t] = add(e, E[t + n_out / 2]);      // the next round's table: the top variable summed out
         const Fr a0w = A[t], a1w = A[t + n_out], s0w = S[t], s1w = S[t + n_out];
         sum9_add(sa0, a0w);
         sum9_add(sa1, a1w);
@@ -668,7 +712,7 @@ __global__ void __launch_bounds__(TPB) k_lookup_round29(Fr* __restrict__ partial
         wide29_mac(wx, fr29_add(ea0, eda), fr29_add(s0, ds));
         if ((++it & 3u) == 0u) { wide29_carry(w0); wide29_carry(w2); wide29_carry(wx); }
         nA[t] = fr29_canon_pack(fr29_add(a0, fr29_mul(vq, da)));
-        nS[t] = fr29_canon_pack(fr29_add(s0r, fr29_mul(vq, ds)));
+        if (pass != 2) nS[t] = fr29_canon_pack(fr29_add(s0r, fr29_mul(vq, ds)));
     }
     Fr acc[5];
     const Fr29 fix = fr29_2_271();
@@ -677,7 +721,7 @@ __global__ void __launch_bounds__(TPB) k_lookup_round29(Fr* __restrict__ partial
     acc[1] = sub(sub(fr29_canon_pack(fr29_mul(wide29_redc(wx), fix)), acc[0]), acc[2]);
     acc[3] = sum9_residue(sa0);
     acc[4] = sub(sum9_residue(sa1), acc[3]);
-    block_reduce_store<5>(acc, partials);
+    block_reduce_store<5>(acc, partials + (size_t)(pass == 0 ? 0 : (pass == 1 ? 5 : 8)) * gridDim.x, pass == 0 ? 5u : 3u);
 }
 
 // k_lookup_round<false, true> for queries given by their int32 forms (HintSrc::hint_ints), with the arithmetic of the common
@@ -1210,23 +1254,6 @@ struct RoundsArgs {
     uint32_t fold_e, e_span;              // fold_e: E is this round's table alone and is summed down from round to round; e_span: its first round's is E[t] + E[t + e_span]
     uint32_t off[RM_ROUNDS];              // where round r's partial sums start
 };
-template <int CTRL> __device__ __forceinline__ uint32_t dpp_plus(uint32_t x) { return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, false); }
-__device__ __forceinline__ void fr29_carry_u(uint32_t (&l)[9]) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        l[i + 1] += l[i] >> 29;
-        l[i] &= R29M;
-    }
-}
-// limb-wise sums over the rows of sixteen lanes (every lane of the wave active), in each row's last lane; limbs 0..7 below 2^29
-__device__ __forceinline__ void fr29_row_sum(uint32_t (&l)[9]) {
-#pragma unroll
-    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x112>(dpp_plus<0x111>(l[i]));      // one, then two lanes to the left
-    fr29_carry_u(l);
-#pragma unroll
-    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x118>(dpp_plus<0x114>(l[i]));      // four, eight
-    fr29_carry_u(l);
-}
 __device__ __forceinline__ void rm_put(int32_t* slot, const Fr29& x) {
     int4* p = reinterpret_cast<int4*>(slot);
     p[0] = make_int4(x.l[0], x.l[1], x.l[2], x.l[3]);
@@ -2678,7 +2705,10 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
             }
             nE = eqbuf[r & 1];
         }
-        if (phase2)
+        const Round29Ptrs rp{cA, cS, cB, cT, cm, w, w + half, w + 2 * half, w + 3 * half, w + 4 * half};
+        if (phase2 && limbs29() && half <= (size_t)256 * nb * TPB)
+            hipLaunchKernelGGL(k_lookup_round29, dim3(nb, 3), dim3(TPB), 0, st, part.as<Fr>(), rp, cE, b, vm, half, nE);
+        else if (phase2)
             hipLaunchKernelGGL((k_lookup_round<true, false>), dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, w + 2 * half, w + 3 * half, w + 4 * half, cA, cS, cB, cT, cm, cE, b, vm, half, nE,
                                HintSrc());
         else if (r == 0 && fuse_first) {
@@ -2713,7 +2743,7 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
                 ZK_HIP(hipEventRecord(t0, st));
             }
             if (limbs29() && half <= (size_t)256 * nb * TPB)       // 29-bit limbs inside the kernel; its unreduced sums hold 256 pairs per lane
-                hipLaunchKernelGGL(k_lookup_round29, dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, cA, cS, cE, b, vm, half, nE);
+                hipLaunchKernelGGL(k_lookup_round29, dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), rp, cE, b, vm, half, nE);
             else
                 hipLaunchKernelGGL((k_lookup_round<false, false>), dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, (Fr*)nullptr, (Fr*)nullptr, (Fr*)nullptr, cA, cS, (const Fr*)nullptr,
                                    (const Fr*)nullptr, (const Fr*)nullptr, cE, b, vm, half, nE, HintSrc());
