@@ -3,12 +3,14 @@
 #include <cstdio>
 #include <cstdlib>
 
+#include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <deque>
 #include <functional>
 #include <optional>
 #include <random>
+#include <thread>
 
 #include "../../include/zkllm_hip.h"
 
@@ -678,11 +680,48 @@ FrTensor llama_layer(const LayerConfig& c, const LayerWeights& w, const FrTensor
 
 static LayerSetupTimes g_setup_times;
 const LayerSetupTimes& layer_setup_times() { return g_setup_times; }
+// out[i] = the nearest integer to scale * N(0, std), what std::normal_distribution<double> draws one after the other (Marsaglia's polar
+// method on 53-bit uniforms of one generator output each).  The generator is serial; the logarithms and roots, three quarters of
+// the time, go to several threads.
+static void normal_ints(std::mt19937_64& rng, std::vector<int>& out, double std_dev, double scale) {
+    struct Pair { double x, y, r2; };
+    const size_t n = out.size(), pairs = (n + 1) / 2;
+    std::vector<Pair> p(pairs);
+    auto uniform = [&] {
+        const double v = (double)rng() / 18446744073709551616.0;
+        return v >= 1.0 ? std::nextafter(1.0, 0.0) : v;
+    };
+    const size_t parts = std::max<size_t>(1, std::min<size_t>({8, std::thread::hardware_concurrency(), pairs >> 14}));
+    std::vector<std::thread> workers;
+    auto convert = [&out, &p, n, std_dev, scale](size_t from, size_t to) {
+        for (size_t i = from; i < to; ++i) {
+            const double mult = std::sqrt(-2 * std::log(p[i].r2) / p[i].r2);
+            out[2 * i] = (int)std::nearbyint((p[i].y * mult * std_dev + 0.0) * scale);
+            if (2 * i + 1 < n) out[2 * i + 1] = (int)std::nearbyint((p[i].x * mult * std_dev + 0.0) * scale);
+        }
+    };
+    size_t from = 0;
+    for (size_t q = 0; q < parts; ++q) {
+        const size_t to = pairs * (q + 1) / parts;
+        for (size_t i = from; i < to; ++i) {
+            Pair& a = p[i];
+            do {
+                a.x = 2.0 * uniform() - 1.0;
+                a.y = 2.0 * uniform() - 1.0;
+                a.r2 = a.x * a.x + a.y * a.y;
+            } while (a.r2 > 1.0 || a.r2 == 0.0);
+        }
+        if (q + 1 < parts) workers.emplace_back(convert, from, to);
+        else convert(from, to);
+        from = to;
+    }
+    for (std::thread& t : workers) t.join();
+}
 static Weight random_weight(std::mt19937_64& rng, uint in_dim, uint out_dim, uint pp_size, bool norm, size_t table_budget) {
     const double t0 = now_ms();
-    std::normal_distribution<double> nd(0.0, 0.02);
     std::vector<int> wi((size_t)in_dim * out_dim);
-    for (auto& x : wi) x = norm ? 65536 : (int)std::nearbyint(nd(rng) * 65536.0);   // scale 2^16 (llama-commit.py:34)
+    if (norm) std::fill(wi.begin(), wi.end(), 65536);
+    else normal_ints(rng, wi, 0.02, 65536.0);          // scale 2^16 (llama-commit.py:34)
     FrTensor weight((uint)wi.size(), wi.data());
     if (!norm) weight.keep_as_matmul_rhs();        // the right operand of the layer's projections, run after run
     weight.keep_for_folds();                       // and folded at a new point by every proof and every opening
