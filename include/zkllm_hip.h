@@ -134,6 +134,7 @@ int zk_fr_dot(uint32_t* out_host, const void* a, const void* b, size_t n, void* 
 /* 1..3 levels of Fr_multi_dim_partial_me_step / Fr_me_step / Fr_partial_me_step in one pass over
  * in[other][cur][window] (fr-tensor.cu:518-560, :588-641).  u: `levels` standard-form challenges. */
 int zk_fr_fold_axis(void* out, const void* in, const uint32_t* u, int levels, size_t other, uint32_t cur, size_t window, void* stream);
+int zk_fr_fold_axis_all(void* out, const void* in, const uint32_t* u, int levels, size_t other, uint32_t cur, size_t window, void* stream);      /* out: other * ceil(cur / 2^levels) * window elements */
 /* A tensor that is folded again and again at new points and never changes (a layer's weight: the multilinear evaluations
  * of zkFC::prove, zkfc.cu:77-78, and the fold over the committed rows at the head of Commitment::me_open, commitment.cu:
  * 118-123), examined once: when every element is a 32-bit signed integer (fixed-point weights are) the handle keeps the int32

@@ -254,4 +254,57 @@ ZK_HD Fr29 wide29_redc(Wide29& w) {
     return fr29_redc<18>([&](int k) { return (int64_t)w.c[k]; });
 }
 
+#if defined(__HIPCC__)
+// ---- sums over lanes -----------------------------------------------------------------------------------------------------
+template <int CTRL, int ROWS = 0xF> __device__ __forceinline__ uint32_t dpp_plus(uint32_t x) {
+    return x + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ void fr29_carry_u(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        l[i + 1] += l[i] >> 29;
+        l[i] &= R29M;
+    }
+}
+// limb-wise sums over the rows of sixteen lanes (every lane of the wave active), in each row's last lane; limbs 0..7 below 2^29
+__device__ __forceinline__ void fr29_row_sum(uint32_t (&l)[9]) {
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x112>(dpp_plus<0x111>(l[i]));      // one, then two lanes to the left
+    fr29_carry_u(l);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x118>(dpp_plus<0x114>(l[i]));      // four, eight
+    fr29_carry_u(l);
+}
+// and over the wave, in its last lane
+__device__ __forceinline__ void fr29_wave_sum(uint32_t (&l)[9]) {
+    fr29_row_sum(l);
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x143, 0xC>(dpp_plus<0x142, 0xA>(l[i]));      // row 0 into 1, 2 into 3, then the lower half into the upper
+    fr29_carry_u(l);
+}
+
+// ---- elements in LDS: twelve words each, so that rows of sixteen lanes read without bank conflicts ------------------------
+__device__ __forceinline__ void rm_put(int32_t* slot, const Fr29& x) {
+    int4* p = reinterpret_cast<int4*>(slot);
+    p[0] = make_int4(x.l[0], x.l[1], x.l[2], x.l[3]);
+    p[1] = make_int4(x.l[4], x.l[5], x.l[6], x.l[7]);
+    slot[8] = x.l[8];
+}
+__device__ __forceinline__ Fr29 rm_get(const int32_t* slot) {
+    const int4* p = reinterpret_cast<const int4*>(slot);
+    const int4 a = p[0], b = p[1];
+    Fr29 x;
+    x.l[0] = a.x; x.l[1] = a.y; x.l[2] = a.z; x.l[3] = a.w;
+    x.l[4] = b.x; x.l[5] = b.y; x.l[6] = b.z; x.l[7] = b.w;
+    x.l[8] = slot[8];
+    return x;
+}
+__device__ __forceinline__ Fr29 fr29_select(bool c, const Fr29& a, const Fr29& b) {
+    Fr29 r;
+#pragma unroll
+    for (int l = 0; l < 9; ++l) r.l[l] = c ? a.l[l] : b.l[l];
+    return r;
+}
+#endif
+
 }  // namespace zk

@@ -7,9 +7,11 @@
 //    product with them costs one Montgomery multiplication instead of two;
 //  * sums of products are accumulated with the R^-1 factor still attached and corrected once;
 //  * folds run several levels per pass (registers) and finish in one workgroup (LDS).
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include "field.hpp"
+#include "fr29.hpp"
 #include "rt.hpp"
 #include "../../include/zkllm_hip.h"
 
@@ -265,6 +267,122 @@ k_fold_axis_dot(Fr* __restrict__ out, const Fr* __restrict__ in, const FrPack<(1
     out[g] = acc;
 }
 
+// ---- a whole axis in one pass ----------------------------------------------------------------------------------------------------
+// Every level of a long axis at once: out = sum_j eq(u, j) in[j].  The weights are a table (k_eq29), a product with one is only
+// summed (Wide29: 81 multiply-adds in 29-bit limbs, one reduction a lane), so the tensor is read once, nothing is written but the
+// result, and a wave's loads run along memory whichever axis it is.  Three levels a pass (k_fold_axis_dot) read 1 1/7 times the tensor
+// and, along the innermost axis, eight elements a lane at 256-byte strides.
+static constexpr int EQ29_MAX = 14;          // levels: three factors of at most five bits
+struct Eq29Tabs { Fr29 t[96]; };             // 32 entries for each factor, with the factor 2^261
+// entry i < n of the eq table with factor 2^261, canonical; SOA: limb l at out[l n + i], else at out[9 i + l]
+template <bool SOA> __global__ void __launch_bounds__(TPB) k_eq29(int32_t* __restrict__ out, const Eq29Tabs tabs, uint32_t n, int b0, int b1) {
+    const uint32_t i = blockIdx.x * TPB + threadIdx.x;
+    if (i >= n) return;
+    const Fr29 e = fr29_canon<2>(fr29_mul(fr29_mul(tabs.t[i & ((1u << b0) - 1u)], tabs.t[32 + ((i >> b0) & ((1u << b1) - 1u))]), tabs.t[64 + (i >> (b0 + b1))]));
+#pragma unroll
+    for (int l = 0; l < 9; ++l) out[SOA ? (size_t)l * n + i : (size_t)i * 9 + l] = e.l[l];
+}
+// innermost axis: out[row] = sum_p E[p] in[row][p].  WPR waves take two rows (an entry of the table serves both), 64 terms a lane at most
+template <int WPR> __global__ void __launch_bounds__(TPB)
+k_fold_rows(Fr* __restrict__ out, const Fr* __restrict__ in, const int32_t* __restrict__ E, size_t rows, uint32_t cur) {
+    __shared__ uint32_t red[2][4][9];
+    const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const size_t r0 = ((size_t)blockIdx.x * (4 / WPR) + wave / WPR) * 2;
+    const size_t ra = r0 < rows ? r0 : rows - 1, rb = r0 + 1 < rows ? r0 + 1 : rows - 1;
+    const Fr *pa = in + ra * cur, *pb = in + rb * cur;
+    Wide29 wa = wide29_zero(), wb = wide29_zero();
+    uint32_t p = (wave % WPR) * 64u + lane, term = 0;
+    Fr xa = big_zero<8>(), xb = xa;
+    Fr29 e = fr29_zero();
+    auto fetch = [&](uint32_t q) {
+        xa = pa[q]; xb = pb[q];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)l * cur + q];
+    };
+    if (p < cur) fetch(p);
+    while (p < cur) {
+        const Fr29 a = fr29_repack(xa), b = fr29_repack(xb), ce = e;
+        p += 64u * WPR;
+        if (p < cur) fetch(p);
+        wide29_mac(wa, ce, a);
+        wide29_mac(wb, ce, b);
+        if ((++term & 3u) == 0) { wide29_carry(wa); wide29_carry(wb); }
+    }
+    uint32_t l9[2][9];
+    const Fr29 sa = fr29_canon<2>(wide29_redc(wa)), sb = fr29_canon<2>(wide29_redc(wb));
+#pragma unroll
+    for (int l = 0; l < 9; ++l) { l9[0][l] = (uint32_t)sa.l[l]; l9[1][l] = (uint32_t)sb.l[l]; }
+    fr29_wave_sum(l9[0]);
+    fr29_wave_sum(l9[1]);
+    if (lane == 63u) {
+#pragma unroll
+        for (int l = 0; l < 9; ++l) { red[0][wave][l] = l9[0][l]; red[1][wave][l] = l9[1][l]; }
+    }
+    __syncthreads();
+    if (threadIdx.x < 8 / WPR) {
+        const uint32_t k = threadIdx.x & 1u, g = threadIdx.x >> 1;
+        const size_t row = ((size_t)blockIdx.x * (4 / WPR) + g) * 2 + k;
+        uint32_t s[9];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) {
+            s[l] = red[k][g * WPR][l];
+#pragma unroll
+            for (int w = 1; w < WPR; ++w) s[l] += red[k][g * WPR + w][l];
+        }
+        fr29_carry_u(s);
+        Fr29 x;
+#pragma unroll
+        for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)s[l];
+        if (row < rows) out[row] = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));
+    }
+}
+// a middle axis: out[z][w] = sum_j E[j] in[z][j][w].  A lane takes one w and J consecutive j (the table's entry is the same for the
+// whole wave), the four waves of a workgroup 4 J of them; grid (w in groups of 64, 4 J at a time, z)
+__global__ void __launch_bounds__(TPB)
+k_fold_cols(Fr* __restrict__ part, const Fr* __restrict__ in, const int32_t* __restrict__ E, uint32_t cur, size_t window, uint32_t J) {
+    __shared__ uint32_t red[3][9][64];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
+    const size_t w = (size_t)blockIdx.x * 64 + lane, wc = w < window ? w : window - 1;
+    const uint32_t j0 = (blockIdx.y * 4 + wave) * J, j1 = j0 + J < cur ? j0 + J : cur;
+    const Fr* base = in + (size_t)blockIdx.z * cur * window + wc;
+    Wide29 acc = wide29_zero();
+    for (uint32_t j = j0; j < j1; j += 4) {
+        Fr x[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = base[(size_t)(j + q < j1 ? j + q : j) * window];
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (j + q < j1) {
+                Fr29 e;
+#pragma unroll
+                for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)(j + q) * 9 + l];
+                wide29_mac(acc, e, fr29_repack(x[q]));
+            }
+        wide29_carry(acc);
+    }
+    Fr29 s = wide29_redc(acc);
+    if (wave) {
+#pragma unroll
+        for (int l = 0; l < 9; ++l) red[wave - 1][l][lane] = (uint32_t)s.l[l];
+    }
+    __syncthreads();
+    if (wave) return;
+    uint32_t l9[9];
+#pragma unroll
+    for (int l = 0; l < 9; ++l) l9[l] = (uint32_t)s.l[l] + red[0][l][lane] + red[1][l][lane] + red[2][l][lane];
+    fr29_carry_u(l9);
+#pragma unroll
+    for (int l = 0; l < 9; ++l) s.l[l] = (int32_t)l9[l];
+    if (w < window) part[((size_t)blockIdx.y * gridDim.z + blockIdx.z) * window + w] = fr29_canon_pack<2>(fr29_mul(s, fr29_2_261()));
+}
+__global__ void __launch_bounds__(TPB) k_sum_partials(Fr* __restrict__ out, const Fr* __restrict__ part, size_t n, uint32_t count) {
+    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (i >= n) return;
+    Fr s = part[i];
+    for (uint32_t c = 1; c < count; ++c) s = add(s, part[(size_t)c * n + i]);
+    out[i] = s;
+}
+
 // Finishes a multilinear evaluation inside one workgroup: n <= 1024 values, k levels.
 struct FrPack12 { Fr x[12]; };
 static constexpr uint32_t ME_SMALL_MAX = 1024;
@@ -357,64 +475,112 @@ __global__ void __launch_bounds__(TPB) k_ip_round_w(Fr* __restrict__ partials, c
     block_reduce_store<3>(acc, partials);
 }
 
-// Whole sumcheck in one workgroup for short vectors (n <= 8192): every round's three sums are
-// written to polys[round*3 + {0,1,2}] (standard form, R^2-corrected), the folded vectors
-// ping-pong through `work` (2 * 2 * n_pow2/2 elements) and the final a, b land in fin[0..1].
-// Challenges are consumed from the back of vs (Montgomery form), as the reference does.
-struct FrPack16 { Fr x[16]; };
-__global__ void __launch_bounds__(1024) k_ip_small(Fr* __restrict__ polys, Fr* __restrict__ fin, Fr* __restrict__ work,
-                                                   const Fr* __restrict__ a_in, const Fr* __restrict__ b_in, const FrPack16 vs, uint32_t n, uint32_t k) {
-    __shared__ uint32_t red[8][1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t half0 = (1u << k) >> 1;
-    const Fr* a = a_in;
-    const Fr* b = b_in;
-    uint32_t n_in = n;
-    const Fr r2 = big_r2<8>();
-    for (uint32_t round = 0; round < k; ++round) {
-        const uint32_t n_out = (1u << (k - round)) >> 1;
-        Fr* na = work + (size_t)(round & 1) * 2 * half0;
-        Fr* nb = na + half0;
-        const Fr v = vs.x[k - 1 - round];
-        Fr acc[3] = {big_zero<8>(), big_zero<8>(), big_zero<8>()};
-        for (uint32_t g = t; g < n_out; g += 1024) {
-            const Fr a0 = (g < n_in) ? a[g] : big_zero<8>();
-            const Fr b0 = (g < n_in) ? b[g] : big_zero<8>();
-            const Fr a1 = (g + n_out < n_in) ? a[g + n_out] : big_zero<8>();
-            const Fr b1 = (g + n_out < n_in) ? b[g + n_out] : big_zero<8>();
-            const Fr da = sub(a1, a0), db = sub(b1, b0);
-            acc[0] = add(acc[0], mont_mul(a0, b0));
-            acc[1] = add(acc[1], add(mont_mul(a0, db), mont_mul(b0, da)));
-            acc[2] = add(acc[2], mont_mul(da, db));
-            na[g] = add(a0, mont_mul(v, da));
-            nb[g] = add(b0, mont_mul(v, db));
-        }
-        for (int q = 0; q < 3; ++q) {
-#pragma unroll
-            for (int l = 0; l < 8; ++l) red[l][t] = acc[q].v[l];
-            __syncthreads();
-            for (uint32_t s = 512; s > 0; s >>= 1) {
-                if (t < s) {
-                    Fr x, y;
-#pragma unroll
-                    for (int l = 0; l < 8; ++l) { x.v[l] = red[l][t]; y.v[l] = red[l][t + s]; }
-                    x = add(x, y);
-#pragma unroll
-                    for (int l = 0; l < 8; ++l) red[l][t] = x.v[l];
-                }
-                __syncthreads();
-            }
-            if (t == 0) {
-                Fr x;
-#pragma unroll
-                for (int l = 0; l < 8; ++l) x.v[l] = red[l][0];
-                polys[round * 3 + q] = mont_mul(x, r2);
-            }
-            __syncthreads();
-        }
-        a = na; b = nb; n_in = n_out;
+// The whole sumcheck of short vectors (n <= 8192) in one or two launches.  The challenges are known before the first round, and a round
+// pairs t with t + n/2 (the top index bit): the elements that agree in their low bits need nobody else for as many rounds as there are
+// high bits.  A workgroup takes the 2^R elements of one low index (R <= 8) of both vectors, in LDS and in 29-bit limbs, and runs R
+// rounds, a barrier each; a second launch of one workgroup runs what is left and adds up the first one's sums.  Every product of a pair
+// has a lane of its own -- sixteen lanes (a row of the data-parallel adds) do one thing for sixteen pairs:
+//   even waves: a0 b0 | a1 b1 | da db | -         odd waves: fold of a | fold of b | - | -
+// so a round is the latency of one product, a row sum and a barrier: about 2 us.  One workgroup that gave a pair to a lane and
+// summed through LDS took 15 us a round, 93 us for 64 elements and 225 us for 4096.  The middle coefficient is a1 b1 - a0 b0 - da db.
+static constexpr int IP_ROUNDS = 8, IP_P = 1 << IP_ROUNDS, IP_W = 12, IP_GROUPS = 8;      // IP_GROUPS: pairs of waves, sixteen pairs each
+struct IpArgs {
+    const Fr *a, *b;
+    Fr *na, *nb;                  // the folded vectors, gridDim.x elements each
+    Fr29 v[IP_ROUNDS];            // in round order, times 2^261
+    uint32_t n, nlow, rounds;     // the vectors' length (zeros behind it), low indices, rounds of this launch
+    Fr* sums;                     // round r's q-th sum at sums[(3 r + q) gridDim.x + workgroup]
+    const Fr* prev; Fr* prev_out; // the sums of a launch before: prev_count times prev_nb of them
+    uint32_t prev_nb, prev_count;
+};
+__global__ void __launch_bounds__(1024) k_ip_rounds(const IpArgs a) {
+    __shared__ int32_t X0[2][IP_P][IP_W], X1[2][IP_P / 2][IP_W];
+    __shared__ uint32_t raw[IP_ROUNDS][IP_GROUPS][3][9];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave & 1u, group = wave >> 1;
+    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u;
+    const uint32_t P = 1u << a.rounds;
+    for (uint32_t i = threadIdx.x; i < 2 * P; i += 1024u) {
+        const uint32_t s = i & (P - 1u), g = s * a.nlow + blockIdx.x;
+        rm_put(X0[i >> a.rounds][s], g < a.n ? fr29_repack((i >> a.rounds ? a.b : a.a)[g]) : fr29_zero());
     }
-    if (t == 0) { fin[0] = a[0]; fin[1] = b[0]; }
+    // the sums of the launch before, on waves that have no pairs here (it has at most 24 of them, of at most 32 parts each)
+    if (a.prev && wave >= 2u && (wave - 2u) * 4u < a.prev_count) {
+        const uint32_t j = (wave - 2u) * 4u + row, jc = j < a.prev_count ? j : 0u;
+        uint32_t l9[9];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) l9[l] = 0;
+        for (uint32_t i = ln; i < a.prev_nb; i += 16u) {
+            const Fr29 x = fr29_repack(a.prev[(size_t)jc * a.prev_nb + i]);
+#pragma unroll
+            for (int l = 0; l < 9; ++l) l9[l] += (uint32_t)x.l[l];
+        }
+        fr29_carry_u(l9);
+        fr29_row_sum(l9);
+        if (ln == 15u && j < a.prev_count) {
+            Fr29 x;
+#pragma unroll
+            for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+            a.prev_out[j] = fr29_canon_pack<2>(fr29_mul(x, fr29_2_261()));
+        }
+    }
+    __syncthreads();
+    for (uint32_t r = 0; r < a.rounds; ++r) {
+        const bool odd = (r & 1u) != 0;
+        const uint32_t half = P >> (r + 1);
+        int32_t* const src = odd ? &X1[0][0][0] : &X0[0][0][0];
+        int32_t* const dst = odd ? &X0[0][0][0] : &X1[0][0][0];
+        const uint32_t ss = (odd ? IP_P / 2 : IP_P) * IP_W, ds = (odd ? IP_P : IP_P / 2) * IP_W;
+        const uint32_t t = group * 16u + ln;
+        if (group * 16u < half) {
+            const bool live = t < half;
+            const uint32_t ta = live ? t : 0u, tb = ta + half;
+            auto rd = [&](uint32_t k, uint32_t slot) { return rm_get(src + k * ss + slot * IP_W); };
+            if (kind == 0) {
+                const Fr29 a0 = rd(0, ta), a1 = rd(0, tb), b0 = rd(1, ta), b1 = rd(1, tb);
+                const Fr29 x = fr29_mul(fr29_select(row == 0, a0, fr29_select(row == 1, a1, fr29_sub_plus_r(a1, a0))),
+                                        fr29_select(row == 0, b0, fr29_select(row == 1, b1, fr29_sub_plus_r(b1, b0))));
+                uint32_t l9[9];
+#pragma unroll
+                for (int l = 0; l < 9; ++l) l9[l] = live ? (uint32_t)x.l[l] : 0u;
+                fr29_row_sum(l9);
+                if (ln == 15u && row < 3u) {
+#pragma unroll
+                    for (int l = 0; l < 9; ++l) raw[r][group][row][l] = l9[l];
+                }
+            } else {
+                const Fr29 x0 = rd(row & 1u, ta), x1 = rd(row & 1u, tb);
+                const Fr29 f = fr29_canon<2>(fr29_add(x0, fr29_mul(a.v[r], fr29_sub_plus_r(x1, x0))));
+                if (live && row < 2u) rm_put(dst + row * ds + t * IP_W, f);
+            }
+        }
+        __syncthreads();
+    }
+    // a product of two elements carries 2^-261 here
+    if (threadIdx.x < 3u * a.rounds) {
+        const uint32_t r = threadIdx.x / 3u, q = threadIdx.x % 3u, half = P >> (r + 1), ng = (half + 15u) / 16u;
+        auto sum = [&](uint32_t role) {
+            uint32_t l9[9];
+#pragma unroll
+            for (int l = 0; l < 9; ++l) {
+                l9[l] = 0;
+                for (uint32_t g = 0; g < ng; ++g) l9[l] += raw[r][g][role][l];
+            }
+            fr29_carry_u(l9);
+            Fr29 x;
+#pragma unroll
+            for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+            return fr29_canon_pack<5>(fr29_mul(x, fr29_2_522()));
+        };
+        Fr o = sum(q == 0 ? 0u : (q == 2 ? 2u : 1u));
+        if (q == 1) o = sub(sub(o, sum(0)), sum(2));
+        a.sums[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = o;
+    }
+    const int32_t* const fin = (a.rounds & 1u) ? &X1[0][0][0] : &X0[0][0][0];
+    const uint32_t fs = ((a.rounds & 1u) ? IP_P / 2 : IP_P) * IP_W;
+    if (threadIdx.x >= 64u && threadIdx.x < 66u) {
+        const uint32_t k = threadIdx.x - 64u;
+        (k ? a.nb : a.na)[blockIdx.x] = fr29_pack(rm_get(fin + k * fs));
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -645,6 +811,75 @@ int zk_fr_fold_axis(void* out, const void* in, const uint32_t* u, int levels, si
     return 0;
 }
 
+// All `levels` of the axis: out has other * ceil(cur / 2^levels) * window elements.  The whole axis in one pass where it is long enough for the table of
+// weights to pay (a launch of its own) and the tensor large enough that its passes and not their launches count (2^15 elements, 1 MB);
+// else three levels a launch.
+int zk_fr_fold_axis_all(void* out, const void* in, const uint32_t* u, int levels, size_t other, uint32_t cur, size_t window, void* stv) {
+    hipStream_t st = (hipStream_t)stv;
+    ZK_ARG(levels >= 1 && levels <= 32 && cur >= 1 && window >= 1, "zk_fr_fold_axis_all: bad axis");
+    ZK_ARG(out != in, "zk_fr_fold_axis_all: out must differ from in");
+    if (other == 0) return 0;
+    if (levels < 32 && cur % (1u << levels) == 0) { other *= cur >> levels; cur = 1u << levels; }      // fewer levels than the axis has: as many axes of 2^levels
+    const bool whole = (uint64_t)cur <= ((uint64_t)1 << levels), rows = window == 1 && cur >= 128, cols = window >= 32 && cur >= 16 && other <= 65535;
+    if (whole && levels <= EQ29_MAX && (rows || cols) && other * cur * window >= ((size_t)1 << 15) && cdiv(other, 2) <= 0x7FFFFFFFu) {
+        Eq29Tabs tabs;
+        const int bits[3] = {(levels + 2) / 3, (levels + 1) / 3, levels / 3};
+        int at = 0;
+        for (int f = 0; f < 3; ++f) {
+            Fr t[32];
+            t[0] = fr29_pack(fr29_2_261());
+            for (int b = 0; b < bits[f]; ++b, ++at) {
+                const Fr x = to_mont(load_fr(u + 8 * at));
+                for (int i = 0; i < (1 << b); ++i) {
+                    t[i + (1 << b)] = mont_mul(t[i], x);
+                    t[i] = sub(t[i], t[i + (1 << b)]);
+                }
+            }
+            for (int i = 0; i < (1 << bits[f]); ++i) tabs.t[32 * f + i] = fr29_repack(t[i]);
+        }
+        Scratch eq(sizeof(int32_t) * 9 * (size_t)cur, st);
+        if (eq.rc) return eq.rc;
+        if (rows) {
+            hipLaunchKernelGGL(k_eq29<true>, dim3(cdiv(cur, TPB)), dim3(TPB), 0, st, eq.as<int32_t>(), tabs, cur, bits[0], bits[1]);
+            // a wave for two rows where that fills the chip (four waves a SIMD) or the rows are short, four waves else
+            if (cur < 512 || (other >= 8192 && cur <= 4096)) hipLaunchKernelGGL(k_fold_rows<1>, dim3(cdiv(other, 8)), dim3(TPB), 0, st, (Fr*)out, (const Fr*)in, eq.as<int32_t>(), other, cur);
+            else hipLaunchKernelGGL(k_fold_rows<4>, dim3(cdiv(other, 2)), dim3(TPB), 0, st, (Fr*)out, (const Fr*)in, eq.as<int32_t>(), other, cur);
+            ZK_LAUNCH_CHECK();
+            return 0;
+        }
+        hipLaunchKernelGGL(k_eq29<false>, dim3(cdiv(cur, TPB)), dim3(TPB), 0, st, eq.as<int32_t>(), tabs, cur, bits[0], bits[1]);
+        // terms of a lane: as many as leave 8192 waves, between 8 and 64 (the reduction at a lane's end costs as much as three terms)
+        const size_t groups = (window + 63) / 64, n_out = other * window;
+        uint32_t J = 64;
+        while (J > 8 && other * groups * ((cur + J - 1) / J) < 8192) J >>= 1;
+        const uint32_t chunks = (cur + 4 * J - 1) / (4 * J);
+        Scratch part(chunks > 1 ? sizeof(Fr) * n_out * chunks : 1, st);
+        if (part.rc) return part.rc;
+        hipLaunchKernelGGL(k_fold_cols, dim3((unsigned)groups, chunks, (unsigned)other), dim3(TPB), 0, st, chunks > 1 ? part.as<Fr>() : (Fr*)out, (const Fr*)in, eq.as<int32_t>(), cur, window, J);
+        ZK_LAUNCH_CHECK();
+        if (chunks > 1) LAUNCH1D(k_sum_partials, n_out, st, (Fr*)out, part.as<Fr>(), n_out, chunks);
+        return 0;
+    }
+    std::unique_ptr<Scratch> keep[2];
+    const void* src = in;
+    for (int done = 0, which = 0; done < levels; which ^= 1) {
+        const int L = std::min(3, levels - done);
+        const uint32_t cur_out = (uint32_t)(((uint64_t)cur + (1u << L) - 1) >> L);
+        void* dst = out;
+        if (done + L < levels) {
+            keep[which].reset(new Scratch(sizeof(Fr) * other * cur_out * window, st));
+            if (keep[which]->rc) return keep[which]->rc;
+            dst = keep[which]->p;
+        }
+        const int rc = zk_fr_fold_axis(dst, src, u + 8 * done, L, other, cur, window, stv);
+        if (rc) return rc;
+        src = dst;
+        cur = cur_out;
+        done += L;
+    }
+    return 0;
+}
+
 // Multilinear extension of a (n elements, zero-extended to 2^k) at u[0..k): index bit j is bound
 // to u[j].  Requires 2^(k-1) < n <= 2^k (k = 0 allowed for n == 1).
 int zk_fr_me(uint32_t* out_host, const void* a, size_t n, const uint32_t* u, int k, void* stv) {
@@ -723,21 +958,37 @@ int zk_ip_round_stacked(uint32_t* poly3_host, const void* a, const void* b, cons
     return 0;
 }
 
-// Complete inner-product sumcheck for n <= 8192 in one launch.  u[0..k) standard form, consumed
+// Complete inner-product sumcheck for n <= 8192 in one or two launches.  u[0..k) standard form, consumed
 // from the back; polys_host gets 3*k coefficients, fin_host the folded a and b.
 int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a, const void* b, uint32_t n, const uint32_t* u, int k, void* stv) {
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(k >= 1 && k <= 13, "zk_ip_sumcheck_small: k must be 1..13");
     ZK_ARG(n >= 1 && n <= (1u << k) && n > ((1u << k) >> 1), "zk_ip_sumcheck_small: need 2^(k-1) < n <= 2^k");
-    FrPack16 p;
-    for (int i = 0; i < 16; ++i) p.x[i] = (i < k) ? to_mont(load_fr(u + 8 * i)) : big_zero<8>();
-    const size_t half0 = ((size_t)1 << k) >> 1;
-    Scratch work(sizeof(Fr) * (4 * half0 + 3 * (size_t)k + 2), st);
+    // out: the sums of all rounds, then the two folded values; behind them what passes from the first launch to the second
+    const int r1 = k <= IP_ROUNDS ? 0 : IP_ROUNDS, r2 = k - r1;
+    const uint32_t nb1 = r1 ? 1u << (k - r1) : 0u;
+    Scratch work(sizeof(Fr) * (3 * (size_t)k + 2 + (3 * (size_t)r1 + 2) * nb1), st);
     if (work.rc) return work.rc;
-    Fr* w = work.as<Fr>();
-    Fr* polys = w + 4 * half0;
-    Fr* fin = polys + 3 * k;
-    hipLaunchKernelGGL(k_ip_small, dim3(1), dim3(1024), 0, st, polys, fin, w, (const Fr*)a, (const Fr*)b, p, n, (uint32_t)k);
+    Fr* polys = work.as<Fr>();
+    Fr* part = polys + 3 * k + 2;
+    Fr* mid = part + 3 * (size_t)r1 * nb1;
+    IpArgs q;
+    memset(&q, 0, sizeof(q));
+    q.a = (const Fr*)a; q.b = (const Fr*)b; q.n = n;
+    auto challenges = [&](int from, int count) {
+        for (int i = 0; i < count; ++i) q.v[i] = fr29_repack(mont_mul(to_mont(load_fr(u + 8 * (size_t)(k - 1 - from - i))), fr29_pack(fr29_2_261())));
+    };
+    if (r1) {
+        challenges(0, r1);
+        q.rounds = (uint32_t)r1; q.nlow = nb1; q.sums = part; q.na = mid; q.nb = mid + nb1;
+        hipLaunchKernelGGL(k_ip_rounds, dim3(nb1), dim3(1024), 0, st, q);
+        ZK_LAUNCH_CHECK();
+        q.a = mid; q.b = mid + nb1; q.n = nb1;
+        q.prev = part; q.prev_out = polys; q.prev_nb = nb1; q.prev_count = 3u * (uint32_t)r1;
+    }
+    challenges(r1, r2);
+    q.rounds = (uint32_t)r2; q.nlow = 1; q.sums = polys + 3 * r1; q.na = polys + 3 * k; q.nb = q.na + 1;
+    hipLaunchKernelGGL(k_ip_rounds, dim3(1), dim3(1024), 0, st, q);
     ZK_LAUNCH_CHECK();
     // one delivery of 3k + 2 values: the round polynomials, then the two fully folded values
     Fr both[3 * 13 + 2];

@@ -445,7 +445,7 @@ vector<Fr_t> FrTensor::me_batch(const vector<const FrTensor*>& ts, const vector<
     return out;
 }
 
-// Folds `u.size()` levels of the middle axis, up to three levels per pass.
+// Folds `u.size()` levels of the middle axis.
 static FrTensor fold_axis_all(const FrTensor& t, const vector<Fr_t>& u, uint cur_dim, size_t window) {
     if (u.empty()) return t;
     if ((size_t)t.size % ((size_t)cur_dim * window) != 0) throw std::runtime_error("t.size % (cur_dim * window_size) != 0");
@@ -462,20 +462,9 @@ static FrTensor fold_axis_all(const FrTensor& t, const vector<Fr_t>& u, uint cur
             return out;
         }
     }
-    const Fr_t* src = t.gpu_data;
-    std::vector<FrTensor> keep;   // intermediates stay alive until the last pass has been queued
-    size_t done = 0;
-    uint cur = cur_dim;
-    while (done < u.size()) {
-        const int L = (int)std::min<size_t>(3, u.size() - done);
-        const uint cur_out = (uint)(((uint64_t)cur + (1u << L) - 1) >> L);
-        keep.emplace_back((uint)(other * cur_out * window));
-        ZKC(zk_fr_fold_axis(keep.back().gpu_data, src, u[done].val, L, other, cur, window, nullptr));
-        src = keep.back().gpu_data;
-        cur = cur_out;
-        done += L;
-    }
-    FrTensor out(std::move(keep.back()));
+    const uint64_t left = u.size() < 32 ? ((uint64_t)cur_dim + (1ull << u.size()) - 1) >> u.size() : 1;
+    FrTensor out((uint)(other * left * window));
+    ZKC(zk_fr_fold_axis_all(out.gpu_data, t.gpu_data, u[0].val, (int)u.size(), other, cur_dim, window, nullptr));
     return out;
 }
 

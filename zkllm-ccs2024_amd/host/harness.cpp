@@ -239,7 +239,7 @@ int zkp_zkip(const u32* claim, void* a, void* b, const u32* u, int k, u32* proof
 // zkFC::prove on existing tensors; challenges come from the seeded stream
 int zkp_zkfc_prove(void* X, void* W, void* Y, u32 in_dim, u32 out_dim, u32* claim_W) {
     ZKP_TRY
-    zkFC fc(in_dim, out_dim, FT(W));
+    zkFC fc(in_dim, out_dim, FrTensor::view(FT(W)));      // the weight outlives the proof
     auto claims = fc.prove(FT(X), FT(Y));
     if (claim_W) memcpy(claim_W, claims[0].claim.val, 32);
     ZKP_END
