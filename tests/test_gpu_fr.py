@@ -151,6 +151,24 @@ def test_partial_me(pv, orc, other, cur, win):
             assert (got == exp[:out_n[0]]).all()
 
 
+# a whole axis in one pass: the innermost one on one wave or four for two rows, odd rows and row lengths; a middle one with one lane's share
+# and less, in one piece and in several, last pieces short
+@pytest.mark.parametrize("other,cur,win", [(1001, 130, 1), (257, 129, 1), (33, 1000, 1), (8193, 512, 1), (3, 11008, 1), (2, 16384, 1), (1, 2049, 32), (2, 600, 70), (40, 16, 65), (1, 11008, 33),
+                                           (3, 129, 100)])
+def test_partial_me_of_a_whole_axis(pv, orc, other, cur, win):
+    n = other * cur * win
+    A = mt_random_vec(np.random.RandomState(cur), n)
+    A[: n // 3] = mt_random_vec(np.random.RandomState(1), 1) if n % 2 else fr_array([R_MOD - 1])      # a long run of one value, the largest one among them
+    k = (cur - 1).bit_length()
+    u = mt_random_vec(np.random.RandomState(8), k)
+    exp = np.zeros((n, 8), np.uint32)
+    out_n = np.zeros(1, np.int64)
+    orc_check(orc.orc_fr_partial_me(A, n, u, k, cur, win, exp, out_n))
+    got = pv.partial_me(pv.from_fr(A), u, cur, win).host()
+    assert got.shape[0] == out_n[0] == other * win
+    assert (got == exp[:out_n[0]]).all()
+
+
 @pytest.mark.parametrize("n,win,k", [(32, 4, 3), (15, 3, 3), (18, 4, 3), (4096 * 16, 4096, 4), (11008 * 8, 8, 14)])
 def test_window_fold(pv, orc, n, win, k):
     A = mt_random_vec(np.random.RandomState(n % 1000), n)
@@ -285,6 +303,12 @@ def test_zkip_matches_oracle(pv, orc, n):
     bad[0] ^= 1
     with pytest.raises(RuntimeError, match="claim != p"):
         pv.zkip(bad, ha, hb, u)
+
+
+# one launch up to 256 elements, two above, the second with one round to five
+@pytest.mark.parametrize("n", [33, 129, 255, 256, 257, 512, 513, 2047, 5000])
+def test_zkip_around_the_launches_of_short_vectors(pv, orc, n):
+    test_zkip_matches_oracle(pv, orc, n)
 
 
 @pytest.mark.parametrize("B,I,O,mode", [(16, 64, 64, 1), (16, 64, 64, 0), (5, 24, 10, 1), (64, 256, 128, 0)])
@@ -447,6 +471,21 @@ def test_matmul_int8_plane_path_on_ragged_stacks_and_wide_operands(pv):
             del os.environ["ZKLLM_MATMUL_PLANES"]
         else:
             os.environ["ZKLLM_MATMUL_PLANES"] = old
+
+
+@pytest.mark.parametrize("num,M,N,P,amax,bmax", [(1, 1, 1, 1, 5, 5), (1, 1, 300, 70, 2 ** 17, 2 ** 13), (2, 67, 129, 65, 0x7F7F7F7F, 0x7F7F), (1, 5, 64, 63, 0x7F7F80, 0x7F80),
+                                                 (3, 4, 127, 3, 0x7F7F7F80, 2 ** 20), (1, 130, 128, 64, 2 ** 36, 2 ** 14), (1, 66, 40, 30, 2 ** 20, 2 ** 31), (1, 9, 3000, 20, 2 ** 34, 0x7F7F)])
+def test_matmul_of_small_integers_of_any_size(pv, num, M, N, P, amax, bmax):
+    """Operands examined and split in one pass (k_examine_split), magnitudes at the edges of one to five digit planes."""
+    rng = np.random.default_rng(M + N)
+    pv.lib.zkp_set_matmul_mode(ctypes.c_int(0))
+    A = rng.integers(-amax, amax + 1, (num, M, N)).astype(np.int64)
+    B = rng.integers(-bmax, bmax + 1, (num, N, P)).astype(np.int64)
+    A[-1, -1, -1], A[0, 0, 0] = amax, -amax
+    B[0, 0, 0], B[-1, -1, -1] = bmax, -bmax
+    got = pv.matmul_stack(pv.from_i64(A), pv.from_i64(B), num, M, N, P).host()
+    assert pv.lib.zkp_last_matmul_path() == 2
+    assert fr_ints(got) == [int(v) % R_MOD for i in range(num) for v in (A[i].astype(object) @ B[i].astype(object)).reshape(-1)]
 
 
 def test_matmul_with_a_kept_right_operand_and_layers_over_views(pv):

@@ -17,6 +17,7 @@
 //    with int32 accumulation (k_gemm_i8_planes_all: v_mfma_i32_32x32x32_i8 tiles), planes of equal weight 2^(8s) accumulate into the same output, and one
 //    pass recombines the outputs in int64.  Exact: a dot product of digits stays below 2^31 (checked), the
 //    recombined value is the true integer result, below 2^62 by the bound above.
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -438,6 +439,110 @@ __global__ void __launch_bounds__(256) k_split_cols(int8_t* __restrict__ planes,
             *reinterpret_cast<v4i*>(planes + ((b * np + j) * P + p0 + row) * Kp + k0 + ch * 16) = *reinterpret_cast<const v4i*>(&tile[j][row][ch * 16]);
 }
 
+// Both operands examined and split in one pass over each: their first four planes -- all there are of 32-bit integers -- and the figures
+// that say what holds (out[0]: largest |a|, out[1]: largest |b|, out[2]: largest row sum of |a|; ~0: not small).  An operand is read
+// once, where finding the figures first and splitting afterwards read it twice: 2048 x 4096 by 4096 x 4096, 0.45 ms -> 0.2 ms.
+// Workgroups below nA take four rows of A, a wave a row; the others a 64 x 64 tile of B, which goes through LDS.
+// The digits of four elements become one word of each plane: on a wave that holds neighbours in neighbouring lanes, the lanes of four
+// exchange their words (quad permutations) and each keeps one plane's bytes.
+struct ExamineArgs { const Fr *A, *B; int8_t *pA, *pB; unsigned long long* out; uint32_t nA, rowsA, M, N, P, Kp, tilesP, tilesK; };
+__device__ __forceinline__ unsigned long long fr_magnitude(const Fr& x, bool& negative) {       // ~0: above 2^62
+    unsigned long long v;
+    negative = (x.v[2] | x.v[3] | x.v[4] | x.v[5] | x.v[6] | x.v[7]) != 0;
+    if (!negative) v = (unsigned long long)x.v[0] | ((unsigned long long)x.v[1] << 32);
+    else {
+        const Fr y = neg(x);
+        v = (y.v[2] | y.v[3] | y.v[4] | y.v[5] | y.v[6] | y.v[7]) ? ~0ull : ((unsigned long long)y.v[0] | ((unsigned long long)y.v[1] << 32));
+    }
+    return v > (1ull << 62) ? ~0ull : v;
+}
+// the balanced digits of a 32-bit integer, one a byte
+__device__ __forceinline__ uint32_t digit_bytes(unsigned long long mag, bool negative) {
+    const uint32_t x = negative ? 0u - (uint32_t)mag : (uint32_t)mag;
+    return (x + 0x80808080u) ^ 0x80808080u;
+}
+__global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
+    __shared__ uint32_t tile[4][64][17];
+    __shared__ unsigned long long red[4];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    auto sat_add = [](unsigned long long x, unsigned long long y) { return (x == ~0ull || y == ~0ull || x + y > (1ull << 62)) ? ~0ull : x + y; };
+    auto raise = [](unsigned long long* p, unsigned long long v) { if (v > __atomic_load_n(p, __ATOMIC_RELAXED)) atomicMax(p, v); };
+    if (blockIdx.x < g.nA) {
+        const uint32_t row = blockIdx.x * 4 + wave;
+        if (row >= g.rowsA) return;
+        const Fr* src = g.A + (size_t)row * g.N;
+        const uint32_t b = row / g.M, m = row - b * g.M, q = lane & 3u, sel = ((4u + q) << 8) | q;
+        int8_t* dst = g.pA + ((size_t)(b * 4 + q) * g.M + m) * g.Kp;
+        unsigned long long mx = 0, sum = 0;
+        for (uint32_t k0 = 0; k0 < g.Kp; k0 += 128) {
+            Fr x[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) x[i] = k0 + 64 * i + lane < g.N ? src[k0 + 64 * i + lane] : big_zero<8>();
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                bool ng;
+                const unsigned long long v = fr_magnitude(x[i], ng);
+                mx = v > mx ? v : mx;
+                sum = sat_add(sum, v);
+                const int w = (int)digit_bytes(v, ng);
+                const uint32_t w0 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x00, 0xF, 0xF, false), w1 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x55, 0xF, 0xF, false);
+                const uint32_t w2 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xAA, 0xF, 0xF, false), w3 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xFF, 0xF, 0xF, false);
+                const uint32_t lo = __builtin_amdgcn_perm(w1, w0, sel), hi = __builtin_amdgcn_perm(w3, w2, sel);
+                *reinterpret_cast<uint32_t*>(dst + k0 + 64 * i + (lane & ~3u)) = (lo & 0xFFFFu) | (hi << 16);
+            }
+        }
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long om = __shfl_xor(mx, off, 64), os = __shfl_xor(sum, off, 64);
+            mx = om > mx ? om : mx;
+            sum = sat_add(sum, os);
+        }
+        if (lane == 0) { raise(g.out, mx); raise(g.out + 2, sum); }
+        return;
+    }
+    const uint32_t idx = blockIdx.x - g.nA, per = g.tilesP * g.tilesK, b = idx / per, r = idx - b * per, tk = r / g.tilesP, tp = r - tk * g.tilesP;
+    const uint32_t p0 = tp * 64, k0 = tk * 64;
+    const Fr* src = g.B + (size_t)b * g.N * g.P;
+    unsigned long long mx = 0;
+    for (uint32_t c = 0; c < 4; ++c) {
+        const uint32_t kk = wave * 16 + c * 4;
+        Fr x[4];
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = (k0 + kk + i < g.N && p0 + lane < g.P) ? src[(size_t)(k0 + kk + i) * g.P + p0 + lane] : big_zero<8>();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bool ng;
+            const unsigned long long v = fr_magnitude(x[i], ng);
+            mx = v > mx ? v : mx;
+            w[i] = digit_bytes(v, ng);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t sel = ((4u + j) << 8) | j;
+            tile[j][lane][kk / 4] = (__builtin_amdgcn_perm(w[1], w[0], sel) & 0xFFFFu) | (__builtin_amdgcn_perm(w[3], w[2], sel) << 16);
+        }
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long om = __shfl_xor(mx, off, 64);
+        mx = om > mx ? om : mx;
+    }
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    if (t == 0) {
+        for (int i = 1; i < 4; ++i) mx = red[i] > mx ? red[i] : mx;
+        raise(g.out + 1, mx);
+    }
+    const uint32_t row = t >> 2, ch = t & 3u;
+    if (p0 + row < g.P)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const v4i v = {(int)tile[j][row][4 * ch], (int)tile[j][row][4 * ch + 1], (int)tile[j][row][4 * ch + 2], (int)tile[j][row][4 * ch + 3]};
+            *reinterpret_cast<v4i*>(g.pB + ((size_t)(b * 4 + j) * g.P + p0 + row) * g.Kp + k0 + 16 * ch) = v;
+        }
+}
+
 // C[b][m][p] = sum_{i,j} 256^(i+j) sum_k PA_i[b][m][k] PB_j[b][p][k], embedded in Fr.
 // One block computes a 128 x 128 tile of C; each of its four waves a 64 x 64 quarter as 2 x 2 tiles of
 // v_mfma_i32_32x32x32_i8.  Plane pairs are taken one after the other: int32 accumulators over the whole contraction
@@ -448,7 +553,8 @@ __global__ void __launch_bounds__(256) k_split_cols(int8_t* __restrict__ planes,
 // both operands alike, so whatever order the instruction takes the bytes in, every product pairs equal k.  Outputs:
 // register r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of the 32 x 32 tile.
 // C64 set: the products are written there as 64-bit integers (8 bytes an element) and C is not written
-struct PlaneGemm { const int8_t* A; const int8_t* B; Fr* C; uint32_t M, P, Kp; int pa, pb; long long* C64; };
+// pa, pb: planes multiplied; sa, sb: planes stored for a matrix of a stack
+struct PlaneGemm { const int8_t* A; const int8_t* B; Fr* C; uint32_t M, P, Kp; int pa, pb; long long* C64; int sa, sb; };
 __device__ __forceinline__ void gemm_store(const PlaneGemm& g, size_t at, long long v) {
     if (g.C64) g.C64[at] = v;
     else g.C[at] = fr_from_i64(v);
@@ -466,8 +572,8 @@ __global__ void __launch_bounds__(256) k_gemm_i8_planes(const PlaneGemm g) {
         for (int r = 0; r < 16; ++r) tot[q][r] = 0;
     for (int i = 0; i < g.pa; ++i)
         for (int j = 0; j < g.pb; ++j) {
-            const int8_t* __restrict__ Ai = g.A + ((b * g.pa + i) * g.M) * (size_t)g.Kp;
-            const int8_t* __restrict__ Bj = g.B + ((b * g.pb + j) * g.P) * (size_t)g.Kp;
+            const int8_t* __restrict__ Ai = g.A + ((b * g.sa + i) * g.M) * (size_t)g.Kp;
+            const int8_t* __restrict__ Bj = g.B + ((b * g.sb + j) * g.P) * (size_t)g.Kp;
             v16i acc[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -536,8 +642,8 @@ template <int PA, int PB> __global__ void __launch_bounds__(256, 2) k_gemm_i8_pl
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
     const uint32_t m0 = blockIdx.y * TB, n0 = blockIdx.x * TB;
     const size_t b = blockIdx.z;
-    const int8_t* __restrict__ A0 = g.A + (b * PA * g.M) * (size_t)g.Kp;
-    const int8_t* __restrict__ B0 = g.B + (b * PB * g.P) * (size_t)g.Kp;
+    const int8_t* __restrict__ A0 = g.A + (b * g.sa * g.M) * (size_t)g.Kp;
+    const int8_t* __restrict__ B0 = g.B + (b * g.sb * g.P) * (size_t)g.Kp;
     const size_t a_plane = (size_t)g.M * g.Kp, b_plane = (size_t)g.P * g.Kp;
     v16i acc[NS];
 #pragma unroll
@@ -589,7 +695,7 @@ template <int PA, int PB> __global__ void __launch_bounds__(256, 2) k_gemm_i8_pl
     for (int r = 0; r < 16; ++r) {
         unsigned long long v = 0;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) v += (unsigned long long)(long long)acc[s][r] << (8 * s);
+        for (int s = 0; s < NS && s < 8; ++s) v += (unsigned long long)(long long)acc[s][r] << (8 * s);
         const uint32_t row = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
         const uint32_t col = n0 + wn * 32 + (lane & 31);
         if (row < g.M && col < g.P) gemm_store(g, (b * g.M + row) * (size_t)g.P + col, (long long)v);
@@ -608,6 +714,8 @@ static bool launch_gemm_all(int pa, int pb, dim3 grid, hipStream_t st, const Pla
         case 1: return launch_gemm_all_b<1>(pb, grid, st, g);
         case 2: return launch_gemm_all_b<2>(pb, grid, st, g);
         case 3: return launch_gemm_all_b<3>(pb, grid, st, g);
+        case 4: return launch_gemm_all_b<4>(pb, grid, st, g);
+        case 5: return launch_gemm_all_b<5>(pb, grid, st, g);
         default: return false;
     }
 }
@@ -632,7 +740,8 @@ static int digits_for(unsigned long long absmax) {      // planes needed for |x|
 struct MatmulRhs { const void* B = nullptr; uint32_t N = 0, P = 0, Kp = 0; unsigned long long mb = ~0ull; int pb = 0; void* planes = nullptr; };
 static int run_int8_plane_path(void* C, const void* A, const void* B, uint32_t batch, uint32_t M, uint32_t N, uint32_t P, unsigned long long ma, unsigned long long mb,
                                hipStream_t st, bool* done, const MatmulRhs* rhs = nullptr, ProdSrc src = ProdSrc{nullptr, nullptr}, long long* C64 = nullptr,
-                               bool b_transposed = false) {
+                               bool b_transposed = false, const int8_t* pa4 = nullptr, const int8_t* pb4 = nullptr) {
+    // pa4, pb4: the operands' first four planes, where an earlier pass has written them
     *done = false;
     const int pa = digits_for(ma), pb = digits_for(mb);
     if (!pa || !pb) return 0;
@@ -641,23 +750,26 @@ static int run_int8_plane_path(void* C, const void* A, const void* B, uint32_t b
     const uint32_t Kp = (N + GBK - 1) / GBK * GBK;
     const size_t rows_a = (size_t)batch * M;
     const bool have_b = rhs && rhs->planes && rhs->pb == pb && rhs->Kp == Kp && batch == 1;
-    Scratch pla(rows_a * pa * Kp, st), plb(have_b ? 1 : (size_t)batch * pb * P * Kp, st);
+    const bool use_a4 = pa4 && pa <= 4, use_b4 = pb4 && pb <= 4;
+    Scratch pla(use_a4 ? 1 : rows_a * pa * Kp, st), plb(have_b || use_b4 ? 1 : (size_t)batch * pb * P * Kp, st);
     if (pla.rc) return pla.rc;
     if (plb.rc) return plb.rc;
-    hipLaunchKernelGGL(k_split_rows, dim3(cdiv(rows_a * (Kp / 4), 256)), dim3(256), 0, st, pla.as<int8_t>(), (const Fr*)A, src, rows_a, M, N, Kp, pa);
+    if (!use_a4) hipLaunchKernelGGL(k_split_rows, dim3(cdiv(rows_a * (Kp / 4), 256)), dim3(256), 0, st, pla.as<int8_t>(), (const Fr*)A, src, rows_a, M, N, Kp, pa);
     // a right operand given transposed ([batch][P][N]) has its planes' layout already: its rows are split like the left operand's
-    if (!have_b && b_transposed)
+    if (have_b || use_b4) {}
+    else if (b_transposed)
         hipLaunchKernelGGL(k_split_rows, dim3(cdiv((size_t)batch * P * (Kp / 4), 256)), dim3(256), 0, st, plb.as<int8_t>(), (const Fr*)B, ProdSrc{nullptr, nullptr}, (size_t)batch * P, P, N, Kp, pb);
-    else if (!have_b) hipLaunchKernelGGL(k_split_cols, dim3(cdiv(P, 64), Kp / 64, batch), dim3(256), 0, st, plb.as<int8_t>(), (const Fr*)B, N, P, Kp, pb);
-    const PlaneGemm g{pla.as<int8_t>(), have_b ? (const int8_t*)rhs->planes : plb.as<int8_t>(), (Fr*)C, M, P, Kp, pa, pb, C64};
+    else hipLaunchKernelGGL(k_split_cols, dim3(cdiv(P, 64), Kp / 64, batch), dim3(256), 0, st, plb.as<int8_t>(), (const Fr*)B, N, P, Kp, pb);
+    const PlaneGemm g{use_a4 ? pa4 : pla.as<int8_t>(), have_b ? (const int8_t*)rhs->planes : (use_b4 ? pb4 : plb.as<int8_t>()), (Fr*)C, M, P, Kp, pa, pb, C64,
+                      use_a4 ? 4 : pa, !have_b && use_b4 ? 4 : pb};
     hipEvent_t t0 = nullptr, t1 = nullptr;
     if (g_gemm_timer.on) {
         ZK_HIP(hipEventCreate(&t0));
         ZK_HIP(hipEventCreate(&t1));
         ZK_HIP(hipEventRecord(t0, st));
     }
-    // up to three planes a side and three pairs' sums within int32: every pair in one pass; else pair by pair
-    const bool all_pairs = pa <= 3 && pb <= 3 && 3ull * N < (1ull << 17) && launch_gemm_all(pa, pb, dim3(cdiv(P, 64), cdiv(M, 64), batch), st, g);
+    // up to five planes by three, the sums of the pairs of equal weight within int32: every pair in one pass; else pair by pair
+    const bool all_pairs = pa <= 5 && pb <= 3 && (unsigned long long)std::min(pa, pb) * N < (1ull << 17) && launch_gemm_all(pa, pb, dim3(cdiv(P, 64), cdiv(M, 64), batch), st, g);
     if (!all_pairs) hipLaunchKernelGGL(k_gemm_i8_planes, dim3(cdiv(P, GBN), cdiv(M, GBM), batch), dim3(256), 0, st, g);
     if (g_gemm_timer.on) {
         ZK_HIP(hipEventRecord(t1, st));
@@ -712,16 +824,42 @@ static int matmul_dispatch(void* C, const void* A, const void* B, uint32_t batch
     ZK_ARG(mode >= 0 && mode <= 2, "zk_fr_matmul: mode must be 0, 1 or 2");
     ZK_ARG(batch <= 65535, "zk_fr_matmul: at most 65535 products per call");
     ZK_ARG((size_t)batch * M < ((size_t)1 << 31), "zk_fr_matmul: too many rows in one call");
+    // ZKLLM_MATMUL_PLANES: log2 of the multiply-accumulates from which on a product may go to the matrix cores, 0 = never.  Unset: always;
+    // 64-bit results from 2^30 (a caller of those falls back to field elements, and smaller scores gain nothing by being kept as integers)
+    const char* planes_env = getenv("ZKLLM_MATMUL_PLANES");           // read at every call: tests set it around single products
+    const int planes_log2 = planes_env ? atoi(planes_env) : (C64 ? 30 : 1);
+    const bool planes_wanted = planes_log2 > 0 && (unsigned __int128)batch * M * N * P >= ((unsigned __int128)1 << planes_log2) && N < (1u << 17);
+    if (C64 && (!planes_wanted || M < 32 || P < 32)) { if (path_used) *path_used = 0; return 0; }
     bool small = false, fits32 = false, b_fits32 = false;
     unsigned long long ma_ = 0, mb_ = 0;
+    std::unique_ptr<Scratch> planes4[2];      // the operands' first four planes, written while they are examined
+    const uint32_t Kp4 = (N + GBK - 1) / GBK * GBK;
+    const uint64_t tiles_b = (uint64_t)cdiv(P, 64) * (Kp4 / 64) * batch;
+    const bool examine = mode != 1 && planes_wanted && !src.a && !b_transposed && cdiv((size_t)batch * M, 4) + tiles_b < (1ull << 31) && tiles_b < (1ull << 31);
     if (mode != 1) {
         Scratch mx(3 * sizeof(unsigned long long), st);
         if (mx.rc) return mx.rc;
         ZK_HIP(hipMemsetAsync(mx.p, 0, 3 * sizeof(unsigned long long), st));
         const size_t nb = (size_t)batch * N * P;
+        if (examine) {
+            planes4[0].reset(new Scratch((size_t)batch * M * 4 * Kp4, st));
+            if (planes4[0]->rc) return planes4[0]->rc;
+            ExamineArgs x;
+            memset(&x, 0, sizeof(x));
+            x.A = (const Fr*)A; x.B = (const Fr*)B; x.pA = planes4[0]->as<int8_t>(); x.out = mx.as<unsigned long long>();
+            x.rowsA = batch * M; x.M = M; x.N = N; x.P = P; x.Kp = Kp4; x.nA = cdiv(x.rowsA, 4);
+            x.tilesP = cdiv(P, 64); x.tilesK = Kp4 / 64;
+            if (!rhs) {
+                planes4[1].reset(new Scratch((size_t)batch * P * 4 * Kp4, st));
+                if (planes4[1]->rc) return planes4[1]->rc;
+                x.pB = planes4[1]->as<int8_t>();
+            }
+            hipLaunchKernelGGL(k_examine_split, dim3(x.nA + (rhs ? 0u : (unsigned)tiles_b)), dim3(256), 0, st, x);
+        } else {
         if (!rhs) hipLaunchKernelGGL(k_absmax, dim3(absmax_grid(nb)), dim3(256), 0, st, mx.as<unsigned long long>() + 1, (const Fr*)B, nb);
         if (src.a) hipLaunchKernelGGL(k_rowabs_prod, dim3(batch * M), dim3(256), 0, st, mx.as<unsigned long long>() + 2, mx.as<unsigned long long>(), src, N);
         else hipLaunchKernelGGL(k_rowabs, dim3(batch * M), dim3(256), 0, st, mx.as<unsigned long long>() + 2, mx.as<unsigned long long>(), (const Fr*)A, N);      // one pass over A for both of its figures
+        }
         ZK_LAUNCH_CHECK();
         void* stage = nullptr;
         int rc = staging(&stage, 24);
@@ -748,13 +886,12 @@ static int matmul_dispatch(void* C, const void* A, const void* B, uint32_t batch
         return 0;
     }
     if (path_used) *path_used = 2;
-    // large products go to the matrix cores as int8 digit planes; below ~1 G multiply-accumulates (over the whole stack)
-    // the conversions outweigh the gain (ZKLLM_MATMUL_PLANES: log2 of that threshold, 0 = never)
-    const char* planes_env = getenv("ZKLLM_MATMUL_PLANES");           // read at every call: tests lower it around single products
-    const int planes_log2 = planes_env ? atoi(planes_env) : 30;
-    if (planes_log2 > 0 && (unsigned __int128)batch * M * N * P >= ((unsigned __int128)1 << planes_log2) && M >= 32 && P >= 32) {
+    // products of small integers go to the matrix cores as int8 digit planes, whatever their size: 300 x 1000 x 2750 takes 217 us on the
+    // vector units and 40 us there, and 16 x 64 x 64 no longer than on the vector units
+    if (planes_wanted) {
         bool done = false;
-        const int rc = run_int8_plane_path(C, A, B, batch, M, N, P, ma_, mb_, st, &done, rhs, src, C64, b_transposed);
+        const int rc = run_int8_plane_path(C, A, B, batch, M, N, P, ma_, mb_, st, &done, rhs, src, C64, b_transposed,
+                                           planes4[0] ? planes4[0]->as<int8_t>() : nullptr, planes4[1] ? planes4[1]->as<int8_t>() : nullptr);
         if (rc) return rc;
         if (done) return 0;
     }
