@@ -210,6 +210,59 @@ ZK_HD bool fq29_is_zero_mod_p(const Fq29& a) {
     return fq29_is_kp(a, k);
 }
 
+// a - b, limb by limb without the carry pass: limbs within +-2^29, for operands of products alone
+ZK_HD Fq29 fq29_sub_raw(const Fq29& a, const Fq29& b) {
+    Fq29 r;
+#pragma unroll
+    for (int i = 0; i < 14; ++i) r.l[i] = a.l[i] - b.l[i];
+    return r;
+}
+// a + p where a is negative
+ZK_HD Fq29 fq29_lift(const Fq29& a) {
+    const int32_t neg = a.l[13] >> 31;
+    Fq29 r;
+    int32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) {
+        const int32_t s = a.l[i] + (fq29_p(i) & neg) + c;
+        r.l[i] = (int32_t)((uint32_t)s & M29);
+        c = s >> 29;
+    }
+    r.l[13] = a.l[13] + (fq29_p(13) & neg) + c;
+    return r;
+}
+// a - b - 2 c in one carry pass
+ZK_HD Fq29 fq29_sub2(const Fq29& a, const Fq29& b, const Fq29& c) {
+    Fq29 r;
+    int32_t k = 0;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) {
+        const int32_t s = a.l[i] - b.l[i] - 2 * c.l[i] + k;
+        r.l[i] = (int32_t)((uint32_t)s & M29);
+        k = s >> 29;
+    }
+    r.l[13] = a.l[13] - b.l[13] - 2 * c.l[13] + k;
+    return r;
+}
+// (a b - c d) / 2^406 mod p with one reduction.  a, b: limbs within +-2^29; c, d: normalised (limbs 0..12 not negative).  A column
+// lies within 28 * 2^58 either way: -28 when a b is at its lowest and nothing is added back, +28 with a b and the reduction's at
+// their highest.
+ZK_HD Fq29 fq29_mul_sub(const Fq29& a, const Fq29& b, const Fq29& c, const Fq29& d) {
+    Fq29 n;
+#pragma unroll
+    for (int i = 0; i < 14; ++i) n.l[i] = -c.l[i];
+    return fq29_redc([&](int k) {
+        int64_t s = 0;
+#pragma unroll
+        for (int i = 0; i < 14; ++i)
+            if (k - i >= 0 && k - i < 14) s += (int64_t)a.l[i] * b.l[k - i];
+#pragma unroll
+        for (int i = 0; i < 14; ++i)
+            if (k - i >= 0 && k - i < 14) s += (int64_t)n.l[i] * d.l[k - i];
+        return s;
+    });
+}
+
 // ---- conversion from / to the 32-bit Montgomery form (R = 2^384, canonical) ---------------------------------------
 ZK_HD Fq29 fq29_repack(const Fp& a) {                   // same integer, 29-bit limbs
     Fq29 r;
@@ -343,6 +396,46 @@ FQ29_POINT_FN J29 j29_add(const J29& a, const J29& b) {
         if (fq29_is_zero_mod_p(rr0)) r = j29_double(a);
         else r = j29_infinity();
     }
+    return r;
+}
+// Points as (X / ZZ, Y / ZZZ) with ZZ^3 = ZZZ^2, for long sums of affine points: a mixed addition (madd-2008-s, dbl-2008-s-1 and
+// mdbl-2008-s-1 of the explicit-formulas database) takes six products, two squares and one reduction over two products -- about 4700
+// instructions against 5700 of the Jacobian one, whose squares and carry passes it does without.
+struct X29 { Fq29 x, y, zz, zzz; uint32_t inf; };
+ZK_HD X29 x29_infinity() { X29 r; r.x = r.y = r.zz = r.zzz = fq29_zero(); r.inf = 1u; return r; }
+ZK_HD void x29_add_mixed(X29& a, const A29& b) {
+    const Fq29 u2 = fq29_mul_inline(b.x, a.zz), s2 = fq29_mul_inline(b.y, a.zzz);
+    const Fq29 h = fq29_sub_raw(u2, a.x), rr = fq29_sub_raw(s2, a.y);
+    const Fq29 hh = fq29_sqr_inline(h), hhh = fq29_mul_inline(h, hh), q = fq29_mul_inline(a.x, hh);
+    X29 r;
+    r.inf = 0u;
+    r.x = fq29_sub2(fq29_sqr_inline(rr), hhh, q);
+    r.y = fq29_mul_sub(rr, fq29_sub_raw(q, r.x), a.y, hhh);
+    r.zz = fq29_mul_inline(a.zz, hh);
+    r.zzz = fq29_mul_inline(a.zzz, hhh);
+    // equal abscissae: hh, a product, is 0 or p (or its neighbourhood's only other multiples of p); the low limb rules that out
+    // except with probability 2^-28
+    if (!a.inf && (hh.l[0] == 0 || hh.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(hh)) {
+        const Fq29 r0 = fq29_sub(s2, a.y);
+        if (fq29_is_zero_mod_p(r0)) {                  // the same point: its double
+            const Fq29 u = fq29_dbl(a.y), v = fq29_sqr(u), w = fq29_mul(u, v), s = fq29_mul(a.x, v), xx = fq29_sqr(a.x), m = fq29_add(fq29_dbl(xx), xx);
+            r.x = fq29_sub(fq29_sqr(m), fq29_dbl(s));
+            r.y = fq29_sub(fq29_mul(m, fq29_sub(s, r.x)), fq29_mul(w, a.y));
+            r.zz = fq29_mul(v, a.zz);
+            r.zzz = fq29_mul(w, a.zzz);
+            if (fq29_is_zero_mod_p(u)) r.inf = 1u;     // a point of order two
+        } else r.inf = 1u;
+    }
+    if (a.inf) { r.x = b.x; r.y = b.y; r.zz = fq29_one(); r.zzz = fq29_one(); }
+    a = r;
+}
+// the same point in Jacobian form, with z = zzz
+FQ29_POINT_FN J29 j29_from_x29(const X29& p) {
+    J29 r;
+    r.inf = p.inf;
+    r.x = fq29_mul(p.x, fq29_sqr(p.zz));
+    r.y = fq29_mul(p.y, fq29_sqr(p.zzz));
+    r.z = p.zzz;
     return r;
 }
 ZK_HD J29 j29_from_jac(const G1Jac& p) {

@@ -11,6 +11,7 @@
 // per-pair doublings and no materialised m*n temporary (the reference writes 144 B per pair).
 // All of it is VALU integer work on 12-limb Fp; results equal the reference's as group elements
 // (a Jacobian triple depends on the order of additions, so bytes are compared after normalising).
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <memory>
@@ -177,10 +178,9 @@ __global__ void __launch_bounds__(256) k_g1aff_to_a29(A29* __restrict__ out, con
 // filled part of every row, row[k + i] = row[i] + row[k - 1] for i < k, k = 1, 2, 4, ...: one launch per k with one lane
 // per new entry, so every launch is dense whatever the row length (rows are as short as 4 entries when few tensor rows
 // share the generators) and the chain of additions is log2(half) deep.
-__global__ void __launch_bounds__(GT) k_msm_table_bases(G1Jac* __restrict__ tab, const G1Jac* __restrict__ gens, size_t ngen, uint32_t c, uint32_t nwin) {
+__global__ void __launch_bounds__(GT) k_msm_table_bases(G1Jac* __restrict__ tab, const G1Jac* __restrict__ gens, size_t ngen, uint32_t c, uint32_t nwin, uint32_t half) {
     const size_t j = (size_t)blockIdx.x * GT + threadIdx.x;
     if (j >= ngen) return;
-    const uint32_t half = 1u << (c - 1);
     G1Jac base = gens[j];
     for (uint32_t w = 0; w < nwin; ++w) {
         tab[((size_t)w * ngen + j) * half] = base;
@@ -194,37 +194,169 @@ __global__ void __launch_bounds__(GT) k_msm_table_fill(G1Jac* __restrict__ tab, 
     G1Jac* row = tab + ((t >> logk) << logh);
     row[k + i] = g1_add(row[i], row[k - 1]);
 }
-// One workgroup per (row, segment): sum_j [s_j] G_j over the segment as mixed additions out of the
-// affine table, in 29-bit limbs (the table is converted once per call).  Scalars are embedded int32 values
-// (commit_int_dev_func, commitment.cu:31-42).
-__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_msm_rows(G1Jac* __restrict__ out, const A29* __restrict__ tab, const int32_t* __restrict__ scalars, size_t ngen, uint32_t c, uint32_t nwin, uint32_t nseg) {
-    const size_t row = blockIdx.x;
-    const uint32_t seg = blockIdx.y;
-    const uint32_t half = 1u << (c - 1);
-    const size_t per = (ngen + nseg - 1) / nseg;
-    const size_t j0 = seg * per, j1 = (j0 + per < ngen) ? j0 + per : ngen;
-    J29 acc29 = j29_infinity();
-    for (size_t j = j0 + threadIdx.x; j < j1; j += GT) {
-        const int32_t s = scalars[row * ngen + j];
-        if (s == 0) continue;
-        const bool negs = s < 0;
-        uint64_t x = negs ? (uint64_t)(-(int64_t)s) : (uint64_t)s;
-        for (uint32_t w = 0; w < nwin && x != 0; ++w) {
-            int64_t d = (int64_t)(x & ((1u << c) - 1));
-            x >>= c;
-            if (d > (int64_t)half) { d -= (int64_t)(1u << c); x += 1; }
-            if (d == 0) continue;
-            const bool nd = (d < 0) != negs;
-            const uint32_t mag = (uint32_t)(d < 0 ? -d : d);
-            A29 p = tab[((size_t)w * ngen + j) * half + (mag - 1)];
-            if (a29_is_inf(p)) continue;
-            if (nd) p.y = fq29_neg(p.y);
-            acc29 = j29_add_mixed(acc29, p);
-        }
+// ---- commit_int: the table in affine 29-bit limbs, and the sums over rows -----------------------------------------------------------
+// Window w of generator j: the multiples d 2^(c w) G_j, d = 1 .. E_w at tab[off_w + j E_w + d - 1].  E_w is 2^(c-1), in the highest window
+// what the largest scalar needs (a power of two).
+struct MsmTable { A29* tab; size_t ngen; uint32_t c, nwin, half, top; };
+__device__ __forceinline__ size_t msm_slot(const MsmTable& T, uint32_t w, size_t j, uint32_t d) {
+    const bool last = w + 1 == T.nwin;
+    return (size_t)w * T.ngen * T.half + j * (last ? T.top : T.half) + (d - 1);
+}
+// the windows' first entries out of the normalised bases (window-major)
+__global__ void __launch_bounds__(256) k_msm_table_place(const MsmTable T, const G1Affine* __restrict__ bases) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= T.ngen * T.nwin) return;
+    const uint32_t w = (uint32_t)(i / T.ngen);
+    T.tab[msm_slot(T, w, i - (size_t)w * T.ngen, 1u)] = a29_from_affine(bases[i]);
+}
+// Entries k + 1 .. 2 k of every window that has them, entry k + i = entry i + entry k: affine additions, whose slopes share an inversion
+// among the CH entries of a lane (an inversion costs a lane about thirteen products, the rest of an entry six).  The entry of the
+// same multiple is a doubling; infinity and opposite points are told apart from the coordinates, whatever the generators are.
+template <int CH> __global__ void __launch_bounds__(GT) k_msm_table_grow(const MsmTable T, uint32_t logk, size_t rows_full, size_t rows) {
+    const uint32_t k = 1u << logk;
+    const size_t n = rows << logk, base = (size_t)blockIdx.x * GT * CH + threadIdx.x;
+    if (base >= n) return;
+    auto row_of = [&](size_t t) {
+        const size_t r = t >> logk;
+        return r < rows_full ? T.tab + r * T.half : T.tab + rows_full * T.half + (r - rows_full) * T.top;
+    };
+    // 0: slope over dx, 1: doubling, 2: a (b is infinity), 3: b, 4: infinity
+    auto kind_of = [&](const A29& a, const A29& b, Fq29& den) {
+        den = fq29_one();
+        if (a29_is_inf(a)) return 3u;
+        if (a29_is_inf(b)) return 2u;
+        const Fq29 dx = fq29_sub(a.x, b.x);
+        if (!fq29_is_zero_mod_p(dx)) { den = dx; return 0u; }
+        const Fq29 y2 = fq29_dbl(a.y);
+        if (!fq29_is_zero_mod_p(fq29_sub(a.y, b.y)) || fq29_is_zero_mod_p(y2)) return 4u;
+        den = y2;
+        return 1u;
+    };
+    Fq29 pre[CH], run = fq29_one();
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const size_t t = base + (size_t)c * GT;
+        pre[c] = run;
+        if (t >= n) continue;
+        const A29* row = row_of(t);
+        Fq29 den;
+        (void)kind_of(row[t & (k - 1)], row[k - 1], den);
+        run = fq29_mul(run, den);
     }
-    const G1Jac acc = block_sum_g1(j29_to_jac(acc29));
-    if (threadIdx.x == 0) out[row * nseg + seg] = acc;
+    Fq29 inv = fq29_from_fp(mont_inverse(fq29_to_fp(run)));
+#pragma unroll
+    for (int c = CH - 1; c >= 0; --c) {
+        const size_t t = base + (size_t)c * GT;
+        if (t >= n) continue;
+        A29* row = const_cast<A29*>(row_of(t));
+        const A29 a = row[t & (k - 1)], b = row[k - 1];
+        Fq29 den;
+        const uint32_t kind = kind_of(a, b, den);
+        const Fq29 di = fq29_mul(inv, pre[c]);
+        inv = fq29_mul(inv, den);
+        Fq29 num;
+        if (kind == 1u) { const Fq29 xx = fq29_sqr(a.x); num = fq29_add(fq29_dbl(xx), xx); }
+        else num = fq29_sub_raw(a.y, b.y);
+        const Fq29 l = fq29_mul(num, di);
+        A29 r;
+        // back to (-eps, p + eps): the coordinates must not grow with the table
+        r.x = fq29_lift(fq29_lift(fq29_sub(fq29_sub(fq29_sqr(l), a.x), b.x)));
+        r.y = fq29_lift(fq29_sub(fq29_mul(l, fq29_sub_raw(a.x, r.x)), a.y));
+        if (kind == 2u) r = a;
+        if (kind == 3u) r = b;
+        if (kind == 4u) { r.x = fq29_zero(); r.y = fq29_zero(); }
+        row[k + (t & (k - 1))] = r;
+    }
+}
+// Sums of [s_j] G_j over segments of the rows (item = segment * m + row, so that a wave's items use the same part of the table), to
+// out[row * nseg + segment].  Sixteen lanes take an item, four items a wave.
+// The scalars' non-zero digits go through a list in LDS, sixteen scalars at a time, and an addition starts when every item of the wave
+// has sixteen: where the second digit of most scalars is zero, lanes that each walked their own scalar's digits would wait for the one
+// in sixty-four that is not.  Sixteen lanes and not the whole wave, because a sum over the lanes of one row is serial: its levels
+// serve four rows at once and are four instead of six.
+// Instruction issue binds it (two waves a SIMD).  11008 rows of 4096 14-bit scalars: 7-bit signed digits of the whole wave's lanes, in
+// Jacobian coordinates, took 17.7 ms; 12-bit digits this way take less than half.
+static constexpr uint32_t MSM_CAP = 256;
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_msm_rows(G1Jac* __restrict__ out, const MsmTable T, const int32_t* __restrict__ scalars, size_t m_rows, uint32_t nseg, uint32_t per) {
+    __shared__ uint32_t list[4][MSM_CAP];
+    __shared__ int32_t sums[43][GT];
+    const uint32_t t = threadIdx.x, grp = t >> 4, ln = t & 15u;
+    const size_t item = (size_t)blockIdx.x * 4 + grp;
+    const bool valid = item < m_rows * nseg;
+    const size_t seg = valid ? item / m_rows : 0, row = valid ? item - seg * m_rows : 0, j0 = valid ? seg * per : 0;
+    const size_t j1 = valid ? (j0 + per < T.ngen ? j0 + per : T.ngen) : 0;
+    const int32_t* src = scalars + row * T.ngen;
+    uint32_t cnt = 0;
+    X29 acc = x29_infinity();
+    const uint32_t room = MSM_CAP - 16u * T.nwin, steps = (per + 15u) / 16u;
+    auto least = [&] {
+        const int v = valid ? (int)cnt : 0x7fffffff;
+        return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)), min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+    };
+    auto most = [&] {
+        const int v = (int)cnt;
+        return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)), max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+    };
+    int32_t s_next = j0 + ln < j1 ? src[j0 + ln] : 0;
+    for (uint32_t step = 0; step <= steps; ++step) {
+        if (step < steps) {
+            const size_t j = j0 + (size_t)step * 16u + ln;
+            const int32_t s = s_next;
+            s_next = j + 16u < j1 ? src[j + 16u] : 0;
+            const bool negs = s < 0;
+            uint64_t x = negs ? (uint64_t)(-(int64_t)s) : (uint64_t)s;
+            for (uint32_t w = 0; w < T.nwin; ++w) {
+                if (__ballot(x != 0) == 0ull) break;
+                int32_t d = (int32_t)(x & (((uint64_t)1 << T.c) - 1));
+                x >>= T.c;
+                if (d > (int32_t)T.half && w + 1 < T.nwin) { d -= (int32_t)(1u << T.c); x += 1; }
+                const uint32_t m = (uint32_t)(__ballot(d != 0) >> (16u * grp)) & 0xFFFFu;
+                if (d != 0) list[grp][cnt + __popc(m & ((1u << ln) - 1u))] = (uint32_t)msm_slot(T, w, j, (uint32_t)(d < 0 ? -d : d)) | ((d < 0) != negs ? 0x80000000u : 0u);
+                cnt += __popc(m);
+            }
+        }
+        __syncthreads();
+        const bool drain = step == steps;
+        for (;;) {
+            const int mx = most();
+            if (drain ? mx == 0 : !(least() >= 16 || mx > (int)room)) break;
+            const uint32_t take = cnt < 16u ? cnt : 16u;
+            cnt -= take;
+            if (ln < take) {
+                const uint32_t e = list[grp][cnt + ln];
+                A29 p = T.tab[e & 0x7FFFFFFFu];
+                if (!a29_is_inf(p)) {
+                    if (e >> 31) p.y = fq29_neg(p.y);
+                    x29_add_mixed(acc, p);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    J29 v = j29_from_x29(acc);
+    for (uint32_t s = 8; s > 0; s >>= 1) {
+        const int32_t* w = reinterpret_cast<const int32_t*>(&v);
+#pragma unroll
+        for (int l = 0; l < 43; ++l) sums[l][t] = w[l];
+        __syncthreads();
+        J29 o;
+        int32_t* wo = reinterpret_cast<int32_t*>(&o);
+        const uint32_t from = (t & 48u) | ((ln + s) & 15u);
+#pragma unroll
+        for (int l = 0; l < 43; ++l) wo[l] = sums[l][from];
+        v = j29_add(v, o);
+        __syncthreads();
+    }
+    if (valid && ln == 0) out[row * nseg + seg] = j29_to_jac(v);
+}
+// out[row] = the sum of row's few parts, a lane a row
+__global__ void __launch_bounds__(GT) k_msm_parts(G1Jac* __restrict__ out, const G1Jac* __restrict__ part, size_t m_rows, uint32_t nseg) {
+    const size_t row = (size_t)blockIdx.x * GT + threadIdx.x;
+    if (row >= m_rows) return;
+    J29 s = j29_from_jac(part[row * nseg]);
+    for (uint32_t i = 1; i < nseg; ++i) s = j29_add(s, j29_from_jac(part[row * nseg + i]));
+    out[row] = j29_to_jac(s);
 }
 // out[i] = [s_i] B for one base point B: additions out of the table of B's multiples d * 2^(8w) B, d = 1..128, w = 0..32
 // (signed 8-bit digits of the 256-bit integer s_i; window 32 only ever holds the last carry).  33 mixed additions at
@@ -249,28 +381,44 @@ k_g1_fixed_base_mul(G1Jac* __restrict__ out, const A29* __restrict__ tab, const 
     }
     out[i] = j29_to_jac(acc29);
 }
-__global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__ out, uint32_t* __restrict__ bad, uint32_t* __restrict__ maxabs, const Fr* __restrict__ in, size_t n) {
-    __shared__ uint32_t wmax[4];
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    uint32_t a = 0;
-    if (i < n) {
-        const Fr x = in[i];
-        // scalar_to_int semantics: values outside the int32 embedding collapse to what the reference reads
-        const int32_t v = fr_to_i32(x);
-        out[i] = v;
-        const Fr back = fr_from_i64((int64_t)v);
-        if (!equal(back, x)) atomicOr(bad, 1u);
-        a = v < 0 ? (uint32_t)(-(int64_t)v) : (uint32_t)v;
+// stats[0]: raised when an element is not the embedding of an int32, [1]: largest magnitude, [2 + b]: of the elements looked at (one in
+// CONV_SAMPLE), those whose magnitude has b bits.  Eight elements a lane in flight: one a lane and an atomic a workgroup ran at 0.8 TB/s
+static constexpr int CONV_SAMPLE = 8, CONV_STATS = 35;
+__global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__ out, uint32_t* __restrict__ stats, const Fr* __restrict__ in, size_t n) {
+    __shared__ uint32_t wmax[4], wbad[4], hist[33];
+    if (threadIdx.x < 33u) hist[threadIdx.x] = 0u;
+    __syncthreads();
+    uint32_t a = 0, bad = 0;
+    const size_t stride = (size_t)gridDim.x * 256;
+    for (size_t i0 = (size_t)blockIdx.x * 256 + threadIdx.x; i0 < n; i0 += CONV_SAMPLE * stride) {
+        Fr x[CONV_SAMPLE];
+#pragma unroll
+        for (int q = 0; q < CONV_SAMPLE; ++q) x[q] = i0 + q * stride < n ? in[i0 + q * stride] : big_zero<8>();
+#pragma unroll
+        for (int q = 0; q < CONV_SAMPLE; ++q) {
+            // scalar_to_int semantics: values outside the int32 embedding collapse to what the reference reads
+            const int32_t v = fr_to_i32(x[q]);
+            if (i0 + q * stride < n) out[i0 + q * stride] = v;
+            bad |= equal(fr_from_i64((int64_t)v), x[q]) ? 0u : 1u;
+            const uint32_t m = v < 0 ? (uint32_t)(-(int64_t)v) : (uint32_t)v;
+            a = m > a ? m : a;
+            if (q == 0) atomicAdd(&hist[m ? 32 - __clz((int)m) : 0], 1u);
+        }
     }
-    // one atomic per workgroup: the largest magnitude of its 256 values
-    for (int off = 32; off >= 1; off >>= 1) { const uint32_t o = (uint32_t)__shfl_xor((int)a, off, 64); a = o > a ? o : a; }
-    if ((threadIdx.x & 63u) == 0) wmax[threadIdx.x >> 6] = a;
+    for (int off = 32; off >= 1; off >>= 1) {
+        const uint32_t o = (uint32_t)__shfl_xor((int)a, off, 64);
+        a = o > a ? o : a;
+        bad |= (uint32_t)__shfl_xor((int)bad, off, 64);
+    }
+    if ((threadIdx.x & 63u) == 0) { wmax[threadIdx.x >> 6] = a; wbad[threadIdx.x >> 6] = bad; }
     __syncthreads();
     if (threadIdx.x == 0) {
         uint32_t m = wmax[0];
-        for (int k = 1; k < 4; ++k) m = wmax[k] > m ? wmax[k] : m;
-        if (m) atomicMax(maxabs, m);
+        for (int k = 1; k < 4; ++k) { m = wmax[k] > m ? wmax[k] : m; bad |= wbad[k]; }
+        if (m > __atomic_load_n(&stats[1], __ATOMIC_RELAXED)) atomicMax(&stats[1], m);
+        if (bad | wbad[0]) atomicOr(&stats[0], 1u);
     }
+    if (threadIdx.x < 33u && hist[threadIdx.x]) atomicAdd(&stats[2 + threadIdx.x], hist[threadIdx.x]);
 }
 
 // ---- opening (Commitment::me_open, commitment.cu:79-129) -------------------------------------------------------------
@@ -1679,6 +1827,44 @@ int zk_g1_normalize(void* out, const void* in, size_t n, void* st) {
     return 0;
 }
 
+// Digit width, windows and segments for m rows of ngen scalars.  seen[b]: how many of the sampled scalars have b bits.  Estimated times in us:
+// an entry of the table costs 0.12 ns and a level of it 60 us at least (one lane's inversion), a base's doubling 12 us of latency, an
+// addition 0.17 ns; a digit beyond the first is an addition where the scalar reaches it.
+struct MsmShape { uint32_t c, nwin, top, nseg; };
+static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs, const uint32_t* seen) {
+    MsmShape best{0, 0, 0, 1};
+    double best_us = 0, total = 0;
+    for (int b = 0; b <= 32; ++b) total += seen[b];
+    if (total < 1) total = 1;
+    for (uint32_t c = 3; c <= 13; ++c) {
+        const uint32_t nwin = bits == 0 ? 1u : (bits + 1 + c - 1) / c, half = 1u << (c - 1);      // a spare bit for the carry of the signed digits
+        uint64_t most = nwin == 1 ? std::max(1u, maxabs) : ((uint64_t)maxabs >> (c * (nwin - 1))) + 1;
+        uint32_t top = 1;
+        while (top < most) top <<= 1;
+        double digits = 0;
+        for (uint32_t w = 0; w < nwin; ++w) {
+            double reach = 0;
+            for (uint32_t b = w ? c * w : 1; b <= 32; ++b) reach += seen[b];
+            digits += reach / total;
+        }
+        double entries = (double)ngen * ((nwin - 1) * (double)half + top);
+        if (entries * sizeof(A29) > 8e9) continue;
+        uint32_t levels = 0;
+        while ((1u << levels) < (nwin > 1 ? std::max(half, top) : top)) ++levels;
+        const double us = 12.0 * c * (nwin - 1) + 60.0 * levels + entries * 1.2e-4 + (double)m * ngen * digits * 1.7e-4;
+        if (!best.c || us < best_us) { best_us = us; best = MsmShape{c, nwin, top, 1}; }
+    }
+    if (!best.c) {      // more generators than the budget of the table allows any width for
+        best.c = 3; best.nwin = bits == 0 ? 1u : (bits + 3) / 3;
+        const uint64_t most = best.nwin == 1 ? std::max(1u, maxabs) : ((uint64_t)maxabs >> (3 * (best.nwin - 1))) + 1;
+        for (best.top = 1; best.top < most; best.top <<= 1) {}
+    }
+    // segments of a row: items (sixteen lanes each) for two waves a SIMD while they keep 32 generators each, and for eight where they keep 512
+    // (a launch of 1.3 times the waves that fit leaves the chip half empty at its end; the sum over an item's lanes costs ten additions)
+    while ((m * best.nseg * 2 <= 8192 && ngen / (best.nseg * 2) >= 32) || (m * best.nseg < 32768 && ngen / (best.nseg * 2) >= 512)) best.nseg *= 2;
+    return best;
+}
+
 // Commitment::commit_int (commitment.cu:50-58): out[row] = sum_j [t[row,j]] gens[j], t = embedded int32 values.
 // scalars: Fr tensor of m*ngen elements.  Values outside the int32 embedding are rejected.
 int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t m, size_t ngen, void* stv) {
@@ -1687,49 +1873,54 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     ZK_ARG(ngen >= 1, "zk_g1_commit_int: no generators");
     ZK_ARG(m <= 0x7fffffffu, "zk_g1_commit_int: too many rows");
     const size_t total = m * ngen;
-    Scratch ints(sizeof(int32_t) * total, st), flags(8, st);
+    Scratch ints(sizeof(int32_t) * total, st), stats(4 * CONV_STATS, st);
     if (ints.rc) return ints.rc;
-    if (flags.rc) return flags.rc;
-    ZK_HIP(hipMemsetAsync(flags.p, 0, 8, st));
-    hipLaunchKernelGGL(k_fr_to_i32_checked, dim3(cdiv(total, 256)), dim3(256), 0, st, ints.as<int32_t>(), flags.as<uint32_t>(), flags.as<uint32_t>() + 1, (const Fr*)scalars_fr, total);
+    if (stats.rc) return stats.rc;
+    ZK_HIP(hipMemsetAsync(stats.p, 0, 4 * CONV_STATS, st));
+    hipLaunchKernelGGL(k_fr_to_i32_checked, dim3((unsigned)std::min<size_t>(cdiv(total, 256), 4096)), dim3(256), 0, st, ints.as<int32_t>(), stats.as<uint32_t>(), (const Fr*)scalars_fr, total);
     ZK_LAUNCH_CHECK();
     void* stage = nullptr;
-    int rc = staging(&stage, 8);
+    int rc = staging(&stage, 4 * CONV_STATS);
     if (rc) return rc;
-    ZK_HIP(hipMemcpyAsync(stage, flags.p, 8, hipMemcpyDeviceToHost, st));
+    ZK_HIP(hipMemcpyAsync(stage, stats.p, 4 * CONV_STATS, hipMemcpyDeviceToHost, st));
     ZK_HIP(hipStreamSynchronize(st));
-    const uint32_t bad = ((uint32_t*)stage)[0], maxabs = ((uint32_t*)stage)[1];
-    ZK_ARG(bad == 0, "zk_g1_commit_int: a scalar is not the embedding of an int32 value");
-    // window width: wide tables pay off when many rows share the generators
-    const uint32_t c = (m >= 256) ? 8u : (m >= 16 ? 5u : 3u);
+    uint32_t seen[CONV_STATS];
+    memcpy(seen, stage, sizeof(seen));
+    const uint32_t maxabs = seen[1];
+    ZK_ARG(seen[0] == 0, "zk_g1_commit_int: a scalar is not the embedding of an int32 value");
     uint32_t bits = 0;
     while (bits < 32 && (maxabs >> bits)) ++bits;
-    uint32_t nwin = (bits + 1 + c - 1) / c;   // one spare bit for the signed-digit carry
-    if (nwin == 0) nwin = 1;
-    const uint32_t half = 1u << (c - 1);
-    const size_t tab_n = (size_t)nwin * ngen * half;
-    Scratch tabj(sizeof(G1Jac) * tab_n, st), taba(sizeof(G1Affine) * tab_n, st);
-    if (tabj.rc) return tabj.rc;
-    if (taba.rc) return taba.rc;
-    hipLaunchKernelGGL(k_msm_table_bases, dim3(cdiv(ngen, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (const G1Jac*)gens, ngen, c, nwin);
-    for (uint32_t logk = 0; logk + 1 < c; ++logk)
-        hipLaunchKernelGGL(k_msm_table_fill, dim3(cdiv(((size_t)nwin * ngen) << logk, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (size_t)nwin * ngen, c - 1, logk);
-    g1_normalize_queue<true>(taba.p, tabj.as<G1Jac>(), tab_n, st);
-    Scratch tab29(sizeof(A29) * tab_n, st);
-    if (tab29.rc) return tab29.rc;
-    hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(tab_n, 256)), dim3(256), 0, st, tab29.as<A29>(), taba.as<G1Affine>(), tab_n);
-    ZK_LAUNCH_CHECK();
-    uint32_t nseg = 1;
-    if (m < 2048) { nseg = (uint32_t)(2048 / m); const uint32_t cap = (uint32_t)((ngen + GT - 1) / GT); if (nseg > cap) nseg = cap; if (nseg < 1) nseg = 1; }
-    if (nseg == 1) {
-        hipLaunchKernelGGL(k_msm_rows, dim3((unsigned)m, 1), dim3(GT), 0, st, (G1Jac*)out, tab29.as<A29>(), ints.as<int32_t>(), ngen, c, nwin, 1u);
-        ZK_LAUNCH_CHECK();
-        return 0;
+    const MsmShape shape = msm_shape(m, ngen, bits, maxabs, seen + 2);
+    MsmTable T;
+    T.ngen = ngen; T.c = shape.c; T.nwin = shape.nwin; T.half = 1u << (shape.c - 1); T.top = shape.top;
+    const size_t nbase = (size_t)T.nwin * ngen, tab_n = (size_t)(T.nwin - 1) * ngen * T.half + ngen * T.top;
+    ZK_ARG(tab_n < ((size_t)1 << 31), "zk_g1_commit_int: too many generators");
+    Scratch tab(sizeof(A29) * tab_n, st), basej(sizeof(G1Jac) * nbase, st), basea(sizeof(G1Affine) * nbase, st);
+    if (tab.rc) return tab.rc;
+    if (basej.rc) return basej.rc;
+    if (basea.rc) return basea.rc;
+    T.tab = tab.as<A29>();
+    hipLaunchKernelGGL(k_msm_table_bases, dim3(cdiv(ngen, GT)), dim3(GT), 0, st, basej.as<G1Jac>(), (const G1Jac*)gens, ngen, T.c, T.nwin, 1u);
+    g1_normalize_queue<true>(basea.p, basej.as<G1Jac>(), nbase, st);
+    hipLaunchKernelGGL(k_msm_table_place, dim3(cdiv(nbase, 256)), dim3(256), 0, st, T, basea.as<G1Affine>());
+    const size_t rows_full = (size_t)(T.nwin - 1) * ngen;
+    for (uint32_t logk = 0; (1u << logk) < std::max(T.top, T.nwin > 1 ? T.half : 1u); ++logk) {
+        const bool with_top = (1u << logk) < T.top;
+        // the windows below the highest are never shorter than it, but a single window is the highest
+        const size_t rows = (T.nwin > 1 ? rows_full : 0) + (with_top ? ngen : 0), n = rows << logk;
+        if (n == 0) continue;
+        // entries a lane: one until every lane of two waves a SIMD has one
+        if (n < ((size_t)1 << 18)) hipLaunchKernelGGL(k_msm_table_grow<1>, dim3(cdiv(n, (size_t)GT)), dim3(GT), 0, st, T, logk, rows_full, rows);
+        else if (n < ((size_t)1 << 19)) hipLaunchKernelGGL(k_msm_table_grow<2>, dim3(cdiv(n, (size_t)GT * 2)), dim3(GT), 0, st, T, logk, rows_full, rows);
+        else hipLaunchKernelGGL(k_msm_table_grow<4>, dim3(cdiv(n, (size_t)GT * 4)), dim3(GT), 0, st, T, logk, rows_full, rows);
     }
-    Scratch part(sizeof(G1Jac) * m * nseg, st);
+    ZK_LAUNCH_CHECK();
+    const size_t per = (ngen + shape.nseg - 1) / shape.nseg, items = m * shape.nseg;
+    Scratch part(shape.nseg > 1 ? sizeof(G1Jac) * items : 1, st);
     if (part.rc) return part.rc;
-    hipLaunchKernelGGL(k_msm_rows, dim3((unsigned)m, nseg), dim3(GT), 0, st, part.as<G1Jac>(), tab29.as<A29>(), ints.as<int32_t>(), ngen, c, nwin, nseg);
-    hipLaunchKernelGGL(k_g1_rowsum, dim3((unsigned)m, 1), dim3(GT), 0, st, (G1Jac*)out, part.as<G1Jac>(), (size_t)nseg, 1u);
+    hipLaunchKernelGGL(k_msm_rows, dim3(cdiv(items, 4)), dim3(GT), 0, st, shape.nseg > 1 ? part.as<G1Jac>() : (G1Jac*)out, T, ints.as<int32_t>(), m, shape.nseg, (uint32_t)per);
+    if (shape.nseg > 16) hipLaunchKernelGGL(k_g1_rowsum, dim3((unsigned)m, 1), dim3(GT), 0, st, (G1Jac*)out, part.as<G1Jac>(), (size_t)shape.nseg, 1u);
+    else if (shape.nseg > 1) hipLaunchKernelGGL(k_msm_parts, dim3(cdiv(m, (size_t)GT)), dim3(GT), 0, st, (G1Jac*)out, part.as<G1Jac>(), m, shape.nseg);
     ZK_LAUNCH_CHECK();
     return 0;
 }
@@ -1757,7 +1948,7 @@ int zk_g1_fixed_base_mul(void* out, const uint32_t* base_host, const void* scala
         if (tabj.rc) return tabj.rc;
         if (taba.rc) return taba.rc;
         ZK_HIP(hipMemcpyAsync(b.p, base_host, sizeof(G1Jac), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(k_msm_table_bases, dim3(1), dim3(GT), 0, st, tabj.as<G1Jac>(), b.as<G1Jac>(), (size_t)1, 8u, FB_WIN);
+        hipLaunchKernelGGL(k_msm_table_bases, dim3(1), dim3(GT), 0, st, tabj.as<G1Jac>(), b.as<G1Jac>(), (size_t)1, 8u, FB_WIN, 128u);
         for (uint32_t logk = 0; logk < 7; ++logk)
             hipLaunchKernelGGL(k_msm_table_fill, dim3(cdiv((size_t)FB_WIN << logk, GT)), dim3(GT), 0, st, tabj.as<G1Jac>(), (size_t)FB_WIN, 7u, logk);
         g1_normalize_queue<true>(taba.p, tabj.as<G1Jac>(), tab_n, st);
