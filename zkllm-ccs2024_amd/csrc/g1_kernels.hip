@@ -210,11 +210,12 @@ __global__ void __launch_bounds__(256) k_msm_table_place(const MsmTable T, const
     T.tab[msm_slot(T, w, i - (size_t)w * T.ngen, 1u)] = a29_from_affine(bases[i]);
 }
 // Entries k + 1 .. 2 k of every window that has them, entry k + i = entry i + entry k: affine additions, whose slopes share an inversion
-// among the CH entries of a lane (an inversion costs a lane about thirteen products, the rest of an entry six).  The entry of the
+// among a lane's entries (an inversion costs a lane about 26 products, the rest of an entry seven).  The entry of the
 // same multiple is a doubling; infinity and opposite points are told apart from the coordinates, whatever the generators are.
-template <int CH> __global__ void __launch_bounds__(GT) k_msm_table_grow(const MsmTable T, uint32_t logk, size_t rows_full, size_t rows) {
+// The products before an entry wait in its slot.
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_grow(const MsmTable T, uint32_t logk, size_t rows_full, size_t rows, uint32_t per_lane) {
     const uint32_t k = 1u << logk;
-    const size_t n = rows << logk, base = (size_t)blockIdx.x * GT * CH + threadIdx.x;
+    const size_t n = rows << logk, base = (size_t)blockIdx.x * GT * per_lane + threadIdx.x;
     if (base >= n) return;
     auto row_of = [&](size_t t) {
         const size_t r = t >> logk;
@@ -232,36 +233,32 @@ template <int CH> __global__ void __launch_bounds__(GT) k_msm_table_grow(const M
         den = y2;
         return 1u;
     };
-    Fq29 pre[CH], run = fq29_one();
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const size_t t = base + (size_t)c * GT;
-        pre[c] = run;
-        if (t >= n) continue;
-        const A29* row = row_of(t);
+    Fq29 run = fq29_one();
+    uint32_t count = 0;
+    for (size_t t = base; count < per_lane && t < n; t += GT, ++count) {
+        A29* row = row_of(t);
         Fq29 den;
         (void)kind_of(row[t & (k - 1)], row[k - 1], den);
-        run = fq29_mul(run, den);
+        row[k + (t & (k - 1))].x = run;
+        run = fq29_mul_inline(run, den);
     }
     Fq29 inv = fq29_from_fp(mont_inverse(fq29_to_fp(run)));
-#pragma unroll
-    for (int c = CH - 1; c >= 0; --c) {
-        const size_t t = base + (size_t)c * GT;
-        if (t >= n) continue;
-        A29* row = const_cast<A29*>(row_of(t));
+    while (count-- > 0) {
+        const size_t t = base + (size_t)count * GT;
+        A29* row = row_of(t);
         const A29 a = row[t & (k - 1)], b = row[k - 1];
         Fq29 den;
         const uint32_t kind = kind_of(a, b, den);
-        const Fq29 di = fq29_mul(inv, pre[c]);
-        inv = fq29_mul(inv, den);
+        const Fq29 di = fq29_mul_inline(inv, row[k + (t & (k - 1))].x);
+        inv = fq29_mul_inline(inv, den);
         Fq29 num;
         if (kind == 1u) { const Fq29 xx = fq29_sqr(a.x); num = fq29_add(fq29_dbl(xx), xx); }
         else num = fq29_sub_raw(a.y, b.y);
-        const Fq29 l = fq29_mul(num, di);
+        const Fq29 l = fq29_mul_inline(num, di);
         A29 r;
         // back to (-eps, p + eps): the coordinates must not grow with the table
-        r.x = fq29_lift(fq29_lift(fq29_sub(fq29_sub(fq29_sqr(l), a.x), b.x)));
-        r.y = fq29_lift(fq29_sub(fq29_mul(l, fq29_sub_raw(a.x, r.x)), a.y));
+        r.x = fq29_lift(fq29_lift(fq29_sub(fq29_sub(fq29_sqr_inline(l), a.x), b.x)));
+        r.y = fq29_lift(fq29_sub(fq29_mul_inline(l, fq29_sub_raw(a.x, r.x)), a.y));
         if (kind == 2u) r = a;
         if (kind == 3u) r = b;
         if (kind == 4u) { r.x = fq29_zero(); r.y = fq29_zero(); }
@@ -707,13 +704,14 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             const uint32_t lenA = cnt[bA] > (uint32_t)MHEAVY ? 0u : cnt[bA], lenB = cnt[bB] > (uint32_t)MHEAVY ? 0u : cnt[bB];
             const uint32_t total = lenA + lenB;
             uint32_t pos = off[bA];
-            J29 acc29 = j29_infinity();
+            X29 acc29 = x29_infinity();
             for (uint32_t i = 0;; ++i) {
                 if (i == lenA) {
                     // the end of the first list: its bucket goes out (added to what earlier chunks of this segment left there)
-                    if (!first) acc29 = j29_add(out[bA], acc29);
-                    out[bA] = acc29;
-                    acc29 = j29_infinity();
+                    J29 v = j29_from_x29(acc29);
+                    if (!first) v = j29_add(out[bA], v);
+                    out[bA] = v;
+                    acc29 = x29_infinity();
                     pos = off[bB];
                 }
                 if (i >= total) break;
@@ -721,10 +719,11 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 A29 pt = A[(size_t)(e0 + (en & 0x7FFFu)) * d.b_mul + d.b_off];
                 if (a29_is_inf(pt)) continue;
                 if (en & 0x8000u) pt.y = fq29_neg(pt.y);
-                acc29 = j29_add_mixed(acc29, pt);
+                x29_add_mixed(acc29, pt);
             }
-            if (!first) acc29 = j29_add(out[bB], acc29);
-            out[bB] = acc29;
+            J29 v = j29_from_x29(acc29);
+            if (!first) v = j29_add(out[bB], v);
+            out[bB] = v;
         }
         __threadfence_block();
         __syncthreads();
@@ -1909,10 +1908,9 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
         // the windows below the highest are never shorter than it, but a single window is the highest
         const size_t rows = (T.nwin > 1 ? rows_full : 0) + (with_top ? ngen : 0), n = rows << logk;
         if (n == 0) continue;
-        // entries a lane: one until every lane of two waves a SIMD has one
-        if (n < ((size_t)1 << 18)) hipLaunchKernelGGL(k_msm_table_grow<1>, dim3(cdiv(n, (size_t)GT)), dim3(GT), 0, st, T, logk, rows_full, rows);
-        else if (n < ((size_t)1 << 19)) hipLaunchKernelGGL(k_msm_table_grow<2>, dim3(cdiv(n, (size_t)GT * 2)), dim3(GT), 0, st, T, logk, rows_full, rows);
-        else hipLaunchKernelGGL(k_msm_table_grow<4>, dim3(cdiv(n, (size_t)GT * 4)), dim3(GT), 0, st, T, logk, rows_full, rows);
+        // entries a lane: one until every lane of two waves a SIMD has one, then as many as leave those waves, up to 32
+        const uint32_t per_lane = (uint32_t)std::min<size_t>(32, std::max<size_t>(1, n >> 17));
+        hipLaunchKernelGGL(k_msm_table_grow, dim3(cdiv(n, (size_t)GT * per_lane)), dim3(GT), 0, st, T, logk, rows_full, rows, per_lane);
     }
     ZK_LAUNCH_CHECK();
     const size_t per = (ngen + shape.nseg - 1) / shape.nseg, items = m * shape.nseg;
