@@ -438,6 +438,99 @@ FQ29_POINT_FN J29 j29_from_x29(const X29& p) {
     r.z = p.zzz;
     return r;
 }
+// ---- Jacobian points for long walks: products inlined, differences that only products read without their carry pass, y with one
+// reduction over two products ----------------------------------------------------------------------------------------------
+template <int SH> ZK_HD Fq29 fq29_shl(const Fq29& a) {      // 2^SH a
+    Fq29 r;
+    int32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) {
+        const uint32_t lo = (uint32_t)a.l[i];                // limbs 0..12 are in [0, 2^29)
+        r.l[i] = (int32_t)(((lo << SH) & M29) | (uint32_t)c);
+        c = (int32_t)(lo >> (29 - SH));
+    }
+    r.l[13] = (int32_t)((uint32_t)a.l[13] << SH) + c;
+    return r;
+}
+// a - 8 b in one carry pass (8 b formed by shifts across the limbs)
+ZK_HD Fq29 fq29_sub8(const Fq29& a, const Fq29& b) { return fq29_sub(a, fq29_shl<3>(b)); }
+// x3 = (3 x^2)^2 - 8 s, y3 = 3 x^2 (4 s - x3) - 8 y^4, z3 = 2 y z with s = x y^2
+ZK_HD void j29_double_walk(J29& p) {
+    const Fq29 a = fq29_sqr_inline(p.x), b = fq29_sqr_inline(p.y), yz = fq29_mul_inline(p.y, p.z);
+    const Fq29 s = fq29_mul_inline(p.x, b), e = fq29_add(fq29_shl<1>(a), a);
+    p.x = fq29_sub8(fq29_sqr_inline(e), s);
+    p.y = fq29_mul_sub(e, fq29_sub_raw(fq29_shl<2>(s), p.x), fq29_shl<3>(b), b);
+    p.z = fq29_shl<1>(yz);
+}
+// madd-2004-hmv
+ZK_HD void j29_add_mixed_walk(J29& a, const A29& b) {
+    const Fq29 zz = fq29_sqr_inline(a.z), u2 = fq29_mul_inline(b.x, zz), s2 = fq29_mul_inline(fq29_mul_inline(b.y, a.z), zz);
+    const Fq29 h = fq29_sub_raw(u2, a.x), rr = fq29_sub_raw(s2, a.y);
+    const Fq29 hh = fq29_sqr_inline(h), hhh = fq29_mul_inline(h, hh), v = fq29_mul_inline(a.x, hh);
+    J29 r;
+    r.inf = 0u;
+    r.z = fq29_mul_inline(a.z, h);
+    r.x = fq29_sub2(fq29_sqr_inline(rr), hhh, v);
+    r.y = fq29_mul_sub(rr, fq29_sub_raw(v, r.x), a.y, hhh);
+    if (!a.inf && (hh.l[0] == 0 || hh.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(hh)) {      // the same point or its opposite
+        if (fq29_is_zero_mod_p(fq29_sub(s2, a.y))) r = j29_double(a);
+        else r.inf = 1u;
+    }
+    if (a.inf) { r.x = b.x; r.y = b.y; r.z = fq29_one(); }
+    a = r;
+}
+#if defined(__HIPCC__)
+// ---- one point on four lanes -------------------------------------------------------------------------------------------------
+// Every lane of four holds the whole point; the independent products of a formula's step go one to a lane and come back by quad
+// permutations.  A doubling is three products deep instead of seven, an addition five instead of sixteen: for chains that a launch
+// waits for while the chip is empty.
+template <int FROM> __device__ __forceinline__ Fq29 quad_get(const Fq29& a) {
+    Fq29 r;
+#pragma unroll
+    for (int i = 0; i < 14; ++i) r.l[i] = __builtin_amdgcn_update_dpp(0, a.l[i], FROM * 0x55, 0xF, 0xF, false);
+    return r;
+}
+__device__ __forceinline__ Fq29 fq29_select(bool c, const Fq29& a, const Fq29& b) {
+    Fq29 r;
+#pragma unroll
+    for (int i = 0; i < 14; ++i) r.l[i] = c ? a.l[i] : b.l[i];
+    return r;
+}
+__device__ __forceinline__ void j29_quad_double(J29& p, uint32_t q) {
+    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 0, p.x, p.y), fq29_select(q == 0, p.x, fq29_select(q == 2, p.z, p.y)));      // x^2 | y^2 | y z | y^2
+    const Fq29 a = quad_get<0>(m1), b = quad_get<1>(m1), yz = quad_get<2>(m1);
+    const Fq29 e = fq29_add(fq29_shl<1>(a), a);
+    const Fq29 m2 = fq29_mul_inline(fq29_select(q == 0, e, fq29_select(q == 1, p.x, b)), fq29_select(q == 0, e, b));                // e^2 | x y^2 | y^4 | y^4
+    const Fq29 s = quad_get<1>(m2), c = quad_get<2>(m2);
+    p.x = fq29_sub8(quad_get<0>(m2), s);
+    p.y = fq29_sub8(fq29_mul_inline(e, fq29_sub_raw(fq29_shl<2>(s), p.x)), c);
+    p.z = fq29_shl<1>(yz);
+}
+__device__ __forceinline__ void j29_quad_add(J29& a, const J29& b, uint32_t q) {
+    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 0, a.z, fq29_select(q == 1, b.z, fq29_select(q == 2, a.y, b.y))),
+                                    fq29_select((q & 1u) != 0, fq29_select(q == 1, b.z, a.z), fq29_select(q == 0, a.z, b.z)));      // z1^2 | z2^2 | y1 z2 | y2 z1
+    const Fq29 z1z1 = quad_get<0>(m1), z2z2 = quad_get<1>(m1);
+    const Fq29 m2 = fq29_mul_inline(fq29_select(q == 0, a.x, fq29_select(q == 1, b.x, m1)), fq29_select((q & 1u) != 0, z1z1, z2z2)); // u1 | u2 | s1 | s2
+    const Fq29 u1 = quad_get<0>(m2), s1 = quad_get<2>(m2);
+    const Fq29 h = fq29_sub_raw(quad_get<1>(m2), u1), rr = fq29_sub_raw(quad_get<3>(m2), s1);
+    const Fq29 m3 = fq29_mul_inline(fq29_select(q == 0, h, fq29_select(q == 1, a.z, rr)), fq29_select(q == 0, h, fq29_select(q == 1, b.z, rr)));      // h^2 | z1 z2 | r^2 | r^2
+    const Fq29 hh = quad_get<0>(m3), zz = quad_get<1>(m3), r2 = quad_get<2>(m3);
+    const Fq29 m4 = fq29_mul_inline(fq29_select(q == 1, u1, fq29_select(q == 2, zz, h)), fq29_select(q == 2, h, hh));                  // h^3 | u1 h^2 | z1 z2 h | h^3
+    const Fq29 hhh = quad_get<0>(m4), v = quad_get<1>(m4);
+    J29 r;
+    r.inf = 0u;
+    r.z = quad_get<2>(m4);
+    r.x = fq29_sub2(r2, hhh, v);
+    r.y = fq29_mul_sub(rr, fq29_sub_raw(v, r.x), s1, hhh);
+    if (a.inf) r = b;
+    else if (b.inf) r = a;
+    else if ((hh.l[0] == 0 || hh.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(hh)) {
+        if ((r2.l[0] == 0 || r2.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(r2)) r = j29_double(a);
+        else r = j29_infinity();
+    }
+    a = r;
+}
+#endif
 ZK_HD J29 j29_from_jac(const G1Jac& p) {
     if (is_zero(p.z)) return j29_infinity();
     J29 r;

@@ -364,7 +364,7 @@ k_g1_fixed_base_mul(G1Jac* __restrict__ out, const A29* __restrict__ tab, const 
     const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i >= n) return;
     const Fr x = scalars[i];
-    J29 acc29 = j29_infinity();
+    X29 acc29 = x29_infinity();
     uint32_t carry = 0;
     for (uint32_t w = 0; w < FB_WIN; ++w) {
         const uint32_t b = (w < 32 ? ((x.v[w >> 2] >> (8 * (w & 3))) & 255u) : 0u) + carry;
@@ -374,9 +374,9 @@ k_g1_fixed_base_mul(G1Jac* __restrict__ out, const A29* __restrict__ tab, const 
         A29 p = tab[w * 128u + (mag - 1)];
         if (a29_is_inf(p)) continue;
         if (carry) p.y = fq29_neg(p.y);
-        acc29 = j29_add_mixed(acc29, p);
+        x29_add_mixed(acc29, p);
     }
-    out[i] = j29_to_jac(acc29);
+    out[i] = j29_to_jac(j29_from_x29(acc29));
 }
 // stats[0]: raised when an element is not the embedding of an int32, [1]: largest magnitude, [2 + b]: of the elements looked at (one in
 // CONV_SAMPLE), those whose magnitude has b bits.  Eight elements a lane in flight: one a lane and an atomic a workgroup ran at 0.8 TB/s
@@ -729,7 +729,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
         __syncthreads();
         for (uint32_t b = 0; b < (uint32_t)MT; ++b) {
             if (cnt[b] <= (uint32_t)MHEAVY) continue;          // the same for every lane
-            J29 h29 = j29_infinity();
+            X29 h29 = x29_infinity();
             for (uint32_t e = e0 + t; e < e1; e += MSL) {
                 const size_t si = (size_t)e * d.s_mul + d.s_off;
                 const int dg = Dw[si];
@@ -737,9 +737,9 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 A29 pt = A[(size_t)e * d.b_mul + d.b_off];
                 if (a29_is_inf(pt)) continue;
                 if ((dg < 0) != (((Df[si] >> half) & 1) != 0)) pt.y = fq29_neg(pt.y);
-                h29 = j29_add_mixed(h29, pt);
+                x29_add_mixed(h29, pt);
             }
-            const J29 h = j29_block_sum<MSL>(pool, h29, t);
+            const J29 h = j29_block_sum<MSL>(pool, j29_from_x29(h29), t);
             if (t == 0) out[b] = j29_add(out[b], h);            // its list was empty: the slot holds what earlier chunks left (or infinity)
         }
         __threadfence_block();
@@ -760,35 +760,62 @@ __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, c
     for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = j29_add(acc, b[(size_t)sg * MT + t]);
     out[((size_t)row * gridDim.y + grp) * MT + t] = acc;
 }
-// The sums of a list from the raw buckets of all their windows, one workgroup per sum: lane t takes bucket (t mod MT) + 1 of one
-// half's windows, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings, the segments of a window added on the way), weights it by
-// its digit, the lanes of the second half apply the endomorphism, and the workgroup's lanes are summed -- one weighting and one
-// lane sum per sum instead of one per window, and no Horner pass of a single lane over window sums afterwards.
-// Raw buckets: buckets[(w nseg + seg) MT + b].  The walk is one lane's chain, so a launch takes what one lane takes whatever the
-// number of sums: all of a job's sums that nothing waits for go into one launch.
-struct PointDesc { const J29* buckets; G1Jac* out; uint32_t nseg, pad; };
-__global__ void __launch_bounds__(2 * MT) k_msm_point(const PointDesc* __restrict__ list) {
-    __shared__ uint32_t pool[J29_WORDS * MT];
-    const uint32_t t = threadIdx.x, half = t / (uint32_t)MT, b = t % (uint32_t)MT;
+// The sums of a list from the raw buckets of all their windows, a workgroup for each half of a sum's windows: four lanes take bucket
+// b + 1, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings, the segments of a window added on the way), weight it by its digit, and
+// the buckets are summed -- one weighting and one lane sum per half instead of one per window, and no Horner pass of a single lane
+// over window sums afterwards.  k_msm_join adds the halves, the endomorphism on the second.
+// Raw buckets: buckets[(w nseg + seg) MT + b]; a half's total goes to its first bucket's place, which only its own workgroup reads.
+// The walk is one chain, so a launch takes what one chain takes whatever the number of sums: all of a job's sums that nothing waits for
+// go into one launch.  On one lane the chain is 1400 products deep, 1.6 ms; four lanes that share a point's products: 0.8 ms.
+struct PointDesc { J29* buckets; G1Jac* out; uint32_t nseg, pad; };
+__global__ void __launch_bounds__(4 * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list) {
+    __shared__ uint32_t pool[J29_WORDS * MT / 2];
+    const uint32_t q = threadIdx.x & 3u, b = threadIdx.x >> 2, half = blockIdx.y;
     const PointDesc d = list[blockIdx.x];
+    J29* const mine = d.buckets + (size_t)half * MWH * d.nseg * MT;
     J29 r = j29_infinity();
     for (int w = MWH - 1; w >= 0; --w) {
         if (__any(!r.inf))
-            for (int k = 0; k < 8; ++k) r = j29_double(r);
-        const J29* row = d.buckets + (size_t)(half * MWH + (uint32_t)w) * d.nseg * MT;
+            for (int k = 0; k < 8; ++k) j29_quad_double(r, q);
+        const J29* row = mine + (size_t)w * d.nseg * MT;
         for (uint32_t sg = 0; sg < d.nseg; ++sg) {
-            const J29 pt = row[(size_t)sg * MT + b];
-            if (!pt.inf) r = j29_add(r, pt);
+            const J29 p = row[(size_t)sg * MT + b];
+            if (__any(!p.inf)) j29_quad_add(r, p, q);
         }
     }
-    J29 q = j29_infinity();
+    J29 s = j29_infinity();
     for (int bit = 7; bit >= 0; --bit) {
-        q = j29_double(q);
-        if (((b + 1) >> bit) & 1u) q = j29_add(q, r);
+        j29_quad_double(s, q);
+        J29 p = r;
+        if (!(((b + 1) >> bit) & 1u)) p.inf = 1u;
+        j29_quad_add(s, p, q);
     }
-    if (half) q.x = fq29_mul(q.x, fq29_from_fp(glv_beta()));
-    q = j29_block_sum<2 * MT>(pool, q, t);
-    if (t == 0) *d.out = j29_to_jac(q);
+    for (uint32_t sd = MT / 2; sd > 0; sd >>= 1) {
+        __syncthreads();
+        if (b >= sd && b < 2 * sd && q == 0) {
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
+#pragma unroll
+            for (int l = 0; l < J29_WORDS; ++l) pool[l * (MT / 2) + b - sd] = src[l];
+        }
+        __syncthreads();
+        if (b < sd) {
+            J29 y;
+            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (MT / 2) + b];
+            j29_quad_add(s, y, q);
+        }
+    }
+    if (threadIdx.x == 0) *mine = s;
+}
+__global__ void __launch_bounds__(GT) k_msm_join(const PointDesc* __restrict__ list, uint32_t n) {
+    const uint32_t i = (blockIdx.x * GT + threadIdx.x) >> 2, q = threadIdx.x & 3u;
+    if (i >= n) return;
+    const PointDesc d = list[i];
+    J29 s = d.buckets[0], y = d.buckets[(size_t)MWH * d.nseg * MT];
+    y.x = fq29_mul(y.x, fq29_from_fp(glv_beta()));
+    j29_quad_add(s, y, q);
+    if (q == 0) *d.out = j29_to_jac(s);
 }
 
 // Sums of an opening's first rounds from commitments of the opened tensor's rows.  The opened vector is the row fold of a
@@ -971,7 +998,7 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
             }
         }
         for (int i = (int)jsf.len - 1; i >= 0; --i) {
-            w = j29_double(w);
+            j29_double_walk(w);
             const uint32_t dg = (jsf.dig[i >> 3] >> ((i & 7) * 4)) & 0xFu;    // (d1 + 1) | (d2 + 1) << 2, the same for every lane
             const int d1 = (int)(dg & 3u) - 1, d2 = (int)(dg >> 2) - 1;
             if (d1 == 0 && d2 == 0) continue;
@@ -992,9 +1019,9 @@ k_open_fold29(const FoldBatch fb, size_t old_size, size_t new_size) {
                 }
             }
             if (negate) t.y = fq29_neg(t.y);
-            w = j29_add_mixed(w, t);
+            j29_add_mixed_walk(w, t);
         }
-        if (!inf1) w = j29_add_mixed(w, a1);
+        if (!inf1) j29_add_mixed_walk(w, a1);
     }
     const A29 o = a29_from_j29(w);
     if (fast) {
@@ -1055,25 +1082,25 @@ k_open_fold_comb(const CombBatch cb, size_t old_size, size_t new_size) {
     if (fast) {
         const Fq29 beta = fq29_from_fp(glv_beta());
         for (int b = COMB_W - 1; b >= 0; --b) {
-            w = j29_double(w);
+            j29_double_walk(w);
 #pragma unroll
             for (int ti = 0; ti < NT; ++ti) {
                 const A29* __restrict__ tb = ti ? tab2 : tab;
                 const uint32_t m1 = ti ? ck2.m1[b] : ck.m1[b], m2 = ti ? ck2.m2[b] : ck.m2[b];          // the same for every lane
                 if (m1) {
                     const A29 t = tb[(size_t)(m1 - 1) * new_size + g];
-                    if (!a29_is_inf(t)) w = j29_add_mixed(w, t);
+                    if (!a29_is_inf(t)) j29_add_mixed_walk(w, t);
                 }
                 if (m2) {
                     A29 t = tb[(size_t)(m2 - 1) * new_size + g];
                     if (!a29_is_inf(t)) {
                         t.x = fq29_mul(t.x, beta);
-                        w = j29_add_mixed(w, t);
+                        j29_add_mixed_walk(w, t);
                     }
                 }
             }
         }
-        if (!inf1) w = j29_add_mixed(w, a1);
+        if (!inf1) j29_add_mixed_walk(w, a1);
     }
     const A29 o = a29_from_j29(w);
     if (fast) new_gens[g] = o;
@@ -1113,47 +1140,47 @@ k_open_fold_jump(const JumpBatch jb, size_t new_size) {
     if (live) {
         const Fq29 beta = fq29_from_fp(glv_beta());
         for (int b = COMB_W - 1; b >= 0; --b) {
-            w = j29_double(w);
+            j29_double_walk(w);
             for (int ti = 0; ti < JUMP_TABS; ++ti) {
                 const A29* __restrict__ tb = it.tab + (size_t)ti * COMB_N * new_size;
                 const uint32_t m1 = it.ck[ti].m1[b], m2 = it.ck[ti].m2[b];          // the same for every lane
                 if (m1) {
                     const A29 t = tb[(size_t)(m1 - 1) * new_size + g];
-                    if (!a29_is_inf(t)) w = j29_add_mixed(w, t);
+                    if (!a29_is_inf(t)) j29_add_mixed_walk(w, t);
                 }
                 if (m2) {
                     A29 t = tb[(size_t)(m2 - 1) * new_size + g];
                     if (!a29_is_inf(t)) {
                         t.x = fq29_mul(t.x, beta);
-                        w = j29_add_mixed(w, t);
+                        j29_add_mixed_walk(w, t);
                     }
                 }
             }
         }
-        if (!inf1) w = j29_add_mixed(w, a1);
+        if (!inf1) j29_add_mixed_walk(w, a1);
     }
     const A29 o = a29_from_j29(w);
     if (live) it.ng[g] = o;
 }
 // ---- three rounds in one without tables ------------------------------------------------------------------------------------------
-// The same combination g^(3)_m = sum_{b<8} c_b g_(8m+b) with nothing prepared: wave b of a workgroup multiplies the b-th generator of
-// 64 results by c_b (one scalar for the wave: the walk of k_open_fold29 over the joint sparse form of the split c_b), and the eight
-// products are added up through LDS.  As much work as three rounds of halving one after the other (8 walks for 7 pairs'), but one
-// walk's latency instead of three: a walk of one wave a SIMD takes 2.4 ms whatever its number of lanes.  65536 generators ... YY.
-struct SpanBatch { A29* ng[OB_MAX]; const A29* g[OB_MAX]; };
+// The same combination g^(3)_m = sum_{b<8} c_b g_(8m+b) with nothing prepared, in two launches.  The joint sparse forms of the eight split
+// c_b are cut into eight slices of `slice` positions.  k_open_span_slices: wave b of a workgroup makes the table of the b-th
+// generator of 64 results (P, phi(P), P - phi(P); P + phi(P) is their x's sum negated), then sums slice b over all eight generators --
+// a walk of `slice` doublings, every digit the same for the wave.  k_open_span_walk: four lanes a result put the slices together, seven
+// times `slice` doublings.  An eighth of the doublings that eight walks beside each other take, and the second launch, whose chain
+// hardly fills the chip, leaves it to the bucket sums.
+struct SpanBatch { A29* ng[OB_MAX]; const A29* g[OB_MAX]; J29* part; };
 __global__ void __launch_bounds__(8 * GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_open_fold_span(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old_size, size_t new_size) {
-    __shared__ int32_t lds[8][4][14][GT];
+k_open_span_slices(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old_size, size_t new_size, uint32_t slice) {
+    __shared__ int32_t tab[8][5][14][GT];      // x, y of P, x of phi(P), x and y of P - phi(P)
+    __shared__ uint8_t flags[8][GT];
     const uint32_t b = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / GT)), t = threadIdx.x % GT;
-    int32_t (*tab)[14][GT] = lds[b];
-    const JsfK& jsf = jsfs[blockIdx.y * 8 + b];
     const size_t m = (size_t)blockIdx.x * GT + t;
-    A29 p;
-    p.x = p.y = fq29_zero();
-    if (m < new_size && 8 * m + b < old_size) p = sb.g[blockIdx.y][8 * m + b];
-    const bool inf = a29_is_inf(p), x0 = !inf && fq29_is_zero_mod_p(p.x);
-    J29 w = j29_infinity();
     {
+        A29 p;
+        p.x = p.y = fq29_zero();
+        if (m < new_size && 8 * m + b < old_size) p = sb.g[blockIdx.y][8 * m + b];
+        const bool inf = a29_is_inf(p), x0 = !inf && fq29_is_zero_mod_p(p.x);
         const Fq29 inv = fq29_inverse((inf || x0) ? fq29_one() : p.x), one29 = fq29_one();
         const Fq29 xQ = fq29_mul(p.x, fq29_from_fp(glv_beta())), xPQ = fq29_mul(p.x, fq29_from_fp(glv_beta2()));
         const Fq29 lam = fq29_mul(fq29_mul(fq29_from_fp(glv_minus2_over_beta_minus_1()), p.y), inv);   // slope of P + (beta x, -y)
@@ -1161,59 +1188,68 @@ k_open_fold_span(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old_s
         const Fq29 yPmQ = fq29_mul(fq29_sub(fq29_mul(lam, fq29_sub(p.x, xPmQ)), p.y), one29);
 #pragma unroll
         for (int l = 0; l < 14; ++l) {
-            tab[0][l][t] = xQ.l[l];
-            tab[1][l][t] = xPQ.l[l];
-            tab[2][l][t] = xPmQ.l[l];
-            tab[3][l][t] = yPmQ.l[l];
+            tab[b][0][l][t] = p.x.l[l];
+            tab[b][1][l][t] = p.y.l[l];
+            tab[b][2][l][t] = xQ.l[l];
+            tab[b][3][l][t] = xPmQ.l[l];
+            tab[b][4][l][t] = yPmQ.l[l];
+        }
+        flags[b][t] = (uint8_t)((inf ? 1 : 0) | (x0 ? 2 : 0));
+    }
+    __syncthreads();
+    const JsfK* const jsf = jsfs + blockIdx.y * 8;
+    J29 w = j29_infinity();
+    for (int i = (int)slice - 1; i >= 0; --i) {
+        if (__any(!w.inf)) j29_double_walk(w);
+        const uint32_t at = b * slice + (uint32_t)i;
+        for (uint32_t k = 0; k < 8; ++k) {
+            if (at >= jsf[k].len) continue;
+            const uint32_t dg = (jsf[k].dig[at >> 3] >> ((at & 7) * 4)) & 0xFu;    // (d1 + 1) | (d2 + 1) << 2, the same for every lane
+            const int d1 = (int)(dg & 3u) - 1, d2 = (int)(dg >> 2) - 1;
+            if (d1 == 0 && d2 == 0) continue;
+            A29 q;
+            bool negate;
+            const bool diff = d1 * d2 < 0;
+            const uint32_t xi = diff ? 3u : (d1 == 0 ? 2u : 0u), yi = diff ? 4u : 1u;
+#pragma unroll
+            for (int l = 0; l < 14; ++l) { q.x.l[l] = tab[k][xi][l][t]; q.y.l[l] = tab[k][yi][l][t]; }
+            if (d1 == d2) {                                                      // P + phi(P) = (beta^2 x, -y), beta^2 = -1 - beta
+                Fq29 s;
+#pragma unroll
+                for (int l = 0; l < 14; ++l) s.l[l] = tab[k][2][l][t];
+                q.x = fq29_neg(fq29_add(q.x, s));
+                negate = d1 > 0;
+            } else negate = d1 == 0 ? d2 < 0 : d1 < 0;
+            if (negate) q.y = fq29_neg(q.y);
+            // a point of abscissa zero is its own image under phi (outside the prime-order subgroup): P - phi(P) is infinity
+            const uint32_t fl = flags[k][t];
+            if (!(fl & 1u) && !((fl & 2u) && diff)) j29_add_mixed_walk(w, q);
         }
     }
-    for (int i = (int)jsf.len - 1; i >= 0; --i) {
-        w = j29_double(w);
-        const uint32_t dg = (jsf.dig[i >> 3] >> ((i & 7) * 4)) & 0xFu;    // (d1 + 1) | (d2 + 1) << 2, the same for every lane
-        const int d1 = (int)(dg & 3u) - 1, d2 = (int)(dg >> 2) - 1;
-        if (d1 == 0 && d2 == 0) continue;
-        A29 q;
-        bool negate;
-        int xi = -1;
-        if (d2 == 0) { q = p; negate = d1 < 0; }
-        else {
-            xi = d1 == 0 ? 0 : (d1 == d2 ? 1 : 2);
+    if (m < new_size) {
+        int32_t* out = reinterpret_cast<int32_t*>(sb.part) + ((size_t)blockIdx.y * 8 + b) * J29_WORDS * new_size + m;
+        const int32_t* src = reinterpret_cast<const int32_t*>(&w);
 #pragma unroll
-            for (int l = 0; l < 14; ++l) q.x.l[l] = tab[xi][l][t];
-            if (xi == 2) {
-#pragma unroll
-                for (int l = 0; l < 14; ++l) q.y.l[l] = tab[3][l][t];
-                negate = d1 < 0;
-            } else {
-                q.y = p.y;
-                negate = xi == 0 ? d2 < 0 : d1 > 0;                          // P + phi(P) = (beta^2 x, -y)
-            }
-        }
-        if (negate) q.y = fq29_neg(q.y);
-        // a point of abscissa zero is its own image under phi (outside the prime-order subgroup): P - phi(P) is infinity
-        if (!inf && !(x0 && xi == 2)) w = j29_add_mixed(w, q);
+        for (int l = 0; l < J29_WORDS; ++l) out[(size_t)l * new_size] = src[l];
     }
-    uint32_t* pool = reinterpret_cast<uint32_t*>(&lds[0][0][0][0]);
-    for (uint32_t sd = 4; sd > 0; sd >>= 1) {
-        __syncthreads();
-        if (b >= sd && b < 2 * sd) {
-            const uint32_t* src = reinterpret_cast<const uint32_t*>(&w);
+}
+__global__ void __launch_bounds__(GT) k_open_span_walk(const SpanBatch sb, size_t new_size, uint32_t slice) {
+    const size_t m = ((size_t)blockIdx.x * GT + threadIdx.x) >> 2;
+    const uint32_t q = threadIdx.x & 3u;
+    if (m >= new_size) return;
+    const int32_t* part = reinterpret_cast<const int32_t*>(sb.part) + (size_t)blockIdx.y * 8 * J29_WORDS * new_size + m;
+    J29 w = j29_infinity();
+    for (int b = 7; b >= 0; --b) {
+        if (__any(!w.inf))
+            for (uint32_t i = 0; i < slice; ++i) j29_quad_double(w, q);
+        J29 s;
+        int32_t* dst = reinterpret_cast<int32_t*>(&s);
 #pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) pool[((b - sd) * J29_WORDS + l) * GT + t] = src[l];
-        }
-        __syncthreads();
-        if (b < sd) {
-            J29 y;
-            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
-#pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[(b * J29_WORDS + l) * GT + t];
-            w = j29_add(w, y);
-        }
+        for (int l = 0; l < J29_WORDS; ++l) dst[l] = part[((size_t)b * J29_WORDS + l) * new_size];
+        j29_quad_add(w, s, q);
     }
-    if (b == 0) {
-        const A29 o = a29_from_j29(w);
-        if (m < new_size) sb.ng[blockIdx.y][m] = o;
-    }
+    const A29 o = a29_from_j29(w);
+    if (q == 0) sb.ng[blockIdx.y][m] = o;
 }
 // the pairs k_open_fold29 left out, by the general Jacobian route in 32-bit limbs (one lane per pair, an inversion each)
 __device__ __forceinline__ G1Affine a29_to_affine(const A29& p) {
@@ -1613,7 +1649,7 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
     hipLaunchKernelGGL(k_msm_seg, dim3(ns, MW, n_msm), dim3(MSL), 0, st, partial.as<J29>(), (const MsmDesc*)dd, ns, cps, chunk);
     // the segments' raw buckets summed eight at a time (a lane per bucket and window: the reduction, one workgroup per sum, then
     // walks single buckets)
-    const J29* cur = partial.as<J29>();
+    J29* cur = partial.as<J29>();
     while (ns > 1) {
         const uint32_t ng = (ns + 7) / 8;
         Scratch& nxt = arena.add(sizeof(J29) * n_msm * MW * (size_t)ng * MT);
@@ -1631,7 +1667,8 @@ static int points_queue(std::vector<PointDesc>& list, JobUploads& up, hipStream_
     const void* dl = nullptr;
     int rc = up.put(list.data(), sizeof(PointDesc) * list.size(), st, &dl);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_msm_point, dim3((unsigned)list.size()), dim3(2 * MT), 0, st, (const PointDesc*)dl);
+    hipLaunchKernelGGL(k_msm_point, dim3((unsigned)list.size(), 2), dim3(4 * MT), 0, st, (const PointDesc*)dl);
+    hipLaunchKernelGGL(k_msm_join, dim3(cdiv(4 * list.size(), (size_t)GT)), dim3(GT), 0, st, (const PointDesc*)dl, (uint32_t)list.size());
     ZK_LAUNCH_CHECK();
     list.clear();
     return 0;
@@ -1728,7 +1765,7 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
 // *scalars: the folded scalars.  pts: the proof points of opening 0 (npts an opening).  no_t_below: T of rounds below it is not summed here.
 static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, int no_t_below, const OpenItem* items, G1Jac* pts, size_t npts,
                              const Fr* U_dev, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later);
-// g^(3) of every opening from its generators in one launch (k_open_fold_span); challenges: rounds r0 .. r0 + 2
+// g^(3) of every opening from its generators (k_open_span_slices, k_open_span_walk); challenges: rounds r0 .. r0 + 2
 static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const OpenItem* items, Arena& arena, JobUploads& up, hipStream_t st);
 
 extern "C" {
@@ -2060,23 +2097,30 @@ static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const 
     const size_t ns = (((n0 + 1) / 2 + 1) / 2 + 1) / 2;
     Scratch& g2 = arena.add(sizeof(A29) * ns * count);
     if (g2.rc) return g2.rc;
+    Scratch& part = arena.add(sizeof(J29) * 8 * ns * count);
+    if (part.rc) return part.rc;
     std::vector<JsfK> jsf((size_t)count * JUMP_SPAN);
     SpanBatch sb;
+    sb.part = part.as<J29>();
     double fp_mults = 0;
+    uint32_t longest = 1;
     for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; sb.ng[i] = g2.as<A29>() + ns * k; sb.g[i] = gens[k]; }
     for (int i = 0; i < count; ++i) {
         Fr c[JUMP_SPAN];
         fold_span_coefficients(c, items[i].u + 8 * (size_t)r0);
         for (int b = 0; b < JUMP_SPAN; ++b) {
             jsf[(size_t)i * JUMP_SPAN + b] = jsf_of(glv_split(c[b]));
-            fp_mults += (fold_fp_mults_per_pair(jsf[(size_t)i * JUMP_SPAN + b]) + 2.0) * (double)ns;      // about what the walk of a pair takes
+            longest = std::max(longest, jsf[(size_t)i * JUMP_SPAN + b].len);
+            fp_mults += (fold_fp_mults_per_pair(jsf[(size_t)i * JUMP_SPAN + b]) + 2.0 - (b ? 7.0 * jsf[(size_t)i * JUMP_SPAN + b].len : 0.0)) * (double)ns;      // about: one of the eight doubles
         }
     }
     const void* dj = nullptr;
     int rc = up.put(jsf.data(), sizeof(JsfK) * jsf.size(), st, &dj);
     if (rc) return rc;
     FoldTimed timed(st);
-    hipLaunchKernelGGL(k_open_fold_span, dim3(cdiv(ns, GT), count), dim3(8 * GT), 0, st, sb, (const JsfK*)dj, n0, ns);
+    const uint32_t slice = (longest + 7) / 8;
+    hipLaunchKernelGGL(k_open_span_slices, dim3(cdiv(ns, GT), count), dim3(8 * GT), 0, st, sb, (const JsfK*)dj, n0, ns, slice);
+    hipLaunchKernelGGL(k_open_span_walk, dim3(cdiv(4 * ns, (size_t)GT), count), dim3(GT), 0, st, sb, ns, slice);
     ZK_LAUNCH_CHECK();
     timed.end(0, fp_mults, ns * (size_t)count * (JUMP_SPAN - 1));
     for (int i = 0; i < count; ++i) gens[i] = g2.as<A29>() + ns * i;
@@ -2115,10 +2159,6 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     if (rc) return rc;
     const A29* before[OB_MAX];
     for (int i = 0; i < count; ++i) before[i] = gens[i];
-    if (!last) {
-        rc = open_span_fold(gens, count, n0, r0, items, arena, up, st);
-        if (rc) return rc;
-    }
     hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, 256), count), dim3(256), 0, aux, coef.as<Fr>(), all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, fin);
     {
         RecodeBatch rb;
@@ -2126,6 +2166,10 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
         hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, 256), 1), dim3(256), 0, aux, rb, ncoef);
     }
     ZK_LAUNCH_CHECK();
+    if (!last) {          // behind the short kernels of the other stream: they would wait for the fold's workgroups otherwise
+        rc = open_span_fold(gens, count, n0, r0, items, arena, up, st);
+        if (rc) return rc;
+    }
     std::vector<MsmDesc> d;
     std::vector<G1Jac*> out;
     for (int it = 0; it < count; ++it)
