@@ -309,6 +309,8 @@ int zk_g1_open_end_batch(void* handle, uint32_t* proof_host, uint32_t* final_sca
 int zk_lookup_index_fr(void* idx_u32, const void* vals_fr, int32_t low, uint32_t table_size, size_t n, void* stream);
 int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32_t table_size, size_t n, void* stream);
 /* multiplicities (tlookup_kernel :10-15): counts[b] = #{i : idx[i] == b}; counts is cleared first */
+/* multiplicities of a table's entries (nbins field elements) from positions, int32 queries or field elements, the first that is not null; idx_out: the positions too, or null */
+int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, void* stream);
 int zk_lookup_hist(void* counts_u32, const void* idx_u32, size_t n, uint32_t nbins, void* stream);
 /* zk_lookup_index_i32 and zk_lookup_hist in one (tLookupRange::prep over queries that keep an int32 form): the counting passes
  * form the positions value - low themselves and no array of positions is written; a value outside [low, low + len) is an error */

@@ -86,6 +86,23 @@ def test_multiplicities_of_many_queries_into_a_large_table(pv, D, low, length, s
     assert (mk[:, 0] == want).all() and not mk[:, 1:].any()
 
 
+@pytest.mark.parametrize("D,low,length", [(1, 7, 16385), (8193, -3, 40001), (70001, -(1 << 15), 1 << 16), ((1 << 20) + 5, 0, 1 << 15), (3000000, -5, 65535)])
+def test_multiplicities_of_tables_counted_in_halves_of_words(pv, D, low, length):
+    """Tables of 16385 to 65536 entries (k_hist_wide): one query, shares of unequal size, all queries of a share in one bin."""
+    rng = np.random.default_rng(D)
+    vals = rng.integers(low, low + length, D)
+    vals[: D // 2] = low + length - 1
+    h = pv.from_i64(vals)
+    want = np.bincount(vals - low, minlength=1 << (length - 1).bit_length()).astype(np.uint32)
+    for kept in (False, True):
+        if kept:
+            pv.keep_for_folds(h)
+        m = pv.range_prep(h, low, length).host()
+        assert (m[:, 0] == want).all() and not m[:, 1:].any()
+    with pytest.raises(RuntimeError, match="outside the table"):
+        pv.range_prep(pv.from_i64(np.append(vals, low + length)), low, length)
+
+
 def test_lookup_out_of_range_is_an_error(pv):
     with pytest.raises(RuntimeError, match="outside the table"):
         pv.range_prep(pv.from_i64(np.array([0, 1, 99])), 0, 8)

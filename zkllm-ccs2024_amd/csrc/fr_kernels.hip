@@ -203,11 +203,8 @@ template <int K> static int finish_to_host(Fr* partials, unsigned nb, Fr* host_o
     void* stage = nullptr;
     int rc = staging(&stage, sizeof(Fr) * K);
     if (rc) return rc;
-    Scratch fin(sizeof(Fr) * K, st);
-    if (fin.rc) return fin.rc;
-    hipLaunchKernelGGL(k_finish_sums, dim3(K), dim3(TPB), 0, st, fin.as<Fr>(), partials, nb);
+    hipLaunchKernelGGL(k_finish_sums, dim3(K), dim3(TPB), 0, st, (Fr*)stage, partials, nb);
     ZK_LAUNCH_CHECK();
-    ZK_HIP(hipMemcpyAsync(stage, fin.p, sizeof(Fr) * K, hipMemcpyDeviceToHost, st));
     ZK_HIP(hipStreamSynchronize(st));
     memcpy(host_out, stage, sizeof(Fr) * K);
     return 0;
@@ -906,13 +903,13 @@ int zk_fr_me(uint32_t* out_host, const void* a, size_t n, const uint32_t* u, int
         FrPack12 p;
         const int rest = k - done;
         for (int i = 0; i < 12; ++i) p.x[i] = (i < rest) ? to_mont(load_fr(u + 8 * (done + i))) : big_zero<8>();
-        Scratch fin(sizeof(Fr), st);
-        rc = fin.rc;
+        Delivery d;
+        rc = deliver_begin(d, 1, 0);
         if (!rc) {
-            hipLaunchKernelGGL(k_me_small, dim3(1), dim3(TPB), 0, st, fin.as<Fr>(), cur_ptr, p, (uint32_t)cur, (uint32_t)rest);
+            hipLaunchKernelGGL(k_me_small, dim3(1), dim3(TPB), 0, st, (Fr*)d.dst, cur_ptr, p, (uint32_t)cur, (uint32_t)rest);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) rc = hip_fail(e, "zk_fr_me", __FILE__, __LINE__);
-            else rc = deliver(st, fin.p, out_host, 1, 0);
+            else rc = deliver_end(d, st, out_host);
         }
     }
     for (int i = 0; i < 2; ++i) if (bufs[i]) pool_free(bufs[i], st);
@@ -933,11 +930,12 @@ int zk_ip_round(uint32_t* poly3_host, const void* a, const void* b, size_t n_in,
     if (part.rc) return part.rc;
     hipLaunchKernelGGL(k_ip_round, dim3(nb), dim3(TPB), 0, (hipStream_t)stv, part.as<Fr>(), (const Fr*)a, (const Fr*)b, n_in, n_out);
     ZK_LAUNCH_CHECK();
-    Scratch fin(sizeof(Fr) * 3, (hipStream_t)stv);
-    if (fin.rc) return fin.rc;
-    hipLaunchKernelGGL(k_finish_sums, dim3(3), dim3(TPB), 0, (hipStream_t)stv, fin.as<Fr>(), part.as<Fr>(), nb);
+    Delivery d;
+    const int rc = deliver_begin(d, 3, 3);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_finish_sums, dim3(3), dim3(TPB), 0, (hipStream_t)stv, (Fr*)d.dst, part.as<Fr>(), nb);
     ZK_LAUNCH_CHECK();
-    return deliver((hipStream_t)stv, fin.p, poly3_host, 3, 3);
+    return deliver_end(d, (hipStream_t)stv, poly3_host);
 }
 
 // Stacked round over [N][D] tensors: rows_in = N, rows_out = 2^ceil(log2 N) / 2, E = eq table over the
@@ -964,13 +962,16 @@ int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(k >= 1 && k <= 13, "zk_ip_sumcheck_small: k must be 1..13");
     ZK_ARG(n >= 1 && n <= (1u << k) && n > ((1u << k) >> 1), "zk_ip_sumcheck_small: need 2^(k-1) < n <= 2^k");
-    // out: the sums of all rounds, then the two folded values; behind them what passes from the first launch to the second
+    // delivered: the sums of all rounds, then the two folded values; work: what passes from the first launch to the second
     const int r1 = k <= IP_ROUNDS ? 0 : IP_ROUNDS, r2 = k - r1;
     const uint32_t nb1 = r1 ? 1u << (k - r1) : 0u;
-    Scratch work(sizeof(Fr) * (3 * (size_t)k + 2 + (3 * (size_t)r1 + 2) * nb1), st);
+    Scratch work(sizeof(Fr) * (3 * (size_t)r1 + 2) * nb1, st);
     if (work.rc) return work.rc;
-    Fr* polys = work.as<Fr>();
-    Fr* part = polys + 3 * k + 2;
+    Delivery d;
+    int rc = deliver_begin(d, 3 * (size_t)k + 2, 0);
+    if (rc) return rc;
+    Fr* polys = (Fr*)d.dst;
+    Fr* part = work.as<Fr>();
     Fr* mid = part + 3 * (size_t)r1 * nb1;
     IpArgs q;
     memset(&q, 0, sizeof(q));
@@ -992,7 +993,7 @@ int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a
     ZK_LAUNCH_CHECK();
     // one delivery of 3k + 2 values: the round polynomials, then the two fully folded values
     Fr both[3 * 13 + 2];
-    int rc = deliver(st, polys, both, 3 * (size_t)k + 2, 0);
+    rc = deliver_end(d, st, both);
     if (rc) return rc;
     memcpy(polys_host, both, sizeof(Fr) * 3 * k);           // (while results are deferred these two are not what the kernel wrote: see zk_defer_begin)
     memcpy(fin_host, both + 3 * k, sizeof(Fr) * 2);

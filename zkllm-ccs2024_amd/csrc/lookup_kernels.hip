@@ -13,6 +13,7 @@
 //    the operands yields every coefficient of the round polynomial and the folded operands; no
 //    term tensor is ever written.
 //  * softmax shift / exp tables use the deterministic exp/log of detmath.hpp.
+#include <algorithm>
 #include <cstring>
 #include <memory>
 #include <vector>
@@ -92,17 +93,32 @@ __global__ void __launch_bounds__(TPB) k_finish(Fr* __restrict__ out, const Fr* 
 // The partial sums of all rounds of a job at once, behind its last round: no round waits for the one before to be summed
 // (the next round needs the fold challenge, not the sums).  Round r's K[r] sums: nb[r] partials each from part + off[r], into
 // sums[r * per_round + k].  grid (most sums of a round, rounds)
+// Results go where the host reads them (pinned memory), with no copy behind the launch; workgroups of the row behind the last round
+// deliver what else a job has: the sum of `extra`'s parts or two values, and a word, behind the rounds' sums.
 static constexpr int FINISH_ROUNDS_MAX = 64;
-struct FinishRounds { uint32_t off[FINISH_ROUNDS_MAX], nb[FINISH_ROUNDS_MAX]; uint8_t k[FINISH_ROUNDS_MAX]; };
+struct FinishRounds {
+    uint32_t off[FINISH_ROUNDS_MAX], nb[FINISH_ROUNDS_MAX];
+    uint8_t k[FINISH_ROUNDS_MAX];
+    const Fr *extra, *v0, *v1;           // extra: extra_nb parts of a sum; v0, v1: two values (null: none)
+    const uint32_t* word;
+    uint32_t extra_nb, slot;             // slot: where they go, in elements
+};
 struct PartSlice { Fr* p; template <class T> T* as() const { return reinterpret_cast<T*>(p); } };      // a round's share of the partial sums
 __global__ void __launch_bounds__(TPB) k_finish_rounds(Fr* __restrict__ sums, const Fr* __restrict__ part, const FinishRounds fr, uint32_t per_round) {
-    const uint32_t r = blockIdx.y;
-    if (blockIdx.x >= fr.k[r]) return;
+    const uint32_t r = blockIdx.y, t = threadIdx.x;
+    const bool behind = r + 1 == gridDim.y;
+    if (behind ? blockIdx.x != 0 : blockIdx.x >= fr.k[r]) return;
+    if (behind) {
+        if (fr.v0 && t < 16) (&sums[fr.slot].v[0])[t] = t < 8 ? fr.v0->v[t] : fr.v1->v[t - 8];
+        if (fr.word && t == 0) sums[fr.slot + (fr.v0 ? 2 : 1)].v[0] = *fr.word;
+        if (!fr.extra) return;
+    }
     Fr acc[1] = {big_zero<8>()};
-    const uint32_t nb = fr.nb[r];
-    const Fr* p = part + fr.off[r] + (size_t)blockIdx.x * nb;
-    for (uint32_t i = threadIdx.x; i < nb; i += TPB) acc[0] = add(acc[0], p[i]);
-    block_reduce_store<1>(acc, sums + (size_t)r * per_round);
+    const uint32_t nb = behind ? fr.extra_nb : fr.nb[r];
+    const Fr* p = behind ? fr.extra : part + fr.off[r] + (size_t)blockIdx.x * nb;
+    for (uint32_t i = t; i < nb; i += TPB) acc[0] = add(acc[0], p[i]);
+    // (block_reduce_store: sum 0 of workgroup blockIdx.x to partials[blockIdx.x])
+    block_reduce_store<1>(acc, sums + (behind ? (size_t)fr.slot : (size_t)r * per_round));
 }
 static inline unsigned reduce_grid(size_t n) {
     size_t b = (n + TPB - 1) / TPB;
@@ -115,18 +131,15 @@ static inline unsigned round_grid(size_t n, unsigned per_lane) {
     const size_t all = reduce_grid(n), want = n / ((size_t)TPB * per_lane);
     return (unsigned)std::min(all, std::max<size_t>(64, want));
 }
-// finish K sums (K x nb partials) and copy them to the host, applying the R correction (to_mont)
+// finish K sums (K x nb partials) where the host reads them, applying the R correction (to_mont)
 // to the first `n_mont` of them
 static int finish_sums(Fr* partials, unsigned nb, int K, int n_mont, Fr* host_out, hipStream_t st) {
-    void* stage = nullptr;
-    int rc = staging(&stage, sizeof(Fr) * K);
+    Delivery d;
+    int rc = deliver_begin(d, (size_t)K, n_mont);
     if (rc) return rc;
-    Scratch fin(sizeof(Fr) * K, st);
-    if (fin.rc) return fin.rc;
-    hipLaunchKernelGGL(k_finish, dim3(K), dim3(TPB), 0, st, fin.as<Fr>(), partials, nb);
+    hipLaunchKernelGGL(k_finish, dim3(K), dim3(TPB), 0, st, (Fr*)d.dst, partials, nb);
     ZK_LAUNCH_CHECK();
-    (void)stage;
-    return deliver(st, fin.p, host_out, (size_t)K, n_mont);
+    return deliver_end(d, st, host_out);
 }
 
 // ---- table index / histogram ---------------------------------------------------------------------------------
@@ -149,10 +162,17 @@ __global__ void __launch_bounds__(TPB) k_index_i32(uint32_t* __restrict__ idx, u
     if (!ok) atomicOr(flag, 1u);
 }
 // Where a counting pass takes its table positions from: an array of them, or the queries themselves in int32 form (position =
-// value - low; a value outside [low, low + len) counts as position 0 and raises *flag in the passes that are asked to check).
-struct KeySrc { const uint32_t* idx; const int32_t* vals; int32_t low; uint32_t len; uint32_t* flag; };
+// value - low; a value outside [low, low + len) counts as position 0 and raises *flag in the passes that are asked to check), or as
+// field elements (fr, low_fr: read eight times the bytes, so by passes that are alone to read them).
+struct KeySrc { const uint32_t* idx; const int32_t* vals; int32_t low; uint32_t len; uint32_t* flag; const Fr* fr = nullptr; Fr low_fr = Fr(); };
 template <bool CHECK> __device__ __forceinline__ uint32_t key_at(const KeySrc& k, size_t i) {
     if (k.idx) return k.idx[i];
+    if (k.fr) {
+        const Fr d = sub(k.fr[i], k.low_fr);
+        const bool ok = !(d.v[1] | d.v[2] | d.v[3] | d.v[4] | d.v[5] | d.v[6] | d.v[7]) && d.v[0] < k.len;
+        if (CHECK && !ok) atomicOr(k.flag, 1u);
+        return ok ? d.v[0] : 0u;
+    }
     const int64_t d = (int64_t)k.vals[i] - (int64_t)k.low;
     const bool ok = d >= 0 && d < (int64_t)k.len;
     if (CHECK && !ok) atomicOr(k.flag, 1u);
@@ -208,15 +228,14 @@ __global__ void __launch_bounds__(TPB) k_hist_global(uint32_t* __restrict__ coun
 // size asks for; global memory sees one atomic per non-empty bin and slice.  Skewed inputs (one partition holding nearly
 // everything) only make that partition's slices hit the same LDS counters, which an LDS serves far faster than L2 does.
 static constexpr uint32_t HP_BITS = 12, HP_BINS = 1u << HP_BITS;   // bins per partition
-static constexpr uint32_t HP_TILE = 65536;                           // queries per workgroup of the partition passes
 static constexpr uint32_t HP_SLICE = 32768;                          // queries per workgroup of the counting pass
 static constexpr uint32_t HP_MAXP = 1024;                            // partitions: tables up to 2^22 bins
 static constexpr size_t HP_MIN_QUERIES = (size_t)1 << 20;
-__global__ void __launch_bounds__(TPB) k_hp_sizes(uint32_t* __restrict__ sizes, const KeySrc idx, size_t n, uint32_t P, uint32_t ntiles) {
+__global__ void __launch_bounds__(TPB) k_hp_sizes(uint32_t* __restrict__ sizes, const KeySrc idx, size_t n, uint32_t P, uint32_t ntiles, uint32_t tile) {
     __shared__ uint32_t c[HP_MAXP];
     for (uint32_t q = threadIdx.x; q < P; q += TPB) c[q] = 0;
     __syncthreads();
-    const size_t base = (size_t)blockIdx.x * HP_TILE, end = base + HP_TILE < n ? base + HP_TILE : n;
+    const size_t base = (size_t)blockIdx.x * tile, end = base + tile < n ? base + tile : n;
     for (size_t i = base + threadIdx.x; i < end; i += TPB) atomicAdd(&c[key_at<true>(idx, i) >> HP_BITS], 1u);
     __syncthreads();
     for (uint32_t q = threadIdx.x; q < P; q += TPB) sizes[(size_t)q * ntiles + blockIdx.x] = c[q];
@@ -275,11 +294,11 @@ __global__ void __launch_bounds__(1024) k_hp_slices(uint32_t* __restrict__ slice
     if (t == 1023u) *nslices = part[1023];
 }
 __global__ void __launch_bounds__(TPB) k_hp_scatter(uint16_t* __restrict__ parted, const uint32_t* __restrict__ offs, const uint32_t* __restrict__ part_off,
-                                                    const KeySrc idx, size_t n, uint32_t P, uint32_t ntiles) {
+                                                    const KeySrc idx, size_t n, uint32_t P, uint32_t ntiles, uint32_t tile) {
     __shared__ uint32_t cur[HP_MAXP];
     for (uint32_t q = threadIdx.x; q < P; q += TPB) cur[q] = part_off[q] + offs[(size_t)q * ntiles + blockIdx.x];
     __syncthreads();
-    const size_t base = (size_t)blockIdx.x * HP_TILE, end = base + HP_TILE < n ? base + HP_TILE : n;
+    const size_t base = (size_t)blockIdx.x * tile, end = base + tile < n ? base + tile : n;
     for (size_t i = base + threadIdx.x; i < end; i += TPB) {
         const uint32_t key = key_at<false>(idx, i);
         const uint32_t pos = atomicAdd(&cur[key >> HP_BITS], 1u);
@@ -303,19 +322,74 @@ __global__ void __launch_bounds__(TPB) k_hp_count(uint32_t* __restrict__ counts,
     }
 }
 static int hist_partitioned(uint32_t* counts, const KeySrc idx, size_t n, uint32_t nbins, hipStream_t st) {
-    const uint32_t P = (nbins + HP_BINS - 1) / HP_BINS, ntiles = cdiv(n, HP_TILE), M = P * ntiles;
+    // queries per workgroup of the partition passes: about a thousand workgroups (64 of them, 65536 queries each, took 120 us for 2^22), of 4096 at least
+    uint32_t tile = 4096;
+    while (tile < 65536 && (size_t)tile << 10 < n) tile <<= 1;
+    const uint32_t P = (nbins + HP_BINS - 1) / HP_BINS, ntiles = cdiv(n, tile), M = P * ntiles;
     const uint32_t max_slices = (uint32_t)(n / HP_SLICE) + P + 1;
     Scratch sizes(sizeof(uint32_t) * (size_t)M, st), part_off(sizeof(uint32_t) * (P + 1), st), totals(sizeof(uint32_t) * P, st), slice_tab(sizeof(uint32_t) * max_slices, st),
         nsl(sizeof(uint32_t), st), parted(sizeof(uint16_t) * n, st);
     for (const Scratch* b : {&sizes, &part_off, &totals, &slice_tab, &nsl, &parted})
         if (b->rc) return b->rc;
-    hipLaunchKernelGGL(k_hp_sizes, dim3(ntiles), dim3(TPB), 0, st, sizes.as<uint32_t>(), idx, n, P, ntiles);
+    hipLaunchKernelGGL(k_hp_sizes, dim3(ntiles), dim3(TPB), 0, st, sizes.as<uint32_t>(), idx, n, P, ntiles, tile);
     hipLaunchKernelGGL(k_hp_rowscan, dim3(P), dim3(TPB), 0, st, sizes.as<uint32_t>(), totals.as<uint32_t>(), ntiles);
     hipLaunchKernelGGL(k_hp_slices, dim3(1), dim3(1024), 0, st, slice_tab.as<uint32_t>(), nsl.as<uint32_t>(), part_off.as<uint32_t>(), totals.as<uint32_t>(), P);
-    hipLaunchKernelGGL(k_hp_scatter, dim3(ntiles), dim3(TPB), 0, st, parted.as<uint16_t>(), sizes.as<uint32_t>(), part_off.as<uint32_t>(), idx, n, P, ntiles);
+    hipLaunchKernelGGL(k_hp_scatter, dim3(ntiles), dim3(TPB), 0, st, parted.as<uint16_t>(), sizes.as<uint32_t>(), part_off.as<uint32_t>(), idx, n, P, ntiles, tile);
     hipLaunchKernelGGL(k_hp_count, dim3(max_slices), dim3(TPB), 0, st, counts, parted.as<uint16_t>(), part_off.as<uint32_t>(), slice_tab.as<uint32_t>(), nsl.as<uint32_t>(), nbins);
     ZK_LAUNCH_CHECK();
     return 0;
+}
+// Tables of 16385 to 65536 entries: a workgroup counts its share of the queries in 16-bit halves of LDS words (64 KB to 128 KB; a share is
+// 32768 queries at most), writes all its counters out, and a second launch adds the workgroups' up and writes the multiplicities.  The
+// counters cross memory once, in lines; adding them to global ones costs an atomic for nearly every query where these spread.
+// 2^22 queries in 2^16 bins: partitioned 163 us, this way 30 us.
+static constexpr uint32_t HW_BINS = 65536, HW_SHARE = 32768, HW_T = 1024, HW_SLICES = 8;
+__global__ void __launch_bounds__(HW_T) k_hist_wide(uint32_t* __restrict__ part, const KeySrc idx, size_t n, uint32_t words) {
+    __shared__ __attribute__((aligned(16))) uint32_t h[HW_BINS / 2];
+    for (uint32_t w = threadIdx.x; w < words; w += HW_T) h[w] = 0;
+    __syncthreads();
+    const size_t share = (n + gridDim.x - 1) / gridDim.x, begin = (size_t)blockIdx.x * share, end = begin + share < n ? begin + share : n;
+    for (size_t i = begin + threadIdx.x; i < end; i += HW_T) {
+        const uint32_t key = key_at<true>(idx, i);
+        atomicAdd(&h[key >> 1], 1u << (16u * (key & 1u)));
+    }
+    __syncthreads();
+    uint32_t* out = part + (size_t)blockIdx.x * words;
+    for (uint32_t w = threadIdx.x; w < words; w += HW_T) out[w] = h[w];
+}
+// m[bin] as field elements; *host_flag = *flag
+__global__ void __launch_bounds__(64 * HW_SLICES) k_hist_wide_sum(Fr* __restrict__ m, const uint32_t* __restrict__ part, uint32_t parts, uint32_t words, uint32_t nbins,
+                                                                  const uint32_t* __restrict__ flag, uint32_t* __restrict__ host_flag) {
+    __shared__ uint32_t s[2][HW_SLICES][64];
+    const uint32_t c = threadIdx.x & 63u, sl = threadIdx.x >> 6, w = blockIdx.x * 64u + c;
+    uint32_t lo = 0, hi = 0;
+    if (w < words)
+        for (uint32_t p = sl; p < parts; p += HW_SLICES) {
+            const uint32_t x = part[(size_t)p * words + w];
+            lo += x & 0xFFFFu;
+            hi += x >> 16;
+        }
+    s[0][sl][c] = lo;
+    s[1][sl][c] = hi;
+    __syncthreads();
+    if (threadIdx.x < 128u) {
+        const uint32_t q = threadIdx.x & 1u, b = threadIdx.x >> 1, bin = 2u * (blockIdx.x * 64u + b) + q;
+        uint32_t total = 0;
+        for (uint32_t k = 0; k < HW_SLICES; ++k) total += s[q][k][b];
+        Fr v = big_zero<8>();
+        v.v[0] = total;
+        if (bin < nbins) m[bin] = v;
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) *host_flag = *flag;
+}
+// counts as field elements; *host_flag = *flag
+__global__ void __launch_bounds__(TPB) k_hist_deliver(Fr* __restrict__ m, const uint32_t* __restrict__ counts, uint32_t nbins, const uint32_t* __restrict__ flag, uint32_t* __restrict__ host_flag) {
+    const uint32_t i = blockIdx.x * TPB + threadIdx.x;
+    if (i == 0) *host_flag = *flag;
+    if (i >= nbins) return;
+    Fr v = big_zero<8>();
+    v.v[0] = counts[i];
+    m[i] = v;
 }
 // table[i] = low + min(i, len-1)  (tlookuprange_init_kernel tlookup.cu:372-380)
 __global__ void __launch_bounds__(TPB) k_range_table(Fr* __restrict__ table, int32_t low, uint32_t len, uint32_t table_size) {
@@ -332,39 +406,53 @@ __global__ void __launch_bounds__(TPB) k_range_table(Fr* __restrict__ table, int
 // inversion for it, and the serial part that such a root has (and three launches at the larger sizes) is gone: 2^16 table entries
 // took 210 us that way.  The inputs are used as they are: Montgomery products of plain numbers carry factors R^-1 that cancel
 // when the product's plain inverse is what comes back down.
+// What a lookup's table wants beside its inverses, in the same launch: each entry and its inverse next to each other (TB), the parts
+// of sum inverse * m, one a workgroup, and a word that a later launch lowers.
+struct InvRiders { Fr* TB; const Fr* m; Fr* dot; uint32_t* word; uint32_t word_value; };
 template <int CH>
-__global__ void __launch_bounds__(256) k_batch_inv(Fr* __restrict__ out, const Fr* __restrict__ in, const Fr beta, size_t n) {
+__global__ void __launch_bounds__(256) k_batch_inv(Fr* __restrict__ out, const Fr* __restrict__ in, const Fr beta, size_t n, const InvRiders ride) {
     const size_t base = (size_t)blockIdx.x * 256 * CH + threadIdx.x;
-    if (base >= n) return;
-    Fr x[CH], pre[CH];
-    uint32_t nz = 0;
-    Fr tot = big_one_mont<8>();
+    if (ride.word && base == 0) *ride.word = ride.word_value;
+    Fr dot[1] = {big_zero<8>()};
+    if (base < n) {
+        Fr x[CH], pre[CH];
+        uint32_t nz = 0;
+        Fr tot = big_one_mont<8>();
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const size_t i = base + (size_t)c * 256;
-        Fr v = big_zero<8>();
-        if (i < n) v = add(in[i], beta);
-        const bool nzc = !is_zero(v);
-        nz |= (nzc ? 1u : 0u) << c;
-        x[c] = nzc ? v : big_one_mont<8>();
-        pre[c] = tot;
-        tot = mont_mul(tot, x[c]);
-    }
-    Fr inv_run = plain_inverse(tot);
+        for (int c = 0; c < CH; ++c) {
+            const size_t i = base + (size_t)c * 256;
+            Fr v = big_zero<8>();
+            if (i < n) v = add(in[i], beta);
+            const bool nzc = !is_zero(v);
+            nz |= (nzc ? 1u : 0u) << c;
+            x[c] = nzc ? v : big_one_mont<8>();
+            pre[c] = tot;
+            tot = mont_mul(tot, x[c]);
+        }
+        Fr inv_run = plain_inverse(tot);
 #pragma unroll
-    for (int c = CH - 1; c >= 0; --c) {
-        const size_t i = base + (size_t)c * 256;
-        const Fr inv_c = mont_mul(inv_run, pre[c]);
-        inv_run = mont_mul(inv_run, x[c]);
-        if (i < n) out[i] = ((nz >> c) & 1u) ? inv_c : big_zero<8>();
+        for (int c = CH - 1; c >= 0; --c) {
+            const size_t i = base + (size_t)c * 256;
+            Fr inv_c = mont_mul(inv_run, pre[c]);
+            inv_run = mont_mul(inv_run, x[c]);
+            if (!((nz >> c) & 1u)) inv_c = big_zero<8>();
+            if (i < n) {
+                out[i] = inv_c;
+                if (ride.TB) { ride.TB[2 * i] = in[i]; ride.TB[2 * i + 1] = inv_c; }
+                if (ride.m) dot[0] = add(dot[0], mont_mul(inv_c, ride.m[i]));
+            }
+        }
     }
+    if (ride.m) block_reduce_store<1>(dot, ride.dot);
 }
+static inline bool batch_inv_narrow(size_t n) { return n <= (size_t)1 << 18; }
+static inline unsigned batch_inv_grid(size_t n) { return cdiv(n, batch_inv_narrow(n) ? 512 : 2048); }
 // queues out = 1 / (in + beta) on st
-static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, hipStream_t st) {
+static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, hipStream_t st, const InvRiders& ride = InvRiders{nullptr, nullptr, nullptr, nullptr, 0}) {
     if (n == 0) return 0;
     // few values a lane while that leaves the chip at two waves a SIMD or less: the launch then takes what one lane takes
-    if (n <= (size_t)1 << 18) hipLaunchKernelGGL(k_batch_inv<2>, dim3(cdiv(n, 512)), dim3(256), 0, st, out, in, beta, n);
-    else hipLaunchKernelGGL(k_batch_inv<8>, dim3(cdiv(n, 2048)), dim3(256), 0, st, out, in, beta, n);
+    if (batch_inv_narrow(n)) hipLaunchKernelGGL(k_batch_inv<2>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
+    else hipLaunchKernelGGL(k_batch_inv<8>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
     ZK_LAUNCH_CHECK();
     return 0;
 }
@@ -397,6 +485,13 @@ __global__ void __launch_bounds__(TPB) k_eq_halves(Fr* __restrict__ lo, Fr* __re
     Fr e = big_one_mont<8>();
     for (int j = 0; j < cnt; ++j) e = mont_mul(e, ((t >> j) & 1u) ? c.u[first + j] : c.omu[first + j]);
     (is_hi ? hi : lo)[t] = e;
+}
+// Up to EQ_TABS_MAX variables in one launch: the host makes the tables over a third of the variables each, an entry is two products
+static constexpr int EQ_TABS_MAX = 15;
+struct EqTabs { Fr t[96]; };          // 32 entries a third, Montgomery form
+__global__ void __launch_bounds__(TPB) k_eq_tabs(Fr* __restrict__ e, const EqTabs tabs, uint32_t n, int b0, int b1) {
+    const uint32_t i = blockIdx.x * TPB + threadIdx.x;
+    if (i < n) e[i] = mont_mul(mont_mul(tabs.t[i & ((1u << b0) - 1u)], tabs.t[32 + ((i >> b0) & ((1u << b1) - 1u))]), tabs.t[64 + (i >> (b0 + b1))]);
 }
 __global__ void __launch_bounds__(TPB) k_eq_outer(Fr* __restrict__ e, const Fr* __restrict__ lo, const Fr* __restrict__ hi, int kl, size_t n) {
     const size_t t = (size_t)blockIdx.x * TPB + threadIdx.x;
@@ -509,10 +604,6 @@ __device__ __forceinline__ Fr query_inv_ints(size_t i, const HintSrc& h, Fr& a, 
     a = inv_plus_beta_alone(sv, h.beta);
     unit = false;
     return sv;
-}
-__global__ void __launch_bounds__(TPB) k_interleave(Fr* __restrict__ out, const Fr* __restrict__ a, const Fr* __restrict__ b, size_t n) {
-    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
-    if (i < n) { out[2 * i] = a[i]; out[2 * i + 1] = b[i]; }
 }
 __global__ void __launch_bounds__(TPB) k_inv_by_hint(Fr* __restrict__ A, const Fr* __restrict__ S, const HintSrc h, size_t D) {
     const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
@@ -1606,6 +1697,25 @@ static int read_flag(uint32_t* dev_flag, uint32_t* host_val, hipStream_t st) {
 
 // eq table of k challenges into out (2^k elements, Montgomery form), queued on the stream; the two half tables live in the arena
 static int eq_table_queue(Fr* out, const uint32_t* u, int k, Arena& arena, hipStream_t st) {
+    if (k <= EQ_TABS_MAX) {
+        EqTabs tabs;
+        const int bits[3] = {(k + 2) / 3, (k + 1) / 3, k / 3};
+        int at = 0;
+        for (int f = 0; f < 3; ++f) {
+            Fr* t = tabs.t + 32 * f;
+            t[0] = big_one_mont<8>();
+            for (int b = 0; b < bits[f]; ++b, ++at) {
+                const Fr x = to_mont(load_fr(u + 8 * at));
+                for (int i = 0; i < (1 << b); ++i) {
+                    t[i + (1 << b)] = mont_mul(t[i], x);
+                    t[i] = sub(t[i], t[i + (1 << b)]);
+                }
+            }
+        }
+        hipLaunchKernelGGL(k_eq_tabs, dim3(cdiv((size_t)1 << k, TPB)), dim3(TPB), 0, st, out, tabs, 1u << k, bits[0], bits[1]);
+        ZK_LAUNCH_CHECK();
+        return 0;
+    }
     EqChallenges c;
     Fr one = big_zero<8>();
     one.v[0] = 1;
@@ -2005,9 +2115,8 @@ int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32
     ZK_ARG(f == 0, "lookup: a value lies outside the table range");
     return 0;
 }
-// counts[0..nbins) = number of occurrences of each index (zeroed here first)
-static int hist_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t nbins, hipStream_t st) {
-    ZK_HIP(hipMemsetAsync(counts, 0, sizeof(uint32_t) * (size_t)nbins, st));
+// counts[0..nbins) += number of occurrences of each index
+static int hist_add_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t nbins, hipStream_t st) {
     if (n == 0) return 0;
     if (nbins <= HIST_LDS_BINS) {
         unsigned blocks = cdiv(n, (size_t)TPB * 16);
@@ -2019,6 +2128,59 @@ static int hist_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t nbi
         hipLaunchKernelGGL(k_hist_global, dim3(cdiv(n, (size_t)TPB * HH_PER_LANE)), dim3(TPB), 0, st, counts, src, n);
     }
     ZK_LAUNCH_CHECK();
+    return 0;
+}
+static int hist_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t nbins, hipStream_t st) {
+    ZK_HIP(hipMemsetAsync(counts, 0, sizeof(uint32_t) * (size_t)nbins, st));
+    return hist_add_queue(counts, src, n, nbins, st);
+}
+// Multiplicities of a table's entries as field elements (m: nbins of them), from table positions (idx), queries in int32 form (vals_i32) or
+// queries as field elements (vals): the first that is not null.  A query outside [low, low + len) is an error.  idx_out (optional): the
+// positions too.  One wait, at the end.
+int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, void* stv) {
+    hipStream_t st = (hipStream_t)stv;
+    ZK_ARG(nbins >= 1 && len >= 1 && len <= nbins, "zk_lookup_multiplicities: need 1 <= len <= nbins");
+    ZK_ARG(m != nullptr && (idx != nullptr || vals_i32 != nullptr || vals != nullptr || n == 0), "zk_lookup_multiplicities: null argument");
+    const bool wide = nbins > HIST_LDS_BINS && nbins <= HW_BINS && n >= 1 && n < ((size_t)1 << 27);
+    const unsigned shares = wide ? (unsigned)std::max<size_t>(std::min<size_t>(cdiv(n, (size_t)8192), 256), cdiv(n, (size_t)HW_SHARE)) : 0u;
+    const uint32_t words = (nbins + 1) / 2;
+    Scratch counts(sizeof(uint32_t) * ((wide ? (size_t)shares * words : (size_t)nbins) + 1), st);      // the first word: the flag
+    if (counts.rc) return counts.rc;
+    uint32_t* const flag = counts.as<uint32_t>();
+    uint32_t* const c = flag + 1;
+    ZK_HIP(hipMemsetAsync(flag, 0, sizeof(uint32_t) * (wide ? 1 : (size_t)nbins + 1), st));
+    void* stage = nullptr;
+    int rc = staging(&stage, 4);
+    if (rc) return rc;
+    KeySrc src{(const uint32_t*)idx, (const int32_t*)vals_i32, low, len, flag};
+    std::unique_ptr<Scratch> own;
+    if (!idx && !vals_i32) {
+        src.fr = (const Fr*)vals;
+        src.low_fr = fr_from_i64((int64_t)low);
+    }
+    const bool several_passes = !wide && nbins > HIST_LDS_BINS && n >= HP_MIN_QUERIES;
+    if (!idx && (idx_out || (src.fr && several_passes))) {
+        if (!idx_out) {
+            own.reset(new Scratch(sizeof(uint32_t) * n, st));
+            if (own->rc) return own->rc;
+            idx_out = own->p;
+        }
+        if (vals_i32) LAUNCH1D(k_index_i32, n, st, (uint32_t*)idx_out, flag, (const int32_t*)vals_i32, low, len, n);
+        else LAUNCH1D(k_index_fr, n, st, (uint32_t*)idx_out, flag, (const Fr*)vals, src.low_fr, len, n);
+        src.idx = (const uint32_t*)idx_out;
+        src.fr = nullptr;
+    }
+    if (wide) {
+        hipLaunchKernelGGL(k_hist_wide, dim3(shares), dim3(HW_T), 0, st, c, src, n, words);
+        hipLaunchKernelGGL(k_hist_wide_sum, dim3(cdiv(words, 64u)), dim3(64 * HW_SLICES), 0, st, (Fr*)m, c, shares, words, nbins, flag, (uint32_t*)stage);
+    } else {
+        rc = hist_add_queue(c, src, n, nbins, st);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_hist_deliver, dim3(cdiv(nbins, (unsigned)TPB)), dim3(TPB), 0, st, (Fr*)m, c, nbins, flag, (uint32_t*)stage);
+    }
+    ZK_LAUNCH_CHECK();
+    ZK_HIP(hipStreamSynchronize(st));
+    ZK_ARG(*(uint32_t*)stage == 0, "lookup: a value lies outside the table range");
     return 0;
 }
 int zk_lookup_hist(void* counts_u32, const void* idx_u32, size_t n, uint32_t nbins, void* stv) {
@@ -2378,13 +2540,17 @@ struct SumJob {
     Arena arena;
     hipStream_t st = nullptr;
     Fr* sums = nullptr;          // rounds x per_round values
-    Fr* extra = nullptr;         // one more value fetched with the sums (lookup: <B, m> with R^-1 attached), or null
+    bool extra = false;          // one more value behind the sums (lookup: <B, m> with R^-1 attached)
+    FinishRounds fin;            // what the last launch adds up and delivers
+    SumJob() { memset(&fin, 0, sizeof(fin)); }
+    ~SumJob() { pinned_release(host); }
+    SumJob(const SumJob&) = delete;
+    SumJob& operator=(const SumJob&) = delete;
     int rounds = 0, per_round = 0, n1 = 0;
     hipEvent_t ready = nullptr;
-    void* host = nullptr;        // jobs on a side stream: pinned buffer the results are copied to behind the last kernel ...
-    hipEvent_t done = nullptr;   // ... and the event behind that copy
-    const uint32_t* n_ok_dev = nullptr;      // lookup jobs over int32 forms: the consistent prefix of the table (HintSrc::n_ok) ...
-    uint32_t n_table = 0;                    // ... and the table's size
+    void* host = nullptr;        // pinned buffer that the last kernels write the results to (sums points to it) ...
+    hipEvent_t done = nullptr;   // ... and, for jobs on a side stream, the event behind them
+    uint32_t n_table = 0;        // lookup jobs over int32 forms (fin.word: the consistent prefix of the table, HintSrc::n_ok): the table's size
     // a job whose launches were handed to the library's launch thread: the ticket to wait for before anything of the job is
     // read, and what that thread's attempt returned
     uint64_t ticket = 0;
@@ -2398,6 +2564,14 @@ struct SumJob {
     std::vector<Fr> eq_scale;
     int tail_from = -1;
 };
+// the pinned buffer of a job's results: rounds x per_round sums, behind them what job.fin delivers
+static int sumjob_results(SumJob& job) {
+    const int rc = pinned_acquire(&job.host);
+    if (rc) return rc;
+    job.sums = (Fr*)job.host;
+    job.fin.slot = (uint32_t)(job.rounds * job.per_round);
+    return 0;
+}
 // eq_scale of a job over `rounds` rounds whose table is eq(u_eq, .) of rounds - 1 challenges (index bit j <-> u_eq[j]); false
 // (and nothing written) if some challenge is 1
 static bool eq_prefix_scales(std::vector<Fr>& out, const uint32_t* u_eq, int rounds) {
@@ -2430,12 +2604,6 @@ static void eq_prefix_apply(const SumJob& job, Fr* sums, uint32_t weighted) {
         for (int i = 0; i < job.per_round; ++i)
             if ((weighted >> i) & 1u) sums[(size_t)r * job.per_round + i] = mont_mul(sums[(size_t)r * job.per_round + i], c);
     }
-}
-__global__ void __launch_bounds__(64) k_u32_set(uint32_t* __restrict__ p, uint32_t v) { if (threadIdx.x == 0) *p = v; }
-__global__ void __launch_bounds__(TPB) k_dot_part(Fr* __restrict__ partials, const Fr* __restrict__ a, const Fr* __restrict__ b, size_t n) {
-    Fr acc[1] = {big_zero<8>()};
-    for (size_t i = (size_t)blockIdx.x * TPB + threadIdx.x; i < n; i += (size_t)gridDim.x * TPB) acc[0] = add(acc[0], mont_mul(a[i], b[i]));
-    block_reduce_store<1>(acc, partials);
 }
 // Optional timing of the hinted first round's launches with events on their own stream (measurement only).
 struct RoundTimer {
@@ -2553,7 +2721,6 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
     job.per_round = 11;
     job.n1 = n1;
     ZK_ARG(rounds <= FINISH_ROUNDS_MAX, "lookup sumcheck: too many rounds");
-    Scratch& sums = job.arena.add(sizeof(Fr) * 11 * rounds);
     // every round keeps its partial sums: one launch sums them all behind the last round
     size_t part_total = 0;
     {
@@ -2565,12 +2732,10 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         part_total += rounds_partials(std::min(D, RM_MAX_N), rounds, 11);
     }
     Scratch& part_all = job.arena.add(sizeof(Fr) * part_total);
-    if (sums.rc) return sums.rc;
     if (part_all.rc) return part_all.rc;
-    job.sums = sums.as<Fr>();
-    ZK_HIP(hipMemsetAsync(sums.p, 0, sizeof(Fr) * 11 * rounds, st));
-    FinishRounds fin;
-    memset(&fin, 0, sizeof(fin));
+    int prc = sumjob_results(job);
+    if (prc) return prc;
+    FinishRounds& fin = job.fin;
     size_t part_at = 0;
     int fin_rounds = 0;              // rounds whose sums come from partials (the rest: the tail kernel's)
     PartSlice part{nullptr};
@@ -2719,7 +2884,7 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         if (nE) cE = nE;
     }
     if (fin_rounds) {
-        hipLaunchKernelGGL(k_finish_rounds, dim3(11, fin_rounds), dim3(TPB), 0, st, sums.as<Fr>(), part_all.as<Fr>(), fin, 11u);
+        hipLaunchKernelGGL(k_finish_rounds, dim3(11, fin_rounds + 1), dim3(TPB), 0, st, job.sums, part_all.as<Fr>(), fin, 11u);
         ZK_LAUNCH_CHECK();
     }
     return 0;
@@ -2731,7 +2896,6 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
     job.rounds = rounds;
     job.per_round = K + 1;
     ZK_ARG(rounds <= FINISH_ROUNDS_MAX, "Hadamard sumcheck: too many rounds");
-    Scratch& sums = job.arena.add(sizeof(Fr) * (K + 1) * rounds);
     size_t part_total = 0;            // every round keeps its partial sums: one launch sums them all behind the last round
     {
         size_t c = N;
@@ -2739,11 +2903,10 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
         part_total += rounds_partials(std::min(N, RM_MAX_N), rounds, (uint32_t)(K + 1));
     }
     Scratch& part_all = job.arena.add(sizeof(Fr) * part_total);
-    if (sums.rc) return sums.rc;
     if (part_all.rc) return part_all.rc;
-    job.sums = sums.as<Fr>();
-    FinishRounds fin;
-    memset(&fin, 0, sizeof(fin));
+    int prc = sumjob_results(job);
+    if (prc) return prc;
+    FinishRounds& fin = job.fin;
     size_t part_at = 0;
     int fin_rounds = 0;
     PartSlice part{nullptr};
@@ -2769,7 +2932,7 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
             TailV vs;
             for (int i = 0; i < TAIL_ROUNDS; ++i) vs.v[i] = i < rest ? to_mont(load_fr(v + 8 * (r + i))) : big_zero<8>();
             Fr* w = work.as<Fr>();
-            Fr* so = sums.as<Fr>() + (size_t)r * (K + 1);
+            Fr* so = job.sums + (size_t)r * (K + 1);
 #define HADS_TAIL(KK)                                                                                                                       \
     case KK: {                                                                                                                              \
         PtrPack<KK> p;                                                                                                                      \
@@ -2822,39 +2985,24 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
         if (nE) cE = nE;
     }
     if (fin_rounds) {
-        hipLaunchKernelGGL(k_finish_rounds, dim3(K + 1, fin_rounds), dim3(TPB), 0, st, sums.as<Fr>(), part_all.as<Fr>(), fin, (uint32_t)(K + 1));
+        hipLaunchKernelGGL(k_finish_rounds, dim3(K + 1, fin_rounds + 1), dim3(TPB), 0, st, job.sums, part_all.as<Fr>(), fin, (uint32_t)(K + 1));
         ZK_LAUNCH_CHECK();
     }
     return 0;
 }
-// waits for the job's stream and copies its sums (and the extra value) to the host
-// a job on a side stream: the copy of its results is queued with it, and collecting waits for that copy only
+// a job on a side stream: its results are there when the event behind its last kernel is reached
 static int sumjob_queue_results(SumJob& job) {
-    const size_t nsum = (size_t)job.rounds * job.per_round;
-    int rc = pinned_acquire(&job.host);
-    if (rc) return rc;
-    ZK_HIP(hipMemcpyAsync(job.host, job.sums, sizeof(Fr) * nsum, hipMemcpyDeviceToHost, job.st));
-    if (job.extra) ZK_HIP(hipMemcpyAsync((Fr*)job.host + nsum, job.extra, sizeof(Fr), hipMemcpyDeviceToHost, job.st));
     ZK_HIP(hipEventCreateWithFlags(&job.done, hipEventDisableTiming));
     ZK_HIP(hipEventRecord(job.done, job.st));
     return 0;
 }
+// waits for the job's last kernel and hands its sums (and the extra value) out
 static int sumjob_collect(SumJob& job, Fr* sums_host, Fr* extra_host) {
     const size_t nsum = (size_t)job.rounds * job.per_round;
-    if (job.done) {
-        ZK_HIP(hipEventSynchronize(job.done));
-        memcpy(sums_host, job.host, sizeof(Fr) * nsum);
-        if (job.extra && extra_host) memcpy(extra_host, (Fr*)job.host + nsum, sizeof(Fr));
-        return 0;
-    }
-    void* stage = nullptr;
-    int rc = staging(&stage, sizeof(Fr) * (nsum + 1));
-    if (rc) return rc;
-    ZK_HIP(hipMemcpyAsync(stage, job.sums, sizeof(Fr) * nsum, hipMemcpyDeviceToHost, job.st));
-    if (job.extra) ZK_HIP(hipMemcpyAsync((Fr*)stage + nsum, job.extra, sizeof(Fr), hipMemcpyDeviceToHost, job.st));
-    ZK_HIP(hipStreamSynchronize(job.st));
-    memcpy(sums_host, stage, sizeof(Fr) * nsum);
-    if (job.extra && extra_host) memcpy(extra_host, (Fr*)stage + nsum, sizeof(Fr));
+    if (job.done) ZK_HIP(hipEventSynchronize(job.done));
+    else ZK_HIP(hipStreamSynchronize(job.st));
+    memcpy(sums_host, job.host, sizeof(Fr) * nsum);
+    if (job.extra && extra_host) memcpy(extra_host, (Fr*)job.host + nsum, sizeof(Fr));
     return 0;
 }
 // the R corrections of the lookup sums: E carries R, each product one R^-1 (same as zk_lookup_round)
@@ -2929,7 +3077,6 @@ static void sumjob_abort(SumJob* job) {
     else if (job->st) (void)hipStreamSynchronize(job->st);
     job->arena.mark_idle();          // the job's kernels have all finished
     if (job->done) (void)hipEventDestroy(job->done);
-    pinned_release(job->host);
     if (job->ready) (void)hipEventDestroy(job->ready);
     delete job;
 }
@@ -2984,29 +3131,30 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     const LookupInts* ints = have_ints ? &li : nullptr;
     hipStream_t st = job->st;
     Scratch& B = job->arena.add(sizeof(Fr) * N);
-    Scratch& dp = job->arena.add(sizeof(Fr) * (reduce_grid(N) + 1));
-    if (B.rc || dp.rc) return B.rc ? B.rc : dp.rc;
-    rc = batch_inv_queue(B.as<Fr>(), (const Fr*)T, b, N, st);
+    Scratch& dp = job->arena.add(sizeof(Fr) * batch_inv_grid(N));
+    Scratch& TB = job->arena.add(hint ? sizeof(Fr) * 2 * N : 1);
+    Scratch& want = job->arena.add(hint && ints ? sizeof(int32_t) * (N + 1) : 1);         // the last slot: n_ok
+    for (const Scratch* x : {&B, &dp, &TB, &want})
+        if (x->rc) return x->rc;
+    uint32_t* const n_ok = hint && ints ? (uint32_t*)(want.as<int32_t>() + N) : nullptr;
+    // ZKLLM_LOOKUP_TRUSTED=0: no entry counts as checked and no output as gathered from the table -- every query goes
+    // through its own comparison (to compare the two paths)
+    static const bool trust = [] { const char* e = getenv("ZKLLM_LOOKUP_TRUSTED"); return !(e && e[0] == '0'); }();
+    // the table's inverses, each beside its entry, and the parts of <B, m>
+    rc = batch_inv_queue(B.as<Fr>(), (const Fr*)T, b, N, st, InvRiders{hint ? TB.as<Fr>() : nullptr, (const Fr*)m, dp.as<Fr>(), n_ok, trust ? 0xFFFFFFFFu : 0u});
+    job->fin.extra = dp.as<Fr>();
+    job->fin.extra_nb = batch_inv_grid(N);
+    job->extra = true;
     const Fr* Aptr = nullptr;
     HintSrc hs;
     if (rc == 0 && hint) {
-        Scratch& TB = job->arena.add(sizeof(Fr) * 2 * N);
-        if (TB.rc) return TB.rc;
-        hipLaunchKernelGGL(k_interleave, dim3(cdiv(N, TPB)), dim3(TPB), 0, st, TB.as<Fr>(), (const Fr*)T, B.as<Fr>(), N);
         hs.TB = TB.as<Fr>(); hs.hint = (const Fr*)hint; hs.low = fr_from_i64((int64_t)low); hs.beta = b; hs.N = (uint32_t)N;
         if (S_out) { hs.S_out = (const Fr*)S_out; hs.r_mont = to_mont(r_val); }
         if (ints) {
-            Scratch& want = job->arena.add(sizeof(int32_t) * (N + 1));         // the last slot: n_ok
-            if (want.rc) return want.rc;
             const int32_t* mi = S_out ? ((const FoldPrepared*)ints->mapped)->ints : nullptr;
-            uint32_t* n_ok = (uint32_t*)(want.as<int32_t>() + N);
-            // ZKLLM_LOOKUP_TRUSTED=0: no entry counts as checked and no output as gathered from the table -- every query goes
-            // through its own comparison (to compare the two paths)
-            static const bool trust = [] { const char* e = getenv("ZKLLM_LOOKUP_TRUSTED"); return !(e && e[0] == '0'); }();
-            hipLaunchKernelGGL(k_u32_set, dim3(1), dim3(64), 0, st, n_ok, trust ? 0xFFFFFFFFu : 0u);      // a kernel, not a memset node: callers may capture this
             hipLaunchKernelGGL(k_lookup_ints_check, dim3(cdiv(N, TPB)), dim3(TPB), 0, st, want.as<int32_t>(), n_ok, TB.as<Fr>(), mi, hs.r_mont, low, (uint32_t)N);
             hs.n_ok = n_ok;
-            job->n_ok_dev = n_ok;
+            job->fin.word = n_ok;
             job->n_table = (uint32_t)N;
             if (S_out) {
                 const FoldPrepared *q = (const FoldPrepared*)ints->queries, *o = (const FoldPrepared*)ints->out, *mp = (const FoldPrepared*)ints->mapped;
@@ -3024,10 +3172,6 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
         Aptr = A.as<Fr>();
     }
     if (rc) return rc;
-    const unsigned nb = reduce_grid(N);
-    hipLaunchKernelGGL(k_dot_part, dim3(nb), dim3(TPB), 0, st, dp.as<Fr>() + 1, B.as<Fr>(), (const Fr*)m, N);
-    hipLaunchKernelGGL(k_finish, dim3(1), dim3(TPB), 0, st, dp.as<Fr>(), dp.as<Fr>() + 1, nb);
-    job->extra = dp.as<Fr>();
     rc = shared_eq_get(job->eq, u_eq, rounds - 1, job->arena, st);
     if (rc) return rc;
     if (eq_prefix_on()) (void)eq_prefix_scales(job->eq_scale, u_eq, rounds);
@@ -3094,9 +3238,10 @@ int zk_lookup_prove_end(void* handle, uint32_t* bm_host, uint32_t* sums_host) {
     if (rc) { sumjob_abort(job); return rc; }
     rc = sumjob_collect(*job, (Fr*)sums_host, &bm);
     g_last_n_ok = g_last_n_table = 0;
-    if (!rc && job->n_ok_dev) {          // the job's kernels have finished
-        uint32_t v = 0;
-        if (hipMemcpy(&v, job->n_ok_dev, sizeof(uint32_t), hipMemcpyDeviceToHost) == hipSuccess) { g_last_n_ok = v < job->n_table ? v : job->n_table; g_last_n_table = job->n_table; }
+    if (!rc && job->fin.word) {
+        const uint32_t v = job->sums[job->fin.slot + 1].v[0];
+        g_last_n_ok = v < job->n_table ? v : job->n_table;
+        g_last_n_table = job->n_table;
     }
     if (!rc) {
         eq_prefix_apply(*job, (Fr*)sums_host, 0x0E7u);      // sums 0..2 and 5..7: sums 3, 4 and 8..10 carry no eq weight
@@ -3218,8 +3363,8 @@ int zk_hadamard_prove_end(void* handle, uint32_t* coefs_host) {
 // hadamard_product_sumcheck (proof.cu:66-109): k rounds over a, b of n elements (2^(k-1) < n <= 2^k), evaluation
 // challenges u and fold challenges v, both in the order the reference consumes them (first challenge first).
 // proof_host: 3k + 2 values -- per round the three evaluated terms, then the fully folded a and b.  Neither input is modified.
-// the launches of hadamard_product_sumcheck on st, its buffers from `arena`; *sums_out: the 3k + 2 values on the device
-static int hp_sumcheck_queue(Fr** sums_out, Arena& arena, const void* a, const void* b, const uint32_t* u, const uint32_t* v, size_t n, int k, hipStream_t st) {
+// the launches of hadamard_product_sumcheck on st, its buffers from `arena`; sums: the 3k + 2 values, in memory that the device writes to
+static int hp_sumcheck_queue(Fr* sums, Arena& arena, const void* a, const void* b, const uint32_t* u, const uint32_t* v, size_t n, int k, hipStream_t st) {
     const size_t half = (n + 1) / 2, etab = (size_t)1 << (k - 1);
     Scratch& E = arena.add(sizeof(Fr) * (etab + etab / 2 + 1));          // eq tables, ping-pong
     Scratch& W = arena.add(sizeof(Fr) * 2 * (half + (half + 1) / 2 + 1));   // folded a, b, ping-pong
@@ -3229,8 +3374,7 @@ static int hp_sumcheck_queue(Fr** sums_out, Arena& arena, const void* a, const v
         for (int r = 0; r < k; ++r) { c = (c + 1) / 2; part_total += 3 * (size_t)reduce_grid(c); }
     }
     Scratch& part = arena.add(sizeof(Fr) * part_total);
-    Scratch& sums = arena.add(sizeof(Fr) * (3 * (size_t)k + 2));
-    if (E.rc || W.rc || part.rc || sums.rc) return E.rc ? E.rc : (W.rc ? W.rc : (part.rc ? part.rc : sums.rc));
+    if (E.rc || W.rc || part.rc) return E.rc ? E.rc : (W.rc ? W.rc : part.rc);
     FinishRounds fin;
     memset(&fin, 0, sizeof(fin));
     size_t part_at = 0;
@@ -3253,11 +3397,9 @@ static int hp_sumcheck_queue(Fr** sums_out, Arena& arena, const void* a, const v
         cur = out;
         ecur /= 2;
     }
-    hipLaunchKernelGGL(k_finish_rounds, dim3(3, k), dim3(TPB), 0, st, sums.as<Fr>(), part.as<Fr>(), fin, 3u);
+    fin.v0 = ca; fin.v1 = cb; fin.slot = 3u * (uint32_t)k;
+    hipLaunchKernelGGL(k_finish_rounds, dim3(3, k + 1), dim3(TPB), 0, st, sums, part.as<Fr>(), fin, 3u);
     ZK_LAUNCH_CHECK();
-    ZK_HIP(hipMemcpyAsync(sums.as<Fr>() + 3 * (size_t)k, ca, sizeof(Fr), hipMemcpyDeviceToDevice, st));
-    ZK_HIP(hipMemcpyAsync(sums.as<Fr>() + 3 * (size_t)k + 1, cb, sizeof(Fr), hipMemcpyDeviceToDevice, st));
-    *sums_out = sums.as<Fr>();
     return 0;
 }
 int zk_hadamard_product_sumcheck(uint32_t* proof_host, const void* a, const void* b, const uint32_t* u, const uint32_t* v, size_t n, int k, void* stv) {
@@ -3265,13 +3407,11 @@ int zk_hadamard_product_sumcheck(uint32_t* proof_host, const void* a, const void
     ZK_ARG(k >= 1 && k <= 30 && n <= ((size_t)1 << k) && n > ((size_t)1 << (k - 1)), "zk_hadamard_product_sumcheck: n does not match the number of challenges");
     ZK_ARG(sizeof(Fr) * (3 * (size_t)k + 2) <= 65536, "zk_hadamard_product_sumcheck: too many rounds for the staging buffer");
     Arena arena(st);
-    Fr* sums = nullptr;
-    int rc = hp_sumcheck_queue(&sums, arena, a, b, u, v, n, k, st);
-    if (rc) { (void)hipStreamSynchronize(st); return rc; }
     void* stage = nullptr;
-    rc = staging(&stage, sizeof(Fr) * (3 * (size_t)k + 2));
+    int rc = staging(&stage, sizeof(Fr) * (3 * (size_t)k + 2));
+    if (rc) return rc;
+    rc = hp_sumcheck_queue((Fr*)stage, arena, a, b, u, v, n, k, st);
     if (rc) { (void)hipStreamSynchronize(st); return rc; }
-    ZK_HIP(hipMemcpyAsync(stage, sums, sizeof(Fr) * (3 * (size_t)k + 2), hipMemcpyDeviceToHost, st));
     ZK_HIP(hipStreamSynchronize(st));
     memcpy(proof_host, stage, sizeof(Fr) * (3 * (size_t)k + 2));
     return 0;
@@ -3290,7 +3430,8 @@ int zk_hadamard_product_sumcheck_begin(void** handle, const void* a, const void*
     job->rounds = 1;
     job->per_round = 3 * k + 2;
     rc = sumjob_launch(job, [=]() -> int {
-        int rc = hp_sumcheck_queue(&job->sums, job->arena, a, b, u_own.data(), v_own.data(), n, k, job->st);
+        int rc = sumjob_results(*job);
+        if (rc == 0) rc = hp_sumcheck_queue(job->sums, job->arena, a, b, u_own.data(), v_own.data(), n, k, job->st);
         if (rc == 0) rc = sumjob_queue_results(*job);
         return rc;
     });

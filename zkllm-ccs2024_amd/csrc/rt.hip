@@ -244,23 +244,28 @@ struct DeferBatch {
 };
 thread_local DeferBatch* g_defer = nullptr;
 }  // namespace
-int deliver(hipStream_t st, const void* dev_src, void* host_dst, size_t count_fr, int n_mont) {
+int deliver_begin(Delivery& d, size_t count_fr, int n_mont) {
     using Fr = Big<8>;
+    d.count = count_fr;
+    d.n_mont = n_mont;
+    d.deferred = false;
     if (DeferBatch* b = g_defer) {
         ZK_ARG((b->used + count_fr) * sizeof(Fr) <= ((size_t)64 << 10), "deferred results: more than 64 KiB in one batch");
-        ZK_HIP(hipMemcpyAsync((Fr*)b->pinned + b->used, dev_src, sizeof(Fr) * count_fr, hipMemcpyDeviceToHost, st));
+        d.deferred = true;
+        d.dst = (Fr*)b->pinned + b->used;
         if (n_mont > 0) b->monts.emplace_back(b->used, n_mont);
         b->used += count_fr;
         return 0;
     }
-    void* stage = nullptr;
-    int rc = staging(&stage, sizeof(Fr) * count_fr);
-    if (rc) return rc;
-    ZK_HIP(hipMemcpyAsync(stage, dev_src, sizeof(Fr) * count_fr, hipMemcpyDeviceToHost, st));
+    return staging(&d.dst, sizeof(Fr) * count_fr);
+}
+int deliver_end(const Delivery& d, hipStream_t st, void* host_dst) {
+    using Fr = Big<8>;
+    if (d.deferred) return 0;
     ZK_HIP(hipStreamSynchronize(st));
     Fr* out = (Fr*)host_dst;
-    memcpy(out, stage, sizeof(Fr) * count_fr);
-    for (int i = 0; i < n_mont; ++i) out[i] = to_mont(out[i]);
+    memcpy(out, d.dst, sizeof(Fr) * d.count);
+    for (int i = 0; i < d.n_mont; ++i) out[i] = to_mont(out[i]);
     return 0;
 }
 

@@ -14,22 +14,23 @@ static const Fr_t TWO_INV{{2147483649u, 2147483647u, 2147429887u, 2849952257u, 8
 tLookup::tLookup(const FrTensor& table) : table(table) {}
 tLookup::tLookup(FrTensor&& table) : table(std::move(table)) {}
 
+// multiplicities of a table's N entries from positions
 static FrTensor counts_to_m(const void* idx, uint D, uint N) {
-    DevBuf counts(sizeof(uint) * (size_t)N);
-    ZKC(zk_lookup_hist(counts.p, idx, D, N, nullptr));
     FrTensor m(N);
-    ZKC(zk_fr_from_u32(m.gpu_data, counts.p, N, nullptr));
-    ZKC(zk_sync(nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, idx, nullptr, nullptr, 0, N, D, N, nullptr));
     return m;
 }
-
 // the same from queries in int32 form: positions value - low formed by the counting passes themselves
 static FrTensor counts_to_m_i32(const void* vals_i32, int low, uint len, uint D, uint N) {
-    DevBuf counts(sizeof(uint) * (size_t)N);
-    ZKC(zk_lookup_hist_i32(counts.p, vals_i32, low, len, D, N, nullptr));
     FrTensor m(N);
-    ZKC(zk_fr_from_u32(m.gpu_data, counts.p, N, nullptr));
-    ZKC(zk_sync(nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, nullptr, vals_i32, nullptr, low, len, D, N, nullptr));
+    return m;
+}
+// and from the queries themselves, their positions with them where idx is given
+static FrTensor counts_to_m(void* idx, const FrTensor& vals, int low, uint len, uint N) {
+    const void* h = vals.kept_ints();
+    FrTensor m(N);
+    ZKC(zk_lookup_multiplicities(m.gpu_data, idx, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, N, nullptr));
     return m;
 }
 
@@ -43,17 +44,7 @@ static FrTensor make_range_table(int low, uint len) {
 tLookupRange::tLookupRange(int low, uint len) : tLookup(make_range_table(low, len)), low(low), len(len) {}
 
 FrTensor tLookupRange::prep(const int* vals, const uint D) { return counts_to_m_i32(vals, low, len, D, table.size); }
-// table positions of the values: from their int32 form when the tensor keeps one
-static void index_of(void* idx, const FrTensor& vals, int low, uint len) {
-    if (const void* h = vals.kept_ints()) ZKC(zk_lookup_index_i32(idx, zk_fr_fold_prepared_ints(h), low, len, vals.size, nullptr));
-    else ZKC(zk_lookup_index_fr(idx, vals.gpu_data, low, len, vals.size, nullptr));
-}
-FrTensor tLookupRange::prep(const FrTensor& vals) {
-    if (const void* h = vals.kept_ints()) return counts_to_m_i32(zk_fr_fold_prepared_ints(h), low, len, vals.size, table.size);
-    DevBuf idx(sizeof(uint) * (size_t)vals.size);
-    index_of(idx.p, vals, low, len);
-    return counts_to_m(idx.p, vals.size, table.size);
-}
+FrTensor tLookupRange::prep(const FrTensor& vals) { return counts_to_m(nullptr, vals, low, len, table.size); }
 
 // mapped values padded by repeating the last one (tlookup.cu:435-444)
 static FrTensor make_mapped(uint len, const FrTensor& mvals) {
@@ -68,11 +59,10 @@ tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mval
 
 pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const int* vals, const uint D) {
     DevBuf idx(sizeof(uint) * (size_t)D);
-    ZKC(zk_lookup_index_i32(idx.p, vals, low, len, D, nullptr));
-    FrTensor m = counts_to_m(idx.p, D, table.size);
+    FrTensor m(table.size);
+    ZKC(zk_lookup_multiplicities(m.gpu_data, idx.p, nullptr, vals, nullptr, low, len, D, table.size, nullptr));
     FrTensor y(D);
     ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, idx.p, D, nullptr));
-    ZKC(zk_sync(nullptr));
     return {std::move(y), std::move(m)};
 }
 pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const FrTensor& vals) { return map(vals, nullptr); }
@@ -80,8 +70,7 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::map(const FrTensor& vals, const Fr
     // queries and mapped values in int32 form: nothing below needs the array of table positions
     const bool by_queries = mapped_vals.kept_ints() && vals.kept_ints();
     DevBuf idx(by_queries ? 4 : sizeof(uint) * (size_t)vals.size);
-    if (!by_queries) index_of(idx.p, vals, low, len);
-    FrTensor m = by_queries ? counts_to_m_i32(zk_fr_fold_prepared_ints(vals.kept_ints()), low, len, vals.size, table.size) : counts_to_m(idx.p, vals.size, table.size);
+    FrTensor m = counts_to_m(by_queries ? nullptr : idx.p, vals, low, len, table.size);
     const bool ints_only_out = unwritten && unwritten->size == vals.size && mapped_vals.kept_ints() && vals.kept_ints();
     FrTensor y = ints_only_out ? FrTensor::view(*unwritten) : FrTensor(vals.size);
     // mapped values that are 32-bit integers: the outputs get their int32 form with them
@@ -91,7 +80,6 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::map(const FrTensor& vals, const Fr
         ZKC(zk_fr_gather_by_queries_ints(ints_only_out ? nullptr : y.gpu_data, const_cast<void*>(y.kept_ints()), vals.kept_ints(), low, th, vals.size, nullptr));
     } else if (th) ZKC(zk_fr_gather_ints(y.gpu_data, y.ints_for_producer(), mapped_vals.gpu_data, th, idx.p, vals.size, nullptr));
     else ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, idx.p, vals.size, nullptr));
-    ZKC(zk_sync(nullptr));
     return {std::move(y), std::move(m)};
 }
 
