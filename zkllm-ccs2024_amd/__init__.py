@@ -26,13 +26,22 @@ def _load(path):
     return _libs[path]
 
 
+def _runtime_started():
+    """Whether this process has the GPU driver open already (torch.cuda.is_available() is enough)."""
+    try:
+        return any(os.readlink(f"/proc/self/fd/{fd}") == "/dev/kfd" for fd in os.listdir("/proc/self/fd") if os.path.islink(f"/proc/self/fd/{fd}"))
+    except OSError:
+        return False
+
+
 def _want_hw_queues():
     """The library keeps up to seven streams busy (the caller's, four for openings, two for sumcheck jobs).  HIP maps
     streams onto GPU_MAX_HW_QUEUES hardware queues (4 unless set) and streams that share a queue run one after the
     other, so ask for at least sixteen (measured when this was added: the decoder layer took 7 % less time with 8 queues than with 4 and another 1 % less with 16).  The HIP runtime reads the variable when it is loaded: this must run before that.
-    ZKLLM_HW_QUEUES=0 leaves the variable alone, ZKLLM_HW_QUEUES=N sets it to N."""
+    ZKLLM_HW_QUEUES=0 leaves the variable alone, ZKLLM_HW_QUEUES=N sets it to N.  Once the runtime has started the variable says how
+    many queues there are (the library chooses its number of streams by it) and is left as it is."""
     want = os.environ.get("ZKLLM_HW_QUEUES", "")
-    if want == "0":
+    if want == "0" or _runtime_started():
         return
     try:
         cur = int(os.environ.get("GPU_MAX_HW_QUEUES", "0"))

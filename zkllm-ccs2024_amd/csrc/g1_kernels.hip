@@ -766,29 +766,38 @@ __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, c
 // over window sums afterwards.  k_msm_join adds the halves, the endomorphism on the second.
 // Raw buckets: buckets[(w nseg + seg) MT + b]; a half's total goes to its first bucket's place, which only its own workgroup reads.
 // The walk is one chain, so a launch takes what one chain takes whatever the number of sums: all of a job's sums that nothing waits for
-// go into one launch.  On one lane the chain is 1400 products deep, 1.6 ms; four lanes that share a point's products: 0.8 ms.
+// go into one launch.  A lane's chain takes 1.5 ms; four lanes that share a point's products take 1.25 ms, and a compute unit holds one
+// such workgroup: LANES is four while all of a launch's fit beside each other, one for longer lists (310 workgroups of four took 2.6 ms).
 struct PointDesc { J29* buckets; G1Jac* out; uint32_t nseg, pad; };
-__global__ void __launch_bounds__(4 * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list) {
+template <int LANES> __device__ __forceinline__ void walk_double(J29& p, uint32_t q) {
+    if constexpr (LANES == 4) j29_quad_double(p, q);
+    else j29_double_walk(p);
+}
+template <int LANES> __device__ __forceinline__ void walk_add(J29& a, const J29& b, uint32_t q) {
+    if constexpr (LANES == 4) j29_quad_add(a, b, q);
+    else a = j29_add(a, b);
+}
+template <int LANES> __global__ void __launch_bounds__(LANES * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list) {
     __shared__ uint32_t pool[J29_WORDS * MT / 2];
-    const uint32_t q = threadIdx.x & 3u, b = threadIdx.x >> 2, half = blockIdx.y;
+    const uint32_t q = threadIdx.x % LANES, b = threadIdx.x / LANES, half = blockIdx.y;
     const PointDesc d = list[blockIdx.x];
     J29* const mine = d.buckets + (size_t)half * MWH * d.nseg * MT;
     J29 r = j29_infinity();
     for (int w = MWH - 1; w >= 0; --w) {
         if (__any(!r.inf))
-            for (int k = 0; k < 8; ++k) j29_quad_double(r, q);
+            for (int k = 0; k < 8; ++k) walk_double<LANES>(r, q);
         const J29* row = mine + (size_t)w * d.nseg * MT;
         for (uint32_t sg = 0; sg < d.nseg; ++sg) {
             const J29 p = row[(size_t)sg * MT + b];
-            if (__any(!p.inf)) j29_quad_add(r, p, q);
+            if (__any(!p.inf)) walk_add<LANES>(r, p, q);
         }
     }
     J29 s = j29_infinity();
     for (int bit = 7; bit >= 0; --bit) {
-        j29_quad_double(s, q);
+        walk_double<LANES>(s, q);
         J29 p = r;
         if (!(((b + 1) >> bit) & 1u)) p.inf = 1u;
-        j29_quad_add(s, p, q);
+        walk_add<LANES>(s, p, q);
     }
     for (uint32_t sd = MT / 2; sd > 0; sd >>= 1) {
         __syncthreads();
@@ -803,7 +812,7 @@ __global__ void __launch_bounds__(4 * MT) __attribute__((amdgpu_waves_per_eu(2, 
             uint32_t* py = reinterpret_cast<uint32_t*>(&y);
 #pragma unroll
             for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (MT / 2) + b];
-            j29_quad_add(s, y, q);
+            walk_add<LANES>(s, y, q);
         }
     }
     if (threadIdx.x == 0) *mine = s;
@@ -1667,7 +1676,8 @@ static int points_queue(std::vector<PointDesc>& list, JobUploads& up, hipStream_
     const void* dl = nullptr;
     int rc = up.put(list.data(), sizeof(PointDesc) * list.size(), st, &dl);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_msm_point, dim3((unsigned)list.size(), 2), dim3(4 * MT), 0, st, (const PointDesc*)dl);
+    if (list.size() <= 96) hipLaunchKernelGGL(k_msm_point<4>, dim3((unsigned)list.size(), 2), dim3(4 * MT), 0, st, (const PointDesc*)dl);
+    else hipLaunchKernelGGL(k_msm_point<1>, dim3((unsigned)list.size(), 2), dim3(MT), 0, st, (const PointDesc*)dl);
     hipLaunchKernelGGL(k_msm_join, dim3(cdiv(4 * list.size(), (size_t)GT)), dim3(GT), 0, st, (const PointDesc*)dl, (uint32_t)list.size());
     ZK_LAUNCH_CHECK();
     list.clear();
@@ -2411,7 +2421,9 @@ int zk_g1_open(uint32_t* proof_host, uint32_t* final_scalar_host, const void* sc
 // must stay alive and unmodified until end, which waits for the opening, delivers its results and releases its buffers.
 static int open_begin_impl(void** handle, const OpenItem* items, int count, size_t n, int rounds, void* stv) {
     ZK_ARG(handle != nullptr, "zk_g1_open_begin: null handle");
-    hipStream_t side = side_stream(0), aux = side_stream(0);      // consecutive streams of the pool: the folds on one, the bucket sums on the other
+    // Consecutive streams of the pool: the folds on one, the bucket sums on the other.  A job whose rounds are one batch has no folds: one
+    // stream, so that the others (and their hardware queues) are left to other jobs.
+    hipStream_t side = side_stream(0), aux = n * (size_t)count <= (size_t)LAST_N && rounds <= TAIL_LEVELS ? side : side_stream(0);
     ZK_ARG(side != nullptr && aux != nullptr, "zk_g1_open_begin: could not create a stream");
     // what open_queue refuses is refused here, before anything is handed to the launch thread
     ZK_ARG(n >= 1, "zk_g1_open: empty input");
