@@ -68,6 +68,7 @@ int zk_defer_wait(void* batch, uint32_t* out_host, size_t max_fr, size_t* n_fr);
 int zk_defer_free(void* batch);
 /* replace cudaMemcpy in ctors, operator()(idx), savebin/loadbin (ioutils.cu:3-45) */
 int zk_memcpy_h2d(void* dst, const void* src_host, size_t bytes, void* stream);
+int zk_upload(void* dst, const void* src, size_t bytes, void* stream);          /* as zk_memcpy_h2d, for data that only work queued on `stream` reads: may return before it is there */
 int zk_memcpy_d2h(void* dst_host, const void* src, size_t bytes, void* stream);
 int zk_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
 int zk_memset(void* dst, int value, size_t bytes, void* stream);
@@ -310,7 +311,7 @@ int zk_lookup_index_fr(void* idx_u32, const void* vals_fr, int32_t low, uint32_t
 int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32_t table_size, size_t n, void* stream);
 /* multiplicities (tlookup_kernel :10-15): counts[b] = #{i : idx[i] == b}; counts is cleared first */
 /* multiplicities of a table's entries (nbins field elements) from positions, int32 queries or field elements, the first that is not null; idx_out: the positions too, or null */
-int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, void* stream);
+int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, int inside, void* stream);      /* inside: the caller knows every query to lie in the table; nothing is checked or waited for */
 int zk_lookup_hist(void* counts_u32, const void* idx_u32, size_t n, uint32_t nbins, void* stream);
 /* zk_lookup_index_i32 and zk_lookup_hist in one (tLookupRange::prep over queries that keep an int32 form): the counting passes
  * form the positions value - low themselves and no array of positions is written; a value outside [low, low + len) is an error */
@@ -407,6 +408,9 @@ int zk_rescale_ints_both(void* out, void* out_ints, int* out_fits_host, void* re
 /* the same with the answer left on the device: *bad_flag_dev (4 bytes of device memory) is cleared, then set by the kernel when a
  * rescaled value does not fit int32; the caller reads it (zk_memcpy_d2h) whenever the kernel is through and a wait costs nothing */
 int zk_rescale_ints_both_flag(void* out, void* out_ints, void* bad_flag_dev, void* rem, void* rem_ints, const void* in, uint32_t scaling_factor, size_t n, void* stream);
+/* out[i] = i < n ? in[i] : *fill for i < n_out; fill on the device (field elements / int32, the latter with the value where fill is null) */
+int zk_fr_pad_from(void* out, const void* in, size_t n, size_t n_out, const void* fill, void* stream);
+int zk_i32_pad_from(void* out_i32, const void* in_i32, size_t n, size_t n_out, const void* fill_i32, int32_t value, void* stream);
 int zk_i32_fill(void* dst_i32, int32_t value, size_t n, void* stream);       /* n int32 slots set to value (padding of an int32 form) */
 /* zkrelu_decomp_kernel zkrelu.cu:8-29: the same rescaling, then sign (1 when the rescaled value is >= 0), magnitude and max(., 0) */
 int zk_relu_decomp(void* res, void* sign, void* mag, void* rem, const void* in, uint32_t scaling_factor, size_t n, void* stream);

@@ -1922,7 +1922,7 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     Scratch ints(sizeof(int32_t) * total, st), stats(4 * CONV_STATS, st);
     if (ints.rc) return ints.rc;
     if (stats.rc) return stats.rc;
-    ZK_HIP(hipMemsetAsync(stats.p, 0, 4 * CONV_STATS, st));
+    if (const int crc = clear_words(stats.p, CONV_STATS, st)) return crc;
     hipLaunchKernelGGL(k_fr_to_i32_checked, dim3((unsigned)std::min<size_t>(cdiv(total, 256), 4096)), dim3(256), 0, st, ints.as<int32_t>(), stats.as<uint32_t>(), (const Fr*)scalars_fr, total);
     ZK_LAUNCH_CHECK();
     void* stage = nullptr;

@@ -380,12 +380,12 @@ __global__ void __launch_bounds__(64 * HW_SLICES) k_hist_wide_sum(Fr* __restrict
         v.v[0] = total;
         if (bin < nbins) m[bin] = v;
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) *host_flag = *flag;
+    if (host_flag && blockIdx.x == 0 && threadIdx.x == 0) *host_flag = *flag;
 }
 // counts as field elements; *host_flag = *flag
 __global__ void __launch_bounds__(TPB) k_hist_deliver(Fr* __restrict__ m, const uint32_t* __restrict__ counts, uint32_t nbins, const uint32_t* __restrict__ flag, uint32_t* __restrict__ host_flag) {
     const uint32_t i = blockIdx.x * TPB + threadIdx.x;
-    if (i == 0) *host_flag = *flag;
+    if (host_flag && i == 0) *host_flag = *flag;
     if (i >= nbins) return;
     Fr v = big_zero<8>();
     v.v[0] = counts[i];
@@ -1517,6 +1517,14 @@ __global__ void __launch_bounds__(TPB) k_rescale(Fr* __restrict__ out, Fr* __res
         if (x_rescaled != (int64_t)(int32_t)x_rescaled) atomicOr(flag, 1u);
     }
 }
+__global__ void __launch_bounds__(TPB) k_fr_pad_from(Fr* __restrict__ out, const Fr* __restrict__ in, size_t n, size_t n_out, const Fr* __restrict__ fill) {
+    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (i < n_out) out[i] = i < n ? in[i] : *fill;
+}
+__global__ void __launch_bounds__(TPB) k_i32_pad_from(int32_t* __restrict__ out, const int32_t* __restrict__ in, size_t n, size_t n_out, const int32_t* __restrict__ fill, int32_t value) {
+    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (i < n_out) out[i] = i < n ? in[i] : (fill ? *fill : value);
+}
 __global__ void __launch_bounds__(TPB) k_i32_fill(int32_t* __restrict__ dst, int32_t v, size_t n) {
     const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
     if (i < n) dst[i] = v;
@@ -2094,7 +2102,7 @@ int zk_lookup_index_fr(void* idx_u32, const void* vals, int32_t low, uint32_t ta
     if (n == 0) return 0;
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     LAUNCH1D(k_index_fr, n, st, (uint32_t*)idx_u32, flag.as<uint32_t>(), (const Fr*)vals, fr_from_i64((int64_t)low), table_size, n);
     uint32_t f = 0;
     int rc = read_flag(flag.as<uint32_t>(), &f, st);
@@ -2107,7 +2115,7 @@ int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32
     if (n == 0) return 0;
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     LAUNCH1D(k_index_i32, n, st, (uint32_t*)idx_u32, flag.as<uint32_t>(), (const int32_t*)vals_i32, low, table_size, n);
     uint32_t f = 0;
     int rc = read_flag(flag.as<uint32_t>(), &f, st);
@@ -2131,13 +2139,13 @@ static int hist_add_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t
     return 0;
 }
 static int hist_queue(uint32_t* counts, const KeySrc src, size_t n, uint32_t nbins, hipStream_t st) {
-    ZK_HIP(hipMemsetAsync(counts, 0, sizeof(uint32_t) * (size_t)nbins, st));
+    if (const int crc = clear_words(counts, nbins, st)) return crc;
     return hist_add_queue(counts, src, n, nbins, st);
 }
 // Multiplicities of a table's entries as field elements (m: nbins of them), from table positions (idx), queries in int32 form (vals_i32) or
 // queries as field elements (vals): the first that is not null.  A query outside [low, low + len) is an error.  idx_out (optional): the
-// positions too.  One wait, at the end.
-int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, void* stv) {
+// positions too.  One wait, at the end; none where `inside` says that no query can lie outside.
+int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, int inside, void* stv) {
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(nbins >= 1 && len >= 1 && len <= nbins, "zk_lookup_multiplicities: need 1 <= len <= nbins");
     ZK_ARG(m != nullptr && (idx != nullptr || vals_i32 != nullptr || vals != nullptr || n == 0), "zk_lookup_multiplicities: null argument");
@@ -2148,10 +2156,10 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
     if (counts.rc) return counts.rc;
     uint32_t* const flag = counts.as<uint32_t>();
     uint32_t* const c = flag + 1;
-    ZK_HIP(hipMemsetAsync(flag, 0, sizeof(uint32_t) * (wide ? 1 : (size_t)nbins + 1), st));
+    if (const int crc = clear_words(flag, wide ? 1 : (size_t)nbins + 1, st)) return crc;
     void* stage = nullptr;
-    int rc = staging(&stage, 4);
-    if (rc) return rc;
+    int rc = 0;
+    if (!inside && (rc = staging(&stage, 4)) != 0) return rc;
     KeySrc src{(const uint32_t*)idx, (const int32_t*)vals_i32, low, len, flag};
     std::unique_ptr<Scratch> own;
     if (!idx && !vals_i32) {
@@ -2179,6 +2187,7 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
         hipLaunchKernelGGL(k_hist_deliver, dim3(cdiv(nbins, (unsigned)TPB)), dim3(TPB), 0, st, (Fr*)m, c, nbins, flag, (uint32_t*)stage);
     }
     ZK_LAUNCH_CHECK();
+    if (inside) return 0;
     ZK_HIP(hipStreamSynchronize(st));
     ZK_ARG(*(uint32_t*)stage == 0, "lookup: a value lies outside the table range");
     return 0;
@@ -2195,7 +2204,7 @@ int zk_lookup_hist_i32(void* counts_u32, const void* vals_i32, int32_t low, uint
     ZK_ARG(vals_i32 != nullptr || n == 0, "zk_lookup_hist_i32: null queries");
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     int rc = hist_queue((uint32_t*)counts_u32, KeySrc{nullptr, (const int32_t*)vals_i32, low, len, flag.as<uint32_t>()}, n, nbins, st);
     if (rc) return rc;
     uint32_t f = 0;
@@ -3468,7 +3477,7 @@ int zk_rescale_ints_both(void* out, void* out_ints, int* out_fits_host, void* re
     if (n == 0) return 0;
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     LAUNCH1D(k_rescale, n, st, (Fr*)out, (Fr*)rem, (int32_t*)rem_ints, (const Fr*)in, (int64_t)scaling_factor, n, (int32_t*)out_ints, flag.as<uint32_t>());
     uint32_t f = 0;
     int rc = read_flag(flag.as<uint32_t>(), &f, st);
@@ -3483,9 +3492,19 @@ int zk_rescale_ints_both_flag(void* out, void* out_ints, void* bad_flag_dev, voi
     ZK_ARG(scaling_factor >= 1, "zk_rescale: scaling factor is 0");
     ZK_ARG(out_ints != nullptr && bad_flag_dev != nullptr, "zk_rescale_ints_both_flag: null argument");
     ZK_ARG(rem != nullptr || rem_ints != nullptr, "zk_rescale_ints_both_flag: the remainders need at least one form");
-    ZK_HIP(hipMemsetAsync(bad_flag_dev, 0, 4, st));
+    if (const int crc = clear_words(bad_flag_dev, 1, st)) return crc;
     if (n == 0) return 0;
     LAUNCH1D(k_rescale, n, st, (Fr*)out, (Fr*)rem, (int32_t*)rem_ints, (const Fr*)in, (int64_t)scaling_factor, n, (int32_t*)out_ints, (uint32_t*)bad_flag_dev);
+    return 0;
+}
+int zk_fr_pad_from(void* out, const void* in, size_t n, size_t n_out, const void* fill, void* st) {
+    ZK_ARG(out != in && n <= n_out && (fill != nullptr || n == n_out), "zk_fr_pad_from: in place, shorter than the input or no value");
+    LAUNCH1D(k_fr_pad_from, n_out, st, (Fr*)out, (const Fr*)in, n, n_out, (const Fr*)fill);
+    return 0;
+}
+int zk_i32_pad_from(void* out, const void* in, size_t n, size_t n_out, const void* fill, int32_t value, void* st) {
+    ZK_ARG(out != in && n <= n_out, "zk_i32_pad_from: in place or shorter than the input");
+    LAUNCH1D(k_i32_pad_from, n_out, st, (int32_t*)out, (const int32_t*)in, n, n_out, (const int32_t*)fill, value);
     return 0;
 }
 int zk_i32_fill(void* dst, int32_t value, size_t n, void* st) {
@@ -3533,7 +3552,7 @@ static int softmax_shift_decompose(void* shift, void* out_shifted, void* const* 
     for (int i = 0; i < K; ++i) ZK_ARG(!ip.p[i] || bs.v[i] <= 0x80000000u, "zk_softmax_decompose_ints: a radix above 2^31 has no int32 plane");
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     hipLaunchKernelGGL(k_softmax_shift, dim3(cdiv(rows, TPB / 64)), dim3(TPB), 0, st, (Fr*)shift, (Fr*)out_shifted, (const Fr*)X, rows, cols, scale, pp, ip, flag.as<uint32_t>(), bs, K,
                        (const int64_t*)X64);
     ZK_LAUNCH_CHECK();
@@ -3560,7 +3579,7 @@ int zk_softmax_decompose_ints(void* const* planes, void* const* int_planes, cons
     for (int i = 0; i < K; ++i) ZK_ARG(bs.v[i] >= 1, "zk_softmax_decompose: zero radix");
     Scratch flag(4, st);
     if (flag.rc) return flag.rc;
-    ZK_HIP(hipMemsetAsync(flag.p, 0, 4, st));
+    if (const int crc = clear_words(flag.p, 1, st)) return crc;
     PlanePtrs pp;
     for (int i = 0; i < 8; ++i) pp.p[i] = i < K ? (Fr*)planes[i] : nullptr;
     for (int i = 0; i < K; ++i) ZK_ARG(pp.p[i] != nullptr, "zk_softmax_decompose: null plane");

@@ -839,7 +839,7 @@ static int matmul_dispatch(void* C, const void* A, const void* B, uint32_t batch
     if (mode != 1) {
         Scratch mx(3 * sizeof(unsigned long long), st);
         if (mx.rc) return mx.rc;
-        ZK_HIP(hipMemsetAsync(mx.p, 0, 3 * sizeof(unsigned long long), st));
+        if (const int crc = clear_words(mx.p, 6, st)) return crc;
         const size_t nb = (size_t)batch * N * P;
         if (examine) {
             planes4[0].reset(new Scratch((size_t)batch * M * 4 * Kp4, st));
@@ -937,7 +937,7 @@ int zk_fr_matmul_rhs_prepare(void** prepared, const void* B, uint32_t N, uint32_
     {
         Scratch mx(sizeof(unsigned long long), st);
         if (mx.rc) return mx.rc;
-        ZK_HIP(hipMemsetAsync(mx.p, 0, sizeof(unsigned long long), st));
+        if (const int crc = clear_words(mx.p, 2, st)) return crc;
         const size_t nb = (size_t)N * P;
         hipLaunchKernelGGL(k_absmax, dim3(absmax_grid(nb)), dim3(256), 0, st, mx.as<unsigned long long>(), (const Fr*)B, nb);
         ZK_LAUNCH_CHECK();

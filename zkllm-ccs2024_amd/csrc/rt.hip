@@ -1,4 +1,5 @@
 // Runtime pieces of the C ABI: device selection, the caching allocator, copies, error text.
+#include <algorithm>
 #include <cstdlib>
 #include <atomic>
 #include <condition_variable>
@@ -356,6 +357,27 @@ int staging(void** host_ptr, size_t bytes) {
     return 0;
 }
 
+// the runtime's own copies and fills cost their caller two to three times a launch
+struct SmallWords { uint32_t v[768]; };
+static __global__ void __launch_bounds__(256) k_small_words(uint32_t* __restrict__ dst, const SmallWords w, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += 256) dst[i] = w.v[i];
+}
+static __global__ void __launch_bounds__(256) k_copy_words(uint32_t* __restrict__ dst, const uint32_t* __restrict__ src, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+static __global__ void __launch_bounds__(256) k_copy_quads(uint4* __restrict__ dst, const uint4* __restrict__ src, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = src[i];
+}
+static __global__ void __launch_bounds__(256) k_clear_words(uint32_t* __restrict__ dst, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = 0u;
+}
+int clear_words(void* dst, size_t words, hipStream_t st) {
+    hipLaunchKernelGGL(k_clear_words, dim3((unsigned)std::min<size_t>(cdiv(words, 256), 4096)), dim3(256), 0, st, (uint32_t*)dst, words);
+    ZK_LAUNCH_CHECK();
+    return 0;
+}
+
 }  // namespace zk
 
 using namespace zk;
@@ -482,19 +504,45 @@ int zk_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream) {
     ZK_HIP(hipStreamSynchronize((hipStream_t)stream));
     return 0;
 }
+// For data that only work queued on `stream` reads: small arrays of words travel as a kernel's arguments, nothing is staged or waited for
+int zk_upload(void* dst, const void* src, size_t bytes, void* stream) {
+    if (bytes == 0 || bytes > sizeof(SmallWords) || bytes % 4 != 0 || (uintptr_t)dst % 4 != 0) return zk_memcpy_h2d(dst, src, bytes, stream);
+    SmallWords w;
+    memcpy(w.v, src, bytes);
+    hipLaunchKernelGGL(k_small_words, dim3(1), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, w, (uint32_t)(bytes / 4));
+    ZK_LAUNCH_CHECK();
+    return 0;
+}
+// up to 64 KiB: a kernel writes them to the thread's pinned buffer
 int zk_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
     if (!bytes) return 0;
+    if (bytes <= ((size_t)64 << 10) && bytes % 4 == 0 && (uintptr_t)src % 4 == 0) {
+        void* stage = nullptr;
+        const int rc = staging(&stage, bytes);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_copy_words, dim3(cdiv(bytes / 4, 256)), dim3(256), 0, (hipStream_t)stream, (uint32_t*)stage, (const uint32_t*)src, bytes / 4);
+        ZK_LAUNCH_CHECK();
+        ZK_HIP(hipStreamSynchronize((hipStream_t)stream));
+        memcpy(dst, stage, bytes);
+        return 0;
+    }
     ZK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, (hipStream_t)stream));
     ZK_HIP(hipStreamSynchronize((hipStream_t)stream));
     return 0;
 }
 int zk_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream) {
     if (!bytes) return 0;
+    if (((uintptr_t)dst | (uintptr_t)src | bytes) % 16 == 0) {
+        hipLaunchKernelGGL(k_copy_quads, dim3((unsigned)std::min<size_t>(cdiv(bytes / 16, 256), 8192)), dim3(256), 0, (hipStream_t)stream, (uint4*)dst, (const uint4*)src, bytes / 16);
+        ZK_LAUNCH_CHECK();
+        return 0;
+    }
     ZK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, (hipStream_t)stream));
     return 0;
 }
 int zk_memset(void* dst, int value, size_t bytes, void* stream) {
     if (!bytes) return 0;
+    if (value == 0 && bytes % 4 == 0 && (uintptr_t)dst % 4 == 0) return clear_words(dst, bytes / 4, (hipStream_t)stream);
     ZK_HIP(hipMemsetAsync(dst, value, bytes, (hipStream_t)stream));
     return 0;
 }

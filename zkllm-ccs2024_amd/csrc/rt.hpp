@@ -89,6 +89,9 @@ struct Delivery { void* dst = nullptr; size_t count = 0; int n_mont = 0; bool de
 int deliver_begin(Delivery& d, size_t count_fr, int n_mont);
 int deliver_end(const Delivery& d, hipStream_t st, void* host_dst);
 
+// `words` 32-bit words set to zero by a kernel (also where the call is captured into a graph)
+int clear_words(void* dst, size_t words, hipStream_t st);
+
 // Looks up, for the current device, the address of the device array behind zk_fr_sum_static (fr_kernels.hip); called
 // by zk_init so that the entry point itself has nothing left to set up.
 int fr_static_scratch_setup();

@@ -66,27 +66,35 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_,
         const bool ints_only = rem_tensor_ptr->kept_ints() && zk_lookup_ints_suffice(padded_size, tl_rem.table.size);
         auto padded = ints_only ? std::make_shared<FrTensor>(padded_size) : std::make_shared<FrTensor>(rem_tensor_ptr->pad({rem_tensor_ptr->size}));
         if (const void* h = rem_tensor_ptr->kept_ints()) {          // the int32 form is padded with the same zeros
-            char* dst = (char*)padded->ints_for_producer();
-            const size_t have = sizeof(int32_t) * (size_t)rem_tensor_ptr->size, all = sizeof(int32_t) * (size_t)padded->size;
-            ZKC(zk_memcpy_d2d(dst, zk_fr_fold_prepared_ints(h), have, nullptr));
-            ZKC(zk_memset(dst + have, 0, all - have, nullptr));
+            ZKC(zk_i32_pad_from(padded->ints_for_producer(), zk_fr_fold_prepared_ints(h), rem_tensor_ptr->size, padded->size, nullptr, 0, nullptr));
         }
         p.rem = padded;
     }
-    p.m.reset(new FrTensor(tl_rem.prep(*p.rem)));
+    p.m.reset(new FrTensor(tl_rem.prep_inside(*p.rem)));          // remainders of a division by the table's length
     // X_(u) and rem(u) in one pass over the two tensors (the padding of the remainders is zeros: the unpadded tensor has the same
     // extension and the others' length).  X = scaling_factor X_ + rem element by element, so X(u) is that combination of the two
     // values: X itself, 32 bytes an element, is read only with ZKLLM_CHECK_CLAIMS=1, which evaluates it and compares as
     // rescaling.cu:52-57 does.
     const char* check_env = getenv("ZKLLM_CHECK_CLAIMS");
     const bool read_X = check_env && check_env[0] == '1';
-    vector<Fr_t> ev = read_X ? FrTensor::me_batch({&X_, rem_tensor_ptr, &X}, u) : FrTensor::me_batch({&X_, rem_tensor_ptr}, u);
-    p.lhs = ev[0] * Fr_t({scaling_factor, 0, 0, 0, 0, 0, 0, 0}) + ev[1];
-    if (read_X && p.lhs != ev[2]) throw std::runtime_error("Error: the rem is not correct.");
+    if (read_X) {
+        const vector<Fr_t> ev = FrTensor::me_batch({&X_, rem_tensor_ptr, &X}, u);
+        p.lhs = ev[0] * Fr_t({scaling_factor, 0, 0, 0, 0, 0, 0, 0}) + ev[1];
+        if (p.lhs != ev[2]) throw std::runtime_error("Error: the rem is not correct.");
+    } else {          // the values are collected with the proof: nothing waits for them before the lookup's job is queued
+        p.evaluated.begin();
+        try { (void)FrTensor::me_batch({&X_, rem_tensor_ptr}, u); } catch (...) { p.evaluated.end(); throw; }
+        p.evaluated.end();
+        p.scaling_factor = scaling_factor;
+    }
     p.look = tl_rem.prove_begin(*p.rem, *p.m, rand_temp[0], rand_temp[1], u, v);
     return p;
 }
 void Rescaling::prove_end(Pending& p) {
+    if (p.evaluated) {
+        const vector<Fr_t> ev = p.evaluated.wait();
+        p.lhs = ev.at(0) * Fr_t({p.scaling_factor, 0, 0, 0, 0, 0, 0, 0}) + ev.at(1);
+    }
     zk_record(p.lhs);
     tLookup::prove_end(p.look);
     cout << "Rescaling proof complete." << endl;

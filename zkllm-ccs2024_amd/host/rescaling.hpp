@@ -32,6 +32,8 @@ class Rescaling {
     // in between may all be begun before the first is ended: challenges and entries keep their order.
     struct Pending {
         Fr_t lhs;
+        DeferredResults evaluated;       // the values lhs is made of, while they are on their way
+        uint scaling_factor = 0;
         std::shared_ptr<FrTensor> rem;   // the remainder tensor itself when its length is a power of two, else a padded copy
         std::unique_ptr<FrTensor> m;
         LookupPending look;

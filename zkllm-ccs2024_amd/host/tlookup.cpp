@@ -17,20 +17,20 @@ tLookup::tLookup(FrTensor&& table) : table(std::move(table)) {}
 // multiplicities of a table's N entries from positions
 static FrTensor counts_to_m(const void* idx, uint D, uint N) {
     FrTensor m(N);
-    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, idx, nullptr, nullptr, 0, N, D, N, nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, idx, nullptr, nullptr, 0, N, D, N, 0, nullptr));
     return m;
 }
 // the same from queries in int32 form: positions value - low formed by the counting passes themselves
 static FrTensor counts_to_m_i32(const void* vals_i32, int low, uint len, uint D, uint N) {
     FrTensor m(N);
-    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, nullptr, vals_i32, nullptr, low, len, D, N, nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, nullptr, vals_i32, nullptr, low, len, D, N, 0, nullptr));
     return m;
 }
 // and from the queries themselves, their positions with them where idx is given
-static FrTensor counts_to_m(void* idx, const FrTensor& vals, int low, uint len, uint N) {
+static FrTensor counts_to_m(void* idx, const FrTensor& vals, int low, uint len, uint N, bool inside = false) {
     const void* h = vals.kept_ints();
     FrTensor m(N);
-    ZKC(zk_lookup_multiplicities(m.gpu_data, idx, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, N, nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, idx, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, N, inside, nullptr));
     return m;
 }
 
@@ -45,12 +45,13 @@ tLookupRange::tLookupRange(int low, uint len) : tLookup(make_range_table(low, le
 
 FrTensor tLookupRange::prep(const int* vals, const uint D) { return counts_to_m_i32(vals, low, len, D, table.size); }
 FrTensor tLookupRange::prep(const FrTensor& vals) { return counts_to_m(nullptr, vals, low, len, table.size); }
+FrTensor tLookupRange::prep_inside(const FrTensor& vals) { return counts_to_m(nullptr, vals, low, len, table.size, true); }
 
 // mapped values padded by repeating the last one (tlookup.cu:435-444)
 static FrTensor make_mapped(uint len, const FrTensor& mvals) {
     if (mvals.size != len) throw std::runtime_error("mvals.size != len");
-    FrTensor out = FrTensor::filled(1u << ceilLog2(len), mvals(mvals.size - 1));
-    ZKC(zk_memcpy_d2d(out.gpu_data, mvals.gpu_data, sizeof(Fr_t) * (size_t)mvals.size, nullptr));
+    FrTensor out(1u << ceilLog2(len));
+    ZKC(zk_fr_pad_from(out.gpu_data, mvals.gpu_data, mvals.size, out.size, mvals.gpu_data + (mvals.size - 1), nullptr));
     return out;
 }
 tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mvals) : tLookupRange(low, len), mapped_vals(make_mapped(len, mvals)) {
@@ -60,7 +61,7 @@ tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mval
 pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const int* vals, const uint D) {
     DevBuf idx(sizeof(uint) * (size_t)D);
     FrTensor m(table.size);
-    ZKC(zk_lookup_multiplicities(m.gpu_data, idx.p, nullptr, vals, nullptr, low, len, D, table.size, nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, idx.p, nullptr, vals, nullptr, low, len, D, table.size, 0, nullptr));
     FrTensor y(D);
     ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, idx.p, D, nullptr));
     return {std::move(y), std::move(m)};
@@ -237,35 +238,23 @@ LookupPending tLookupRangeMapping::prove_begin(const FrTensor& S_in, const FrTen
     if (D != (1u << ceilLog2(D))) {
         // pad the queries with the first table entry and account for them in m[0] (tlookup.cu:502-510)
         const uint Dp = 1u << ceilLog2(D);
-        const Fr_t t0 = table(0), v0 = mapped_vals(0);
         // Queries that keep int32 forms are padded in that form; where the job reads nothing else (zk_lookup_ints_suffice) the
         // padded field elements are not written at all.
-        auto small = [](const Fr_t& x, int32_t& out) {          // x as an int32, if it is one
-            const Fr_t n = Fr_t{{0, 0, 0, 0, 0, 0, 0, 0}} - x;
-            auto one_limb = [](const Fr_t& y) { return !(y.val[1] | y.val[2] | y.val[3] | y.val[4] | y.val[5] | y.val[6] | y.val[7]) && y.val[0] < 0x80000000u; };
-            if (one_limb(x)) { out = (int32_t)x.val[0]; return true; }
-            if (one_limb(n)) { out = -(int32_t)n.val[0]; return true; }
-            return false;
-        };
-        int32_t t0i = 0, v0i = 0;
-        const bool ints = S_in.kept_ints() && S_out.kept_ints() && mapped_vals.kept_ints() && small(t0, t0i) && small(v0, v0i);
+        const bool ints = S_in.kept_ints() && S_out.kept_ints() && mapped_vals.kept_ints();
         const bool ints_only = ints && zk_lookup_ints_suffice(Dp, table.size);
-        auto padded = [&](const FrTensor& t, const Fr_t& fill, int32_t fill_i) {
-            FrTensor* p = ints_only ? new FrTensor(Dp) : new FrTensor(t.pad({D}, fill));
+        auto padded = [&](const FrTensor& t, const FrTensor& fill_from, const void* fill_ints) {
+            FrTensor* p = new FrTensor(Dp);
             keep.emplace_back(p);
-            if (ints) {
-                char* dst = (char*)p->ints_for_producer();
-                ZKC(zk_memcpy_d2d(dst, zk_fr_fold_prepared_ints(t.kept_ints()), sizeof(int32_t) * (size_t)D, nullptr));
-                ZKC(zk_i32_fill(dst + sizeof(int32_t) * (size_t)D, fill_i, Dp - D, nullptr));
-            }
+            if (!ints_only) ZKC(zk_fr_pad_from(p->gpu_data, t.gpu_data, D, Dp, fill_from.gpu_data, nullptr));
+            if (ints) ZKC(zk_i32_pad_from(p->ints_for_producer(), zk_fr_fold_prepared_ints(t.kept_ints()), D, Dp, fill_ints, low, nullptr));
             return p;
         };
-        si = padded(S_in, t0, t0i);
-        so = padded(S_out, v0, v0i);
+        si = padded(S_in, table, nullptr);          // the first table entry is low
+        so = padded(S_out, mapped_vals, ints ? zk_fr_fold_prepared_ints(mapped_vals.kept_ints()) : nullptr);
         keep.emplace_back(new FrTensor(m));
         FrTensor* m_ = keep.back().get();
-        Fr_t m0 = (*m_)(0) + Fr_t{{(1u << ceilLog2(D)) - D, 0, 0, 0, 0, 0, 0, 0}};
-        ZKC(zk_memcpy_h2d(m_->gpu_data, &m0, sizeof(Fr_t), nullptr));
+        const Fr_t more{{Dp - D, 0, 0, 0, 0, 0, 0, 0}};
+        ZKC(zk_fr_add_s(m_->gpu_data, m_->gpu_data, more.val, 1, nullptr));
         mm = m_;
     }
     const uint N = mm->size;

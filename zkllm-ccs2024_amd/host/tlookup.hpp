@@ -50,6 +50,7 @@ class tLookupRange : public tLookup {
 
     FrTensor prep(const int* vals, const uint D);   // vals: device pointer
     FrTensor prep(const FrTensor& vals);
+    FrTensor prep_inside(const FrTensor& vals);      // addition: for values known to lie in the range (no check, no wait)
 
     // the queries of a range lookup are their own hints for the table position (value - low)
     Fr_t prove(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v, vector<Polynomial>& proof);
