@@ -169,6 +169,12 @@ def test_partial_me_of_a_whole_axis(pv, orc, other, cur, win):
     assert (got == exp[:out_n[0]]).all()
 
 
+# short axes of small tensors in one launch: 16, 64 and 256 lanes an output, one term a lane and four, a window around them
+@pytest.mark.parametrize("other,cur,win", [(1, 1024, 1), (2, 1000, 3), (3, 257, 1), (5, 256, 2), (17, 65, 1), (1, 64, 500), (33, 33, 7), (100, 32, 10), (7, 17, 1), (1, 2, 1), (2000, 16, 1)])
+def test_partial_me_of_small_tensors(pv, orc, other, cur, win):
+    test_partial_me_of_a_whole_axis(pv, orc, other, cur, win)
+
+
 @pytest.mark.parametrize("n,win,k", [(32, 4, 3), (15, 3, 3), (18, 4, 3), (4096 * 16, 4096, 4), (11008 * 8, 8, 14)])
 def test_window_fold(pv, orc, n, win, k):
     A = mt_random_vec(np.random.RandomState(n % 1000), n)

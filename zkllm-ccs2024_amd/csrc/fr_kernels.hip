@@ -380,43 +380,68 @@ __global__ void __launch_bounds__(TPB) k_sum_partials(Fr* __restrict__ out, cons
     out[i] = s;
 }
 
-// Finishes a multilinear evaluation inside one workgroup: n <= 1024 values, k levels.
-struct FrPack12 { Fr x[12]; };
-static constexpr uint32_t ME_SMALL_MAX = 1024;
-__global__ void __launch_bounds__(TPB) k_me_small(Fr* __restrict__ out, const Fr* __restrict__ in, const FrPack12 xs, uint32_t n, uint32_t k) {
-    __shared__ uint32_t buf[8][ME_SMALL_MAX];
-    const uint32_t t = threadIdx.x;
-    for (uint32_t i = t; i < ME_SMALL_MAX; i += TPB) {
-        Fr v = (i < n) ? in[i] : big_zero<8>();
-#pragma unroll
-        for (int l = 0; l < 8; ++l) buf[l][i] = v.v[l];
+// Short axes of small tensors in one launch, where a launch's cost counts and not what it does: LANES lanes take an output, at most four
+// terms each, the weights out of two tables in the launch's arguments (lo: five bits, hi: the rest).
+struct EqSmall { Fr29 lo[32], hi[32]; };
+static constexpr uint32_t FOLD_SMALL_CUR = 1024;
+static constexpr size_t FOLD_SMALL_MAX = (size_t)1 << 15;
+template <int LANES> __global__ void __launch_bounds__(TPB) k_fold_small(Fr* __restrict__ out, const Fr* __restrict__ in, const EqSmall eq, uint32_t n_out, uint32_t n_in, uint32_t cur, uint32_t window) {
+    __shared__ uint32_t red[4][9];
+    const uint32_t t = threadIdx.x, ln = t % LANES, o = (blockIdx.x * TPB + t) / LANES;
+    const bool live = o < n_out;
+    const uint32_t z = live ? o / window : 0u, base = z * cur * window + (live ? o - z * window : 0u);
+    Wide29 acc = wide29_zero();
+    for (uint32_t j = ln; j < cur; j += LANES) {
+        const uint32_t at = base + j * window;
+        if (!live || at >= n_in) continue;
+        Fr29 e = eq.lo[j & 31u];
+        if (cur > 32u) e = fr29_mul(e, eq.hi[j >> 5]);
+        wide29_mac(acc, e, fr29_repack(in[at]));
     }
-    __syncthreads();
-    uint32_t cur = 1u << k;    // zero-extended length
-    for (uint32_t lvl = 0; lvl < k; ++lvl) {
-        const uint32_t half = cur >> 1;
-        Fr r[ME_SMALL_MAX / 2 / TPB];
-        int cnt = 0;
-        for (uint32_t j = t; j < half; j += TPB, ++cnt) {
-            Fr a, b;
+    const Fr29 s = fr29_canon<2>(wide29_redc(acc));
+    uint32_t l9[9];
 #pragma unroll
-            for (int l = 0; l < 8; ++l) { a.v[l] = buf[l][2 * j]; b.v[l] = buf[l][2 * j + 1]; }
-            r[cnt] = add(a, mont_mul(xs.x[lvl], sub(b, a)));
+    for (int l = 0; l < 9; ++l) l9[l] = (uint32_t)s.l[l];
+    if (LANES == 16) fr29_row_sum(l9);
+    else fr29_wave_sum(l9);
+    if (LANES == 256) {
+        if ((t & 63u) == 63u) {
+#pragma unroll
+            for (int l = 0; l < 9; ++l) red[t >> 6][l] = l9[l];
         }
         __syncthreads();
-        cnt = 0;
-        for (uint32_t j = t; j < half; j += TPB, ++cnt) {
+        if (t != TPB - 1) return;
 #pragma unroll
-            for (int l = 0; l < 8; ++l) buf[l][j] = r[cnt].v[l];
-        }
-        __syncthreads();
-        cur = half;
+        for (int l = 0; l < 9; ++l) l9[l] = red[0][l] + red[1][l] + red[2][l] + red[3][l];
+        fr29_carry_u(l9);
     }
-    if (t == 0) {
-        Fr v;
+    if (!live || ln != LANES - 1) return;
+    Fr29 x;
 #pragma unroll
-        for (int l = 0; l < 8; ++l) v.v[l] = buf[l][0];
-        out[0] = v;
+    for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+    out[o] = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));
+}
+// the eq tables of up to ten challenges, with the factor 2^261
+static void eq_small_tables(EqSmall& e, const Fr* u_mont, int levels);
+static int fold_small_queue(Fr* out, const Fr* in, const EqSmall& eq, uint32_t n_out, uint32_t n_in, uint32_t cur, uint32_t window, hipStream_t st) {
+    if (cur <= 64) hipLaunchKernelGGL(k_fold_small<16>, dim3(cdiv((size_t)n_out * 16, TPB)), dim3(TPB), 0, st, out, in, eq, n_out, n_in, cur, window);
+    else if (cur <= 256) hipLaunchKernelGGL(k_fold_small<64>, dim3(cdiv((size_t)n_out * 64, TPB)), dim3(TPB), 0, st, out, in, eq, n_out, n_in, cur, window);
+    else hipLaunchKernelGGL(k_fold_small<256>, dim3(n_out), dim3(TPB), 0, st, out, in, eq, n_out, n_in, cur, window);
+    ZK_LAUNCH_CHECK();
+    return 0;
+}
+static void eq_small_tables(EqSmall& e, const Fr* u_mont, int levels) {
+    int at = 0;
+    for (int f = 0; f < 2; ++f) {
+        Fr t[32];
+        t[0] = fr29_pack(fr29_2_261());
+        const int bits = f == 0 ? std::min(5, levels) : std::max(0, levels - 5);
+        for (int b = 0; b < bits; ++b, ++at)
+            for (int i = 0; i < (1 << b); ++i) {
+                t[i + (1 << b)] = mont_mul(t[i], u_mont[at]);
+                t[i] = sub(t[i], t[i + (1 << b)]);
+            }
+        for (int i = 0; i < (1 << bits); ++i) (f ? e.hi : e.lo)[i] = fr29_repack(t[i]);
     }
 }
 
@@ -857,6 +882,13 @@ int zk_fr_fold_axis_all(void* out, const void* in, const uint32_t* u, int levels
         if (chunks > 1) LAUNCH1D(k_sum_partials, n_out, st, (Fr*)out, part.as<Fr>(), n_out, chunks);
         return 0;
     }
+    if (whole && cur <= FOLD_SMALL_CUR && levels <= 10 && other * cur * window <= FOLD_SMALL_MAX) {
+        Fr um[10];
+        for (int i = 0; i < levels; ++i) um[i] = to_mont(load_fr(u + 8 * i));
+        EqSmall eq;
+        eq_small_tables(eq, um, levels);
+        return fold_small_queue((Fr*)out, (const Fr*)in, eq, (uint32_t)(other * window), (uint32_t)(other * cur * window), cur, (uint32_t)window, st);
+    }
     std::unique_ptr<Scratch> keep[2];
     const void* src = in;
     for (int done = 0, which = 0; done < levels; which ^= 1) {
@@ -888,7 +920,7 @@ int zk_fr_me(uint32_t* out_host, const void* a, size_t n, const uint32_t* u, int
     int done = 0;
     void* bufs[2] = {nullptr, nullptr};
     int which = 0, rc = 0;
-    while (cur > ME_SMALL_MAX && rc == 0) {
+    while (cur > FOLD_SMALL_CUR && rc == 0) {
         const int L = 3;
         const size_t next = (cur + 7) >> 3;
         if (!bufs[which]) rc = pool_alloc(&bufs[which], next * sizeof(Fr), st);
@@ -900,16 +932,16 @@ int zk_fr_me(uint32_t* out_host, const void* a, size_t n, const uint32_t* u, int
         done += L;
     }
     if (rc == 0) {
-        FrPack12 p;
         const int rest = k - done;
-        for (int i = 0; i < 12; ++i) p.x[i] = (i < rest) ? to_mont(load_fr(u + 8 * (done + i))) : big_zero<8>();
+        Fr um[10];
+        for (int i = 0; i < rest; ++i) um[i] = to_mont(load_fr(u + 8 * (done + i)));
+        EqSmall eq;
+        eq_small_tables(eq, um, rest);
         Delivery d;
         rc = deliver_begin(d, 1, 0);
         if (!rc) {
-            hipLaunchKernelGGL(k_me_small, dim3(1), dim3(TPB), 0, st, (Fr*)d.dst, cur_ptr, p, (uint32_t)cur, (uint32_t)rest);
-            hipError_t e = hipGetLastError();
-            if (e != hipSuccess) rc = hip_fail(e, "zk_fr_me", __FILE__, __LINE__);
-            else rc = deliver_end(d, st, out_host);
+            rc = fold_small_queue((Fr*)d.dst, cur_ptr, eq, 1u, (uint32_t)cur, (uint32_t)cur, 1u, st);
+            if (!rc) rc = deliver_end(d, st, out_host);
         }
     }
     for (int i = 0; i < 2; ++i) if (bufs[i]) pool_free(bufs[i], st);

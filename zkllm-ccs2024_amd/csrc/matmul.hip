@@ -445,7 +445,9 @@ __global__ void __launch_bounds__(256) k_split_cols(int8_t* __restrict__ planes,
 // Workgroups below nA take four rows of A, a wave a row; the others a 64 x 64 tile of B, which goes through LDS.
 // The digits of four elements become one word of each plane: on a wave that holds neighbours in neighbouring lanes, the lanes of four
 // exchange their words (quad permutations) and each keeps one plane's bytes.
-struct ExamineArgs { const Fr *A, *B; int8_t *pA, *pB; unsigned long long* out; uint32_t nA, rowsA, M, N, P, Kp, tilesP, tilesK; };
+// slots set: each wave of A (its largest magnitude and row sum) and behind them each workgroup of B (its largest) leaves its figures there
+// (pinned memory; the host takes the maxima) and out is not used: no clearing, no atomics and no copy for small products
+struct ExamineArgs { const Fr *A, *B; int8_t *pA, *pB; unsigned long long *out, *slots; uint32_t nA, rowsA, M, N, P, Kp, tilesP, tilesK; };
 __device__ __forceinline__ unsigned long long fr_magnitude(const Fr& x, bool& negative) {       // ~0: above 2^62
     unsigned long long v;
     negative = (x.v[2] | x.v[3] | x.v[4] | x.v[5] | x.v[6] | x.v[7]) != 0;
@@ -497,7 +499,10 @@ __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
             mx = om > mx ? om : mx;
             sum = sat_add(sum, os);
         }
-        if (lane == 0) { raise(g.out, mx); raise(g.out + 2, sum); }
+        if (lane == 0) {
+            if (g.slots) { g.slots[2 * row] = mx; g.slots[2 * row + 1] = sum; }
+            else { raise(g.out, mx); raise(g.out + 2, sum); }
+        }
         return;
     }
     const uint32_t idx = blockIdx.x - g.nA, per = g.tilesP * g.tilesK, b = idx / per, r = idx - b * per, tk = r / g.tilesP, tp = r - tk * g.tilesP;
@@ -532,7 +537,8 @@ __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
     __syncthreads();
     if (t == 0) {
         for (int i = 1; i < 4; ++i) mx = red[i] > mx ? red[i] : mx;
-        raise(g.out + 1, mx);
+        if (g.slots) g.slots[2 * g.rowsA + idx] = mx;
+        else raise(g.out + 1, mx);
     }
     const uint32_t row = t >> 2, ch = t & 3u;
     if (p0 + row < g.P)
@@ -837,16 +843,22 @@ static int matmul_dispatch(void* C, const void* A, const void* B, uint32_t batch
     const uint64_t tiles_b = (uint64_t)cdiv(P, 64) * (Kp4 / 64) * batch;
     const bool examine = mode != 1 && planes_wanted && !src.a && !b_transposed && cdiv((size_t)batch * M, 4) + tiles_b < (1ull << 31) && tiles_b < (1ull << 31);
     if (mode != 1) {
+        const size_t nslots = 2 * (size_t)batch * M + (rhs ? 0 : (size_t)tiles_b);
+        const bool by_slots = examine && nslots * sizeof(unsigned long long) <= ((size_t)16 << 10);
+        void* stage = nullptr;
+        int rc = staging(&stage, by_slots ? nslots * sizeof(unsigned long long) : 24);
+        if (rc) return rc;
         Scratch mx(3 * sizeof(unsigned long long), st);
         if (mx.rc) return mx.rc;
-        if (const int crc = clear_words(mx.p, 6, st)) return crc;
+        if (!by_slots)
+            if (const int crc = clear_words(mx.p, 6, st)) return crc;
         const size_t nb = (size_t)batch * N * P;
         if (examine) {
             planes4[0].reset(new Scratch((size_t)batch * M * 4 * Kp4, st));
             if (planes4[0]->rc) return planes4[0]->rc;
             ExamineArgs x;
             memset(&x, 0, sizeof(x));
-            x.A = (const Fr*)A; x.B = (const Fr*)B; x.pA = planes4[0]->as<int8_t>(); x.out = mx.as<unsigned long long>();
+            x.A = (const Fr*)A; x.B = (const Fr*)B; x.pA = planes4[0]->as<int8_t>(); x.out = mx.as<unsigned long long>(); x.slots = by_slots ? (unsigned long long*)stage : nullptr;
             x.rowsA = batch * M; x.M = M; x.N = N; x.P = P; x.Kp = Kp4; x.nA = cdiv(x.rowsA, 4);
             x.tilesP = cdiv(P, 64); x.tilesK = Kp4 / 64;
             if (!rhs) {
@@ -861,12 +873,18 @@ static int matmul_dispatch(void* C, const void* A, const void* B, uint32_t batch
         else hipLaunchKernelGGL(k_rowabs, dim3(batch * M), dim3(256), 0, st, mx.as<unsigned long long>() + 2, mx.as<unsigned long long>(), (const Fr*)A, N);      // one pass over A for both of its figures
         }
         ZK_LAUNCH_CHECK();
-        void* stage = nullptr;
-        int rc = staging(&stage, 24);
-        if (rc) return rc;
-        ZK_HIP(hipMemcpyAsync(stage, mx.p, 24, hipMemcpyDeviceToHost, st));
-        ZK_HIP(hipStreamSynchronize(st));
-        const unsigned long long ma = ((unsigned long long*)stage)[0], mb = rhs ? rhs->mb : ((unsigned long long*)stage)[1], ra = ((unsigned long long*)stage)[2];
+        unsigned long long fig[3] = {0, 0, 0};
+        if (by_slots) {
+            ZK_HIP(hipStreamSynchronize(st));
+            const unsigned long long* slot = (const unsigned long long*)stage;
+            for (size_t i = 0; i < (size_t)batch * M; ++i) { fig[0] = std::max(fig[0], slot[2 * i]); fig[2] = std::max(fig[2], slot[2 * i + 1]); }
+            for (size_t i = 2 * (size_t)batch * M; i < nslots; ++i) fig[1] = std::max(fig[1], slot[i]);
+        } else {
+            ZK_HIP(hipMemcpyAsync(stage, mx.p, 24, hipMemcpyDeviceToHost, st));
+            ZK_HIP(hipStreamSynchronize(st));
+            memcpy(fig, stage, 24);
+        }
+        const unsigned long long ma = fig[0], mb = rhs ? rhs->mb : fig[1], ra = fig[2];
         if (ma != ~0ull && mb != ~0ull && ra != ~0ull) {
             // |sum_j a_ij b_jk| <= (max_i sum_j |a_ij|) * max|b| must stay below 2^62
             const unsigned __int128 bound = (unsigned __int128)ra * mb;

@@ -487,6 +487,16 @@ Fr_t FrTensor::multi_dim_me(const vector<vector<Fr_t>>& us, const vector<uint>& 
     if (shape.size() != us.size()) throw std::runtime_error("Incompatible dimensions");
     if (shape.size() == 0) return (*this)(0);
     if (shape.size() == 1) return (*this)(us[0]);
+    // a small tensor whose inner dimensions are full is one axis: one launch
+    if (size <= 1024) {
+        bool full = true;
+        for (size_t i = 1; i < shape.size(); ++i) full = full && shape[i] == (1u << us[i].size());
+        if (full) {
+            vector<Fr_t> flat;
+            for (size_t i = us.size(); i-- > 0;) flat.insert(flat.end(), us[i].begin(), us[i].end());
+            return (*this)(flat);
+        }
+    }
     FrTensor t_new = this->partial_me(us.back(), shape.back(), 1);
     return t_new.multi_dim_me({us.begin(), us.end() - 1}, {shape.begin(), shape.end() - 1});
 }
