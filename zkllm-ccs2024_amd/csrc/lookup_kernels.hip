@@ -126,10 +126,11 @@ static inline unsigned reduce_grid(size_t n) {
     if (b < 1) b = 1;
     return (unsigned)b;
 }
-// the grid of a round that gives a lane `per_lane` pairs where the round has them: at least 64 workgroups, at most reduce_grid's
+// the grid of a round that gives a lane `per_lane` pairs where the round has them: at least 256 workgroups (one a CU: with 64, rounds
+// of 2^14 to 2^18 pairs left most of the chip idle -- a lookup of 2^22 queries 721 us, with 256 692), at most reduce_grid's
 static inline unsigned round_grid(size_t n, unsigned per_lane) {
     const size_t all = reduce_grid(n), want = n / ((size_t)TPB * per_lane);
-    return (unsigned)std::min(all, std::max<size_t>(64, want));
+    return (unsigned)std::min(all, std::max<size_t>(256, want));
 }
 // finish K sums (K x nb partials) where the host reads them, applying the R correction (to_mont)
 // to the first `n_mont` of them
