@@ -227,6 +227,27 @@ def test_open_with_equal_scalars(pv, orc, n, val):
     assert (norm(orc, proof) == norm(orc, exp_proof)).all()
 
 
+@pytest.mark.parametrize("counts", [[96, 97, 107], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
+def test_open_with_several_digits_shared_by_many_scalars(pv, orc, counts):
+    """Buckets about the size from which a workgroup shares them out, one and several of them, whose ends fall inside and at
+    the ends of the lanes' shares."""
+    n = sum(counts)
+    gens = oracle_gens(orc, 41 + n, n)
+    t = np.repeat(np.arange(1, len(counts) + 1), counts)
+    t[::3] *= -1
+    T = fr_array([int(x) % R_MOD for x in np.random.default_rng(n).permutation(t)])
+    k = (n - 1).bit_length()
+    u = mt_random_vec(np.random.RandomState(18), k)
+    exp_proof = np.zeros((3 * k + 1, 36), np.uint32)
+    exp_val = np.zeros(8, np.uint32)
+    orc_check(orc.orc_open(gens, n, T, n, 1, u, k, exp_proof, exp_val))
+    hG, hT = pv.g1_from_host(gens), pv.from_fr(T)
+    com = pv.commit_int(hG, hT)
+    val_got, proof = pv.open(hG, hT, com, u)
+    assert (val_got == exp_val).all()
+    assert (norm(orc, proof) == norm(orc, exp_proof)).all()
+
+
 def test_open_with_equal_opposite_and_infinite_generators_in_the_first_round(pv, orc):
     """More generators than the batched rest takes, so the first round halves them on the device: pairs of equal
     generators (their sum is a doubling), of opposite ones (their sum is infinity), with an infinite member, and an

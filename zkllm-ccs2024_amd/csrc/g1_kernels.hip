@@ -438,7 +438,7 @@ static constexpr int MWH = MW / 2;
 static constexpr int MT = 128;       // buckets of a window (digit magnitudes 1..128)
 static constexpr int MSEG = 4096;    // most elements of a chunk (12-bit list entries)
 static constexpr int MSL = 64;       // lanes of a bucket-accumulation workgroup (one wave): each takes two buckets of its chunk
-static constexpr int MHEAVY = 256;   // a bucket above this many elements of a chunk is summed by the whole workgroup
+static constexpr int MHEAVY = 96;    // a bucket above this many elements of a chunk is shared out over the workgroup
 struct MsmDesc { const int8_t* digits; const A29* base; uint32_t dstride, count, s_mul, s_off, b_mul, b_off; };   // element i: recoded scalar i*s_mul+s_off of dstride, point base[i*b_mul+b_off]
 static constexpr int OB_MAX = 8;           // openings of equal size that share their rounds' launches
 static constexpr int TABLE_MIN_N = 1024;   // results of a fold below which no fold tables are made for it
@@ -609,31 +609,8 @@ __global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t
     msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i]);
 }
 
-// sum over the NT lanes of a workgroup through the LDS pool (43 x NT words); lane 0 returns the total
 static constexpr int J29_WORDS = 43;
 static_assert(sizeof(J29) == 4 * J29_WORDS, "a point is its coordinates and its flag");
-template <int NT> __device__ __forceinline__ J29 j29_block_sum(uint32_t* pool, const J29& v, uint32_t t) {
-    J29 x = v;
-    for (uint32_t sd = NT / 2; sd > 0; sd >>= 1) {
-        __syncthreads();
-        if (t >= sd && t < 2 * sd) {
-            const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
-#pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) pool[l * (NT / 2) + t - sd] = src[l];
-        }
-        __syncthreads();
-        if (t < sd) {
-            J29 y;
-            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
-#pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (NT / 2) + t];
-            x = j29_add(x, y);
-        }
-    }
-    __syncthreads();
-    return x;
-}
-
 // One segment's share of sum over elements of digit_w(s) * base: the segment's MT raw buckets,
 // partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold / k_msm_point reduce them).
 // One wave per workgroup.  Per chunk of `chunk` elements (at most MSEG):
@@ -643,14 +620,19 @@ template <int NT> __device__ __forceinline__ J29 j29_block_sum(uint32_t* pool, c
 //     digits are Poisson(32), the largest of 64 is ~47, while the 64 pair sums all lie within a few elements of 64 -- the
 //     lanes walk their two lists as one sequence of mixed additions, in lockstep, and 96 % of the lane-steps add a point
 //     (67 % with one bucket per lane);
-//  3. a bucket with more than MHEAVY elements (scalars that share a digit: equal values, a common high byte) is left out
-//     of the lists and summed by all lanes together, each over its own share of the chunk.
+//  3. buckets with more than MHEAVY elements (scalars that share a digit: equal values, small integers, a common high byte) stand
+//     together at the end of the list, which the lanes divide evenly: a lane's share is shorter than such a bucket, so it holds parts of
+//     at most two.  A bucket that ends inside a share goes out there; the rest is a segmented scan over the lanes, six additions for
+//     all of them together.  An opening of 1 x 16384 small integers: 10.7 ms with a tree of six additions a bucket above 256
+//     elements and one lane's walk below, 5.0 ms so.
 __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(J29* __restrict__ partial, const MsmDesc* __restrict__ descs, uint32_t nseg, uint32_t chunks_per_seg, uint32_t chunk) {
     __shared__ uint32_t cnt[MT], off[MT], cursor[MT];
-    __shared__ uint8_t order[MT];
-    __shared__ uint32_t pool[J29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the point tree of the heavy buckets
+    __shared__ uint8_t order[MT], heavy[MT];
+    __shared__ uint32_t pool[J29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the points of the heavy buckets' scan
     static_assert(J29_WORDS * MSL * 4 >= MSEG * 2, "pool too small for the list");
     static_assert(MSEG <= 4096, "12-bit list entries");
+    static_assert(MSEG / MSL < MHEAVY, "a lane's share of the heavy buckets' list touches two of them at most");
+    static_assert(MT == 2 * MSL, "a lane counts two buckets");
     uint16_t* list = reinterpret_cast<uint16_t*>(pool);
     const MsmDesc d = descs[blockIdx.z];
     const A29* __restrict__ A = d.base;
@@ -671,12 +653,28 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             if (dg != 0) atomicAdd(&cnt[(dg < 0 ? -dg : dg) - 1], 1u);
         }
         __syncthreads();
-        if (t == 0) {
-            uint32_t run = 0;
-            for (uint32_t b = 0; b < (uint32_t)MT; ++b) {
-                off[b] = run; cursor[b] = run;
-                run += cnt[b] > (uint32_t)MHEAVY ? 0u : cnt[b];
+        // the lists one after the other, those of the heavy buckets last: lane t places buckets 2t and 2t + 1
+        uint32_t n_light, n_heavy, n_hb;
+        {
+            const uint32_t c0 = cnt[2 * t], c1 = cnt[2 * t + 1];
+            const bool h0 = c0 > (uint32_t)MHEAVY, h1 = c1 > (uint32_t)MHEAVY;
+            const uint32_t mine = (h0 ? 0u : c0) + (h1 ? 0u : c1);                                      // at most 2 MHEAVY
+            const uint32_t mine_h = (h0 ? c0 : 0u) + (h1 ? c1 : 0u);
+            uint32_t run = mine, run_h = mine_h | ((uint32_t)h0 + (uint32_t)h1) << 16;                   // elements, and buckets above bit 16
+            for (int sd = 1; sd < MSL; sd <<= 1) {
+                const uint32_t a = __shfl_up(run, sd), ah = __shfl_up(run_h, sd);
+                if (t >= (uint32_t)sd) { run += a; run_h += ah; }
             }
+            n_light = __shfl(run, MSL - 1);
+            n_heavy = __shfl(run_h, MSL - 1) & 0xFFFFu;
+            n_hb = __shfl(run_h, MSL - 1) >> 16;
+            const uint32_t l0 = run - mine, g0 = n_light + (run_h & 0xFFFFu) - mine_h;
+            const uint32_t o0 = h0 ? g0 : l0, o1 = h1 ? g0 + (h0 ? c0 : 0u) : l0 + (h0 ? 0u : c0);
+            off[2 * t] = o0; cursor[2 * t] = o0;
+            off[2 * t + 1] = o1; cursor[2 * t + 1] = o1;
+            const uint32_t k0 = (run_h >> 16) - (uint32_t)h0 - (uint32_t)h1;
+            if (h0) heavy[k0] = (uint8_t)(2 * t);
+            if (h1) heavy[k0 + (uint32_t)h0] = (uint8_t)(2 * t + 1);
         }
         // rank of a bucket by list length (heavy buckets have none), ties by index: a permutation
         for (uint32_t b = t; b < (uint32_t)MT; b += MSL) {
@@ -694,7 +692,6 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             const int dg = Dw[si];
             if (dg == 0) continue;
             const uint32_t mag = (uint32_t)(dg < 0 ? -dg : dg);
-            if (cnt[mag - 1] > (uint32_t)MHEAVY) continue;
             const uint32_t pos = atomicAdd(&cursor[mag - 1], 1u);
             list[pos] = (uint16_t)((e - e0) | (((dg < 0) != (((Df[si] >> half) & 1) != 0)) ? 0x8000u : 0u));
         }
@@ -727,20 +724,58 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
         }
         __threadfence_block();
         __syncthreads();
-        for (uint32_t b = 0; b < (uint32_t)MT; ++b) {
-            if (cnt[b] <= (uint32_t)MHEAVY) continue;          // the same for every lane
-            X29 h29 = x29_infinity();
-            for (uint32_t e = e0 + t; e < e1; e += MSL) {
-                const size_t si = (size_t)e * d.s_mul + d.s_off;
-                const int dg = Dw[si];
-                if ((uint32_t)(dg < 0 ? -dg : dg) != b + 1) continue;
-                A29 pt = A[(size_t)e * d.b_mul + d.b_off];
+        if (n_hb) {                                         // the same for every lane
+            const uint32_t share = (n_heavy + MSL - 1) / MSL, end = n_light + n_heavy;
+            const uint32_t p0 = min(n_light + t * share, end), p1 = min(p0 + share, end);
+            uint32_t k = 0;
+            while (k + 1 < n_hb && off[heavy[k + 1]] <= p0) ++k;
+            uint32_t b = heavy[k], b_end = off[b] + cnt[b];
+            bool start = p0 >= end || p0 == off[b];          // what the lane holds begins its bucket (or is nothing)
+            bool lacks = false;                             // bucket `split` went out without the shares before this lane's
+            uint32_t split = 0;
+            X29 acc29 = x29_infinity();
+            for (uint32_t pos = p0; pos < p1; ++pos) {
+                if (pos == b_end) {
+                    J29 v = j29_from_x29(acc29);
+                    if (!first) v = j29_add(out[b], v);
+                    out[b] = v;
+                    split = b; lacks = !start; start = true;
+                    acc29 = x29_infinity();
+                    b = heavy[++k]; b_end = off[b] + cnt[b];
+                }
+                const uint32_t en = list[pos];
+                A29 pt = A[(size_t)(e0 + (en & 0x7FFFu)) * d.b_mul + d.b_off];
                 if (a29_is_inf(pt)) continue;
-                if ((dg < 0) != (((Df[si] >> half) & 1) != 0)) pt.y = fq29_neg(pt.y);
-                x29_add_mixed(h29, pt);
+                if (en & 0x8000u) pt.y = fq29_neg(pt.y);
+                x29_add_mixed(acc29, pt);
             }
-            const J29 h = j29_block_sum<MSL>(pool, j29_from_x29(h29), t);
-            if (t == 0) out[b] = j29_add(out[b], h);            // its list was empty: the slot holds what earlier chunks left (or infinity)
+            const bool whole = p1 > p0 && p1 == b_end;       // the bucket ends with this share
+            // inclusive scan of the shares' last parts, begun anew where a bucket begins; the last step moves the sums up by a lane
+            J29 x = j29_from_x29(acc29);
+            uint32_t begun = start ? 1u : 0u;
+            for (uint32_t sd = 1; sd <= (uint32_t)MSL; sd <<= 1) {
+                const bool last = sd == (uint32_t)MSL;
+                const uint32_t from = last ? 1u : sd;
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
+                __syncthreads();
+#pragma unroll
+                for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
+                __syncthreads();
+                const uint32_t before = __shfl_up(begun, from);
+                if (last && whole) {
+                    if (!first) x = j29_add(out[b], x);
+                    out[b] = x;
+                }
+                if (last ? lacks : (t >= from && !begun)) {
+                    J29 y;
+                    uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+                    for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - from];
+                    if (last) out[split] = j29_add(out[split], y);
+                    else x = j29_add(x, y);
+                }
+                if (!last && t >= from) begun |= before;
+            }
         }
         __threadfence_block();
         __syncthreads();
