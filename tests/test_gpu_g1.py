@@ -227,9 +227,9 @@ def test_open_with_equal_scalars(pv, orc, n, val):
     assert (norm(orc, proof) == norm(orc, exp_proof)).all()
 
 
-@pytest.mark.parametrize("counts", [[96, 97, 107], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
+@pytest.mark.parametrize("counts", [[1, 64], [96, 97, 107], [400, 113], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
 def test_open_with_several_digits_shared_by_many_scalars(pv, orc, counts):
-    """Buckets about the size from which a workgroup shares them out, one and several of them, whose ends fall inside and at
+    """Few scalars (512 at most, a path of its own) and many: buckets about the size from which a workgroup shares them out, whose ends fall inside and at
     the ends of the lanes' shares."""
     n = sum(counts)
     gens = oracle_gens(orc, 41 + n, n)

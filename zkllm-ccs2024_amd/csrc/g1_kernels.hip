@@ -611,6 +611,44 @@ __global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t
 
 static constexpr int J29_WORDS = 43;
 static_assert(sizeof(J29) == 4 * J29_WORDS, "a point is its coordinates and its flag");
+// The end of a list of points in bucket order that a wave's lanes have divided evenly (lane t the t-th share).  x: the sum of the last part of
+// the lane's share, which belongs to bucket b; begun: the bucket begins in this share (or the share is empty); whole: it ends with this
+// share; lacks: bucket `split`, the first part's, went out already without the shares before this one.  A segmented inclusive scan, as
+// long as a bucket spans further lanes, then the sums to `out` (added to what is there unless fresh).  All lanes call it; pool: 43 x 64 words.
+__device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, J29 x, bool begun, bool whole, uint32_t b, bool lacks, uint32_t split, J29* __restrict__ out, bool fresh, uint32_t t) {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
+    for (uint32_t sd = 1; sd < (uint32_t)MSL && !__all(begun); sd <<= 1) {
+        __syncthreads();
+#pragma unroll
+        for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
+        __syncthreads();
+        const bool before = __shfl_up(begun ? 1 : 0, sd) != 0;
+        if (t >= sd && !begun) {
+            J29 y;
+            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - sd];
+            x = j29_add(x, y);
+            begun = before;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
+    __syncthreads();
+    if (whole) {
+        if (!fresh) x = j29_add(out[b], x);
+        out[b] = x;
+    }
+    if (lacks) {
+        J29 y;
+        uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+        for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - 1];
+        out[split] = j29_add(out[split], y);
+    }
+}
+
 // One segment's share of sum over elements of digit_w(s) * base: the segment's MT raw buckets,
 // partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold / k_msm_point reduce them).
 // One wave per workgroup.  Per chunk of `chunk` elements (at most MSEG):
@@ -750,32 +788,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 x29_add_mixed(acc29, pt);
             }
             const bool whole = p1 > p0 && p1 == b_end;       // the bucket ends with this share
-            // inclusive scan of the shares' last parts, begun anew where a bucket begins; the last step moves the sums up by a lane
-            J29 x = j29_from_x29(acc29);
-            uint32_t begun = start ? 1u : 0u;
-            for (uint32_t sd = 1; sd <= (uint32_t)MSL; sd <<= 1) {
-                const bool last = sd == (uint32_t)MSL;
-                const uint32_t from = last ? 1u : sd;
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
-                __syncthreads();
-#pragma unroll
-                for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
-                __syncthreads();
-                const uint32_t before = __shfl_up(begun, from);
-                if (last && whole) {
-                    if (!first) x = j29_add(out[b], x);
-                    out[b] = x;
-                }
-                if (last ? lacks : (t >= from && !begun)) {
-                    J29 y;
-                    uint32_t* py = reinterpret_cast<uint32_t*>(&y);
-#pragma unroll
-                    for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - from];
-                    if (last) out[split] = j29_add(out[split], y);
-                    else x = j29_add(x, y);
-                }
-                if (!last && t >= from) begun |= before;
-            }
+            bucket_shares_merge(pool, j29_from_x29(acc29), start, whole, b, lacks, split, out, first, t);
         }
         __threadfence_block();
         __syncthreads();
@@ -786,6 +799,79 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
         out[t + MSL] = j29_infinity();
     }
 }
+// The same for sums of few elements: the 8-bit digits taken as two signed 4-bit digits each, so that a sum has 512 buckets (64 windows
+// of 8) instead of 4096 and the walk over its buckets, which is most of such a sum's work, fits two waves instead of sixteen.  A wave
+// takes nw windows, sorts their elements by bucket in LDS and divides that list evenly over its lanes, whatever the digits are.
+// nw (1, 2, 4 or 8) gives a lane about eight elements, so that the scan behind them costs less than they do.
+// FEW_MAX: an element costs 64 additions here and 32 there, a sum 32 walks here and 256 there; at 512 elements an opening alone takes the
+// same time both ways (1.87 ms), and of a layer of small products, whose 250 sums then leave the chip to the rest, 7.2 ms instead of 7.7.
+static constexpr int FEW_MAX = 512, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T, FEW_GROUP = MT / (4 * FEW_T);     // FEW_GROUP: the sums that k_msm_point takes in a workgroup
+// grid (64 / nw, sums); buckets[(sum * 64 + window) * 8 + magnitude - 1]
+__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_few(J29* __restrict__ buckets, const MsmDesc* __restrict__ descs, uint32_t nw) {
+    __shared__ uint32_t cnt[MSL], off[MSL], cursor[MSL];
+    __shared__ uint32_t pool[J29_WORDS * MSL];      // the sorted list (u16), then the points of the shares' scan
+    static_assert(FEW_MAX <= 4096 && FEW_MAX * 2 <= J29_WORDS * MSL * 4 && 8 * FEW_T == MSL, "list entries, the pool and a lane for each bucket");
+    uint16_t* list = reinterpret_cast<uint16_t*>(pool);
+    const MsmDesc d = descs[blockIdx.y];
+    const A29* __restrict__ A = d.base;
+    const uint32_t t = threadIdx.x, v0 = blockIdx.x * nw, half = v0 / (FEW_WINDOWS / 2);
+    const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
+    J29* __restrict__ out = buckets + ((size_t)blockIdx.y * FEW_WINDOWS + v0) * FEW_T;
+    cnt[t] = 0;
+    if (t < nw * FEW_T) out[t] = j29_infinity();
+    __syncthreads();
+    auto digit = [&](uint32_t v, size_t si) {
+        const int dg = d.digits[(size_t)(v >> 1) * d.dstride + si], hi = (dg + 8) >> 4;
+        return (v & 1u) ? hi : dg - 16 * hi;
+    };
+    for (uint32_t j = 0; j < nw; ++j)
+        for (uint32_t e = t; e < d.count; e += MSL) {
+            const int g = digit(v0 + j, (size_t)e * d.s_mul + d.s_off);
+            if (g != 0) atomicAdd(&cnt[j * FEW_T + (g < 0 ? -g : g) - 1], 1u);
+        }
+    __syncthreads();
+    uint32_t run = cnt[t];
+    for (int sd = 1; sd < MSL; sd <<= 1) {
+        const uint32_t a = __shfl_up(run, sd);
+        if (t >= (uint32_t)sd) run += a;
+    }
+    off[t] = cursor[t] = run - cnt[t];
+    const uint32_t total = __shfl(run, MSL - 1);
+    __syncthreads();
+    for (uint32_t j = 0; j < nw; ++j)
+        for (uint32_t e = t; e < d.count; e += MSL) {
+            const size_t si = (size_t)e * d.s_mul + d.s_off;
+            const int g = digit(v0 + j, si);
+            if (g == 0) continue;
+            const uint32_t pos = atomicAdd(&cursor[j * FEW_T + (g < 0 ? -g : g) - 1], 1u);
+            list[pos] = (uint16_t)(e | (((g < 0) != (((Df[si] >> half) & 1) != 0)) ? 0x8000u : 0u));
+        }
+    __threadfence_block();
+    __syncthreads();
+    if (total == 0) return;                                 // the same for every lane
+    const uint32_t share = (total + MSL - 1) / MSL, p0 = min(t * share, total), p1 = min(p0 + share, total);
+    uint32_t b = 0;                                         // the last bucket that begins at p0 or before: it holds entry p0, if there is one
+    for (uint32_t sd = MSL / 2; sd > 0; sd >>= 1)
+        if (off[b + sd] <= p0) b += sd;
+    uint32_t b_end = off[b] + cnt[b], split = 0;
+    bool start = p0 >= total || p0 == off[b], lacks = false;
+    X29 acc29 = x29_infinity();
+    for (uint32_t pos = p0; pos < p1; ++pos) {
+        if (pos == b_end) {
+            out[b] = j29_from_x29(acc29);
+            if (!start) { split = b; lacks = true; start = true; }
+            acc29 = x29_infinity();
+            do ++b; while (cnt[b] == 0);
+            b_end = off[b] + cnt[b];
+        }
+        const uint32_t en = list[pos];
+        A29 pt = A[(size_t)(en & 0x7FFFu) * d.b_mul + d.b_off];
+        if (a29_is_inf(pt)) continue;
+        if (en & 0x8000u) pt.y = fq29_neg(pt.y);
+        x29_add_mixed(acc29, pt);
+    }
+    bucket_shares_merge(pool, j29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
+}
 // raw buckets of up to 8 consecutive segments summed: out[(row * gridDim.y + group) * MT + t], row = sum * MW + w
 __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, const J29* __restrict__ buckets, uint32_t nseg) {
     const uint32_t t = threadIdx.x, row = blockIdx.x, grp = blockIdx.y;
@@ -795,15 +881,17 @@ __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, c
     for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = j29_add(acc, b[(size_t)sg * MT + t]);
     out[((size_t)row * gridDim.y + grp) * MT + t] = acc;
 }
-// The sums of a list from the raw buckets of all their windows, a workgroup for each half of a sum's windows: four lanes take bucket
-// b + 1, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings, the segments of a window added on the way), weight it by its digit, and
-// the buckets are summed -- one weighting and one lane sum per half instead of one per window, and no Horner pass of a single lane
-// over window sums afterwards.  k_msm_join adds the halves, the endomorphism on the second.
-// Raw buckets: buckets[(w nseg + seg) MT + b]; a half's total goes to its first bucket's place, which only its own workgroup reads.
+// The sums of a list from the raw buckets of all their windows, 128 walks for each half of a sum's windows: four lanes take bucket
+// b + 1, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings), weight it by its digit, and the buckets are summed -- one weighting and
+// one lane sum per half instead of one per window, and no Horner pass of a single lane over window sums afterwards.  A sum of few
+// elements has two sets of 8 buckets a window, weighted 1 .. 8 and 16 .. 128: 16 walks a half.  k_msm_join adds the halves, the
+// endomorphism on the second.
+// Raw buckets: buckets[w MT + b] (k_msm_few's: [w 16 + b]); a half's total goes to its first bucket's place, which only its own walks read.
 // The walk is one chain, so a launch takes what one chain takes whatever the number of sums: all of a job's sums that nothing waits for
-// go into one launch.  A lane's chain takes 1.5 ms; four lanes that share a point's products take 1.25 ms, and a compute unit holds one
-// such workgroup: LANES is four while all of a launch's fit beside each other, one for longer lists (310 workgroups of four took 2.6 ms).
-struct PointDesc { J29* buckets; G1Jac* out; uint32_t nseg, pad; };
+// go into one launch, those of few elements behind the others (first_few), four to a workgroup.  A lane's chain takes 1.5 ms; four lanes
+// that share a point's products take 1.25 ms, and a compute unit holds one such workgroup: LANES is four while all of a launch's fit
+// beside each other, one for longer lists (310 workgroups of four took 2.6 ms).
+struct PointDesc { J29* buckets; G1Jac* out; uint32_t half_off, few; };     // half_off: where the second half's buckets begin
 template <int LANES> __device__ __forceinline__ void walk_double(J29& p, uint32_t q) {
     if constexpr (LANES == 4) j29_quad_double(p, q);
     else j29_double_walk(p);
@@ -812,51 +900,57 @@ template <int LANES> __device__ __forceinline__ void walk_add(J29& a, const J29&
     if constexpr (LANES == 4) j29_quad_add(a, b, q);
     else a = j29_add(a, b);
 }
-template <int LANES> __global__ void __launch_bounds__(LANES * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list) {
+template <int LANES> __global__ void __launch_bounds__(LANES * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list, uint32_t first_few, uint32_t n) {
     __shared__ uint32_t pool[J29_WORDS * MT / 2];
-    const uint32_t q = threadIdx.x % LANES, b = threadIdx.x / LANES, half = blockIdx.y;
-    const PointDesc d = list[blockIdx.x];
-    J29* const mine = d.buckets + (size_t)half * MWH * d.nseg * MT;
+    const uint32_t q = threadIdx.x % LANES, walk = threadIdx.x / LANES;
+    const bool few = blockIdx.x >= 2 * first_few;           // the same for the workgroup
+    const uint32_t width = few ? 2 * FEW_T : MT, group = walk / width, b = walk % width;
+    const uint32_t sum = few ? first_few + (blockIdx.x - 2 * first_few) * FEW_GROUP + group / 2 : blockIdx.x >> 1;
+    const uint32_t half = few ? group & 1u : blockIdx.x & 1u;
+    const uint32_t weight = few && b >= FEW_T ? (b - FEW_T + 1) * 16 : b + 1;
+    const bool live = sum < n;
+    J29* mine = nullptr;
+    if (live) { const PointDesc d = list[sum]; mine = d.buckets + half * d.half_off; }
     J29 r = j29_infinity();
-    for (int w = MWH - 1; w >= 0; --w) {
+    for (uint32_t w = MWH; w-- > 0;) {
+        J29 p = j29_infinity();
+        if (LANES == 4 && live) p = mine[w * width + b];    // on its way during the doublings (a single lane has no registers left for it)
         if (__any(!r.inf))
             for (int k = 0; k < 8; ++k) walk_double<LANES>(r, q);
-        const J29* row = mine + (size_t)w * d.nseg * MT;
-        for (uint32_t sg = 0; sg < d.nseg; ++sg) {
-            const J29 p = row[(size_t)sg * MT + b];
-            if (__any(!p.inf)) walk_add<LANES>(r, p, q);
-        }
+        if (LANES == 1 && live) p = mine[w * width + b];
+        if (__any(!p.inf)) walk_add<LANES>(r, p, q);
     }
-    J29 s = j29_infinity();
-    for (int bit = 7; bit >= 0; --bit) {
+    J29 s = r;
+    if (!(weight & 128u)) s.inf = 1u;
+    for (int bit = 6; bit >= 0; --bit) {
         walk_double<LANES>(s, q);
         J29 p = r;
-        if (!(((b + 1) >> bit) & 1u)) p.inf = 1u;
+        if (!((weight >> bit) & 1u)) p.inf = 1u;
         walk_add<LANES>(s, p, q);
     }
-    for (uint32_t sd = MT / 2; sd > 0; sd >>= 1) {
+    for (uint32_t sd = width / 2; sd > 0; sd >>= 1) {
         __syncthreads();
         if (b >= sd && b < 2 * sd && q == 0) {
             const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
 #pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) pool[l * (MT / 2) + b - sd] = src[l];
+            for (int l = 0; l < J29_WORDS; ++l) pool[l * (MT / 2) + group * sd + b - sd] = src[l];
         }
         __syncthreads();
         if (b < sd) {
             J29 y;
             uint32_t* py = reinterpret_cast<uint32_t*>(&y);
 #pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (MT / 2) + b];
+            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (MT / 2) + group * sd + b];
             walk_add<LANES>(s, y, q);
         }
     }
-    if (threadIdx.x == 0) *mine = s;
+    if (live && b == 0 && q == 0) *mine = s;
 }
 __global__ void __launch_bounds__(GT) k_msm_join(const PointDesc* __restrict__ list, uint32_t n) {
     const uint32_t i = (blockIdx.x * GT + threadIdx.x) >> 2, q = threadIdx.x & 3u;
     if (i >= n) return;
     const PointDesc d = list[i];
-    J29 s = d.buckets[0], y = d.buckets[(size_t)MWH * d.nseg * MT];
+    J29 s = d.buckets[0], y = d.buckets[d.half_off];
     y.x = fq29_mul(y.x, fq29_from_fp(glv_beta()));
     j29_quad_add(s, y, q);
     if (q == 0) *d.out = j29_to_jac(s);
@@ -1678,6 +1772,19 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
                              std::vector<PointDesc>& later) {
     const uint32_t n_msm = (uint32_t)d.size();
     if (n_msm == 0) return 0;
+    if (count_max <= (size_t)FEW_MAX) {
+        uint32_t nw = 8;
+        while (nw > 1 && nw * count_max > 8 * MSL) nw /= 2;
+        const void* dd = nullptr;
+        int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
+        if (rc) return rc;
+        Scratch& buckets = arena.add(sizeof(J29) * (size_t)n_msm * FEW_BUCKETS);
+        if (buckets.rc) return buckets.rc;
+        hipLaunchKernelGGL(k_msm_few, dim3(FEW_WINDOWS / nw, n_msm), dim3(MSL), 0, st, buckets.as<J29>(), (const MsmDesc*)dd, nw);
+        ZK_LAUNCH_CHECK();
+        for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<J29>() + (size_t)z * FEW_BUCKETS, out[z], FEW_BUCKETS / 2, 1u});
+        return 0;
+    }
     // One chunk per workgroup, and chunks short enough for two workgroups a SIMD where there are few elements: a workgroup's time is its
     // chunk's elements over 64 lanes.  Very large inputs take more chunks per workgroup to bound the bucket storage.
     uint32_t chunk = MSEG;
@@ -1703,17 +1810,20 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
         ns = ng;
     }
     ZK_LAUNCH_CHECK();
-    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], 1u, 0u});
+    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], MWH * MT, 0u});
     return 0;
 }
 static int points_queue(std::vector<PointDesc>& list, JobUploads& up, hipStream_t st) {
     if (list.empty()) return 0;
+    const uint32_t n = (uint32_t)list.size();
+    const uint32_t first_few = (uint32_t)(std::stable_partition(list.begin(), list.end(), [](const PointDesc& d) { return d.few == 0; }) - list.begin());
     const void* dl = nullptr;
-    int rc = up.put(list.data(), sizeof(PointDesc) * list.size(), st, &dl);
+    int rc = up.put(list.data(), sizeof(PointDesc) * n, st, &dl);
     if (rc) return rc;
-    if (list.size() <= 96) hipLaunchKernelGGL(k_msm_point<4>, dim3((unsigned)list.size(), 2), dim3(4 * MT), 0, st, (const PointDesc*)dl);
-    else hipLaunchKernelGGL(k_msm_point<1>, dim3((unsigned)list.size(), 2), dim3(MT), 0, st, (const PointDesc*)dl);
-    hipLaunchKernelGGL(k_msm_join, dim3(cdiv(4 * list.size(), (size_t)GT)), dim3(GT), 0, st, (const PointDesc*)dl, (uint32_t)list.size());
+    const unsigned groups = 2 * first_few + cdiv(n - first_few, FEW_GROUP);
+    if (groups <= 192) hipLaunchKernelGGL(k_msm_point<4>, dim3(groups), dim3(4 * MT), 0, st, (const PointDesc*)dl, first_few, n);
+    else hipLaunchKernelGGL(k_msm_point<1>, dim3(groups), dim3(MT), 0, st, (const PointDesc*)dl, first_few, n);
+    hipLaunchKernelGGL(k_msm_join, dim3(cdiv(4 * (size_t)n, (size_t)GT)), dim3(GT), 0, st, (const PointDesc*)dl, n);
     ZK_LAUNCH_CHECK();
     list.clear();
     return 0;
