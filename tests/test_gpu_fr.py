@@ -826,6 +826,49 @@ def _hip_streams(n):
     return rt, out
 
 
+def test_copies_and_clears_take_any_memory_and_refuse_null(hip):
+    """zk_memcpy_d2h / _d2d, zk_memset(0) and zk_upload run as kernels inside the allocator's own blocks only: another allocator's device
+    memory gives the same values through the runtime, a null pointer is an error of the call, and the calls behind it work."""
+    with open("/proc/self/maps") as f:                           # the runtime that the library runs on
+        runtime = ctypes.CDLL(next(x.split()[-1] for x in f if "libamdhip64" in x))
+    P = lambda p: ctypes.c_void_p(p)
+    n = 1000
+    data = np.random.default_rng(3).integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    own = hip.upload(data)
+    theirs = ctypes.c_void_p()
+    assert runtime.hipMalloc(ctypes.byref(theirs), ctypes.c_size_t(4 * (n + 3))) == 0
+    out = np.zeros(n, np.uint32)
+    size = ctypes.c_size_t
+    refused = [("zk_memcpy_d2h", lambda b: (out, None, size(b), None)), ("zk_memcpy_d2h", lambda b: (None, P(own), size(b), None)),
+               ("zk_memcpy_d2d", lambda b: (None, P(own), size(b), None)), ("zk_memcpy_d2d", lambda b: (P(own), None, size(b), None)),
+               ("zk_memset", lambda b: (None, ctypes.c_int(0), size(b), None)), ("zk_upload", lambda b: (None, data, size(b), None)),
+               ("zk_upload", lambda b: (P(own), None, size(b), None))]
+    for bytes_ in (64, 61):                                      # a kernel's sizes and the runtime's
+        for name, args in refused:
+            with pytest.raises(RuntimeError):
+                hip.call(name, *args(bytes_))
+            assert (hip.download(own, n, np.uint32) == data).all(), name
+    # offsets inside a block, aligned to a word, to 16 bytes and not at all
+    for off, count in ((0, n), (1, n - 1), (4, 64), (7, 1), (n - 1, 1)):
+        assert (hip.download(own + 4 * off, count, np.uint32) == data[off:off + count]).all()
+    assert (hip.download(own + 2, 4 * (n - 1), np.uint8) == data.view(np.uint8)[2:4 * (n - 1) + 2]).all()
+    # memory of another allocator, both ways
+    for off in (0, 3):
+        t = theirs.value + 4 * off
+        hip.call("zk_memcpy_d2d", P(t), P(own), size(4 * n), None)
+        assert (hip.download(t, n, np.uint32) == data).all()
+        back = hip.malloc(4 * n)
+        hip.call("zk_memcpy_d2d", P(back), P(t), size(4 * n), None)
+        assert (hip.download(back, n, np.uint32) == data).all()
+        hip.call("zk_memset", P(t), ctypes.c_int(0), size(4 * 500), None)
+        assert not hip.download(t, 500, np.uint32).any() and (hip.download(t + 2000, n - 500, np.uint32) == data[500:]).all()
+        hip.call("zk_upload", P(t), data[:100].copy(), size(400), None)
+        assert (hip.download(t, 100, np.uint32) == data[:100]).all()
+        hip.free(back)
+    hip.free(own)
+    assert runtime.hipFree(theirs) == 0
+
+
 def test_scratch_blocks_reused_on_another_stream_wait_for_their_last_user(hip):
     """Two matrix products of one shape on two streams back to back: the second call gets the scratch blocks that the first
     call has just given back while its kernels are still queued, and must not overwrite them early."""

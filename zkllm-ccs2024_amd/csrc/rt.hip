@@ -7,7 +7,6 @@
 #include <map>
 #include <mutex>
 #include <thread>
-#include <unordered_map>
 #include <utility>
 #include <vector>
 #include <cstdio>
@@ -26,14 +25,15 @@ int hip_fail(hipError_t e, const char* what, const char* file, int line) {
     char buf[512];
     snprintf(buf, sizeof(buf), "%s failed: %s (%s:%d)", what, hipGetErrorString(e), file, line);
     set_error((int)e, buf);
+    (void)hipGetLastError();          // reported: the check behind the next launch must not find it again
     return (int)e;
 }
 
-struct Block { size_t size; hipStream_t last; bool idle; uint64_t freed_tick; hipEvent_t ev; bool ev_set; };
+struct Block { size_t size; hipStream_t last; bool idle; uint64_t freed_tick; hipEvent_t ev; bool ev_set; int device; };
 struct Pool {
     std::mutex mu;
     std::map<size_t, std::vector<void*>> free_lists;
-    std::unordered_map<void*, Block> live;      // every block we own -> rounded size and last user
+    std::map<void*, Block> live;                // every block we own -> rounded size and last user; ordered: an address inside one is found too
     size_t cached_bytes = 0, live_bytes = 0;
     hipEvent_t events[32] = {};
     unsigned next_event = 0;
@@ -136,8 +136,10 @@ int pool_alloc(void** out, size_t bytes, hipStream_t stream, const hipStream_t* 
         e = hipMalloc(&p, sz);
         if (e != hipSuccess) return hip_fail(e, "hipMalloc", __FILE__, __LINE__);
     }
+    int device = -1;
+    if (hipGetDevice(&device) != hipSuccess) (void)hipGetLastError();
     std::lock_guard<std::mutex> lk(P.mu);
-    P.live[p] = Block{sz, stream, true, 0, nullptr, false};
+    P.live[p] = Block{sz, stream, true, 0, nullptr, false, device};
     P.live_bytes += sz;
     *out = p;
     return 0;
@@ -372,6 +374,29 @@ static __global__ void __launch_bounds__(256) k_copy_quads(uint4* __restrict__ d
 static __global__ void __launch_bounds__(256) k_clear_words(uint32_t* __restrict__ dst, size_t n) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) dst[i] = 0u;
 }
+// Whether a kernel on `st` may take [p, p + bytes) in place of a copy or fill of the runtime's: a part of one of the allocator's blocks, on
+// the device that the stream and the caller are on.  Anything else -- null, host memory, another device's, another allocator's -- is the
+// runtime's to handle or to refuse; a kernel that touched it could fault.
+static bool in_own_block(const void* p, size_t bytes, hipStream_t st) {
+    int device = -1, stream_device = -1;
+    if (hipGetDevice(&device) != hipSuccess) { (void)hipGetLastError(); return false; }
+    if (st == nullptr) stream_device = device;
+    else if (hipStreamGetDevice(st, &stream_device) != hipSuccess) { (void)hipGetLastError(); return false; }
+    Pool& P = pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    auto it = P.live.upper_bound(const_cast<void*>(p));
+    if (it == P.live.begin()) return false;
+    --it;
+    const size_t at = (size_t)((const char*)p - (const char*)it->first);
+    return at <= it->second.size && bytes <= it->second.size - at && it->second.device == device && stream_device == device;
+}
+// Whether the host itself may read or write p: memory that the runtime does not know, or pinned
+static bool host_memory(const void* p) {
+    if (p == nullptr) return false;
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) { (void)hipGetLastError(); return true; }
+    return a.type == hipMemoryTypeUnregistered || a.type == hipMemoryTypeHost;
+}
 int clear_words(void* dst, size_t words, hipStream_t st) {
     hipLaunchKernelGGL(k_clear_words, dim3((unsigned)std::min<size_t>(cdiv(words, 256), 4096)), dim3(256), 0, st, (uint32_t*)dst, words);
     ZK_LAUNCH_CHECK();
@@ -506,7 +531,8 @@ int zk_memcpy_h2d(void* dst, const void* src, size_t bytes, void* stream) {
 }
 // For data that only work queued on `stream` reads: small arrays of words travel as a kernel's arguments, nothing is staged or waited for
 int zk_upload(void* dst, const void* src, size_t bytes, void* stream) {
-    if (bytes == 0 || bytes > sizeof(SmallWords) || bytes % 4 != 0 || (uintptr_t)dst % 4 != 0) return zk_memcpy_h2d(dst, src, bytes, stream);
+    if (bytes == 0 || bytes > sizeof(SmallWords) || bytes % 4 != 0 || (uintptr_t)dst % 4 != 0 || !host_memory(src) || !in_own_block(dst, bytes, (hipStream_t)stream))
+        return zk_memcpy_h2d(dst, src, bytes, stream);
     SmallWords w;
     memcpy(w.v, src, bytes);
     hipLaunchKernelGGL(k_small_words, dim3(1), dim3(256), 0, (hipStream_t)stream, (uint32_t*)dst, w, (uint32_t)(bytes / 4));
@@ -516,7 +542,7 @@ int zk_upload(void* dst, const void* src, size_t bytes, void* stream) {
 // up to 64 KiB: a kernel writes them to the thread's pinned buffer
 int zk_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
     if (!bytes) return 0;
-    if (bytes <= ((size_t)64 << 10) && bytes % 4 == 0 && (uintptr_t)src % 4 == 0) {
+    if (bytes <= ((size_t)64 << 10) && bytes % 4 == 0 && (uintptr_t)src % 4 == 0 && host_memory(dst) && in_own_block(src, bytes, (hipStream_t)stream)) {
         void* stage = nullptr;
         const int rc = staging(&stage, bytes);
         if (rc) return rc;
@@ -532,7 +558,7 @@ int zk_memcpy_d2h(void* dst, const void* src, size_t bytes, void* stream) {
 }
 int zk_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream) {
     if (!bytes) return 0;
-    if (((uintptr_t)dst | (uintptr_t)src | bytes) % 16 == 0) {
+    if (((uintptr_t)dst | (uintptr_t)src | bytes) % 16 == 0 && in_own_block(dst, bytes, (hipStream_t)stream) && in_own_block(src, bytes, (hipStream_t)stream)) {
         hipLaunchKernelGGL(k_copy_quads, dim3((unsigned)std::min<size_t>(cdiv(bytes / 16, 256), 8192)), dim3(256), 0, (hipStream_t)stream, (uint4*)dst, (const uint4*)src, bytes / 16);
         ZK_LAUNCH_CHECK();
         return 0;
@@ -542,7 +568,7 @@ int zk_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream) {
 }
 int zk_memset(void* dst, int value, size_t bytes, void* stream) {
     if (!bytes) return 0;
-    if (value == 0 && bytes % 4 == 0 && (uintptr_t)dst % 4 == 0) return clear_words(dst, bytes / 4, (hipStream_t)stream);
+    if (value == 0 && bytes % 4 == 0 && (uintptr_t)dst % 4 == 0 && in_own_block(dst, bytes, (hipStream_t)stream)) return clear_words(dst, bytes / 4, (hipStream_t)stream);
     ZK_HIP(hipMemsetAsync(dst, value, bytes, (hipStream_t)stream));
     return 0;
 }
