@@ -1,5 +1,7 @@
 """GPU parity: multiplicities, batch inversion, the two-phase lookup sumcheck, range / mapping tables,
 rescaling, multi-Hadamard sumcheck, stacked inner-product sumcheck and zkSoftmax -- bit-exact against the oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 from ctypes import c_uint64 as c_u64
@@ -18,6 +20,30 @@ def pv():
 @pytest.fixture(scope="module")
 def orc():
     return load_oracle()
+
+
+def test_tensors_are_on_the_device_when_their_constructor_or_the_mapping_returns(pv):
+    """The constructors from host arrays and tLookupRangeMapping::operator() leave nothing queued on the default stream that a caller's own
+    non-blocking stream would have to wait for: not the conversion, also behind a long product, and not the gather."""
+    with open("/proc/self/maps") as f:                           # the runtime that the library runs on
+        runtime = ctypes.CDLL(next(x.split()[-1] for x in f if "libamdhip64" in x))
+    idle = lambda: runtime.hipStreamQuery(None) == 0
+    rng = np.random.default_rng(2)
+    a = pv.from_fr(mt_random_vec(np.random.RandomState(1), 512 * 512))
+    for n in (1, 24, 96, 97, 700, 50000):                        # through a kernel's arguments and through a staged copy
+        ints = rng.integers(-1000, 1000, n)
+        for make in (lambda: pv.from_fr(fr_array([int(x) % R_MOD for x in ints])), lambda: pv.from_i32(ints), lambda: pv.from_i64(ints),
+                     lambda: pv.from_f32(ints.astype(np.float32), 1), lambda: pv.from_f64(ints.astype(np.float64), 1)):
+            product = pv.matmul(a, a, 512, 512, 512)             # milliseconds on the default stream
+            t = make()
+            assert idle(), n
+            assert (t.host() == fr_array([int(x) % R_MOD for x in ints])).all()
+            del product
+    q = pv.from_i32(rng.integers(0, 256, 1 << 22))
+    y, m, _ = pv.mapping(q, 0, 256, pv.from_i32(np.arange(256) * 7))
+    assert idle()
+    del y, m
+
 
 
 def ch(seed, n):

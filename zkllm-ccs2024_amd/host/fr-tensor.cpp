@@ -215,28 +215,34 @@ static Fr_t* fr_alloc(size_t n) {
 }
 
 FrTensor::FrTensor(uint size) : gpu_data(fr_alloc(size)), size(size) {}
+// The constructors from host arrays return when the data is on the device: a caller may read gpu_data on any stream
 FrTensor::FrTensor(uint size, const Fr_t* cpu_data) : gpu_data(fr_alloc(size)), size(size) {
     ZKC(zk_upload(gpu_data, cpu_data, sizeof(Fr_t) * size, nullptr));
+    ZKC(zk_sync(nullptr));
 }
 FrTensor::FrTensor(uint size, const int* cpu_data) : gpu_data(fr_alloc(size)), size(size) {
     DevBuf tmp(sizeof(int) * (size_t)size);
     ZKC(zk_upload(tmp.p, cpu_data, sizeof(int) * (size_t)size, nullptr));
     ZKC(zk_fr_from_i32(gpu_data, tmp.p, size, nullptr));
+    ZKC(zk_sync(nullptr));
 }
 FrTensor::FrTensor(uint size, const long* cpu_data) : gpu_data(fr_alloc(size)), size(size) {
     DevBuf tmp(sizeof(long) * (size_t)size);
     ZKC(zk_upload(tmp.p, cpu_data, sizeof(long) * (size_t)size, nullptr));
     ZKC(zk_fr_from_i64(gpu_data, tmp.p, size, nullptr));
+    ZKC(zk_sync(nullptr));
 }
 FrTensor::FrTensor(uint size, const float* cpu_data, unsigned long sf) : gpu_data(fr_alloc(size)), size(size) {
     DevBuf tmp(sizeof(float) * (size_t)size);
     ZKC(zk_upload(tmp.p, cpu_data, sizeof(float) * (size_t)size, nullptr));
     ZKC(zk_fr_from_f32(gpu_data, tmp.p, sf, size, nullptr));
+    ZKC(zk_sync(nullptr));
 }
 FrTensor::FrTensor(uint size, const double* cpu_data, unsigned long sf) : gpu_data(fr_alloc(size)), size(size) {
     DevBuf tmp(sizeof(double) * (size_t)size);
     ZKC(zk_upload(tmp.p, cpu_data, sizeof(double) * (size_t)size, nullptr));
     ZKC(zk_fr_from_f64(gpu_data, tmp.p, sf, size, nullptr));
+    ZKC(zk_sync(nullptr));
 }
 FrTensor::FrTensor(const FrTensor& t) : gpu_data(fr_alloc(t.size)), size(t.size) {
     ZKC(zk_memcpy_d2d(gpu_data, t.gpu_data, sizeof(Fr_t) * (size_t)size, nullptr));

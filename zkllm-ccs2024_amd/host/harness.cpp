@@ -396,7 +396,8 @@ int zkp_range_prove(void* S, int low, u32 len, const u32* alpha, const u32* beta
 int zkp_mapping(void* S_in, int low, u32 len, void* mvals, const u32* r, const u32* alpha, const u32* beta, const u32* u, const u32* v, void** y_out, void** m_out, u32* final_claim) {
     ZKP_TRY
     tLookupRangeMapping t(low, len, FT(mvals));
-    auto p = t(FT(S_in));
+    // a proof of more than one query ends behind the outputs that it was begun on
+    auto p = final_claim && FT(S_in).size > 1 ? t.map_queued(FT(S_in)) : t(FT(S_in));
     if (final_claim) {
         const int k = (int)ceilLog2(FT(S_in).size);
         std::vector<Polynomial> proof;

@@ -461,7 +461,7 @@ const FrTensor& FfnBlock::forward() {
     up_out_.emplace(up_rescale.rescale(*up_out, true));            // int32 forms: the activation lookup and the product below read them
     gate_out.emplace(gate_layer(input));
     gate_out_.emplace(gate_rescale.rescale(*gate_out, true));
-    auto p = swiglu(*gate_out_);
+    auto p = swiglu.map_queued(*gate_out_);
     swiglu_out.emplace(std::move(p.first));
     swiglu_m.emplace(std::move(p.second));
     down_in.emplace(*swiglu_out * *up_out_);

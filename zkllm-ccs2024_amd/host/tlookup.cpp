@@ -64,10 +64,16 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const int* vals, const 
     ZKC(zk_lookup_multiplicities(m.gpu_data, idx.p, nullptr, vals, nullptr, low, len, D, table.size, 0, nullptr));
     FrTensor y(D);
     ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, idx.p, D, nullptr));
+    ZKC(zk_sync(nullptr));
     return {std::move(y), std::move(m)};
 }
 pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const FrTensor& vals) { return map(vals, nullptr); }
 pair<FrTensor, FrTensor> tLookupRangeMapping::map(const FrTensor& vals, const FrTensor* unwritten) {
+    auto p = map_queued(vals, unwritten);
+    ZKC(zk_sync(nullptr));
+    return p;
+}
+pair<FrTensor, FrTensor> tLookupRangeMapping::map_queued(const FrTensor& vals, const FrTensor* unwritten) {
     // queries and mapped values in int32 form: nothing below needs the array of table positions
     const bool by_queries = mapped_vals.kept_ints() && vals.kept_ints();
     DevBuf idx(by_queries ? 4 : sizeof(uint) * (size_t)vals.size);

@@ -71,6 +71,8 @@ class tLookupRangeMapping : public tLookupRange {
     // it) with an int32 form of its own.  For a caller whose every reader of the outputs takes the int32 form (the proof of a
     // large lookup does: zk_lookup_ints_suffice; evaluations do; products of two such tensors do).
     pair<FrTensor, FrTensor> map(const FrTensor& vals, const FrTensor* unwritten);
+    // map() without its wait: the outputs may still be on their way.  For a caller that goes on on the default stream.
+    pair<FrTensor, FrTensor> map_queued(const FrTensor& vals, const FrTensor* unwritten = nullptr);
 
     Fr_t prove(const FrTensor& S_in, const FrTensor& S_out, const FrTensor& m, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u,
                const vector<Fr_t>& v, vector<Polynomial>& proof);

@@ -92,7 +92,7 @@ FrTensor zkSoftmax::compute_rows(uint m, const FrTensor& X, FrTensor& shift, FrT
     for (uint i = 0; i < K; ++i) lean_tensors_last += ints_only[i] ? 1 : 0;
     for (uint i = 0; i < L; ++i) m_segments.push_back(least_significant_segments[i].prep(X_segments[i]));
     for (uint i = L; i < K; ++i) {
-        auto p = other_segments[i - L].map(X_segments[i], lean_out ? unwritten.get() : nullptr);
+        auto p = other_segments[i - L].map_queued(X_segments[i], lean_out ? unwritten.get() : nullptr);
         Y_segments.push_back(std::move(p.first));
         m_segments.push_back(std::move(p.second));
     }
