@@ -30,3 +30,13 @@ def test_every_reference_header_name_has_a_forwarding_header(tmp_path):
     inc = os.path.join(ROOT, "zkllm-ccs2024_amd", "host", "compat")
     r = subprocess.run(["g++", "-std=c++17", "-x", "c++", "-fsyntax-only", "-w", "-I" + inc, "-"], input=src, text=True, capture_output=True, cwd=tmp_path)
     assert r.returncode == 0, r.stderr[:2000]
+
+
+def test_the_host_layer_is_built_with_the_compiler_that_the_environment_names():
+    """CXX from the environment and from the command line; neither given, the toolchain's clang where it is there."""
+    where = os.path.join(ROOT, "zkllm-ccs2024_amd", "host")
+    clang = "/opt/rocm/llvm/bin/clang++"
+    env = {k: v for k, v in os.environ.items() if k not in ("CXX", "MAKEFLAGS", "MAKELEVEL")}
+    for more, args, compiler in (({"CXX": "some-c++"}, [], "some-c++"), ({}, ["CXX=other-c++"], "other-c++"), ({}, [], clang if os.path.exists(clang) else "g++")):
+        r = subprocess.run(["make", "-n", "-B", "fr-tensor.o"] + args, env={**env, **more}, text=True, capture_output=True, cwd=where)
+        assert r.returncode == 0 and r.stdout.split()[0] == compiler, (r.stdout, r.stderr)
