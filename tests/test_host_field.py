@@ -1,12 +1,14 @@
 """The product's own limb arithmetic (zkllm-ccs2024_amd/csrc/field.hpp -- one source for the GPU kernels
 and the prover's host-side scalar work), run on the CPU through the class-layer library and compared
 with python big-int closed forms and with the oracle.  No GPU needed."""
+import os
 import random
+import subprocess
 
 import numpy as np
 
 from gpuhelp import _np_ptr, pkg
-from zkhelp import FP_R, FR_R, P_MOD, R_MOD, fp_array, fp_ints, fr_array, fr_ints, load_oracle, orc_check
+from zkhelp import FP_R, FR_R, P_MOD, R_MOD, ROOT, fp_array, fp_ints, fr_array, fr_ints, load_oracle, orc_check
 
 import ctypes
 
@@ -121,3 +123,21 @@ def test_host_polynomial_eval_matches_horner():
     C, X = fr_array(coefs), fr_array([x])
     assert lib.zkp_poly_eval(_np_ptr(C), ctypes.c_int(5), _np_ptr(X), _np_ptr(out)) == 0
     assert fr_ints(out) == [sum(c * pow(x, i, R_MOD) for i, c in enumerate(coefs)) % R_MOD]
+
+
+def test_the_two_streams_of_an_opening_are_two_apart(tmp_path):
+    """stream_pair (rt.hpp) for every pool size that ZKLLM_SIDE_STREAMS allows: two streams wherever there are two, of four or more neither
+    neighbours nor four apart, and every stream of the default pools in turn."""
+    src = tmp_path / "pairs.cpp"
+    src.write_text('#include <cstdio>\n#include "rt.hpp"\nint main() { for (unsigned c = 1; c <= 24; ++c) for (unsigned j = 0; j < 48; ++j) {'
+                   ' unsigned p[2]; zk::stream_pair(j, c, p); printf("%u %u %u\\n", c, p[0], p[1]); } }\n')
+    csrc = os.path.join(ROOT, "zkllm-ccs2024_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + csrc, str(src), "-o", str(tmp_path / "pairs")], check=True)
+    pairs = [tuple(map(int, x.split())) for x in subprocess.run([str(tmp_path / "pairs")], check=True, capture_output=True, text=True).stdout.splitlines()]
+    assert len(pairs) == 24 * 48
+    for count, a, b in pairs:
+        assert a < count and b < count and (a != b or count == 1)
+        if count >= 4:
+            assert (b - a) % count == 2
+    for count in (4, 8):
+        assert {x for c, a, b in pairs if c == count for x in (a, b)} == set(range(count))

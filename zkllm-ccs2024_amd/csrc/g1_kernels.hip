@@ -2566,9 +2566,11 @@ int zk_g1_open(uint32_t* proof_host, uint32_t* final_scalar_host, const void* sc
 // must stay alive and unmodified until end, which waits for the opening, delivers its results and releases its buffers.
 static int open_begin_impl(void** handle, const OpenItem* items, int count, size_t n, int rounds, void* stv) {
     ZK_ARG(handle != nullptr, "zk_g1_open_begin: null handle");
-    // Consecutive streams of the pool: the folds on one, the bucket sums on the other.  A job whose rounds are one batch has no folds: one
-    // stream, so that the others (and their hardware queues) are left to other jobs.
-    hipStream_t side = side_stream(0), aux = n * (size_t)count <= (size_t)LAST_N && rounds <= TAIL_LEVELS ? side : side_stream(0);
+    // The folds on one stream, the bucket sums on another.  A job whose rounds are one batch has no folds: one stream, so that the others
+    // (and their hardware queues) are left to other jobs.
+    hipStream_t side = nullptr, aux = nullptr;
+    if (n * (size_t)count <= (size_t)LAST_N && rounds <= TAIL_LEVELS) aux = side = side_stream(0);
+    else opening_streams(&side, &aux);
     ZK_ARG(side != nullptr && aux != nullptr, "zk_g1_open_begin: could not create a stream");
     // what open_queue refuses is refused here, before anything is handed to the launch thread
     ZK_ARG(n >= 1, "zk_g1_open: empty input");

@@ -190,31 +190,50 @@ int pool_trim() {
     return 0;
 }
 
-hipStream_t side_stream(int pool) {
-    std::lock_guard<std::mutex> lk(g_side_mu);
-    static unsigned next[2] = {0, 0};
+// A stream of a pool, called with g_side_mu held: `job` counts calls (`pair`: which of a job's two streams, -1 for a job of one).  The streams
+// are all made at the first use of any, the openings' first, so that which of them share a hardware queue does not hang on the order of
+// the jobs (4 queues: a layer of 2048 x 2048 takes 55.1 ms when its sumchecks' streams come first, 53.9 ms behind the openings').
+static hipStream_t side_stream_locked(int pool, int pair, unsigned job) {
     static int count[2] = {0, 0}, shared = 0;
     if (!count[0]) {
-        // An opening job takes two consecutive streams of pool 0 (folds / bucket sums), four jobs in flight.  With few hardware queues (the
-        // runtime's four) the streams beyond them share one with the caller's, whose short kernels then wait for an opening's: half as
-        // many (a small layer 9.9 -> 8.7 ms, the layer of 2048 x 2048 60 -> 56 ms).
+        // Four streams for openings while there are fewer than eight hardware queues (the runtime's default is four), else eight.  Streams
+        // beyond the queues share one with the caller's, whose short kernels then wait for an opening's: with 4 queues a layer of 2048 x 2048
+        // takes 55.1 ms on four and 56.2 ms on eight, two openings of 2^16 generators in flight 12.3 and 14.9 ms.  With 8 queues, and with 16,
+        // the layer takes the same on both (55.3 and 55.6; 55.7 and 56.0 ms) and four such openings in flight 25.3 and 22.2 ms; with 5 to 7 queues
+        // neither number is better throughout (5: the layer 55.8 and 56.7 ms, two such openings 13.0 and 14.0, four 25.4 and 23.4).
         int queues = 4;
         if (const char* e = getenv("GPU_MAX_HW_QUEUES")) queues = atoi(e);
-        count[0] = queues >= 11 ? 8 : 4; count[1] = 2;
+        count[0] = queues >= 8 ? 8 : 4; count[1] = 2;
         if (const char* e = getenv("ZKLLM_SIDE_STREAMS")) {          // "openings,sumchecks[,shared]" (experiments)
             int a = 0, b2 = 0, c = 0;
             if (sscanf(e, "%d,%d,%d", &a, &b2, &c) >= 2 && a >= 1 && a <= 24 && b2 >= 1 && b2 <= 24) { count[0] = a; count[1] = b2; shared = c; }
         }
     }
     const int q = (pool && !shared) ? 1 : 0;
-    const unsigned i = next[q]++ % (unsigned)count[q];
-    hipStream_t& s = g_side_streams[q][i];
     // ZKLLM_SIDE_STREAMS_BLOCKING=1 (measurement only): streams that the default stream waits for and that wait for it; with
     // ZKLLM_SIDE_STREAMS=1,1,1 and a caller on the default stream no two kernels of the library overlap, so a kernel trace
     // shows what each costs alone
     static const bool blocking = [] { const char* e = getenv("ZKLLM_SIDE_STREAMS_BLOCKING"); return e && e[0] == '1'; }();
-    if (!s && hipStreamCreateWithFlags(&s, blocking ? hipStreamDefault : hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); s = nullptr; return nullptr; }
-    return s;
+    for (int k = 0; k < (shared ? 1 : 2); ++k)
+        for (int i = 0; i < count[k]; ++i) {
+            hipStream_t& s = g_side_streams[k][i];
+            if (!s && hipStreamCreateWithFlags(&s, blocking ? hipStreamDefault : hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); s = nullptr; }
+        }
+    unsigned both[2];
+    stream_pair(job, (unsigned)count[q], both);
+    return g_side_streams[q][pair < 0 ? job % (unsigned)count[q] : both[pair]];
+}
+hipStream_t side_stream(int pool) {
+    std::lock_guard<std::mutex> lk(g_side_mu);
+    static unsigned next[2] = {0, 0};
+    return side_stream_locked(pool, -1, next[pool ? 1 : 0]++);
+}
+void opening_streams(hipStream_t* folds, hipStream_t* sums) {
+    std::lock_guard<std::mutex> lk(g_side_mu);
+    static unsigned next = 0;
+    *folds = side_stream_locked(0, 0, next);
+    *sums = side_stream_locked(0, 1, next);
+    ++next;
 }
 
 // hooks are registered by static initialisers of the other files: the list is made on first use and never destroyed
