@@ -444,7 +444,7 @@ static constexpr int OB_MAX = 8;           // openings of equal size that share 
 static constexpr int TABLE_MIN_N = 1024;   // results of a fold below which no fold tables are made for it
 static constexpr int LAST_N = 16384;       // generators of a job (all its openings together) at which the remaining rounds are computed in one batch
 static constexpr int TAIL_LEVELS = 20;     // most rounds the batch takes
-static constexpr int SPAN_MAX_N = 1 << 17; // generators of a job up to which three rounds are taken as a batch of sums beside one fold
+static constexpr int SPAN_MAX_N = 3 << 15; // generators of a job up to which three rounds are taken as a batch of sums beside one fold
 struct GlvK { uint32_t k1[4], k2[4]; };
 
 __device__ __forceinline__ bool aff_is_inf(const G1Affine& p) { return is_zero(p.x) && is_zero(p.y); }   // normalised infinity: all-zero limbs
@@ -2471,7 +2471,8 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         bool comb = r <= 1;
         for (int i = 0; i < count; ++i) comb = comb && (r == 0 ? items[i].comb : items[i].comb2) != nullptr;
         // Three rounds as a batch of sums beside one fold where a round's fold would leave the chip half empty and take one walk's
-        // latency (2.4 ms) all the same; above that a round at a time, which sums over fewer points.
+        // latency (2.4 ms) all the same; above that a round at a time, which sums over fewer points.  Openings of 16 rows, the first round
+        // alone / in a span: 70000 generators 9.2 / 8.1 ms, 100000 10.4 / 10.5, 2^17 11.1 / 11.5, 2^18 17.7 / 18.8.
         if (!comb && r >= cross_r && rounds - r >= JUMP_ROUNDS && size * (size_t)count <= (size_t)SPAN_MAX_N) {
             int rc = open_batch_launch(cs, cg, count, size, JUMP_ROUNDS, false, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, aux, job.events, later);
             if (rc) return rc;
