@@ -1,6 +1,7 @@
 """GPU parity: G1 tensor kernels, Pedersen commitment (fixed-base windowed MSM) and its opening, compared
 with the CPU oracle as group elements (both sides normalised to z = ONE, which makes them byte-equal)."""
 import random
+from operator import mul
 
 import numpy as np
 import pytest
@@ -183,10 +184,8 @@ def test_commit_int_rejects_non_integer_scalars_and_is_linear(pv, orc):
 
 
 # 300 x 1: raw small integers, whose negative embeddings share their high bytes (one bucket receives whole chunks);
-# 4500 x 2: more than one chunk of the bucket kernel and odd sizes in several rounds; 20000 x 2: two halving rounds
-# (the second takes T from the first round's points) before the batched rest; 70000 x 1: four halving rounds, so T of
-# rounds 1..3 are combinations of up to seven earlier points, with an odd size (4375 pairs + 1) on the way
-# 9001 x 1: an odd size in the first halving round, whose T is the sum over pairs with one element left alone
+# up to 9001 x 1: all rounds in one batch of sums over the generators, 4500 x 2 with more than one chunk of the bucket kernel and
+# odd sizes on the way; 20000 x 2 and 70000 x 1: three rounds as one fold beside the batch of their sums, then the batched rest
 @pytest.mark.parametrize("n,m", [(4, 2), (8, 1), (16, 4), (5, 3), (1, 2), (300, 1), (4500, 2), (9001, 1), (20000, 2), (70000, 1)])
 def test_open_value_and_g1_transcript(pv, orc, n, m):
     gens = oracle_gens(orc, 15 + n, n)
@@ -249,9 +248,9 @@ def test_open_with_several_digits_shared_by_many_scalars(pv, orc, counts):
 
 
 def test_open_with_equal_opposite_and_infinite_generators_in_the_first_round(pv, orc):
-    """More generators than the batched rest takes, so the first round halves them on the device: pairs of equal
-    generators (their sum is a doubling), of opposite ones (their sum is infinity), with an infinite member, and an
-    infinite pair, in the pair sums that give T, in the fold and in the bucket sums."""
+    """Pairs of equal generators (their sum is a doubling), of opposite ones (their sum is infinity), with an infinite
+    member, and an infinite pair, in the bucket sums: 8200 generators take all their rounds as one batch.  The folds meet such
+    generators in test_open_follows_the_logarithms_of_its_generators and its batched counterpart."""
     n = 8200
     gens = oracle_gens(orc, 77, n)
     neg = np.zeros((1, 36), np.uint32)
@@ -310,10 +309,10 @@ def test_open_begin_end_matches_open_through_the_c_abi(orc):
 
 def test_open_batch_over_prepared_generators_matches_single_openings(orc):
     """zk_g1_open_begin_batch (openings of one size as ONE job: every round's kernels launched once for all of them) over
-    generators prepared with zk_g1_open_prepare delivers, opening by opening, the bytes of zk_g1_open.  Sizes on both
-    sides of the batched last rounds, a ragged one (odd halves: its first two rounds run on the prepared tables), special
-    generators (equal, opposite, infinite, also among the second round's prepared points) in one member of the batch,
-    and zk_g1_open_begin_prepared alone."""
+    generators prepared with zk_g1_open_prepare delivers, opening by opening, the bytes of zk_g1_open.  Jobs on both
+    sides of the 16384 generators (all openings together) from which on every round is in one batch: above, the first round runs on the
+    prepared tables.  Special generators (equal, opposite, infinite) in one member of the batch, and zk_g1_open_begin_prepared
+    alone.  (A second round on its tables: test_open_batches_follow_the_logarithms_of_their_generators.)"""
     import ctypes
     from gpuhelp import Hip, c_void_p, c_size_t, c_int
     hip = Hip()
@@ -375,24 +374,26 @@ def test_open_batch_over_prepared_generators_matches_single_openings(orc):
             hip.free(x)
 
 
-def test_open_batch_with_row_commitments_delivers_the_points_of_the_plain_opening(pv):
+# two openings a job: 5000: all rounds in one batch; 9000: one round on the prepared table, or three in a span; 50000: two rounds on the tables
+# and a span, or one round without tables and a span
+@pytest.mark.parametrize("n,tables", [(5000, 2), (9000, 2), (9000, 0), (50000, 2), (50000, 0)])
+def test_open_batch_with_row_commitments_delivers_the_points_of_the_plain_opening(pv, n, tables):
     """zk_g1_open_begin_batch_rows takes the first round's T from the tensors' row commitments (sum_r eq(u_rows, r) C_r)
     instead of summing over all generators: for commitments made by commit_int of the same tensors every point of the
     proof, T of the first round included, equals zk_g1_open's on the row-folded vector.  One tensor with a number of
-    rows that is no power of two, one with a single row (no row challenge), more generators than the batched last
-    rounds take; and with another tensor's commitments only the T of the halving rounds change."""
+    rows that is no power of two, one with a single row (no row challenge); and with another tensor's commitments only the
+    T of the rounds over more than 1024 generators change."""
     import ctypes
     from gpuhelp import Hip, c_void_p, c_size_t, c_int
     hip = Hip()
     pv.lib.zkp_g1_devptr.restype = ctypes.c_void_p
-    n = 5000
     k = (n - 1).bit_length()
     npts = 3 * k + 1
     pv.seed(77)
     gens = pv.commitment_random(n)
     dG = pv.lib.zkp_g1_devptr(c_void_p(gens.h))
     prep = c_void_p()
-    hip.call("zk_g1_open_prepare", ctypes.byref(prep), c_void_p(dG), c_size_t(n), None)
+    hip.call("zk_g1_open_prepare_tables", ctypes.byref(prep), c_void_p(dG), c_size_t(n), c_int(tables), None)
     rng = np.random.default_rng(5)
     keep, folded, coms, urows, us = [], [], [], [], []
     exp_p = np.zeros((2, npts, 36), np.uint32)
@@ -431,27 +432,31 @@ def test_open_batch_with_row_commitments_delivers_the_points_of_the_plain_openin
     assert (got_v == exp_v).all()
     assert (got_p == exp_p).all()
     # the statement "these are the tensor's row commitments" is the caller's: with the other tensor's, T of the first round
-    # is what those commitments give, and with it T of the later halving rounds, which follow from the earlier rounds' points
-    # (5000 -> 2500 -> 1250 -> 625 generators, then the batched last rounds, which sum over the generators); T0, T1 of
-    # every round, the folded generator and the value do not depend on them
+    # is what those commitments give, and with it T of the later rounds over more than 1024 generators, which follow from the earlier
+    # rounds' points (the rest are sums over the generators); T0, T1 of every round, the folded generator and the value do not
+    # depend on them
     got_p, got_v = run((1, 0))
     assert (got_v == exp_v).all()
+    sizes = [n]
+    while sizes[-1] > 1:
+        sizes.append((sizes[-1] + 1) // 2)
+    unrolled = [3 * r for r, size in enumerate(sizes) if size > 1024]
     same = np.ones(npts, bool)
-    same[[0, 3, 6]] = False
+    same[unrolled] = False
     assert (got_p[:, same] == exp_p[:, same]).all()
     for i in range(2):
-        assert not (got_p[i, 0] == exp_p[i, 0]).all() and not (got_p[i, 3] == exp_p[i, 3]).all() and not (got_p[i, 6] == exp_p[i, 6]).all()
+        assert not any((got_p[i, j] == exp_p[i, j]).all() for j in unrolled)
     hip.call("zk_g1_open_prepared_free", prep)
 
 
-@pytest.mark.parametrize("n,R,tables", [(8192, 2, 2), (16384, 3, 3), (32768, 3, 3)])
+# two openings a job.  8192: all rounds in one batch of sums over the generators, which needs no commitments; 16384: one round before that batch, or three as one fold; 32768: two rounds, or that fold
+@pytest.mark.parametrize("n,R,tables", [(8192, 2, 2), (16384, 3, 3), (16384, 2, 2), (32768, 3, 3), (32768, 2, 2), (32768, 3, 2), (32768, 3, 0)])
 def test_open_batch_with_cross_commitments_needs_no_sum_over_the_generators(pv, orc, n, R, tables):
     """With the cross commitments of its first R rounds -- commitments of every 2nd / 4th / 8th column of the tensor's rows
     under every 2nd / 4th / 8th generator, made here with commit_int on slices -- zk_g1_open_begin_batch_rows forms T, T0 and
-    T1 of those rounds from rows x patterns points: of the three halvings of 8192 generators before the batched last rounds
-    only the third sums over its generators.  With three rounds of them and the tables of zk_g1_open_prepare_tables(.., 3) the
-    three rounds are one fold (16384 generators: that fold, one ordinary round and the batched last rounds; 32768: two ordinary
-    rounds behind it).  Every point of the proof equals zk_g1_open's on the row-folded vector, and at 16384 generators also the
+    T1 of those rounds from rows x patterns points, for the rounds that come before the batch which takes all the rest (16384 generators
+    of the whole job).  With three rounds of them the three rounds are one fold, from the tables of zk_g1_open_prepare_tables(.., 3)
+    or, with other tables or none, as a span.  Every point of the proof equals zk_g1_open's on the row-folded vector, and at 16384 generators also the
     oracle's own opening of the padded tensor (Commitment::open, commitment.cu:133-141: row fold, then me_open), point by
     point after normalisation, so the batched path is compared with the reference's algorithm directly."""
     import ctypes
@@ -493,7 +498,7 @@ def test_open_batch_with_cross_commitments_needs_no_sum_over_the_generators(pv, 
         hip.call("zk_g1_open", exp_p[i], exp_v[i], c_void_p(f.devptr), c_void_p(dG), c_size_t(n), u, c_int(k), None)
         keep += [W, f]
         folded.append(f); urows.append(np.ascontiguousarray(ur, dtype=np.uint32)); us.append(u)
-        if n == 16384:
+        if n == 16384 and R == 3:
             rows_p = 1 << kr
             Tp = np.zeros((rows_p * n, 8), np.uint32)
             Tp[:nrows * n] = fr_array([int(x) % R_MOD for x in Wi.ravel()])
@@ -521,6 +526,138 @@ def test_open_batch_with_cross_commitments_needs_no_sum_over_the_generators(pv, 
     hip.call("zk_g1_open_prepared_free", prep)
     for x in cross:
         hip.free(x)
+
+
+def opening_logarithms(a, s, u):
+    """The opening of the scalars s over the generators [a_i] G with the challenges u (Commitment::me_open, commitment.cu:109-129) in the
+    exponent: the logarithms of T, T0, T1 of every round and of the folded generator, and the folded scalar."""
+    out = []
+    for x in u:
+        if len(a) % 2:
+            a, s = a + [0], s + [0]
+        a0, a1, s0, s1 = a[0::2], a[1::2], s[0::2], s[1::2]
+        t0, t1 = sum(map(mul, s0, a1)) % R_MOD, sum(map(mul, s1, a0)) % R_MOD
+        out += [(sum(map(mul, s0, a0)) + sum(map(mul, s1, a1))) % R_MOD, t0, t1]
+        a = [(q + x * (p - q)) % R_MOD for p, q in zip(a0, a1)]
+        s = [(p + x * (q - p)) % R_MOD for p, q in zip(s0, s1)]
+    return out + a, s[0]
+
+
+def special_logarithms(seed, n, shift=0):
+    """n random logarithms, among them equal, opposite and infinite generators in pairs, in pairs of pairs and in eights, also eights that
+    are one generator throughout, that cancel, that hold one generator alone and, a wave's worth and more, none at all"""
+    a = fr_ints(mt_random_vec(np.random.RandomState(seed), n))
+    b = a[:]
+    b[1], b[3], b[5], b[6], b[7] = b[0], -b[2], 0, 0, 0
+    b[15], b[18], b[19], b[23] = b[13], b[16], b[17], -b[21]         # special only in the second round
+    b[24:32] = [b[24]] * 8
+    b[32:40] = [b[32], -b[32]] * 4
+    b[40:48] = [0] * 8
+    b[48:56] = [0] * 5 + [b[53]] + [0] * 2
+    b[64:72] = [b[64], 0, 0, 0, -b[64], 0, 0, 0]
+    b[1024:2048] = [0] * 1024
+    if n % 2:
+        b[n - 1] = 0 if shift else b[n - 2]
+    b[:2048] = b[shift:2048] + b[:shift]
+    return [x % R_MOD for x in b]
+
+
+def known_generators(hip, a):
+    from gpuhelp import c_size_t, c_void_p
+    dA, dG = hip.upload(fr_array(a)), hip.malloc(144 * len(a))
+    hip.call("zk_g1_fixed_base_mul", c_void_p(dG), np.ascontiguousarray(affine_to_jac((G1_X, G1_Y)), dtype=np.uint32), c_void_p(dA), c_size_t(len(a)), None)
+    hip.sync()
+    hip.free(dA)
+    return dG
+
+
+def assert_points_are(points, logarithms):
+    assert len(points) == len(logarithms)
+    for i, (p, l) in enumerate(zip(points, logarithms)):
+        assert jac_to_affine(p) == (ec_mul(l, (G1_X, G1_Y)) if l else None), i
+
+
+# 16385 .. 98304: three rounds in a span, then the batched rest (70001 with odd sizes throughout); above: one round alone (98305: its last
+# generator has no partner), two at 2^18 + 3, then a span
+@pytest.mark.parametrize("n", [16385, 20000, 70001, 98304, 98305, 131072, 140001, (1 << 18) + 3])
+def test_open_follows_the_logarithms_of_its_generators(n):
+    """An unprepared opening over generators of known logarithm, special ones among them, point by point in big-integer arithmetic."""
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    k = (n - 1).bit_length()
+    a = special_logarithms(90, n)
+    S, u = mt_random_vec(np.random.RandomState(91), n), mt_random_vec(np.random.RandomState(92), k)
+    dG, dS = known_generators(hip, a), hip.upload(S)
+    points, value = np.zeros((3 * k + 1, 36), np.uint32), np.zeros(8, np.uint32)
+    print(f"zk_g1_open n={n}", flush=True)
+    hip.call("zk_g1_open", points, value, c_void_p(dS), c_void_p(dG), c_size_t(n), u, c_int(k), None)
+    logs, exp_value = opening_logarithms(a, fr_ints(S), fr_ints(u))
+    assert fr_ints(value)[0] == exp_value
+    assert_points_are(points, logs)
+    hip.free(dG)
+    hip.free(dS)
+
+
+@pytest.mark.parametrize("slice_bits,sign,first", [(b, s, None) for b in (15, 16, 17) for s in (1, -1)] + [(0, 1, f) for f in ((0, 0, 0), (1, 1, 1), (1, 0, 1), (R_MOD - 1, 2, 1))])
+def test_span_of_rounds_whose_slices_meet_themselves(slice_bits, sign, first):
+    """The slices of a span's combination added to one another as equal and as opposite points: with u = 2/3, 2/3 and 9/4 * 2^slice the
+    first generator's coefficient is 2^slice, one digit in the second slice, and those of the next two are 2^(slice - 1), in the first: the
+    first slice's point, +-2^slice times the generator, meets the second slice's after its doublings.  Which width a slice has follows from
+    the longest of all coefficients: one of the three.  Then challenges that leave single or short coefficients."""
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    n = 16400
+    k = (n - 1).bit_length()
+    u = fr_ints(mt_random_vec(np.random.RandomState(93), k))
+    inv = lambda x: pow(x, -1, R_MOD)
+    u[:3] = first if first is not None else (2 * inv(3) % R_MOD, 2 * inv(3) % R_MOD, 9 * inv(4) * (1 << slice_bits) % R_MOD)
+    a = special_logarithms(94, n)
+    for m in range(512, 600):
+        a[8 * m:8 * m + 8] = [a[8 * m], sign * a[8 * m] % R_MOD, sign * a[8 * m] % R_MOD, 0, 0, 0, 0, 0]
+    S = mt_random_vec(np.random.RandomState(95), n)
+    dG, dS = known_generators(hip, a), hip.upload(S)
+    points, value = np.zeros((3 * k + 1, 36), np.uint32), np.zeros(8, np.uint32)
+    print(f"zk_g1_open n={n} slice {slice_bits} sign {sign} first {first}", flush=True)
+    hip.call("zk_g1_open", points, value, c_void_p(dS), c_void_p(dG), c_size_t(n), fr_array(u), c_int(k), None)
+    logs, exp_value = opening_logarithms(a, fr_ints(S), u)
+    assert fr_ints(value)[0] == exp_value
+    assert_points_are(points, logs)
+    hip.free(dG)
+    hip.free(dS)
+
+
+# 4099 x 8 and 33001: the first and the second round on their tables (odd halves); 12300 x 8: the first alone without tables, or on its table;
+# 40000 x 3: three, the third without a table; 2051 x 8: the first on its table and no table for the second
+@pytest.mark.parametrize("n,count,tables", [(4099, 8, 2), (33001, 1, 2), (12300, 8, 0), (12300, 8, 1), (12300, 8, 2), (40000, 3, 2), (2051, 8, 2)])
+def test_open_batches_follow_the_logarithms_of_their_generators(n, count, tables):
+    """zk_g1_open_begin_batch over prepared generators of known logarithm, special ones at another place in each member."""
+    import ctypes
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    k = (n - 1).bit_length()
+    a, S, u, preps, keep = [], [], [], [], []
+    for i in range(count):
+        a.append(special_logarithms(100 + i, n, i % 3))
+        S.append(mt_random_vec(np.random.RandomState(110 + i), n))
+        u.append(mt_random_vec(np.random.RandomState(120 + i), k))
+        dG = known_generators(hip, a[i])
+        preps.append(c_void_p())
+        hip.call("zk_g1_open_prepare_tables", ctypes.byref(preps[i]), c_void_p(dG), c_size_t(n), c_int(tables), None)
+        hip.free(dG)
+        keep.append(hip.upload(S[i]))
+    h = c_void_p()
+    print(f"zk_g1_open_begin_batch n={n} count={count} tables={tables}", flush=True)
+    hip.call("zk_g1_open_begin_batch", ctypes.byref(h), c_int(count), (c_void_p * count)(*[c_void_p(x) for x in keep]), (c_void_p * count)(*preps),
+             np.ascontiguousarray(np.concatenate(u), dtype=np.uint32), c_int(k), None)
+    points, values = np.zeros((count, 3 * k + 1, 36), np.uint32), np.zeros((count, 8), np.uint32)
+    hip.call("zk_g1_open_end_batch", h, points, values)
+    for i in range(count):
+        logs, exp_value = opening_logarithms(a[i], fr_ints(S[i]), fr_ints(u[i]))
+        assert fr_ints(values[i])[0] == exp_value
+        assert_points_are(points[i], logs)
+    for pr, p in zip(preps, keep):
+        hip.call("zk_g1_open_prepared_free", pr)
+        hip.free(p)
 
 
 def test_fixed_base_multiplication_equals_the_generic_one_and_big_integer_arithmetic(orc):
