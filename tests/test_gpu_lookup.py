@@ -82,7 +82,7 @@ def test_multiplicities(pv, D, low, length):
     rng = np.random.default_rng(D)
     vals = rng.integers(low, low + length, D)
     vals[: D // 3] = low + length // 2               # a long run of equal values (wave aggregation path)
-    # queries that keep an int32 form are counted from it, positions formed by the counting passes (zk_lookup_hist_i32)
+    # queries that keep an int32 form are counted from it, positions formed by the counting passes
     hk = pv.from_i64(vals)
     pv.keep_for_folds(hk)
     assert pv.folds_from_ints(hk) == 1
@@ -91,6 +91,78 @@ def test_multiplicities(pv, D, low, length):
     assert (mk == m).all()
     size = 1 << max(0, (length - 1).bit_length())
     assert fr_ints(m) == [int(c) for c in np.bincount(vals - low, minlength=size)]
+
+
+@pytest.mark.parametrize("D,low,length", [(1, 7, 1), (64, -5, 11), (5000, -(1 << 31), 1 << 14), (70001, -(1 << 15), 16385), ((1 << 20) + 5, 1000, (1 << 17) + 3)])
+def test_positions_and_counts_through_the_c_abi(D, low, length):
+    """The entry points that the class layer has no call for any more, beside the one that it has: table positions (zk_lookup_index_fr, _i32),
+    counts (zk_lookup_hist, _hist_i32), conversion of counts (zk_fr_from_u32) and zk_lookup_multiplicities from positions, int32 queries and
+    field elements, with its positions and without its check.  A query on either side of the table is refused by each that sees it."""
+    from gpuhelp import Hip, c_int, c_size_t, c_uint, c_void_p
+    hip = Hip()
+    P = c_void_p
+    rng = np.random.default_rng(D)
+    vals = rng.integers(low, low + length, D)
+    vals[: D // 3] = low + length - 1
+    want, counts = vals - low, np.bincount(vals - low, minlength=length)
+    L, N, n = c_int(low), c_uint(length), c_size_t(D)
+    i32 = hip.upload(vals.astype(np.int32))
+    i64, fr, idx, cnt, m = hip.upload(vals.astype(np.int64)), hip.malloc(32 * D), hip.malloc(4 * D), hip.malloc(4 * length), hip.malloc(32 * length)
+    hip.call("zk_fr_from_i64", P(fr), P(i64), n, None)
+    sources = (("zk_lookup_index_i32", i32), ("zk_lookup_index_fr", fr))
+    for name, src in sources:
+        hip.call("zk_memset", P(idx), c_int(255), c_size_t(4 * D), None)
+        hip.call(name, P(idx), P(src), L, N, n, None)
+        assert (hip.download(idx, D, np.uint32) == want).all(), name
+    for name, args in (("zk_lookup_hist", (P(cnt), P(idx), n, N, None)), ("zk_lookup_hist_i32", (P(cnt), P(i32), L, N, n, N, None))):
+        hip.call("zk_memset", P(cnt), c_int(255), c_size_t(4 * length), None)
+        hip.call(name, *args)
+        assert (hip.download(cnt, length, np.uint32) == counts).all(), name
+    for positions, ints, elements in ((idx, None, None), (None, i32, None), (None, None, fr)):
+        for out in (None, hip.malloc(4 * D)):
+            for inside in (0, 1):
+                hip.call("zk_memset", P(m), c_int(255), c_size_t(32 * length), None)
+                hip.call("zk_lookup_multiplicities", P(m), P(out), P(positions), P(ints), P(elements), L, N, n, N, c_int(inside), None)
+                got = hip.download(m, (length, 8), np.uint32)
+                assert (got[:, 0] == counts).all() and not got[:, 1:].any()
+                if out and not positions:
+                    assert (hip.download(out, D, np.uint32) == want).all()
+            if out:
+                hip.free(out)
+    for outside in (low - 1, low + length):
+        if not -(1 << 31) <= outside < 1 << 31:
+            continue
+        vals[D // 2] = outside
+        hip.call("zk_memcpy_h2d", P(i32), vals.astype(np.int32), c_size_t(4 * D), None)
+        hip.call("zk_memcpy_h2d", P(i64), vals.astype(np.int64), c_size_t(8 * D), None)
+        hip.call("zk_fr_from_i64", P(fr), P(i64), n, None)
+        for name, src in sources:
+            with pytest.raises(RuntimeError, match="outside the table"):
+                hip.call(name, P(idx), P(src), L, N, n, None)
+        with pytest.raises(RuntimeError, match="outside the table"):
+            hip.call("zk_lookup_hist_i32", P(cnt), P(i32), L, N, n, N, None)
+        for ints, elements in ((i32, None), (None, fr)):
+            with pytest.raises(RuntimeError, match="outside the table"):
+                hip.call("zk_lookup_multiplicities", P(m), None, None, P(ints), P(elements), L, N, n, N, c_int(0), None)
+    whole = np.array([0, 1, (1 << 31) - 1, 1 << 31, (1 << 32) - 1] + list(range(D % 700)), np.uint32)
+    du, df = hip.upload(whole), hip.malloc(32 * whole.size)
+    hip.call("zk_fr_from_u32", P(df), P(du), c_size_t(whole.size), None)
+    assert fr_ints(hip.download(df, (whole.size, 8), np.uint32)) == [int(x) for x in whole]
+    for p in (i32, i64, fr, idx, cnt, m, du, df):
+        hip.free(p)
+
+
+@pytest.mark.parametrize("n,value", [(1, -1), (257, 7), (100003, -(1 << 31))])
+def test_int32_fill_through_the_c_abi(n, value):
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    d = hip.upload(np.full(n + 1, 5, np.int32))
+    hip.call("zk_i32_fill", c_void_p(d), c_int(value), c_size_t(n), None)
+    got = hip.download(d, n + 1, np.int32)
+    assert (got[:n] == value).all() and got[n] == 5
+    hip.call("zk_i32_fill", c_void_p(d), c_int(9), c_size_t(0), None)
+    assert hip.download(d, 1, np.int32)[0] == value
+    hip.free(d)
 
 
 @pytest.mark.parametrize("D,low,length,skew", [((1 << 21) + 12345, -5, (1 << 18) + 777, 3), (1500000, 0, 1 << 20, 1), ((1 << 20) + 1, -9, 1 << 22, 0)])
