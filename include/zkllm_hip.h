@@ -68,7 +68,8 @@ int zk_defer_wait(void* batch, uint32_t* out_host, size_t max_fr, size_t* n_fr);
 int zk_defer_free(void* batch);
 /* replace cudaMemcpy in ctors, operator()(idx), savebin/loadbin (ioutils.cu:3-45) */
 int zk_memcpy_h2d(void* dst, const void* src_host, size_t bytes, void* stream);
-int zk_upload(void* dst, const void* src, size_t bytes, void* stream);          /* as zk_memcpy_h2d, for data that only work queued on `stream` reads: may return before it is there */
+/* as zk_memcpy_h2d, for data that only work queued on `stream` reads: may return before it is there */
+int zk_upload(void* dst, const void* src_host, size_t bytes, void* stream);
 int zk_memcpy_d2h(void* dst_host, const void* src, size_t bytes, void* stream);
 int zk_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream);
 int zk_memset(void* dst, int value, size_t bytes, void* stream);
@@ -264,7 +265,8 @@ int zk_g1_open_end(void* handle, uint32_t* proof_host, uint32_t* final_scalar_ho
  * bytes; nothing in it depends on the opened tensor) and, above 1024 generators, the fixed-base tables of the
  * first two rounds' folds (255 points per generator pair for the first round, as much again for the second when it
  * folds more than 1024 generators: 28 KB per generator in all, kept until the handle is freed; building them takes
- * about as much again in temporaries).  zk_g1_open_begin_prepared is zk_g1_open_begin with
+ * about as much again in temporaries).  A job of at most 16384 generators, all its openings together, folds none and reads no table: for
+ * sets of that size that are opened alone, tables = 0 below makes the same proofs in the same time.  zk_g1_open_begin_prepared is zk_g1_open_begin with
  * such generators; the handle must outlive every opening started with it and is released with
  * zk_g1_open_prepared_free. */
 int zk_g1_open_prepare(void** prepared, const void* gens, size_t n, void* stream);
@@ -295,11 +297,13 @@ int zk_g1_open_begin_batch(void** handle, int count, const void* const* scalars,
  * 4^q of T1_q, X[r] = sum_j W[r][2^(q+1) j + 2^q + a] g_(2^(q+1) j + b): 1 + 2 (4^R - 1) / 3 patterns in all (the host
  * layer's Commitment::cross_commitments makes them with commit_int over strided parts).  u_rows[i]: the k_rows[i] challenges
  * the rows were folded with, lowest row bit first, 2^k_rows >= nrows.
- * T of the first round is then sum_r eq(u_rows, r) C_r, and T0, T1 of the first R halving rounds are the combinations
+ * T of the first round is then sum_r eq(u_rows, r) C_r, and T0, T1 of the first R rounds are the combinations
  * of the cross patterns with the products of the earlier rounds' challenges -- sums over rows x patterns points instead
- * of bucket sums over all generators; those rounds then consist of their fold alone.  The points equal the sums over the
+ * of bucket sums over all generators; those rounds then consist of their fold alone.  (Only rounds that fold: from 16384 generators of the
+ * job on all rounds are one batch of sums over the generators.)  With R = 0, T of the later rounds over more than 1024 generators
+ * follows from the earlier rounds' points.  The points equal the sums over the
  * generators whenever rows[i] are such commitments of the tensor under these generators -- the caller's statement;
- * with other points T, T0, T1 of the halving rounds differ from zk_g1_open_begin_batch's, nothing else does. */
+ * with other points T, T0, T1 of those rounds differ from zk_g1_open_begin_batch's, nothing else does. */
 int zk_g1_open_begin_batch_rows(void** handle, int count, const void* const* scalars, const void* const* prepared, const uint32_t* u, int rounds,
                                 const void* const* rows, const uint32_t* nrows, const uint32_t* const* u_rows, const int* k_rows, int cross_rounds, void* stream);
 int zk_g1_open_end_batch(void* handle, uint32_t* proof_host, uint32_t* final_scalar_host);
@@ -309,11 +313,14 @@ int zk_g1_open_end_batch(void* handle, uint32_t* proof_host, uint32_t* final_sca
  * unlike the reference, a value outside [low, low+table_size) is an error instead of an unchecked access */
 int zk_lookup_index_fr(void* idx_u32, const void* vals_fr, int32_t low, uint32_t table_size, size_t n, void* stream);
 int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32_t table_size, size_t n, void* stream);
-/* multiplicities (tlookup_kernel :10-15): counts[b] = #{i : idx[i] == b}; counts is cleared first */
-/* multiplicities of a table's entries (nbins field elements) from positions, int32 queries or field elements, the first that is not null; idx_out: the positions too, or null */
-int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, int inside, void* stream);      /* inside: the caller knows every query to lie in the table; nothing is checked or waited for */
+/* multiplicities of a table's nbins entries as field elements (tlookup_kernel :10-15, count_to_m :17-20) from table positions (idx; not
+ * checked, as there), int32 queries or queries as field elements, the first that is not null; idx_out: the positions too, or null.  A query
+ * outside [low, low + len) is an error, known when the call returns.  inside: the caller knows every query to lie in the table; nothing is
+ * checked or waited for */
+int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins, int inside, void* stream);
+/* the counts alone, as 32-bit integers: counts[b] = #{i : idx[i] == b}; counts is cleared first */
 int zk_lookup_hist(void* counts_u32, const void* idx_u32, size_t n, uint32_t nbins, void* stream);
-/* zk_lookup_index_i32 and zk_lookup_hist in one (tLookupRange::prep over queries that keep an int32 form): the counting passes
+/* zk_lookup_index_i32 and zk_lookup_hist in one: the counting passes
  * form the positions value - low themselves and no array of positions is written; a value outside [low, low + len) is an error */
 int zk_lookup_hist_i32(void* counts_u32, const void* vals_i32, int32_t low, uint32_t len, size_t n, uint32_t nbins, void* stream);
 int zk_range_table(void* table_fr, int32_t low, uint32_t len, uint32_t table_size, void* stream);   /* tlookuprange_init_kernel :372-380 */
@@ -336,7 +343,8 @@ int zk_lookup_round(uint32_t* sums_host, void* new_A, void* new_S, void* new_B, 
 int zk_hadamard_round(uint32_t* coefs_host, void* const* new_Xs, const void* const* Xs, int K, const void* E, const uint32_t* v, size_t n_out, void* stream);
 /* both sumchecks whole, queued without a host round trip (all rounds' sums come back in one copy): their challenges
  * are fixed before the first round (tLookup::prove tlookup.cu:150-176 and multi_hadamard_sumchecks proof.cu:191-241 take
- * u and v as arguments).  Rounds on short tensors (<= 512 pairs) run inside one launch.  Lookup: A, S of
+ * u and v as arguments).  The rounds on at most 2^16 pairs share
+ * a few launches.  Lookup: A, S of
  * D elements, B, T, m of N (D/N a power of two), E of D/2; v: rounds x 8 limbs in round order; sums_host: rounds x 11.
  * Hadamard: K tensors of N elements (a power of two), E of N/2; coefs_host: log2(N) x (K+1).  Inputs are not modified. */
 int zk_lookup_sumcheck(uint32_t* sums_host, const void* A, const void* S, const void* B, const void* T, const void* m, const void* E, const uint32_t* beta,

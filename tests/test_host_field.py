@@ -34,7 +34,7 @@ def test_host_fr_ops_match_bigint_and_oracle():
         assert fr_ints(got) == [f(x, y) for x, y in zip(a, b)], f"host fr op {op}"
         orc_check(orc.orc_fr_op(op, A, B, exp, len(a)))
         assert (got == exp).all(), f"host fr op {op} vs oracle"
-    # Montgomery inverse (binary algorithm in the product, exponentiation in the oracle): x = aR -> a^-1 R = x^-1 R^2
+    # Montgomery inverse (Lehmer's algorithm in the product, exponentiation in the oracle): x = aR -> a^-1 R = x^-1 R^2
     inv_in = a + [1 << k for k in range(0, 255, 7)] + [R_MOD - (1 << k) for k in range(0, 254, 9)] + [(1 << 254) + 1, 3, R_MOD // 2, R_MOD // 2 + 1]
     IA = fr_array(inv_in)
     got, exp = np.zeros_like(IA), np.zeros_like(IA)

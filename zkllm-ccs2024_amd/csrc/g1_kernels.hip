@@ -890,7 +890,9 @@ __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, c
 // The walk is one chain, so a launch takes what one chain takes whatever the number of sums: all of a job's sums that nothing waits for
 // go into one launch, those of few elements behind the others (first_few), four to a workgroup.  A lane's chain takes 1.5 ms; four lanes
 // that share a point's products take 1.25 ms, and a compute unit holds one such workgroup: LANES is four while all of a launch's fit
-// beside each other, one for longer lists (310 workgroups of four took 2.6 ms).
+// beside each other and beside what else runs, one for longer lists (310 workgroups of four took 2.6 ms).  192 workgroups: an opening of
+// 2^17 generators (18 and 86 workgroups) takes 11.9 ms on four lanes and 13.1 on one, one of 16384 5.1 and 5.3; a layer of small products
+// 6.9 to 7.1 ms with the line at 96 or 192, 7.4 on one lane or on four throughout, and the layer of 2048 x 2048 54.6, 54.8 and 55.4.
 struct PointDesc { J29* buckets; G1Jac* out; uint32_t half_off, few; };     // half_off: where the second half's buckets begin
 template <int LANES> __device__ __forceinline__ void walk_double(J29& p, uint32_t q) {
     if constexpr (LANES == 4) j29_quad_double(p, q);
@@ -2662,9 +2664,9 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
     {
         Arena arena(st);
         rc = open_prep_build((A29*)pr->a29, (const G1Jac*)gens, n, arena, st);
-        // The combs of the first two rounds, for each round that is a fold (more generators than the batched last rounds
-        // take): entry-major tables of the subset sums of 2^(j COMB_W) P over the round's prepared points P (the pair
-        // differences D; for the second round F and H, see k_open_fold_comb), built from elementwise point kernels -- the
+        // The combs of the first two rounds, for each round over more than TABLE_MIN_N generators: how many openings share a job is not known
+        // here, and a job of more than LAST_N generators in all folds these rounds.  Entry-major tables of the subset sums of
+        // 2^(j COMB_W) P over the round's prepared points P (the pair differences D; for the second round F and H, see k_open_fold_comb), built from elementwise point kernels -- the
         // teeth by repeated doubling (an addition of an array to itself), entry m = entry (m without its lowest bit) + entry
         // (that bit).
         // The tables only make the folds cheaper: ZKLLM_OPEN_TABLES = 0 or 1 keeps none or the first round's alone (28 KB
@@ -2673,7 +2675,7 @@ static int open_prepare_impl(void** prepared, const void* gens, size_t n, int ta
         static const int env_rounds = [] { const char* e = getenv("ZKLLM_OPEN_TABLES"); return e ? atoi(e) : -1; }();
         const int table_rounds = env_rounds >= 0 ? env_rounds : table_mode;
         // mode 3: the seven tables of k_open_fold_jump in place of those two (as large as both together); only for a power of
-        // two of generators that leaves more than the batched last rounds take after three folds
+        // two of generators that leaves at least TABLE_MIN_N after three folds
         const bool jump = table_rounds >= 3 && !(n & (n - 1)) && (n >> JUMP_ROUNDS) >= (size_t)TABLE_MIN_N;
         if (rc == 0 && jump) {
             const size_t no = n >> JUMP_ROUNDS, ne = no * COMB_N * JUMP_TABS;

@@ -636,9 +636,9 @@ __global__ void __launch_bounds__(256) k_gemm_i8_planes(const PlaneGemm g) {
             if (row < g.M && col < g.P) gemm_store(g, (b * g.M + row) * (size_t)g.P + col, tot[q][r]);
         }
 }
-// The same product for up to three planes a side (every projection and attention product of the LLaMa layer): all plane pairs
-// are multiplied while a K tile lies in LDS, pairs of equal weight 256^(i+j) into one int32 accumulator (at most three pairs
-// of at most K * 2^14 each; the caller keeps 3 K below 2^17), and the int64 recombination happens once, in the epilogue.
+// The same product for up to five planes on the left and three on the right (every matrix product of the LLaMa layer): all plane pairs
+// are multiplied while a K tile lies in LDS, pairs of equal weight 256^(i+j) into one int32 accumulator (at most min(PA, PB) pairs
+// of at most K * 2^14 each; the caller keeps min(PA, PB) K below 2^17), and the int64 recombination happens once, in the epilogue.
 // Against the pair-by-pair kernel: one pass over the operands instead of PA * PB, PA * PB times the matrix instructions per
 // barrier, no int64 totals held through the loop.  Block tile 64 x 64, one 32 x 32 tile per wave, two blocks per CU.
 template <int PA, int PB> __global__ void __launch_bounds__(256, 2) k_gemm_i8_planes_all(const PlaneGemm g) {
