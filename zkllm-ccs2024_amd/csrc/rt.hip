@@ -190,9 +190,9 @@ int pool_trim() {
     return 0;
 }
 
-// A stream of a pool, called with g_side_mu held: `job` counts calls (`pair`: which of a job's two streams, -1 for a job of one).  The streams
-// are all made at the first use of any, the openings' first, so that which of them share a hardware queue does not hang on the order of
-// the jobs (4 queues: a layer of 2048 x 2048 takes 55.1 ms when its sumchecks' streams come first, 53.9 ms behind the openings').
+// A stream of a pool, called with g_side_mu held: `job` counts calls (`pair`: which of a job's two streams, -1 for a job of one).  A pool's
+// streams are made in order, and none before a job needs it or one behind it: a stream's own hardware queue costs 5 ms to make, which a
+// process that proves once would pay for every stream.
 static hipStream_t side_stream_locked(int pool, int pair, unsigned job) {
     static int count[2] = {0, 0}, shared = 0;
     if (!count[0]) {
@@ -214,14 +214,14 @@ static hipStream_t side_stream_locked(int pool, int pair, unsigned job) {
     // ZKLLM_SIDE_STREAMS=1,1,1 and a caller on the default stream no two kernels of the library overlap, so a kernel trace
     // shows what each costs alone
     static const bool blocking = [] { const char* e = getenv("ZKLLM_SIDE_STREAMS_BLOCKING"); return e && e[0] == '1'; }();
-    for (int k = 0; k < (shared ? 1 : 2); ++k)
-        for (int i = 0; i < count[k]; ++i) {
-            hipStream_t& s = g_side_streams[k][i];
-            if (!s && hipStreamCreateWithFlags(&s, blocking ? hipStreamDefault : hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); s = nullptr; }
-        }
     unsigned both[2];
     stream_pair(job, (unsigned)count[q], both);
-    return g_side_streams[q][pair < 0 ? job % (unsigned)count[q] : both[pair]];
+    const unsigned want = pair < 0 ? job % (unsigned)count[q] : both[pair], last = pair < 0 ? want : std::max(both[0], both[1]);
+    for (unsigned i = 0; i <= last; ++i) {
+        hipStream_t& s = g_side_streams[q][i];
+        if (!s && hipStreamCreateWithFlags(&s, blocking ? hipStreamDefault : hipStreamNonBlocking) != hipSuccess) { (void)hipGetLastError(); s = nullptr; }
+    }
+    return g_side_streams[q][want];
 }
 hipStream_t side_stream(int pool) {
     std::lock_guard<std::mutex> lk(g_side_mu);

@@ -73,9 +73,9 @@ struct Arena {
 hipStream_t side_stream(int pool);
 // The two streams of an opening that folds (null on failure): folds on one, bucket sums on the other.
 void opening_streams(hipStream_t* folds, hipStream_t* sums);
-// Which two of a pool's `count` streams job `job` takes: two apart.  Of streams made one after the other the last may have got the hardware
-// queue of the one before it (measured: the fourth of four with 4 queues, the eighth of eight with 8; an opening of 2^17 generators on
-// such a pair takes 14.3 ms instead of 11.5), and a pair four apart takes 12.5 ms where every stream has a queue of its own.
+// Which two of a pool's `count` streams job `job` takes: two apart.  Of two streams made one after the other the second may get the
+// hardware queue of the first (the first stream beyond the queues does: measured with 4 queues and with 8); an opening of 2^17
+// generators on such a pair takes 14.3 ms instead of 11.5, and on a pair four apart 12.5 ms where every stream has a queue of its own.
 static inline void stream_pair(unsigned job, unsigned count, unsigned both[2]) {
     both[0] = count >= 4 ? (job / 2 * 4 + job % 2) % count : 2 * job % count;
     both[1] = (both[0] + (count >= 4 ? 2u : 1u)) % count;
