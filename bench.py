@@ -490,8 +490,9 @@ def main():
                                  "one launch per round for all openings of a size)",
                        "bound": "valu-int", "achieved": fold_tops, "peak": VALU_PEAK_TOPS, "unit": "T MAD32/s", "frac": fold_tops / VALU_PEAK_TOPS,
                        "traffic": fold_traffic / max(1, fold_launches), "algorithmic_bytes_per_launch": FOLD_ALGO_BYTES_PER_PAIR * fold_pairs / max(1, fold_launches),
-                       "traffic_note": "bytes per launch from the counters of each kernel ALONE (FETCH_SIZE x 2.000 + WRITE_SIZE per pair: walk 764 B, comb 6991 B, "
-                                       "three-round fold 3937 B -- the table-driven folds read their fixed-base table entries, 112 B each) times the pairs of the "
+                       "traffic_note": "bytes per launch from the counters of each kernel ALONE (FETCH_SIZE x 2.000 + WRITE_SIZE per pair: walk %.0f B, comb %.0f B, "
+                                       "three-round fold %.0f B -- " % (FOLD_TRAFFIC_BYTES_PER_PAIR_AT_262144, COMB_TRAFFIC_BYTES_PER_PAIR, JUMP_TRAFFIC_BYTES_PER_PAIR) +
+                                       "the table-driven folds read their fixed-base table entries, 112 B each) times the pairs of the "
                                        "timed launches; counters of a kernel inside the layer cannot be told apart from its neighbours'",
                        "by_method": fold_methods,
                        "launches": int(fold_launches), "avg_launch_ms": fold_ms / max(1, fold_launches),
@@ -499,7 +500,7 @@ def main():
                        "note": "algorithmic work = Fp multiplications of the point formulas x 300 MAD32 (12-limb schoolbook product and reduction; the kernel "
                                "itself works on 14 limbs of 29 bits: 392 multiply-adds and ~110 other instructions per product, 301 per square); "
                                "peak = 256 CU x 4 SIMD x 16 lanes x 2.4 GHz.  The launches are of every size (524288 pairs in the first round of the "
-                               "two 2^19 openings down to 1024 in the last halving round) and run beside the bucket sums of their own job, beside up to three other opening jobs and beside "
+                               "two 2^19 openings on) and run beside the bucket sums of their own job, beside up to three other opening jobs and beside "
                                "the rest of the proof; traffic was measured for the kernel alone at 262144 pairs (roofline_fold_alone)"}
     if lk_launches:
         out["roofline_lookup_round_in_layer"] = {
@@ -575,17 +576,19 @@ def main():
     msm_s = (time.perf_counter() - t0) / reps
     out["g1_msm_points_per_s"] = 11008 * 4096 / msm_s
     out["g1_msm_ms"] = msm_s * 1e3
-    # algorithmic work of the commitment: one mixed addition (11 Fp multiplications) per c-bit window of the bits the data covers
-    msm_c = 8
+    # algorithmic work of the commitment: one mixed addition (11 Fp multiplications) per signed c-bit digit that is not zero; c = 12 is
+    # the width that zk_g1_commit_int takes for these scalars
+    msm_c = 12
     msm_bits = int(np.abs(Wm).max()).bit_length()
-    msm_windows = (msm_bits + 1 + msm_c - 1) // msm_c      # one spare bit for the signed digits' carry, as zk_g1_commit_int counts them
-    msm_tops = 11008 * 4096 * msm_windows * 11 * MAD_PER_FP_MUL / msm_s / 1e12
+    low = ((Wm + 2048) & 4095) - 2048
+    msm_digits = float((low != 0).mean() + (Wm != low).mean())
+    msm_tops = 11008 * 4096 * msm_digits * 11 * MAD_PER_FP_MUL / msm_s / 1e12
     out["roofline_msm"] = {"kernel": "zk_g1_commit_int (k_msm_rows and the table build, conversion and row sums around it), 11008 x 4096 scalars over 4096 generators",
                            "bound": "valu-int", "achieved": msm_tops, "peak": VALU_PEAK_TOPS, "unit": "T MAD32/s", "frac": msm_tops / VALU_PEAK_TOPS, "traffic": None,
-                           "window_bits_c": msm_c, "scalar_bits_b": msm_bits, "windows": msm_windows,
-                           "note": "algorithmic work = ceil((b + 1) / c) windows x 11 Fp multiplications (one mixed addition) x 300 MAD32 per (scalar, generator) pair, "
-                                   "b = bits of the largest |scalar| in the data, c = 8; the time is the whole commit_int call (fixed-base table of the "
-                                   "generators' multiples built and normalised, scalars range-checked, row sums) -- what g1_msm_points_per_s is quoted on"}
+                           "window_bits_c": msm_c, "scalar_bits_b": msm_bits, "digits_per_scalar": msm_digits,
+                           "note": "algorithmic work = non-zero signed 12-bit digits of the data x 11 Fp multiplications (one mixed addition) x 300 MAD32, "
+                                   "b = bits of the largest |scalar|; the time is the whole commit_int call (fixed-base table of the "
+                                   "generators' multiples built, scalars range-checked, row sums) -- what g1_msm_points_per_s is quoted on"}
     del com, hW, gens
 
     # ---- Fr mul/s: n independent Montgomery products on resident operands ------------------------------------------------------
