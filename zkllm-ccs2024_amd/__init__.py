@@ -35,9 +35,10 @@ def _runtime_started():
 
 
 def _want_hw_queues():
-    """The library keeps up to seven streams busy (the caller's, four for openings, two for sumcheck jobs).  HIP maps
-    streams onto GPU_MAX_HW_QUEUES hardware queues (4 unless set) and streams that share a queue run one after the
-    other, so ask for at least sixteen (measured when this was added: the decoder layer took 7 % less time with 8 queues than with 4 and another 1 % less with 16).  The HIP runtime reads the variable when it is loaded: this must run before that.
+    """HIP maps streams onto GPU_MAX_HW_QUEUES hardware queues (4 unless set) and streams that share a queue run one after the
+    other; the library has up to eleven (the caller's, eight for openings, two for sumcheck jobs), so ask for at least sixteen: the
+    7B-shape decoder layer with its openings at their claims takes 104 ms then and 109 with 4 (started ahead of them 97.7 and 95.5, several openings
+    of 2^16 generators in flight 10 % less with 16).  The HIP runtime reads the variable when it starts: this must run before that.
     ZKLLM_HW_QUEUES=0 leaves the variable alone, ZKLLM_HW_QUEUES=N sets it to N.  Once the runtime has started the variable says how
     many queues there are (the library chooses its number of streams by it) and is left as it is."""
     want = os.environ.get("ZKLLM_HW_QUEUES", "")
