@@ -887,9 +887,10 @@ __global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, c
 // elements has two sets of 8 buckets a window, weighted 1 .. 8 and 16 .. 128: 16 walks a half.  k_msm_join adds the halves, the
 // endomorphism on the second.
 // Raw buckets: buckets[w MT + b] (k_msm_few's: [w 16 + b]); a half's total goes to its first bucket's place, which only its own walks read.
-// The walk is one chain, so a launch takes what one chain takes whatever the number of sums: all of a job's sums that nothing waits for
+// A launch takes what one workgroup takes whatever the number of sums: all of a job's sums that nothing waits for
 // go into one launch, those of few elements behind the others (first_few), four to a workgroup.  A lane's chain takes 1.5 ms; four lanes
-// that share a point's products take 1.25 ms, and a compute unit holds one such workgroup: LANES is four while all of a launch's fit
+// that share a point's products take 1.2 ms (eight waves a workgroup, two a SIMD, 339 k instructions each: a SIMD's whole issue rate, on
+// one compute unit), and a compute unit holds one such workgroup: LANES is four while all of a launch's fit
 // beside each other and beside what else runs, one for longer lists (310 workgroups of four took 2.6 ms).  192 workgroups: an opening of
 // 2^17 generators (18 and 86 workgroups) takes 11.9 ms on four lanes and 13.1 on one, one of 16384 5.1 and 5.3; a layer of small products
 // 6.9 to 7.1 ms with the line at 96 or 192, 7.4 on one lane or on four throughout, and the layer of 2048 x 2048 54.6, 54.8 and 55.4.
