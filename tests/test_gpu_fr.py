@@ -869,6 +869,43 @@ def test_copies_and_clears_take_any_memory_and_refuse_null(hip):
     assert runtime.hipFree(theirs) == 0
 
 
+def test_copies_and_clears_in_a_captured_graph_are_kernels(hip):
+    """zk_memset(0), zk_memcpy_d2d and zk_upload on the allocator's blocks, captured on a stream of the caller's: kernel nodes only, and every
+    replay gives what the eager calls give."""
+    with open("/proc/self/maps") as f:                           # the runtime that the library runs on
+        runtime = ctypes.CDLL(next(x.split()[-1] for x in f if "libamdhip64" in x))
+    P, size, ref = ctypes.c_void_p, ctypes.c_size_t, ctypes.byref
+    n = 1000
+    data = np.random.default_rng(4).integers(0, 1 << 32, n, dtype=np.uint64).astype(np.uint32)
+    few = np.arange(16, dtype=np.uint32) + 7
+    a, b, stream, graph, execute, count = hip.upload(data), hip.malloc(4 * n), P(), P(), P(), size()
+    assert runtime.hipStreamCreateWithFlags(ref(stream), ctypes.c_uint(1)) == 0
+    assert runtime.hipStreamBeginCapture(stream, ctypes.c_int(1)) == 0
+    hip.call("zk_memcpy_d2d", P(b), P(a), size(4 * n), stream)
+    hip.call("zk_memset", P(b + 400), ctypes.c_int(0), size(800), stream)
+    hip.call("zk_upload", P(b + 2000), few, size(64), stream)
+    assert runtime.hipStreamEndCapture(stream, ref(graph)) == 0
+    assert runtime.hipGraphGetNodes(graph, None, ref(count)) == 0 and count.value == 3
+    nodes = (P * 3)()
+    assert runtime.hipGraphGetNodes(graph, nodes, ref(count)) == 0
+    for node in nodes:
+        kind = ctypes.c_int(-1)
+        assert runtime.hipGraphNodeGetType(P(node), ref(kind)) == 0 and kind.value == 0          # a kernel
+    assert runtime.hipGraphInstantiate(ref(execute), graph, None, None, size(0)) == 0
+    want = data.copy()
+    want[100:300] = 0
+    want[500:516] = few
+    for i in range(4):
+        hip.call("zk_memset", P(b), ctypes.c_int(255), size(4 * n), None)
+        hip.sync()
+        assert runtime.hipGraphLaunch(execute, stream) == 0
+        hip.call("zk_sync", stream)
+        assert (hip.download(b, n, np.uint32) == want).all(), i
+    assert runtime.hipGraphExecDestroy(execute) == 0 and runtime.hipGraphDestroy(graph) == 0 and runtime.hipStreamDestroy(stream) == 0
+    hip.free(a)
+    hip.free(b)
+
+
 def test_scratch_blocks_reused_on_another_stream_wait_for_their_last_user(hip):
     """Two matrix products of one shape on two streams back to back: the second call gets the scratch blocks that the first
     call has just given back while its kernels are still queued, and must not overwrite them early."""
