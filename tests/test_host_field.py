@@ -71,6 +71,24 @@ def test_29_bit_limb_products_match_bigint():
     assert fr_ints(got) == [v % R_MOD for v in signed]
 
 
+def test_barrett_product_matches_bigint():
+    """fr_mul_barrett (the elementwise product of two tensors), run on the CPU, against big integers: edge operands, products just
+    below, at and above multiples of r (where the quotient's estimate is one short), random ones, and any 256-bit integers."""
+    lib = _lib()
+    rng = random.Random(30)
+    edge = [0, 1, 2, R_MOD - 1, R_MOD - 2, (1 << 29) - 1, 1 << 29, (1 << 232) - 1, 1 << 232, 1 << 254, R_MOD, R_MOD + 1, (1 << 256) - 1, (1 << 256) - (1 << 232), 2 * R_MOD - 1]
+    pairs = [(x, y) for x in edge for y in edge]
+    for _ in range(2000):
+        x = rng.randrange(1, R_MOD)
+        i = pow(x, -1, R_MOD)
+        pairs += [(x, i), (x, R_MOD - i), (x, 2 * i % R_MOD), (x, rng.randrange(R_MOD)), (rng.randrange(1 << 256), rng.randrange(1 << 256))]
+    A, B = (np.array([[(v >> (32 * k)) & 0xFFFFFFFF for k in range(8)] for v in col], dtype=np.uint32) for col in zip(*pairs))
+    got, K = np.zeros_like(A), np.zeros(len(pairs), np.uint64)
+    lib.zkp_host_fr29_op.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_long]
+    assert lib.zkp_host_fr29_op(3, _np_ptr(A), _np_ptr(B), K.ctypes.data, _np_ptr(got), len(pairs)) == 0
+    assert fr_ints(got) == [x * y % R_MOD for x, y in pairs]
+
+
 def test_unreduced_sums_of_products_reduce_to_the_sum_of_montgomery_products():
     """wide_mac / wide_redc (the sumcheck rounds' accumulator: products added as 512-bit integers, one reduction at the end)
     against big integers: sum a_i b_i / R mod r for operands below r, for arbitrary 256-bit operands (the accumulator does

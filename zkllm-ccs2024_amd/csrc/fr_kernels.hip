@@ -31,7 +31,7 @@ template <int OP> __global__ void __launch_bounds__(TPB) k_ew(Fr* __restrict__ o
     Fr r;
     if (OP == EW_ADD) r = add(x, y);
     else if (OP == EW_SUB) r = sub(x, y);
-    else if (OP == EW_MUL) r = fr_mul_std(x, y);
+    else if (OP == EW_MUL) r = fr_mul_barrett(x, y);
     else r = mont_mul(x, y);
     out[i] = r;
 }

@@ -105,6 +105,7 @@ int zkp_host_fr29_op(int op, const u32* a, const u32* b, const unsigned long lon
             case 0: r = zk::fr29_mul(zk::fr29_repack(x), zk::fr29_repack(y)); break;
             case 1: r = zk::fr29_mul_small(zk::fr29_repack(x), (u32)(k[i] & zk::R29M), (u32)(k[i] >> 29)); break;
             case 2: r = zk::fr29_from_small((long long)k[i]); break;
+            case 3: r = zk::fr29_repack(zk::fr_mul_barrett(x, y)); break;
             default: throw std::runtime_error("bad op");
         }
         const zk::Fr c = zk::fr29_canon_pack(r);
