@@ -8,7 +8,7 @@ import subprocess
 import numpy as np
 
 from gpuhelp import _np_ptr, pkg
-from zkhelp import FP_R, FR_R, P_MOD, R_MOD, ROOT, fp_array, fp_ints, fr_array, fr_ints, load_oracle, orc_check
+from zkhelp import FP_R, FR_R, G1_X, G1_Y, P_MOD, R_MOD, ROOT, affine_to_jac, ec_add, ec_mul, fp_array, fp_ints, jac_to_affine, fr_array, fr_ints, load_oracle, orc_check
 
 import ctypes
 
@@ -159,3 +159,32 @@ def test_the_two_streams_of_an_opening_are_two_apart(tmp_path):
             assert (b - a) % count == 2
     for count in (4, 8):
         assert {x for c, a, b in pairs if c == count for x in (a, b)} == set(range(count))
+
+
+def test_complete_projective_additions_match_the_affine_group_law():
+    """p29_add (the bucket reductions' addition: no special cases), run on the CPU, against the affine group law: random points, a point and
+    itself, its opposite, infinity on either side and both, and points outside the subgroup of order r, those of order three among them."""
+    lib = _lib()
+    G = (G1_X, G1_Y)
+    neg = lambda p: p and (p[0], (-p[1]) % P_MOD)
+    pts = [ec_mul(k, G) for k in (1, 2, 3, 12345, R_MOD - 1, R_MOD // 2)]
+    rng = random.Random(31)
+    while len(pts) < 10:                               # any points of the curve
+        x = rng.randrange(P_MOD)
+        y = pow(x ** 3 + 4, (P_MOD + 1) // 4, P_MOD)
+        if y * y % P_MOD == (x ** 3 + 4) % P_MOD:
+            pts.append((x, y))
+    pts += [(0, 2), (0, P_MOD - 2), None] + [neg(p) for p in pts[:4]]
+    pairs = [(p, q) for p in pts for q in pts]
+
+    def scaled(p):                                      # a Jacobian form with another z
+        if p is None:
+            return affine_to_jac(None)
+        z = rng.randrange(1, P_MOD)
+        return np.concatenate([fp_array([v * FP_R % P_MOD])[0] for v in (p[0] * z * z, p[1] * z ** 3, z)])
+    A = np.ascontiguousarray(np.stack([scaled(p) for p, _ in pairs]), dtype=np.uint32)
+    B = np.ascontiguousarray(np.stack([scaled(q) for _, q in pairs]), dtype=np.uint32)
+    for op in (0, 1):
+        got = np.zeros_like(A)
+        assert lib.zkp_host_p29_add(ctypes.c_int(op), _np_ptr(A), _np_ptr(B), _np_ptr(got), ctypes.c_long(len(pairs))) == 0
+        assert [jac_to_affine(g) for g in got] == [ec_add(p, q) for p, q in pairs]

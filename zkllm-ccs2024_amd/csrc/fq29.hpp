@@ -479,56 +479,118 @@ ZK_HD void j29_add_mixed_walk(J29& a, const A29& b) {
     if (a.inf) { r.x = b.x; r.y = b.y; r.z = fq29_one(); }
     a = r;
 }
+// ---- homogeneous projective points ----------------------------------------------------------------------------------------------
+// (X / Z, Y / Z), infinity (0 : y : 0).  The complete formulas of Renes, Costello and Batina (2016, algorithms 7 and 9, a = 0, b = 4) hold for
+// every pair of points of a curve without a point of order two, which this one is: its group has odd order.  So there are no cases, and
+// nothing to keep beside the coordinates.  An addition takes six products and three reductions over two products each, 4116 limb products
+// against 5817 of the Jacobian one, and is three products deep where that is five; a doubling is two deep instead of three.
+struct P29 { Fq29 x, y, z; };
+ZK_HD P29 p29_infinity() { P29 r; r.x = r.z = fq29_zero(); r.y = fq29_one(); return r; }
+ZK_HD P29 p29_from_x29(const X29& p) {
+    P29 r;
+    r.x = fq29_mul(p.x, p.zzz);
+    r.y = fq29_mul(p.y, p.zz);
+    r.z = fq29_mul(p.zz, p.zzz);
+    if (p.inf) r = p29_infinity();
+    return r;
+}
+ZK_HD P29 p29_from_j29(const J29& p) {
+    P29 r;
+    r.x = fq29_mul(p.x, p.z);
+    r.y = p.y;
+    r.z = fq29_mul(fq29_sqr(p.z), p.z);
+    if (p.inf) r = p29_infinity();
+    return r;
+}
+ZK_HD G1Jac p29_to_jac(const P29& p) {
+    if (fq29_is_zero_mod_p(p.z)) return g1_infinity();
+    G1Jac r;
+    r.x = fq29_to_fp(fq29_mul(p.x, p.z));
+    r.y = fq29_to_fp(fq29_mul(p.y, fq29_sqr(p.z)));
+    r.z = fq29_to_fp(p.z);
+    return r;
+}
+// ka a + kb b for small factors, in one carry pass
+ZK_HD Fq29 fq29_lin(const Fq29& a, int32_t ka, const Fq29& b, int32_t kb) {
+    Fq29 r;
+    int64_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) {
+        c += (int64_t)a.l[i] * ka + (int64_t)b.l[i] * kb;
+        r.l[i] = (int32_t)((uint32_t)c & M29);
+        c >>= 29;
+    }
+    r.l[13] = a.l[13] * ka + b.l[13] * kb + (int32_t)c;
+    return r;
+}
+// a - b - c in one carry pass
+ZK_HD Fq29 fq29_sub_both(const Fq29& a, const Fq29& b, const Fq29& c) {
+    Fq29 r;
+    int32_t k = 0;
+#pragma unroll
+    for (int i = 0; i < 13; ++i) {
+        const int32_t s = a.l[i] - b.l[i] - c.l[i] + k;
+        r.l[i] = (int32_t)((uint32_t)s & M29);
+        k = s >> 29;
+    }
+    r.l[13] = a.l[13] - b.l[13] - c.l[13] + k;
+    return r;
+}
+// a + b on one lane.  INL: everything inlined, for kernels that do little else; otherwise products by calls
+template <bool INL> ZK_HD P29 p29_add(const P29& a, const P29& b) {
+    auto mul = [](const Fq29& x, const Fq29& y) { if constexpr (INL) return fq29_mul_inline(x, y); else return fq29_mul(x, y); };
+    auto mul_sub = [](const Fq29& x, const Fq29& y, const Fq29& z, const Fq29& w) { if constexpr (INL) return fq29_mul_sub(x, y, z, w); else return fq29_sub(fq29_mul(x, y), fq29_mul(z, w)); };
+    const Fq29 t0 = mul(a.x, b.x), t1 = mul(a.y, b.y), t2 = mul(a.z, b.z);
+    const Fq29 xy = fq29_sub_both(mul(fq29_add(a.x, a.y), fq29_add(b.x, b.y)), t0, t1);
+    const Fq29 yz = fq29_sub_both(mul(fq29_add(a.y, a.z), fq29_add(b.y, b.z)), t1, t2);
+    const Fq29 xz = fq29_sub_both(mul(fq29_add(a.x, a.z), fq29_add(b.x, b.z)), t0, t2);
+    const Fq29 u = fq29_lin(t1, 1, t2, 12), v = fq29_lin(t1, 1, t2, -12), w = fq29_lin(t0, -3, t0, 0), g = fq29_lin(xz, 12, xz, 0);
+    P29 r;
+    r.x = mul_sub(xy, v, yz, g);
+    r.y = mul_sub(u, v, w, g);
+    r.z = mul_sub(yz, u, w, xy);
+    return r;
+}
 #if defined(__HIPCC__)
 // ---- one point on four lanes -------------------------------------------------------------------------------------------------
 // Every lane of four holds the whole point; the independent products of a formula's step go one to a lane and come back by quad
-// permutations.  A doubling is three products deep instead of seven, an addition five instead of sixteen: for chains that a launch
-// waits for while the chip is empty.
-template <int FROM> __device__ __forceinline__ Fq29 quad_get(const Fq29& a) {
+// permutations: two products one after the other for a doubling, three for an addition.  For chains that a launch waits for while the
+// chip is empty: a wave alone issues one instruction every six to seven cycles, so the instructions of one lane are what takes the time.
+template <int CTRL> __device__ __forceinline__ Fq29 quad_perm(const Fq29& a) {
     Fq29 r;
 #pragma unroll
-    for (int i = 0; i < 14; ++i) r.l[i] = __builtin_amdgcn_update_dpp(0, a.l[i], FROM * 0x55, 0xF, 0xF, false);
+    for (int i = 0; i < 14; ++i) r.l[i] = __builtin_amdgcn_update_dpp(0, a.l[i], CTRL, 0xF, 0xF, false);
     return r;
 }
+template <int FROM> __device__ __forceinline__ Fq29 quad_get(const Fq29& a) { return quad_perm<FROM * 0x55>(a); }
 __device__ __forceinline__ Fq29 fq29_select(bool c, const Fq29& a, const Fq29& b) {
     Fq29 r;
 #pragma unroll
     for (int i = 0; i < 14; ++i) r.l[i] = c ? a.l[i] : b.l[i];
     return r;
 }
-__device__ __forceinline__ void j29_quad_double(J29& p, uint32_t q) {
-    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 0, p.x, p.y), fq29_select(q == 0, p.x, fq29_select(q == 2, p.z, p.y)));      // x^2 | y^2 | y z | y^2
-    const Fq29 a = quad_get<0>(m1), b = quad_get<1>(m1), yz = quad_get<2>(m1);
-    const Fq29 e = fq29_add(fq29_shl<1>(a), a);
-    const Fq29 m2 = fq29_mul_inline(fq29_select(q == 0, e, fq29_select(q == 1, p.x, b)), fq29_select(q == 0, e, b));                // e^2 | x y^2 | y^4 | y^4
-    const Fq29 s = quad_get<1>(m2), c = quad_get<2>(m2);
-    p.x = fq29_sub8(quad_get<0>(m2), s);
-    p.y = fq29_sub8(fq29_mul_inline(e, fq29_sub_raw(fq29_shl<2>(s), p.x)), c);
-    p.z = fq29_shl<1>(yz);
+// with A = y^2, B = z^2: x3 = 2 xy (A - 36 B), y3 = (A + 12 B)(A - 36 B) + 96 A B, z3 = 8 A yz
+__device__ __forceinline__ void p29_quad_double(P29& p, uint32_t q) {
+    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 1, p.z, fq29_select(q == 2, p.x, p.y)), fq29_select((q & 1u) != 0, p.z, p.y));      // A | B | x y | y z
+    const Fq29 a = quad_get<0>(m1), b = quad_get<1>(m1), own = quad_perm<0xD2>(m1);                                                       // own: x y | A | B | y z
+    const int32_t k = q == 0 ? 2 : (q == 1 ? 1 : (q == 2 ? 96 : 8)), kb = q == 1 ? 12 : 0, kr = q < 2 ? -36 : 0;
+    const Fq29 m2 = fq29_mul_inline(fq29_lin(own, k, b, kb), fq29_lin(a, 1, b, kr));
+    p.x = quad_get<0>(m2);
+    p.y = fq29_add(quad_get<1>(m2), quad_get<2>(m2));
+    p.z = quad_get<3>(m2);
 }
-__device__ __forceinline__ void j29_quad_add(J29& a, const J29& b, uint32_t q) {
-    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 0, a.z, fq29_select(q == 1, b.z, fq29_select(q == 2, a.y, b.y))),
-                                    fq29_select((q & 1u) != 0, fq29_select(q == 1, b.z, a.z), fq29_select(q == 0, a.z, b.z)));      // z1^2 | z2^2 | y1 z2 | y2 z1
-    const Fq29 z1z1 = quad_get<0>(m1), z2z2 = quad_get<1>(m1);
-    const Fq29 m2 = fq29_mul_inline(fq29_select(q == 0, a.x, fq29_select(q == 1, b.x, m1)), fq29_select((q & 1u) != 0, z1z1, z2z2)); // u1 | u2 | s1 | s2
-    const Fq29 u1 = quad_get<0>(m2), s1 = quad_get<2>(m2);
-    const Fq29 h = fq29_sub_raw(quad_get<1>(m2), u1), rr = fq29_sub_raw(quad_get<3>(m2), s1);
-    const Fq29 m3 = fq29_mul_inline(fq29_select(q == 0, h, fq29_select(q == 1, a.z, rr)), fq29_select(q == 0, h, fq29_select(q == 1, b.z, rr)));      // h^2 | z1 z2 | r^2 | r^2
-    const Fq29 hh = quad_get<0>(m3), zz = quad_get<1>(m3), r2 = quad_get<2>(m3);
-    const Fq29 m4 = fq29_mul_inline(fq29_select(q == 1, u1, fq29_select(q == 2, zz, h)), fq29_select(q == 2, h, hh));                  // h^3 | u1 h^2 | z1 z2 h | h^3
-    const Fq29 hhh = quad_get<0>(m4), v = quad_get<1>(m4);
-    J29 r;
-    r.inf = 0u;
-    r.z = quad_get<2>(m4);
-    r.x = fq29_sub2(r2, hhh, v);
-    r.y = fq29_mul_sub(rr, fq29_sub_raw(v, r.x), s1, hhh);
-    if (a.inf) r = b;
-    else if (b.inf) r = a;
-    else if ((hh.l[0] == 0 || hh.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(hh)) {
-        if ((r2.l[0] == 0 || r2.l[0] == fq29_p(0)) && fq29_is_zero_mod_p(r2)) r = j29_double(a);
-        else r = j29_infinity();
-    }
-    a = r;
+__device__ __forceinline__ void p29_quad_add(P29& a, const P29& b, uint32_t q) {
+    const Fq29 m1 = fq29_mul_inline(fq29_select(q == 0, a.x, fq29_select(q == 1, a.y, fq29_select(q == 2, a.z, fq29_add(a.x, a.y)))),
+                                    fq29_select(q == 0, b.x, fq29_select(q == 1, b.y, fq29_select(q == 2, b.z, fq29_add(b.x, b.y)))));    // t0 | t1 | t2 | (x + y)(x + y)
+    const Fq29 m2 = fq29_mul_inline(fq29_add(fq29_select(q == 0, a.y, a.x), a.z), fq29_add(fq29_select(q == 0, b.y, b.x), b.z));          // (y + z)(y + z) | (x + z)(x + z) | -- | --
+    const Fq29 t0 = quad_get<0>(m1), t1 = quad_get<1>(m1), t2 = quad_get<2>(m1);
+    const Fq29 xy = fq29_sub_both(quad_get<3>(m1), t0, t1), yz = fq29_sub_both(quad_get<0>(m2), t1, t2), xz = fq29_sub_both(quad_get<1>(m2), t0, t2);
+    const Fq29 w = fq29_lin(t0, -3, t0, 0), g = fq29_lin(xz, 12, xz, 0);
+    const Fq29 m3 = fq29_mul_sub(fq29_select(q == 0, xy, fq29_select(q == 1, fq29_lin(t1, 1, t2, 12), yz)), fq29_lin(t1, 1, t2, q == 2 ? 12 : -12),
+                                 fq29_select(q == 0, yz, w), fq29_select(q == 2, xy, g));                                                 // x3 | y3 | z3 | --
+    a.x = quad_get<0>(m3);
+    a.y = quad_get<1>(m3);
+    a.z = quad_get<2>(m3);
 }
 #endif
 ZK_HD J29 j29_from_jac(const G1Jac& p) {

@@ -609,48 +609,48 @@ __global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t
     msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i]);
 }
 
-static constexpr int J29_WORDS = 43;
-static_assert(sizeof(J29) == 4 * J29_WORDS, "a point is its coordinates and its flag");
+static constexpr int P29_WORDS = 42;
+static_assert(sizeof(P29) == 4 * P29_WORDS, "a point is its coordinates");
 // The end of a list of points in bucket order that a wave's lanes have divided evenly (lane t the t-th share).  x: the sum of the last part of
 // the lane's share, which belongs to bucket b; begun: the bucket begins in this share (or the share is empty); whole: it ends with this
 // share; lacks: bucket `split`, the first part's, went out already without the shares before this one.  A segmented inclusive scan, as
-// long as a bucket spans further lanes, then the sums to `out` (added to what is there unless fresh).  All lanes call it; pool: 43 x 64 words.
-__device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, J29 x, bool begun, bool whole, uint32_t b, bool lacks, uint32_t split, J29* __restrict__ out, bool fresh, uint32_t t) {
+// long as a bucket spans further lanes, then the sums to `out` (added to what is there unless fresh).  All lanes call it; pool: 42 x 64 words.
+__device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, P29 x, bool begun, bool whole, uint32_t b, bool lacks, uint32_t split, P29* __restrict__ out, bool fresh, uint32_t t) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
     for (uint32_t sd = 1; sd < (uint32_t)MSL && !__all(begun); sd <<= 1) {
         __syncthreads();
 #pragma unroll
-        for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
+        for (int l = 0; l < P29_WORDS; ++l) pool[l * MSL + t] = src[l];
         __syncthreads();
         const bool before = __shfl_up(begun ? 1 : 0, sd) != 0;
         if (t >= sd && !begun) {
-            J29 y;
+            P29 y;
             uint32_t* py = reinterpret_cast<uint32_t*>(&y);
 #pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - sd];
-            x = j29_add(x, y);
+            for (int l = 0; l < P29_WORDS; ++l) py[l] = pool[l * MSL + t - sd];
+            x = p29_add<false>(x, y);
             begun = before;
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int l = 0; l < J29_WORDS; ++l) pool[l * MSL + t] = src[l];
+    for (int l = 0; l < P29_WORDS; ++l) pool[l * MSL + t] = src[l];
     __syncthreads();
     if (whole) {
-        if (!fresh) x = j29_add(out[b], x);
+        if (!fresh) x = p29_add<false>(out[b], x);
         out[b] = x;
     }
     if (lacks) {
-        J29 y;
+        P29 y;
         uint32_t* py = reinterpret_cast<uint32_t*>(&y);
 #pragma unroll
-        for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * MSL + t - 1];
-        out[split] = j29_add(out[split], y);
+        for (int l = 0; l < P29_WORDS; ++l) py[l] = pool[l * MSL + t - 1];
+        out[split] = p29_add<false>(out[split], y);
     }
 }
 
 // One segment's share of sum over elements of digit_w(s) * base: the segment's MT raw buckets,
-// partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold / k_msm_point reduce them).
+// partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold, k_msm_windows and k_msm_horner reduce them).
 // One wave per workgroup.  Per chunk of `chunk` elements (at most MSEG):
 //  1. the bucket sizes are counted (one LDS atomic per element) and the elements are sorted by bucket into one list in
 //     LDS (counting sort: 12-bit position in the chunk + sign);
@@ -663,11 +663,11 @@ __device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, J29 x, bool 
 //     at most two.  A bucket that ends inside a share goes out there; the rest is a segmented scan over the lanes, six additions for
 //     all of them together.  An opening of 1 x 16384 small integers: 10.7 ms with a tree of six additions a bucket above 256
 //     elements and one lane's walk below, 5.0 ms so.
-__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(J29* __restrict__ partial, const MsmDesc* __restrict__ descs, uint32_t nseg, uint32_t chunks_per_seg, uint32_t chunk) {
+__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(P29* __restrict__ partial, const MsmDesc* __restrict__ descs, uint32_t nseg, uint32_t chunks_per_seg, uint32_t chunk) {
     __shared__ uint32_t cnt[MT], off[MT], cursor[MT];
     __shared__ uint8_t order[MT], heavy[MT];
-    __shared__ uint32_t pool[J29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the points of the heavy buckets' scan
-    static_assert(J29_WORDS * MSL * 4 >= MSEG * 2, "pool too small for the list");
+    __shared__ uint32_t pool[P29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the points of the heavy buckets' scan
+    static_assert(P29_WORDS * MSL * 4 >= MSEG * 2, "pool too small for the list");
     static_assert(MSEG <= 4096, "12-bit list entries");
     static_assert(MSEG / MSL < MHEAVY, "a lane's share of the heavy buckets' list touches two of them at most");
     static_assert(MT == 2 * MSL, "a lane counts two buckets");
@@ -678,7 +678,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int8_t* __restrict__ Dw = d.digits + (size_t)w * d.dstride;
     const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
     const uint32_t half = w / (uint32_t)MWH;
-    J29* __restrict__ out = partial + (((size_t)zz * MW + w) * nseg + seg) * MT;
+    P29* __restrict__ out = partial + (((size_t)zz * MW + w) * nseg + seg) * MT;
     bool first = true;                                  // nothing written to `out` yet (the same for every lane)
     for (uint32_t ch = 0; ch < chunks_per_seg; ++ch) {
         const uint32_t e0 = (seg * chunks_per_seg + ch) * chunk;
@@ -743,8 +743,8 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             for (uint32_t i = 0;; ++i) {
                 if (i == lenA) {
                     // the end of the first list: its bucket goes out (added to what earlier chunks of this segment left there)
-                    J29 v = j29_from_x29(acc29);
-                    if (!first) v = j29_add(out[bA], v);
+                    P29 v = p29_from_x29(acc29);
+                    if (!first) v = p29_add<false>(out[bA], v);
                     out[bA] = v;
                     acc29 = x29_infinity();
                     pos = off[bB];
@@ -756,8 +756,8 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 if (en & 0x8000u) pt.y = fq29_neg(pt.y);
                 x29_add_mixed(acc29, pt);
             }
-            J29 v = j29_from_x29(acc29);
-            if (!first) v = j29_add(out[bB], v);
+            P29 v = p29_from_x29(acc29);
+            if (!first) v = p29_add<false>(out[bB], v);
             out[bB] = v;
         }
         __threadfence_block();
@@ -774,8 +774,8 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
             X29 acc29 = x29_infinity();
             for (uint32_t pos = p0; pos < p1; ++pos) {
                 if (pos == b_end) {
-                    J29 v = j29_from_x29(acc29);
-                    if (!first) v = j29_add(out[b], v);
+                    P29 v = p29_from_x29(acc29);
+                    if (!first) v = p29_add<false>(out[b], v);
                     out[b] = v;
                     split = b; lacks = !start; start = true;
                     acc29 = x29_infinity();
@@ -788,15 +788,15 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
                 x29_add_mixed(acc29, pt);
             }
             const bool whole = p1 > p0 && p1 == b_end;       // the bucket ends with this share
-            bucket_shares_merge(pool, j29_from_x29(acc29), start, whole, b, lacks, split, out, first, t);
+            bucket_shares_merge(pool, p29_from_x29(acc29), start, whole, b, lacks, split, out, first, t);
         }
         __threadfence_block();
         __syncthreads();
         first = false;
     }
     if (first) {                                       // a segment past the end of this sum: empty buckets
-        out[t] = j29_infinity();
-        out[t + MSL] = j29_infinity();
+        out[t] = p29_infinity();
+        out[t + MSL] = p29_infinity();
     }
 }
 // The same for sums of few elements: the 8-bit digits taken as two signed 4-bit digits each, so that a sum has 512 buckets (64 windows
@@ -805,20 +805,20 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
 // nw (1, 2, 4 or 8) gives a lane about eight elements, so that the scan behind them costs less than they do.
 // FEW_MAX: an element costs 64 additions here and 32 there, a sum 32 walks here and 256 there; at 512 elements an opening alone takes the
 // same time both ways (1.87 ms), and of a layer of small products, whose 250 sums then leave the chip to the rest, 7.2 ms instead of 7.7.
-static constexpr int FEW_MAX = 512, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T, FEW_GROUP = MT / (4 * FEW_T);     // FEW_GROUP: the sums that k_msm_point takes in a workgroup
+static constexpr int FEW_MAX = 512, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T;
 // grid (64 / nw, sums); buckets[(sum * 64 + window) * 8 + magnitude - 1]
-__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_few(J29* __restrict__ buckets, const MsmDesc* __restrict__ descs, uint32_t nw) {
+__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_few(P29* __restrict__ buckets, const MsmDesc* __restrict__ descs, uint32_t nw) {
     __shared__ uint32_t cnt[MSL], off[MSL], cursor[MSL];
-    __shared__ uint32_t pool[J29_WORDS * MSL];      // the sorted list (u16), then the points of the shares' scan
-    static_assert(FEW_MAX <= 4096 && FEW_MAX * 2 <= J29_WORDS * MSL * 4 && 8 * FEW_T == MSL, "list entries, the pool and a lane for each bucket");
+    __shared__ uint32_t pool[P29_WORDS * MSL];      // the sorted list (u16), then the points of the shares' scan
+    static_assert(FEW_MAX <= 4096 && FEW_MAX * 2 <= P29_WORDS * MSL * 4 && 8 * FEW_T == MSL, "list entries, the pool and a lane for each bucket");
     uint16_t* list = reinterpret_cast<uint16_t*>(pool);
     const MsmDesc d = descs[blockIdx.y];
     const A29* __restrict__ A = d.base;
     const uint32_t t = threadIdx.x, v0 = blockIdx.x * nw, half = v0 / (FEW_WINDOWS / 2);
     const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
-    J29* __restrict__ out = buckets + ((size_t)blockIdx.y * FEW_WINDOWS + v0) * FEW_T;
+    P29* __restrict__ out = buckets + ((size_t)blockIdx.y * FEW_WINDOWS + v0) * FEW_T;
     cnt[t] = 0;
-    if (t < nw * FEW_T) out[t] = j29_infinity();
+    if (t < nw * FEW_T) out[t] = p29_infinity();
     __syncthreads();
     auto digit = [&](uint32_t v, size_t si) {
         const int dg = d.digits[(size_t)(v >> 1) * d.dstride + si], hi = (dg + 8) >> 4;
@@ -858,7 +858,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
     X29 acc29 = x29_infinity();
     for (uint32_t pos = p0; pos < p1; ++pos) {
         if (pos == b_end) {
-            out[b] = j29_from_x29(acc29);
+            out[b] = p29_from_x29(acc29);
             if (!start) { split = b; lacks = true; start = true; }
             acc29 = x29_infinity();
             do ++b; while (cnt[b] == 0);
@@ -870,93 +870,111 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (en & 0x8000u) pt.y = fq29_neg(pt.y);
         x29_add_mixed(acc29, pt);
     }
-    bucket_shares_merge(pool, j29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
+    bucket_shares_merge(pool, p29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
 }
 // raw buckets of up to 8 consecutive segments summed: out[(row * gridDim.y + group) * MT + t], row = sum * MW + w
-__global__ void __launch_bounds__(MT) k_msm_bucket_fold(J29* __restrict__ out, const J29* __restrict__ buckets, uint32_t nseg) {
+__global__ void __launch_bounds__(MT) k_msm_bucket_fold(P29* __restrict__ out, const P29* __restrict__ buckets, uint32_t nseg) {
     const uint32_t t = threadIdx.x, row = blockIdx.x, grp = blockIdx.y;
     const uint32_t s0 = grp * 8, s1 = (s0 + 8 < nseg) ? s0 + 8 : nseg;
-    const J29* b = buckets + (size_t)row * nseg * MT;
-    J29 acc = b[(size_t)s0 * MT + t];
-    for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = j29_add(acc, b[(size_t)sg * MT + t]);
+    const P29* b = buckets + (size_t)row * nseg * MT;
+    P29 acc = b[(size_t)s0 * MT + t];
+    for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = p29_add<true>(acc, b[(size_t)sg * MT + t]);
     out[((size_t)row * gridDim.y + grp) * MT + t] = acc;
 }
-// The sums of a list from the raw buckets of all their windows, 128 walks for each half of a sum's windows: four lanes take bucket
-// b + 1, sum_w 2^(8w) B[w] (one Horner walk of 120 doublings), weight it by its digit, and the buckets are summed -- one weighting and
-// one lane sum per half instead of one per window, and no Horner pass of a single lane over window sums afterwards.  A sum of few
-// elements has two sets of 8 buckets a window, weighted 1 .. 8 and 16 .. 128: 16 walks a half.  k_msm_join adds the halves, the
-// endomorphism on the second.
-// Raw buckets: buckets[w MT + b] (k_msm_few's: [w 16 + b]); a half's total goes to its first bucket's place, which only its own walks read.
-// A launch takes what one workgroup takes whatever the number of sums: all of a job's sums that nothing waits for
-// go into one launch, those of few elements behind the others (first_few), four to a workgroup.  A lane's chain takes 1.5 ms; four lanes
-// that share a point's products take 1.2 ms (eight waves a workgroup, two a SIMD, 339 k instructions each: a SIMD's whole issue rate, on
-// one compute unit), and a compute unit holds one such workgroup: LANES is four while all of a launch's fit
-// beside each other and beside what else runs, one for longer lists (310 workgroups of four took 2.6 ms).  192 workgroups: an opening of
-// 2^17 generators (18 and 86 workgroups) takes 11.9 ms on four lanes and 13.1 on one, one of 16384 5.1 and 5.3; a layer of small products
-// 6.9 to 7.1 ms with the line at 96 or 192, 7.4 on one lane or on four throughout, and the layer of 2048 x 2048 54.6, 54.8 and 55.4.
-struct PointDesc { J29* buckets; G1Jac* out; uint32_t half_off, few; };     // half_off: where the second half's buckets begin
-template <int LANES> __device__ __forceinline__ void walk_double(J29& p, uint32_t q) {
-    if constexpr (LANES == 4) j29_quad_double(p, q);
-    else j29_double_walk(p);
-}
-template <int LANES> __device__ __forceinline__ void walk_add(J29& a, const J29& b, uint32_t q) {
-    if constexpr (LANES == 4) j29_quad_add(a, b, q);
-    else a = j29_add(a, b);
-}
-template <int LANES> __global__ void __launch_bounds__(LANES * MT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_point(const PointDesc* __restrict__ list, uint32_t first_few, uint32_t n) {
-    __shared__ uint32_t pool[J29_WORDS * MT / 2];
-    const uint32_t q = threadIdx.x % LANES, walk = threadIdx.x / LANES;
-    const bool few = blockIdx.x >= 2 * first_few;           // the same for the workgroup
-    const uint32_t width = few ? 2 * FEW_T : MT, group = walk / width, b = walk % width;
-    const uint32_t sum = few ? first_few + (blockIdx.x - 2 * first_few) * FEW_GROUP + group / 2 : blockIdx.x >> 1;
-    const uint32_t half = few ? group & 1u : blockIdx.x & 1u;
-    const uint32_t weight = few && b >= FEW_T ? (b - FEW_T + 1) * 16 : b + 1;
-    const bool live = sum < n;
-    J29* mine = nullptr;
-    if (live) { const PointDesc d = list[sum]; mine = d.buckets + half * d.half_off; }
-    J29 r = j29_infinity();
-    for (uint32_t w = MWH; w-- > 0;) {
-        J29 p = j29_infinity();
-        if (LANES == 4 && live) p = mine[w * width + b];    // on its way during the doublings (a single lane has no registers left for it)
-        if (__any(!r.inf))
-            for (int k = 0; k < 8; ++k) walk_double<LANES>(r, q);
-        if (LANES == 1 && live) p = mine[w * width + b];
-        if (__any(!p.inf)) walk_add<LANES>(r, p, q);
-    }
-    J29 s = r;
-    if (!(weight & 128u)) s.inf = 1u;
-    for (int bit = 6; bit >= 0; --bit) {
-        walk_double<LANES>(s, q);
-        J29 p = r;
-        if (!((weight >> bit) & 1u)) p.inf = 1u;
-        walk_add<LANES>(s, p, q);
-    }
-    for (uint32_t sd = width / 2; sd > 0; sd >>= 1) {
-        __syncthreads();
-        if (b >= sd && b < 2 * sd && q == 0) {
-            const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
+// The sums of a list from the raw buckets of all their windows, in two launches.  k_msm_windows: a wave takes a window, sum_b (b + 1) B[b]:
+// each four lanes the running sums over eight neighbouring buckets (fourteen additions), then a tree over the sixteen of them in which one
+// of four lanes carries the weighted sum and one the plain sum times the buckets below it (eight additions).  A sum of few elements has two sets of 8
+// buckets a window, weighted 1 .. 8 and 16 .. 128: a wave takes eight of its windows.  k_msm_horner: four lanes walk the sixteen windows of a
+// half, 120 doublings, and the halves are added, the endomorphism on the second.
+// All of a job's sums that nothing waits for go into one launch each, those of few elements behind the others (first_few).  Both are chains of one wave's
+// instructions; the windows are summed before the walk so that 32 waves and two walks of four lanes do what took 256 walks a sum.
+struct PointDesc { P29* buckets; G1Jac* out; uint32_t few, pad; };
+__device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
+    P29 r;
+    const int32_t* src = reinterpret_cast<const int32_t*>(&a);
+    int32_t* dst = reinterpret_cast<int32_t*>(&r);
 #pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) pool[l * (MT / 2) + group * sd + b - sd] = src[l];
+    for (int l = 0; l < P29_WORDS; ++l) dst[l] = __shfl(src[l], lane, 64);
+    return r;
+}
+// win[sum * MW + w]: the windows' sums.  grid: MW workgroups a sum, then MW / 8 a sum of few elements
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_windows(P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t first_few) {
+    __shared__ int32_t pool[3][16][44];                     // of each four lanes: S, V, T below
+    const uint32_t q = threadIdx.x & 3u, g = threadIdx.x >> 2;
+    const bool few = blockIdx.x >= MW * first_few;          // the same for the workgroup
+    const uint32_t at = few ? blockIdx.x - MW * first_few : blockIdx.x, per = few ? MW / 8 : MW;
+    const uint32_t sum = (few ? first_few : 0u) + at / per, w = few ? at % per * 8 + g / 2 : at % per;
+    const P29* __restrict__ B = list[sum].buckets + (few ? w * (2 * FEW_T) + (g & 1u) * FEW_T : w * MT + g * 8);
+    enum : uint32_t { S = 0, V = 1, T = 2 };                // the running sum, the sum of the running sums, half a step of the tree
+    auto get = [&](uint32_t slot, uint32_t of) {
+        P29 r;
+        int32_t* dst = reinterpret_cast<int32_t*>(&r);
+#pragma unroll
+        for (int l = 0; l < P29_WORDS; ++l) dst[l] = pool[slot][of & 15u][l];
+        return r;
+    };
+    auto put = [&](uint32_t slot, const P29& v) {
+        const int32_t* src = reinterpret_cast<const int32_t*>(&v);
+        if (q == 0) {
+#pragma unroll
+            for (int l = 0; l < P29_WORDS; ++l) pool[slot][g][l] = src[l];
+        }
+    };
+    {
+        const P29 top = B[7];
+        put(S, top);
+        put(V, top);
+    }
+    P29 nxt = B[6];
+    const uint32_t steps = few ? 19 : 25;
+    for (uint32_t step = 0; step < steps; ++step) {         // one addition, whatever it is for, so that its instructions are there once
+        uint32_t xs, ys, yg = g, to;
+        const bool odd = (g & 1u) != 0;
+        bool bucket = false;
+        if (step < 14) {
+            bucket = !(step & 1u);
+            xs = (step & 1u) ? V : S; ys = S; to = xs;
+        } else if (step < (few ? 18u : 17u)) {              // eight times the plain sum; of few elements sixteen times the weighted one
+            xs = ys = few && step == 14 ? V : S; to = S;
+        } else if (few) {                                   // the upper set's to the lower's
+            xs = V; ys = S; yg = g ^ 1u; to = V;
+        } else {                                            // level k of the tree: the left half's first four lanes carry the weighted sum, its second the plain one
+            const uint32_t k = (step - 17) >> 1;
+            if (step & 1u) {
+                xs = ys = k == 0 && odd ? S : V; yg = k == 0 ? g ^ 1u : g + (1u << k); to = T;
+            } else {                                        // and the right half's plain sum to the weighted; the plain sum doubled
+                xs = T; ys = odd ? T : (k == 0 ? S : V); yg = odd ? g : (k == 0 ? g ^ 1u : g + (1u << k) + 1u); to = V;
+            }
         }
         __syncthreads();
-        if (b < sd) {
-            J29 y;
-            uint32_t* py = reinterpret_cast<uint32_t*>(&y);
-#pragma unroll
-            for (int l = 0; l < J29_WORDS; ++l) py[l] = pool[l * (MT / 2) + group * sd + b];
-            walk_add<LANES>(s, y, q);
+        P29 x = get(xs, g), y;
+        if (bucket) y = nxt;
+        else {
+            y = get(ys, yg);
+            if (step < 13) nxt = B[5 - (step >> 1)];
         }
+        p29_quad_add(x, y, q);
+        put(to, x);
+        if (step + 1 == steps && q == 0 && (few ? !odd : g == 0)) win[(size_t)sum * MW + w] = x;
     }
-    if (live && b == 0 && q == 0) *mine = s;
 }
-__global__ void __launch_bounds__(GT) k_msm_join(const PointDesc* __restrict__ list, uint32_t n) {
-    const uint32_t i = (blockIdx.x * GT + threadIdx.x) >> 2, q = threadIdx.x & 3u;
-    if (i >= n) return;
-    const PointDesc d = list[i];
-    J29 s = d.buckets[0], y = d.buckets[d.half_off];
-    y.x = fq29_mul(y.x, fq29_from_fp(glv_beta()));
-    j29_quad_add(s, y, q);
-    if (q == 0) *d.out = j29_to_jac(s);
+// grid: eight sums a wave
+__global__ void __launch_bounds__(GT) k_msm_horner(const P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t n) {
+    const uint32_t q = threadIdx.x & 3u, sum = (blockIdx.x * GT + threadIdx.x) >> 3, half = (threadIdx.x >> 2) & 1u;
+    const P29* __restrict__ W = win + (size_t)(sum < n ? sum : n - 1) * MW + half * MWH;
+    P29 r = W[MWH - 1];
+    for (int w = MWH - 2; w >= -1; --w) {
+        P29 p;
+        if (w >= 0) {
+            p = W[w];                                       // on its way during the doublings
+            for (int k = 0; k < 8; ++k) p29_quad_double(r, q);
+        } else {                                            // the halves: [lambda] of the second
+            if (half) r.x = fq29_mul(r.x, fq29_from_fp(glv_beta()));
+            p = p29_shfl(r, (int)(threadIdx.x ^ 4u));
+        }
+        p29_quad_add(r, p, q);
+    }
+    if (sum < n && half == 0 && q == 0) *list[sum].out = p29_to_jac(r);
 }
 
 // Sums of an opening's first rounds from commitments of the opened tensor's rows.  The opened vector is the row fold of a
@@ -1069,6 +1087,17 @@ __device__ __forceinline__ A29 a29_from_j29(const J29& w) {
         const Fq29 zi2 = fq29_sqr(zi);
         o.x = fq29_canon(fq29_mul(w.x, zi2));
         o.y = fq29_canon(fq29_mul(fq29_mul(w.y, zi2), zi));
+    }
+    return o;
+}
+__device__ __forceinline__ A29 a29_from_p29(const P29& w) {
+    A29 o;
+    o.x = o.y = fq29_zero();
+    const bool inf = fq29_is_zero_mod_p(w.z);
+    const Fq29 zi = fq29_inverse(inf ? fq29_one() : w.z);
+    if (!inf) {
+        o.x = fq29_canon(fq29_mul(w.x, zi));
+        o.y = fq29_canon(fq29_mul(w.y, zi));
     }
     return o;
 }
@@ -1310,7 +1339,7 @@ k_open_fold_jump(const JumpBatch jb, size_t new_size) {
 // a walk of `slice` doublings, every digit the same for the wave.  k_open_span_walk: four lanes a result put the slices together, seven
 // times `slice` doublings.  An eighth of the doublings that eight walks beside each other take, and the second launch, whose chain
 // hardly fills the chip, leaves it to the bucket sums.
-struct SpanBatch { A29* ng[OB_MAX]; const A29* g[OB_MAX]; J29* part; };
+struct SpanBatch { A29* ng[OB_MAX]; const A29* g[OB_MAX]; P29* part; };
 __global__ void __launch_bounds__(8 * GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_open_span_slices(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old_size, size_t new_size, uint32_t slice) {
     __shared__ int32_t tab[8][5][14][GT];      // x, y of P, x of phi(P), x and y of P - phi(P)
@@ -1368,28 +1397,29 @@ k_open_span_slices(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old
         }
     }
     if (m < new_size) {
-        int32_t* out = reinterpret_cast<int32_t*>(sb.part) + ((size_t)blockIdx.y * 8 + b) * J29_WORDS * new_size + m;
-        const int32_t* src = reinterpret_cast<const int32_t*>(&w);
+        int32_t* out = reinterpret_cast<int32_t*>(sb.part) + ((size_t)blockIdx.y * 8 + b) * P29_WORDS * new_size + m;
+        const P29 v = p29_from_j29(w);
+        const int32_t* src = reinterpret_cast<const int32_t*>(&v);
 #pragma unroll
-        for (int l = 0; l < J29_WORDS; ++l) out[(size_t)l * new_size] = src[l];
+        for (int l = 0; l < P29_WORDS; ++l) out[(size_t)l * new_size] = src[l];
     }
 }
 __global__ void __launch_bounds__(GT) k_open_span_walk(const SpanBatch sb, size_t new_size, uint32_t slice) {
     const size_t m = ((size_t)blockIdx.x * GT + threadIdx.x) >> 2;
     const uint32_t q = threadIdx.x & 3u;
     if (m >= new_size) return;
-    const int32_t* part = reinterpret_cast<const int32_t*>(sb.part) + (size_t)blockIdx.y * 8 * J29_WORDS * new_size + m;
-    J29 w = j29_infinity();
+    const int32_t* part = reinterpret_cast<const int32_t*>(sb.part) + (size_t)blockIdx.y * 8 * P29_WORDS * new_size + m;
+    P29 w = p29_infinity();
     for (int b = 7; b >= 0; --b) {
-        if (__any(!w.inf))
-            for (uint32_t i = 0; i < slice; ++i) j29_quad_double(w, q);
-        J29 s;
+        if (b != 7)
+            for (uint32_t i = 0; i < slice; ++i) p29_quad_double(w, q);
+        P29 s;
         int32_t* dst = reinterpret_cast<int32_t*>(&s);
 #pragma unroll
-        for (int l = 0; l < J29_WORDS; ++l) dst[l] = part[((size_t)b * J29_WORDS + l) * new_size];
-        j29_quad_add(w, s, q);
+        for (int l = 0; l < P29_WORDS; ++l) dst[l] = part[((size_t)b * P29_WORDS + l) * new_size];
+        p29_quad_add(w, s, q);
     }
-    const A29 o = a29_from_j29(w);
+    const A29 o = a29_from_p29(w);
     if (q == 0) sb.ng[blockIdx.y][m] = o;
 }
 // the pairs k_open_fold29 left out, by the general Jacobian route in 32-bit limbs (one lane per pair, an inversion each)
@@ -1781,11 +1811,11 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
         const void* dd = nullptr;
         int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
         if (rc) return rc;
-        Scratch& buckets = arena.add(sizeof(J29) * (size_t)n_msm * FEW_BUCKETS);
+        Scratch& buckets = arena.add(sizeof(P29) * (size_t)n_msm * FEW_BUCKETS);
         if (buckets.rc) return buckets.rc;
-        hipLaunchKernelGGL(k_msm_few, dim3(FEW_WINDOWS / nw, n_msm), dim3(MSL), 0, st, buckets.as<J29>(), (const MsmDesc*)dd, nw);
+        hipLaunchKernelGGL(k_msm_few, dim3(FEW_WINDOWS / nw, n_msm), dim3(MSL), 0, st, buckets.as<P29>(), (const MsmDesc*)dd, nw);
         ZK_LAUNCH_CHECK();
-        for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<J29>() + (size_t)z * FEW_BUCKETS, out[z], FEW_BUCKETS / 2, 1u});
+        for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<P29>() + (size_t)z * FEW_BUCKETS, out[z], 1u, 0u});
         return 0;
     }
     // One chunk per workgroup, and chunks short enough for two workgroups a SIMD where there are few elements: a workgroup's time is its
@@ -1798,35 +1828,35 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
     const void* dd = nullptr;
     int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
     if (rc) return rc;
-    Scratch& partial = arena.add(sizeof(J29) * n_msm * MW * (size_t)ns * MT);
+    Scratch& partial = arena.add(sizeof(P29) * n_msm * MW * (size_t)ns * MT);
     if (partial.rc) return partial.rc;
-    hipLaunchKernelGGL(k_msm_seg, dim3(ns, MW, n_msm), dim3(MSL), 0, st, partial.as<J29>(), (const MsmDesc*)dd, ns, cps, chunk);
+    hipLaunchKernelGGL(k_msm_seg, dim3(ns, MW, n_msm), dim3(MSL), 0, st, partial.as<P29>(), (const MsmDesc*)dd, ns, cps, chunk);
     // the segments' raw buckets summed eight at a time (a lane per bucket and window: the reduction, one workgroup per sum, then
     // walks single buckets)
-    J29* cur = partial.as<J29>();
+    P29* cur = partial.as<P29>();
     while (ns > 1) {
         const uint32_t ng = (ns + 7) / 8;
-        Scratch& nxt = arena.add(sizeof(J29) * n_msm * MW * (size_t)ng * MT);
+        Scratch& nxt = arena.add(sizeof(P29) * n_msm * MW * (size_t)ng * MT);
         if (nxt.rc) return nxt.rc;
-        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, st, nxt.as<J29>(), cur, ns);
-        cur = nxt.as<J29>();
+        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, st, nxt.as<P29>(), cur, ns);
+        cur = nxt.as<P29>();
         ns = ng;
     }
     ZK_LAUNCH_CHECK();
-    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], MWH * MT, 0u});
+    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], 0u, 0u});
     return 0;
 }
-static int points_queue(std::vector<PointDesc>& list, JobUploads& up, hipStream_t st) {
+static int points_queue(std::vector<PointDesc>& list, Arena& arena, JobUploads& up, hipStream_t st) {
     if (list.empty()) return 0;
     const uint32_t n = (uint32_t)list.size();
     const uint32_t first_few = (uint32_t)(std::stable_partition(list.begin(), list.end(), [](const PointDesc& d) { return d.few == 0; }) - list.begin());
     const void* dl = nullptr;
     int rc = up.put(list.data(), sizeof(PointDesc) * n, st, &dl);
     if (rc) return rc;
-    const unsigned groups = 2 * first_few + cdiv(n - first_few, FEW_GROUP);
-    if (groups <= 192) hipLaunchKernelGGL(k_msm_point<4>, dim3(groups), dim3(4 * MT), 0, st, (const PointDesc*)dl, first_few, n);
-    else hipLaunchKernelGGL(k_msm_point<1>, dim3(groups), dim3(MT), 0, st, (const PointDesc*)dl, first_few, n);
-    hipLaunchKernelGGL(k_msm_join, dim3(cdiv(4 * (size_t)n, (size_t)GT)), dim3(GT), 0, st, (const PointDesc*)dl, n);
+    Scratch& win = arena.add(sizeof(P29) * MW * (size_t)n);
+    if (win.rc) return win.rc;
+    hipLaunchKernelGGL(k_msm_windows, dim3(MW * first_few + MW / 8 * (n - first_few)), dim3(GT), 0, st, win.as<P29>(), (const PointDesc*)dl, first_few);
+    hipLaunchKernelGGL(k_msm_horner, dim3(cdiv(8 * (size_t)n, (size_t)GT)), dim3(GT), 0, st, (const P29*)win.as<P29>(), (const PointDesc*)dl, n);
     ZK_LAUNCH_CHECK();
     list.clear();
     return 0;
@@ -2177,7 +2207,7 @@ int zk_g1_open_round(void* new_scalars, void* new_gens, uint32_t* sums_host, con
     std::vector<PointDesc> later;
     const RoundItem item{(Fr*)new_scalars, n29.as<A29>(), (const Fr*)scalars, g29.as<A29>(), load_fr(u), nullptr};
     rc = open_round_launch(&item, 1, old_size, 0, 0, pts.as<G1Jac>(), 3, arena, up, st, st, evs, later);
-    if (rc == 0) rc = points_queue(later, up, st);
+    if (rc == 0) rc = points_queue(later, arena, up, st);
     if (rc) { (void)hipStreamSynchronize(st); return rc; }
     hipLaunchKernelGGL(k_a29_to_jac, dim3(cdiv(new_size, GT)), dim3(GT), 0, st, (G1Jac*)new_gens, n29.as<A29>(), new_size);
     g1_normalize_queue<false>(pts.p, pts.as<G1Jac>(), (size_t)3, st);
@@ -2255,11 +2285,11 @@ static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const 
     const size_t ns = (((n0 + 1) / 2 + 1) / 2 + 1) / 2;
     Scratch& g2 = arena.add(sizeof(A29) * ns * count);
     if (g2.rc) return g2.rc;
-    Scratch& part = arena.add(sizeof(J29) * 8 * ns * count);
+    Scratch& part = arena.add(sizeof(P29) * 8 * ns * count);
     if (part.rc) return part.rc;
     std::vector<JsfK> jsf((size_t)count * JUMP_SPAN);
     SpanBatch sb;
-    sb.part = part.as<J29>();
+    sb.part = part.as<P29>();
     double fp_mults = 0;
     uint32_t longest = 1;
     for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; sb.ng[i] = g2.as<A29>() + ns * k; sb.g[i] = gens[k]; }
@@ -2466,7 +2496,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         if (last_batch(size, r)) {
             std::vector<PointDesc> mine;
             int rc = open_batch_launch(cs, cg, count, size, rounds - r, true, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, st, job.events, mine);
-            if (rc == 0) rc = points_queue(mine, job.up, st);
+            if (rc == 0) rc = points_queue(mine, job.arena, job.up, st);
             if (rc) return rc;
             tail_done = true;
             break;
@@ -2502,7 +2532,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         ++r;
     }
     {
-        int rc = points_queue(later, job.up, aux);
+        int rc = points_queue(later, job.arena, job.up, aux);
         if (rc == 0) rc = join_streams(aux, st, job.events);
         if (rc) return rc;
     }
@@ -2525,7 +2555,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R);
         std::vector<PointDesc> mine;
         int rc = bucket_sums_queue(d, out, np, job.arena, job.up, st, mine);
-        if (rc == 0) rc = points_queue(mine, job.up, st);
+        if (rc == 0) rc = points_queue(mine, job.arena, job.up, st);
         if (rc) return rc;
     }
     if (!tail_done)

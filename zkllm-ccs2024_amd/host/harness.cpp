@@ -8,6 +8,7 @@
 #include "../../include/zkllm_hip.h"
 #include "../csrc/field.hpp"
 #include "../csrc/fr29.hpp"
+#include "../csrc/fq29.hpp"
 #include "fr-tensor.hpp"
 #include "polynomial.hpp"
 #include "proof.hpp"
@@ -130,6 +131,19 @@ int zkp_host_fp_op(int op, const u32* a, const u32* b, u32* out, long n) {
             default: throw std::runtime_error("bad op");
         }
         memcpy(out + 12 * i, r.v, 48);
+    }
+    ZKP_END
+}
+// a + b of Jacobian points by the complete projective formulas (p29_add): op 0 with the products inlined, 1 with calls
+int zkp_host_p29_add(int op, const u32* a, const u32* b, u32* out, long n) {
+    ZKP_TRY
+    for (long i = 0; i < n; ++i) {
+        zk::G1Jac x, y;
+        memcpy(&x, a + 36 * i, 144);
+        memcpy(&y, b + 36 * i, 144);
+        const zk::P29 p = zk::p29_from_j29(zk::j29_from_jac(x)), q = zk::p29_from_j29(zk::j29_from_jac(y));
+        const zk::G1Jac r = zk::p29_to_jac(op == 0 ? zk::p29_add<true>(p, q) : zk::p29_add<false>(p, q));
+        memcpy(out + 36 * i, &r, 144);
     }
     ZKP_END
 }
