@@ -577,8 +577,8 @@ def assert_points_are(points, logarithms):
         assert jac_to_affine(p) == (ec_mul(l, (G1_X, G1_Y)) if l else None), i
 
 
-# 16385 .. 98304: three rounds in a span, then the batched rest (70001 with odd sizes throughout); above: one round alone (98305: its last
-# generator has no partner), two at 2^18 + 3, then a span
+# 16385 .. 131072: three rounds in a span, then the batched rest (70001 with odd sizes throughout, 98305 with a last generator that has no
+# partner); above: one round alone (2^18 + 3: two), then a span
 @pytest.mark.parametrize("n", [16385, 20000, 70001, 98304, 98305, 131072, 140001, (1 << 18) + 3])
 def test_open_follows_the_logarithms_of_its_generators(n):
     """An unprepared opening over generators of known logarithm, special ones among them, point by point in big-integer arithmetic."""

@@ -14,6 +14,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <mutex>
 #include <utility>
@@ -444,7 +445,8 @@ static constexpr int OB_MAX = 8;           // openings of equal size that share 
 static constexpr int TABLE_MIN_N = 1024;   // results of a fold below which no fold tables are made for it
 static constexpr int LAST_N = 16384;       // generators of a job (all its openings together) at which the remaining rounds are computed in one batch
 static constexpr int TAIL_LEVELS = 20;     // most rounds the batch takes
-static constexpr int SPAN_MAX_N = 3 << 15; // generators of a job up to which three rounds are taken as a batch of sums beside one fold
+static constexpr int T_SUM_MAX_N = 8192;    // generators of a job's last batch up to which it sums its rounds' T itself
+static constexpr int SPAN_MAX_N = 1 << 17; // generators of a job up to which three rounds are taken as a batch of sums beside one fold
 struct GlvK { uint32_t k1[4], k2[4]; };
 
 __device__ __forceinline__ bool aff_is_inf(const G1Affine& p) { return is_zero(p.x) && is_zero(p.y); }   // normalised infinity: all-zero limbs
@@ -987,87 +989,64 @@ __global__ void __launch_bounds__(GT) k_msm_horner(const P29* __restrict__ win, 
 //   T0_q = sum_j s^(q)_(2j) g^(q)_(2j+1) = sum_{a,b} c(a,b) sum_j s_(2^(q+1) j + a) g_(2^(q+1) j + 2^q + b),   T1_q likewise with the halves exchanged,
 // and T of round 0 is the same combination of the row commitments themselves.  `pts`: [pattern][row] points, pattern 0 the row
 // commitments, then for q = 0 .. cross_rounds - 1 the 4^q patterns (a 2^q + b) of T0_q followed by those of T1_q.
-// T of the later rounds r follows from these points as well: unrolling
-//   T_r = u(1-u) T_(r-1) + (1-u)^2 T0_(r-1) + u^2 T1_(r-1)   (u = the challenge of round r-1)
-// down to round 0 makes T_r the sum over all patterns of the rounds before r, with the products of those coefficients.
-// Target t of an opening with `full` rounds: 0 = T of round 0, 1 + 2q + side = T0_q / T1_q, 2 full + r = T_r (1 <= r < full).  The sums equal
-// the sums over all generators exactly when `pts` are such commitments of the opened tensor -- what the caller states by
-// passing them.
+// Target t of an opening with `full` rounds: 0 = T of round 0, 1 + 2q + side = T0_q / T1_q.  The sums equal the sums over all generators
+// exactly when `pts` are such commitments of the opened tensor -- what the caller states by passing them.
 __host__ __device__ __forceinline__ uint32_t cross_patterns(uint32_t rounds) { return 1u + 2u * (((1u << (2 * rounds)) - 1u) / 3u); }
-// first_pattern, npat: the points of target t; first_term: its coefficients' place (in patterns) among the terms; slot: its place in the proof
-__host__ __device__ __forceinline__ void cross_target(uint32_t t, uint32_t full, uint32_t& first_pattern, uint32_t& npat, uint32_t& first_term, uint32_t& slot) {
-    if (t == 0) { first_pattern = first_term = 0; npat = 1; slot = 0; return; }
-    if (t > 2 * full) {
-        const uint32_t r = t - 2 * full;
-        first_pattern = 0;
-        npat = cross_patterns(r);
-        first_term = cross_patterns(full);
-        for (uint32_t j = 1; j < r; ++j) first_term += cross_patterns(j);
-        slot = 3 * r;
-        return;
-    }
+// first_pattern, npat: the points of target t; slot: its place in the proof
+__host__ __device__ __forceinline__ void cross_target(uint32_t t, uint32_t& first_pattern, uint32_t& npat, uint32_t& slot) {
+    if (t == 0) { first_pattern = 0; npat = 1; slot = 0; return; }
     const uint32_t q = (t - 1) >> 1, side = (t - 1) & 1u;
     npat = 1u << (2 * q);
-    first_pattern = first_term = cross_patterns(q) + side * npat;
+    first_pattern = cross_patterns(q) + side * npat;
     slot = 3 * q + 1 + side;
 }
 // These sums are bucket multi-scalar multiplications.  Term g = pattern * nrows + row of an opening, in the order `pts`
 // lays the points out, has the coefficient eq(u_rows, row) * c(pattern) -- c = 1 for the row commitments, the product of the
-// earlier rounds' challenges for a cross pattern; the terms of T_1, T_2, ... follow, pattern by pattern again -- and a target is
-// the sum over a contiguous range of terms: one bucket sum per target over the normalised points, with the digits of all
+// earlier rounds' challenges for a cross pattern -- and a target is the sum over a contiguous range of terms: one bucket sum per target over the normalised points, with the digits of all
 // terms written once, as k_msm_recode writes them (D: (MW + 1) x terms bytes).  A term costs 32 mixed additions (a scalar
 // multiplication of its own would cost a 129-step walk).
 struct CrossDigitItem { int8_t* D; const Fr* u_rows; const Fr* u; uint32_t nrows, k_rows; };
 struct CrossDigitBatch { CrossDigitItem it[OB_MAX]; };
 // grid (ceil(most terms / 256), openings)
-__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t full, uint32_t nterm_patterns) {
+__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t npatterns) {
     const CrossDigitItem& it = cb.it[blockIdx.y];
-    const size_t terms = (size_t)nterm_patterns * it.nrows, i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    const size_t terms = (size_t)npatterns * it.nrows, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= terms) return;
-    uint32_t p = (uint32_t)(i / it.nrows), t_round = 0;
-    const uint32_t row = (uint32_t)(i - (size_t)p * it.nrows);
-    if (p >= cross_patterns(full)) {                    // a term of T_r, r = t_round
-        p -= cross_patterns(full);
-        for (t_round = 1; p >= cross_patterns(t_round); ++t_round) p -= cross_patterns(t_round);
-    }
+    const uint32_t p = (uint32_t)(i / it.nrows), row = (uint32_t)(i - (size_t)p * it.nrows);
     const Fr one = big_one_mont<8>();
     Fr coef = one;
     for (uint32_t j = 0; j < it.k_rows; ++j) coef = mont_mul(coef, ((row >> j) & 1u) ? it.u_rows[j] : sub(one, it.u_rows[j]));
-    uint32_t k0 = 0;                                    // the T_r expansion multiplies by u (1 - u) of the rounds from here on
     if (p != 0) {
         uint32_t q = 0;                                 // the patterns of round q: T0's 4^q, then T1's
         while (p >= cross_patterns(q + 1)) ++q;
-        const uint32_t in_q = p - cross_patterns(q), pl = in_q & ((1u << (2 * q)) - 1u), a = pl >> q, b = pl & ((1u << q) - 1u);
+        const uint32_t pl = (p - cross_patterns(q)) & ((1u << (2 * q)) - 1u), a = pl >> q, b = pl & ((1u << q) - 1u);
         for (uint32_t k = 0; k < q; ++k) {
             const Fr uk = it.u[k], nk = sub(one, uk);
             coef = mont_mul(coef, mont_mul(((a >> k) & 1u) ? uk : nk, ((b >> k) & 1u) ? nk : uk));
         }
-        if (t_round) {
-            const Fr f = (in_q >> (2 * q)) ? it.u[q] : sub(one, it.u[q]);
-            coef = mont_mul(coef, mont_mul(f, f));
-            k0 = q + 1;
-        }
     }
-    for (uint32_t k = k0; k < t_round; ++k) coef = mont_mul(coef, mont_mul(it.u[k], sub(one, it.u[k])));
     msm_recode_store(it.D, terms, i, from_mont(coef));
 }
-// Row commitments without cross patterns give T of round 0 alone; T of the rounds behind it follows from it and from T0, T1 of the rounds
-// before by the same unrolling.  Those points lie in the proof itself: the digits of T_1 .. T_(R-1) as bucket sums over an opening's
-// first 3 R proof points (T, T0, T1 a round; the T of later rounds take no part: zeros).  U: the challenges, opening y's at U + y * ustride
-__global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__ D0, const Fr* __restrict__ U, uint32_t ustride, uint32_t R) {
-    const uint32_t terms = (R - 1) * 3 * R, i = blockIdx.x * 256 + threadIdx.x;
+// T of the rounds behind the first follows from T of round 0 and from T0, T1 of the rounds before:
+//   T_r = u(1-u) T_(r-1) + (1-u)^2 T0_(r-1) + u^2 T1_(r-1)   (u = the challenge of round r-1)
+// unrolled down to round 0, with the products of those coefficients.  Those points lie in the proof itself: the digits of T_1 .. T_(R-1) as
+// bucket sums over an opening's first 3 (R - 1) proof points (T, T0, T1 a round; the T of later rounds take no part: zeros).  A round's T
+// is a sum over as many generators as its T0 and T1 together, so this halves what is summed.  T of the rounds above `again` (0: none) is unrolled
+// from T of round `again`.  U: the challenges, opening y's at U + y * ustride
+__global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__ D0, const Fr* __restrict__ U, uint32_t ustride, uint32_t R, uint32_t again) {
+    const uint32_t np = 3 * (R - 1), terms = (R - 1) * np, i = blockIdx.x * 256 + threadIdx.x;
     if (i >= terms) return;
     const Fr* __restrict__ u = U + (size_t)blockIdx.y * ustride;
-    const uint32_t r = 1 + i / (3 * R), m = i % (3 * R), k = m / 3, j = m % 3;
+    const uint32_t r = 1 + i / np, m = i % np, k = m / 3, j = m % 3, from = again && r > again ? again : 0u;
     const Fr one = big_one_mont<8>();
     Fr c = big_zero<8>();
-    if (m == 0 || (j != 0 && k < r)) {
+    if (k >= from && k < r && (j != 0 || k == from)) {
         c = one;
-        if (m != 0) {
+        if (j != 0) {
             const Fr f = j == 2 ? u[k] : sub(one, u[k]);
             c = mont_mul(f, f);
         }
-        for (uint32_t q = m == 0 ? 0u : k + 1; q < r; ++q) c = mont_mul(c, mont_mul(u[q], sub(one, u[q])));
+        for (uint32_t q = j == 0 ? k : k + 1; q < r; ++q) c = mont_mul(c, mont_mul(u[q], sub(one, u[q])));
     }
     msm_recode_store(D0 + (size_t)blockIdx.y * (MW + 1) * terms, terms, i, from_mont(c));
 }
@@ -1863,8 +1842,8 @@ static int points_queue(std::vector<PointDesc>& list, Arena& arena, JobUploads& 
 }
 // One halving round: the scalars' digits and the fold on st, the bucket sums on aux (their reductions are appended to `later`).
 // pts: where the round's T, T0, T1 of opening 0 go; opening i's npts further.
-// given: what of this round's sums comes from commitments of the tensor's rows (open_cross_sums_queue, k_open_unroll_digits) and is not
-// summed here: 0 nothing, 1 T, 2 T0 and T1 as well (no bucket sums at all: the round is its fold)
+// given: what of this round's sums comes from commitments of the tensor's rows or from the rounds before (open_cross_sums_queue,
+// open_unroll_queue) and is not summed here: 0 nothing, 1 T, 2 T0 and T1 as well (no bucket sums at all: the round is its fold)
 // comb_round: 0 the first round (fold table RoundItem::comb, when all items have one), 1 the second (comb2), 2 a later one
 static int open_round_launch(const RoundItem* items, int count, size_t old_size, int comb_round, int given, G1Jac* pts, size_t npts, Arena& arena, JobUploads& up,
                              hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
@@ -1950,8 +1929,8 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
 // `levels` rounds (r0 .. r0 + levels - 1 of `rounds`) in one batch over n0 generators: the scalars of all levels on st, then T, T0, T1 of
 // those rounds as bucket sums with formed coefficients on aux.  last: the batch takes all rounds that are left and the final
 // generator is one more sum; otherwise (three levels) the generators are folded three times at once on st and *gens names the results.
-// *scalars: the folded scalars.  pts: the proof points of opening 0 (npts an opening).  no_t_below: T of rounds below it is not summed here.
-static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, int no_t_below, const OpenItem* items, G1Jac* pts, size_t npts,
+// *scalars: the folded scalars.  pts: the proof points of opening 0 (npts an opening).  t_given: the rounds whose T is not summed here.
+static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, const std::function<bool(int)>& t_given, const OpenItem* items, G1Jac* pts, size_t npts,
                              const Fr* U_dev, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later);
 // g^(3) of every opening from its generators (k_open_span_slices, k_open_span_walk); challenges: rounds r0 .. r0 + 2
 static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const OpenItem* items, Arena& arena, JobUploads& up, hipStream_t st);
@@ -2239,25 +2218,21 @@ struct OpenJob {
     std::string queue_err;
     OpenJob() { up.arena = &arena; }
 };
-// The targets of every opening of a batch (T of round 0; T0, T1 of the first `full` rounds; T of those rounds behind the first) as
-// bucket sums over the openings' [pattern][row] points, on aux.
+// The targets of every opening of a batch (T of round 0; T0, T1 of the first `full` rounds) as bucket sums over the openings' [pattern][row] points, on aux.
 static int open_cross_sums_queue(const OpenItem* items, int count, uint32_t full, G1Jac* pts, size_t npts, const Fr* const* urow_dev, const Fr* U_dev, int rounds, Arena& arena,
                                  JobUploads& up, hipStream_t aux, std::vector<PointDesc>& later) {
-    const uint32_t ntargets = 1u + 2u * full + (full > 1 ? full - 1 : 0u);
-    const uint32_t npatterns = cross_patterns(full);
-    uint32_t nterm_patterns = npatterns;
-    for (uint32_t r = 1; r < full; ++r) nterm_patterns += cross_patterns(r);
+    const uint32_t ntargets = 1u + 2u * full, npatterns = cross_patterns(full);
     CrossDigitBatch db;
     const A29* base[OB_MAX];
     const int8_t* digs[OB_MAX];
     size_t most_terms = 0, most_count = 0;
     for (int i = 0; i < count; ++i) {
-        const size_t points = (size_t)npatterns * items[i].nrows, terms = (size_t)nterm_patterns * items[i].nrows;
-        ZK_ARG(items[i].nrows >= 1 && terms < (1ull << 31), "zk_g1_open: bad row count");
-        most_terms = std::max(most_terms, terms);
+        const size_t points = (size_t)npatterns * items[i].nrows;          // and as many terms
+        ZK_ARG(items[i].nrows >= 1 && points < (1ull << 31), "zk_g1_open: bad row count");
+        most_terms = std::max(most_terms, points);
         Scratch& aff = arena.add(sizeof(G1Affine) * points);
         Scratch& a29 = arena.add(sizeof(A29) * points);
-        Scratch& dg = arena.add((size_t)(MW + 1) * terms);
+        Scratch& dg = arena.add((size_t)(MW + 1) * points);
         if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
         g1_normalize_queue<true>(aff.p, (const G1Jac*)items[i].rows, points, aux);
         hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(points, 256)), dim3(256), 0, aux, a29.as<A29>(), aff.as<G1Affine>(), points);
@@ -2266,17 +2241,17 @@ static int open_cross_sums_queue(const OpenItem* items, int count, uint32_t full
         db.it[i] = CrossDigitItem{dg.as<int8_t>(), urow_dev[i], U_dev + (size_t)i * rounds, items[i].nrows, (uint32_t)items[i].k_rows};
     }
     for (int i = count; i < OB_MAX; ++i) db.it[i] = db.it[0];
-    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, full, nterm_patterns);
+    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, npatterns);
     ZK_LAUNCH_CHECK();
     std::vector<MsmDesc> d;
     std::vector<G1Jac*> out;
     for (int i = 0; i < count; ++i)
         for (uint32_t t = 0; t < ntargets; ++t) {
-            uint32_t p0, npat, t0, slot;
-            cross_target(t, full, p0, npat, t0, slot);
+            uint32_t p0, npat, slot;
+            cross_target(t, p0, npat, slot);
             const uint32_t nr = items[i].nrows;
             most_count = std::max(most_count, (size_t)npat * nr);
-            d.push_back(MsmDesc{digs[i], base[i], nterm_patterns * nr, npat * nr, 1u, t0 * nr, 1u, p0 * nr});
+            d.push_back(MsmDesc{digs[i], base[i], npatterns * nr, npat * nr, 1u, p0 * nr, 1u, p0 * nr});
             out.push_back(pts + npts * i + slot);
         }
     return bucket_sums_queue(d, out, most_count, arena, up, aux, later);
@@ -2314,7 +2289,7 @@ static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const 
     for (int i = 0; i < count; ++i) gens[i] = g2.as<A29>() + ns * i;
     return 0;
 }
-static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, int no_t_below, const OpenItem* items, G1Jac* pts, size_t npts,
+static int open_batch_launch(const Fr** scalars, const A29** gens, int count, size_t n0, int levels, bool last, int r0, int rounds, const std::function<bool(int)>& t_given, const OpenItem* items, G1Jac* pts, size_t npts,
                              const Fr* U_dev, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
     const uint32_t fin = last ? 1u : 0u, n_msm = 3 * (uint32_t)levels + fin;
     const size_t sl_n = n0 + (size_t)levels + 1;
@@ -2362,7 +2337,7 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     std::vector<G1Jac*> out;
     for (int it = 0; it < count; ++it)
         for (uint32_t i = 0; i < n_msm; ++i) {
-            if (i < 3 * (uint32_t)levels && i % 3 == 0 && r0 + (int)(i / 3) < no_t_below) continue;
+            if (i < 3 * (uint32_t)levels && i % 3 == 0 && t_given(r0 + (int)(i / 3))) continue;
             d.push_back(MsmDesc{dig.as<int8_t>(), before[it], (uint32_t)ncoef, (uint32_t)n0, 1u, (uint32_t)(((size_t)it * n_msm + i) * n0), 1u, 0u});
             out.push_back(pts + npts * it + (i == 3 * (uint32_t)levels ? 3 * (size_t)rounds : 3 * (size_t)r0 + i));
         }
@@ -2370,6 +2345,32 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     if (rc) return rc;
     for (int it = 0; it < count; ++it) scalars[it] = sl.as<Fr>() + sl_n * it + off;
     return 0;
+}
+// T of the rounds 1 .. rounds_t - 1 but `again` of every opening from its T of round 0 (above `again`, of that round) and T0, T1 of the rounds below, on st
+static int open_unroll_queue(G1Jac* pts, size_t npts, int count, int rounds_t, int again, const Fr* U_dev, int rounds, Arena& arena, JobUploads& up, hipStream_t st) {
+    if (rounds_t <= 1 || (rounds_t == 2 && again == 1)) return 0;
+    const uint32_t R = (uint32_t)rounds_t, np = 3 * (R - 1), terms = (R - 1) * np;
+    Scratch& aff = arena.add(sizeof(G1Affine) * np);
+    Scratch& a29 = arena.add(sizeof(A29) * np * count);
+    Scratch& dg = arena.add((size_t)(MW + 1) * terms * count);
+    if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
+    std::vector<MsmDesc> d;
+    std::vector<G1Jac*> out;
+    for (int i = 0; i < count; ++i) {
+        g1_normalize_queue<true>(aff.p, pts + npts * i, np, st);
+        hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(np, 256)), dim3(256), 0, st, a29.as<A29>() + (size_t)np * i, aff.as<G1Affine>(), (size_t)np);
+        for (uint32_t q = 1; q < R; ++q) {
+            if ((int)q == again) continue;
+            d.push_back(MsmDesc{dg.as<int8_t>() + (size_t)(MW + 1) * terms * i, a29.as<A29>() + (size_t)np * i, terms, np, 1u, (q - 1) * np, 1u, 0u});
+            out.push_back(pts + npts * i + 3 * q);
+        }
+    }
+    hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R, (uint32_t)again);
+    ZK_LAUNCH_CHECK();
+    std::vector<PointDesc> mine;
+    int rc = bucket_sums_queue(d, out, np, arena, up, st, mine);
+    if (rc == 0) rc = points_queue(mine, arena, up, st);
+    return rc;
 }
 // rows (optional): commitments of the opened tensor's rows, [pattern][row] as open_cross_sums_queue takes them -- the row
 // commitments alone (cross_rounds = 0) or with the cross patterns of the first cross_rounds rounds
@@ -2419,11 +2420,13 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     }
     auto last_batch = [&](size_t size, int r) { return size * (size_t)count <= (size_t)LAST_N && rounds - r <= TAIL_LEVELS; };
     // commitments of the tensors' rows: which sums they replace (all openings of the batch must bring them)
-    bool with_rows = true, comb3 = true;
+    bool with_rows = rounds > 0 && n > (size_t)TABLE_MIN_N, comb3 = true, comb1 = true, comb2 = true;
     int cross_r = 64;
     for (int i = 0; i < count; ++i) {
         with_rows = with_rows && items[i].rows != nullptr;
         cross_r = std::min(cross_r, items[i].cross_rounds);
+        comb1 = comb1 && items[i].comb != nullptr;
+        comb2 = comb2 && items[i].comb2 != nullptr;
         comb3 = comb3 && items[i].comb3 != nullptr;
     }
     int halving = 0;
@@ -2431,18 +2434,46 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         size_t sz = n;
         for (int r = 0; r < rounds && !last_batch(sz, r); ++r) { ++halving; sz = (sz + 1) / 2; }
     }
-    // row commitments alone: T of the first round from them, T of the rounds over more than TABLE_MIN_N generators unrolled from it
-    int rows_t = 0;
-    if (with_rows && cross_r == 0)
-        for (size_t sz = n; rows_t < rounds && sz > (size_t)TABLE_MIN_N; sz = (sz + 1) / 2) ++rows_t;
     if (!with_rows || halving == 0) cross_r = 0;
     // three rounds as one fold: their sums all come from cross commitments
     const bool jump = halving > 0 && with_rows && cross_r >= JUMP_ROUNDS && rounds >= JUMP_ROUNDS && !(n & (n - 1)) && n >= (size_t)JUMP_SPAN;
     if (jump) cross_r = JUMP_ROUNDS;
     else cross_r = std::min(cross_r, halving);
+    // What round r over `size` generators begins.  Three rounds as a batch of sums beside one fold where a round's fold would leave the chip
+    // half empty and take one walk's latency all the same; above that a round at a time, which sums over fewer points.  Openings of 128 x 2^17,
+    // the first round alone / in a span: 9.9 / 9.2 ms; of 16 x 2^18, two rounds alone / one and a span: 14.7 / 14.9.
+    enum Step { LAST, SPAN, ROUND };
+    auto step_of = [&](size_t size, int r) {
+        if (last_batch(size, r)) return LAST;
+        const bool comb = r == 0 ? comb1 : (r == 1 && comb2);
+        return !comb && r >= cross_r && rounds - r >= JUMP_ROUNDS && size * (size_t)count <= (size_t)SPAN_MAX_N ? SPAN : ROUND;
+    };
+    // T of round 0 from the row commitments or summed; T of the rounds from 1 to t_rounds - 1 unrolled from it.  The tensor's commitments say what
+    // T is for the rounds they have cross patterns for, or else while a round has more than TABLE_MIN_N generators: the first round behind those,
+    // t_again, has its T summed, and the rounds behind it follow from that.  A last batch that is so small that its own T cost less than the
+    // unrolling's chain of launches behind it sums them, and the unrolling of the rounds before it runs beside it: openings of 1024 and 4096
+    // generators 1.8 and 2.5 ms by sums, 2.6 and 2.9 unrolled, of 16384 4.3 and 3.8.
+    int t_rounds = rounds, t_again = 0;
+    bool unroll_early = false;
+    {
+        if (cross_r > 0) t_again = cross_r;
+        else if (with_rows)
+            for (size_t sz = n; t_again < rounds && sz > (size_t)TABLE_MIN_N; sz = (sz + 1) / 2) ++t_again;
+        size_t sz = n;
+        int r = 0;
+        if (jump) { sz = n >> JUMP_ROUNDS; r = JUMP_ROUNDS; }
+        while (r < rounds && step_of(sz, r) != LAST)
+            for (int q = step_of(sz, r) == SPAN ? JUMP_ROUNDS : 1; q > 0; --q) { sz = (sz + 1) / 2; ++r; }
+        if (r < rounds && sz * (size_t)count <= (size_t)T_SUM_MAX_N) {
+            t_rounds = std::min(std::max(r + 1, t_again), rounds);
+            unroll_early = t_rounds == r + 1;
+        }
+        if (t_again >= t_rounds) t_again = 0;
+    }
+    auto t_given = [&](int r) { return r == 0 ? with_rows : r < t_rounds && r != t_again; };
     std::vector<PointDesc> later;        // bucket reductions that nothing waits for before the end: one launch behind the last round
-    if (rows_t > 1) GLAUNCH(k_g1_fill, npts * count, st, job.pts, g1_infinity(), npts * count);
-    if (cross_r > 0 || rows_t > 0) {
+    if (t_rounds > 1) GLAUNCH(k_g1_fill, npts * count, st, job.pts, g1_infinity(), npts * count);
+    if (with_rows) {
         int rc = join_streams(st, aux, job.events);          // the challenges travel on st
         if (rc == 0) rc = open_cross_sums_queue(items, count, (uint32_t)cross_r, job.pts, npts, urow_dev, U_dev, rounds, job.arena, job.up, aux, later);
         if (rc) return rc;
@@ -2492,22 +2523,27 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         size = ns;
         r = JUMP_ROUNDS;
     }
+    auto reductions = [&]() {            // on aux: the sums that nothing waited for, and T of the rounds that follow from them
+        int rc = points_queue(later, job.arena, job.up, aux);
+        if (rc == 0 && unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, rounds, job.arena, job.up, aux);
+        return rc;
+    };
     while (r < rounds) {
-        if (last_batch(size, r)) {
+        const Step step = step_of(size, r);
+        if (step == LAST) {
+            if (unroll_early && aux != st) {
+                int rc = reductions();
+                if (rc) return rc;
+            }
             std::vector<PointDesc> mine;
-            int rc = open_batch_launch(cs, cg, count, size, rounds - r, true, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, st, job.events, mine);
+            int rc = open_batch_launch(cs, cg, count, size, rounds - r, true, r, rounds, t_given, items, job.pts, npts, U_dev, job.arena, job.up, st, st, job.events, mine);
             if (rc == 0) rc = points_queue(mine, job.arena, job.up, st);
             if (rc) return rc;
             tail_done = true;
             break;
         }
-        bool comb = r <= 1;
-        for (int i = 0; i < count; ++i) comb = comb && (r == 0 ? items[i].comb : items[i].comb2) != nullptr;
-        // Three rounds as a batch of sums beside one fold where a round's fold would leave the chip half empty and take one walk's
-        // latency (2.4 ms) all the same; above that a round at a time, which sums over fewer points.  Openings of 16 rows, the first round
-        // alone / in a span: 70000 generators 9.2 / 8.1 ms, 100000 10.4 / 10.5, 2^17 11.1 / 11.5, 2^18 17.7 / 18.8.
-        if (!comb && r >= cross_r && rounds - r >= JUMP_ROUNDS && size * (size_t)count <= (size_t)SPAN_MAX_N) {
-            int rc = open_batch_launch(cs, cg, count, size, JUMP_ROUNDS, false, r, rounds, rows_t, items, job.pts, npts, U_dev, job.arena, job.up, st, aux, job.events, later);
+        if (step == SPAN) {
+            int rc = open_batch_launch(cs, cg, count, size, JUMP_ROUNDS, false, r, rounds, t_given, items, job.pts, npts, U_dev, job.arena, job.up, st, aux, job.events, later);
             if (rc) return rc;
             size = (((size + 1) / 2 + 1) / 2 + 1) / 2;
             r += JUMP_ROUNDS;
@@ -2524,7 +2560,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
             if (r == 0) ri[i].comb = items[i].comb;
             if (r == 1) { ri[i].comb2 = items[i].comb2; ri[i].u_prev = load_fr(items[i].u + 8 * (r - 1)); }
         }
-        const int given = r < cross_r ? 2 : (r < rows_t ? 1 : 0);
+        const int given = r < cross_r ? 2 : (t_given(r) ? 1 : 0);
         int rc = open_round_launch(ri, count, size, std::min(r, 2), given, job.pts + 3 * (size_t)r, npts, job.arena, job.up, st, aux, job.events, later);
         if (rc) return rc;
         for (int i = 0; i < count; ++i) { cs[i] = ri[i].new_scalars; cg[i] = ri[i].new_gens; }
@@ -2532,30 +2568,9 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
         ++r;
     }
     {
-        int rc = points_queue(later, job.arena, job.up, aux);
+        int rc = unroll_early && aux != st && tail_done ? 0 : reductions();
         if (rc == 0) rc = join_streams(aux, st, job.events);
-        if (rc) return rc;
-    }
-    if (rows_t > 1) {
-        const uint32_t R = (uint32_t)rows_t, np = 3 * R, terms = (R - 1) * np;
-        Scratch& aff = job.arena.add(sizeof(G1Affine) * np);
-        Scratch& a29 = job.arena.add(sizeof(A29) * np * count);
-        Scratch& dg = job.arena.add((size_t)(MW + 1) * terms * count);
-        if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
-        std::vector<MsmDesc> d;
-        std::vector<G1Jac*> out;
-        for (int i = 0; i < count; ++i) {
-            g1_normalize_queue<true>(aff.p, job.pts + npts * i, np, st);
-            hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(np, 256)), dim3(256), 0, st, a29.as<A29>() + (size_t)np * i, aff.as<G1Affine>(), (size_t)np);
-            for (uint32_t q = 1; q < R; ++q) {
-                d.push_back(MsmDesc{dg.as<int8_t>() + (size_t)(MW + 1) * terms * i, a29.as<A29>() + (size_t)np * i, terms, np, 1u, (q - 1) * np, 1u, 0u});
-                out.push_back(job.pts + npts * i + 3 * q);
-            }
-        }
-        hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R);
-        std::vector<PointDesc> mine;
-        int rc = bucket_sums_queue(d, out, np, job.arena, job.up, st, mine);
-        if (rc == 0) rc = points_queue(mine, job.arena, job.up, st);
+        if (rc == 0 && !unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, rounds, job.arena, job.up, st);
         if (rc) return rc;
     }
     if (!tail_done)
