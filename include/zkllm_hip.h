@@ -380,6 +380,12 @@ int zk_lookup_prove_begin_hinted_ints(void** handle, const void* S, const void* 
 int zk_lookup_prove_begin_mapped_ints(void** handle, const void* S_in, const void* S_in_prepared, const void* S_out, const void* S_out_prepared, const void* mapped_prepared,
                                       const uint32_t* r, const void* T, const void* m, int32_t low, const uint32_t* beta, const uint32_t* u_eq, const uint32_t* v, size_t D,
                                       size_t N, int rounds, void* stream);
+/* zk_lookup_prove_begin_mapped with the outputs' and the mapped values' int32 forms alone, where the queries keep none: a job whose first
+ * round is the fused one (zk_lookup_ints_suffice) reads the queries as field elements and the outputs in that form only; any other job is
+ * zk_lookup_prove_begin_mapped's. */
+int zk_lookup_prove_begin_mapped_out_ints(void** handle, const void* S_in, const void* S_out, const void* S_out_prepared, const void* mapped_prepared, const uint32_t* r,
+                                          const void* T, const void* m, int32_t low, const uint32_t* beta, const uint32_t* u_eq, const uint32_t* v, size_t D, size_t N, int rounds,
+                                          void* stream);
 int zk_lookup_prove_end(void* handle, uint32_t* bm_host, uint32_t* sums_host);
 /* Diagnostics of the job zk_lookup_prove_end collected last (no counterpart in the reference): *n_ok = how many leading table
  * entries were what the integers say -- the queries naming one of them took the first round's short path, the others their own

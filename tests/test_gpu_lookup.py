@@ -1234,6 +1234,67 @@ def test_lookup_jobs_that_read_int32_forms_equal_the_plain_one(k):
         hip.free(q)
 
 
+@pytest.mark.parametrize("k", [13, 17, 19])
+def test_lookup_jobs_that_read_integers_off_field_elements_equal_the_plain_one(k):
+    """zk_lookup_prove_begin_hinted over queries that are their own hints, and zk_lookup_prove_begin_mapped_out_ints (the fused first round, from
+    2^17 queries on, takes the queries' integers from the field elements), against zk_lookup_prove_begin: queries outside the table, at
+    the ends of the 32-bit integers and just beyond them, that are no integers, -beta, and a table entry that is not what its position says."""
+    import ctypes
+    from gpuhelp import Hip, c_void_p, c_size_t, c_int
+    hip = Hip()
+    D, N, low = 1 << k, 64, -9
+    rng = np.random.default_rng(2000 + k)
+    mapped = [int(x) for x in rng.integers(-2 ** 31, 2 ** 31, N)]
+    r_fr, beta = ch(72, 1)[0], ch(73, 1)[0]
+    r, b = fr_ints(r_fr.reshape(1, 8))[0], fr_ints(beta.reshape(1, 8))[0]
+    pos = rng.integers(0, N, D)
+    s_in, s_out = [int(p) + low for p in pos], [mapped[int(p)] for p in pos]
+    odd = rng.choice(np.arange(D), 200, replace=False)
+    ends = [0, -1, 1, 2 ** 31 - 1, 2 ** 31, -2 ** 31, -2 ** 31 - 1, 2 ** 32 - 1, 2 ** 32, -2 ** 32, -2 ** 32 + 1, 2 ** 33, low - 1, low + N, 1 << 64, 1 << 224, R_MOD // 2, -b]
+    for i, x in zip(odd, ends + [int(y) for y in fr_ints(ch(76, 200 - len(ends)))]):
+        s_in[int(i)] = x
+    for i in odd[:40:2]:
+        s_out[int(i)] = 12345 + int(i)
+    Tr = [(low + j) % R_MOD for j in range(N)]
+    Tr[13] = (Tr[13] + 5) % R_MOD
+    Tc = [(low + j + r * mapped[j]) % R_MOD for j in range(N)]
+    Tc[7] = (Tc[7] + 1) % R_MOD
+    S_com = [(x + r * y) % R_MOD for x, y in zip(s_in, s_out)]
+    m, u, v = fr_array([int(c) for c in np.bincount(pos, minlength=N)]), ch(74, k - 1), ch(75, k)
+    bufs = [hip.upload(fr_array([x % R_MOD for x in col])) for col in (s_in, s_out, mapped, Tr, Tc, S_com)]
+    dSi, dSo, dMp, dTr, dTc, dS = (c_void_p(x) for x in bufs)
+    bufs.append(hip.upload(m))
+    dm = c_void_p(bufs[-1])
+    prep = []
+    for dev, n in ((dSo, D), (dMp, N)):
+        h = c_void_p()
+        hip.call("zk_fr_fold_prepare", ctypes.byref(h), dev, c_size_t(n), None)
+        assert h.value
+        prep.append(h)
+    tail = (beta, u, v, c_size_t(D), c_size_t(N), c_int(k), None)
+    # the outputs' field elements are not read where the first round is the fused one
+    bufs.append(hip.upload(ch(77, D)))
+    fSo = c_void_p(bufs[-1]) if hip.lib.zk_lookup_ints_suffice(c_size_t(D), c_size_t(N)) == 1 else dSo
+    jobs = {"range, plain": ("zk_lookup_prove_begin", dSi, dTr, dm), "range": ("zk_lookup_prove_begin_hinted", dSi, dTr, dm, dSi, c_int(low)),
+            "mapping, plain": ("zk_lookup_prove_begin", dS, dTc, dm),
+            "mapping": ("zk_lookup_prove_begin_mapped_out_ints", dSi, fSo, prep[0], prep[1], r_fr, dTc, dm, c_int(low))}
+    res = {}
+    for name, (entry, *args) in jobs.items():
+        print(name, flush=True)
+        h = c_void_p()
+        hip.call(entry, ctypes.byref(h), *args, *tail)
+        bm, sums = np.zeros(8, np.uint32), np.zeros((k * 11, 8), np.uint32)
+        hip.call("zk_lookup_prove_end", h, bm, sums)
+        res[name] = (bm, sums)
+    for name in ("range", "mapping"):
+        plain = res[name + ", plain"]
+        assert plain[1].any() and (plain[0] == res[name][0]).all() and (plain[1] == res[name][1]).all(), name
+    for h in prep:
+        hip.call("zk_fr_fold_prepared_free", h)
+    for x in bufs:
+        hip.free(x)
+
+
 @pytest.mark.parametrize("n", [3007, 1 << 16])
 def test_int32_forms_written_with_the_tensors_serve_index_gather_and_evaluations(n):
     """zk_softmax_decompose_ints writes every digit plane as field elements and as int32 (both checked against divmod);

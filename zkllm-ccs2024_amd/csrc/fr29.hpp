@@ -35,6 +35,7 @@ ZK_HD Fr29 fr29_2_527() { constexpr int32_t t[9] = {238450677, 105123874, 285095
 ZK_HD Fr29 fr29_2_266() { constexpr int32_t t[9] = {536868651, 18087, 526333248, 216203804, 294598241, 8484555, 89016444, 271483280, 1968430}; return fr29_const(t); }     // 2^266 mod r
 ZK_HD Fr29 fr29_2_271() { constexpr int32_t t[9] = {536798552, 578879, 254716416, 35656607, 98837070, 269398762, 12757061, 312906888, 2209941}; return fr29_const(t); }     // 2^271 mod r
 ZK_HD Fr29 fr29_2_522() { constexpr int32_t t[9] = {175223744, 489824382, 375642521, 475708563, 62229572, 199455800, 136968049, 375395230, 2620817}; return fr29_const(t); }   // 2^522 mod r
+ZK_HD Fr29 fr29_2_532() { constexpr int32_t t[9] = {114228895, 142738518, 3129318, 211945681, 138120195, 474365025, 94583408, 180499405, 1807122}; return fr29_const(t); }     // 2^532 mod r
 ZK_HD Fr29 fr29_zero() {
     Fr29 r;
 #pragma unroll
@@ -321,6 +322,79 @@ __device__ __forceinline__ void fr29_wave_sum(uint32_t (&l)[9]) {
 #pragma unroll
     for (int i = 0; i < 9; ++i) l[i] = dpp_plus<0x143, 0xC>(dpp_plus<0x142, 0xA>(l[i]));      // row 0 into 1, 2 into 3, then the lower half into the upper
     fr29_carry_u(l);
+}
+
+// ---- sums over a workgroup that are reduced once -------------------------------------------------------------------------
+// A lane's sums stay integers in 29-bit limbs while they are added up over the lanes; the residues are taken of the workgroup's sums, a lane
+// a sum in one of its waves.  (Reduced a lane first, the five sums of a round took 4000 instructions a wave, what two pairs cost.)
+static constexpr int RAW_LIMBS = 19;                      // 2^522 a lane, 256 lanes
+// the wave's sum of N limbs (the top one small enough for 64 of it) to slot; every lane of the wave active
+template <int N> __device__ __forceinline__ void raw_wave_sum(uint32_t (&l)[N], uint32_t* slot) {
+    auto carry = [&]() {
+#pragma unroll
+        for (int i = 0; i < N - 1; ++i) {
+            l[i + 1] += l[i] >> 29;
+            l[i] &= R29M;
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < N; ++i) l[i] = dpp_plus<0x112>(dpp_plus<0x111>(l[i]));
+    carry();
+#pragma unroll
+    for (int i = 0; i < N; ++i) l[i] = dpp_plus<0x118>(dpp_plus<0x114>(l[i]));
+    carry();
+#pragma unroll
+    for (int i = 0; i < N; ++i) l[i] = dpp_plus<0x143, 0xC>(dpp_plus<0x142, 0xA>(l[i]));
+    carry();
+    if ((threadIdx.x & 63u) == 63u) {
+#pragma unroll
+        for (int i = 0; i < RAW_LIMBS; ++i) slot[i] = i < N ? l[i] : 0u;
+    }
+}
+__device__ __forceinline__ void raw_put(Wide29& w, uint32_t* slot) {      // below 2^522
+    wide29_carry(w);
+    uint32_t l[19];
+#pragma unroll
+    for (int i = 0; i < 18; ++i) l[i] = (uint32_t)w.c[i];
+    l[18] = 0u;
+    raw_wave_sum(l, slot);
+}
+__device__ __forceinline__ void raw_put(const uint32_t (&words)[9], uint32_t* slot) {      // a sum of up to 2^12 elements as nine 32-bit words
+    uint32_t l[10];
+#pragma unroll
+    for (int i = 0; i < 10; ++i) {
+        const int off = 29 * i, w = off >> 5, sh = off & 31;
+        uint32_t v = words[w] >> sh;
+        if (sh > 3 && w + 1 < 9) v |= words[w + 1] << (32 - sh);
+        l[i] = i < 9 ? v & R29M : v;
+    }
+    raw_wave_sum(l, slot);
+}
+__device__ __forceinline__ void raw_put(const Fr29& x, uint32_t* slot) {      // limb 8 below 2^31
+    uint32_t l[10];
+#pragma unroll
+    for (int i = 0; i < 9; ++i) l[i] = (uint32_t)x.l[i];
+    l[9] = l[8] >> 29;
+    l[8] &= R29M;
+    raw_wave_sum(l, slot);
+}
+// V fix 2^-522 mod r, canonical, of a workgroup's sum V; slot: its first wave's, the others' `stride` words apart
+template <int WAVES> __device__ __forceinline__ Fr raw_residue(const uint32_t* slot, uint32_t stride, const Fr29& fix) {
+    uint32_t v[RAW_LIMBS];
+#pragma unroll
+    for (int i = 0; i < RAW_LIMBS; ++i) {
+        v[i] = slot[i];
+#pragma unroll
+        for (int w = 1; w < WAVES; ++w) v[i] += slot[(uint32_t)w * stride + i];
+    }
+#pragma unroll
+    for (int i = 0; i < RAW_LIMBS - 1; ++i) {
+        v[i + 1] += v[i] >> 29;
+        v[i] &= R29M;
+    }
+    const Fr29 top = fr29_2_522();
+    const Fr29 t = fr29_redc<18>([&](int k) { return (int64_t)v[k] + (k < 9 ? (int64_t)v[18] * top.l[k < 9 ? k : 0] : 0); });
+    return fr29_canon_pack<3>(fr29_mul(t, fix));
 }
 
 // ---- elements in LDS: twelve words each, so that rows of sixteen lanes read without bank conflicts ------------------------

@@ -126,10 +126,17 @@ static inline unsigned reduce_grid(size_t n) {
     if (b < 1) b = 1;
     return (unsigned)b;
 }
+// Two workgroups a CU hold their registers (or their LDS) in the large rounds' kernels: the 512 that run side by side, while a lane's
+// unreduced sums hold its share (256 of them); a second half behind them would begin and end anew.  2^22 queries, the first two rounds in one
+// pass: 227 us on 1024 workgroups whose lanes reduced their own sums, 182 on 512 that reduce them once; 2^20 pairs of the next round 87 and 49.
+static inline unsigned resident_grid(size_t n) {
+    const unsigned all = reduce_grid(n);
+    return n <= (size_t)256 * 512 * TPB ? std::min(all, 512u) : all;
+}
 // the grid of a round that gives a lane `per_lane` pairs where the round has them: at least 256 workgroups (one a CU: with 64, rounds
-// of 2^14 to 2^18 pairs left most of the chip idle -- a lookup of 2^22 queries 721 us, with 256 692), at most reduce_grid's
+// of 2^14 to 2^18 pairs left most of the chip idle -- a lookup of 2^22 queries 721 us, with 256 692)
 static inline unsigned round_grid(size_t n, unsigned per_lane) {
-    const size_t all = reduce_grid(n), want = n / ((size_t)TPB * per_lane);
+    const size_t all = resident_grid(n), want = n / ((size_t)TPB * per_lane);
     return (unsigned)std::min(all, std::max<size_t>(256, want));
 }
 // finish K sums (K x nb partials) where the host reads them, applying the R correction (to_mont)
@@ -544,7 +551,10 @@ struct HintSrc { const Fr* TB; const Fr* hint; Fr low; Fr beta; uint32_t N; cons
                  // (zk_fr_gather_by_queries_ints).  A query that names an entry below *n_ok then needs neither its output nor the
                  // entry's expected integer (for a plain table; for a mapping table with trusted outputs): nothing is gathered but
                  // the table record.
-                 const uint32_t* n_ok = nullptr; bool trusted_out = false; };
+                 const uint32_t* n_ok = nullptr; bool trusted_out = false;
+                 // fr_queries: hint_ints is null and the queries' integers are taken from the field elements in hint (a query that is no
+                 // 32-bit integer is inverted on its own)
+                 bool fr_queries = false; };
 static constexpr int32_t INTS_POISON = (int32_t)0x80000000;
 __device__ __forceinline__ Fr hinted_query(const Fr* __restrict__ S, size_t i, const HintSrc& h) {
     return h.S_out ? add(h.hint[i], mont_mul(h.r_mont, h.S_out[i])) : S[i];
@@ -580,12 +590,29 @@ __global__ void __launch_bounds__(TPB) k_lookup_ints_check(int32_t* __restrict__
     want[j] = ok ? (mapped_ints ? mapped_ints[j] : 0) : INTS_POISON;
     if (!ok) atomicMin(n_ok, j);          // *n_ok starts at 0xFFFFFFFF
 }
-// query i and 1 / (query + beta) from the int32 forms (HintSrc); unit as in inv_by_hint
-__device__ __forceinline__ Fr query_inv_ints(size_t i, const HintSrc& h, Fr& a, bool& unit, int32_t* query = nullptr) {
-    const int32_t hi = __builtin_nontemporal_load(h.hint_ints + i);
+// whether x is a 32-bit integer v (v itself, or r - |v|)
+__device__ __forceinline__ bool fr_is_i32(const Fr& x, int32_t& v) {
+    uint32_t high = 0, high_neg = 0;
+#pragma unroll
+    for (int l = 2; l < 8; ++l) { high |= x.v[l]; high_neg |= x.v[l] ^ FrK::P(l); }
+    const bool pos = (high | x.v[1]) == 0 && !(x.v[0] >> 31);
+    const uint32_t d = x.v[0] - 1u;                    // r = 1 + (2^32 - 1) 2^32 + ...: r - k has 1 - k in its low word, with a borrow for k > 1
+    const bool neg = high_neg == 0 && (x.v[1] == 0xFFFFFFFEu ? (d >> 31) != 0 : (x.v[1] == 0xFFFFFFFFu && x.v[0] == 0));
+    v = (int32_t)(pos ? x.v[0] : d);
+    return pos || neg;
+}
+// query i and 1 / (query + beta) from the int32 forms (HintSrc), FRQ: of the queries' field elements; unit as in inv_by_hint
+template <bool FRQ = false> __device__ __forceinline__ Fr query_inv_ints(size_t i, const HintSrc& h, Fr& a, bool& unit, int32_t* query = nullptr) {
+    int32_t hi;
+    bool is_int = true;
+    Fr x;
+    if constexpr (FRQ) {
+        x = ld_stream(h.hint + i);
+        is_int = fr_is_i32(x, hi);
+    } else hi = __builtin_nontemporal_load(h.hint_ints + i);
     if (query) *query = hi;
     const int64_t d = (int64_t)hi - (int64_t)h.low_int;
-    const bool in_table = d >= 0 && d < (int64_t)h.N;
+    const bool in_table = is_int && d >= 0 && d < (int64_t)h.N;
     const uint32_t j = in_table ? (uint32_t)d : 0u;
     const bool sure = in_table && j < *h.n_ok && (!h.sout_ints || h.trusted_out);
     int32_t so = 0;
@@ -600,7 +627,7 @@ __device__ __forceinline__ Fr query_inv_ints(size_t i, const HintSrc& h, Fr& a, 
         unit = !is_zero(a);
         return h.TB[2 * (size_t)j];
     }
-    Fr sv = fr_from_i64((int64_t)hi);
+    Fr sv = FRQ ? x : fr_from_i64((int64_t)hi);
     if (h.sout_ints) sv = add(sv, mont_mul(h.r_mont, fr_from_i64((int64_t)so)));
     a = inv_plus_beta_alone(sv, h.beta);
     unit = false;
@@ -724,20 +751,23 @@ k_lookup_round(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ 
 }
 
 // ---- the same round with the arithmetic in 29-bit limbs (fr29.hpp) ----------------------------------------------------------
-// sum of up to 2^32 - 1 canonical elements as a plain 288-bit integer (nine words), and its residue
+__device__ __forceinline__ Fr fr_shfl(const Fr& x, int lane) {
+    Fr r;
+#pragma unroll
+    for (int l = 0; l < 8; ++l) r.v[l] = (uint32_t)__shfl((int)x.v[l], lane, 64);
+    return r;
+}
+// lanes at .. at + 2 hold the weighted sums of a0 s0, of (a0 + da)(s0 + ds) and of da ds: the middle coefficient comes of the three
+__device__ __forceinline__ Fr raw_middle(const Fr& x, uint32_t at) {
+    const Fr first = fr_shfl(x, (int)at), last = fr_shfl(x, (int)at + 2), m = sub(sub(x, first), last);
+    return threadIdx.x == at + 1 ? m : x;
+}
+// sum of up to 2^32 - 1 canonical elements as a plain 288-bit integer (nine words)
 __device__ __forceinline__ void sum9_add(uint32_t (&acc)[9], const Fr& x) {
     uint32_t c = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] = addc32(acc[i], x.v[i], c);
     acc[8] += c;
-}
-__device__ __forceinline__ Fr sum9_residue(const uint32_t (&acc)[9]) {
-    Fr lo, hi = big_zero<8>();
-#pragma unroll
-    for (int i = 0; i < 8; ++i) lo.v[i] = acc[i];
-    lo = reduce_once(reduce_once(lo));          // below 2^256 < 3 r
-    hi.v[0] = acc[8];
-    return add(lo, mont_mul(hi, big_r2<8>()));  // hi * 2^256
 }
 // k_lookup_round<false, false> (phase 1, inverses given) for rounds of many pairs: same inputs, same outputs (folded tensors
 // canonical, the five sums as that kernel leaves them), about a quarter fewer vector instructions.  The eq weight e arrives
@@ -780,14 +810,23 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(2, 2))
         nA[t] = fr29_canon_pack(fr29_add(a0, fr29_mul(vq, da)));
         if (pass != 2) nS[t] = fr29_canon_pack(fr29_add(s0r, fr29_mul(vq, ds)));
     }
-    Fr acc[5];
-    const Fr29 fix = fr29_2_271();
-    acc[0] = fr29_canon_pack(fr29_mul(wide29_redc(w0), fix));
-    acc[2] = fr29_canon_pack(fr29_mul(wide29_redc(w2), fix));
-    acc[1] = sub(sub(fr29_canon_pack(fr29_mul(wide29_redc(wx), fix)), acc[0]), acc[2]);
-    acc[3] = sum9_residue(sa0);
-    acc[4] = sub(sum9_residue(sa1), acc[3]);
-    block_reduce_store<5>(acc, partials + (size_t)(pass == 0 ? 0 : (pass == 1 ? 5 : 8)) * gridDim.x, pass == 0 ? 5u : 3u);
+    __shared__ uint32_t raw[TPB / 64][5][RAW_LIMBS];
+    const uint32_t wv = threadIdx.x >> 6, k = threadIdx.x, keep = pass == 0 ? 5u : 3u;
+    raw_put(w0, raw[wv][0]);
+    raw_put(wx, raw[wv][1]);
+    raw_put(w2, raw[wv][2]);
+    if (pass == 0) {
+        raw_put(sa0, raw[wv][3]);
+        raw_put(sa1, raw[wv][4]);
+    }
+    __syncthreads();
+    if (k < keep) {
+        Fr x = raw_residue<TPB / 64>(raw[0][k], 5 * RAW_LIMBS, fr29_select(k < 3, fr29_2_271(), fr29_2_522()));
+        x = raw_middle(x, 0);
+        const Fr f = fr_shfl(x, 3);
+        if (k == 4) x = sub(x, f);                          // the second half's sum less the first's
+        partials[(size_t)((pass == 0 ? 0u : (pass == 1 ? 5u : 8u)) + k) * gridDim.x + blockIdx.x] = x;
+    }
 }
 
 // k_lookup_round<false, true> for queries given by their int32 forms (HintSrc::hint_ints), with the arithmetic of the common
@@ -796,7 +835,7 @@ __global__ void __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(2, 2))
 // with an inverse of its own (a query that is no table entry, or -beta) takes the formulas of the other kernel in 32-bit limbs.
 // Same inputs, same outputs (folded tensors canonical, the five sums with the factors that kernel leaves on them).  At most
 // 512 pairs per lane (the unreduced sum holds 2^522): the launch site checks.
-__global__ void __launch_bounds__(TPB) k_lookup_first29(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ nS, const Fr* __restrict__ E, const Fr beta, const Fr v_mont,
+template <bool FRQ> __global__ void __launch_bounds__(TPB) k_lookup_first29(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ nS, const Fr* __restrict__ E, const Fr beta, const Fr v_mont,
                                                         size_t n_out, Fr* __restrict__ nE, const HintSrc hs) {
     const Fr29 vq = fr29_mul(fr29_repack(v_mont), fr29_2_266());      // v 2^261
     const Fr29 b2 = fr29_repack(add(beta, beta));
@@ -811,8 +850,8 @@ __global__ void __launch_bounds__(TPB) k_lookup_first29(Fr* __restrict__ partial
         if (nE && t < n_out / 2) st_stream(nE + t, add(e, ld_stream(E + t + n_out / 2)));      // the next round's table: the top variable summed out
         Fr s0w, s1w, a0w, a1w;
         bool unit0 = false, unit1 = false;
-        s0w = query_inv_ints(t, hs, a0w, unit0);
-        s1w = query_inv_ints(t + n_out, hs, a1w, unit1);
+        s0w = query_inv_ints<FRQ>(t, hs, a0w, unit0);
+        s1w = query_inv_ints<FRQ>(t + n_out, hs, a1w, unit1);
         sum9_add(sa0, a0w);
         sum9_add(sa1, a1w);
         if (unit0 && unit1) {
@@ -834,21 +873,27 @@ __global__ void __launch_bounds__(TPB) k_lookup_first29(Fr* __restrict__ partial
             st_stream(nS + t, add(s0w, mont_mul(v_mont, ds)));
         }
     }
-    Fr acc[5];
-    // E M 2^-5 summed; reduced (2^-261) and brought to the factor 2^-256 of the other kernel's products by 2^271 (2^-261 again)
-    const Fr acc_em = fr29_canon_pack(fr29_mul(wide29_redc(wx), fr29_2_271()));
-    // E is in Montgomery form and the sums carry R^-1: sum(E) R^-2 through one product with R^-1
-    constexpr uint32_t RINV[8] = {4269129792u, 334977897u, 165441631u, 2876230287u, 1333208682u, 1912866698u, 805346647u, 465471123u};
-    Fr k;
-#pragma unroll
-    for (int l = 0; l < 8; ++l) k.v[l] = RINV[l];
-    const Fr one = mont_mul(sum9_residue(se), k), two = add(one, one), four = add(two, two);
-    acc[0] = add(c0s, one);
-    acc[1] = add(c1s, sub(acc_em, four));
-    acc[2] = add(c2s, sub(four, acc_em));
-    acc[3] = sum9_residue(sa0);
-    acc[4] = sub(sum9_residue(sa1), acc[3]);
-    block_reduce_store<5>(acc, partials);
+    __shared__ uint32_t raw[TPB / 64][7][RAW_LIMBS];
+    const uint32_t wv = threadIdx.x >> 6, k = threadIdx.x;
+    raw_put(wx, raw[wv][0]);
+    raw_put(se, raw[wv][1]);
+    raw_put(sa0, raw[wv][2]);
+    raw_put(sa1, raw[wv][3]);
+    raw_put(fr29_repack(c0s), raw[wv][4]);
+    raw_put(fr29_repack(c1s), raw[wv][5]);
+    raw_put(fr29_repack(c2s), raw[wv][6]);
+    __syncthreads();
+    if (k < 8) {
+        // E M 2^-5 summed: 2^-522 2^271 is the factor 2^-256 of the other kernel's products.  E is in Montgomery form and the sums carry
+        // R^-1: sum(E) R^-2 = sum(E) 2^10 2^-522.  The others as they are.
+        Fr29 ten = fr29_zero();
+        ten.l[0] = 1 << 10;
+        const Fr x = raw_residue<TPB / 64>(raw[0][k < 7 ? k : 6], 7 * RAW_LIMBS, fr29_select(k == 0, fr29_2_271(), fr29_select(k == 1, ten, fr29_2_522())));
+        const Fr em = fr_shfl(x, 0), one = fr_shfl(x, 1), two = add(one, one), four = add(two, two), s0 = fr_shfl(x, 2), s1 = fr_shfl(x, 3);
+        const Fr c0 = fr_shfl(x, 4), c1 = fr_shfl(x, 5), c2 = fr_shfl(x, 6);
+        const Fr o = k == 0 ? add(c0, one) : (k == 1 ? add(c1, sub(em, four)) : (k == 2 ? add(c2, sub(four, em)) : (k == 3 ? s0 : sub(s1, s0))));
+        if (k < 5) partials[(size_t)k * gridDim.x + blockIdx.x] = o;
+    }
 }
 
 // The first TWO rounds of such a job in one pass: the folded tensors of the first round are never written or read back.
@@ -894,7 +939,7 @@ static First2Consts first2_consts(const Fr& beta, const Fr& v1_mont, const Fr& v
     c.nvs1 = sf.nvs;
     return c;
 }
-template <bool PLAIN> __global__ void __launch_bounds__(TPB) k_lookup_first2_29(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ nS, const Fr* __restrict__ E, const Fr beta,
+template <bool PLAIN, bool FRQ> __global__ void __launch_bounds__(TPB) k_lookup_first2_29(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ nS, const Fr* __restrict__ E, const Fr beta,
                                                           const Fr v1_mont, const First2Consts cs, size_t h2, Fr* __restrict__ nE3, const HintSrc hs) {
     __shared__ uint32_t rare[3][8][TPB];                               // round 1: the three weighted terms of the pairs with an inverse of their own, per lane
     const size_t h1 = 2 * h2;
@@ -924,12 +969,6 @@ template <bool PLAIN> __global__ void __launch_bounds__(TPB) k_lookup_first2_29(
 #pragma unroll
         for (int l = 0; l < 9; ++l) qsum[k][l][threadIdx.x] = acc[l];
     };
-    auto qsum_residue = [&](int k) {
-        uint32_t acc[9];
-#pragma unroll
-        for (int l = 0; l < 9; ++l) acc[l] = qsum[k][l][threadIdx.x];
-        return sum9_residue(acc);
-    };
     Fr29 t0 = fr29_zero(), t2 = fr29_zero(), tx = fr29_zero();         // round 2: the three weighted sums, times 2^-266
     uint32_t it = 0;
     for (size_t t = (size_t)blockIdx.x * TPB + threadIdx.x; t < h2; t += (size_t)gridDim.x * TPB) {
@@ -941,8 +980,8 @@ template <bool PLAIN> __global__ void __launch_bounds__(TPB) k_lookup_first2_29(
             Fr s0w, s1w, a0w, a1w;
             bool unit0 = false, unit1 = false;
             int32_t q0 = 0, q1 = 0;
-            s0w = query_inv_ints(i, hs, a0w, unit0, &q0);
-            s1w = query_inv_ints(i + h1, hs, a1w, unit1, &q1);
+            s0w = query_inv_ints<FRQ>(i, hs, a0w, unit0, &q0);
+            s1w = query_inv_ints<FRQ>(i + h1, hs, a1w, unit1, &q1);
             qsum_add(qa, a0w);
             qsum_add(qb, a1w);
             if constexpr (PLAIN) { if (unit0 && unit1) {
@@ -995,46 +1034,46 @@ template <bool PLAIN> __global__ void __launch_bounds__(TPB) k_lookup_first2_29(
         st_stream(nA + t, fr29_canon_pack<3>(fr29_add(fa0, fr29_mul(vq2, da))));
         st_stream(nS + t, fr29_canon_pack<3>(fr29_add(fs0, fr29_mul(vq2, ds))));
     }
-    const Fr29 fix = fr29_2_271();
-    // round 1
-    {
-        Fr acc[5];
-        Fr29 em29 = fr29_mul(wide29_redc(wx), fix);
-        if (plain) {
-            // The inverses are inverses under the Montgomery product, a (s + beta) = 2^256, and M is such a product:
-            // M - 4 = (a0 - a1) d 2^-261 in this file's 29-bit form.  The small products left 2^-58: 2^-203 is missing.
-            Fr29 two58 = fr29_zero();
-            two58.l[2] = 1;
-            em29 = fr29_mul(em29, two58);
-        }
-        const Fr acc_em = fr29_canon_pack(em29);
-        constexpr uint32_t RINV[8] = {4269129792u, 334977897u, 165441631u, 2876230287u, 1333208682u, 1912866698u, 805346647u, 465471123u};
-        Fr k;
+    // the workgroup's sums: 0 E M, 1 E, 2 .. 4 the rare pairs' terms, 5 .. 7 the second round's, 8 .. 11 the quarters of the inverses
+    __shared__ uint32_t raw[TPB / 64][12][RAW_LIMBS];
+    const uint32_t wv = threadIdx.x >> 6, k = threadIdx.x;
+    raw_put(wx, raw[wv][0]);
+    raw_put(se, raw[wv][1]);
 #pragma unroll
-        for (int l = 0; l < 8; ++l) k.v[l] = RINV[l];
-        const Fr one = mont_mul(sum9_residue(se), k), two = add(one, one), four = plain ? big_zero<8>() : add(two, two);      // plain: acc_em is the sum of E (M - 4) already
-        Fr c0s, c1s, c2s;
+    for (int c = 0; c < 3; ++c) {
+        Fr x;
 #pragma unroll
-        for (int l = 0; l < 8; ++l) { c0s.v[l] = rare[0][l][threadIdx.x]; c1s.v[l] = rare[1][l][threadIdx.x]; c2s.v[l] = rare[2][l][threadIdx.x]; }
-        acc[0] = add(c0s, one);
-        acc[1] = add(c1s, sub(acc_em, four));
-        acc[2] = add(c2s, sub(four, acc_em));
-        acc[3] = add(qsum_residue(0), qsum_residue(1));
-        acc[4] = sub(add(qsum_residue(2), qsum_residue(3)), acc[3]);
-        block_reduce_store<5>(acc, partials);
+        for (int l = 0; l < 8; ++l) x.v[l] = rare[c][l][threadIdx.x];
+        raw_put(fr29_repack(x), raw[wv][2 + c]);
     }
-    // round 2
-    {
-        Fr acc[5];
-        acc[0] = fr29_canon_pack(fr29_mul(t0, fix));
-        acc[2] = fr29_canon_pack(fr29_mul(t2, fix));
-        acc[1] = sub(sub(fr29_canon_pack(fr29_mul(tx, fix)), acc[0]), acc[2]);
-        const Fr r00 = qsum_residue(0), r01 = qsum_residue(1);
-        const Fr sA = add(r00, mont_mul(v1_mont, sub(qsum_residue(2), r00)));      // sum of fa0 over the lane's quads
-        const Fr sB = add(r01, mont_mul(v1_mont, sub(qsum_residue(3), r01)));      // sum of fa1
-        acc[3] = sA;
-        acc[4] = sub(sB, sA);
-        block_reduce_store<5>(acc, partials + 5 * (size_t)gridDim.x);
+    raw_put(t0, raw[wv][5]);
+    raw_put(tx, raw[wv][6]);
+    raw_put(t2, raw[wv][7]);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        uint32_t acc[9];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) acc[l] = qsum[c][l][threadIdx.x];
+        raw_put(acc, raw[wv][8 + c]);
+    }
+    __syncthreads();
+    if (k < 16) {
+        // Round 1: E M 2^-5 summed, 2^-522 2^271 is the factor 2^-256 of the other kernels' products.  A plain table: the inverses are inverses under
+        // the Montgomery product, a (s + beta) = 2^256, and M is such a product: M - 4 = (a0 - a1) d 2^-261 in this file's 29-bit form; the
+        // small products left 2^-58, so 2^-203 is missing: 2^68.  E is in Montgomery form and the sums carry R^-1: sum(E) R^-2 =
+        // sum(E) 2^10 2^-522.  Round 2: E a s 2^-266 summed, 2^532.  The others as they are.
+        Fr29 small = fr29_zero();
+        small.l[0] = k == 1 ? 1 << 10 : 0;
+        small.l[2] = k == 0 ? 1 << 10 : 0;
+        const Fr29 fix = fr29_select(k == 1 || (plain && k == 0), small, fr29_select(k == 0, fr29_2_271(), fr29_select(k >= 5 && k < 8, fr29_2_532(), fr29_2_522())));
+        const Fr x = raw_middle(raw_residue<TPB / 64>(raw[0][k < 12 ? k : 11], 12 * RAW_LIMBS, fix), 5);
+        const Fr em = fr_shfl(x, 0), one = fr_shfl(x, 1), two = add(one, one), four = plain ? big_zero<8>() : add(two, two);      // plain: em is the sum of E (M - 4) already
+        const Fr q0 = fr_shfl(x, 8), q1 = fr_shfl(x, 9), q2 = fr_shfl(x, 10), q3 = fr_shfl(x, 11), s0 = add(q0, q1);
+        const Fr sA = add(q0, mont_mul(v1_mont, sub(q2, q0))), sB = add(q1, mont_mul(v1_mont, sub(q3, q1)));      // sums of fa0 and of fa1
+        const Fr c = fr_shfl(x, (int)(k < 3 ? 2 + k : (k < 8 ? k : 7)));
+        const Fr o = k == 0 ? add(c, one) : (k == 1 ? add(c, sub(em, four)) : (k == 2 ? add(c, sub(four, em)) : (k == 3 ? s0 : (k == 4 ? sub(add(q2, q3), s0) :
+                     (k < 8 ? c : (k == 8 ? sA : sub(sB, sA)))))));
+        if (k < 10) partials[(size_t)k * gridDim.x + blockIdx.x] = o;
     }
 }
 
@@ -1140,8 +1179,7 @@ k_hadamard_round(Fr* __restrict__ partials, const PtrPack<K> p, const Fr* __rest
 
 // k_hadamard_round<2> for rounds of many pairs with the arithmetic in 29-bit limbs, as k_lookup_round29 does it: the weight
 // arrives as E 2^256, e x0 and e dx come out as E x0 / 32 and E dx / 32, the three sums of products stay unreduced, are
-// reduced once per lane (2^-261 again) and brought to standard form by 2^271 (2^-261 once more: R^-1 in all) and R^2.
-// Same inputs, same outputs (folded tensors canonical).  At most 256 pairs per lane: the launch site checks.
+// reduced once per workgroup (2^-522) and brought to standard form by 2^527.  Same inputs, same outputs (folded tensors canonical).  At most 256 pairs per lane: the launch site checks.
 __global__ void __launch_bounds__(TPB) k_hadamard_round29(Fr* __restrict__ partials, Fr* __restrict__ nX, Fr* __restrict__ nY, const Fr* __restrict__ X, const Fr* __restrict__ Y,
                                                           const Fr* __restrict__ E, const Fr v_mont, size_t n_out, Fr* __restrict__ nE) {
     const Fr29 vq = fr29_mul(fr29_repack(v_mont), fr29_2_266());      // v 2^261
@@ -1161,15 +1199,13 @@ __global__ void __launch_bounds__(TPB) k_hadamard_round29(Fr* __restrict__ parti
         nX[t] = fr29_canon_pack(fr29_add(x0, fr29_mul(vq, dx)));
         nY[t] = fr29_canon_pack(fr29_add(y0, fr29_mul(vq, dy)));
     }
-    Fr acc[3];
-    const Fr29 fix = fr29_2_271();
-    acc[0] = fr29_canon_pack(fr29_mul(wide29_redc(w0), fix));
-    acc[2] = fr29_canon_pack(fr29_mul(wide29_redc(w2), fix));
-    acc[1] = sub(sub(fr29_canon_pack(fr29_mul(wide29_redc(wx), fix)), acc[0]), acc[2]);
-    const Fr r2 = big_r2<8>();
-#pragma unroll
-    for (int j = 0; j < 3; ++j) acc[j] = mont_mul(acc[j], r2);
-    block_reduce_store<3>(acc, partials);
+    __shared__ uint32_t raw[TPB / 64][3][RAW_LIMBS];
+    const uint32_t wv = threadIdx.x >> 6, k = threadIdx.x;
+    raw_put(w0, raw[wv][0]);
+    raw_put(wx, raw[wv][1]);
+    raw_put(w2, raw[wv][2]);
+    __syncthreads();
+    if (k < 3) partials[(size_t)k * gridDim.x + blockIdx.x] = raw_middle(raw_residue<TPB / 64>(raw[0][k], 3 * RAW_LIMBS, fr29_2_527()), 0);
 }
 
 // The first round for two tensors given by their int32 forms (the mapped outputs of a softmax's segments): 4 bytes per
@@ -2763,11 +2799,11 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
             fin_rounds = rounds;
             break;
         }
-        if (r == 0 && !phase2 && fuse_first && hs->hint_ints && limbs29() && two_rounds_on() && n1 >= 2 && rounds >= 2 && (half >> 1) > (size_t)SPLIT_HALF &&
-            (half >> 1) <= (size_t)256 * reduce_grid(half >> 1) * TPB) {
+        if (r == 0 && !phase2 && fuse_first && (hs->hint_ints || hs->fr_queries) && limbs29() && two_rounds_on() && n1 >= 2 && rounds >= 2 && (half >> 1) > (size_t)SPLIT_HALF &&
+            (half >> 1) <= (size_t)256 * resident_grid(half >> 1) * TPB) {
             // queries in int32 form, two large phase-1 rounds ahead: both in one pass (k_lookup_first2_29)
             const size_t h2 = half >> 1;
-            const unsigned nb2 = reduce_grid(h2);
+            const unsigned nb2 = resident_grid(h2);
             Scratch& nx2 = job.arena.add(sizeof(Fr) * h2 * 2);
             if (nx2.rc) return nx2.rc;
             Fr* w2 = nx2.as<Fr>();
@@ -2788,16 +2824,18 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
                 ZK_HIP(hipEventCreate(&t1));
                 ZK_HIP(hipEventRecord(t0, st));
             }
-            if (hs->sout_ints) hipLaunchKernelGGL(k_lookup_first2_29<false>, dim3(nb2), dim3(TPB), 0, st, part.as<Fr>(), w2, w2 + h2, cE, b, vm, cs, h2, nE3, *hs);
-            else hipLaunchKernelGGL(k_lookup_first2_29<true>, dim3(nb2), dim3(TPB), 0, st, part.as<Fr>(), w2, w2 + h2, cE, b, vm, cs, h2, nE3, *hs);
+#define FIRST2(PLAIN, FRQ) hipLaunchKernelGGL((k_lookup_first2_29<PLAIN, FRQ>), dim3(nb2), dim3(TPB), 0, st, part.as<Fr>(), w2, w2 + h2, cE, b, vm, cs, h2, nE3, *hs)
+            if (hs->fr_queries) { if (hs->sout_ints) FIRST2(false, true); else FIRST2(true, true); }
+            else { if (hs->sout_ints) FIRST2(false, false); else FIRST2(true, false); }
+#undef FIRST2
             if (g_round_timer.on) {
                 ZK_HIP(hipEventRecord(t1, st));
                 std::lock_guard<std::mutex> lk(g_round_timer.mu);
                 g_round_timer.ev.emplace_back(t0, t1);
                 g_round_timer.pairs += half;
-                // per quad: four queries in int32 form (and their outputs where those are read), two eq weights, two folded values
+                // per quad: four queries (in int32 form, or as field elements; and their outputs' int32 form where it is read), two eq weights, two folded values
                 // written, half a share of the next table (two more weights read, one written)
-                const double q = (hs->sout_ints && !hs->trusted_out) ? 32.0 : 16.0;
+                const double q = (hs->fr_queries ? 128.0 : 16.0) + (hs->sout_ints && !hs->trusted_out ? 16.0 : 0.0);
                 g_round_timer.bytes += (double)h2 * (q + 64.0 + 64.0 + (nE3 ? 48.0 : 0.0));
             }
             ZK_LAUNCH_CHECK();
@@ -2815,11 +2853,10 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         Scratch& nx = job.arena.add(sizeof(Fr) * half * (phase2 ? 5 : 2));
         if (nx.rc) return nx.rc;
         Fr* w = nx.as<Fr>();
-        // A lane ends with a fixed tail -- its unreduced sums reduced, the workgroup's tree over five or eleven sums: what two to three
-        // pairs cost -- so a one-lane-per-pair round with a pair or two per lane pays it per pair.  Those rounds (not the first, whose
-        // grid the fused passes choose) take fewer lanes: eight pairs a lane in phase 1, four in phase 2, where the round has them.
+        // A lane ends with a fixed tail, its sums added up over the workgroup: what a pair costs.  Rounds of few pairs (not the first, whose grid the
+        // fused passes choose) take fewer lanes: four pairs a lane in phase 1, two in phase 2, where the round has them.
         unsigned nb = reduce_grid(half);
-        if (!(r == 0 && fuse_first)) nb = round_grid(half, phase2 ? 4 : 8);
+        if (!(r == 0 && fuse_first)) nb = round_grid(half, phase2 ? 2 : 4);
         const Fr vm = to_mont(load_fr(v + 8 * r));
         // the next round's eq table is written by this round's kernel (ping-pong between two buffers of the job)
         Fr* nE = nullptr;
@@ -2846,8 +2883,9 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
                 ZK_HIP(hipEventCreate(&t1));
                 ZK_HIP(hipEventRecord(t0, st));
             }
-            if (hs->hint_ints && limbs29() && half <= (size_t)512 * nb * TPB)      // queries in int32 form: the common pair in 29-bit limbs
-                hipLaunchKernelGGL(k_lookup_first29, dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, cE, b, vm, half, nE, *hs);
+            const bool wide_ok = limbs29() && half <= (size_t)512 * nb * TPB;      // the common pair in 29-bit limbs
+            if (hs->hint_ints && wide_ok) hipLaunchKernelGGL(k_lookup_first29<false>, dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, cE, b, vm, half, nE, *hs);
+            else if (hs->fr_queries && wide_ok) hipLaunchKernelGGL(k_lookup_first29<true>, dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, cE, b, vm, half, nE, *hs);
             else
                 hipLaunchKernelGGL((k_lookup_round<false, true>), dim3(nb), dim3(TPB), 0, st, part.as<Fr>(), w, w + half, (Fr*)nullptr, (Fr*)nullptr, (Fr*)nullptr, (const Fr*)nullptr, cS,
                                    (const Fr*)nullptr, (const Fr*)nullptr, (const Fr*)nullptr, cE, b, vm, half, nE, *hs);
@@ -2859,7 +2897,8 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
                 // per pair: two queries (32 B each; a mapping table's query is two tensors), the eq weight (32 B), two folded values
                 // written (64 B), the next round's eq table (16 B)
                 // (queries read from their int32 forms: 4 B each)
-                const double q = hs->hint_ints ? ((hs->sout_ints && !hs->trusted_out) ? 16.0 : 8.0) : (hs->S_out ? 128.0 : 64.0);      // (trusted outputs are not read)
+                const double out_ints = hs->sout_ints && !hs->trusted_out ? 8.0 : 0.0;      // (trusted outputs are not read)
+                const double q = hs->hint_ints ? 8.0 + out_ints : (hs->fr_queries ? 64.0 + out_ints : (hs->S_out ? 128.0 : 64.0));
                 g_round_timer.bytes += (double)half * (q + 32.0 + 64.0 + (nE ? 16.0 : 0.0));
             }
         }
@@ -2959,7 +2998,7 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
         Scratch& nx = job.arena.add(sizeof(Fr) * half * K);
         if (nx.rc) return nx.rc;
         Fr* w = nx.as<Fr>();
-        const unsigned nb = reduce_grid(half);
+        const unsigned nb = K == 2 ? resident_grid(half) : reduce_grid(half);
         const Fr vm = to_mont(load_fr(v + 8 * r));
         Fr* nE = nullptr;
         if (r + 1 < rounds && job.eq_scale.empty()) {      // (with eq_scale every round reads the first table's prefix)
@@ -3123,7 +3162,7 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     if (rc) return rc;
     if (ints) {
         const FoldPrepared *q = (const FoldPrepared*)ints->queries, *o = (const FoldPrepared*)ints->out, *mp = (const FoldPrepared*)ints->mapped;
-        ZK_ARG(q != nullptr && q->n == D, "lookup sumcheck: the queries' int32 form has another size");
+        ZK_ARG(q == nullptr ? S_out != nullptr : q->n == D, "lookup sumcheck: the queries' int32 form has another size");
         ZK_ARG(!S_out || (o != nullptr && o->n == D && mp != nullptr && mp->n == N), "lookup sumcheck: a mapping table's int32 forms are missing or of another size");
     }
     SumJob* job = new SumJob;
@@ -3143,10 +3182,14 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     Scratch& B = job->arena.add(sizeof(Fr) * N);
     Scratch& dp = job->arena.add(sizeof(Fr) * batch_inv_grid(N));
     Scratch& TB = job->arena.add(hint ? sizeof(Fr) * 2 * N : 1);
-    Scratch& want = job->arena.add(hint && ints ? sizeof(int32_t) * (N + 1) : 1);         // the last slot: n_ok
+    // The queries as integers: their int32 forms, or, where the first round is the fused one, read off the field elements by it (a mapping
+    // table then needs the outputs' and its own int32 forms beside them).
+    const bool fr_queries = hint && zk_lookup_ints_suffice(D, N) && (ints ? ints->queries == nullptr : (!S_out && S == hint));
+    const bool by_ints = fr_queries || (hint && ints && ints->queries);
+    Scratch& want = job->arena.add(by_ints ? sizeof(int32_t) * (N + 1) : 1);         // the last slot: n_ok
     for (const Scratch* x : {&B, &dp, &TB, &want})
         if (x->rc) return x->rc;
-    uint32_t* const n_ok = hint && ints ? (uint32_t*)(want.as<int32_t>() + N) : nullptr;
+    uint32_t* const n_ok = by_ints ? (uint32_t*)(want.as<int32_t>() + N) : nullptr;
     // ZKLLM_LOOKUP_TRUSTED=0: no entry counts as checked and no output as gathered from the table -- every query goes
     // through its own comparison (to compare the two paths)
     static const bool trust = [] { const char* e = getenv("ZKLLM_LOOKUP_TRUSTED"); return !(e && e[0] == '0'); }();
@@ -3160,17 +3203,20 @@ static int lookup_prove_begin(void** handle, const void* S, const void* T, const
     if (rc == 0 && hint) {
         hs.TB = TB.as<Fr>(); hs.hint = (const Fr*)hint; hs.low = fr_from_i64((int64_t)low); hs.beta = b; hs.N = (uint32_t)N;
         if (S_out) { hs.S_out = (const Fr*)S_out; hs.r_mont = to_mont(r_val); }
-        if (ints) {
+        if (by_ints) {
             const int32_t* mi = S_out ? ((const FoldPrepared*)ints->mapped)->ints : nullptr;
             hipLaunchKernelGGL(k_lookup_ints_check, dim3(cdiv(N, TPB)), dim3(TPB), 0, st, want.as<int32_t>(), n_ok, TB.as<Fr>(), mi, hs.r_mont, low, (uint32_t)N);
             hs.n_ok = n_ok;
-            job->fin.word = n_ok;
-            job->n_table = (uint32_t)N;
-            if (S_out) {
+            hs.fr_queries = fr_queries;
+            if (!fr_queries) {
+                job->fin.word = n_ok;
+                job->n_table = (uint32_t)N;
+            }
+            if (S_out && !fr_queries) {
                 const FoldPrepared *q = (const FoldPrepared*)ints->queries, *o = (const FoldPrepared*)ints->out, *mp = (const FoldPrepared*)ints->mapped;
                 hs.trusted_out = trust && o->src_queries != 0 && o->src_queries == q->id && o->src_table == mp->id && o->src_low == low;
             }
-            hs.hint_ints = ((const FoldPrepared*)ints->queries)->ints;
+            if (!fr_queries) hs.hint_ints = ((const FoldPrepared*)ints->queries)->ints;
             hs.sout_ints = S_out ? ((const FoldPrepared*)ints->out)->ints : nullptr;
             hs.want = want.as<int32_t>();
             hs.low_int = low;
@@ -3212,6 +3258,16 @@ int zk_lookup_prove_begin_mapped(void** handle, const void* S_in, const void* S_
                                  const uint32_t* u_eq, const uint32_t* v, size_t D, size_t N, int rounds, void* stv) {
     ZK_ARG(S_in != nullptr && S_out != nullptr && r != nullptr, "zk_lookup_prove_begin_mapped: null queries or challenge");
     return lookup_prove_begin(handle, nullptr, T, m, S_in, low, beta, u_eq, v, D, N, rounds, stv, S_out, r);
+}
+// zk_lookup_prove_begin_mapped with the int32 forms of the outputs and of the mapped values, where the queries have none: the first round takes the
+// queries' integers from the field elements
+int zk_lookup_prove_begin_mapped_out_ints(void** handle, const void* S_in, const void* S_out, const void* S_out_prepared, const void* mapped_prepared, const uint32_t* r, const void* T,
+                                          const void* m, int32_t low, const uint32_t* beta, const uint32_t* u_eq, const uint32_t* v, size_t D, size_t N, int rounds, void* stv) {
+    ZK_ARG(S_in != nullptr && S_out != nullptr && r != nullptr, "zk_lookup_prove_begin_mapped_out_ints: null queries or challenge");
+    ZK_ARG(S_out_prepared != nullptr && mapped_prepared != nullptr, "zk_lookup_prove_begin_mapped_out_ints: null int32 form");
+    LookupInts li;
+    li.out = S_out_prepared; li.mapped = mapped_prepared;
+    return lookup_prove_begin(handle, nullptr, T, m, S_in, low, beta, u_eq, v, D, N, rounds, stv, S_out, r, &li);
 }
 // 1 when a job of this shape takes its queries from their int32 forms alone (its first round is the fused one): the
 // field-element tensor given beside them is then never read

@@ -142,6 +142,9 @@ static LookupPending sumcheck_begin(const FrTensor& S0, const FrTensor& T0, cons
     if (S_out && qi && oi && mapped_ints)
         ZKC(zk_lookup_prove_begin_mapped_ints(&p.handle, S0.gpu_data, qi, S_out->gpu_data, oi, mapped_ints, r->val, T0.gpu_data, m0.gpu_data, low, beta.val, u[0].val, vs[0].val,
                                               D, N, (int)k, nullptr));
+    else if (S_out && oi && mapped_ints)
+        ZKC(zk_lookup_prove_begin_mapped_out_ints(&p.handle, S0.gpu_data, S_out->gpu_data, oi, mapped_ints, r->val, T0.gpu_data, m0.gpu_data, low, beta.val, u[0].val, vs[0].val,
+                                                  D, N, (int)k, nullptr));
     else if (S_out) ZKC(zk_lookup_prove_begin_mapped(&p.handle, S0.gpu_data, S_out->gpu_data, r->val, T0.gpu_data, m0.gpu_data, low, beta.val, u[0].val, vs[0].val, D, N, (int)k, nullptr));
     else if (hint == &S0 && qi)
         ZKC(zk_lookup_prove_begin_hinted_ints(&p.handle, S0.gpu_data, qi, T0.gpu_data, m0.gpu_data, low, beta.val, u[0].val, vs[0].val, D, N, (int)k, nullptr));
@@ -244,19 +247,19 @@ LookupPending tLookupRangeMapping::prove_begin(const FrTensor& S_in, const FrTen
     if (D != (1u << ceilLog2(D))) {
         // pad the queries with the first table entry and account for them in m[0] (tlookup.cu:502-510)
         const uint Dp = 1u << ceilLog2(D);
-        // Queries that keep int32 forms are padded in that form; where the job reads nothing else (zk_lookup_ints_suffice) the
+        // Queries and outputs that keep int32 forms are padded in that form; where the job reads nothing else (zk_lookup_ints_suffice) the
         // padded field elements are not written at all.
-        const bool ints = S_in.kept_ints() && S_out.kept_ints() && mapped_vals.kept_ints();
-        const bool ints_only = ints && zk_lookup_ints_suffice(Dp, table.size);
-        auto padded = [&](const FrTensor& t, const FrTensor& fill_from, const void* fill_ints) {
+        const bool out_ints = S_out.kept_ints() && mapped_vals.kept_ints(), in_ints = out_ints && S_in.kept_ints();
+        const bool suffice = zk_lookup_ints_suffice(Dp, table.size) != 0;
+        auto padded = [&](const FrTensor& t, const FrTensor& fill_from, bool ints, const void* fill_ints) {
             FrTensor* p = new FrTensor(Dp);
             keep.emplace_back(p);
-            if (!ints_only) ZKC(zk_fr_pad_from(p->gpu_data, t.gpu_data, D, Dp, fill_from.gpu_data, nullptr));
+            if (!(ints && suffice)) ZKC(zk_fr_pad_from(p->gpu_data, t.gpu_data, D, Dp, fill_from.gpu_data, nullptr));
             if (ints) ZKC(zk_i32_pad_from(p->ints_for_producer(), zk_fr_fold_prepared_ints(t.kept_ints()), D, Dp, fill_ints, low, nullptr));
             return p;
         };
-        si = padded(S_in, table, nullptr);          // the first table entry is low
-        so = padded(S_out, mapped_vals, ints ? zk_fr_fold_prepared_ints(mapped_vals.kept_ints()) : nullptr);
+        si = padded(S_in, table, in_ints, nullptr);          // the first table entry is low
+        so = padded(S_out, mapped_vals, out_ints, out_ints ? zk_fr_fold_prepared_ints(mapped_vals.kept_ints()) : nullptr);
         keep.emplace_back(new FrTensor(m));
         FrTensor* m_ = keep.back().get();
         const Fr_t more{{Dp - D, 0, 0, 0, 0, 0, 0, 0}};
