@@ -1345,7 +1345,7 @@ template <int K> __device__ __forceinline__ void tail_block_sum(Fr (&acc)[K], Fr
 // coefficients (da s0 + a0 ds and the like) are a1 s1 - a0 s0 - da ds.
 // What binds: instruction issue of the sixteen waves on one compute unit while a round has 64 pairs, the chain of two products
 // below.  These rounds took 17 us each in a workgroup that gave a pair's products to four lanes, 14 us each as launches.
-static constexpr int RM_ROUNDS = 8, RM_P = 1 << RM_ROUNDS, RM_W = 12, RM_ROWS = 16, RM_GROUPS = 4;      // RM_W: words of an element in LDS (rows of sixteen read without conflicts)
+static constexpr int RM_ROUNDS = 8, RM_P = 1 << RM_ROUNDS, RM_W = 12, RM_ROWS = 16, RM_GROUPS = 4, RM_WIDE_ROUNDS = 3;      // RM_W: words of an element in LDS (rows of sixteen read without conflicts)
 static constexpr size_t RM_MAX_N = (size_t)1 << 17;      // elements from which on a sumcheck's rounds run in such launches
 struct RoundsArgs {
     const Fr *A, *S, *B, *T, *m, *E;
@@ -1356,13 +1356,13 @@ struct RoundsArgs {
     uint32_t fold_e, e_span;              // fold_e: E is this round's table alone and is summed down from round to round; e_span: its first round's is E[t] + E[t + e_span]
     uint32_t off[RM_ROUNDS];              // where round r's partial sums start
 };
-template <bool PHASE2> __global__ void __launch_bounds__(1024)
+template <bool PHASE2, int GROUPS> __global__ void __launch_bounds__(256 * GROUPS)
 k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
-    constexpr int NT = PHASE2 ? 5 : 2;
-    __shared__ int32_t X0[NT][RM_P][RM_W], X1[NT][RM_P / 2][RM_W], XE[RM_P / 2][RM_W];
-    __shared__ uint32_t raw[RM_ROUNDS][RM_GROUPS][RM_ROWS][9];
+    constexpr int NT = PHASE2 ? 5 : 2, PM = RM_P / RM_GROUPS * GROUPS, MAXR = GROUPS == RM_GROUPS ? RM_ROUNDS : RM_WIDE_ROUNDS;
+    __shared__ int32_t X0[NT][PM][RM_W], X1[NT][PM / 2][RM_W], XE[PM / 2][RM_W];
+    __shared__ uint32_t raw[MAXR][GROUPS][RM_ROWS][9];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave & 3u, group = wave >> 2;
-    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u, T = 1024u;
+    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u, T = 256u * GROUPS;
     const uint32_t nb = gridDim.x, c = 1u << a.log_c;
     // neighbouring workgroups read neighbouring elements of the same lines: keep them on one die (workgroups go to the eight dies in turn)
     const uint32_t blk = (nb & 7u) == 0 ? (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
@@ -1384,7 +1384,7 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
             if (a.e_span) e = add(e, a.E[g + a.e_span]);
             rm_put(XE[s], fr29_repack(e));
         }
-        for (uint32_t i = threadIdx.x; i < RM_ROUNDS * RM_GROUPS * RM_ROWS * 9; i += T) (&raw[0][0][0][0])[i] = 0u;
+        for (uint32_t i = threadIdx.x; i < MAXR * GROUPS * RM_ROWS * 9; i += T) (&raw[0][0][0][0])[i] = 0u;
     }
     __syncthreads();
     for (uint32_t r = 0; r < a.rounds; ++r) {
@@ -1392,13 +1392,13 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
         const uint32_t half = P >> (r + 1);
         int32_t* const src = odd ? &X1[0][0][0] : &X0[0][0][0];
         int32_t* const dst = odd ? &X0[0][0][0] : &X1[0][0][0];
-        const uint32_t ss = (odd ? RM_P / 2 : RM_P) * RM_W, ds = (odd ? RM_P : RM_P / 2) * RM_W;
+        const uint32_t ss = (odd ? PM / 2 : PM) * RM_W, ds = (odd ? PM : PM / 2) * RM_W;
         auto rd = [&](uint32_t k, uint32_t slot) { return rm_get(src + k * ss + slot * RM_W); };
         if (group * 16u < half && (phase2 || !(kind & 1u))) {
             uint32_t acc[9];
 #pragma unroll
             for (int l = 0; l < 9; ++l) acc[l] = 0;
-            for (uint32_t t0 = group * 16u; t0 < half; t0 += 16u * RM_GROUPS) {
+            for (uint32_t t0 = group * 16u; t0 < half; t0 += 16u * GROUPS) {
                 const uint32_t t = t0 + ln;
                 const bool live = t < half;
                 const uint32_t ta = live ? t : 0u, tb = ta + half;
@@ -1440,35 +1440,48 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
     }
     // the sums with the factors the other round kernels leave on them: a product of two elements carries 2^-261 here, another with E = e 2^256
     // leaves e x y 2^-266; the sums of E's products are e x y 2^-256 there (k_hadamard_round: no factor), of m b 2^-256, of a alone as they are
+    // Every sum's residue on a lane of its own, then the middle coefficients and the differences from the neighbours' in LDS.
     const uint32_t per = a.hadamard ? 3u : (PHASE2 ? 11u : 5u);
+    __shared__ uint32_t res[MAXR * 11][8];
     for (uint32_t i = threadIdx.x; i < per * a.rounds; i += T) {
         const uint32_t r = i / per, k = i % per;
         if (!a.hadamard && k >= 5 && r < a.phase2_from) continue;
-        auto sum = [&](uint32_t role, const Fr29& fix) {
-            uint32_t l9[9];
+        // the sums' rows of sixteen lanes: 0 1 2 | 8 9 | 4 5 6 | 12 13 14, the middle of three being x1 y1
+        const uint32_t role = k < 3 ? k : (k < 5 ? 5u + k : (k < 8 ? k - 1u : 4u + k));
+        uint32_t l9[9];
 #pragma unroll
-            for (int l = 0; l < 9; ++l) l9[l] = raw[r][0][role][l] + raw[r][1][role][l] + raw[r][2][role][l] + raw[r][3][role][l];
-            fr29_carry_u(l9);
-            Fr29 x;
+        for (int l = 0; l < 9; ++l) {
+            l9[l] = raw[r][0][role][l];
 #pragma unroll
-            for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
-            return fr29_canon_pack<5>(fr29_mul(x, fix));
-        };
-        Fr o;
-        if (k == 3 || k == 4) {
-            o = sum(8, fr29_2_261());
-            if (k == 4) o = sub(sum(9, fr29_2_261()), o);
-        } else {
-            const uint32_t base = k < 3 ? 0u : (k < 8 ? 4u : 12u), which = k < 3 ? k : (k < 8 ? k - 5 : k - 8);
-            const Fr29 fix = k >= 8 ? fr29_2_266() : (a.hadamard ? fr29_2_527() : fr29_2_271());
-            o = sum(base + (which == 0 ? 0u : (which == 2 ? 2u : 1u)), fix);
-            if (which == 1) o = sub(sub(o, sum(base, fix)), sum(base + 2, fix));
+            for (int g = 1; g < GROUPS; ++g) l9[l] += raw[r][g][role][l];
         }
+        fr29_carry_u(l9);
+        Fr29 x;
+#pragma unroll
+        for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+        const Fr29 fix = fr29_select(k == 3 || k == 4, fr29_2_261(), fr29_select(k >= 8, fr29_2_266(), fr29_select(a.hadamard != 0, fr29_2_527(), fr29_2_271())));
+        const Fr o = fr29_canon_pack<3>(fr29_mul(x, fix));          // up to 128 pairs of values below 1.07 r: below 3 r
+#pragma unroll
+        for (int l = 0; l < 8; ++l) res[i][l] = o.v[l];
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < per * a.rounds; i += T) {
+        const uint32_t r = i / per, k = i % per;
+        if (!a.hadamard && k >= 5 && r < a.phase2_from) continue;
+        auto at = [&](uint32_t q) {
+            Fr x;
+#pragma unroll
+            for (int l = 0; l < 8; ++l) x.v[l] = res[q][l];
+            return x;
+        };
+        Fr o = at(i);
+        if (k == 1 || k == 6 || k == 9) o = sub(sub(o, at(i - 1)), at(i + 1));
+        else if (k == 4) o = sub(o, at(i - 1));
         partials[(size_t)a.off[r] + (size_t)k * nb + blockIdx.x] = o;
     }
     if (a.nA) {
         const int32_t* const fin = (a.rounds & 1u) ? &X1[0][0][0] : &X0[0][0][0];
-        const uint32_t fs = ((a.rounds & 1u) ? RM_P / 2 : RM_P) * RM_W, nt = PHASE2 && a.phase2_from < a.rounds ? 5u : 2u;
+        const uint32_t fs = ((a.rounds & 1u) ? PM / 2 : PM) * RM_W, nt = PHASE2 && a.phase2_from < a.rounds ? 5u : 2u;
         for (uint32_t i = threadIdx.x; i < nt * c; i += T) {
             const uint32_t k = i >> a.log_c, s = i & (c - 1);
             Fr* d = k == 0 ? a.nA : (k == 1 ? a.nS : (k == 2 ? a.nB : (k == 3 ? a.nT : a.nm)));
@@ -2695,8 +2708,9 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
         // a full one: three rounds then; all that the workgroup's elements allow, evenly split over the launches, where each has a unit
         // of its own.
         const int left = rounds - r;
-        int R = std::min(3, left);
+        int R = std::min(RM_WIDE_ROUNDS, left), P = RM_P / RM_GROUPS;
         if (n <= (size_t)256 * RM_P) {
+            P = RM_P;
             const int launches = (left + RM_ROUNDS - 1) / RM_ROUNDS;
             R = (left + launches - 1) / launches;
         }
@@ -2704,7 +2718,7 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
         memset(&a, 0, sizeof(a));
         a.rounds = (uint32_t)R;
         a.nlow = (uint32_t)(n >> R);
-        while (((size_t)2 << (a.log_c + R)) <= (size_t)RM_P && (2u << a.log_c) <= a.nlow) ++a.log_c;
+        while (((size_t)2 << (a.log_c + R)) <= (size_t)P && (2u << a.log_c) <= a.nlow) ++a.log_c;
         const uint32_t nb = a.nlow >> a.log_c;
         a.A = A; a.S = S; a.B = B; a.T = T; a.m = m; a.E = E;
         a.beta = fr29_repack(beta);
@@ -2726,8 +2740,13 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
             if (nx.rc) return nx.rc;
             a.nA = nx.as<Fr>(); a.nS = a.nA + o; a.nB = a.nS + o; a.nT = a.nB + o; a.nm = a.nT + o; a.nE = a.nm + o;
         }
-        if (phase2) hipLaunchKernelGGL(k_sum_rounds<true>, dim3(nb), dim3(1024), 0, job.st, part_all, a);
-        else hipLaunchKernelGGL(k_sum_rounds<false>, dim3(nb), dim3(1024), 0, job.st, part_all, a);
+        if (P < RM_P) {
+            if (phase2) hipLaunchKernelGGL((k_sum_rounds<true, 1>), dim3(nb), dim3(256), 0, job.st, part_all, a);
+            else hipLaunchKernelGGL((k_sum_rounds<false, 1>), dim3(nb), dim3(256), 0, job.st, part_all, a);
+        } else {
+            if (phase2) hipLaunchKernelGGL((k_sum_rounds<true, RM_GROUPS>), dim3(nb), dim3(256 * RM_GROUPS), 0, job.st, part_all, a);
+            else hipLaunchKernelGGL((k_sum_rounds<false, RM_GROUPS>), dim3(nb), dim3(256 * RM_GROUPS), 0, job.st, part_all, a);
+        }
         ZK_LAUNCH_CHECK();
         A = a.nA; S = a.nS;
         if (phase2) { B = a.nB; T = a.nT; m = a.nm; }
@@ -2737,8 +2756,8 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
     }
     return 0;
 }
-// partial sums that rounds_queue may need for the rounds of n elements: a workgroup holds 128 pairs of a launch's first round where there are as many
-static size_t rounds_partials(size_t n, int rounds, uint32_t k) { return (size_t)rounds * k * (n / RM_P + 1); }
+// partial sums that rounds_queue may need for the rounds of n elements: a workgroup holds 32 pairs of a launch's first round where there are as many
+static size_t rounds_partials(size_t n, int rounds, uint32_t k) { return (size_t)rounds * k * (n / (RM_P / RM_GROUPS) + 1); }
 static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& b, const uint32_t* v, size_t D, size_t N, int rounds,
                         const HintSrc* hs = nullptr) {
     hipStream_t st = job.st;
