@@ -453,13 +453,15 @@ __global__ void __launch_bounds__(256) k_batch_inv(Fr* __restrict__ out, const F
     }
     if (ride.m) block_reduce_store<1>(dot, ride.dot);
 }
-static inline bool batch_inv_narrow(size_t n) { return n <= (size_t)1 << 18; }
-static inline unsigned batch_inv_grid(size_t n) { return cdiv(n, batch_inv_narrow(n) ? 512 : 2048); }
+// values a lane: few while that leaves the chip at two waves a SIMD or less (the launch then takes what one lane takes, and a lane's products
+// are part of it: 2^16 entries 42 us with two, 36 with one)
+static inline unsigned batch_inv_chunk(size_t n) { return n <= (size_t)1 << 16 ? 1u : (n <= (size_t)1 << 18 ? 2u : 8u); }
+static inline unsigned batch_inv_grid(size_t n) { return cdiv(n, 256 * batch_inv_chunk(n)); }
 // queues out = 1 / (in + beta) on st
 static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, hipStream_t st, const InvRiders& ride = InvRiders{nullptr, nullptr, nullptr, nullptr, 0}) {
     if (n == 0) return 0;
-    // few values a lane while that leaves the chip at two waves a SIMD or less: the launch then takes what one lane takes
-    if (batch_inv_narrow(n)) hipLaunchKernelGGL(k_batch_inv<2>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
+    if (batch_inv_chunk(n) == 1) hipLaunchKernelGGL(k_batch_inv<1>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
+    else if (batch_inv_chunk(n) == 2) hipLaunchKernelGGL(k_batch_inv<2>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
     else hipLaunchKernelGGL(k_batch_inv<8>, dim3(batch_inv_grid(n)), dim3(256), 0, st, out, in, beta, n, ride);
     ZK_LAUNCH_CHECK();
     return 0;
