@@ -71,6 +71,8 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_,
         p.rem = padded;
     }
     p.m.reset(new FrTensor(tl_rem.prep_inside(*p.rem)));          // remainders of a division by the table's length
+    // the lookup's job first: its kernels wait for what is queued here so far, and the evaluations below run beside them
+    p.look = tl_rem.prove_begin(*p.rem, *p.m, rand_temp[0], rand_temp[1], u, v);
     // X_(u) and rem(u) in one pass over the two tensors (the padding of the remainders is zeros: the unpadded tensor has the same
     // extension and the others' length).  X = scaling_factor X_ + rem element by element, so X(u) is that combination of the two
     // values: X itself, 32 bytes an element, is read only with ZKLLM_CHECK_CLAIMS=1, which evaluates it and compares as
@@ -81,13 +83,12 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_,
         const vector<Fr_t> ev = FrTensor::me_batch({&X_, rem_tensor_ptr, &X}, u);
         p.lhs = ev[0] * Fr_t({scaling_factor, 0, 0, 0, 0, 0, 0, 0}) + ev[1];
         if (p.lhs != ev[2]) throw std::runtime_error("Error: the rem is not correct.");
-    } else {          // the values are collected with the proof: nothing waits for them before the lookup's job is queued
+    } else {          // the values are collected with the proof: nothing waits for them here
         p.evaluated.begin();
         try { (void)FrTensor::me_batch({&X_, rem_tensor_ptr}, u); } catch (...) { p.evaluated.end(); throw; }
         p.evaluated.end();
         p.scaling_factor = scaling_factor;
     }
-    p.look = tl_rem.prove_begin(*p.rem, *p.m, rand_temp[0], rand_temp[1], u, v);
     return p;
 }
 void Rescaling::prove_end(Pending& p) {
