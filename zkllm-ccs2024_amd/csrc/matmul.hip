@@ -375,34 +375,29 @@ template <typename T> static int run_int_path(void* C, const void* A, const void
 
 // ---- int8-plane path: digit planes and a GEMM on the matrix cores ------------------------------------------------------
 // Balanced base-256 digits of a small signed integer: x = sum_j d_j 256^j, d_j in [-128, 127].  Both operands are laid
-// out with the contraction index fastest and padded with zeros to a multiple of the GEMM's K tile:
-//   planes of A[b][m][k]:  PA[((b * pa + i) * M + m) * Kp + k]
-//   planes of B[b][k][p]:  PB[((b * pb + j) * P + p) * Kp + k]      (transposed on the way)
-// so that every operand fragment of the matrix instruction is 16 consecutive bytes.
+// out as planes of rows along the contraction index, padded with zeros to a multiple of the GEMM's K tile Kp, A[b][m][k] in rows m of the
+// planes b * pa + i and B[b][k][p], transposed on the way, in rows p of the planes b * pb + j.  A plane stands in blocks of 32 contraction
+// bytes of all its rows (plane_at): every operand fragment of the matrix instruction is 16 consecutive bytes, and the 32 rows of a step
+// that a wave brings to LDS at once are 1 KB in one piece.
+__host__ __device__ __forceinline__ size_t plane_at(size_t rows, size_t row, uint32_t k) { return ((size_t)(k >> 5) * rows + row) * 32 + (k & 31u); }
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
-static constexpr int GBM = 128, GBN = 128, GBK = 128;      // block tile of the GEMM: 4 waves, 64 x 64 outputs each
+static constexpr int GBM = 128, GBN = 128, GBK = 128;      // block tile of the pair-by-pair GEMM: 4 waves, 64 x 64 outputs each
 static constexpr int GLD = GBK + 16;                       // LDS row stride in bytes: 16-byte aligned rows whose 16-byte reads spread over all banks
 
 // src: the operand as a product of int32 forms when src.a is set (a is then not read)
 __global__ void __launch_bounds__(256) k_split_rows(int8_t* __restrict__ planes, const Fr* __restrict__ a, const ProdSrc src, size_t rows, uint32_t M, uint32_t N, uint32_t Kp, int np) {
-    const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const uint32_t groups = Kp / 4;
-    // 32-bit divisions where the launch has fewer than 2^32 lanes (the same for every lane; rows is below 2^31): a 64-bit
-    // division costs more than forming a plane's four digits
-    size_t row;
-    uint32_t k;
-    if (rows * (size_t)groups <= 0xFFFFFFFFull) {
-        const uint32_t g32 = (uint32_t)gid, r32 = g32 / groups;
-        row = r32;
-        k = 4 * (g32 - r32 * groups);
-    } else {
-        row = gid / groups;
-        k = 4 * (uint32_t)(gid % groups);
-    }
-    if (row >= rows) return;
-    const uint32_t b32 = (uint32_t)row / M;
-    const size_t b = b32, m = (uint32_t)row - b32 * M;
+    // lanes in the order of the words that they write: eight to a row's 32 bytes, then the rows, then the blocks of 32.  32-bit divisions
+    // where the launch has fewer than 2^32 lanes (the same for every lane): a 64-bit division costs more than forming a plane's four digits
+    const size_t gid = (size_t)blockIdx.x * 256 + threadIdx.x, r = gid >> 3;
+    if (r >= rows * (size_t)(Kp / 32)) return;
+    const uint32_t blocks = Kp / 32;
+    size_t at;                                  // the matrix of the stack times its blocks, plus the block
+    uint32_t m;
+    if (rows * (size_t)Kp <= 0xFFFFFFFFull) { const uint32_t q = (uint32_t)r / M; m = (uint32_t)r - q * M; at = q; }
+    else { at = r / M; m = (uint32_t)(r % M); }
+    const size_t b = (uint32_t)at / blocks, row = b * M + m;
+    const uint32_t k = ((uint32_t)at - (uint32_t)b * blocks) * 32 + 4 * ((uint32_t)gid & 7u);
     long long x[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) x[e] = (k + e < N) ? (src.a ? prod_at(src, row * N + k + e) : fr_to_i64(a[row * N + k + e])) : 0ll;
@@ -414,7 +409,7 @@ __global__ void __launch_bounds__(256) k_split_rows(int8_t* __restrict__ planes,
             x[e] = (x[e] - d) >> 8;
             packed |= (uint32_t)(uint8_t)d << (8 * e);
         }
-        *reinterpret_cast<uint32_t*>(planes + ((b * np + j) * M + m) * Kp + k) = packed;
+        *reinterpret_cast<uint32_t*>(planes + (b * np + j) * M * (size_t)Kp + plane_at(M, m, k)) = packed;
     }
 }
 // grid (P tiles of 64, K tiles of 64, batch): a 64 x 64 tile of B goes through LDS so that reads run along p and writes along k
@@ -436,7 +431,7 @@ __global__ void __launch_bounds__(256) k_split_cols(int8_t* __restrict__ planes,
     const uint32_t row = t >> 2, ch = t & 3;
     if (p0 + row < P)
         for (int j = 0; j < np; ++j)
-            *reinterpret_cast<v4i*>(planes + ((b * np + j) * P + p0 + row) * Kp + k0 + ch * 16) = *reinterpret_cast<const v4i*>(&tile[j][row][ch * 16]);
+            *reinterpret_cast<v4i*>(planes + (b * np + j) * P * (size_t)Kp + plane_at(P, p0 + row, k0 + ch * 16)) = *reinterpret_cast<const v4i*>(&tile[j][row][ch * 16]);
 }
 
 // Both operands examined and split in one pass over each: their first four planes -- all there are of 32-bit integers -- and the figures
@@ -463,6 +458,7 @@ __device__ __forceinline__ uint32_t digit_bytes(unsigned long long mag, bool neg
     const uint32_t x = negative ? 0u - (uint32_t)mag : (uint32_t)mag;
     return (x + 0x80808080u) ^ 0x80808080u;
 }
+static constexpr int EX_ROW = 4;      // elements a lane of A has on their way at once
 __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
     __shared__ uint32_t tile[4][64][17];
     __shared__ unsigned long long red[4];
@@ -474,14 +470,15 @@ __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
         if (row >= g.rowsA) return;
         const Fr* src = g.A + (size_t)row * g.N;
         const uint32_t b = row / g.M, m = row - b * g.M, q = lane & 3u, sel = ((4u + q) << 8) | q;
-        int8_t* dst = g.pA + ((size_t)(b * 4 + q) * g.M + m) * g.Kp;
+        int8_t* dst = g.pA + (size_t)(b * 4 + q) * g.M * g.Kp + plane_at(g.M, m, lane & ~3u);      // 64 further along k: 64 M bytes
         unsigned long long mx = 0, sum = 0;
-        for (uint32_t k0 = 0; k0 < g.Kp; k0 += 128) {
-            Fr x[2];
+        for (uint32_t k0 = 0; k0 < g.Kp; k0 += 64 * EX_ROW) {
+            Fr x[EX_ROW];
 #pragma unroll
-            for (int i = 0; i < 2; ++i) x[i] = k0 + 64 * i + lane < g.N ? src[k0 + 64 * i + lane] : big_zero<8>();
+            for (int i = 0; i < EX_ROW; ++i) x[i] = k0 + 64 * i + lane < g.N ? src[k0 + 64 * i + lane] : big_zero<8>();
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < EX_ROW; ++i) {
+                if (k0 + 64 * i >= g.Kp) break;
                 bool ng;
                 const unsigned long long v = fr_magnitude(x[i], ng);
                 mx = v > mx ? v : mx;
@@ -490,7 +487,7 @@ __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
                 const uint32_t w0 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x00, 0xF, 0xF, false), w1 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0x55, 0xF, 0xF, false);
                 const uint32_t w2 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xAA, 0xF, 0xF, false), w3 = (uint32_t)__builtin_amdgcn_update_dpp(0, w, 0xFF, 0xF, 0xF, false);
                 const uint32_t lo = __builtin_amdgcn_perm(w1, w0, sel), hi = __builtin_amdgcn_perm(w3, w2, sel);
-                *reinterpret_cast<uint32_t*>(dst + k0 + 64 * i + (lane & ~3u)) = (lo & 0xFFFFu) | (hi << 16);
+                *reinterpret_cast<uint32_t*>(dst + (size_t)(k0 / 64 + i) * g.M * 64) = (lo & 0xFFFFu) | (hi << 16);
             }
         }
 #pragma unroll
@@ -545,7 +542,7 @@ __global__ void __launch_bounds__(256) k_examine_split(const ExamineArgs g) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const v4i v = {(int)tile[j][row][4 * ch], (int)tile[j][row][4 * ch + 1], (int)tile[j][row][4 * ch + 2], (int)tile[j][row][4 * ch + 3]};
-            *reinterpret_cast<v4i*>(g.pB + ((size_t)(b * 4 + j) * g.P + p0 + row) * g.Kp + k0 + 16 * ch) = v;
+            *reinterpret_cast<v4i*>(g.pB + (size_t)(b * 4 + j) * g.P * g.Kp + plane_at(g.P, p0 + row, k0 + 16 * ch)) = v;
         }
 }
 
@@ -591,8 +588,8 @@ __global__ void __launch_bounds__(256) k_gemm_i8_planes(const PlaneGemm g) {
                 for (int q = 0; q < 4; ++q) {
                     const uint32_t c = t + 256 * q, row = c >> 3, kc = c & 7;
                     const v4i zero = {0, 0, 0, 0};
-                    ra[q] = (m0 + row < g.M) ? *reinterpret_cast<const v4i*>(Ai + (size_t)(m0 + row) * g.Kp + k0 + kc * 16) : zero;
-                    rb[q] = (n0 + row < g.P) ? *reinterpret_cast<const v4i*>(Bj + (size_t)(n0 + row) * g.Kp + k0 + kc * 16) : zero;
+                    ra[q] = (m0 + row < g.M) ? *reinterpret_cast<const v4i*>(Ai + plane_at(g.M, m0 + row, k0 + kc * 16)) : zero;
+                    rb[q] = (n0 + row < g.P) ? *reinterpret_cast<const v4i*>(Bj + plane_at(g.P, n0 + row, k0 + kc * 16)) : zero;
                 }
             };
             fetch(0);
@@ -640,88 +637,150 @@ __global__ void __launch_bounds__(256) k_gemm_i8_planes(const PlaneGemm g) {
 // are multiplied while a K tile lies in LDS, pairs of equal weight 256^(i+j) into one int32 accumulator (at most min(PA, PB) pairs
 // of at most K * 2^14 each; the caller keeps min(PA, PB) K below 2^17), and the int64 recombination happens once, in the epilogue.
 // Against the pair-by-pair kernel: one pass over the operands instead of PA * PB, PA * PB times the matrix instructions per
-// barrier, no int64 totals held through the loop.  Block tile 64 x 64, one 32 x 32 tile per wave, two blocks per CU.
-template <int PA, int PB> __global__ void __launch_bounds__(256, 2) k_gemm_i8_planes_all(const PlaneGemm g) {
-    constexpr int NS = PA + PB - 1, TB = 64;
-    __shared__ __attribute__((aligned(16))) int8_t sA[PA][TB * GLD];
-    __shared__ __attribute__((aligned(16))) int8_t sB[PB][TB * GLD];
-    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6, wm = wave >> 1, wn = wave & 1;
-    const uint32_t m0 = blockIdx.y * TB, n0 = blockIdx.x * TB;
+// barrier, no int64 totals held through the loop.
+// Block tile 64 x TN, a wave 32 x TN / 2, two blocks a CU.  TN = 128: a wave's seven fragments of three and two planes serve twelve matrix
+// instructions, and a tile is read for twice the outputs; TN = 64 for more accumulators than that leaves registers for, and for
+// products of few tiles.  Steps of 32 contraction bytes, one matrix instruction a pair of fragments, go from memory to LDS without passing through
+// registers, three steps ahead in four buffers: a step takes a CU's two blocks half a microsecond, less than an L2 under this load takes
+// to answer.  A wave brings the step's 32-row pieces wave, wave + 4, ... (the last one again where they do not come out even: every wave then has
+// as many loads on their way, and "all but the last two steps'" is a constant).  The two 16-byte halves of a row change places every
+// eight rows (the source addresses do: a direct load writes LDS in lane order), so that the fragments' reads spread over all banks.
+// 2048 x 4096 by 4096 x 4096, three planes by two: 251 us with tiles of 64 x 64 through registers, 225 so; the matrix units alone, on
+// random bytes, 129 us (3.2 POP/s: what the card's power allows them), the loads alone 123 (17 TB/s out of the L2), the 268 MB of results 48,
+// which two blocks that run in step do not hide.
+static constexpr int GKT = 32, GBUF = 4;
+__device__ __forceinline__ uint32_t gemm_half(uint32_t row, uint32_t h) { return h ^ ((row >> 3) & 1u); }
+__device__ __forceinline__ void load_to_lds(const int8_t* src, int8_t* dst) {       // 16 bytes a lane, dst: the wave's first byte
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint32_t*)src, (__attribute__((address_space(3))) uint32_t*)dst, 16, 0, 0);
+}
+template <int PA, int PB, int TN> __global__ void __launch_bounds__(256, 2) k_gemm_i8_planes_all(const PlaneGemm g) {
+    constexpr int NS = PA + PB - 1, TM = 64, NT = TN / 64, PIECES = 2 * PA + 2 * NT * PB, SHARE = (PIECES + 3) / 4, BYTES = (PA * TM + PB * TN) * GKT;      // NT: a wave's 32 x 32 tiles
+    // a variable a buffer: the compiler waits for a direct load before every read of the variable that it writes
+    __shared__ __attribute__((aligned(16))) int8_t s0[BYTES], s1[BYTES], s2[BYTES], s3[BYTES];
+    const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), wm = wave >> 1, wn = wave & 1;
+    // Workgroups go to the eight dies in turn: a die takes a run of tiles in groups of eight rows of them, which share operands in its L2
+    uint32_t tm = blockIdx.y, tn = blockIdx.x;
+    {
+        const uint32_t nx = gridDim.x, ny = gridDim.y, total = nx * ny, id = blockIdx.y * nx + blockIdx.x;
+        if ((total & 7u) == 0 && total >= 64) {
+            const uint32_t lin = (id & 7u) * (total >> 3) + (id >> 3), group = lin / (8 * nx), first = group * 8, rows = ny - first < 8 ? ny - first : 8u, in = lin - group * 8 * nx;
+            tm = first + in % rows;
+            tn = in / rows;
+        }
+    }
+    const uint32_t m0 = tm * TM, n0 = tn * TN;
     const size_t b = blockIdx.z;
-    const int8_t* __restrict__ A0 = g.A + (b * g.sa * g.M) * (size_t)g.Kp;
-    const int8_t* __restrict__ B0 = g.B + (b * g.sb * g.P) * (size_t)g.Kp;
-    const size_t a_plane = (size_t)g.M * g.Kp, b_plane = (size_t)g.P * g.Kp;
-    v16i acc[NS];
+    v16i acc[NS][NT];
 #pragma unroll
     for (int s = 0; s < NS; ++s)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[s][r] = 0;
-    v4i ra[PA][2], rb[PB][2];
-    auto fetch = [&](uint32_t k0) {
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const uint32_t c = t + 256 * q, row = c >> 3, kc = c & 7;
-            const v4i zero = {0, 0, 0, 0};
-            const bool in_a = m0 + row < g.M, in_b = n0 + row < g.P;
-            const size_t oa = (size_t)(m0 + row) * g.Kp + k0 + kc * 16, ob = (size_t)(n0 + row) * g.Kp + k0 + kc * 16;
+            for (int r = 0; r < 16; ++r) acc[s][q][r] = 0;
+    // The wave's pieces: 32 rows of a plane each, A's planes' two and then B's 2 NT a plane.  Rows beyond the matrix read its last one (their outputs are
+    // not stored).
+    const int8_t* src[SHARE];
+    uint32_t dst[SHARE];
+    size_t step[SHARE];
 #pragma unroll
-            for (int i = 0; i < PA; ++i) ra[i][q] = in_a ? *reinterpret_cast<const v4i*>(A0 + i * a_plane + oa) : zero;
+    for (int q = 0; q < SHARE; ++q) {
+        const uint32_t c = min(wave + 4 * q, (uint32_t)PIECES - 1), lr = lane >> 1;
+        const bool in_a = c < 2 * PA;
+        const uint32_t cb = in_a ? 0u : c - 2 * PA, plane = in_a ? c >> 1 : cb / (2 * NT), r = (in_a ? (c & 1u) : cb % (2 * NT)) * 32 + lr;
+        const uint32_t rows = in_a ? g.M : g.P, at = (in_a ? m0 : n0) + r;
+        const int8_t* base = in_a ? g.A + (b * g.sa + plane) * g.M * (size_t)g.Kp : g.B + (b * g.sb + plane) * g.P * (size_t)g.Kp;
+        src[q] = base + (size_t)(at < rows ? at : rows - 1) * GKT + gemm_half(r, lane & 1u) * 16;
+        dst[q] = (in_a ? plane * TM : PA * TM + plane * TN) * GKT + (r - lr) * GKT;
+        step[q] = (size_t)rows * GKT;
+    }
+    const uint32_t rowA = wm * 32 + (lane & 31), rowB = wn * 32 * NT + (lane & 31), half = lane >> 5, steps = g.Kp / GKT;
+    uint32_t fetched = 0;
+    auto fetch = [&](int8_t* buf) {                            // the next step; behind the last one that again, into buffers nobody reads any more
 #pragma unroll
-            for (int j = 0; j < PB; ++j) rb[j][q] = in_b ? *reinterpret_cast<const v4i*>(B0 + j * b_plane + ob) : zero;
-        }
+        for (int q = 0; q < SHARE; ++q) load_to_lds(src[q], buf + dst[q]);
+        ++fetched;
+#pragma unroll
+        for (int q = 0; q < SHARE; ++q) src[q] += fetched < steps ? step[q] : 0;
     };
-    fetch(0);
-    for (uint32_t k0 = 0; k0 < g.Kp; k0 += GBK) {
-        __syncthreads();                    // every wave is done with the previous tile
+    auto multiply = [&](const int8_t* buf) {
+        v4i fa[PA], fb[PB][NT];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const uint32_t c = t + 256 * q, row = c >> 3, kc = c & 7;
+        for (int i = 0; i < PA; ++i) fa[i] = *reinterpret_cast<const v4i*>(buf + (i * TM + rowA) * GKT + gemm_half(rowA, half) * 16);
 #pragma unroll
-            for (int i = 0; i < PA; ++i) *reinterpret_cast<v4i*>(&sA[i][row * GLD + kc * 16]) = ra[i][q];
+        for (int j = 0; j < PB; ++j)
 #pragma unroll
-            for (int j = 0; j < PB; ++j) *reinterpret_cast<v4i*>(&sB[j][row * GLD + kc * 16]) = rb[j][q];
-        }
-        __syncthreads();
-        if (k0 + GBK < g.Kp) fetch(k0 + GBK);
+            for (int q = 0; q < NT; ++q) fb[j][q] = *reinterpret_cast<const v4i*>(buf + (PA * TM + j * TN + rowB + 32 * q) * GKT + gemm_half(rowB + 32 * q, half) * 16);
 #pragma unroll
-        for (int ks = 0; ks < GBK / 32; ++ks) {
-            const uint32_t ko = ks * 32 + 16 * (lane >> 5);
-            v4i fa[PA], fb[PB];
+        for (int i = 0; i < PA; ++i)
 #pragma unroll
-            for (int i = 0; i < PA; ++i) fa[i] = *reinterpret_cast<const v4i*>(&sA[i][(wm * 32 + (lane & 31)) * GLD + ko]);
+            for (int j = 0; j < PB; ++j)
 #pragma unroll
-            for (int j = 0; j < PB; ++j) fb[j] = *reinterpret_cast<const v4i*>(&sB[j][(wn * 32 + (lane & 31)) * GLD + ko]);
-#pragma unroll
-            for (int i = 0; i < PA; ++i)
-#pragma unroll
-                for (int j = 0; j < PB; ++j) acc[i + j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j], acc[i + j], 0, 0, 0);
-        }
+                for (int q = 0; q < NT; ++q) acc[i + j][q] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[j][q], acc[i + j][q], 0, 0, 0);
+    };
+    // The wave's share of the oldest step is in LDS when no more than the two younger ones' loads are on their way; behind the barrier everybody's is,
+    // and everybody has read the buffer of the step before (lgkmcnt 0), which the next fetch fills.
+    auto arrived = [&] {
+        constexpr int YOUNGER = 2 * SHARE;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt((YOUNGER & 15) | (YOUNGER >> 4) << 14 | 7 << 4);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    fetch(s0);
+    fetch(s1);
+    fetch(s2);
+    for (uint32_t t = 0; t < steps; t += GBUF) {               // Kp is a multiple of 128
+        arrived();
+        fetch(s3);
+        multiply(s0);
+        arrived();
+        fetch(s0);
+        multiply(s1);
+        arrived();
+        fetch(s1);
+        multiply(s2);
+        arrived();
+        fetch(s2);
+        multiply(s3);
     }
+    __builtin_amdgcn_s_waitcnt(7 << 4 | 15 << 8);              // vmcnt 0: no load into LDS outlives the workgroup
+    asm volatile("" ::: "memory");
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        unsigned long long v = 0;
+    for (int q = 0; q < NT; ++q)
 #pragma unroll
-        for (int s = 0; s < NS && s < 8; ++s) v += (unsigned long long)(long long)acc[s][r] << (8 * s);
-        const uint32_t row = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const uint32_t col = n0 + wn * 32 + (lane & 31);
-        if (row < g.M && col < g.P) gemm_store(g, (b * g.M + row) * (size_t)g.P + col, (long long)v);
-    }
+        for (int r = 0; r < 16; ++r) {
+            unsigned long long v = 0;
+#pragma unroll
+            for (int s = 0; s < NS && s < 8; ++s) v += (unsigned long long)(long long)acc[s][q][r] << (8 * s);
+            const uint32_t row = m0 + wm * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
+            const uint32_t col = n0 + (wn * NT + q) * 32 + (lane & 31);
+            if (row < g.M && col < g.P) gemm_store(g, (b * g.M + row) * (size_t)g.P + col, (long long)v);
+        }
 }
-template <int PA> static bool launch_gemm_all_b(int pb, dim3 grid, hipStream_t st, const PlaneGemm& g) {
+template <int PA, int PB> static void launch_gemm_all_n(uint32_t batch, hipStream_t st, const PlaneGemm& g) {
+    // tiles of 128 columns where there are enough of them for two a CU
+    if constexpr (PA + PB <= 6)
+        if ((size_t)cdiv(g.P, 128) * cdiv(g.M, 64) * batch >= 512) {
+            hipLaunchKernelGGL((k_gemm_i8_planes_all<PA, PB, 128>), dim3(cdiv(g.P, 128), cdiv(g.M, 64), batch), dim3(256), 0, st, g);
+            return;
+        }
+    hipLaunchKernelGGL((k_gemm_i8_planes_all<PA, PB, 64>), dim3(cdiv(g.P, 64), cdiv(g.M, 64), batch), dim3(256), 0, st, g);
+}
+template <int PA> static bool launch_gemm_all_b(int pb, uint32_t batch, hipStream_t st, const PlaneGemm& g) {
     switch (pb) {
-        case 1: hipLaunchKernelGGL((k_gemm_i8_planes_all<PA, 1>), grid, dim3(256), 0, st, g); return true;
-        case 2: hipLaunchKernelGGL((k_gemm_i8_planes_all<PA, 2>), grid, dim3(256), 0, st, g); return true;
-        case 3: hipLaunchKernelGGL((k_gemm_i8_planes_all<PA, 3>), grid, dim3(256), 0, st, g); return true;
+        case 1: launch_gemm_all_n<PA, 1>(batch, st, g); return true;
+        case 2: launch_gemm_all_n<PA, 2>(batch, st, g); return true;
+        case 3: launch_gemm_all_n<PA, 3>(batch, st, g); return true;
         default: return false;
     }
 }
-static bool launch_gemm_all(int pa, int pb, dim3 grid, hipStream_t st, const PlaneGemm& g) {
+static bool launch_gemm_all(int pa, int pb, uint32_t batch, hipStream_t st, const PlaneGemm& g) {
     switch (pa) {
-        case 1: return launch_gemm_all_b<1>(pb, grid, st, g);
-        case 2: return launch_gemm_all_b<2>(pb, grid, st, g);
-        case 3: return launch_gemm_all_b<3>(pb, grid, st, g);
-        case 4: return launch_gemm_all_b<4>(pb, grid, st, g);
-        case 5: return launch_gemm_all_b<5>(pb, grid, st, g);
+        case 1: return launch_gemm_all_b<1>(pb, batch, st, g);
+        case 2: return launch_gemm_all_b<2>(pb, batch, st, g);
+        case 3: return launch_gemm_all_b<3>(pb, batch, st, g);
+        case 4: return launch_gemm_all_b<4>(pb, batch, st, g);
+        case 5: return launch_gemm_all_b<5>(pb, batch, st, g);
         default: return false;
     }
 }
@@ -775,7 +834,7 @@ static int run_int8_plane_path(void* C, const void* A, const void* B, uint32_t b
         ZK_HIP(hipEventRecord(t0, st));
     }
     // up to five planes by three, the sums of the pairs of equal weight within int32: every pair in one pass; else pair by pair
-    const bool all_pairs = pa <= 5 && pb <= 3 && (unsigned long long)std::min(pa, pb) * N < (1ull << 17) && launch_gemm_all(pa, pb, dim3(cdiv(P, 64), cdiv(M, 64), batch), st, g);
+    const bool all_pairs = pa <= 5 && pb <= 3 && (unsigned long long)std::min(pa, pb) * N < (1ull << 17) && launch_gemm_all(pa, pb, batch, st, g);
     if (!all_pairs) hipLaunchKernelGGL(k_gemm_i8_planes, dim3(cdiv(P, GBN), cdiv(M, GBM), batch), dim3(256), 0, st, g);
     if (g_gemm_timer.on) {
         ZK_HIP(hipEventRecord(t1, st));
