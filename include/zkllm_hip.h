@@ -55,7 +55,7 @@ int zk_shutdown(void);
 int zk_set_async_jobs(int on);
 int zk_async_jobs(void);
 /* No counterpart in the reference.  Deferred results: between zk_defer_begin and zk_defer_end (same host thread), the entry points
- * that hand a few field elements back to the host -- zk_fr_me, zk_fr_me_multi(_ints), zk_ip_round, zk_ip_sumcheck_small -- queue
+ * that hand a few field elements back to the host -- zk_fr_me, zk_fr_me_multi(_ints), zk_ip_round, zk_ip_sumcheck_small, zk_matmul_sumcheck -- queue
  * their kernels and the copy of their results and return WITHOUT waiting and WITHOUT writing their host output arguments;
  * zk_defer_end records an event on `stream` (the stream those calls were given) and zk_defer_wait waits for it and writes every
  * result, in the order of the calls and with each call's own layout, to out_host (n_fr: how many field elements; at most 2048
@@ -219,6 +219,12 @@ int zk_ip_round(uint32_t* poly3_host, const void* a, const void* b, size_t n_in,
 int zk_ip_round_stacked(uint32_t* poly3_host, const void* a, const void* b, const void* E, size_t D, size_t rows_in, size_t rows_out, void* stream);
 /* all rounds of zkip (zkfc.cu:140-151) in one launch, n <= 8192 */
 int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a, const void* b, uint32_t n, const uint32_t* u, int k, void* stream);
+/* The device side of zkFC::prove (zkfc.cu:61-87) for Y [B][O] = X [B][D] W [D][O]: claim = Y at (u_batch, u_output); X folded at u_batch and W
+ * at u_output; every round of zkip on the two vectors (3 kd coefficients); the folded values, which are X and W at the proof's point.
+ * Field for field what zk_fr_fold_axis_all, zk_fr_me and zk_ip_sumcheck_small give.  2^(k-1) < n <= 2^k on every axis; kb and
+ * ko at most 14, kd 1 to 13.  While results are deferred it delivers 3 kd + 3 elements in the order of its arguments. */
+int zk_matmul_sumcheck(uint32_t* claim_host, uint32_t* polys_host, uint32_t* fin_host, const void* X, const void* W, const void* Y, uint32_t B, uint32_t D, uint32_t O,
+                       const uint32_t* u_batch, int kb, const uint32_t* u_input, int kd, const uint32_t* u_output, int ko, void* stream);
 
 /* ---- G1 tensors (g1-tensor.cu) ------------------------------------------------------------------------ */
 int zk_g1_fill(void* out, const uint32_t* point36, size_t n, void* stream);               /* G1Jacobian_assign_broadcast :140 */

@@ -394,6 +394,37 @@ def test_deferred_results_arrive_in_call_order_with_the_values_of_the_immediate_
         hip.free(p)
 
 
+# the batch and output axes at the line of nine challenges (tables in the arguments, or in memory), at one and four waves for two rows, with one and several
+# parts of X; the inner axis at one launch of rounds and two
+@pytest.mark.parametrize("B,D,O", [(1, 2, 1), (1, 3, 2), (2, 256, 33), (16, 64, 64), (63, 257, 511), (65, 100, 512), (512, 130, 512), (512, 5, 513), (513, 70, 5), (300, 1000, 700), (1, 8192, 520),
+                                   (1025, 65, 1), (2049, 2, 1000), (16384, 3, 3), (2, 4, 16384)])
+def test_the_sumcheck_of_a_matrix_product_equals_its_separate_steps(hip, B, D, O):
+    """zk_matmul_sumcheck on any three tensors (Y need not be the product): the values of zk_fr_fold_axis_all, zk_fr_me and zk_ip_sumcheck_small."""
+    sz, i = ctypes.c_size_t, ctypes.c_int
+    kb, kd, ko = ((n - 1).bit_length() for n in (B, D, O))
+    X, W, Y = (mt_random_vec(np.random.RandomState(B + s), n) for s, n in enumerate((B * D, D * O, B * O)))
+    X[: len(X) // 2] = fr_array([R_MOD - 1])
+    u_b, u_i, u_o = (mt_random_vec(np.random.RandomState(40 + s), max(k, 1)) for s, k in enumerate((kb, kd, ko)))
+    dX, dW, dY, xf, wf, yf = (hip.upload(t) for t in (X, W, Y, X[:1].repeat(D, 0), X[:1].repeat(D, 0), X[:1].repeat(B, 0)))
+
+    def fold(out, t, u, k, other, cur, win):
+        if k == 0:
+            return t
+        hip.call("zk_fr_fold_axis_all", ctypes.c_void_p(out), ctypes.c_void_p(t), u, i(k), sz(other), ctypes.c_uint32(cur), sz(win), None)
+        return out
+
+    want = [np.zeros((n, 8), np.uint32) for n in (1, 3 * kd, 2)]
+    hip.call("zk_fr_me", want[0], ctypes.c_void_p(fold(yf, dY, u_o, ko, B, O, 1)), sz(B), u_b, i(kb), None)
+    a, b = fold(xf, dX, u_b, kb, 1, B, D), fold(wf, dW, u_o, ko, D, O, 1)
+    hip.call("zk_ip_sumcheck_small", want[1], want[2], ctypes.c_void_p(a), ctypes.c_void_p(b), ctypes.c_uint32(D), u_i, i(kd), None)
+    got = [np.zeros((n, 8), np.uint32) for n in (1, 3 * kd, 2)]
+    hip.call("zk_matmul_sumcheck", *got, *(ctypes.c_void_p(t) for t in (dX, dW, dY)), *(ctypes.c_uint32(n) for n in (B, D, O)), u_b, i(kb), u_i, i(kd), u_o, i(ko), None)
+    for g, w in zip(got, want):
+        assert (g == w).all()
+    for p in (dX, dW, dY, xf, wf, yf):
+        hip.free(p)
+
+
 def test_row_sums_of_squares_in_double_follow_a_plain_loop():
     """zk_row_sumsq_f64 must round exactly as `for j: acc += (x[j] / scale) ** 2` does: Python floats are IEEE doubles and
     every operation involved is exactly rounded, so the device result is compared bit for bit."""

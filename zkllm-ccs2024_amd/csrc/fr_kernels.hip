@@ -280,26 +280,44 @@ template <bool SOA> __global__ void __launch_bounds__(TPB) k_eq29(int32_t* __res
     for (int l = 0; l < 9; ++l) out[SOA ? (size_t)l * n + i : (size_t)i * 9 + l] = e.l[l];
 }
 // innermost axis: out[row] = sum_p E[p] in[row][p].  WPR waves take two rows (an entry of the table serves both), 64 terms a lane at most
-template <int WPR> __global__ void __launch_bounds__(TPB)
-k_fold_rows(Fr* __restrict__ out, const Fr* __restrict__ in, const int32_t* __restrict__ E, size_t rows, uint32_t cur) {
-    __shared__ uint32_t red[2][4][9];
+struct EqSoa {
+    const int32_t* E;
+    uint32_t n;
+    __device__ __forceinline__ Fr29 operator()(uint32_t i) const {
+        Fr29 e;
+#pragma unroll
+        for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)l * n + i];
+        return e;
+    }
+};
+struct EqAos {
+    const int32_t* E;
+    __device__ __forceinline__ Fr29 operator()(uint32_t i) const {
+        Fr29 e;
+#pragma unroll
+        for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)i * 9 + l];
+        return e;
+    }
+};
+using FoldRowsLds = uint32_t[2][4][9];
+template <class EQ> __device__ __forceinline__ void
+fold_rows_block(FoldRowsLds& red, Fr* __restrict__ out, const Fr* __restrict__ in, const EQ& eq, size_t rows, uint32_t cur, const uint32_t wpr, uint32_t block) {
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    const size_t r0 = ((size_t)blockIdx.x * (4 / WPR) + wave / WPR) * 2;
+    const size_t r0 = ((size_t)block * (4 / wpr) + wave / wpr) * 2;
     const size_t ra = r0 < rows ? r0 : rows - 1, rb = r0 + 1 < rows ? r0 + 1 : rows - 1;
     const Fr *pa = in + ra * cur, *pb = in + rb * cur;
     Wide29 wa = wide29_zero(), wb = wide29_zero();
-    uint32_t p = (wave % WPR) * 64u + lane, term = 0;
+    uint32_t p = (wave % wpr) * 64u + lane, term = 0;
     Fr xa = big_zero<8>(), xb = xa;
     Fr29 e = fr29_zero();
     auto fetch = [&](uint32_t q) {
         xa = pa[q]; xb = pb[q];
-#pragma unroll
-        for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)l * cur + q];
+        e = eq(q);
     };
     if (p < cur) fetch(p);
     while (p < cur) {
         const Fr29 a = fr29_repack(xa), b = fr29_repack(xb), ce = e;
-        p += 64u * WPR;
+        p += 64u * wpr;
         if (p < cur) fetch(p);
         wide29_mac(wa, ce, a);
         wide29_mac(wb, ce, b);
@@ -316,15 +334,15 @@ k_fold_rows(Fr* __restrict__ out, const Fr* __restrict__ in, const int32_t* __re
         for (int l = 0; l < 9; ++l) { red[0][wave][l] = l9[0][l]; red[1][wave][l] = l9[1][l]; }
     }
     __syncthreads();
-    if (threadIdx.x < 8 / WPR) {
+    if (threadIdx.x < 8 / wpr) {
         const uint32_t k = threadIdx.x & 1u, g = threadIdx.x >> 1;
-        const size_t row = ((size_t)blockIdx.x * (4 / WPR) + g) * 2 + k;
+        const size_t row = ((size_t)block * (4 / wpr) + g) * 2 + k;
         uint32_t s[9];
 #pragma unroll
         for (int l = 0; l < 9; ++l) {
-            s[l] = red[k][g * WPR][l];
+            s[l] = red[k][g * wpr][l];
 #pragma unroll
-            for (int w = 1; w < WPR; ++w) s[l] += red[k][g * WPR + w][l];
+            for (uint32_t w = 1; w < wpr; ++w) s[l] += red[k][g * wpr + w][l];
         }
         fr29_carry_u(s);
         Fr29 x;
@@ -333,15 +351,21 @@ k_fold_rows(Fr* __restrict__ out, const Fr* __restrict__ in, const int32_t* __re
         if (row < rows) out[row] = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));
     }
 }
+template <int WPR> __global__ void __launch_bounds__(TPB)
+k_fold_rows(Fr* __restrict__ out, const Fr* __restrict__ in, const int32_t* __restrict__ E, size_t rows, uint32_t cur) {
+    __shared__ FoldRowsLds red;
+    fold_rows_block(red, out, in, EqSoa{E, cur}, rows, cur, WPR, blockIdx.x);
+}
 // a middle axis: out[z][w] = sum_j E[j] in[z][j][w].  A lane takes one w and J consecutive j (the table's entry is the same for the
 // whole wave), the four waves of a workgroup 4 J of them; grid (w in groups of 64, 4 J at a time, z)
-__global__ void __launch_bounds__(TPB)
-k_fold_cols(Fr* __restrict__ part, const Fr* __restrict__ in, const int32_t* __restrict__ E, uint32_t cur, size_t window, uint32_t J) {
-    __shared__ uint32_t red[3][9][64];
+using FoldColsLds = uint32_t[3][9][64];
+template <class EQ> __device__ __forceinline__ void
+fold_cols_block(FoldColsLds& red, Fr* __restrict__ part, const Fr* __restrict__ in, const EQ& eq, uint32_t e0, uint32_t cur, size_t window, uint32_t J,
+                uint32_t bx, uint32_t by, uint32_t bz, uint32_t nz) {      // eq's first entry is e0's
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = threadIdx.x & 63u;
-    const size_t w = (size_t)blockIdx.x * 64 + lane, wc = w < window ? w : window - 1;
-    const uint32_t j0 = (blockIdx.y * 4 + wave) * J, j1 = j0 + J < cur ? j0 + J : cur;
-    const Fr* base = in + (size_t)blockIdx.z * cur * window + wc;
+    const size_t w = (size_t)bx * 64 + lane, wc = w < window ? w : window - 1;
+    const uint32_t j0 = (by * 4 + wave) * J, j1 = j0 + J < cur ? j0 + J : cur;
+    const Fr* base = in + (size_t)bz * cur * window + wc;
     Wide29 acc = wide29_zero();
     for (uint32_t j = j0; j < j1; j += 4) {
         Fr x[4];
@@ -350,9 +374,7 @@ k_fold_cols(Fr* __restrict__ part, const Fr* __restrict__ in, const int32_t* __r
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             if (j + q < j1) {
-                Fr29 e;
-#pragma unroll
-                for (int l = 0; l < 9; ++l) e.l[l] = E[(size_t)(j + q) * 9 + l];
+                const Fr29 e = eq(j + q - e0);
                 wide29_mac(acc, e, fr29_repack(x[q]));
             }
         wide29_carry(acc);
@@ -370,7 +392,92 @@ k_fold_cols(Fr* __restrict__ part, const Fr* __restrict__ in, const int32_t* __r
     fr29_carry_u(l9);
 #pragma unroll
     for (int l = 0; l < 9; ++l) s.l[l] = (int32_t)l9[l];
-    if (w < window) part[((size_t)blockIdx.y * gridDim.z + blockIdx.z) * window + w] = fr29_canon_pack<2>(fr29_mul(s, fr29_2_261()));
+    if (w < window) part[((size_t)by * nz + bz) * window + w] = fr29_canon_pack<2>(fr29_mul(s, fr29_2_261()));
+}
+__global__ void __launch_bounds__(TPB)
+k_fold_cols(Fr* __restrict__ part, const Fr* __restrict__ in, const int32_t* __restrict__ E, uint32_t cur, size_t window, uint32_t J) {
+    __shared__ FoldColsLds red;
+    fold_cols_block(red, part, in, EqAos{E}, 0u, cur, window, J, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
+}
+// ---- the folds of a matrix product's proof, Y = X W ---------------------------------------------------------------------------------
+// X over its rows at u_batch (Xf, xchunks parts of it for the reader to add up), W and Y over their columns at u_output (Wf, Yf): they need nothing of
+// one another, and for all but the largest tensors each is a launch that does not fill the chip.  One launch takes the three, one before it
+// both tables of weights; the parts of Xf and the value of Yf at u_batch are left to the sumcheck's launch.  Loads in flight bind
+// it.  300 x 1000 x 2750: 73 us in eight launches, now 36 in two; 2048 x 4096 x 4096: 288 us in nine, now 232.
+// SMALL (u of at most nine bits): the tables' two factors come in the arguments, a workgroup makes the entries that it needs in LDS, and one more
+// leaves the table of u_batch for the reader of Yf.
+struct EqArgs {
+    Fr29 lo[32], hi[16];
+    __device__ __forceinline__ Fr29 operator()(uint32_t i) const { return fr29_canon<2>(fr29_mul(lo[i & 31u], hi[i >> 5])); }
+};
+static constexpr int FC_SMALL_BITS = 9;
+struct FcFolds {
+    const Fr *X, *W, *Y;
+    Fr *Xf, *Wf, *Yf;
+    int32_t *Eb, *Eo;              // u_batch: nine limbs an entry; u_output: an entry's limbs O apart
+    uint32_t B, D, O;
+    uint32_t J, xgroups, xchunks;  // as k_fold_cols
+    uint32_t wwaves, ywaves;       // waves that take two rows of W and Y (1 or 4)
+    uint32_t wblocks, yblocks;     // workgroups: W's, Y's, then X's
+};
+template <bool SMALL> struct FcEq { };
+template <> struct FcEq<true> { EqArgs batch, output; };
+template <bool SMALL> __global__ void __launch_bounds__(TPB) k_fc_folds(const FcFolds a, const FcEq<SMALL> eq) {
+    __shared__ union { FoldRowsLds rows; FoldColsLds cols; } lds;
+    __shared__ int32_t tab[SMALL ? 9 << FC_SMALL_BITS : 1];
+    uint32_t b = blockIdx.x;
+    if (b < a.wblocks + a.yblocks) {
+        const bool w = b < a.wblocks;
+        if (!w) b -= a.wblocks;
+        if constexpr (SMALL) {
+            for (uint32_t i = threadIdx.x; i < a.O; i += TPB) {
+                const Fr29 e = eq.output(i);
+#pragma unroll
+                for (int l = 0; l < 9; ++l) tab[l * a.O + i] = e.l[l];
+            }
+            __syncthreads();
+        }
+        fold_rows_block(lds.rows, w ? a.Wf : a.Yf, w ? a.W : a.Y, EqSoa{SMALL ? (const int32_t*)tab : (const int32_t*)a.Eo, a.O}, w ? a.D : a.B, a.O, w ? a.wwaves : a.ywaves, b);
+        return;
+    }
+    b -= a.wblocks + a.yblocks;
+    const uint32_t by = b / a.xgroups, bx = b - by * a.xgroups;
+    if constexpr (SMALL) {
+        const bool all = by == a.xchunks;                   // the workgroup behind X's
+        const uint32_t j0 = all ? 0u : by * 4 * a.J, n = all ? a.B : (a.B - j0 < 4 * a.J ? a.B - j0 : 4 * a.J);
+        for (uint32_t i = threadIdx.x; i < n; i += TPB) {
+            const Fr29 e = eq.batch(j0 + i);
+#pragma unroll
+            for (int l = 0; l < 9; ++l) (all ? a.Eb : tab)[i * 9 + l] = e.l[l];
+        }
+        if (all) return;
+        __syncthreads();
+        fold_cols_block(lds.cols, a.Xf, a.X, EqAos{tab}, j0, a.B, a.D, a.J, bx, by, 0u, 1u);
+    } else fold_cols_block(lds.cols, a.Xf, a.X, EqAos{a.Eb}, 0u, a.B, a.D, a.J, bx, by, 0u, 1u);
+}
+// both tables in one launch: four factors of at most four bits each
+struct EqTwoTabs { Fr29 t[2][48]; uint32_t n[2]; int bits[2][4]; };
+__global__ void __launch_bounds__(TPB) k_eq29_two(int32_t* __restrict__ Eb, int32_t* __restrict__ Eo, const EqTwoTabs a, uint32_t first) {
+    const uint32_t which = blockIdx.x < first ? 0u : 1u, n = a.n[which];
+    uint32_t i = (blockIdx.x - (which ? first : 0u)) * TPB + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t at = i;
+    uint32_t base = 0;
+    Fr29 e = a.t[which][0];
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        const uint32_t bits = (uint32_t)a.bits[which][f];
+        const Fr29 x = a.t[which][base + (i & ((1u << bits) - 1u))];
+        e = f ? fr29_mul(e, x) : x;
+        i >>= bits;
+        base += 1u << bits;
+    }
+    e = fr29_canon<2>(e);
+#pragma unroll
+    for (int l = 0; l < 9; ++l) {
+        if (which) Eo[(size_t)l * n + at] = e.l[l];
+        else Eb[(size_t)at * 9 + l] = e.l[l];
+    }
 }
 __global__ void __launch_bounds__(TPB) k_sum_partials(Fr* __restrict__ out, const Fr* __restrict__ part, size_t n, uint32_t count) {
     const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
@@ -504,26 +611,66 @@ __global__ void __launch_bounds__(TPB) k_ip_round_w(Fr* __restrict__ partials, c
 // has a lane of its own -- sixteen lanes (a row of the data-parallel adds) do one thing for sixteen pairs:
 //   even waves: a0 b0 | a1 b1 | da db | -         odd waves: fold of a | fold of b | - | -
 // so a round is the latency of one product, a row sum and a barrier: about 2 us.  One workgroup that gave a pair to a lane and
-// summed through LDS took 15 us a round, 93 us for 64 elements and 225 us for 4096.  The middle coefficient is a1 b1 - a0 b0 - da db.
+// summed through LDS took 15 us a round, 93 us for 64 elements and 225 us for 4096.  A further workgroup of the first launch may take an
+// evaluation that nothing here waits for (ip_evaluate).  The middle coefficient is a1 b1 - a0 b0 - da db.
 static constexpr int IP_ROUNDS = 8, IP_P = 1 << IP_ROUNDS, IP_W = 12, IP_GROUPS = 8;      // IP_GROUPS: pairs of waves, sixteen pairs each
 struct IpArgs {
     const Fr *a, *b;
-    Fr *na, *nb;                  // the folded vectors, gridDim.x elements each
+    Fr *na, *nb;                  // the folded vectors, nlow elements each
     Fr29 v[IP_ROUNDS];            // in round order, times 2^261
     uint32_t n, nlow, rounds;     // the vectors' length (zeros behind it), low indices, rounds of this launch
-    Fr* sums;                     // round r's q-th sum at sums[(3 r + q) gridDim.x + workgroup]
+    Fr* sums;                     // round r's q-th sum at sums[(3 r + q) nlow + workgroup]
     const Fr* prev; Fr* prev_out; // the sums of a launch before: prev_count times prev_nb of them
     uint32_t prev_nb, prev_count;
+    uint32_t a_parts;             // a is the sum of so many vectors, one behind the other
+    const Fr* ev; const int32_t* ev_E; Fr* ev_out;      // for a workgroup more than nlow: sum_i ev_E[i] ev[i], i < ev_n
+    uint32_t ev_n;
 };
+__device__ __forceinline__ void ip_evaluate(uint32_t (&red)[3][9], const IpArgs& a) {      // 256 lanes, at most 64 terms each
+    const uint32_t t = threadIdx.x;
+    Wide29 acc = wide29_zero();
+    uint32_t term = 0;
+    if (t < 256u)
+        for (uint32_t i = t; i < a.ev_n; i += 256u) {
+            wide29_mac(acc, EqAos{a.ev_E}(i), fr29_repack(a.ev[i]));
+            if ((++term & 3u) == 0) wide29_carry(acc);
+        }
+    const Fr29 s = fr29_canon<2>(wide29_redc(acc));
+    uint32_t l9[9];
+#pragma unroll
+    for (int l = 0; l < 9; ++l) l9[l] = (uint32_t)s.l[l];
+    fr29_wave_sum(l9);
+    if ((t & 63u) == 63u && t < 255u) {
+#pragma unroll
+        for (int l = 0; l < 9; ++l) red[t >> 6][l] = l9[l];
+    }
+    __syncthreads();
+    if (t != 255u) return;
+#pragma unroll
+    for (int l = 0; l < 9; ++l) l9[l] += red[0][l] + red[1][l] + red[2][l];
+    fr29_carry_u(l9);
+    Fr29 x;
+#pragma unroll
+    for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+    *a.ev_out = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));
+}
 __global__ void __launch_bounds__(1024) k_ip_rounds(const IpArgs a) {
     __shared__ int32_t X0[2][IP_P][IP_W], X1[2][IP_P / 2][IP_W];
     __shared__ uint32_t raw[IP_ROUNDS][IP_GROUPS][3][9];
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave & 1u, group = wave >> 1;
     const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u;
     const uint32_t P = 1u << a.rounds;
+    if (blockIdx.x == a.nlow) { ip_evaluate(raw[0][0], a); return; }
     for (uint32_t i = threadIdx.x; i < 2 * P; i += 1024u) {
         const uint32_t s = i & (P - 1u), g = s * a.nlow + blockIdx.x;
-        rm_put(X0[i >> a.rounds][s], g < a.n ? fr29_repack((i >> a.rounds ? a.b : a.a)[g]) : fr29_zero());
+        Fr x = big_zero<8>();
+        if (g < a.n) {
+            x = (i >> a.rounds ? a.b : a.a)[g];
+            if (!(i >> a.rounds))
+#pragma unroll 4
+                for (uint32_t k = 1; k < a.a_parts; ++k) x = add(x, a.a[(size_t)k * a.n + g]);
+        }
+        rm_put(X0[i >> a.rounds][s], fr29_repack(x));
     }
     // the sums of the launch before, on waves that have no pairs here (it has at most 24 of them, of at most 32 parts each)
     if (a.prev && wave >= 2u && (wave - 2u) * 4u < a.prev_count) {
@@ -577,25 +724,28 @@ __global__ void __launch_bounds__(1024) k_ip_rounds(const IpArgs a) {
         }
         __syncthreads();
     }
-    // a product of two elements carries 2^-261 here
-    if (threadIdx.x < 3u * a.rounds) {
-        const uint32_t r = threadIdx.x / 3u, q = threadIdx.x % 3u, half = P >> (r + 1), ng = (half + 15u) / 16u;
-        auto sum = [&](uint32_t role) {
-            uint32_t l9[9];
+    // a product of two elements carries 2^-261 here.  Lane 3 r + q adds up round r's q-th sum; the middle coefficient takes its neighbours'
+    if (threadIdx.x < 64u) {
+        const uint32_t i = threadIdx.x < 3u * a.rounds ? threadIdx.x : 0u, r = i / 3u, q = i - 3u * r, half = P >> (r + 1), ng = (half + 15u) / 16u;
+        uint32_t l9[9];
 #pragma unroll
-            for (int l = 0; l < 9; ++l) {
-                l9[l] = 0;
-                for (uint32_t g = 0; g < ng; ++g) l9[l] += raw[r][g][role][l];
-            }
-            fr29_carry_u(l9);
-            Fr29 x;
+        for (int l = 0; l < 9; ++l) {
+            l9[l] = 0;
+            for (uint32_t g = 0; g < ng; ++g) l9[l] += raw[r][g][q][l];
+        }
+        fr29_carry_u(l9);
+        Fr29 x;
 #pragma unroll
-            for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
-            return fr29_canon_pack<5>(fr29_mul(x, fr29_2_522()));
-        };
-        Fr o = sum(q == 0 ? 0u : (q == 2 ? 2u : 1u));
-        if (q == 1) o = sub(sub(o, sum(0)), sum(2));
-        a.sums[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = o;
+        for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+        Fr o = fr29_canon_pack<5>(fr29_mul(x, fr29_2_522()));
+        Fr before, behind;
+#pragma unroll
+        for (int l = 0; l < 8; ++l) {
+            before.v[l] = (uint32_t)__shfl_up((int)o.v[l], 1, 64);
+            behind.v[l] = (uint32_t)__shfl_down((int)o.v[l], 1, 64);
+        }
+        if (q == 1) o = sub(sub(o, before), behind);
+        if (threadIdx.x < 3u * a.rounds) a.sums[(size_t)threadIdx.x * a.nlow + blockIdx.x] = o;
     }
     const int32_t* const fin = (a.rounds & 1u) ? &X1[0][0][0] : &X0[0][0][0];
     const uint32_t fs = ((a.rounds & 1u) ? IP_P / 2 : IP_P) * IP_W;
@@ -988,47 +1138,131 @@ int zk_ip_round_stacked(uint32_t* poly3_host, const void* a, const void* b, cons
     return 0;
 }
 
+// The launches of a complete inner-product sumcheck for n <= 8192.  work: ip_work(k) elements; out: 3 k sums, then the folded a and b.
+struct IpEval { const Fr* v; const int32_t* E; uint32_t n; Fr* out; };
+static size_t ip_work(int k) { return k <= IP_ROUNDS ? 0 : (3 * (size_t)IP_ROUNDS + 2) << (k - IP_ROUNDS); }
+static int ip_rounds_queue(Fr* work, Fr* out, const Fr* a, uint32_t a_parts, const Fr* b, uint32_t n, const uint32_t* u, int k, const IpEval* ev, hipStream_t st) {
+    // work: what passes from the first launch to the second
+    const int r1 = k <= IP_ROUNDS ? 0 : IP_ROUNDS, r2 = k - r1;
+    const uint32_t nb1 = r1 ? 1u << (k - r1) : 0u;
+    Fr* part = work;
+    Fr* mid = part + 3 * (size_t)r1 * nb1;
+    IpArgs q;
+    memset(&q, 0, sizeof(q));
+    q.a = a; q.b = b; q.n = n; q.a_parts = a_parts;
+    if (ev) { q.ev = ev->v; q.ev_E = ev->E; q.ev_n = ev->n; q.ev_out = ev->out; }
+    auto challenges = [&](int from, int count) {
+        for (int i = 0; i < count; ++i) q.v[i] = fr29_repack(mont_mul(to_mont(load_fr(u + 8 * (size_t)(k - 1 - from - i))), fr29_pack(fr29_2_261())));
+    };
+    uint32_t extra = ev ? 1u : 0u;
+    if (r1) {
+        challenges(0, r1);
+        q.rounds = (uint32_t)r1; q.nlow = nb1; q.sums = part; q.na = mid; q.nb = mid + nb1;
+        hipLaunchKernelGGL(k_ip_rounds, dim3(nb1 + extra), dim3(1024), 0, st, q);
+        ZK_LAUNCH_CHECK();
+        q.a = mid; q.b = mid + nb1; q.n = nb1; q.a_parts = 1;
+        q.prev = part; q.prev_out = out; q.prev_nb = nb1; q.prev_count = 3u * (uint32_t)r1;
+        extra = 0;
+    }
+    challenges(r1, r2);
+    q.rounds = (uint32_t)r2; q.nlow = 1; q.sums = out + 3 * r1; q.na = out + 3 * k; q.nb = q.na + 1;
+    hipLaunchKernelGGL(k_ip_rounds, dim3(1 + extra), dim3(1024), 0, st, q);
+    ZK_LAUNCH_CHECK();
+    return 0;
+}
 // Complete inner-product sumcheck for n <= 8192 in one or two launches.  u[0..k) standard form, consumed
 // from the back; polys_host gets 3*k coefficients, fin_host the folded a and b.
 int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a, const void* b, uint32_t n, const uint32_t* u, int k, void* stv) {
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(k >= 1 && k <= 13, "zk_ip_sumcheck_small: k must be 1..13");
     ZK_ARG(n >= 1 && n <= (1u << k) && n > ((1u << k) >> 1), "zk_ip_sumcheck_small: need 2^(k-1) < n <= 2^k");
-    // delivered: the sums of all rounds, then the two folded values; work: what passes from the first launch to the second
-    const int r1 = k <= IP_ROUNDS ? 0 : IP_ROUNDS, r2 = k - r1;
-    const uint32_t nb1 = r1 ? 1u << (k - r1) : 0u;
-    Scratch work(sizeof(Fr) * (3 * (size_t)r1 + 2) * nb1, st);
+    Scratch work(sizeof(Fr) * ip_work(k), st);
     if (work.rc) return work.rc;
+    // one delivery of 3k + 2 values: the round polynomials, then the two fully folded values
     Delivery d;
     int rc = deliver_begin(d, 3 * (size_t)k + 2, 0);
     if (rc) return rc;
-    Fr* polys = (Fr*)d.dst;
-    Fr* part = work.as<Fr>();
-    Fr* mid = part + 3 * (size_t)r1 * nb1;
-    IpArgs q;
-    memset(&q, 0, sizeof(q));
-    q.a = (const Fr*)a; q.b = (const Fr*)b; q.n = n;
-    auto challenges = [&](int from, int count) {
-        for (int i = 0; i < count; ++i) q.v[i] = fr29_repack(mont_mul(to_mont(load_fr(u + 8 * (size_t)(k - 1 - from - i))), fr29_pack(fr29_2_261())));
-    };
-    if (r1) {
-        challenges(0, r1);
-        q.rounds = (uint32_t)r1; q.nlow = nb1; q.sums = part; q.na = mid; q.nb = mid + nb1;
-        hipLaunchKernelGGL(k_ip_rounds, dim3(nb1), dim3(1024), 0, st, q);
-        ZK_LAUNCH_CHECK();
-        q.a = mid; q.b = mid + nb1; q.n = nb1;
-        q.prev = part; q.prev_out = polys; q.prev_nb = nb1; q.prev_count = 3u * (uint32_t)r1;
-    }
-    challenges(r1, r2);
-    q.rounds = (uint32_t)r2; q.nlow = 1; q.sums = polys + 3 * r1; q.na = polys + 3 * k; q.nb = q.na + 1;
-    hipLaunchKernelGGL(k_ip_rounds, dim3(1), dim3(1024), 0, st, q);
-    ZK_LAUNCH_CHECK();
-    // one delivery of 3k + 2 values: the round polynomials, then the two fully folded values
+    rc = ip_rounds_queue(work.as<Fr>(), (Fr*)d.dst, (const Fr*)a, 1u, (const Fr*)b, n, u, k, nullptr, st);
+    if (rc) return rc;
     Fr both[3 * 13 + 2];
     rc = deliver_end(d, st, both);
     if (rc) return rc;
     memcpy(polys_host, both, sizeof(Fr) * 3 * k);           // (while results are deferred these two are not what the kernel wrote: see zk_defer_begin)
     memcpy(fin_host, both + 3 * k, sizeof(Fr) * 2);
+    return 0;
+}
+// the factors of an eq table, with the factor 2^261: entry i = t_0[low bits of i] t_1[the next] ..., factor f with bits[f] bits
+static void eq_factors(Fr29* out, const uint32_t* u, const int* bits, int nf) {
+    for (int f = 0; f < nf; ++f) {
+        Fr t[32];
+        t[0] = fr29_pack(fr29_2_261());
+        for (int b = 0; b < bits[f]; ++b, u += 8) {
+            const Fr x = to_mont(load_fr(u));
+            for (int i = 0; i < (1 << b); ++i) {
+                t[i + (1 << b)] = mont_mul(t[i], x);
+                t[i] = sub(t[i], t[i + (1 << b)]);
+            }
+        }
+        for (int i = 0; i < (1 << bits[f]); ++i) *out++ = fr29_repack(t[i]);
+    }
+}
+int zk_matmul_sumcheck(uint32_t* claim_host, uint32_t* polys_host, uint32_t* fin_host, const void* X, const void* W, const void* Y, uint32_t B, uint32_t D, uint32_t O,
+                       const uint32_t* u_batch, int kb, const uint32_t* u_input, int kd, const uint32_t* u_output, int ko, void* stv) {
+    hipStream_t st = (hipStream_t)stv;
+    auto fits = [](uint32_t n, int k, int most) { return k >= 0 && k <= most && n >= 1 && n <= (1u << k) && n > ((1u << k) >> 1); };
+    ZK_ARG(kd >= 1 && fits(D, kd, 13), "zk_matmul_sumcheck: inner axis: 1 to 13 challenges, 2^(k-1) < D <= 2^k");
+    ZK_ARG(fits(B, kb, EQ29_MAX) && fits(O, ko, EQ29_MAX), "zk_matmul_sumcheck: outer axes: at most 14 challenges, 2^(k-1) < n <= 2^k");
+    FcFolds a;
+    a.X = (const Fr*)X; a.W = (const Fr*)W; a.Y = (const Fr*)Y;
+    a.B = B; a.D = D; a.O = O;
+    // X: sixteen terms a lane, fewer where the axis is that short, more where there would be more than eight parts to add up
+    a.J = B < 64 ? (B + 15) / 16 * 4 : 16;
+    while (a.J < 64 && B > 32 * a.J) a.J *= 2;
+    a.xgroups = (D + 63) / 64; a.xchunks = (B + 4 * a.J - 1) / (4 * a.J);
+    auto waves = [&](uint32_t rows) { return O < 512 || (rows >= 8192 && O <= 4096) ? 1u : 4u; };      // as zk_fr_fold_axis_all
+    a.wwaves = waves(D); a.ywaves = waves(B);
+    a.wblocks = a.wwaves == 1 ? cdiv(D, 8) : cdiv(D, 2);
+    a.yblocks = a.ywaves == 1 ? cdiv(B, 8) : cdiv(B, 2);
+    const size_t words = 9 * ((size_t)B + O), elems = (size_t)a.xchunks * D + D + B + ip_work(kd);
+    Scratch work(sizeof(Fr) * elems + sizeof(int32_t) * words, st);
+    if (work.rc) return work.rc;
+    a.Xf = work.as<Fr>(); a.Wf = a.Xf + (size_t)a.xchunks * D; a.Yf = a.Wf + D;
+    Fr* ip = a.Yf + B;
+    a.Eb = (int32_t*)(ip + ip_work(kd)); a.Eo = a.Eb + 9 * (size_t)B;
+    Delivery d;
+    int rc = deliver_begin(d, 3 * (size_t)kd + 3, 0);
+    if (rc) return rc;
+    if (kb <= FC_SMALL_BITS && ko <= FC_SMALL_BITS) {
+        FcEq<true> eq;
+        const int bb[2] = {std::min(kb, 5), std::max(kb - 5, 0)}, bo[2] = {std::min(ko, 5), std::max(ko - 5, 0)};
+        auto factors = [](EqArgs& e, const uint32_t* u, const int* bits) {
+            eq_factors(e.lo, u, bits, 1);
+            eq_factors(e.hi, u + 8 * bits[0], bits + 1, 1);
+        };
+        factors(eq.batch, u_batch, bb);
+        factors(eq.output, u_output, bo);
+        hipLaunchKernelGGL(k_fc_folds<true>, dim3(a.wblocks + a.yblocks + a.xgroups * a.xchunks + 1), dim3(TPB), 0, st, a, eq);
+    } else {
+        EqTwoTabs t;
+        auto split = [](int* bits, int k) { for (int f = 0; f < 4; ++f) bits[f] = (k + 3 - f) / 4; };
+        split(t.bits[0], kb); split(t.bits[1], ko);
+        t.n[0] = B; t.n[1] = O;
+        eq_factors(t.t[0], u_batch, t.bits[0], 4);
+        eq_factors(t.t[1], u_output, t.bits[1], 4);
+        const uint32_t first = cdiv(B, TPB);
+        hipLaunchKernelGGL(k_eq29_two, dim3(first + cdiv(O, TPB)), dim3(TPB), 0, st, a.Eb, a.Eo, t, first);
+        hipLaunchKernelGGL(k_fc_folds<false>, dim3(a.wblocks + a.yblocks + a.xgroups * a.xchunks), dim3(TPB), 0, st, a, FcEq<false>{});
+    }
+    ZK_LAUNCH_CHECK();
+    const IpEval ev{a.Yf, a.Eb, B, (Fr*)d.dst};
+    rc = ip_rounds_queue(ip, (Fr*)d.dst + 1, a.Xf, a.xchunks, a.Wf, D, u_input, kd, &ev, st);
+    if (rc) return rc;
+    Fr all[3 * 13 + 3];
+    rc = deliver_end(d, st, all);
+    if (rc) return rc;
+    memcpy(claim_host, all, sizeof(Fr));
+    memcpy(polys_host, all + 1, sizeof(Fr) * 3 * kd);
+    memcpy(fin_host, all + 1 + 3 * kd, sizeof(Fr) * 2);
     return 0;
 }
 

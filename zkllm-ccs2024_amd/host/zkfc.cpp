@@ -95,6 +95,22 @@ zkFC::Pending zkFC::prove_begin(const FrTensor& X, const FrTensor& Y, const Chal
     if (Y.size != p.batchSize * outputSize) throw std::runtime_error("zkFC::prove: Y does not match the shapes");
     p.keep.reserve(2 * u_input.size() + 4);
     p.results.begin();
+    // plain tensors: all of it in a few launches (a tensor that is kept for folds has a form that is cheaper to read)
+    const bool sizes = X.size == p.batchSize * inputSize && weights.size == inputSize * outputSize && inputSize <= 8192;
+    if (sizes && !X.fold_cache && !weights.fold_cache && !Y.fold_cache && std::max(u_batch.size(), u_output.size()) <= 14) {
+        try {
+            Fr_t unused_claim, unused_polys[3 * 13], unused_fin[2];
+            auto first = [](const vector<Fr_t>& u) { return u.empty() ? nullptr : u[0].val; };
+            ZKC(zk_matmul_sumcheck(unused_claim.val, unused_polys[0].val, unused_fin[0].val, X.gpu_data, weights.gpu_data, Y.gpu_data, p.batchSize, inputSize, outputSize,
+                                   first(u_batch), (int)u_batch.size(), first(u_input), (int)u_input.size(), first(u_output), (int)u_output.size(), nullptr));
+            p.small_rounds = (uint)u_input.size();
+        } catch (...) {
+            p.results.end();
+            throw;
+        }
+        p.results.end();
+        return p;
+    }
     try {
         // result 0: Y at (u_batch, u_output)
         (void)Y.multi_dim_me({u_batch, u_output}, {p.batchSize, outputSize});
