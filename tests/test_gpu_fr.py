@@ -525,6 +525,24 @@ def test_matmul_of_small_integers_of_any_size(pv, num, M, N, P, amax, bmax):
     assert fr_ints(got) == [int(v) % R_MOD for i in range(num) for v in (A[i].astype(object) @ B[i].astype(object)).reshape(-1)]
 
 
+@pytest.mark.parametrize("num,M,N,P,amax,bmax", [(1, 2113, 131, 2050, 2 ** 17, 2 ** 13), (3, 1000, 33, 1921, 100, 100), (1, 4100, 63, 1000, 2 ** 38, 100), (2, 1025, 64, 2176, 2 ** 17, 2 ** 20), (1, 2113, 40, 2050, 2 ** 30, 2 ** 20)])
+def test_matmul_on_tiles_of_128_columns(pv, num, M, N, P, amax, bmax):
+    """Products of 512 tiles and more: ragged rows, columns and inner dimensions, stacks, plane counts on both sides of the wide tile's line."""
+    rng = np.random.default_rng(M)
+    pv.lib.zkp_set_matmul_mode(ctypes.c_int(0))
+    A = rng.integers(-amax, amax + 1, (num, M, N)).astype(np.int64)
+    B = rng.integers(-bmax, bmax + 1, (num, N, P)).astype(np.int64)
+    got = pv.matmul_stack(pv.from_i64(A), pv.from_i64(B), num, M, N, P).host().reshape(num, M, P, 8)
+    assert pv.lib.zkp_last_matmul_path() == 2
+    want = A @ B                                            # below 2^63
+    low = got[..., 0].astype(np.uint64) | got[..., 1].astype(np.uint64) << np.uint64(32)
+    neg = want < 0
+    r_low = np.uint64(R_MOD & (2 ** 64 - 1))
+    assert (low == np.where(neg, r_low + want.astype(np.uint64), want.astype(np.uint64))).all()
+    high = np.array([(R_MOD >> (32 * i)) & 0xFFFFFFFF for i in range(2, 8)], np.uint32)
+    assert (got[..., 2:] == np.where(neg[..., None], high, np.uint32(0))).all()
+
+
 def test_matmul_with_a_kept_right_operand_and_layers_over_views(pv):
     """A weight kept as the right operand of matrix products (FrTensor::keep_as_matmul_rhs: largest magnitude and digit planes
     computed once, zk_fr_matmul_rhs_prepare / zk_fr_matmul_rhs) gives the products of the plain path, on the matrix-core path and
