@@ -479,11 +479,18 @@ __global__ void __launch_bounds__(TPB) k_eq29_two(int32_t* __restrict__ Eb, int3
         else Eb[(size_t)at * 9 + l] = e.l[l];
     }
 }
+// out[i] = sum of the count parts of i, sixteen lanes an output: one lane's loads behind one another took 24 us for 128 outputs of 64 parts
 __global__ void __launch_bounds__(TPB) k_sum_partials(Fr* __restrict__ out, const Fr* __restrict__ part, size_t n, uint32_t count) {
-    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= n) return;
-    Fr s = part[i];
-    for (uint32_t c = 1; c < count; ++c) s = add(s, part[(size_t)c * n + i]);
+    __shared__ Fr red[TPB / 16 - 1][16];
+    const uint32_t q = threadIdx.x >> 4, o = threadIdx.x & 15u;
+    const size_t i = (size_t)blockIdx.x * 16 + o;
+    Fr s = big_zero<8>();
+    if (i < n)
+        for (uint32_t c = q; c < count; c += TPB / 16) s = add(s, part[(size_t)c * n + i]);
+    if (q) red[q - 1][o] = s;
+    __syncthreads();
+    if (q || i >= n) return;
+    for (uint32_t k = 0; k < TPB / 16 - 1; ++k) s = add(s, red[k][o]);
     out[i] = s;
 }
 
@@ -1029,7 +1036,10 @@ int zk_fr_fold_axis_all(void* out, const void* in, const uint32_t* u, int levels
         if (part.rc) return part.rc;
         hipLaunchKernelGGL(k_fold_cols, dim3((unsigned)groups, chunks, (unsigned)other), dim3(TPB), 0, st, chunks > 1 ? part.as<Fr>() : (Fr*)out, (const Fr*)in, eq.as<int32_t>(), cur, window, J);
         ZK_LAUNCH_CHECK();
-        if (chunks > 1) LAUNCH1D(k_sum_partials, n_out, st, (Fr*)out, part.as<Fr>(), n_out, chunks);
+        if (chunks > 1) {
+            hipLaunchKernelGGL(k_sum_partials, dim3(cdiv(n_out, 16)), dim3(TPB), 0, st, (Fr*)out, part.as<Fr>(), n_out, chunks);
+            ZK_LAUNCH_CHECK();
+        }
         return 0;
     }
     if (whole && cur <= FOLD_SMALL_CUR && levels <= 10 && other * cur * window <= FOLD_SMALL_MAX) {
