@@ -167,6 +167,30 @@ def test_commit_int_matches_oracle(pv, orc, m, n, lim):
     assert (norm(orc, got) == norm(orc, exp)).all()
 
 
+@pytest.mark.parametrize("m,n,lim", [(40, 100, 1), (2, 8192, 3), (1, 5000, 2 ** 31 - 1), (3, 129, 9), (200, 300, 2 ** 12), (9, 33, 2 ** 20)])
+def test_commit_int_tables_of_every_shape_match_the_oracle(pv, orc, m, n, lim):
+    """Tables whose first entries (k_msm_table_first) are all of a window, none, or as many as two waves a SIMD have lanes for; one generator is infinity, two are equal."""
+    gens = oracle_gens(orc, 90 + n, n)
+    gens[1] = 0
+    gens[2] = gens[3]
+    rng = np.random.default_rng(m * n)
+    t = rng.integers(-lim, lim, m * n, endpoint=True).astype(np.int64)
+    t[0], t[5], t[n - 1] = -lim, -2 ** 31 if lim > 2 ** 30 else lim, lim
+    T = fr_array([int(x) % R_MOD for x in t])
+    exp = np.zeros((m, 36), np.uint32)
+    orc_check(orc.orc_commit_int(gens, n, T, m * n, exp))
+    assert (norm(orc, pv.commit_int(pv.g1_from_host(gens), pv.from_fr(T)).host()) == norm(orc, exp)).all()
+
+
+@pytest.mark.parametrize("bad", [2 ** 31, R_MOD - 2 ** 31 - 1, 2 ** 32, 2 ** 64, R_MOD - 2 ** 64, 1 << 224, (R_MOD >> 64) << 64, R_MOD - (1 << 224)])
+def test_commit_int_refuses_what_is_no_int32(pv, orc, bad):
+    gens = pv.g1_from_host(oracle_gens(orc, 14, 8))
+    ok = [0, 1, 2 ** 31 - 1, R_MOD - 1, R_MOD - 2 ** 31, 5, 6, 7]
+    pv.commit_int(gens, pv.from_fr(fr_array(ok)))
+    with pytest.raises(RuntimeError, match="int32"):
+        pv.commit_int(gens, pv.from_fr(fr_array(ok[:7] + [bad])))
+
+
 def test_commit_int_rejects_non_integer_scalars_and_is_linear(pv, orc):
     gens = oracle_gens(orc, 14, 8)
     hG = pv.g1_from_host(gens)

@@ -175,17 +175,17 @@ __global__ void __launch_bounds__(256) k_g1aff_to_a29(A29* __restrict__ out, con
 
 // ---- fixed-base table for commit_int -------------------------------------------------------------------------
 // table (Jacobian, before normalisation): tab[(w * ngen + j) * half + (d-1)] = d * 2^(c*w) * G_j, d = 1..half.
-// Bases first, one lane per generator walking up the windows by c doublings each; then the multiples by doubling the
+// Bases first, one lane per generator walking up the windows by c doublings each (7 us each, in 29-bit limbs; 14 in 32-bit ones); then the multiples by doubling the
 // filled part of every row, row[k + i] = row[i] + row[k - 1] for i < k, k = 1, 2, 4, ...: one launch per k with one lane
 // per new entry, so every launch is dense whatever the row length (rows are as short as 4 entries when few tensor rows
 // share the generators) and the chain of additions is log2(half) deep.
 __global__ void __launch_bounds__(GT) k_msm_table_bases(G1Jac* __restrict__ tab, const G1Jac* __restrict__ gens, size_t ngen, uint32_t c, uint32_t nwin, uint32_t half) {
     const size_t j = (size_t)blockIdx.x * GT + threadIdx.x;
     if (j >= ngen) return;
-    G1Jac base = gens[j];
+    J29 base = j29_from_jac(gens[j]);
     for (uint32_t w = 0; w < nwin; ++w) {
-        tab[((size_t)w * ngen + j) * half] = base;
-        if (w + 1 < nwin) for (uint32_t k = 0; k < c; ++k) base = g1_double(base);
+        tab[((size_t)w * ngen + j) * half] = w ? j29_to_jac(base) : gens[j];
+        if (w + 1 < nwin) for (uint32_t k = 0; k < c; ++k) j29_double_walk(base);
     }
 }
 __global__ void __launch_bounds__(GT) k_msm_table_fill(G1Jac* __restrict__ tab, size_t nrows, uint32_t logh, uint32_t logk) {
@@ -203,12 +203,30 @@ __device__ __forceinline__ size_t msm_slot(const MsmTable& T, uint32_t w, size_t
     const bool last = w + 1 == T.nwin;
     return (size_t)w * T.ngen * T.half + j * (last ? T.top : T.half) + (d - 1);
 }
-// the windows' first entries out of the normalised bases (window-major)
-__global__ void __launch_bounds__(256) k_msm_table_place(const MsmTable T, const G1Affine* __restrict__ bases) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= T.ngen * T.nwin) return;
-    const uint32_t w = (uint32_t)(i / T.ngen);
-    T.tab[msm_slot(T, w, i - (size_t)w * T.ngen, 1u)] = a29_from_affine(bases[i]);
+__device__ __forceinline__ Fq29 fq29_inverse(const Fq29& v) { return fq29_from_fp(mont_inverse(fq29_to_fp(v))); }
+// The first 2^logs entries of every window (those that it has) out of the normalised bases (window-major), a lane an entry: doublings and additions
+// of the base along the bits of the multiple, and an inversion.  A level of k_msm_table_grow takes what one lane's inversion and
+// its launch take however few its entries are: the first four of 8192 rows took 252 us, so they take 170.
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_first(const MsmTable T, const G1Affine* __restrict__ bases, uint32_t logs) {
+    const size_t i = (size_t)blockIdx.x * GT + threadIdx.x, r = i >> logs, rows_full = (size_t)(T.nwin - 1) * T.ngen;
+    const uint32_t d = (uint32_t)(i & ((1u << logs) - 1u)) + 1u;
+    const bool full = r < rows_full;
+    if (r >= T.ngen * T.nwin || d > (full ? T.half : T.top)) return;
+    const A29 base = a29_from_affine(bases[r]);
+    A29 out = base;
+    if (d > 1u && !a29_is_inf(base)) {
+        J29 p;
+        p.x = base.x; p.y = base.y; p.z = fq29_one(); p.inf = 0u;
+        for (int b = 30 - __clz((int)d); b >= 0; --b) {
+            j29_double_walk(p);
+            if ((d >> b) & 1u) j29_add_mixed_walk(p, base);
+        }
+        const Fq29 zi = fq29_inverse(p.z), zi2 = fq29_sqr(zi);
+        out.x = fq29_mul(p.x, zi2);
+        out.y = fq29_mul(p.y, fq29_mul(zi2, zi));
+        if (p.inf) { out.x = fq29_zero(); out.y = fq29_zero(); }
+    }
+    (full ? T.tab + r * T.half : T.tab + rows_full * T.half + (r - rows_full) * T.top)[d - 1u] = out;
 }
 // Entries k + 1 .. 2 k of every window that has them, entry k + i = entry i + entry k: affine additions, whose slopes share an inversion
 // among a lane's entries (an inversion costs a lane about 26 products, the rest of an entry seven).  The entry of the
@@ -243,7 +261,7 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
         row[k + (t & (k - 1))].x = run;
         run = fq29_mul_inline(run, den);
     }
-    Fq29 inv = fq29_from_fp(mont_inverse(fq29_to_fp(run)));
+    Fq29 inv = fq29_inverse(run);
     while (count-- > 0) {
         const size_t t = base + (size_t)count * GT;
         A29* row = row_of(t);
@@ -380,8 +398,9 @@ k_g1_fixed_base_mul(G1Jac* __restrict__ out, const A29* __restrict__ tab, const 
     out[i] = j29_to_jac(j29_from_x29(acc29));
 }
 // stats[0]: raised when an element is not the embedding of an int32, [1]: largest magnitude, [2 + b]: of the elements looked at (one in
-// CONV_SAMPLE), those whose magnitude has b bits.  Eight elements a lane in flight: one a lane and an atomic a workgroup ran at 0.8 TB/s
-static constexpr int CONV_SAMPLE = 8, CONV_STATS = 35;
+// CONV_SAMPLE), those whose magnitude has b bits.  Eight elements a lane in flight: one a lane and an atomic a workgroup ran at 0.8 TB/s; the words looked at
+// instead of the embedding formed again, and one round of workgroups at four waves a SIMD: 45 million elements 425 -> 338 us, 4.8 TB/s
+static constexpr int CONV_SAMPLE = 8, CONV_STATS = 35, CONV_GRID = 1024;
 __global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__ out, uint32_t* __restrict__ stats, const Fr* __restrict__ in, size_t n) {
     __shared__ uint32_t wmax[4], wbad[4], hist[33];
     if (threadIdx.x < 33u) hist[threadIdx.x] = 0u;
@@ -394,11 +413,15 @@ __global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__
         for (int q = 0; q < CONV_SAMPLE; ++q) x[q] = i0 + q * stride < n ? in[i0 + q * stride] : big_zero<8>();
 #pragma unroll
         for (int q = 0; q < CONV_SAMPLE; ++q) {
-            // scalar_to_int semantics: values outside the int32 embedding collapse to what the reference reads
-            const int32_t v = fr_to_i32(x[q]);
-            if (i0 + q * stride < n) out[i0 + q * stride] = v;
-            bad |= equal(fr_from_i64((int64_t)v), x[q]) ? 0u : 1u;
-            const uint32_t m = v < 0 ? (uint32_t)(-(int64_t)v) : (uint32_t)v;
+            // x itself, or r - |x|: the words from the third on are zero or r's (r's two low words leave 2^31 room, so nothing borrows from above)
+            uint32_t high = 0, high_neg = 0;
+#pragma unroll
+            for (int l = 2; l < 8; ++l) { high |= x[q].v[l]; high_neg |= x[q].v[l] ^ FrK::P(l); }
+            const uint64_t low = (uint64_t)x[q].v[1] << 32 | x[q].v[0], r_low = (uint64_t)FrK::P(1) << 32 | FrK::P(0);
+            const uint64_t mag = high ? r_low - low : low;
+            if (i0 + q * stride < n) out[i0 + q * stride] = (int32_t)(high ? 0u - (uint32_t)mag : (uint32_t)mag);
+            bad |= (high ? high_neg == 0 && mag - 1 < 0x80000000ull : mag < 0x80000000ull) ? 0u : 1u;
+            const uint32_t m = (uint32_t)mag;
             a = m > a ? m : a;
             if (q == 0) atomicAdd(&hist[m ? 32 - __clz((int)m) : 0], 1u);
         }
@@ -1056,7 +1079,6 @@ __global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__
 // normalisation or conversion pass between two rounds.
 // 1 / v, every lane its own: all lanes of a wave execute the inversion's instructions in any case, so a product tree over the
 // lanes around one inversion only adds to them.  v must not be 0 mod p (lanes with nothing to invert pass one).
-__device__ __forceinline__ Fq29 fq29_inverse(const Fq29& v) { return fq29_from_fp(mont_inverse(fq29_to_fp(v))); }
 // w as an affine point with canonical limbs (infinity: all zero)
 __device__ __forceinline__ A29 a29_from_j29(const J29& w) {
     A29 o;
@@ -2030,9 +2052,15 @@ int zk_g1_normalize(void* out, const void* in, size_t n, void* st) {
     return 0;
 }
 
+// levels that k_msm_table_first takes: as many entries a window as two waves a SIMD have lanes for
+static uint32_t msm_first_levels(size_t rows, uint32_t levels) {
+    uint32_t logs = 0;
+    while (logs < levels && rows << (logs + 1) <= (size_t)1 << 17) ++logs;
+    return logs;
+}
 // Digit width, windows and segments for m rows of ngen scalars.  seen[b]: how many of the sampled scalars have b bits.  Estimated times in us:
-// an entry of the table costs 0.12 ns and a level of it 60 us at least (one lane's inversion), a base's doubling 12 us of latency, an
-// addition 0.17 ns; a digit beyond the first is an addition where the scalar reaches it.
+// an entry of the table costs 0.12 ns, a level of it 60 us at least (one lane's inversion) or 30 among the first ones (k_msm_table_first, 50 us besides),
+// a base's doubling 7 us of latency, an addition 0.17 ns; a digit beyond the first is an addition where the scalar reaches it.
 struct MsmShape { uint32_t c, nwin, top, nseg; };
 static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs, const uint32_t* seen) {
     MsmShape best{0, 0, 0, 1};
@@ -2054,7 +2082,8 @@ static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs,
         if (entries * sizeof(A29) > 8e9) continue;
         uint32_t levels = 0;
         while ((1u << levels) < (nwin > 1 ? std::max(half, top) : top)) ++levels;
-        const double us = 12.0 * c * (nwin - 1) + 60.0 * levels + entries * 1.2e-4 + (double)m * ngen * digits * 1.7e-4;
+        const uint32_t first = msm_first_levels(ngen * nwin, levels);
+        const double us = 7.0 * c * (nwin - 1) + 60.0 * (levels - first) + (first ? 50.0 + 30.0 * first : 0.0) + entries * 1.2e-4 + (double)m * ngen * digits * 1.7e-4;
         if (!best.c || us < best_us) { best_us = us; best = MsmShape{c, nwin, top, 1}; }
     }
     if (!best.c) {      // more generators than the budget of the table allows any width for
@@ -2080,7 +2109,7 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     if (ints.rc) return ints.rc;
     if (stats.rc) return stats.rc;
     if (const int crc = clear_words(stats.p, CONV_STATS, st)) return crc;
-    hipLaunchKernelGGL(k_fr_to_i32_checked, dim3((unsigned)std::min<size_t>(cdiv(total, 256), 4096)), dim3(256), 0, st, ints.as<int32_t>(), stats.as<uint32_t>(), (const Fr*)scalars_fr, total);
+    hipLaunchKernelGGL(k_fr_to_i32_checked, dim3((unsigned)std::min<size_t>(cdiv(total, 256), CONV_GRID)), dim3(256), 0, st, ints.as<int32_t>(), stats.as<uint32_t>(), (const Fr*)scalars_fr, total);
     ZK_LAUNCH_CHECK();
     void* stage = nullptr;
     int rc = staging(&stage, 4 * CONV_STATS);
@@ -2105,9 +2134,12 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     T.tab = tab.as<A29>();
     hipLaunchKernelGGL(k_msm_table_bases, dim3(cdiv(ngen, GT)), dim3(GT), 0, st, basej.as<G1Jac>(), (const G1Jac*)gens, ngen, T.c, T.nwin, 1u);
     g1_normalize_queue<true>(basea.p, basej.as<G1Jac>(), nbase, st);
-    hipLaunchKernelGGL(k_msm_table_place, dim3(cdiv(nbase, 256)), dim3(256), 0, st, T, basea.as<G1Affine>());
     const size_t rows_full = (size_t)(T.nwin - 1) * ngen;
-    for (uint32_t logk = 0; (1u << logk) < std::max(T.top, T.nwin > 1 ? T.half : 1u); ++logk) {
+    uint32_t levels = 0;
+    while ((1u << levels) < std::max(T.top, T.nwin > 1 ? T.half : 1u)) ++levels;
+    const uint32_t logs = msm_first_levels(nbase, levels);
+    hipLaunchKernelGGL(k_msm_table_first, dim3(cdiv(nbase << logs, GT)), dim3(GT), 0, st, T, basea.as<G1Affine>(), logs);
+    for (uint32_t logk = logs; (1u << logk) < std::max(T.top, T.nwin > 1 ? T.half : 1u); ++logk) {
         const bool with_top = (1u << logk) < T.top;
         // the windows below the highest are never shorter than it, but a single window is the highest
         const size_t rows = (T.nwin > 1 ? rows_full : 0) + (with_top ? ngen : 0), n = rows << logk;
