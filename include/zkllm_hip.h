@@ -88,6 +88,7 @@ int zk_fr_neg(void* out, const void* a, size_t n, void* stream);
 int zk_fr_add_s(void* out, const void* a, const uint32_t* s, size_t n, void* stream);
 int zk_fr_sub_s(void* out, const void* a, const uint32_t* s, size_t n, void* stream);
 int zk_fr_mul_s(void* out, const void* a, const uint32_t* s, size_t n, void* stream);
+int zk_fr_add_mul_s(void* out, const void* a, const void* b, const uint32_t* s, size_t n, void* stream);      /* a + s b */
 int zk_fr_mont(void* out, const void* a, size_t n, void* stream);                     /* a*R  */
 int zk_fr_unmont(void* out, const void* a, size_t n, void* stream);                   /* a/R  */
 int zk_fr_fill(void* out, const uint32_t* s, size_t n, void* stream);

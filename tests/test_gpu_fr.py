@@ -61,6 +61,18 @@ def test_elementwise_ops_bit_exact(hip, orc):
         assert (got == exp).all(), name
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 5000])
+def test_a_sum_with_a_multiple_is_its_product_and_its_sum(hip, n):
+    A, B = seeded(n, 3)[-n:].copy(), seeded(n, 4)[:n].copy()
+    for s in (0, 1, R_MOD - 12345):
+        a, b, out = hip.upload(A), hip.upload(B), hip.malloc(32 * n)
+        hip.call("zk_fr_add_mul_s", ctypes.c_void_p(out), ctypes.c_void_p(a), ctypes.c_void_p(b), fr_array([s]), ctypes.c_size_t(n), None)
+        got = hip.download(out, (n, 8), np.uint32)
+        assert fr_ints(got) == [(x + s * y) % R_MOD for x, y in zip(fr_ints(A), fr_ints(B))]
+        for p in (a, b, out):
+            hip.free(p)
+
+
 def test_empty_and_single_element(hip, pv):
     empty = np.zeros((0, 8), np.uint32)
     assert hip.fr_binary("zk_fr_add", empty, empty).shape == (0, 8)

@@ -46,6 +46,11 @@ template <int OP> __global__ void __launch_bounds__(TPB) k_ew_s(Fr* __restrict__
     else r = mont_mul(x, s);
     out[i] = r;
 }
+// a + s b (s in Montgomery form) in one pass: 2^20 elements 72 us as a product and a sum that read it back
+__global__ void __launch_bounds__(TPB) k_add_mul_s(Fr* __restrict__ out, const Fr* __restrict__ a, const Fr* __restrict__ b, const Fr s, size_t n) {
+    const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
+    if (i < n) out[i] = add(a[i], mont_mul(b[i], s));
+}
 __global__ void __launch_bounds__(TPB) k_neg(Fr* __restrict__ out, const Fr* __restrict__ a, size_t n) {
     const size_t i = (size_t)blockIdx.x * TPB + threadIdx.x;
     if (i < n) out[i] = neg(a[i]);
@@ -846,6 +851,10 @@ int zk_fr_sub_s(void* out, const void* a, const uint32_t* s, size_t n, void* st)
 int zk_fr_mul_s(void* out, const void* a, const uint32_t* s, size_t n, void* st) {
     const Fr sm = to_mont(load_fr(s));
     LAUNCH1D(k_ew_s<EW_MUL>, n, st, (Fr*)out, (const Fr*)a, sm, n);
+    return 0;
+}
+int zk_fr_add_mul_s(void* out, const void* a, const void* b, const uint32_t* s, size_t n, void* st) {
+    LAUNCH1D(k_add_mul_s, n, st, (Fr*)out, (const Fr*)a, (const Fr*)b, to_mont(load_fr(s)), n);
     return 0;
 }
 // a*R (Scalar_mont) is a Montgomery product with R^2; a*R^-1 (Scalar_unmont) one with 1.

@@ -269,8 +269,10 @@ LookupPending tLookupRangeMapping::prove_begin(const FrTensor& S_in, const FrTen
     const uint N = mm->size;
     if (N != (1u << ceilLog2(N)) || si->size % N != 0) throw std::runtime_error("N is not power of 2, or D is not divisible by N");
     // S_com = S_in + r * S_out (tlookup.cu:517) is formed by the job itself; T_com is small
-    keep.emplace_back(new FrTensor(table + mapped_vals * r));
-    const FrTensor* T_com = keep.back().get();
+    if (mapped_vals.size != table.size) throw std::runtime_error("Incompatible dimensions");
+    FrTensor* T_com = new FrTensor(table.size);
+    keep.emplace_back(T_com);
+    ZKC(zk_fr_add_mul_s(T_com->gpu_data, table.gpu_data, mapped_vals.gpu_data, r.val, T_com->size, nullptr));
     LookupPending p = sumcheck_begin(*si, *T_com, *mm, alpha, beta, u, v, si, low, so, &r, mapped_vals.kept_ints());
     p.keep = std::move(keep);
     return p;
