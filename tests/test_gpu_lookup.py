@@ -184,6 +184,26 @@ def test_multiplicities_of_many_queries_into_a_large_table(pv, D, low, length, s
     assert (mk[:, 0] == want).all() and not mk[:, 1:].any()
 
 
+@pytest.mark.parametrize("D,low,length", [(1 << 17, 0, 1 << 17), (300001, -7, 200000), (1 << 18, 3, 1 << 18), ((1 << 18) - 1, -9, 1 << 18), (2000003, 5, (1 << 18) - 1), (600000, -3, (1 << 17) + 1)])
+def test_multiplicities_of_tables_counted_in_ranges_of_bins(pv, D, low, length):
+    """Two and four workgroups a share of the queries (k_hist_wide's ranges), the sizes where that begins and ends, whole shares in one bin at a range's edge."""
+    rng = np.random.default_rng(D)
+    vals = rng.integers(low, low + length, D)
+    vals[: D // 3] = low + 65535
+    vals[D // 3: D // 2] = low + 65536
+    vals[-1] = low + length - 1
+    h = pv.from_i64(vals)
+    want = np.bincount(vals - low, minlength=1 << (length - 1).bit_length()).astype(np.uint32)
+    for kept in (False, True):
+        if kept:
+            pv.keep_for_folds(h)
+        m = pv.range_prep(h, low, length).host()
+        assert (m[:, 0] == want).all() and not m[:, 1:].any()
+    vals[D // 2] = low + length
+    with pytest.raises(RuntimeError, match="outside the table"):
+        pv.range_prep(pv.from_i64(vals), low, length)
+
+
 @pytest.mark.parametrize("D,low,length", [(1, 7, 16385), (8193, -3, 40001), (70001, -(1 << 15), 1 << 16), ((1 << 20) + 5, 0, 1 << 15), (3000000, -5, 65535)])
 def test_multiplicities_of_tables_counted_in_halves_of_words(pv, D, low, length):
     """Tables of 16385 to 65536 entries (k_hist_wide): one query, shares of unequal size, all queries of a share in one bin."""

@@ -173,18 +173,46 @@ __global__ void __launch_bounds__(TPB) k_index_i32(uint32_t* __restrict__ idx, u
 // value - low; a value outside [low, low + len) counts as position 0 and raises *flag in the passes that are asked to check), or as
 // field elements (fr, low_fr: read eight times the bytes, so by passes that are alone to read them).
 struct KeySrc { const uint32_t* idx; const int32_t* vals; int32_t low; uint32_t len; uint32_t* flag; const Fr* fr = nullptr; Fr low_fr = Fr(); };
-template <bool CHECK> __device__ __forceinline__ uint32_t key_at(const KeySrc& k, size_t i) {
-    if (k.idx) return k.idx[i];
-    if (k.fr) {
-        const Fr d = sub(k.fr[i], k.low_fr);
-        const bool ok = !(d.v[1] | d.v[2] | d.v[3] | d.v[4] | d.v[5] | d.v[6] | d.v[7]) && d.v[0] < k.len;
-        if (CHECK && !ok) atomicOr(k.flag, 1u);
-        return ok ? d.v[0] : 0u;
-    }
-    const int64_t d = (int64_t)k.vals[i] - (int64_t)k.low;
+template <bool CHECK> __device__ __forceinline__ uint32_t key_of(const KeySrc& k, const Fr& x) {
+    const Fr d = sub(x, k.low_fr);
+    const bool ok = !(d.v[1] | d.v[2] | d.v[3] | d.v[4] | d.v[5] | d.v[6] | d.v[7]) && d.v[0] < k.len;
+    if (CHECK && !ok) atomicOr(k.flag, 1u);
+    return ok ? d.v[0] : 0u;
+}
+template <bool CHECK> __device__ __forceinline__ uint32_t key_of(const KeySrc& k, int32_t x) {
+    const int64_t d = (int64_t)x - (int64_t)k.low;
     const bool ok = d >= 0 && d < (int64_t)k.len;
     if (CHECK && !ok) atomicOr(k.flag, 1u);
     return ok ? (uint32_t)d : 0u;
+}
+template <bool CHECK> __device__ __forceinline__ uint32_t key_at(const KeySrc& k, size_t i) {
+    if (k.idx) return k.idx[i];
+    return k.fr ? key_of<CHECK>(k, k.fr[i]) : key_of<CHECK>(k, k.vals[i]);
+}
+// positions i, i + step, ... below end, their loads in flight together; ~0: none
+template <int N> __device__ __forceinline__ void keys_at(uint32_t (&key)[N], const KeySrc& k, size_t i, size_t step, size_t end) {
+    auto all = [&](auto read) {
+        decltype(read((size_t)0)) x[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = read(i + q * step < end ? i + q * step : i);
+        return [=](int q) { return x[q]; };
+    };
+    if (k.idx) {
+        const auto x = all([&](size_t j) { return k.idx[j]; });
+#pragma unroll
+        for (int q = 0; q < N; ++q) key[q] = x(q);
+    } else if (k.fr) {
+        const auto x = all([&](size_t j) { return k.fr[j]; });
+#pragma unroll
+        for (int q = 0; q < N; ++q) key[q] = key_of<true>(k, x(q));
+    } else {
+        const auto x = all([&](size_t j) { return k.vals[j]; });
+#pragma unroll
+        for (int q = 0; q < N; ++q) key[q] = key_of<true>(k, x(q));
+    }
+#pragma unroll
+    for (int q = 0; q < N; ++q)
+        if (i + q * step >= end) key[q] = ~0u;
 }
 static constexpr uint32_t HIST_LDS_BINS = 16384;
 __global__ void __launch_bounds__(TPB) k_hist_lds(uint32_t* __restrict__ counts, const KeySrc idx, size_t n, uint32_t nbins) {
@@ -351,19 +379,27 @@ static int hist_partitioned(uint32_t* counts, const KeySrc idx, size_t n, uint32
 // 32768 queries at most), writes all its counters out, and a second launch adds the workgroups' up and writes the multiplicities.  The
 // counters cross memory once, in lines; adding them to global ones costs an atomic for nearly every query where these spread.
 // 2^22 queries in 2^16 bins: partitioned 163 us, this way 30 us.
-static constexpr uint32_t HW_BINS = 65536, HW_SHARE = 32768, HW_T = 1024, HW_SLICES = 8;
+// Up to four times as many entries: a workgroup for every 65536 of them reads the same share and counts those that are its own, where there are
+// as many queries as entries.  825000 queries in 2^18 bins: 42 us by global atomics, 22 this way.
+static constexpr uint32_t HW_BINS = 65536, HW_SHARE = 32768, HW_T = 1024, HW_SLICES = 8, HW_RANGES = 4, HW_AHEAD = 4;
 __global__ void __launch_bounds__(HW_T) k_hist_wide(uint32_t* __restrict__ part, const KeySrc idx, size_t n, uint32_t words) {
     __shared__ __attribute__((aligned(16))) uint32_t h[HW_BINS / 2];
-    for (uint32_t w = threadIdx.x; w < words; w += HW_T) h[w] = 0;
+    const uint32_t first = blockIdx.y * (HW_BINS / 2), own = words - first < HW_BINS / 2 ? words - first : HW_BINS / 2;
+    for (uint32_t w = threadIdx.x; w < own; w += HW_T) h[w] = 0;
     __syncthreads();
     const size_t share = (n + gridDim.x - 1) / gridDim.x, begin = (size_t)blockIdx.x * share, end = begin + share < n ? begin + share : n;
-    for (size_t i = begin + threadIdx.x; i < end; i += HW_T) {
-        const uint32_t key = key_at<true>(idx, i);
-        atomicAdd(&h[key >> 1], 1u << (16u * (key & 1u)));
+    for (size_t i = begin + threadIdx.x; i < end; i += HW_AHEAD * HW_T) {
+        uint32_t key[HW_AHEAD];
+        keys_at(key, idx, i, HW_T, end);
+#pragma unroll
+        for (uint32_t q = 0; q < HW_AHEAD; ++q) {
+            const uint32_t k = key[q] - 2 * first;
+            if (k < 2 * own) atomicAdd(&h[k >> 1], 1u << (16u * (k & 1u)));
+        }
     }
     __syncthreads();
-    uint32_t* out = part + (size_t)blockIdx.x * words;
-    for (uint32_t w = threadIdx.x; w < words; w += HW_T) out[w] = h[w];
+    uint32_t* out = part + (size_t)blockIdx.x * words + first;
+    for (uint32_t w = threadIdx.x; w < own; w += HW_T) out[w] = h[w];
 }
 // m[bin] as field elements; *host_flag = *flag
 __global__ void __launch_bounds__(64 * HW_SLICES) k_hist_wide_sum(Fr* __restrict__ m, const uint32_t* __restrict__ part, uint32_t parts, uint32_t words, uint32_t nbins,
@@ -2201,8 +2237,9 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
     hipStream_t st = (hipStream_t)stv;
     ZK_ARG(nbins >= 1 && len >= 1 && len <= nbins, "zk_lookup_multiplicities: need 1 <= len <= nbins");
     ZK_ARG(m != nullptr && (idx != nullptr || vals_i32 != nullptr || vals != nullptr || n == 0), "zk_lookup_multiplicities: null argument");
-    const bool wide = nbins > HIST_LDS_BINS && nbins <= HW_BINS && n >= 1 && n < ((size_t)1 << 27);
-    const unsigned shares = wide ? (unsigned)std::max<size_t>(std::min<size_t>(cdiv(n, (size_t)8192), 256), cdiv(n, (size_t)HW_SHARE)) : 0u;
+    const unsigned ranges = cdiv(nbins, HW_BINS);
+    const bool wide = nbins > HIST_LDS_BINS && n >= 1 && n < ((size_t)1 << 27) && (ranges == 1 || (ranges <= HW_RANGES && n >= nbins));
+    const unsigned shares = wide ? (unsigned)std::max<size_t>(std::min<size_t>(cdiv(n, (size_t)8192), 256 / ranges), cdiv(n, (size_t)HW_SHARE)) : 0u;
     const uint32_t words = (nbins + 1) / 2;
     Scratch counts(sizeof(uint32_t) * ((wide ? (size_t)shares * words : (size_t)nbins) + 1), st);      // the first word: the flag
     if (counts.rc) return counts.rc;
@@ -2218,7 +2255,7 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
         src.fr = (const Fr*)vals;
         src.low_fr = fr_from_i64((int64_t)low);
     }
-    const bool several_passes = !wide && nbins > HIST_LDS_BINS && n >= HP_MIN_QUERIES;
+    const bool several_passes = wide ? ranges > 1 : nbins > HIST_LDS_BINS && n >= HP_MIN_QUERIES;
     if (!idx && (idx_out || (src.fr && several_passes))) {
         if (!idx_out) {
             own.reset(new Scratch(sizeof(uint32_t) * n, st));
@@ -2231,7 +2268,7 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
         src.fr = nullptr;
     }
     if (wide) {
-        hipLaunchKernelGGL(k_hist_wide, dim3(shares), dim3(HW_T), 0, st, c, src, n, words);
+        hipLaunchKernelGGL(k_hist_wide, dim3(shares, ranges), dim3(HW_T), 0, st, c, src, n, words);
         hipLaunchKernelGGL(k_hist_wide_sum, dim3(cdiv(words, 64u)), dim3(64 * HW_SLICES), 0, st, (Fr*)m, c, shares, words, nbins, flag, (uint32_t*)stage);
     } else {
         rc = hist_add_queue(c, src, n, nbins, st);
