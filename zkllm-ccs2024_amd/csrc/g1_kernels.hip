@@ -28,6 +28,9 @@ using namespace zk;
 static constexpr int GT = 64;   // threads per workgroup for point kernels (one wave; ~200 VGPRs per lane)
 
 // ---- elementwise -------------------------------------------------------------------------------------
+// For kernels of a few waves that a chain of launches waits for: their instructions go before those of the wide kernels of other streams that
+// share their SIMDs: an opening of 128 x 131072, with the workgroups of one wave that k_tail_levels explains, 9.13 -> 8.70 ms
+__device__ __forceinline__ void urgent() { __builtin_amdgcn_s_setprio(3); }
 __global__ void __launch_bounds__(GT) k_g1_fill(G1Jac* __restrict__ out, const G1Jac p, size_t n) {
     const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i < n) out[i] = p;
@@ -124,6 +127,7 @@ __global__ void __launch_bounds__(GT) k_g1_me_step(G1Jac* __restrict__ out, cons
 // Each lane owns CH points, GT apart: prefix products of z, one inversion, back-substitution.
 // Infinity (z == 0) is skipped in the product and written as all-zero limbs.
 template <bool AFFINE_OUT, int CH> __global__ void __launch_bounds__(GT) k_g1_normalize(void* outv, const G1Jac* in, size_t n) {
+    urgent();
     const size_t base = (size_t)blockIdx.x * GT * CH + threadIdx.x;
     if (base >= n) return;
     Fp pre[CH];
@@ -628,8 +632,8 @@ __device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t 
     }
     D[(size_t)MW * n + i] = (int8_t)((flip != neg1 ? 1 : 0) | (flip ? 2 : 0));
 }
-__global__ void __launch_bounds__(256) k_msm_recode(const RecodeBatch rb, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(GT) k_msm_recode(const RecodeBatch rb, size_t n) {      // one wave a workgroup: as k_tail_levels
+    const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i >= n) return;
     msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i]);
 }
@@ -898,8 +902,10 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
     bucket_shares_merge(pool, p29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
 }
 // raw buckets of up to 8 consecutive segments summed: out[(row * gridDim.y + group) * MT + t], row = sum * MW + w
-__global__ void __launch_bounds__(MT) k_msm_bucket_fold(P29* __restrict__ out, const P29* __restrict__ buckets, uint32_t nseg) {
-    const uint32_t t = threadIdx.x, row = blockIdx.x, grp = blockIdx.y;
+__global__ void __launch_bounds__(GT) k_msm_bucket_fold(P29* __restrict__ out, const P29* __restrict__ buckets, uint32_t nseg) {
+    urgent();
+    constexpr uint32_t PER = MT / GT;                      // workgroups of one wave a row (as k_tail_levels)
+    const uint32_t t = (blockIdx.x % PER) * GT + threadIdx.x, row = blockIdx.x / PER, grp = blockIdx.y;
     const uint32_t s0 = grp * 8, s1 = (s0 + 8 < nseg) ? s0 + 8 : nseg;
     const P29* b = buckets + (size_t)row * nseg * MT;
     P29 acc = b[(size_t)s0 * MT + t];
@@ -924,6 +930,7 @@ __device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
 }
 // win[sum * MW + w]: the windows' sums.  grid: MW workgroups a sum, then MW / 8 a sum of few elements
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_windows(P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t first_few) {
+    urgent();
     __shared__ int32_t pool[3][16][44];                     // of each four lanes: S, V, T below
     const uint32_t q = threadIdx.x & 3u, g = threadIdx.x >> 2;
     const bool few = blockIdx.x >= MW * first_few;          // the same for the workgroup
@@ -985,6 +992,7 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
 }
 // grid: eight sums a wave
 __global__ void __launch_bounds__(GT) k_msm_horner(const P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t n) {
+    urgent();
     const uint32_t q = threadIdx.x & 3u, sum = (blockIdx.x * GT + threadIdx.x) >> 3, half = (threadIdx.x >> 2) & 1u;
     const P29* __restrict__ W = win + (size_t)(sum < n ? sum : n - 1) * MW + half * MWH;
     P29 r = W[MWH - 1];
@@ -1057,6 +1065,7 @@ __global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch
 // is a sum over as many generators as its T0 and T1 together, so this halves what is summed.  T of the rounds above `again` (0: none) is unrolled
 // from T of round `again`.  U: the challenges, opening y's at U + y * ustride
 __global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__ D0, const Fr* __restrict__ U, uint32_t ustride, uint32_t R, uint32_t again) {
+    urgent();
     const uint32_t np = 3 * (R - 1), terms = (R - 1) * np, i = blockIdx.x * 256 + threadIdx.x;
     if (i >= terms) return;
     const Fr* __restrict__ u = U + (size_t)blockIdx.y * ustride;
@@ -1406,6 +1415,7 @@ k_open_span_slices(const SpanBatch sb, const JsfK* __restrict__ jsfs, size_t old
     }
 }
 __global__ void __launch_bounds__(GT) k_open_span_walk(const SpanBatch sb, size_t new_size, uint32_t slice) {
+    urgent();
     const size_t m = ((size_t)blockIdx.x * GT + threadIdx.x) >> 2;
     const uint32_t q = threadIdx.x & 3u;
     if (m >= new_size) return;
@@ -1511,43 +1521,49 @@ __global__ void __launch_bounds__(256) k_a29_canon(A29* __restrict__ a, size_t n
 // final generator are multi-scalar multiplications over the same n0 affine points with coefficients that are plain field
 // arithmetic; they run as one launch instead of a chain of rounds that each wait for a scalar multiplication.
 // Folded scalars of all levels: level 0 is S itself, level j >= 1 sits at SL + sum_{1<=i<j} n_i, n_i = ceil(n0 / 2^i).
-struct TailPtrs { Fr* SL[OB_MAX]; const Fr* S[OB_MAX]; };      // per opening of a batch (blockIdx.x of k_tail_scalars, blockIdx.y of k_tail_scalars3 and k_tail_coeffs)
-// three levels at once, a lane for every eight scalars
-__global__ void __launch_bounds__(256) k_tail_scalars3(const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0) {
-    const uint32_t g = blockIdx.x * 256 + threadIdx.x, n1 = (n0 + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2;
-    if (g >= n3) return;
+struct TailPtrs { Fr* SL[OB_MAX]; const Fr* S[OB_MAX]; };      // per opening of a batch (blockIdx.x of k_tail_scalars, blockIdx.y of k_tail_levels and k_tail_coeffs)
+// One wave a workgroup: beside a kernel of many single waves that hold every SIMD's registers, four waves at once found no room on a compute unit until
+// that kernel's queue had drained (in an opening of 128 x 131072: 670 to 1370 us for 16384 scalars, 13 alone and 56 so).
+static constexpr int TAIL_T = 64;
+// L levels at once, a lane for every 2^L scalars
+template <int L> __global__ void __launch_bounds__(TAIL_T) k_tail_levels(const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0) {
+    urgent();
+    uint32_t n[L + 1];
+    n[0] = n0;
+#pragma unroll
+    for (int k = 0; k < L; ++k) n[k + 1] = (n[k] + 1) / 2;
+    const uint32_t g = blockIdx.x * TAIL_T + threadIdx.x;
+    if (g >= n[L]) return;
     const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
     const Fr* __restrict__ S = tp.S[blockIdx.y];
-    Fr* __restrict__ L1 = tp.SL[blockIdx.y];
-    Fr* __restrict__ L2 = L1 + n1;
-    Fr* __restrict__ L3 = L2 + n2;
-    Fr v[8];
+    Fr* __restrict__ out = tp.SL[blockIdx.y];
+    Fr v[1 << L];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = 8 * g + i < n0 ? S[8 * g + i] : big_zero<8>();      // a missing scalar counts as zero: s0 - u s0
+    for (int i = 0; i < (1 << L); ++i) v[i] = (g << L) + i < n0 ? S[(g << L) + i] : big_zero<8>();      // a missing scalar counts as zero: s0 - u s0
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
+    for (int k = 0; k < L; ++k) {
         const Fr u = usu[k];
-        const uint32_t nk = k == 0 ? n1 : (k == 1 ? n2 : n3), per = 4u >> k;
-        Fr* __restrict__ L = k == 0 ? L1 : (k == 1 ? L2 : L3);
 #pragma unroll
-        for (int i = 0; i < (4 >> k); ++i) {
+        for (int i = 0; i < (1 << (L - 1 - k)); ++i) {
+            const uint32_t at = (g << (L - 1 - k)) + i;
             v[i] = add(v[2 * i], mont_mul(u, sub(v[2 * i + 1], v[2 * i])));
-            if (per * g + i < nk) L[per * g + i] = v[i];
+            if (at < n[k + 1]) out[at] = v[i];
         }
+        out += n[k + 1];
     }
 }
 // U: the tail's challenges (Montgomery form), opening y's at U + y * ustride
-// One workgroup per opening (the levels follow each other behind a barrier) of TAIL_SCALAR_T lanes: four waves find room on
-// a compute unit whose SIMDs each hold a point kernel's waves; the sixteen of a 1024-lane workgroup waited milliseconds for it.
-static constexpr int TAIL_SCALAR_T = 256;
-__global__ void __launch_bounds__(TAIL_SCALAR_T) k_tail_scalars(const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels) {
+// the last levels, of at most TAIL_SHORT scalars: one wave per opening
+static constexpr size_t TAIL_SHORT = 512;
+__global__ void __launch_bounds__(TAIL_T) k_tail_scalars(const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels) {
+    urgent();
     const Fr* __restrict__ usu = U + (size_t)blockIdx.x * ustride;
     const Fr* cur = tp.S[blockIdx.x];
     Fr* nxt = tp.SL[blockIdx.x];
     uint32_t n = n0;
     for (uint32_t j = 0; j < levels; ++j) {
         const uint32_t ns = (n + 1) / 2;
-        for (uint32_t g = threadIdx.x; g < ns; g += TAIL_SCALAR_T) {
+        for (uint32_t g = threadIdx.x; g < ns; g += TAIL_T) {
             const Fr s0 = cur[2 * g];
             nxt[g] = (2 * g + 1 < n) ? add(s0, mont_mul(usu[j], sub(cur[2 * g + 1], s0))) : sub(s0, mont_mul(usu[j], s0));
         }
@@ -1559,8 +1575,9 @@ __global__ void __launch_bounds__(TAIL_SCALAR_T) k_tail_scalars(const TailPtrs t
 }
 // C[(3j+0)*n0 + k] = s_j[k>>j] W_j(k); C[(3j+1)*n0 + k] = s_j[(k>>j)-1] W_j(k) for odd k>>j; C[(3j+2)*n0 + k] = s_j[(k>>j)+1] W_j(k)
 // for even k>>j with a partner; zero elsewhere.  C[3*levels*n0 + k] = W_levels(k) when `final_gen`.
-__global__ void __launch_bounds__(256) k_tail_coeffs(Fr* __restrict__ C0, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels, uint32_t final_gen) {
-    const uint32_t k = blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(TAIL_T) k_tail_coeffs(Fr* __restrict__ C0, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels, uint32_t final_gen) {
+    urgent();
+    const uint32_t k = blockIdx.x * TAIL_T + threadIdx.x;
     if (k >= n0) return;
     const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
     Fr* __restrict__ C = C0 + (size_t)blockIdx.y * (3 * levels + final_gen) * n0;
@@ -1839,7 +1856,7 @@ static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1
         const uint32_t ng = (ns + 7) / 8;
         Scratch& nxt = arena.add(sizeof(P29) * n_msm * MW * (size_t)ng * MT);
         if (nxt.rc) return nxt.rc;
-        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW, ng), dim3(MT), 0, st, nxt.as<P29>(), cur, ns);
+        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW * (MT / GT), ng), dim3(GT), 0, st, nxt.as<P29>(), cur, ns);
         cur = nxt.as<P29>();
         ns = ng;
     }
@@ -1880,7 +1897,7 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
         digits = dig.as<int8_t>();
         RecodeBatch rb;
         for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>() + dig_bytes * (i < count ? i : 0); rb.S[i] = items[i < count ? i : 0].scalars; }
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(old_size, 256), count), dim3(256), 0, st, rb, old_size);
+        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(old_size, GT), count), dim3(GT), 0, st, rb, old_size);
         ZK_LAUNCH_CHECK();
         int rc = join_streams(st, aux, events);
         if (rc) return rc;
@@ -2336,15 +2353,20 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     const TailPtrs all = tp;
     size_t n = n0, off = 0;               // off: where the level just formed starts
     for (int j = 0; j < levels;) {
-        if (levels - j >= 3 && (n > 2048 || levels == 3)) {
-            hipLaunchKernelGGL(k_tail_scalars3, dim3(cdiv((n + 7) / 8, 256), count), dim3(256), 0, st, tp, U_dev + r0 + j, (uint32_t)rounds, (uint32_t)n);
-            const size_t n1 = (n + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2;
-            for (int i = 0; i < OB_MAX; ++i) { tp.S[i] = tp.SL[i] + n1 + n2; tp.SL[i] += n1 + n2 + n3; }
+        if (n > TAIL_SHORT) {
+            const int L = std::min(3, levels - j);
+            const dim3 grid(cdiv((n + (1u << L) - 1) >> L, TAIL_T), count);
+            const Fr* u = U_dev + r0 + j;
+            if (L == 3) hipLaunchKernelGGL(k_tail_levels<3>, grid, dim3(TAIL_T), 0, st, tp, u, (uint32_t)rounds, (uint32_t)n);
+            else if (L == 2) hipLaunchKernelGGL(k_tail_levels<2>, grid, dim3(TAIL_T), 0, st, tp, u, (uint32_t)rounds, (uint32_t)n);
+            else hipLaunchKernelGGL(k_tail_levels<1>, grid, dim3(TAIL_T), 0, st, tp, u, (uint32_t)rounds, (uint32_t)n);
+            size_t before = 0;            // the levels in front of the last one
+            for (int k = 0; k < L; ++k) { n = (n + 1) / 2; if (k + 1 < L) before += n; }
+            for (int i = 0; i < OB_MAX; ++i) { tp.S[i] = tp.SL[i] + before; tp.SL[i] += before + n; }
             off = (size_t)(tp.S[0] - sl.as<Fr>());
-            n = n3;
-            j += 3;
+            j += L;
         } else {
-            hipLaunchKernelGGL(k_tail_scalars, dim3(count), dim3(TAIL_SCALAR_T), 0, st, tp, U_dev + r0 + j, (uint32_t)rounds, (uint32_t)n, (uint32_t)(levels - j));
+            hipLaunchKernelGGL(k_tail_scalars, dim3(count), dim3(TAIL_T), 0, st, tp, U_dev + r0 + j, (uint32_t)rounds, (uint32_t)n, (uint32_t)(levels - j));
             off = (size_t)(tp.SL[0] - sl.as<Fr>());
             for (; j < levels; ++j) { n = (n + 1) / 2; if (j + 1 < levels) off += n; }
         }
@@ -2354,11 +2376,11 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     if (rc) return rc;
     const A29* before[OB_MAX];
     for (int i = 0; i < count; ++i) before[i] = gens[i];
-    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, 256), count), dim3(256), 0, aux, coef.as<Fr>(), all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, fin);
+    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, TAIL_T), count), dim3(TAIL_T), 0, aux, coef.as<Fr>(), all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, fin);
     {
         RecodeBatch rb;
         for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>(); rb.S[i] = coef.as<Fr>(); }
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, 256), 1), dim3(256), 0, aux, rb, ncoef);
+        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, GT), 1), dim3(GT), 0, aux, rb, ncoef);
     }
     ZK_LAUNCH_CHECK();
     if (!last) {          // behind the short kernels of the other stream: they would wait for the fold's workgroups otherwise
@@ -2546,7 +2568,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
             if (sl.rc) return sl.rc;
             TailPtrs tp;
             for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; tp.SL[i] = sl.as<Fr>() + sl_n * k; tp.S[i] = cs[k]; }
-            hipLaunchKernelGGL(k_tail_scalars3, dim3(cdiv(ns, 256), count), dim3(256), 0, st, tp, U_dev, (uint32_t)rounds, (uint32_t)n);
+            hipLaunchKernelGGL(k_tail_levels<3>, dim3(cdiv(ns, TAIL_T), count), dim3(TAIL_T), 0, st, tp, U_dev, (uint32_t)rounds, (uint32_t)n);
             ZK_LAUNCH_CHECK();
             int rc = open_span_fold(cg, count, n, 0, items, job.arena, job.up, st);
             if (rc) return rc;
