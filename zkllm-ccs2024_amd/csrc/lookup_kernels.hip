@@ -380,8 +380,10 @@ static int hist_partitioned(uint32_t* counts, const KeySrc idx, size_t n, uint32
 // counters cross memory once, in lines; adding them to global ones costs an atomic for nearly every query where these spread.
 // 2^22 queries in 2^16 bins: partitioned 163 us, this way 30 us.
 // Up to four times as many entries: a workgroup for every 65536 of them reads the same share and counts those that are its own, where there are
-// as many queries as entries.  825000 queries in 2^18 bins: 42 us by global atomics, 22 this way.
+// as many queries as entries and fewer than 2^23.  A mapping's proof into 2^18 bins: 300 x 2750 queries 496 us by global atomics, 472 this way; 2^20 650 us
+// partitioned, 570 this way, 2^22 800 and 770, 16 million 2.11 and 2.16 ms (every range reads the queries).
 static constexpr uint32_t HW_BINS = 65536, HW_SHARE = 32768, HW_T = 1024, HW_SLICES = 8, HW_RANGES = 4, HW_AHEAD = 4;
+static constexpr size_t HWR_MAX_QUERIES = (size_t)1 << 23;
 __global__ void __launch_bounds__(HW_T) k_hist_wide(uint32_t* __restrict__ part, const KeySrc idx, size_t n, uint32_t words) {
     __shared__ __attribute__((aligned(16))) uint32_t h[HW_BINS / 2];
     const uint32_t first = blockIdx.y * (HW_BINS / 2), own = words - first < HW_BINS / 2 ? words - first : HW_BINS / 2;
@@ -2238,7 +2240,7 @@ int zk_lookup_multiplicities(void* m, void* idx_out, const void* idx, const void
     ZK_ARG(nbins >= 1 && len >= 1 && len <= nbins, "zk_lookup_multiplicities: need 1 <= len <= nbins");
     ZK_ARG(m != nullptr && (idx != nullptr || vals_i32 != nullptr || vals != nullptr || n == 0), "zk_lookup_multiplicities: null argument");
     const unsigned ranges = cdiv(nbins, HW_BINS);
-    const bool wide = nbins > HIST_LDS_BINS && n >= 1 && n < ((size_t)1 << 27) && (ranges == 1 || (ranges <= HW_RANGES && n >= nbins));
+    const bool wide = nbins > HIST_LDS_BINS && n >= 1 && n < ((size_t)1 << 27) && (ranges == 1 || (ranges <= HW_RANGES && n >= nbins && n < HWR_MAX_QUERIES));
     const unsigned shares = wide ? (unsigned)std::max<size_t>(std::min<size_t>(cdiv(n, (size_t)8192), 256 / ranges), cdiv(n, (size_t)HW_SHARE)) : 0u;
     const uint32_t words = (nbins + 1) / 2;
     Scratch counts(sizeof(uint32_t) * ((wide ? (size_t)shares * words : (size_t)nbins) + 1), st);      // the first word: the flag
