@@ -211,7 +211,7 @@ class FrTensor {
 };
 
 // Results that arrive later (zk_defer_begin / _end / _wait of the C ABI).  Between begin() and end() the calling thread's
-// evaluations and inner-product rounds (FrTensor::operator()(u), multi_dim_me, zk_ip_round, zk_ip_sumcheck_small) only queue
+// evaluations and inner-product rounds (FrTensor::operator()(u), multi_dim_me, zk_ip_round, zk_ip_sumcheck_small, zk_matmul_sumcheck) only queue
 // their kernels: what they return is NOT their result.  wait() delivers the results of those calls in call order, each with
 // the layout of its C entry point.  For proofs whose challenges are all known up front: the device side is queued in one go,
 // the host side (checks, transcript entries) runs when the values are collected.
