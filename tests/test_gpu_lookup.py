@@ -1,6 +1,9 @@
 """GPU parity: multiplicities, batch inversion, the two-phase lookup sumcheck, range / mapping tables,
 rescaling, multi-Hadamard sumcheck, stacked inner-product sumcheck and zkSoftmax -- bit-exact against the oracle."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -401,6 +404,44 @@ def test_mapping_lookup_with_int32_forms(pv, orc, D, low, length):
     assert (y.host() == e_y).all() and (m.host() == e_m).all() and (fin == e_fin).all()
     t = pv.transcript()
     assert t.shape == e_t.shape and (t == e_t).all()
+
+
+def mapping_against_the_oracle(D, low, length, kept):
+    """One mapping proof in this process: queries with an int32 form or without, the blocks that its padded copies get full of other elements."""
+    from gpuhelp import Prover
+    pv, orc = Prover(), load_oracle()
+    rng = np.random.default_rng(D + 2)
+    vals = rng.integers(low, low + length, D)
+    mv = fr_array([int(v) % R_MOD for v in rng.integers(-2 ** 31, 2 ** 31, length)])
+    S = fr_array([int(v) % R_MOD for v in vals])
+    k = (D - 1).bit_length()
+    r, alpha, beta, u, v = ch(7, 1)[0], ch(8, 1)[0], ch(9, 1)[0], ch(10, k), ch(11, k)
+    e_y, e_m, e_fin = np.zeros((D, 8), np.uint32), np.zeros((1 << (length - 1).bit_length(), 8), np.uint32), np.zeros(8, np.uint32)
+    orc.orc_transcript_clear()
+    orc_check(orc.orc_mapping(S, D, low, length, mv, r, alpha, beta, u, v, e_y, e_m, e_fin))
+    e_t = orc_transcript(orc)
+    hS, hv = pv.from_i64(vals.astype(np.int64)), pv.from_fr(mv)
+    if kept:
+        pv.keep_for_folds(hS)
+    junk = [pv.from_fr(ch(12 + i, 1 << k)) for i in range(4)]
+    del junk
+    pv.transcript_begin()
+    y, m, fin = pv.mapping(hS, low, length, hv, r, alpha, beta, u, v)
+    pv.lib.zkp_transcript_end()
+    assert (y.host() == e_y).all() and (m.host() == e_m).all() and (fin == e_fin).all()
+    t = pv.transcript()
+    assert t.shape == e_t.shape and (t == e_t).all()
+
+
+@pytest.mark.parametrize("switch", ["ZKLLM_FR_LIMBS=32", "ZKLLM_LOOKUP_TWO_ROUNDS=0", "ZKLLM_LOOKUP_TRUSTED=0"])
+def test_mapping_lookup_of_padded_queries_on_every_first_round(switch):
+    """The first rounds that the environment chooses between (read once a process, so each runs in a child): the padded outputs exist in their
+    int32 form alone, whether the queries keep one or not, and none of these rounds may read their field elements.  70001 queries: one
+    first round of its own (padded to 2^17); 300000: the size of the first two rounds in one pass (2^19)."""
+    code = "import test_gpu_lookup as t\nfor D in (70001, 300000):\n    for kept in (False, True):\n        print(D, kept, flush=True)\n        t.mapping_against_the_oracle(D, -16, 32, kept)\n"
+    name, value = switch.split("=")
+    r = subprocess.run([sys.executable, "-c", code], cwd=os.path.dirname(os.path.abspath(__file__)), env=dict(os.environ, **{name: value}), capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout[-300:] + r.stderr[-1500:]
 
 
 @pytest.mark.parametrize("D,low,length", [(1 << 17, -(1 << 9), 1 << 10), (1 << 18, -(1 << 7), 1 << 8), (1 << 19, -(1 << 15), 1 << 16)])

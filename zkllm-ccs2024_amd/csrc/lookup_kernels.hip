@@ -593,7 +593,7 @@ struct HintSrc { const Fr* TB; const Fr* hint; Fr low; Fr beta; uint32_t N; cons
                  // the table record.
                  const uint32_t* n_ok = nullptr; bool trusted_out = false;
                  // fr_queries: hint_ints is null and the queries' integers are taken from the field elements in hint (a query that is no
-                 // 32-bit integer is inverted on its own)
+                 // 32-bit integer is inverted on its own); S_out, where there is one, need hold nothing: every first round reads sout_ints
                  bool fr_queries = false; };
 static constexpr int32_t INTS_POISON = (int32_t)0x80000000;
 __device__ __forceinline__ Fr hinted_query(const Fr* __restrict__ S, size_t i, const HintSrc& h) {
@@ -715,6 +715,9 @@ k_lookup_round(Fr* __restrict__ partials, Fr* __restrict__ nA, Fr* __restrict__ 
             if (HINTED && hs.hint_ints) {
                 s0r = query_inv_ints(t, hs, a0, unit0);
                 s1 = query_inv_ints(t + n_out, hs, a1, unit1);
+            } else if (HINTED && hs.fr_queries) {      // (a mapping table's outputs may exist in their int32 form alone)
+                s0r = query_inv_ints<true>(t, hs, a0, unit0);
+                s1 = query_inv_ints<true>(t + n_out, hs, a1, unit1);
             } else {
                 s0r = HINTED ? hinted_query(S, t, hs) : S[t];
                 s1 = HINTED ? hinted_query(S, t + n_out, hs) : S[t + n_out];
