@@ -223,7 +223,8 @@ int zk_ip_sumcheck_small(uint32_t* polys_host, uint32_t* fin_host, const void* a
 /* The device side of zkFC::prove (zkfc.cu:61-87) for Y [B][O] = X [B][D] W [D][O]: claim = Y at (u_batch, u_output); X folded at u_batch and W
  * at u_output; every round of zkip on the two vectors (3 kd coefficients); the folded values, which are X and W at the proof's point.
  * Field for field what zk_fr_fold_axis_all, zk_fr_me and zk_ip_sumcheck_small give.  2^(k-1) < n <= 2^k on every axis; kb and
- * ko at most 14, kd 1 to 13.  While results are deferred it delivers 3 kd + 3 elements in the order of its arguments. */
+ * ko at most 14, kd 1 to 13.  While results are deferred it delivers 3 kd + 3 elements in the order of its arguments, and the host pointers
+ * for them may be null. */
 int zk_matmul_sumcheck(uint32_t* claim_host, uint32_t* polys_host, uint32_t* fin_host, const void* X, const void* W, const void* Y, uint32_t B, uint32_t D, uint32_t O,
                        const uint32_t* u_batch, int kb, const uint32_t* u_input, int kd, const uint32_t* u_output, int ko, void* stream);
 

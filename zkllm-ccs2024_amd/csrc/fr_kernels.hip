@@ -1231,6 +1231,9 @@ int zk_matmul_sumcheck(uint32_t* claim_host, uint32_t* polys_host, uint32_t* fin
     auto fits = [](uint32_t n, int k, int most) { return k >= 0 && k <= most && n >= 1 && n <= (1u << k) && n > ((1u << k) >> 1); };
     ZK_ARG(kd >= 1 && fits(D, kd, 13), "zk_matmul_sumcheck: inner axis: 1 to 13 challenges, 2^(k-1) < D <= 2^k");
     ZK_ARG(fits(B, kb, EQ29_MAX) && fits(O, ko, EQ29_MAX), "zk_matmul_sumcheck: outer axes: at most 14 challenges, 2^(k-1) < n <= 2^k");
+    ZK_ARG(X != nullptr && W != nullptr && Y != nullptr, "zk_matmul_sumcheck: null operand or result");
+    ZK_ARG(u_input != nullptr && (kb == 0 || u_batch != nullptr) && (ko == 0 || u_output != nullptr), "zk_matmul_sumcheck: null challenges");
+    ZK_ARG(deferring() || (claim_host != nullptr && polys_host != nullptr && fin_host != nullptr), "zk_matmul_sumcheck: null output");      // (deferred: delivered elsewhere)
     FcFolds a;
     a.X = (const Fr*)X; a.W = (const Fr*)W; a.Y = (const Fr*)Y;
     a.B = B; a.D = D; a.O = O;

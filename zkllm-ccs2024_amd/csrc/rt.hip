@@ -271,6 +271,7 @@ struct DeferBatch {
 };
 thread_local DeferBatch* g_defer = nullptr;
 }  // namespace
+bool deferring() { return g_defer != nullptr; }
 int deliver_begin(Delivery& d, size_t count_fr, int n_mont) {
     using Fr = Big<8>;
     d.count = count_fr;

@@ -95,6 +95,7 @@ int staging(void** host_ptr, size_t bytes);
 // thread has a batch of deferred results open (zk_defer_begin) the place is in the batch's buffer, nothing is waited for, host_dst is NOT
 // written, and zk_defer_wait hands the values out later, in the order of the deliver_begin calls.
 struct Delivery { void* dst = nullptr; size_t count = 0; int n_mont = 0; bool deferred = false; };
+bool deferring();
 int deliver_begin(Delivery& d, size_t count_fr, int n_mont);
 int deliver_end(const Delivery& d, hipStream_t st, void* host_dst);
 
