@@ -6,7 +6,8 @@ GPU with weights, generators, commitments and the input already resident in HBM:
 projections, 32 attention heads (QK^T, zkSoftmax, YV), SwiGLU FFN, every rescaling / lookup / sumcheck and
 the opening of all nine weight commitments.  `value` is seconds per layer.
 
-The same JSON line also carries the layer time without the openings and with the nine commitments included, the
+One JSON line on standard output carries the figures; the full record, with a note on what each of them is, goes to standard error ahead of it.
+The line also has the layer time without the openings and with the nine commitments included, the
 two throughput figures of the headline metric (G1 MSM points/s on the 4096 x 11008 commitment workload, Fr
 multiplications/s) with their roofline fractions, a roofline entry for the kernel with the largest share of the
 layer's GPU time (timed with HIP events around its launches inside the timed region), roofline entries of the first
@@ -133,6 +134,40 @@ def drivers_leg(seq):
     finally:
         shutil.rmtree(tmp, ignore_errors=True)
     return out
+
+
+CONTRACT = ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling", "vs_baseline", "dtype", "data")
+LINE_MAX = 7800      # whoever records the line keeps the last 8000 characters of the output: a longer one loses its head, and with it the figure
+
+
+def line_of(out):
+    """The record as the one line of output: every figure (those beside the headline to six digits), texts cut to 72 characters, notes left out.
+    Entries that would take it past LINE_MAX characters are left out, the last first, and named in "left_out"."""
+    def short(x):
+        if isinstance(x, bool) or x is None or isinstance(x, int):
+            return x
+        if isinstance(x, float):
+            return float("%.6g" % x)
+        if isinstance(x, str):
+            return x if len(x) <= 72 else x[:69] + "..."
+        if isinstance(x, dict):
+            return {k: short(v) for k, v in x.items() if k != "note" and not k.endswith("_note")}
+        return [short(v) for v in x]
+    line = {k: v if k in CONTRACT else short(v) for k, v in out.items()}
+    chain = line.get("drivers_chain")
+    if isinstance(chain, dict) and "runs" in chain:      # the phases of every run are in the full record
+        line["drivers_chain"] = {"wall_s": [[r["run"], r["wall_s"]] for r in chain["runs"]], **{k: chain[k] for k in ("chain_wall_s", "chain_prove_s", "setup_s") if k in chain}}
+    left_out = []
+    while len(json.dumps(line)) > LINE_MAX and any(k not in CONTRACT + ("config", "left_out") for k in line):
+        left_out.insert(0, [k for k in line if k not in CONTRACT + ("config", "left_out")][-1])
+        del line[left_out[0]]
+        line["left_out"] = left_out
+    return json.dumps(line)
+
+
+def emit(out):
+    print("full record: " + json.dumps(out), file=sys.stderr, flush=True)
+    print(line_of(out), flush=True)
 
 
 def main():
@@ -445,7 +480,8 @@ def main():
         "vs_baseline": None,
         "dtype": "u32",
         "data": "synthetic",
-        "config": {"workload": f"C5: LLaMa-2-7B-shape decoder layer proof, seq {seq}, hidden 4096, 32 heads x 128, FFN 11008, "
+        "config": {"model": "LLaMa-2-7B decoder layer", "global_batch": 1, "seq_len": seq, "parallelism": "one GPU",
+                   "workload": f"C5: LLaMa-2-7B-shape decoder layer proof, seq {seq}, hidden 4096, 32 heads x 128, FFN 11008, "
                                "random-init fixed-point weights (scale 2^16), generators of size out_features<<5, all nine weight openings included "
                                "(value: their points are read ahead from the seeded challenge stream, so all nine run from the start of the layer, batched by "
                                "generator size; layer_openings_at_claim_s: the same layer with every opening started at its claim and the attention proof, which opens nothing, queued and collected behind the last block; layer_openings_at_claim_blocks_in_turn_s: that, and every "
@@ -526,7 +562,7 @@ def main():
                     "multiply-add peak; the launches share the device with each other, with the openings and with the main stream.  Alone at 2^25 pairs the "
                     "kernel takes 2.12 ms: 3.8 TB/s and 70 % of the vector issue slots -- both sides bind"}
     if args.skip_extras:
-        print(json.dumps(out))
+        emit(out)
         return
 
     # ---- the same fold kernel alone at its largest per-opening shape in the layer: one halving of 2^19 generators ----
@@ -814,7 +850,7 @@ def main():
             out["drivers_chain"] = drivers_leg(args.seq)
         except Exception as e:          # never loses the headline line
             out["drivers_chain"] = {"error": str(e)[:600]}
-    print(json.dumps(out))
+    emit(out)
     lib.zk_shutdown()
 
 
