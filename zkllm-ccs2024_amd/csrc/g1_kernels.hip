@@ -2076,8 +2076,12 @@ static uint32_t msm_first_levels(size_t rows, uint32_t levels) {
     return logs;
 }
 // Digit width, windows and segments for m rows of ngen scalars.  seen[b]: how many of the sampled scalars have b bits.  Estimated times in us:
-// an entry of the table costs 0.12 ns, a level of it 60 us at least (one lane's inversion) or 30 among the first ones (k_msm_table_first, 50 us besides),
+// a level of the table counts 60 us (one lane's inversion) or 30 among the first ones (k_msm_table_first, 50 us besides) and 0.12 ns an entry,
 // a base's doubling 7 us of latency, an addition 0.17 ns; a digit beyond the first is an addition where the scalar reaches it.
+// These are weights for the choice and not the kernels' times: in k_msm_table_grow an entry of a large level takes 0.24 ns, its 60 us included, and an
+// addition 0.18 (11008 x 4096 of 13 bits).  Every width timed, 1 to 11008 rows of 64 to 4096 generators and scalars of 13 and of 28 bits (48 shapes):
+// the one chosen here takes 4 % longer than the best on average.  The furthest off are 28-bit scalars in few rows of 64 generators, 14 % (3 bits chosen,
+// 7 are best), 512 rows of 4096, 12 % (9, 7), and many rows of 28 bits, 7 % (13, 9); the same model fitted to those times chooses no better (5 %).
 struct MsmShape { uint32_t c, nwin, top, nseg; };
 static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs, const uint32_t* seen) {
     MsmShape best{0, 0, 0, 1};
@@ -2495,7 +2499,9 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     else cross_r = std::min(cross_r, halving);
     // What round r over `size` generators begins.  Three rounds as a batch of sums beside one fold where a round's fold would leave the chip
     // half empty and take one walk's latency all the same; above that a round at a time, which sums over fewer points.  Openings of 128 x 2^17,
-    // the first round alone / in a span: 9.9 / 9.2 ms; of 16 x 2^18, two rounds alone / one and a span: 14.7 / 14.9.
+    // the first round alone / in a span: 9.9 / 9.2 ms; of 16 x 2^18, two rounds alone / one and a span: 14.7 / 14.9.  One opening with the line at 2^16, 2^17
+    // and 2^18 generators of a job, in ms: of 147456 generators 11.0, 10.4, 11.3; 163840 11.2, 10.8, 11.8; 196608 12.8, 11.8, 12.8; 229376 14.0, 13.4,
+    // 14.0; 2^18 14.9, 14.2, 15.3; of 2^17 9.0, 8.9.  Three of 65536 at once 12.8, 12.4, 12.4; five of 32768 11.5, 11.0, 12.0; six 13.5, 12.7, 13.3.
     enum Step { LAST, SPAN, ROUND };
     auto step_of = [&](size_t size, int r) {
         if (last_batch(size, r)) return LAST;

@@ -382,6 +382,8 @@ static int hist_partitioned(uint32_t* counts, const KeySrc idx, size_t n, uint32
 // Up to four times as many entries: a workgroup for every 65536 of them reads the same share and counts those that are its own, where there are
 // as many queries as entries and fewer than 2^23.  A mapping's proof into 2^18 bins: 300 x 2750 queries 496 us by global atomics, 472 this way; 2^20 650 us
 // partitioned, 570 this way, 2^22 800 and 770, 16 million 2.11 and 2.16 ms (every range reads the queries).
+// More ranges than four would not pay: into 2^19 bins 825000 queries 587 us by the ways below, 568 in ranges, 2^21 653 and 635, 2^22 equal, 2^23 - 1 1.33
+// and 1.43 ms; into 2^20 bins 2^20 715 and 694, 2^21 800 and 808, 2^22 973 and 1080, 2^23 - 1 1.48 and 1.74 ms.
 static constexpr uint32_t HW_BINS = 65536, HW_SHARE = 32768, HW_T = 1024, HW_SLICES = 8, HW_RANGES = 4, HW_AHEAD = 4;
 static constexpr size_t HWR_MAX_QUERIES = (size_t)1 << 23;
 __global__ void __launch_bounds__(HW_T) k_hist_wide(uint32_t* __restrict__ part, const KeySrc idx, size_t n, uint32_t words) {
