@@ -686,7 +686,7 @@ def main():
     hip.check(lib.zk_prof_gemm_read(ctypes.byref(g_ms), ctypes.byref(g_launches), ctypes.byref(g_macs)))
     if g_launches.value:
         g_tops = 2 * g_macs.value / (g_ms.value * 1e-3) / 1e12
-        out["roofline_matmul_mfma"] = {"kernel": "k_gemm_i8_planes_all<3,2> (v_mfma_i32_32x32x32_i8 over base-256 digit planes: three of the activations, two of the weights; 2048x4096x4096, exact)", "bound": "mfma",
+        out["roofline_matmul_mfma"] = {"kernel": "k_gemm_i8_planes_all<3, 2, 128> (v_mfma_i32_32x32x32_i8 over base-256 digit planes: three of the activations, two of the weights; 2048x4096x4096, exact)", "bound": "mfma",
                                        "achieved": g_tops, "peak": 5000.0, "unit": "TOP/s", "frac": g_tops / 5000.0, "traffic": None,
                                        "avg_launch_ms": g_ms.value / g_launches.value, "plane_pairs": g_macs.value / g_launches.value / (M * N * P),
                                        "whole_product_ms": mm_call_ms,

@@ -1508,13 +1508,6 @@ __global__ void __launch_bounds__(GT) k_a29_to_jac(G1Jac* __restrict__ out, cons
     if (i >= n) return;
     out[i] = a29_is_inf(in[i]) ? g1_infinity() : aff_to_jac(a29_to_affine(in[i]));
 }
-__global__ void __launch_bounds__(256) k_a29_canon(A29* __restrict__ a, size_t n) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    A29 v = a[i];
-    v.x = fq29_canon(v.x); v.y = fq29_canon(v.y);
-    a[i] = v;
-}
 // ---- rounds in one batch ------------------------------------------------------------------------------------------------
 // Over n0 generators, every later round's generators are fixed linear combinations of these n0 points: g at level j, block i, is
 // sum over k in block i of W_j(k) g_k with W_j(k) = prod_{b<j} (bit_b(k) ? 1-u_b : u_b).  So T, T0, T1 of any number of rounds and the

@@ -508,14 +508,7 @@ static int batch_inv_queue(Fr* out, const Fr* in, const Fr& beta, size_t n, hipS
 }
 
 // ---- eq tables ----------------------------------------------------------------------------------------------------------
-// E[t] = prod_j (u_j if bit_j(t) else 1-u_j), Montgomery form.  Built by doubling: level j appends bit j.
-__global__ void __launch_bounds__(TPB) k_eq_double(Fr* __restrict__ e, const Fr u_mont, const Fr one_minus_u_mont, size_t half) {
-    const size_t t = (size_t)blockIdx.x * TPB + threadIdx.x;
-    if (t >= half) return;
-    const Fr x = e[t];
-    e[t + half] = mont_mul(x, u_mont);
-    e[t] = mont_mul(x, one_minus_u_mont);
-}
+// E[t] = prod_j (u_j if bit_j(t) else 1-u_j), Montgomery form: the products of two half tables' entries (k_eq_halves, k_eq_outer) or of three small ones' (k_eq_tabs)
 // dropping the top variable: E'[t] = E[t] + E[t + n_out]
 __global__ void __launch_bounds__(TPB) k_eq_halve(Fr* __restrict__ out, const Fr* __restrict__ in, size_t n_out) {
     const size_t t = (size_t)blockIdx.x * TPB + threadIdx.x;
@@ -3383,7 +3376,7 @@ int zk_lookup_prove_end(void* handle, uint32_t* bm_host, uint32_t* sums_host) {
     sumjob_abort(job);
     return rc;
 }
-// Measurement: time every launch of the hinted first round (k_lookup_round<false, true>) between begin and read, with events
+// Measurement: time every launch of a first round over hinted queries (k_lookup_first2_29, k_lookup_first29, k_lookup_round<false, true>) between begin and read, with events
 // on the launch stream.  bytes: the algorithmic traffic of those launches.
 static void round_timer_begin(RoundTimer& T) {
     std::lock_guard<std::mutex> lk(T.mu);
