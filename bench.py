@@ -194,7 +194,7 @@ def main():
     args = ap.parse_args()
     if args.gpus != 1:
         print("bench.py: this prover runs on one GPU; every configuration of the benchmark fits a single MI355X, "
-              "so --gpus must be 1 (no multi-GPU path exists in this build)", file=sys.stderr)
+              "so --gpus must be 1 (it has no multi-GPU path)", file=sys.stderr)
         sys.exit(2)
 
     if args.drivers_only:

@@ -2,7 +2,7 @@
 //
 // Nothing that ships (the HIP library, the host class layer, the drivers) may include,
 // link or call this file; only tests/, the smoke check and the benchmark's cpu_baseline
-// leg use it, as the checker.
+// leg use it, to compare against.
 //
 // Plain host C++ restatement of the reference's BLS12-381 field and curve routines:
 //   Fr  (8 x u32 limbs, R = 2^256)  bls12-381.cu:245-300 (gte/eq/add_/sub_/add/sub),
