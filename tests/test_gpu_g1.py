@@ -252,7 +252,7 @@ def test_open_with_equal_scalars(pv, orc, n, val):
 
 @pytest.mark.parametrize("counts", [[1, 64], [96, 97, 107], [400, 113], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
 def test_open_with_several_digits_shared_by_many_scalars(pv, orc, counts):
-    """Few scalars (512 at most, a path of its own) and many: buckets about the size from which a workgroup shares them out, whose ends fall inside and at
+    """Few scalars (256 at most, a path of its own) and many: buckets about the size from which a workgroup shares them out, whose ends fall inside and at
     the ends of the lanes' shares."""
     n = sum(counts)
     gens = oracle_gens(orc, 41 + n, n)
@@ -648,6 +648,56 @@ def test_span_of_rounds_whose_slices_meet_themselves(slice_bits, sign, first):
     assert_points_are(points, logs)
     hip.free(dG)
     hip.free(dS)
+
+
+# one batch of sums of 2^13 to 2^14 generators, whose T all follow from the final generator and scalar, unless a challenge is 0 or 1
+@pytest.mark.parametrize("n", [8193, 16384])
+@pytest.mark.parametrize("at,to", [(0, None), (0, 0), (12, 1), (5, R_MOD - 1)])
+def test_open_whose_sums_follow_from_its_last_round(n, at, to):
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    k = (n - 1).bit_length()
+    a, S, u = special_logarithms(96, n), mt_random_vec(np.random.RandomState(97), n), fr_ints(mt_random_vec(np.random.RandomState(98), k))
+    if to is not None:
+        u[at] = to
+    dG, dS = known_generators(hip, a), hip.upload(S)
+    points, value = np.zeros((3 * k + 1, 36), np.uint32), np.zeros(8, np.uint32)
+    print(f"zk_g1_open n={n} u[{at}] = {to}", flush=True)
+    hip.call("zk_g1_open", points, value, c_void_p(dS), c_void_p(dG), c_size_t(n), fr_array(u), c_int(k), None)
+    logs, exp_value = opening_logarithms(a, fr_ints(S), u)
+    assert fr_ints(value)[0] == exp_value
+    assert_points_are(points, logs)
+    hip.free(dG)
+    hip.free(dS)
+
+
+def test_open_round_whose_lists_are_sorted_a_few_windows_at_a_time():
+    """One round over so many generators that the lists of all windows of its three sums do not fit the sorting's space: small and large scalars, every eighth of them zero."""
+    from gpuhelp import Hip, c_int, c_size_t, c_void_p
+    hip = Hip()
+    n, period = 1600000, 1 << 12
+    a = special_logarithms(130, period)
+    S = np.random.RandomState(131).randint(0, 1 << 32, (n, 8), dtype=np.uint64).astype(np.uint32)
+    S[:, 7] %= 1944954707
+    S[::8] = 0
+    S[::3, 1:] = 0
+    reps = -(-n // period)
+    dA, dG = hip.upload(np.tile(fr_array(a), (reps, 1))[:n]), hip.malloc(144 * n)
+    hip.call("zk_g1_fixed_base_mul", c_void_p(dG), np.ascontiguousarray(affine_to_jac((G1_X, G1_Y)), dtype=np.uint32), c_void_p(dA), c_size_t(n), None)
+    hip.sync()
+    dS, u = hip.upload(S), mt_random_vec(np.random.RandomState(132), 1)
+    points, value = np.zeros((4, 36), np.uint32), np.zeros(8, np.uint32)
+    print(f"zk_g1_open n={n}, one round", flush=True)
+    hip.call("zk_g1_open", points, value, c_void_p(dS), c_void_p(dG), c_size_t(n), u, c_int(1), None)
+    # the generators repeat with the period: the sum of all scalars that meet one of them
+    tot = np.zeros((period, 8), np.int64)
+    pad = np.concatenate([S, np.zeros((reps * period - n, 8), np.uint32)]).reshape(reps, period, 8)
+    tot = pad.astype(np.int64).sum(axis=0)
+    s = [sum(int(v) << (32 * l) for l, v in enumerate(row)) for row in tot]
+    exp = [sum(map(mul, s, a)) % R_MOD, sum(map(mul, s[0::2], a[1::2])) % R_MOD, sum(map(mul, s[1::2], a[0::2])) % R_MOD]
+    assert_points_are(points[:3], exp)
+    for p in (dA, dG, dS):
+        hip.free(p)
 
 
 # 4099 x 8 and 33001: the first and the second round on their tables (odd halves); 12300 x 8: the first alone without tables, or on its table;

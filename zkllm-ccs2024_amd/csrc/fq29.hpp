@@ -559,7 +559,7 @@ template <bool INL> ZK_HD P29 p29_add(const P29& a, const P29& b) {
 template <int CTRL> __device__ __forceinline__ Fq29 quad_perm(const Fq29& a) {
     Fq29 r;
 #pragma unroll
-    for (int i = 0; i < 14; ++i) r.l[i] = __builtin_amdgcn_update_dpp(0, a.l[i], CTRL, 0xF, 0xF, false);
+    for (int i = 0; i < 14; ++i) r.l[i] = __builtin_amdgcn_mov_dpp(a.l[i], CTRL, 0xF, 0xF, true);      // every lane of a quad is there: no old value to keep
     return r;
 }
 template <int FROM> __device__ __forceinline__ Fq29 quad_get(const Fq29& a) { return quad_perm<FROM * 0x55>(a); }

@@ -452,22 +452,28 @@ __global__ void __launch_bounds__(256) k_fr_to_i32_checked(int32_t* __restrict__
 // and publishes T = sum [s_j] g_j, T0 = sum [s_2i] g_2i+1, T1 = sum [s_2i+1] g_2i.  The reference spends five
 // 255-bit scalar multiplications per pair on this.  Here
 //  * T0 and T1 (and T of the first round) are bucket multi-scalar multiplications over the affine-normalised
-//    generators: 8-bit signed windows, one workgroup per (sum, window, segment), one bucket per lane;
+//    generators: signed windows of 8 to 12 bits, the elements sorted by bucket, one bucket per lane;
 //  * T of every later round follows from the previous round's three points, because <s', g'> expands to
-//    u(1-u) T + (1-u)^2 T0 + u^2 T1;
+//    u(1-u) T + (1-u)^2 T0 + u^2 T1, or all T from the last round's result the other way round;
 //  * the one remaining scalar multiplication per pair, by the round's common challenge u, uses the curve
 //    endomorphism (x, y) -> (beta x, y) = [lambda](x, y): u = k1 + k2 lambda with k1, k2 < 2^128 (r = lambda^2 +
 //    lambda + 1, so this is one integer division on the host), then 128 doublings instead of 255.
 // The endomorphism and the expansion of T hold for points of the order-r subgroup, which is where the
 // generators live (Commitment::random draws multiples of the group generator, commitment.cu:9-20).
 // All rounds are queued without a host round trip; the proof points come back in one copy, normalised to z = 1.
-static constexpr int MW = 32;        // 8-bit signed windows of a scalar split as k1 + k2 lambda: 16 of each half
+static constexpr int MW = 32;        // bytes of a scalar split as k1 + k2 lambda: 16 of each half
 static constexpr int MWH = MW / 2;
-static constexpr int MT = 128;       // buckets of a window (digit magnitudes 1..128)
-static constexpr int MSEG = 4096;    // most elements of a chunk (12-bit list entries)
-static constexpr int MSL = 64;       // lanes of a bucket-accumulation workgroup (one wave): each takes two buckets of its chunk
-static constexpr int MHEAVY = 96;    // a bucket above this many elements of a chunk is shared out over the workgroup
-struct MsmDesc { const int8_t* digits; const A29* base; uint32_t dstride, count, s_mul, s_off, b_mul, b_off; };   // element i: recoded scalar i*s_mul+s_off of dstride, point base[i*b_mul+b_off]
+static constexpr int MT = 128;       // buckets that a wave of k_msm_windows reduces
+static constexpr int MSL = 64;       // lanes of a bucket-accumulation workgroup (one wave)
+static constexpr int MHB = 2048;     // most buckets of a window
+static constexpr int MPIECE = 128;   // most elements of a bucket that one lane adds up
+static constexpr int MFEWP = 8;      // most pieces that one lane puts together
+// element i: recoded scalar i*s_mul+s_off of dstride, point base[i*b_mul+b_off]; list_at: the counts of the sums before this one
+struct MsmDesc { const void* digits; const A29* base; uint32_t dstride, count, s_mul, s_off, b_mul, b_off, list_at, pad; };
+// How scalars are written for their sums: nwh windows a half, the first 128 % nwh of them one bit wider than the rest (bias: a half of every
+// window's range), or (nwh = 0) the bytes that k_msm_few reads
+struct DigitPlan { uint32_t nwh, bias[4]; };
+static inline size_t digit_bytes(const DigitPlan& p) { return p.nwh ? 4 * (size_t)p.nwh : (size_t)MW + 1; }       // of a scalar
 static constexpr int OB_MAX = 8;           // openings of equal size that share their rounds' launches
 static constexpr int TABLE_MIN_N = 1024;   // results of a fold below which no fold tables are made for it
 static constexpr int LAST_N = 16384;       // generators of a job (all its openings together) at which the remaining rounds are computed in one batch
@@ -529,14 +535,18 @@ static __device__ __attribute__((noinline)) G1Jac g1_mul_glv(const G1Jac& P, con
     return out;
 }
 
-// Signed 8-bit digits of every scalar, written window-major: the scalar is split as +-k1 +-k2 lambda with |k1|, |k2| < 2^127
-// ([lambda](x, y) = (beta x, y), see glv_beta), D[w*n + i] in [-128, 127] is digit w of |k1| for w < MWH and digit w - MWH of |k2|
-// above, and D[MW*n + i] says which halves are subtracted (bit 0: k1, bit 1: k2).  The halves share the points they are summed over;
-// what the split buys is the end of a sum, whose Horner walk over the windows is 120 doublings instead of 248.
+// Signed digits of every scalar, written window-major: the scalar is split as +-k1 +-k2 lambda with |k1|, |k2| < 2^127
+// ([lambda](x, y) = (beta x, y), see glv_beta).  The halves share the points they are summed over;
+// what the split buys is the end of a sum, whose Horner walk over the windows is about 117 doublings instead of 248.
 // The smaller of s and r - s is split (weights are embedded as small values of either sign: a value below lambda / 2 is its own k1,
-// and its high windows are empty).  A window byte above 127 becomes byte - 256 and carries one into the next window; the top byte
-// of a half is at most 0x57, so the carry ends there.
-struct RecodeBatch { int8_t* D[OB_MAX]; const Fr* S[OB_MAX]; };      // blockIdx.y names the pair
+// and its high windows are empty).
+// A plan of nwh windows a half: D (int16) [w*n + i] is digit w of +-k1 for w < nwh and digit w - nwh of +-k2 above.  With half of every
+// window's range added to |k| beforehand, the digits are bits of that sum less the half range, without carries from window to window:
+// |k| is at most 2^126.44 and the halves together below 2^127.02, so the sum has 128 bits.
+// The bytes of k_msm_few: D[w*n + i] in [-128, 127] is digit w of |k1| for w < MWH and digit w - MWH of |k2| above, and D[MW*n + i] says
+// which halves are subtracted (bit 0: k1, bit 1: k2).  A window byte above 127 becomes byte - 256 and carries one into the next window; the
+// top byte of a half is at most 0x57, so the carry ends there.
+struct RecodeBatch { void* D[OB_MAX]; const Fr* S[OB_MAX]; };      // blockIdx.y names the pair
 // a = round(x / lambda) and k1 = x - a lambda for x < 2^254: the quotient's estimate is the high half of x times 2^256 / lambda, at
 // most one short, and the remainder's comparison with lambda / 2 mends it.  k1 comes as magnitude and sign.
 __device__ __forceinline__ void glv_split_centred(const uint32_t* x, uint32_t (&k1)[4], bool& k1_neg, uint32_t (&a)[4]) {
@@ -602,7 +612,7 @@ __device__ __forceinline__ void glv_split_centred(const uint32_t* x, uint32_t (&
     }
 }
 // the digits of scalar i of n (standard form)
-__device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t n, size_t i, const Fr& sv) {
+__device__ __forceinline__ void msm_recode_store(void* __restrict__ Dv, size_t n, size_t i, const Fr& sv, const DigitPlan& plan) {
     Fr ng;
     uint32_t br = 0;
 #pragma unroll
@@ -616,6 +626,27 @@ __device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t 
 #pragma unroll
     for (int l = 0; l < 8; ++l) x[l] = flip ? ng.v[l] : sv.v[l];
     glv_split_centred(x, k1, neg1, k2);
+    if (plan.nwh) {
+        int16_t* __restrict__ D = reinterpret_cast<int16_t*>(Dv);
+        const uint32_t q = 128u / plan.nwh, rem = 128u % plan.nwh;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool neg = h ? flip : flip != neg1;
+            uint32_t v[4], c = 0;
+#pragma unroll
+            for (int l = 0; l < 4; ++l) v[l] = addc32(h ? k2[l] : k1[l], plan.bias[l], c);
+            for (uint32_t w = 0; w < plan.nwh; ++w) {
+                const uint32_t width = q + (w < rem ? 1u : 0u), range = 1u << width;
+                const int dg = (int)(v[0] & (range - 1u)) - (int)(range >> 1);
+                D[(size_t)(h * plan.nwh + w) * n + i] = (int16_t)(neg ? -dg : dg);
+#pragma unroll
+                for (int l = 0; l < 3; ++l) v[l] = v[l] >> width | v[l + 1] << (32u - width);
+                v[3] >>= width;
+            }
+        }
+        return;
+    }
+    int8_t* __restrict__ D = reinterpret_cast<int8_t*>(Dv);
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         uint32_t carry = 0;
@@ -632,10 +663,17 @@ __device__ __forceinline__ void msm_recode_store(int8_t* __restrict__ D, size_t 
     }
     D[(size_t)MW * n + i] = (int8_t)((flip != neg1 ? 1 : 0) | (flip ? 2 : 0));
 }
-__global__ void __launch_bounds__(GT) k_msm_recode(const RecodeBatch rb, size_t n) {      // one wave a workgroup: as k_tail_levels
+// What the sums behind a recoding count with (SortState), cleared by its first workgroup
+__device__ __forceinline__ void clear_state(uint32_t* __restrict__ state, uint32_t words) {
+    if (blockIdx.x == 0 && blockIdx.y == 0)
+        for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) state[i] = 0u;
+}
+__global__ void __launch_bounds__(GT) k_msm_recode(const RecodeBatch rb, size_t n, const DigitPlan plan, uint32_t* __restrict__ state, uint32_t state_words) {      // one wave a workgroup: as k_tail_levels
+    urgent();
+    clear_state(state, state_words);
     const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
     if (i >= n) return;
-    msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i]);
+    msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i], plan);
 }
 
 static constexpr int P29_WORDS = 42;
@@ -678,163 +716,202 @@ __device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, P29 x, bool 
     }
 }
 
-// One segment's share of sum over elements of digit_w(s) * base: the segment's MT raw buckets,
-// partial[((sum * MW + w) * nseg + seg) * MT + b] for bucket magnitude b + 1 (k_msm_bucket_fold, k_msm_windows and k_msm_horner reduce them).
-// One wave per workgroup.  Per chunk of `chunk` elements (at most MSEG):
-//  1. the bucket sizes are counted (one LDS atomic per element) and the elements are sorted by bucket into one list in
-//     LDS (counting sort: 12-bit position in the chunk + sign);
-//  2. the buckets are ranked by size and lane j takes the j-th largest and the j-th smallest: list lengths of uniform
-//     digits are Poisson(32), the largest of 64 is ~47, while the 64 pair sums all lie within a few elements of 64 -- the
-//     lanes walk their two lists as one sequence of mixed additions, in lockstep, and 96 % of the lane-steps add a point
-//     (67 % with one bucket per lane);
-//  3. buckets with more than MHEAVY elements (scalars that share a digit: equal values, small integers, a common high byte) stand
-//     together at the end of the list, which the lanes divide evenly: a lane's share is shorter than such a bucket, so it holds parts of
-//     at most two.  A bucket that ends inside a share goes out there; the rest is a segmented scan over the lanes, six additions for
-//     all of them together.  An opening of 1 x 16384 small integers: 10.7 ms with a tree of six additions a bucket above 256
-//     elements and one lane's walk below, 5.0 ms so.
-__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_seg(P29* __restrict__ partial, const MsmDesc* __restrict__ descs, uint32_t nseg, uint32_t chunks_per_seg, uint32_t chunk) {
-    __shared__ uint32_t cnt[MT], off[MT], cursor[MT];
-    __shared__ uint8_t order[MT], heavy[MT];
-    __shared__ uint32_t pool[P29_WORDS * MSL];     // the sorted list (u16 x MSEG), then the points of the heavy buckets' scan
-    static_assert(P29_WORDS * MSL * 4 >= MSEG * 2, "pool too small for the list");
-    static_assert(MSEG <= 4096, "12-bit list entries");
-    static_assert(MSEG / MSL < MHEAVY, "a lane's share of the heavy buckets' list touches two of them at most");
-    static_assert(MT == 2 * MSL, "a lane counts two buckets");
-    uint16_t* list = reinterpret_cast<uint16_t*>(pool);
-    const MsmDesc d = descs[blockIdx.z];
-    const A29* __restrict__ A = d.base;
-    const uint32_t w = blockIdx.y, seg = blockIdx.x, t = threadIdx.x, zz = blockIdx.z;
-    const int8_t* __restrict__ Dw = d.digits + (size_t)w * d.dstride;
-    const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
-    const uint32_t half = w / (uint32_t)MWH;
-    P29* __restrict__ out = partial + (((size_t)zz * MW + w) * nseg + seg) * MT;
-    bool first = true;                                  // nothing written to `out` yet (the same for every lane)
-    for (uint32_t ch = 0; ch < chunks_per_seg; ++ch) {
-        const uint32_t e0 = (seg * chunks_per_seg + ch) * chunk;
-        if (e0 >= d.count) break;
-        const uint32_t e1 = (e0 + chunk < d.count) ? e0 + chunk : d.count;
-        cnt[t] = 0; cnt[t + MSL] = 0;
-        __syncthreads();
-        for (uint32_t e = e0 + t; e < e1; e += MSL) {
-            const int dg = Dw[(size_t)e * d.s_mul + d.s_off];
-            if (dg != 0) atomicAdd(&cnt[(dg < 0 ? -dg : dg) - 1], 1u);
-        }
-        __syncthreads();
-        // the lists one after the other, those of the heavy buckets last: lane t places buckets 2t and 2t + 1
-        uint32_t n_light, n_heavy, n_hb;
-        {
-            const uint32_t c0 = cnt[2 * t], c1 = cnt[2 * t + 1];
-            const bool h0 = c0 > (uint32_t)MHEAVY, h1 = c1 > (uint32_t)MHEAVY;
-            const uint32_t mine = (h0 ? 0u : c0) + (h1 ? 0u : c1);                                      // at most 2 MHEAVY
-            const uint32_t mine_h = (h0 ? c0 : 0u) + (h1 ? c1 : 0u);
-            uint32_t run = mine, run_h = mine_h | ((uint32_t)h0 + (uint32_t)h1) << 16;                   // elements, and buckets above bit 16
-            for (int sd = 1; sd < MSL; sd <<= 1) {
-                const uint32_t a = __shfl_up(run, sd), ah = __shfl_up(run_h, sd);
-                if (t >= (uint32_t)sd) { run += a; run_h += ah; }
-            }
-            n_light = __shfl(run, MSL - 1);
-            n_heavy = __shfl(run_h, MSL - 1) & 0xFFFFu;
-            n_hb = __shfl(run_h, MSL - 1) >> 16;
-            const uint32_t l0 = run - mine, g0 = n_light + (run_h & 0xFFFFu) - mine_h;
-            const uint32_t o0 = h0 ? g0 : l0, o1 = h1 ? g0 + (h0 ? c0 : 0u) : l0 + (h0 ? 0u : c0);
-            off[2 * t] = o0; cursor[2 * t] = o0;
-            off[2 * t + 1] = o1; cursor[2 * t + 1] = o1;
-            const uint32_t k0 = (run_h >> 16) - (uint32_t)h0 - (uint32_t)h1;
-            if (h0) heavy[k0] = (uint8_t)(2 * t);
-            if (h1) heavy[k0 + (uint32_t)h0] = (uint8_t)(2 * t + 1);
-        }
-        // rank of a bucket by list length (heavy buckets have none), ties by index: a permutation
-        for (uint32_t b = t; b < (uint32_t)MT; b += MSL) {
-            const uint32_t cb = cnt[b] > (uint32_t)MHEAVY ? 0u : cnt[b];
-            uint32_t r = 0;
-            for (uint32_t o = 0; o < (uint32_t)MT; ++o) {
-                const uint32_t co = cnt[o] > (uint32_t)MHEAVY ? 0u : cnt[o];
-                r += (co > cb || (co == cb && o < b)) ? 1u : 0u;
-            }
-            order[r] = (uint8_t)b;
-        }
-        __syncthreads();
-        for (uint32_t e = e0 + t; e < e1; e += MSL) {
-            const size_t si = (size_t)e * d.s_mul + d.s_off;
-            const int dg = Dw[si];
-            if (dg == 0) continue;
-            const uint32_t mag = (uint32_t)(dg < 0 ? -dg : dg);
-            const uint32_t pos = atomicAdd(&cursor[mag - 1], 1u);
-            list[pos] = (uint16_t)((e - e0) | (((dg < 0) != (((Df[si] >> half) & 1) != 0)) ? 0x8000u : 0u));
-        }
-        __syncthreads();
-        {
-            const uint32_t bA = order[t], bB = order[MT - 1 - t];
-            const uint32_t lenA = cnt[bA] > (uint32_t)MHEAVY ? 0u : cnt[bA], lenB = cnt[bB] > (uint32_t)MHEAVY ? 0u : cnt[bB];
-            const uint32_t total = lenA + lenB;
-            uint32_t pos = off[bA];
-            X29 acc29 = x29_infinity();
-            for (uint32_t i = 0;; ++i) {
-                if (i == lenA) {
-                    // the end of the first list: its bucket goes out (added to what earlier chunks of this segment left there)
-                    P29 v = p29_from_x29(acc29);
-                    if (!first) v = p29_add<false>(out[bA], v);
-                    out[bA] = v;
-                    acc29 = x29_infinity();
-                    pos = off[bB];
-                }
-                if (i >= total) break;
-                const uint32_t en = list[pos++];
-                A29 pt = A[(size_t)(e0 + (en & 0x7FFFu)) * d.b_mul + d.b_off];
-                if (a29_is_inf(pt)) continue;
-                if (en & 0x8000u) pt.y = fq29_neg(pt.y);
-                x29_add_mixed(acc29, pt);
-            }
-            P29 v = p29_from_x29(acc29);
-            if (!first) v = p29_add<false>(out[bB], v);
-            out[bB] = v;
-        }
-        __threadfence_block();
-        __syncthreads();
-        if (n_hb) {                                         // the same for every lane
-            const uint32_t share = (n_heavy + MSL - 1) / MSL, end = n_light + n_heavy;
-            const uint32_t p0 = min(n_light + t * share, end), p1 = min(p0 + share, end);
-            uint32_t k = 0;
-            while (k + 1 < n_hb && off[heavy[k + 1]] <= p0) ++k;
-            uint32_t b = heavy[k], b_end = off[b] + cnt[b];
-            bool start = p0 >= end || p0 == off[b];          // what the lane holds begins its bucket (or is nothing)
-            bool lacks = false;                             // bucket `split` went out without the shares before this lane's
-            uint32_t split = 0;
-            X29 acc29 = x29_infinity();
-            for (uint32_t pos = p0; pos < p1; ++pos) {
-                if (pos == b_end) {
-                    P29 v = p29_from_x29(acc29);
-                    if (!first) v = p29_add<false>(out[b], v);
-                    out[b] = v;
-                    split = b; lacks = !start; start = true;
-                    acc29 = x29_infinity();
-                    b = heavy[++k]; b_end = off[b] + cnt[b];
-                }
-                const uint32_t en = list[pos];
-                A29 pt = A[(size_t)(e0 + (en & 0x7FFFu)) * d.b_mul + d.b_off];
-                if (a29_is_inf(pt)) continue;
-                if (en & 0x8000u) pt.y = fq29_neg(pt.y);
-                x29_add_mixed(acc29, pt);
-            }
-            const bool whole = p1 > p0 && p1 == b_end;       // the bucket ends with this share
-            bucket_shares_merge(pool, p29_from_x29(acc29), start, whole, b, lacks, split, out, first, t);
-        }
-        __threadfence_block();
-        __syncthreads();
-        first = false;
+// Bucket sums, [(sum * 2 nwh + w) * hb + b] for magnitude b + 1 of window w of a sum, in four launches over the windows w0 .. w0 + gridDim.x - 1:
+//  1. k_msm_sort: a workgroup a window sorts the sum's elements by bucket (counting sort in LDS) into one list in memory, the point's index and
+//     the digit's sign an entry, and counts the buckets by size.  A bucket above `most` elements (scalars that share a digit: equal values,
+//     small integers) is cut into pieces of equal size.
+//  2. k_msm_tasks: the buckets and pieces of ALL sums and windows ordered by size, the longest first.
+//  3. k_msm_lists: a lane adds up the points of one bucket or piece.  The 64 of a wave are of one size, so its lanes are busy to the end, and
+//     the waves get shorter towards the end of the launch, so that the chip empties at once.
+//  4. k_msm_merge: a lane puts the pieces of a bucket together, a wave those of a bucket in many.
+// Bound by the instructions of 3.  That the lists lie in memory is what lets windows be wider than 8 bits (22 additions an element with 11 windows a half instead
+// of 32).  The sums of an opening of 128 x 131072 alone: 0.20 ms of sorting and 2.3 ms of k_msm_lists at 76 % of the issue slots; with 8-bit windows, a wave for the 128 buckets of a chunk and
+// a window sorted in LDS, and the chunks' buckets added up, 5.5 + 0.3 ms at 66 %: the whole opening 8.7 -> 6.8 ms, of 16 x 4096 2.19 -> 1.45 ms.
+static constexpr uint32_t SORT_CURSOR = MPIECE + 1, SORT_PARTS = 2 * (MPIECE + 1), SORT_CUT = SORT_PARTS + 1, SORT_HEAVY = SORT_CUT + 1, SORT_WORDS = SORT_HEAVY + 1;
+// what the four launches share; state: tasks of each size, how many of a size are placed, pieces, cut buckets
+// heavy: buckets of few pieces from the front, those of more than MFEWP from the back of `cuts` entries
+struct SortSpace { uint32_t* state; uint4* info; uint32_t* lists; uint4* heavy; uint4* tasks; P29* buckets; uint32_t nwh, hb, w0, total, most, parts_at, cuts; };
+__device__ __forceinline__ uint32_t sort_wave_scan(uint32_t v, uint32_t lane) {      // inclusive
+    for (int sd = 1; sd < 64; sd <<= 1) {
+        const uint32_t a = __shfl_up(v, sd);
+        if (lane >= (uint32_t)sd) v += a;
     }
-    if (first) {                                       // a segment past the end of this sum: empty buckets
-        out[t] = p29_infinity();
-        out[t + MSL] = p29_infinity();
+    return v;
+}
+template <int BT> __global__ void __launch_bounds__(BT) k_msm_sort(const SortSpace sp, const MsmDesc* __restrict__ descs) {
+    urgent();
+    __shared__ uint32_t cursor[MHB], sizes[MPIECE + 1], wave_sum[3][BT / 64], at_part, at_cut, at_heavy;
+    constexpr int AHEAD = 8;
+    const MsmDesc d = descs[blockIdx.y];
+    const uint32_t t = threadIdx.x, w = sp.w0 + blockIdx.x, row = blockIdx.y * 2 * sp.nwh + w, list0 = blockIdx.x * sp.total + d.list_at;
+    const int16_t* __restrict__ Dw = reinterpret_cast<const int16_t*>(d.digits) + (size_t)w * d.dstride + d.s_off;
+    for (uint32_t b = t; b < sp.hb; b += BT) cursor[b] = 0;
+    for (uint32_t b = t; b <= (uint32_t)MPIECE; b += BT) sizes[b] = 0;
+    __syncthreads();
+    for (uint32_t e = t; e < d.count; e += BT * AHEAD) {
+        int dg[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) dg[k] = e + k * BT < d.count ? (int)Dw[(size_t)(e + k * BT) * d.s_mul] : 0;
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+            if (dg[k] != 0) atomicAdd(&cursor[(dg[k] < 0 ? -dg[k] : dg[k]) - 1], 1u);
+    }
+    __syncthreads();
+    const uint32_t per = (sp.hb + BT - 1) / BT, b0 = min(t * per, sp.hb), b1 = min(b0 + per, sp.hb);
+    uint32_t mine = 0, parts = 0, cuts = 0;                 // elements, pieces, cut buckets and above bit 16 those of more than MFEWP pieces
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t c = cursor[b], np = (c + sp.most - 1) / sp.most;
+        mine += c;
+        if (np > 1) { parts += np; cuts += np > (uint32_t)MFEWP ? 0x10000u : 1u; }
+    }
+    uint32_t run = sort_wave_scan(mine, t & 63u), run_parts = sort_wave_scan(parts, t & 63u), run_cuts = sort_wave_scan(cuts, t & 63u);
+    if ((t & 63u) == 63u) { wave_sum[0][t >> 6] = run; wave_sum[1][t >> 6] = run_parts; wave_sum[2][t >> 6] = run_cuts; }
+    __syncthreads();
+    run -= mine; run_parts -= parts; run_cuts -= cuts;
+    for (uint32_t k = 0; k < t >> 6; ++k) { run += wave_sum[0][k]; run_parts += wave_sum[1][k]; run_cuts += wave_sum[2][k]; }
+    if (t == BT - 1 && run_parts + parts) {
+        const uint32_t c = run_cuts + cuts;
+        at_part = atomicAdd(&sp.state[SORT_PARTS], run_parts + parts);
+        at_cut = atomicAdd(&sp.state[SORT_CUT], c & 0xFFFFu);
+        at_heavy = atomicAdd(&sp.state[SORT_HEAVY], c >> 16);
+    }
+    __syncthreads();
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t c = cursor[b], np = (c + sp.most - 1) / sp.most, at = row * sp.hb + b;
+        uint32_t slot = 0;
+        cursor[b] = run;
+        if (np == 1) atomicAdd(&sizes[c], 1u);
+        else if (np > 1) {
+            const uint32_t len = c / np, more = c % np;
+            if (more) atomicAdd(&sizes[len + 1], more);
+            atomicAdd(&sizes[len], np - more);
+            const bool many = np > (uint32_t)MFEWP;
+            slot = at_part + run_parts;
+            sp.heavy[many ? sp.cuts - 1 - (at_heavy + (run_cuts >> 16)) : at_cut + (run_cuts & 0xFFFFu)] = make_uint4(at, sp.parts_at + slot, np, 0u);
+            run_parts += np;
+            run_cuts += many ? 0x10000u : 1u;
+        } else sp.buckets[at] = p29_infinity();
+        sp.info[at] = make_uint4(list0 + run, c, sp.parts_at + slot, 0u);
+        run += c;
+    }
+    __syncthreads();
+    if (t <= (uint32_t)MPIECE && sizes[t]) atomicAdd(&sp.state[t], sizes[t]);
+    for (uint32_t e = t; e < d.count; e += BT * AHEAD) {
+        int dg[AHEAD];
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k) dg[k] = e + k * BT < d.count ? (int)Dw[(size_t)(e + k * BT) * d.s_mul] : 0;
+#pragma unroll
+        for (int k = 0; k < AHEAD; ++k)
+            if (dg[k] != 0) sp.lists[list0 + atomicAdd(&cursor[(dg[k] < 0 ? -dg[k] : dg[k]) - 1], 1u)] = ((e + k * BT) * d.b_mul + d.b_off) | (dg[k] < 0 ? 0x80000000u : 0u);
     }
 }
-// The same for sums of few elements: the 8-bit digits taken as two signed 4-bit digits each, so that a sum has 512 buckets (64 windows
+static constexpr int TASK_T = 256;
+static_assert(TASK_T > MPIECE, "a lane for every size");
+__global__ void __launch_bounds__(TASK_T) k_msm_tasks(const SortSpace sp) {
+    urgent();
+    __shared__ uint32_t all[MPIECE + 1], at[MPIECE + 1], own[MPIECE + 1];
+    const uint32_t t = threadIdx.x, row = blockIdx.y * 2 * sp.nwh + sp.w0 + blockIdx.x;
+    const uint4* __restrict__ info = sp.info + (size_t)row * sp.hb;
+    if (t <= (uint32_t)MPIECE) { all[t] = sp.state[t]; own[t] = 0; }
+    __syncthreads();
+    for (uint32_t b = t; b < sp.hb; b += TASK_T) {
+        const uint32_t c = info[b].y, np = (c + sp.most - 1) / sp.most;
+        if (np == 0) continue;
+        const uint32_t len = c / np, more = c % np;
+        if (more) atomicAdd(&own[len + 1], more);
+        atomicAdd(&own[len], np - more);
+    }
+    __syncthreads();
+    if (t <= (uint32_t)MPIECE && own[t]) {
+        uint32_t before = 0;
+        for (uint32_t l = t + 1; l <= (uint32_t)MPIECE; ++l) before += all[l];
+        at[t] = before + atomicAdd(&sp.state[SORT_CURSOR + t], own[t]);
+        own[t] = 0;
+    }
+    __syncthreads();
+    for (uint32_t b = t; b < sp.hb; b += TASK_T) {
+        const uint4 in = info[b];
+        const uint32_t np = (in.y + sp.most - 1) / sp.most;
+        if (np == 0) continue;
+        const uint32_t len = in.y / np, more = in.y % np;
+        uint32_t from = in.x;
+        for (uint32_t p = 0; p < np; ++p) {
+            const uint32_t l = len + (p < more ? 1u : 0u);
+            sp.tasks[at[l] + atomicAdd(&own[l], 1u)] = make_uint4(from, l, np == 1 ? row * sp.hb + b : in.z + p, blockIdx.y);
+            from += l;
+        }
+    }
+}
+__global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_lists(const SortSpace sp, const MsmDesc* __restrict__ descs) {
+    const uint32_t t = threadIdx.x, id = blockIdx.x * MSL + t;
+    uint32_t n = 0;                                         // tasks
+    for (uint32_t l = t; l <= (uint32_t)MPIECE; l += MSL) n += sp.state[l];
+    for (int sd = 1; sd < MSL; sd <<= 1) n += __shfl_xor(n, sd);
+    if (id >= n) return;
+    const uint4 task = sp.tasks[id];
+    const A29* __restrict__ A = descs[task.w].base;
+    const uint32_t* __restrict__ list = sp.lists + task.x;
+    // an entry is sent for two additions ahead, its point one
+    uint32_t en = list[0], en2 = list[min(1u, task.y - 1)];
+    A29 next = A[en & 0x7FFFFFFFu];
+    X29 acc;
+    for (uint32_t i = 0; i < task.y; ++i) {
+        A29 pt = next;
+        if (en >> 31) pt.y = fq29_neg(pt.y);
+        if (i + 1 < task.y) {
+            en = en2;
+            next = A[en & 0x7FFFFFFFu];
+            en2 = list[min(i + 2, task.y - 1)];
+        }
+        if (i == 0) {
+            acc.x = pt.x; acc.y = pt.y;
+            acc.zz = acc.zzz = fq29_one();
+            acc.inf = a29_is_inf(pt) ? 1u : 0u;             // infinity stays infinity when its sign is changed
+        } else if (!a29_is_inf(pt)) x29_add_mixed(acc, pt);
+    }
+    sp.buckets[task.z] = p29_from_x29(acc);
+}
+__global__ void __launch_bounds__(MSL) k_msm_merge(const SortSpace sp) {
+    urgent();
+    __shared__ uint32_t pool[P29_WORDS * MSL];
+    const uint32_t t = threadIdx.x, n = sp.state[SORT_HEAVY], few = sp.state[SORT_CUT];
+    for (uint32_t k = blockIdx.x * MSL + t; k < few; k += gridDim.x * MSL) {
+        const uint4 h = sp.heavy[k];
+        P29 x = sp.buckets[h.y];
+        for (uint32_t p = 1; p < h.z; ++p) x = p29_add<false>(x, sp.buckets[h.y + p]);
+        sp.buckets[h.x] = x;
+    }
+    for (uint32_t k = blockIdx.x; k < n; k += gridDim.x) {
+        const uint4 h = sp.heavy[sp.cuts - 1 - k];
+        const P29* __restrict__ part = sp.buckets + h.y;
+        P29 x = t < h.z ? part[t] : p29_infinity();
+        for (uint32_t p = t + MSL; p < h.z; p += MSL) x = p29_add<false>(x, part[p]);
+        uint32_t* src = reinterpret_cast<uint32_t*>(&x);
+        uint32_t sd = 1;
+        while (sd < (uint32_t)MSL / 2 && 2 * sd < h.z) sd <<= 1;
+        for (; sd > 0; sd >>= 1) {                          // lanes sd .. 2 sd - 1 to those below
+            __syncthreads();
+#pragma unroll
+            for (int l = 0; l < P29_WORDS; ++l) pool[l * MSL + t] = src[l];
+            __syncthreads();
+            if (t < sd) {
+                P29 y;
+                uint32_t* py = reinterpret_cast<uint32_t*>(&y);
+#pragma unroll
+                for (int l = 0; l < P29_WORDS; ++l) py[l] = pool[l * MSL + t + sd];
+                x = p29_add<false>(x, y);
+            }
+        }
+        if (t == 0) sp.buckets[h.x] = x;
+    }
+}
+// Bucket sums of few elements: the 8-bit digits taken as two signed 4-bit digits each, so that a sum has 512 buckets (64 windows
 // of 8) instead of 4096 and the walk over its buckets, which is most of such a sum's work, fits two waves instead of sixteen.  A wave
 // takes nw windows, sorts their elements by bucket in LDS and divides that list evenly over its lanes, whatever the digits are.
 // nw (1, 2, 4 or 8) gives a lane about eight elements, so that the scan behind them costs less than they do.
-// FEW_MAX: an element costs 64 additions here and 32 there, a sum 32 walks here and 256 there; at 512 elements an opening alone takes the
-// same time both ways (1.87 ms), and of a layer of small products, whose 250 sums then leave the chip to the rest, 7.2 ms instead of 7.7.
-static constexpr int FEW_MAX = 512, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T;
+// FEW_MAX: an element costs 64 additions here and 32 there, a sum 512 buckets here and 4096 there; an opening of 8 x 512 alone takes
+// 1.00 ms here, 0.93 sorted, one of 4 x 256 0.91 here.
+static constexpr int FEW_MAX = 256, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T;
 // grid (64 / nw, sums); buckets[(sum * 64 + window) * 8 + magnitude - 1]
 __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_few(P29* __restrict__ buckets, const MsmDesc* __restrict__ descs, uint32_t nw) {
     __shared__ uint32_t cnt[MSL], off[MSL], cursor[MSL];
@@ -844,13 +921,14 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
     const MsmDesc d = descs[blockIdx.y];
     const A29* __restrict__ A = d.base;
     const uint32_t t = threadIdx.x, v0 = blockIdx.x * nw, half = v0 / (FEW_WINDOWS / 2);
-    const int8_t* __restrict__ Df = d.digits + (size_t)MW * d.dstride;
+    const int8_t* __restrict__ D8 = reinterpret_cast<const int8_t*>(d.digits);
+    const int8_t* __restrict__ Df = D8 + (size_t)MW * d.dstride;
     P29* __restrict__ out = buckets + ((size_t)blockIdx.y * FEW_WINDOWS + v0) * FEW_T;
     cnt[t] = 0;
     if (t < nw * FEW_T) out[t] = p29_infinity();
     __syncthreads();
     auto digit = [&](uint32_t v, size_t si) {
-        const int dg = d.digits[(size_t)(v >> 1) * d.dstride + si], hi = (dg + 8) >> 4;
+        const int dg = D8[(size_t)(v >> 1) * d.dstride + si], hi = (dg + 8) >> 4;
         return (v & 1u) ? hi : dg - 16 * hi;
     };
     for (uint32_t j = 0; j < nw; ++j)
@@ -901,25 +979,16 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
     bucket_shares_merge(pool, p29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
 }
-// raw buckets of up to 8 consecutive segments summed: out[(row * gridDim.y + group) * MT + t], row = sum * MW + w
-__global__ void __launch_bounds__(GT) k_msm_bucket_fold(P29* __restrict__ out, const P29* __restrict__ buckets, uint32_t nseg) {
-    urgent();
-    constexpr uint32_t PER = MT / GT;                      // workgroups of one wave a row (as k_tail_levels)
-    const uint32_t t = (blockIdx.x % PER) * GT + threadIdx.x, row = blockIdx.x / PER, grp = blockIdx.y;
-    const uint32_t s0 = grp * 8, s1 = (s0 + 8 < nseg) ? s0 + 8 : nseg;
-    const P29* b = buckets + (size_t)row * nseg * MT;
-    P29 acc = b[(size_t)s0 * MT + t];
-    for (uint32_t sg = s0 + 1; sg < s1; ++sg) acc = p29_add<true>(acc, b[(size_t)sg * MT + t]);
-    out[((size_t)row * gridDim.y + grp) * MT + t] = acc;
-}
-// The sums of a list from the raw buckets of all their windows, in two launches.  k_msm_windows: a wave takes a window, sum_b (b + 1) B[b]:
-// each four lanes the running sums over eight neighbouring buckets (fourteen additions), then a tree over the sixteen of them in which one
-// of four lanes carries the weighted sum and one the plain sum times the buckets below it (eight additions).  A sum of few elements has two sets of 8
-// buckets a window, weighted 1 .. 8 and 16 .. 128: a wave takes eight of its windows.  k_msm_horner: four lanes walk the sixteen windows of a
-// half, 120 doublings, and the halves are added, the endomorphism on the second.
-// All of a job's sums that nothing waits for go into one launch each, those of few elements behind the others (first_few).  Both are chains of one wave's
+// The sums of a list from the raw buckets of all their windows, in two launches, three for windows of more than 128 buckets.  k_msm_windows: a wave takes 128 buckets,
+// sum_b (b + 1) B[b]: each four lanes the running sums over eight neighbouring buckets (fourteen additions), then a tree over the sixteen of them in which one
+// of four lanes carries the weighted sum and one the plain sum times the buckets below it (eight additions).
+// Wider windows: the weighted sums and 128 times the plain sums of their blocks of 128 (BLOCKS), then the same tree over those.  A sum of few elements has two sets of 8
+// buckets a window, weighted 1 .. 8 and 16 .. 128: a wave takes eight of its windows.  k_msm_horner: four lanes walk the windows of a
+// half, 128 doublings less the top window's width, and the halves are added, the endomorphism on the second.
+// All of a job's sums that nothing waits for go into one launch each.  Both are chains of one wave's
 // instructions; the windows are summed before the walk so that 32 waves and two walks of four lanes do what took 256 walks a sum.
-struct PointDesc { P29* buckets; G1Jac* out; uint32_t few, pad; };
+// The list: sums of one number of windows stand together and begin at a multiple of eight (a wave of k_msm_horner; gaps: out = null), those of few elements last.
+struct PointDesc { P29* buckets; P29* blocks; G1Jac* out; uint32_t few, nwh, hb, pad; };
 __device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
     P29 r;
     const int32_t* src = reinterpret_cast<const int32_t*>(&a);
@@ -929,14 +998,20 @@ __device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
     return r;
 }
 // win[sum * MW + w]: the windows' sums.  grid: MW workgroups a sum, then MW / 8 a sum of few elements
-__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_windows(P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t first_few) {
+// BLOCKS: grid (blocks of a sum, sums), the first of the list; blocks[2 (w * hb / MT + block)]: the two sums of a block
+template <bool BLOCKS> __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_windows(P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t first_few) {
     urgent();
     __shared__ int32_t pool[3][16][44];                     // of each four lanes: S, V, T below
     const uint32_t q = threadIdx.x & 3u, g = threadIdx.x >> 2;
-    const bool few = blockIdx.x >= MW * first_few;          // the same for the workgroup
+    const bool few = !BLOCKS && blockIdx.x >= MW * first_few;          // the same for the workgroup
     const uint32_t at = few ? blockIdx.x - MW * first_few : blockIdx.x, per = few ? MW / 8 : MW;
-    const uint32_t sum = (few ? first_few : 0u) + at / per, w = few ? at % per * 8 + g / 2 : at % per;
-    const P29* __restrict__ B = list[sum].buckets + (few ? w * (2 * FEW_T) + (g & 1u) * FEW_T : w * MT + g * 8);
+    const uint32_t sum = BLOCKS ? blockIdx.y : (few ? first_few : 0u) + at / per;
+    const PointDesc& desc = list[sum];
+    const uint32_t w = BLOCKS ? blockIdx.x : (few ? at % per * 8 + g / 2 : at % per);      // BLOCKS: the block's number among all
+    const uint32_t nblk = desc.hb / MT;
+    if (desc.out == nullptr || (!few && w >= 2 * desc.nwh * (BLOCKS ? nblk : 1u))) return;
+    const bool tree = !BLOCKS && !few && nblk > 1;
+    const P29* __restrict__ B = desc.buckets + (few ? w * (2 * FEW_T) + (g & 1u) * FEW_T : w * MT + g * 8);
     enum : uint32_t { S = 0, V = 1, T = 2 };                // the running sum, the sum of the running sums, half a step of the tree
     auto get = [&](uint32_t slot, uint32_t of) {
         P29 r;
@@ -952,14 +1027,19 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
             for (int l = 0; l < P29_WORDS; ++l) pool[slot][g][l] = src[l];
         }
     };
-    {
+    P29 nxt = p29_infinity();
+    if (tree) {
+        const P29* __restrict__ b2 = desc.blocks + 2 * (size_t)(w * nblk + (g < nblk ? g : 0u));
+        put(V, g < nblk ? b2[0] : nxt);
+        put(S, g < nblk ? b2[1] : nxt);
+    } else {
         const P29 top = B[7];
         put(S, top);
         put(V, top);
+        nxt = B[6];
     }
-    P29 nxt = B[6];
-    const uint32_t steps = few ? 19 : 25;
-    for (uint32_t step = 0; step < steps; ++step) {         // one addition, whatever it is for, so that its instructions are there once
+    const uint32_t steps = few ? 19 : (tree ? 17 + 2 * (31 - __builtin_clz(nblk)) : 25);
+    for (uint32_t step = tree ? 17 : 0; step < steps; ++step) {         // one addition, whatever it is for, so that its instructions are there once
         uint32_t xs, ys, yg = g, to;
         const bool odd = (g & 1u) != 0;
         bool bucket = false;
@@ -987,27 +1067,33 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
         p29_quad_add(x, y, q);
         put(to, x);
-        if (step + 1 == steps && q == 0 && (few ? !odd : g == 0)) win[(size_t)sum * MW + w] = x;
+        if (step + 1 == steps && q == 0) {
+            if constexpr (BLOCKS) {
+                if (g < 2) desc.blocks[2 * (size_t)w + g] = x;
+            } else if (few ? !odd : g == 0) win[(size_t)sum * MW + w] = x;
+        }
     }
 }
 // grid: eight sums a wave
 __global__ void __launch_bounds__(GT) k_msm_horner(const P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t n) {
     urgent();
     const uint32_t q = threadIdx.x & 3u, sum = (blockIdx.x * GT + threadIdx.x) >> 3, half = (threadIdx.x >> 2) & 1u;
-    const P29* __restrict__ W = win + (size_t)(sum < n ? sum : n - 1) * MW + half * MWH;
-    P29 r = W[MWH - 1];
-    for (int w = MWH - 2; w >= -1; --w) {
+    const uint32_t nwh = list[blockIdx.x * (GT / 8)].nwh, width = 128u / nwh, wider = 128u % nwh;      // of the wave's sums
+    G1Jac* __restrict__ out = sum < n ? list[sum].out : nullptr;
+    const P29* __restrict__ W = win + (size_t)(out ? sum : blockIdx.x * (GT / 8)) * MW + half * nwh;
+    P29 r = W[nwh - 1];
+    for (int w = (int)nwh - 2; w >= -1; --w) {
         P29 p;
         if (w >= 0) {
             p = W[w];                                       // on its way during the doublings
-            for (int k = 0; k < 8; ++k) p29_quad_double(r, q);
+            for (uint32_t k = width + ((uint32_t)w < wider ? 1u : 0u); k > 0; --k) p29_quad_double(r, q);
         } else {                                            // the halves: [lambda] of the second
             if (half) r.x = fq29_mul(r.x, fq29_from_fp(glv_beta()));
             p = p29_shfl(r, (int)(threadIdx.x ^ 4u));
         }
         p29_quad_add(r, p, q);
     }
-    if (sum < n && half == 0 && q == 0) *list[sum].out = p29_to_jac(r);
+    if (out && half == 0 && q == 0) *out = p29_to_jac(r);
 }
 
 // Sums of an opening's first rounds from commitments of the opened tensor's rows.  The opened vector is the row fold of a
@@ -1034,12 +1120,13 @@ __host__ __device__ __forceinline__ void cross_target(uint32_t t, uint32_t& firs
 // These sums are bucket multi-scalar multiplications.  Term g = pattern * nrows + row of an opening, in the order `pts`
 // lays the points out, has the coefficient eq(u_rows, row) * c(pattern) -- c = 1 for the row commitments, the product of the
 // earlier rounds' challenges for a cross pattern -- and a target is the sum over a contiguous range of terms: one bucket sum per target over the normalised points, with the digits of all
-// terms written once, as k_msm_recode writes them (D: (MW + 1) x terms bytes).  A term costs 32 mixed additions (a scalar
+// terms written once, as k_msm_recode writes them.  A term costs at most 32 mixed additions (a scalar
 // multiplication of its own would cost a 129-step walk).
-struct CrossDigitItem { int8_t* D; const Fr* u_rows; const Fr* u; uint32_t nrows, k_rows; };
+struct CrossDigitItem { void* D; const Fr* u_rows; const Fr* u; uint32_t nrows, k_rows; };
 struct CrossDigitBatch { CrossDigitItem it[OB_MAX]; };
 // grid (ceil(most terms / 256), openings)
-__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t npatterns) {
+__global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch cb, uint32_t npatterns, const DigitPlan plan, uint32_t* __restrict__ state, uint32_t state_words) {
+    clear_state(state, state_words);
     const CrossDigitItem& it = cb.it[blockIdx.y];
     const size_t terms = (size_t)npatterns * it.nrows, i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= terms) return;
@@ -1056,7 +1143,7 @@ __global__ void __launch_bounds__(256) k_open_cross_digits(const CrossDigitBatch
             coef = mont_mul(coef, mont_mul(((a >> k) & 1u) ? uk : nk, ((b >> k) & 1u) ? nk : uk));
         }
     }
-    msm_recode_store(it.D, terms, i, from_mont(coef));
+    msm_recode_store(it.D, terms, i, from_mont(coef), plan);
 }
 // T of the rounds behind the first follows from T of round 0 and from T0, T1 of the rounds before:
 //   T_r = u(1-u) T_(r-1) + (1-u)^2 T0_(r-1) + u^2 T1_(r-1)   (u = the challenge of round r-1)
@@ -1080,7 +1167,31 @@ __global__ void __launch_bounds__(256) k_open_unroll_digits(int8_t* __restrict__
         }
         for (uint32_t q = j == 0 ? k : k + 1; q < r; ++q) c = mont_mul(c, mont_mul(u[q], sub(one, u[q])));
     }
-    msm_recode_store(D0 + (size_t)blockIdx.y * (MW + 1) * terms, terms, i, from_mont(c));
+    msm_recode_store(D0 + (size_t)blockIdx.y * (MW + 1) * terms, terms, i, from_mont(c), DigitPlan{});
+}
+// The same the other way round, for openings whose T is not given for any round: behind the last round T_R = [s] g of the final scalar and generator, and
+//   T_r = (T_(r+1) - (1-u)^2 T0_r - u^2 T1_r) / (u(1-u))   (u = the challenge of round r, neither 0 nor 1)
+// so no round's T is summed at all: the sum over all generators in the first round was a quarter of the sums of an opening of 128 x 131072.
+// The digits of T_0 .. T_(R-1) over the 3 R + 1 proof points (T's: zeros).  V: 1 / (u(1-u)) of every round, as U
+struct FinalScalars { const Fr* s[OB_MAX]; };
+__global__ void __launch_bounds__(256) k_open_back_digits(int8_t* __restrict__ D0, const Fr* __restrict__ U, const Fr* __restrict__ V, const FinalScalars fs, uint32_t R) {
+    urgent();
+    const uint32_t np = 3 * R + 1, terms = R * np, i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= terms) return;
+    const Fr* __restrict__ u = U + (size_t)blockIdx.y * R;
+    const Fr* __restrict__ v = V + (size_t)blockIdx.y * R;
+    const uint32_t r = i / np, m = i % np, k = m / 3, j = m % 3;
+    const Fr one = big_one_mont<8>();
+    Fr c = big_zero<8>();
+    if (m == 3 * R || (j != 0 && k >= r)) {
+        if (m == 3 * R) c = to_mont(*fs.s[blockIdx.y]);
+        else {
+            const Fr f = j == 2 ? u[k] : sub(one, u[k]);
+            c = sub(c, mont_mul(f, f));
+        }
+        for (uint32_t q = r; q < (m == 3 * R ? R : k + 1); ++q) c = mont_mul(c, v[q]);
+    }
+    msm_recode_store(D0 + (size_t)blockIdx.y * (MW + 1) * terms, terms, i, from_mont(c), DigitPlan{});
 }
 // ---- the fold on 29-bit-limb affine points ----------------------------------------------------------------------------------
 // The rounds of an opening keep the generators in ONE form: affine, 29-bit limbs (A29; all-zero limbs = infinity), canonical
@@ -1566,35 +1677,33 @@ __global__ void __launch_bounds__(TAIL_T) k_tail_scalars(const TailPtrs tp, cons
         n = ns;
     }
 }
-// C[(3j+0)*n0 + k] = s_j[k>>j] W_j(k); C[(3j+1)*n0 + k] = s_j[(k>>j)-1] W_j(k) for odd k>>j; C[(3j+2)*n0 + k] = s_j[(k>>j)+1] W_j(k)
-// for even k>>j with a partner; zero elsewhere.  C[3*levels*n0 + k] = W_levels(k) when `final_gen`.
-__global__ void __launch_bounds__(TAIL_T) k_tail_coeffs(Fr* __restrict__ C0, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels, uint32_t final_gen) {
+// The digits (k_msm_recode) of C[(3j+0)*n0 + k] = s_j[k>>j] W_j(k); C[(3j+1)*n0 + k] = s_j[(k>>j)-1] W_j(k) for odd k>>j; C[(3j+2)*n0 + k] = s_j[(k>>j)+1] W_j(k)
+// for even k>>j with a partner; zero elsewhere.  C[3*levels*n0 + k] = W_levels(k), the final generator's.  A lane forms its own W: the products cost less than a chain of
+// all levels' recodings on one lane.  blockIdx.z: which of these; given: the levels whose first is not wanted.  An opening's coefficients stand behind those
+// of the one before, ncoef of all of them.
+__global__ void __launch_bounds__(TAIL_T) k_tail_coeffs(void* __restrict__ D, size_t ncoef, const TailPtrs tp, const Fr* __restrict__ U, uint32_t ustride, uint32_t n0, uint32_t levels, uint32_t given,
+                                                        const DigitPlan plan, uint32_t* __restrict__ state, uint32_t state_words) {
     urgent();
-    const uint32_t k = blockIdx.x * TAIL_T + threadIdx.x;
-    if (k >= n0) return;
+    if (blockIdx.z == 0) clear_state(state, state_words);
+    const uint32_t k = blockIdx.x * TAIL_T + threadIdx.x, j = blockIdx.z / 3, kind = blockIdx.z % 3;
+    if (k >= n0 || (j < levels && kind == 0 && (given >> j & 1u))) return;
     const Fr* __restrict__ usu = U + (size_t)blockIdx.y * ustride;
-    Fr* __restrict__ C = C0 + (size_t)blockIdx.y * (3 * levels + final_gen) * n0;
-    const Fr* __restrict__ SL = tp.SL[blockIdx.y];
-    const Fr* __restrict__ S = tp.S[blockIdx.y];
     const Fr one_m = big_one_mont<8>();
     Fr W = one_m;                 // Montgomery form
-    const Fr* sj = S;
-    const Fr* nxt = SL;
+    const Fr* sj = tp.S[blockIdx.y];
     uint32_t n = n0;
-    const Fr zero = big_zero<8>();
-    for (uint32_t j = 0; j < levels; ++j) {
-        const uint32_t i = k >> j;
-        // mont_mul(Montgomery W, standard s) is the standard-form product
-        C[(size_t)(3 * j) * n0 + k] = mont_mul(W, sj[i]);
-        C[(size_t)(3 * j + 1) * n0 + k] = (i & 1u) ? mont_mul(W, sj[i - 1]) : zero;
-        C[(size_t)(3 * j + 2) * n0 + k] = (!(i & 1u) && i + 1 < n) ? mont_mul(W, sj[i + 1]) : zero;
-        W = mont_mul(W, (i & 1u) ? sub(one_m, usu[j]) : usu[j]);
-        const uint32_t ns = (n + 1) / 2;
-        sj = nxt;
-        nxt += ns;
-        n = ns;
+    for (uint32_t i = 0; i < j; ++i) {
+        const Fr f = (k >> i & 1u) ? sub(one_m, usu[i]) : usu[i];
+        W = i == 0 ? f : mont_mul(W, f);
+        sj = i == 0 ? tp.SL[blockIdx.y] : sj + n;
+        n = (n + 1) / 2;
     }
-    if (final_gen) C[(size_t)(3 * levels) * n0 + k] = from_mont(W);
+    const uint32_t i = k >> j;
+    Fr c = big_zero<8>();
+    if (j == levels) c = from_mont(W);
+    else if (kind == 0 || (kind == 1 ? (i & 1u) != 0 : !(i & 1u) && i + 1 < n))
+        c = mont_mul(W, sj[kind == 0 ? i : (kind == 1 ? i - 1 : i + 1)]);      // Montgomery W times standard s: the product's standard form
+    msm_recode_store(D, ncoef, ((size_t)blockIdx.y * gridDim.z + blockIdx.z) * n0 + k, c, plan);
 }
 __global__ void __launch_bounds__(64) k_u32_zero(uint32_t* __restrict__ p, uint32_t n, size_t stride) {      // p[i * stride] = 0, i < n
     for (uint32_t i = threadIdx.x; i < n; i += 64) p[(size_t)i * stride] = 0u;
@@ -1811,65 +1920,132 @@ static int join_streams(hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>
     ZK_HIP(hipStreamWaitEvent(aux, ev, 0));
     return 0;
 }
-// The bucket accumulation of some sums of at most count_max elements on st; their reductions, sum z into out[z], are appended to `later`.
-static int bucket_sums_queue(const std::vector<MsmDesc>& d, const std::vector<G1Jac*>& out, size_t count_max, Arena& arena, JobUploads& up, hipStream_t st,
-                             std::vector<PointDesc>& later) {
+// How some sums are taken, decided before their scalars' digits are written.  n: the sums; count_max, terms: elements of the longest, and about how many of
+// them have a scalar other than zero; total: elements of all of them.
+struct SumsPlan { DigitPlan digits{}; uint32_t hb = 0, most = 0, group = 0, state_words = 0; size_t total = 0; uint32_t* state = nullptr; };
+// Windows of a half, and the longest list of one lane: two and a half times the mean of the wide windows' buckets, which cuts outliers alone; buckets a bit narrower have twice the mean,
+// start first and leave the shorter ones to fill up.
+// In instructions of a lane: an element costs an addition of 4700 a window (the first of a list none), a list 1700 and a bucket about 1350 for each step
+// of its wave in k_msm_windows.  The time of these on the whole chip at three quarters of its issue slots, half a list of the last waves, and the launch that
+// windows of more than 128 buckets add.
+static uint32_t msm_windows_of_half(size_t terms, uint32_t n, uint32_t* most) {
+    uint32_t best = 0;
+    double best_us = 0;
+    for (uint32_t nwh : {16u, 13u, 12u, 11u}) {
+        const uint32_t q = 128u / nwh, rem = 128u % nwh, hb = 1u << (q - 1 + (rem ? 1u : 0u));
+        const double buckets = 2.0 * ((double)rem * (1u << q) + (double)(nwh - rem) * (1u << (q - 1))), mean = std::min((double)terms / hb, (double)MPIECE);
+        const double all = (double)n * (std::max(0.0, (double)terms * 2.0 * nwh - buckets) * 4700.0 + buckets * (1700.0 + 1350.0 * (hb > 128 ? 29.0 : 25.0)));
+        const double us = all * 4.0 / 64.0 / (1024.0 * 2400.0) / 0.75 + 6.0 * mean + (hb > 128u ? 80.0 : 0.0);
+        if (best == 0 || us < best_us) {
+            best = nwh; best_us = us;
+            *most = (uint32_t)std::min(std::max(2.5 * mean, 32.0), (double)MPIECE);
+        }
+    }
+    return best;
+}
+static int sums_plan(SumsPlan& p, uint32_t n, size_t count_max, size_t terms, size_t total, Arena& arena) {
+    if (n == 0 || count_max <= (size_t)FEW_MAX) return 0;
+    ZK_ARG(total < (1ull << 32), "opening: too many elements");
+    const uint32_t nwh = msm_windows_of_half(terms, n, &p.most), q = 128u / nwh, rem = 128u % nwh;
+    p.total = total;
+    p.digits.nwh = nwh;
+    for (uint32_t w = 0, off = 0; w < nwh; ++w) {
+        off += q + (w < rem ? 1u : 0u);
+        p.digits.bias[(off - 1) / 32] |= 1u << ((off - 1) % 32);
+    }
+    p.hb = 1u << (q - 1 + (rem ? 1u : 0u));
+    // windows at a time, equally many: lists of at most 256 MiB (or one window's), which 1.5 M generators in a round alone exceed
+    const uint32_t most_windows = (uint32_t)std::min<size_t>(std::max<size_t>((1ull << 26) / std::max<size_t>(total, 1), 1), 2 * nwh);
+    p.group = (uint32_t)cdiv(2 * nwh, cdiv(2 * nwh, most_windows));
+    p.state_words = (uint32_t)cdiv(2 * nwh, p.group) * SORT_WORDS;
+    Scratch& st = arena.add(sizeof(uint32_t) * p.state_words);
+    p.state = st.as<uint32_t>();
+    return st.rc;
+}
+// The bucket accumulation of some sums of at most count_max elements on aux, which waits for st; their reductions, sum z into out[z], are appended to `later`.
+// The sorting goes on st: what st holds next and the sums fill the chip together, and in front of both the short launches find room.
+static int bucket_sums_queue(std::vector<MsmDesc> d, const std::vector<G1Jac*>& out, size_t count_max, const SumsPlan& plan, Arena& arena, JobUploads& up, hipStream_t st, hipStream_t aux,
+                             std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
     const uint32_t n_msm = (uint32_t)d.size();
     if (n_msm == 0) return 0;
-    if (count_max <= (size_t)FEW_MAX) {
-        uint32_t nw = 8;
-        while (nw > 1 && nw * count_max > 8 * MSL) nw /= 2;
-        const void* dd = nullptr;
-        int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
-        if (rc) return rc;
-        Scratch& buckets = arena.add(sizeof(P29) * (size_t)n_msm * FEW_BUCKETS);
-        if (buckets.rc) return buckets.rc;
-        hipLaunchKernelGGL(k_msm_few, dim3(FEW_WINDOWS / nw, n_msm), dim3(MSL), 0, st, buckets.as<P29>(), (const MsmDesc*)dd, nw);
-        ZK_LAUNCH_CHECK();
-        for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<P29>() + (size_t)z * FEW_BUCKETS, out[z], 1u, 0u});
-        return 0;
-    }
-    // One chunk per workgroup, and chunks short enough for two workgroups a SIMD where there are few elements: a workgroup's time is its
-    // chunk's elements over 64 lanes.  Very large inputs take more chunks per workgroup to bound the bucket storage.
-    uint32_t chunk = MSEG;
-    while (chunk > 256 && (size_t)n_msm * MW * cdiv(count_max, chunk / 2) <= 2048) chunk /= 2;
-    const uint32_t chunks = count_max ? cdiv(count_max, chunk) : 1u;
-    const uint32_t cps = (chunks + 255u) / 256u;
-    uint32_t ns = (chunks + cps - 1) / cps;
+    size_t total = 0;
+    for (MsmDesc& m : d) { m.list_at = (uint32_t)total; total += m.count; }
     const void* dd = nullptr;
     int rc = up.put(d.data(), sizeof(MsmDesc) * n_msm, st, &dd);
     if (rc) return rc;
-    Scratch& partial = arena.add(sizeof(P29) * n_msm * MW * (size_t)ns * MT);
-    if (partial.rc) return partial.rc;
-    hipLaunchKernelGGL(k_msm_seg, dim3(ns, MW, n_msm), dim3(MSL), 0, st, partial.as<P29>(), (const MsmDesc*)dd, ns, cps, chunk);
-    // the segments' raw buckets summed eight at a time (a lane per bucket and window: the reduction, one workgroup per sum, then
-    // walks single buckets)
-    P29* cur = partial.as<P29>();
-    while (ns > 1) {
-        const uint32_t ng = (ns + 7) / 8;
-        Scratch& nxt = arena.add(sizeof(P29) * n_msm * MW * (size_t)ng * MT);
-        if (nxt.rc) return nxt.rc;
-        hipLaunchKernelGGL(k_msm_bucket_fold, dim3(n_msm * MW * (MT / GT), ng), dim3(GT), 0, st, nxt.as<P29>(), cur, ns);
-        cur = nxt.as<P29>();
-        ns = ng;
+    if (plan.digits.nwh == 0) {
+        uint32_t nw = 8;
+        while (nw > 1 && nw * count_max > 8 * MSL) nw /= 2;
+        Scratch& buckets = arena.add(sizeof(P29) * (size_t)n_msm * FEW_BUCKETS);
+        if (buckets.rc) return buckets.rc;
+        rc = join_streams(st, aux, events);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_msm_few, dim3(FEW_WINDOWS / nw, n_msm), dim3(MSL), 0, aux, buckets.as<P29>(), (const MsmDesc*)dd, nw);
+        ZK_LAUNCH_CHECK();
+        for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<P29>() + (size_t)z * FEW_BUCKETS, nullptr, out[z], 1u, (uint32_t)MWH, (uint32_t)MT, 0u});
+        return 0;
     }
-    ZK_LAUNCH_CHECK();
-    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{cur + (size_t)z * MW * MT, out[z], 0u, 0u});
+    ZK_ARG(total <= plan.total, "opening: more elements than planned");
+    const uint32_t nw = 2 * plan.digits.nwh;
+    const size_t entries = (size_t)plan.group * total, cut = entries / plan.most + 1;               // of a launch; buckets above `most` at most
+    const size_t rows = (size_t)n_msm * nw, nb = rows * plan.hb, max_tasks = std::min((size_t)n_msm * plan.group * plan.hb + 2 * cut, entries);
+    ZK_ARG(nb + 2 * cut < (1ull << 32), "opening: too many sums");
+    Scratch& info = arena.add(sizeof(uint4) * nb);
+    Scratch& lists = arena.add(sizeof(uint32_t) * entries);
+    Scratch& heavy = arena.add(sizeof(uint4) * cut);
+    Scratch& tasks = arena.add(sizeof(uint4) * max_tasks);
+    Scratch& buckets = arena.add(sizeof(P29) * (nb + 2 * cut));                                      // a cut bucket has less than twice as many pieces as it is longer than `most`
+    if (info.rc || lists.rc || heavy.rc || tasks.rc || buckets.rc) return info.rc ? info.rc : (lists.rc ? lists.rc : (heavy.rc ? heavy.rc : (tasks.rc ? tasks.rc : buckets.rc)));
+    SortSpace sp{plan.state, info.as<uint4>(), lists.as<uint32_t>(), heavy.as<uint4>(), tasks.as<uint4>(), buckets.as<P29>(), plan.digits.nwh, plan.hb, 0u, (uint32_t)total, plan.most, (uint32_t)nb, (uint32_t)cut};
+    for (sp.w0 = 0; sp.w0 < nw; sp.w0 += plan.group, sp.state += SORT_WORDS) {
+        const dim3 grid(std::min(plan.group, nw - sp.w0), n_msm);
+        const hipStream_t sort_on = sp.w0 ? aux : st;
+        // a workgroup passes over its sum's digits twice: more lanes for long ones
+        if (count_max > 8192) hipLaunchKernelGGL(k_msm_sort<1024>, grid, dim3(1024), 0, sort_on, sp, (const MsmDesc*)dd);
+        else hipLaunchKernelGGL(k_msm_sort<256>, grid, dim3(256), 0, sort_on, sp, (const MsmDesc*)dd);
+        hipLaunchKernelGGL(k_msm_tasks, grid, dim3(TASK_T), 0, sort_on, sp);
+        if (sp.w0 == 0) rc = join_streams(st, aux, events);
+        if (rc) return rc;
+        hipLaunchKernelGGL(k_msm_lists, dim3(cdiv(max_tasks, MSL)), dim3(MSL), 0, aux, sp, (const MsmDesc*)dd);
+        hipLaunchKernelGGL(k_msm_merge, dim3((uint32_t)std::min<size_t>(cut, 256)), dim3(MSL), 0, aux, sp);
+        ZK_LAUNCH_CHECK();
+    }
+    for (uint32_t z = 0; z < n_msm; ++z) later.push_back(PointDesc{buckets.as<P29>() + (size_t)z * nw * plan.hb, nullptr, out[z], 0u, plan.digits.nwh, plan.hb, 0u});
     return 0;
 }
-static int points_queue(std::vector<PointDesc>& list, Arena& arena, JobUploads& up, hipStream_t st) {
-    if (list.empty()) return 0;
+static int points_queue(std::vector<PointDesc>& sums, Arena& arena, JobUploads& up, hipStream_t st) {
+    if (sums.empty()) return 0;
+    // fewer windows (of more buckets) first, few elements last
+    std::stable_sort(sums.begin(), sums.end(), [](const PointDesc& a, const PointDesc& b) { return a.few != b.few ? a.few < b.few : a.nwh < b.nwh; });
+    std::vector<PointDesc> list;
+    size_t blocks_n = 0;
+    uint32_t wide = 0, blocks_max = 0;                       // entries up to the last sum of wide windows; most blocks of one
+    for (const PointDesc& d : sums) {
+        if (!list.empty() && list.back().nwh != d.nwh)
+            while (list.size() % (GT / 8)) { PointDesc gap = list.back(); gap.out = nullptr; list.push_back(gap); }
+        list.push_back(d);
+        if (d.hb > (uint32_t)MT) {
+            wide = (uint32_t)list.size();
+            blocks_max = std::max(blocks_max, 2 * d.nwh * d.hb / MT);
+            blocks_n += 2 * (size_t)(2 * d.nwh * d.hb / MT);
+        }
+    }
     const uint32_t n = (uint32_t)list.size();
-    const uint32_t first_few = (uint32_t)(std::stable_partition(list.begin(), list.end(), [](const PointDesc& d) { return d.few == 0; }) - list.begin());
+    uint32_t first_few = n;
+    while (first_few > 0 && list[first_few - 1].few) --first_few;
+    Scratch& win = arena.add(sizeof(P29) * (MW * (size_t)n + blocks_n));
+    if (win.rc) return win.rc;
+    P29* blocks = win.as<P29>() + MW * (size_t)n;
+    for (PointDesc& d : list)
+        if (d.hb > (uint32_t)MT && d.out) { d.blocks = blocks; blocks += 2 * (size_t)(2 * d.nwh * d.hb / MT); }
     const void* dl = nullptr;
     int rc = up.put(list.data(), sizeof(PointDesc) * n, st, &dl);
     if (rc) return rc;
-    Scratch& win = arena.add(sizeof(P29) * MW * (size_t)n);
-    if (win.rc) return win.rc;
-    hipLaunchKernelGGL(k_msm_windows, dim3(MW * first_few + MW / 8 * (n - first_few)), dim3(GT), 0, st, win.as<P29>(), (const PointDesc*)dl, first_few);
+    if (wide) hipLaunchKernelGGL(k_msm_windows<true>, dim3(blocks_max, wide), dim3(GT), 0, st, win.as<P29>(), (const PointDesc*)dl, 0u);
+    hipLaunchKernelGGL(k_msm_windows<false>, dim3(MW * first_few + MW / 8 * (n - first_few)), dim3(GT), 0, st, win.as<P29>(), (const PointDesc*)dl, first_few);
     hipLaunchKernelGGL(k_msm_horner, dim3(cdiv(8 * (size_t)n, (size_t)GT)), dim3(GT), 0, st, (const P29*)win.as<P29>(), (const PointDesc*)dl, n);
     ZK_LAUNCH_CHECK();
-    list.clear();
+    sums.clear();
     return 0;
 }
 // One halving round: the scalars' digits and the fold on st, the bucket sums on aux (their reductions are appended to `later`).
@@ -1882,17 +2058,33 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
     ZK_ARG(old_size < (1ull << 31), "opening: more than 2^31 generators");
     ZK_ARG(count >= 1 && count <= OB_MAX, "opening: bad batch size");
     const size_t new_size = (old_size + 1) / 2;
-    const size_t dig_bytes = (size_t)(MW + 1) * old_size;
-    const int8_t* digits = nullptr;
+    SumsPlan plan;
     if (given < 2) {
+        const char* digits = nullptr;
+        size_t dig_bytes = 0;
+        const size_t half = old_size / 2;
+        int rc = sums_plan(plan, (given == 0 ? 3u : 2u) * (uint32_t)count, given == 0 ? old_size : half, half, count * (2 * half + (given == 0 ? old_size : 0)), arena);
+        if (rc) return rc;
+        dig_bytes = digit_bytes(plan.digits) * old_size;
         Scratch& dig = arena.add(dig_bytes * count);
         if (dig.rc) return dig.rc;
-        digits = dig.as<int8_t>();
+        digits = dig.as<char>();
         RecodeBatch rb;
-        for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>() + dig_bytes * (i < count ? i : 0); rb.S[i] = items[i < count ? i : 0].scalars; }
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(old_size, GT), count), dim3(GT), 0, st, rb, old_size);
+        for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<char>() + dig_bytes * (i < count ? i : 0); rb.S[i] = items[i < count ? i : 0].scalars; }
+        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(old_size, GT), count), dim3(GT), 0, st, rb, old_size, plan.digits, plan.state, plan.state_words);
         ZK_LAUNCH_CHECK();
-        int rc = join_streams(st, aux, events);
+        // ---- side chain (aux): nothing here feeds the fold ----
+        std::vector<MsmDesc> d;
+        std::vector<G1Jac*> out;
+        const uint32_t ds = (uint32_t)old_size, dh = (uint32_t)half;
+        for (int i = 0; i < count; ++i) {
+            const char* dg = digits + dig_bytes * i;
+            G1Jac* o = pts + npts * i;
+            if (given == 0) { d.push_back(MsmDesc{dg, items[i].gens, ds, ds, 1u, 0u, 1u, 0u, 0u, 0u}); out.push_back(o); }
+            d.push_back(MsmDesc{dg, items[i].gens, ds, dh, 2u, 0u, 2u, 1u, 0u, 0u}); out.push_back(o + 1);
+            d.push_back(MsmDesc{dg, items[i].gens, ds, dh, 2u, 1u, 2u, 0u, 0u, 0u}); out.push_back(o + 2);
+        }
+        rc = bucket_sums_queue(d, out, given == 0 ? old_size : half, plan, arena, up, st, aux, events, later);
         if (rc) return rc;
     }
     // ---- critical chain (st): the fold ----
@@ -1941,20 +2133,6 @@ static int open_round_launch(const RoundItem* items, int count, size_t old_size,
     timed.end((use_comb || use_comb2) ? 1 : 0, fp_mults, new_size * (size_t)count);
     hipLaunchKernelGGL(k_open_fold_special, dim3(16, count), dim3(GT), 0, st, sb, old_size);
     ZK_LAUNCH_CHECK();
-    // ---- side chain (aux): nothing here feeds the next fold ----
-    if (given < 2) {
-        std::vector<MsmDesc> d;
-        std::vector<G1Jac*> out;
-        const uint32_t half = (uint32_t)(old_size / 2), ds = (uint32_t)old_size;
-        for (int i = 0; i < count; ++i) {
-            const int8_t* dg = digits + dig_bytes * i;
-            G1Jac* o = pts + npts * i;
-            if (given == 0) { d.push_back(MsmDesc{dg, items[i].gens, ds, ds, 1u, 0u, 1u, 0u}); out.push_back(o); }
-            d.push_back(MsmDesc{dg, items[i].gens, ds, half, 2u, 0u, 2u, 1u}); out.push_back(o + 1);
-            d.push_back(MsmDesc{dg, items[i].gens, ds, half, 2u, 1u, 2u, 0u}); out.push_back(o + 2);
-        }
-        return bucket_sums_queue(d, out, given == 0 ? old_size : half, arena, up, aux, later);
-    }
     return 0;
 }
 
@@ -2266,28 +2444,39 @@ struct OpenJob {
 };
 // The targets of every opening of a batch (T of round 0; T0, T1 of the first `full` rounds) as bucket sums over the openings' [pattern][row] points, on aux.
 static int open_cross_sums_queue(const OpenItem* items, int count, uint32_t full, G1Jac* pts, size_t npts, const Fr* const* urow_dev, const Fr* U_dev, int rounds, Arena& arena,
-                                 JobUploads& up, hipStream_t aux, std::vector<PointDesc>& later) {
+                                 JobUploads& up, hipStream_t aux, std::vector<hipEvent_t>& events, std::vector<PointDesc>& later) {
     const uint32_t ntargets = 1u + 2u * full, npatterns = cross_patterns(full);
     CrossDigitBatch db;
     const A29* base[OB_MAX];
-    const int8_t* digs[OB_MAX];
-    size_t most_terms = 0, most_count = 0;
+    const void* digs[OB_MAX];
+    size_t most_terms = 0, most_count = 0, all_terms = 0;
+    for (int i = 0; i < count; ++i) {
+        all_terms += (size_t)npatterns * items[i].nrows;
+        for (uint32_t t = 0; t < ntargets; ++t) {
+            uint32_t p0, npat, slot;
+            cross_target(t, p0, npat, slot);
+            most_count = std::max(most_count, (size_t)npat * items[i].nrows);
+        }
+    }
+    SumsPlan plan;
+    int rc = sums_plan(plan, ntargets * (uint32_t)count, most_count, all_terms / (ntargets * (uint32_t)count), all_terms, arena);
+    if (rc) return rc;
     for (int i = 0; i < count; ++i) {
         const size_t points = (size_t)npatterns * items[i].nrows;          // and as many terms
         ZK_ARG(items[i].nrows >= 1 && points < (1ull << 31), "zk_g1_open: bad row count");
         most_terms = std::max(most_terms, points);
         Scratch& aff = arena.add(sizeof(G1Affine) * points);
         Scratch& a29 = arena.add(sizeof(A29) * points);
-        Scratch& dg = arena.add((size_t)(MW + 1) * points);
+        Scratch& dg = arena.add(digit_bytes(plan.digits) * points);
         if (aff.rc || a29.rc || dg.rc) return aff.rc ? aff.rc : (a29.rc ? a29.rc : dg.rc);
         g1_normalize_queue<true>(aff.p, (const G1Jac*)items[i].rows, points, aux);
         hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(points, 256)), dim3(256), 0, aux, a29.as<A29>(), aff.as<G1Affine>(), points);
         base[i] = a29.as<A29>();
-        digs[i] = dg.as<int8_t>();
-        db.it[i] = CrossDigitItem{dg.as<int8_t>(), urow_dev[i], U_dev + (size_t)i * rounds, items[i].nrows, (uint32_t)items[i].k_rows};
+        digs[i] = dg.p;
+        db.it[i] = CrossDigitItem{dg.p, urow_dev[i], U_dev + (size_t)i * rounds, items[i].nrows, (uint32_t)items[i].k_rows};
     }
     for (int i = count; i < OB_MAX; ++i) db.it[i] = db.it[0];
-    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, npatterns);
+    hipLaunchKernelGGL(k_open_cross_digits, dim3(cdiv(most_terms, 256), count), dim3(256), 0, aux, db, npatterns, plan.digits, plan.state, plan.state_words);
     ZK_LAUNCH_CHECK();
     std::vector<MsmDesc> d;
     std::vector<G1Jac*> out;
@@ -2296,11 +2485,10 @@ static int open_cross_sums_queue(const OpenItem* items, int count, uint32_t full
             uint32_t p0, npat, slot;
             cross_target(t, p0, npat, slot);
             const uint32_t nr = items[i].nrows;
-            most_count = std::max(most_count, (size_t)npat * nr);
-            d.push_back(MsmDesc{digs[i], base[i], npatterns * nr, npat * nr, 1u, p0 * nr, 1u, p0 * nr});
+            d.push_back(MsmDesc{digs[i], base[i], npatterns * nr, npat * nr, 1u, p0 * nr, 1u, p0 * nr, 0u, 0u});
             out.push_back(pts + npts * i + slot);
         }
-    return bucket_sums_queue(d, out, most_count, arena, up, aux, later);
+    return bucket_sums_queue(d, out, most_count, plan, arena, up, aux, aux, events, later);
 }
 static int open_span_fold(const A29** gens, int count, size_t n0, int r0, const OpenItem* items, Arena& arena, JobUploads& up, hipStream_t st) {
     const size_t ns = (((n0 + 1) / 2 + 1) / 2 + 1) / 2;
@@ -2341,10 +2529,17 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
     const size_t sl_n = n0 + (size_t)levels + 1;
     Scratch& sl = arena.add(sizeof(Fr) * sl_n * count);
     const size_t ncoef = (size_t)n_msm * n0 * count;
-    Scratch& coef = arena.add(sizeof(Fr) * ncoef);
-    Scratch& dig = arena.add((size_t)(MW + 1) * ncoef);
-    if (sl.rc || coef.rc || dig.rc) return sl.rc ? sl.rc : (coef.rc ? coef.rc : dig.rc);
     ZK_ARG(ncoef < (1ull << 32), "opening: batched rounds too large");
+    uint32_t given = 0, summed = fin;                          // levels whose T is not summed; sums of an opening
+    for (int j = 0; j < levels; ++j) {
+        if (t_given(r0 + j)) given |= 1u << j;
+        summed += t_given(r0 + j) ? 2 : 3;
+    }
+    SumsPlan plan;
+    int rc = sums_plan(plan, summed * (uint32_t)count, n0, (n0 + 1) / 2, (size_t)summed * count * n0, arena);
+    if (rc) return rc;
+    Scratch& dig = arena.add(digit_bytes(plan.digits) * ncoef);
+    if (sl.rc || dig.rc) return sl.rc ? sl.rc : dig.rc;
     TailPtrs tp;
     for (int i = 0; i < OB_MAX; ++i) { const int k = i < count ? i : 0; tp.SL[i] = sl.as<Fr>() + sl_n * k; tp.S[i] = scalars[k]; }
     const TailPtrs all = tp;
@@ -2369,38 +2564,33 @@ static int open_batch_launch(const Fr** scalars, const A29** gens, int count, si
         }
     }
     ZK_LAUNCH_CHECK();
-    int rc = join_streams(st, aux, events);
-    if (rc) return rc;
     const A29* before[OB_MAX];
     for (int i = 0; i < count; ++i) before[i] = gens[i];
-    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, TAIL_T), count), dim3(TAIL_T), 0, aux, coef.as<Fr>(), all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, fin);
-    {
-        RecodeBatch rb;
-        for (int i = 0; i < OB_MAX; ++i) { rb.D[i] = dig.as<int8_t>(); rb.S[i] = coef.as<Fr>(); }
-        hipLaunchKernelGGL(k_msm_recode, dim3(cdiv(ncoef, GT), 1), dim3(GT), 0, aux, rb, ncoef);
-    }
+    hipLaunchKernelGGL(k_tail_coeffs, dim3(cdiv(n0, TAIL_T), count, n_msm), dim3(TAIL_T), 0, st, dig.p, ncoef, all, U_dev + r0, (uint32_t)rounds, (uint32_t)n0, (uint32_t)levels, given, plan.digits,
+                       plan.state, plan.state_words);
     ZK_LAUNCH_CHECK();
-    if (!last) {          // behind the short kernels of the other stream: they would wait for the fold's workgroups otherwise
-        rc = open_span_fold(gens, count, n0, r0, items, arena, up, st);
-        if (rc) return rc;
-    }
     std::vector<MsmDesc> d;
     std::vector<G1Jac*> out;
     for (int it = 0; it < count; ++it)
         for (uint32_t i = 0; i < n_msm; ++i) {
-            if (i < 3 * (uint32_t)levels && i % 3 == 0 && t_given(r0 + (int)(i / 3))) continue;
-            d.push_back(MsmDesc{dig.as<int8_t>(), before[it], (uint32_t)ncoef, (uint32_t)n0, 1u, (uint32_t)(((size_t)it * n_msm + i) * n0), 1u, 0u});
+            if (i < 3 * (uint32_t)levels && i % 3 == 0 && (given >> (i / 3) & 1u)) continue;
+            d.push_back(MsmDesc{dig.p, before[it], (uint32_t)ncoef, (uint32_t)n0, 1u, (uint32_t)(((size_t)it * n_msm + i) * n0), 1u, 0u, 0u, 0u});
             out.push_back(pts + npts * it + (i == 3 * (uint32_t)levels ? 3 * (size_t)rounds : 3 * (size_t)r0 + i));
         }
-    rc = bucket_sums_queue(d, out, n0, arena, up, aux, later);
+    rc = bucket_sums_queue(d, out, n0, plan, arena, up, st, aux, events, later);
     if (rc) return rc;
+    if (!last) {
+        rc = open_span_fold(gens, count, n0, r0, items, arena, up, st);
+        if (rc) return rc;
+    }
     for (int it = 0; it < count; ++it) scalars[it] = sl.as<Fr>() + sl_n * it + off;
     return 0;
 }
-// T of the rounds 1 .. rounds_t - 1 but `again` of every opening from its T of round 0 (above `again`, of that round) and T0, T1 of the rounds below, on st
-static int open_unroll_queue(G1Jac* pts, size_t npts, int count, int rounds_t, int again, const Fr* U_dev, int rounds, Arena& arena, JobUploads& up, hipStream_t st) {
-    if (rounds_t <= 1 || (rounds_t == 2 && again == 1)) return 0;
-    const uint32_t R = (uint32_t)rounds_t, np = 3 * (R - 1), terms = (R - 1) * np;
+// T of the rounds 1 .. rounds_t - 1 but `again` of every opening from its T of round 0 (above `again`, of that round) and T0, T1 of the rounds below, on st;
+// with V_dev of all rounds from the final generators, the final scalars and T0, T1
+static int open_unroll_queue(G1Jac* pts, size_t npts, int count, int rounds_t, int again, const Fr* U_dev, const Fr* V_dev, const Fr* const* finals, int rounds, Arena& arena, JobUploads& up, hipStream_t st) {
+    if (!V_dev && (rounds_t <= 1 || (rounds_t == 2 && again == 1))) return 0;
+    const uint32_t R = (uint32_t)rounds_t, first = V_dev ? 0u : 1u, np = V_dev ? 3 * R + 1 : 3 * (R - 1), terms = (R - first) * np;
     Scratch& aff = arena.add(sizeof(G1Affine) * np);
     Scratch& a29 = arena.add(sizeof(A29) * np * count);
     Scratch& dg = arena.add((size_t)(MW + 1) * terms * count);
@@ -2410,16 +2600,22 @@ static int open_unroll_queue(G1Jac* pts, size_t npts, int count, int rounds_t, i
     for (int i = 0; i < count; ++i) {
         g1_normalize_queue<true>(aff.p, pts + npts * i, np, st);
         hipLaunchKernelGGL(k_g1aff_to_a29, dim3(cdiv(np, 256)), dim3(256), 0, st, a29.as<A29>() + (size_t)np * i, aff.as<G1Affine>(), (size_t)np);
-        for (uint32_t q = 1; q < R; ++q) {
-            if ((int)q == again) continue;
-            d.push_back(MsmDesc{dg.as<int8_t>() + (size_t)(MW + 1) * terms * i, a29.as<A29>() + (size_t)np * i, terms, np, 1u, (q - 1) * np, 1u, 0u});
+        for (uint32_t q = first; q < R; ++q) {
+            if (!V_dev && (int)q == again) continue;
+            d.push_back(MsmDesc{dg.as<int8_t>() + (size_t)(MW + 1) * terms * i, a29.as<A29>() + (size_t)np * i, terms, np, 1u, (q - first) * np, 1u, 0u, 0u, 0u});
             out.push_back(pts + npts * i + 3 * q);
         }
     }
-    hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R, (uint32_t)again);
+    if (V_dev) {
+        FinalScalars fs;
+        for (int i = 0; i < OB_MAX; ++i) fs.s[i] = finals[i < count ? i : 0];
+        hipLaunchKernelGGL(k_open_back_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, V_dev, fs, R);
+    } else hipLaunchKernelGGL(k_open_unroll_digits, dim3(cdiv(terms, 256), count), dim3(256), 0, st, dg.as<int8_t>(), U_dev, (uint32_t)rounds, R, (uint32_t)again);
     ZK_LAUNCH_CHECK();
+    static_assert(3 * 64 + 1 <= FEW_MAX, "the points of a proof are few");
     std::vector<PointDesc> mine;
-    int rc = bucket_sums_queue(d, out, np, arena, up, st, mine);
+    std::vector<hipEvent_t> none;                             // one stream
+    int rc = bucket_sums_queue(d, out, np, SumsPlan{}, arena, up, st, st, none, mine);
     if (rc == 0) rc = points_queue(mine, arena, up, st);
     return rc;
 }
@@ -2504,10 +2700,11 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     // T of round 0 from the row commitments or summed; T of the rounds from 1 to t_rounds - 1 unrolled from it.  The tensor's commitments say what
     // T is for the rounds they have cross patterns for, or else while a round has more than TABLE_MIN_N generators: the first round behind those,
     // t_again, has its T summed, and the rounds behind it follow from that.  A last batch that is so small that its own T cost less than the
-    // unrolling's chain of launches behind it sums them, and the unrolling of the rounds before it runs beside it: openings of 1024 and 4096
-    // generators 1.8 and 2.5 ms by sums, 2.6 and 2.9 unrolled, of 16384 4.3 and 3.8.
+    // unrolling's chain of launches behind it sums them, and the unrolling of the rounds before it runs beside it: openings of 8192
+    // generators 2.15 ms by sums, 2.68 unrolled, of 16384 3.20 and 2.83.
+    // An opening without row commitments whose last batch is larger has all T from its final generator and scalar, behind the last batch as well.
     int t_rounds = rounds, t_again = 0;
-    bool unroll_early = false;
+    bool unroll_early = false, back = false;
     {
         if (cross_r > 0) t_again = cross_r;
         else if (with_rows)
@@ -2522,13 +2719,36 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
             unroll_early = t_rounds == r + 1;
         }
         if (t_again >= t_rounds) t_again = 0;
+        size_t left = n;
+        for (int q = 0; q < rounds && left > 1; ++q) left = (left + 1) / 2;
+        back = !with_rows && !unroll_early && r < rounds && left == 1;
     }
-    auto t_given = [&](int r) { return r == 0 ? with_rows : r < t_rounds && r != t_again; };
+    const Fr* V_dev = nullptr;
+    if (back) {                                              // 1 / (u (1 - u)), all by one inversion
+        const size_t m = (size_t)rounds * count;
+        std::vector<Fr> w(m), v(m);
+        Fr run = big_one_mont<8>();
+        for (size_t i = 0; i < m; ++i) {
+            w[i] = mont_mul(hu[i], sub(big_one_mont<8>(), hu[i]));
+            v[i] = run;
+            run = mont_mul(run, w[i]);
+        }
+        back = !is_zero(run);
+        if (back) {
+            run = mont_inverse(run);
+            for (size_t i = m; i-- > 0;) { v[i] = mont_mul(v[i], run); run = mont_mul(run, w[i]); }
+            const void* vd = nullptr;
+            int rc = job.up.put(v.data(), sizeof(Fr) * m, st, &vd);
+            if (rc) return rc;
+            V_dev = (const Fr*)vd;
+        }
+    }
+    auto t_given = [&](int r) { return back || (r == 0 ? with_rows : r < t_rounds && r != t_again); };
     std::vector<PointDesc> later;        // bucket reductions that nothing waits for before the end: one launch behind the last round
-    if (t_rounds > 1) GLAUNCH(k_g1_fill, npts * count, st, job.pts, g1_infinity(), npts * count);
+    if (t_rounds > 1 || back) GLAUNCH(k_g1_fill, npts * count, st, job.pts, g1_infinity(), npts * count);
     if (with_rows) {
         int rc = join_streams(st, aux, job.events);          // the challenges travel on st
-        if (rc == 0) rc = open_cross_sums_queue(items, count, (uint32_t)cross_r, job.pts, npts, urow_dev, U_dev, rounds, job.arena, job.up, aux, later);
+        if (rc == 0) rc = open_cross_sums_queue(items, count, (uint32_t)cross_r, job.pts, npts, urow_dev, U_dev, rounds, job.arena, job.up, aux, job.events, later);
         if (rc) return rc;
     }
     size_t size = n;
@@ -2578,7 +2798,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     }
     auto reductions = [&]() {            // on aux: the sums that nothing waited for, and T of the rounds that follow from them
         int rc = points_queue(later, job.arena, job.up, aux);
-        if (rc == 0 && unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, rounds, job.arena, job.up, aux);
+        if (rc == 0 && unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, nullptr, nullptr, rounds, job.arena, job.up, aux);
         return rc;
     };
     while (r < rounds) {
@@ -2623,7 +2843,7 @@ static int open_queue(OpenJob& job, const OpenItem* items, int count, size_t n, 
     {
         int rc = unroll_early && aux != st && tail_done ? 0 : reductions();
         if (rc == 0) rc = join_streams(aux, st, job.events);
-        if (rc == 0 && !unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, rounds, job.arena, job.up, st);
+        if (rc == 0 && !unroll_early) rc = open_unroll_queue(job.pts, npts, count, t_rounds, t_again, U_dev, V_dev, cs, rounds, job.arena, job.up, st);
         if (rc) return rc;
     }
     if (!tail_done)
