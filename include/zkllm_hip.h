@@ -147,6 +147,8 @@ int zk_fr_fold_axis_all(void* out, const void* in, const uint32_t* u, int levels
  * in[other][cur][window] with cur <= 2^levels (elements beyond cur count as zero):
  * out[o][w] = sum_j eq(u, j) in[o][j][w], u[0] on the lowest bit of j; bit-identical to the level-by-level fold. */
 int zk_fr_fold_prepare(void** prepared, const void* t, size_t n, void* stream);
+/* without the wait: *bad_flag_dev (4 bytes of device memory) is raised if some element is no 32-bit integer; the handle is then to be freed unused */
+int zk_fr_fold_prepare_queue(void** prepared, void* bad_flag_dev, const void* t, size_t n, void* stream);
 int zk_fr_fold_axis_prepared(void* out, const void* prepared, const uint32_t* u, int levels, size_t other, uint32_t cur, size_t window, void* stream);
 /* the same fold of the elementwise product of two such tensors (handles of equal size): out[o][w] = sum_j eq(u, j) a[o][j][w] b[o][j][w] */
 int zk_fr_fold_axis_prod(void* out, const void* a_prepared, const void* b_prepared, const uint32_t* u, int levels, size_t other, uint32_t cur, size_t window, void* stream);
@@ -323,6 +325,11 @@ int zk_g1_open_end_batch(void* handle, uint32_t* proof_host, uint32_t* final_sca
  * unlike the reference, a value outside [low, low+table_size) is an error instead of an unchecked access */
 int zk_lookup_index_fr(void* idx_u32, const void* vals_fr, int32_t low, uint32_t table_size, size_t n, void* stream);
 int zk_lookup_index_i32(void* idx_u32, const void* vals_i32, int32_t low, uint32_t table_size, size_t n, void* stream);
+/* zk_lookup_multiplicities in two halves, for a caller that has other work to queue before it needs to know whether every query lies in the
+ * table: begin queues the counting, end waits for it and returns the error.  Every handle must be ended exactly once. */
+int zk_lookup_multiplicities_begin(void** check, void* m, void* idx_out, const void* idx, const void* vals_i32, const void* vals, int32_t low, uint32_t len, size_t n, uint32_t nbins,
+                                   void* stream);
+int zk_lookup_multiplicities_end(void* check);
 /* multiplicities of a table's nbins entries as field elements (tlookup_kernel :10-15, count_to_m :17-20) from table positions (idx; not
  * checked, as there), int32 queries or queries as field elements, the first that is not null; idx_out: the positions too, or null.  A query
  * outside [low, low + len) is an error, known when the call returns.  inside: the caller knows every query to lie in the table; nothing is
@@ -396,6 +403,17 @@ int zk_lookup_prove_begin_mapped_ints(void** handle, const void* S_in, const voi
 int zk_lookup_prove_begin_mapped_out_ints(void** handle, const void* S_in, const void* S_out, const void* S_out_prepared, const void* mapped_prepared, const uint32_t* r,
                                           const void* T, const void* m, int32_t low, const uint32_t* beta, const uint32_t* u_eq, const uint32_t* v, size_t D, size_t N, int rounds,
                                           void* stream);
+/* A lookup job in two steps: _open inverts the table (N >= 2 entries T + beta) on the job's stream, behind what `stream` holds; what the
+ * caller queues next runs beside that.  _begin_opened is zk_lookup_prove_begin_hinted(_ints) (S_out, r null; S_prepared null or the queries'
+ * int32 form) or _mapped, _mapped_ints and _mapped_out_ints (by the int32 forms that are given) on it, with the same T, beta and N: a job that is begun belongs to *handle,
+ * after an error and without a begin the opened one goes to _open_drop.  queries_ready: everything but m was in place when the job was
+ * opened, and only the rounds over the table wait for what `stream` holds at begin.  launch_here: the launches are queued by the calling
+ * thread, whether or not zk_async_jobs is on. */
+int zk_lookup_open(void** opened, const void* T, const uint32_t* beta, size_t N, void* stream);
+int zk_lookup_open_drop(void* opened);
+int zk_lookup_prove_begin_opened(void** handle, void* opened, const void* S, const void* S_prepared, const void* S_out, const void* S_out_prepared, const void* mapped_prepared,
+                                 const uint32_t* r, const void* T, const void* m, int32_t low, const uint32_t* beta, const uint32_t* u_eq, const uint32_t* v, size_t D, size_t N,
+                                 int rounds, int queries_ready, int launch_here, void* stream);
 int zk_lookup_prove_end(void* handle, uint32_t* bm_host, uint32_t* sums_host);
 /* Diagnostics of the job zk_lookup_prove_end collected last (no counterpart in the reference): *n_ok = how many leading table
  * entries were what the integers say -- the queries naming one of them took the first round's short path, the others their own
@@ -434,6 +452,8 @@ int zk_rescale_ints_both(void* out, void* out_ints, int* out_fits_host, void* re
 int zk_rescale_ints_both_flag(void* out, void* out_ints, void* bad_flag_dev, void* rem, void* rem_ints, const void* in, uint32_t scaling_factor, size_t n, void* stream);
 /* out[i] = i < n ? in[i] : *fill for i < n_out; fill on the device (field elements / int32, the latter with the value where fill is null) */
 int zk_fr_pad_from(void* out, const void* in, size_t n, size_t n_out, const void* fill, void* stream);
+/* out = in, its first element plus `more` (a canonical field element): the padding queries of a mapping table in its multiplicities */
+int zk_fr_copy_add_first(void* out, const void* in, const uint32_t* more, size_t n, void* stream);
 int zk_i32_pad_from(void* out_i32, const void* in_i32, size_t n, size_t n_out, const void* fill_i32, int32_t value, void* stream);
 int zk_i32_fill(void* dst_i32, int32_t value, size_t n, void* stream);       /* n int32 slots set to value (padding of an int32 form) */
 /* zkrelu_decomp_kernel zkrelu.cu:8-29: the same rescaling, then sign (1 when the rescaled value is >= 0), magnitude and max(., 0) */

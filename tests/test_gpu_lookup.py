@@ -787,6 +787,91 @@ def test_hinted_lookup_job_equals_the_plain_one_whatever_the_hints(k):
         hip.free(p)
 
 
+# tables of two entries, as many entries as queries (no phase-1 round), a first round that writes the inverses out, that forms them, and two rounds in one
+@pytest.mark.parametrize("k,N", [(1, 2), (6, 64), (6, 2), (13, 64), (17, 64), (19, 1 << 15)])
+def test_lookup_job_opened_ahead_equals_the_one_begun_at_once(k, N):
+    """zk_lookup_open and zk_lookup_prove_begin_opened against zk_lookup_prove_begin_hinted: multiplicities counted behind the opening, queries outside the table."""
+    import ctypes
+    from gpuhelp import Hip, c_void_p, c_size_t, c_int
+    hip = Hip()
+    D, low = 1 << k, -(N // 2)
+    rng = np.random.default_rng(k)
+    vals = rng.integers(low, low + N, D)
+    good = fr_array([int(x) % R_MOD for x in vals])
+    S = good.copy()
+    if D > 64:
+        S[5], S[D - 1] = fr_array([low + N + 3])[0], ch(46, 1)[0]
+    T = fr_array([(low + i) % R_MOD for i in range(N)])
+    beta, u, v = ch(43, 1)[0], ch(44, max(k - 1, 1)), ch(45, k)
+    dS, dG, dT, dm, dn = hip.upload(S), hip.upload(good), hip.upload(T), hip.malloc(32 * N), hip.malloc(32 * N)
+    sizes = (c_size_t(D), c_size_t(N), c_int(k))
+
+    def end(h):
+        bm, sums = np.zeros(8, np.uint32), np.zeros((k * 11, 8), np.uint32)
+        hip.call("zk_lookup_prove_end", h, bm, sums)
+        return bm, sums
+    hip.call("zk_lookup_multiplicities", c_void_p(dm), None, None, None, c_void_p(dG), c_int(low), c_int(N), c_size_t(D), c_int(N), c_int(0), None)
+    h = c_void_p()
+    hip.call("zk_lookup_prove_begin_hinted", ctypes.byref(h), c_void_p(dS), c_void_p(dT), c_void_p(dm), c_void_p(dS), c_int(low), beta, u, v, *sizes, None)
+    bm, sums = end(h)
+    inv = [pow((low + i + fr_ints(beta.reshape(1, 8))[0]) % R_MOD, -1, R_MOD) for i in range(N)]
+    counts = np.bincount(vals - low, minlength=N)
+    assert fr_ints(bm.reshape(1, 8))[0] == sum(int(c) * b for c, b in zip(counts, inv)) % R_MOD
+    for ready in (0, 1):
+        for here in (0, 1):
+            o, h, check = c_void_p(), c_void_p(), c_void_p()
+            hip.call("zk_lookup_open", ctypes.byref(o), c_void_p(dT), beta, c_size_t(N), None)
+            hip.call("zk_lookup_multiplicities_begin", ctypes.byref(check), c_void_p(dn), None, None, None, c_void_p(dG), c_int(low), c_int(N), c_size_t(D), c_int(N), None)
+            hip.call("zk_lookup_prove_begin_opened", ctypes.byref(h), o, c_void_p(dS), None, None, None, None, None, c_void_p(dT), c_void_p(dn), c_int(low), beta, u, v, *sizes,
+                     c_int(ready), c_int(here), None)
+            hip.call("zk_lookup_multiplicities_end", check)
+            got = end(h)
+            assert (got[0] == bm).all() and (got[1] == sums).all(), (ready, here)
+    # a job that is refused stays the caller's, and one that is never begun is dropped; a query outside the table is reported by the second half
+    o, h, check = c_void_p(), c_void_p(), c_void_p()
+    hip.call("zk_lookup_open", ctypes.byref(o), c_void_p(dT), beta, c_size_t(N), None)
+    with pytest.raises(RuntimeError, match="no opened job"):
+        hip.call("zk_lookup_prove_begin_opened", ctypes.byref(h), o, c_void_p(dS), None, None, None, None, None, c_void_p(dT), c_void_p(dn), c_int(low), beta, u, v, c_size_t(D), c_size_t(2 * N),
+                 c_int(k), c_int(1), c_int(1), None)
+    hip.call("zk_lookup_open_drop", o)
+    if D > 64:
+        hip.call("zk_lookup_multiplicities_begin", ctypes.byref(check), c_void_p(dn), None, None, None, c_void_p(dS), c_int(low), c_int(N), c_size_t(D), c_int(N), None)
+        with pytest.raises(RuntimeError, match="outside the table"):
+            hip.call("zk_lookup_multiplicities_end", check)
+    for p in (dS, dG, dT, dm, dn):
+        hip.free(p)
+
+
+def test_range_proof_of_a_query_outside_its_table_is_an_error_and_leaves_nothing_behind(pv):
+    """The proof has begun when the range check is read: the job is dropped, nothing is recorded, and the next proof is the same as before."""
+    D, low, length = 1 << 13, -32, 60
+    vals = np.random.default_rng(7).integers(low, low + length, D)
+    S = fr_array([int(x) % R_MOD for x in vals])
+    bad = S.copy()
+    bad[D // 3] = fr_array([low + length])[0]          # in the padded table, outside the range
+    mv = ch(6, length)
+    k = D.bit_length() - 1
+    r, alpha, beta, u, v = ch(7, 1)[0], ch(8, 1)[0], ch(9, 1)[0], ch(10, k), ch(11, k)
+
+    def good():
+        pv.transcript_begin()
+        fin = pv.range_prove(pv.from_fr(S), low, length, alpha, beta, u, v)
+        y, m, fin2 = pv.mapping(pv.from_fr(S), low, length, pv.from_fr(mv), r, alpha, beta, u, v)
+        t = pv.transcript()
+        pv.lib.zkp_transcript_end()
+        return fin, fin2, y.host(), m.host(), t
+    first = good()
+    pv.transcript_begin()
+    with pytest.raises(RuntimeError, match="outside the table"):
+        pv.range_prove(pv.from_fr(bad), low, length, alpha, beta, u, v)
+    with pytest.raises(RuntimeError, match="outside the table"):
+        pv.mapping(pv.from_fr(bad), low, length, pv.from_fr(mv), r, alpha, beta, u, v)
+    assert pv.transcript().shape[0] == 0
+    pv.lib.zkp_transcript_end()
+    for a, b in zip(first, good()):
+        assert a.shape == b.shape and (a == b).all()
+
+
 def test_jobs_launched_by_the_library_thread_equal_those_launched_by_the_caller():
     """zk_set_async_jobs: with it on, begin hands a job's launches to the library's launch thread and returns; off, the caller
     queues them itself.  Four lookup jobs and two Hadamard jobs begun back to back (more jobs than streams of that kind, so

@@ -290,6 +290,13 @@ void FrTensor::keep_for_folds() {
         ZKC(zk_fr_fold_prepare(&fold_cache->prepared, gpu_data, size, nullptr));
     }
 }
+void FrTensor::keep_for_folds_queued() {
+    if (!fold_cache) fold_cache = std::make_shared<FoldCache>();
+    if (fold_cache->tried) return;
+    ZKC(zk_malloc(&fold_cache->unchecked, 4));
+    ZKC(zk_fr_fold_prepare_queue(&fold_cache->prepared, fold_cache->unchecked, gpu_data, size, nullptr));
+    fold_cache->tried = true;
+}
 void* FrTensor::ints_for_producer() {
     if (!fold_cache) fold_cache = std::make_shared<FoldCache>();
     fold_cache->reset();

@@ -182,6 +182,7 @@ class FrTensor {
     // holds 32-bit integers, fold its int32 form (bit-identical results).  Every operation that changes the elements drops
     // what was kept.
     void keep_for_folds();
+    void keep_for_folds_queued();      // without its wait: whether every element is a 32-bit integer is read at the first question for that form
     void drop_kept();       // what keep_as_matmul_rhs and keep_for_folds hold, after the elements have changed
     // A tensor whose int32 form is written by the kernel that writes the tensor: allocates that form (zk_fr_fold_prepared_new)
     // and keeps it as keep_for_folds would; returns its device address for the kernel.  Call before the kernel is queued.

@@ -400,10 +400,10 @@ void* zkp_batch_inv(void* in, const u32* beta) {
 int zkp_range_prove(void* S, int low, u32 len, const u32* alpha, const u32* beta, const u32* u, const u32* v, u32* final_claim) {
     ZKP_TRY
     tLookupRange t(low, len);
-    FrTensor m = t.prep(FT(S));
     const int k = (int)ceilLog2(FT(S).size);
-    std::vector<Polynomial> proof;
-    Fr_t f = t.prove(FT(S), m, fr1(alpha), fr1(beta), frs(u, k), frs(v, k), proof);
+    std::unique_ptr<FrTensor> m;
+    LookupPending p = t.count_and_prove_begin(FT(S), m, false, fr1(alpha), fr1(beta), frs(u, k), frs(v, k), true);
+    Fr_t f = tLookupRange::prove_end(p);
     memcpy(final_claim, f.val, 32);
     ZKP_END
 }
@@ -411,8 +411,16 @@ int zkp_range_prove(void* S, int low, u32 len, const u32* alpha, const u32* beta
 int zkp_mapping(void* S_in, int low, u32 len, void* mvals, const u32* r, const u32* alpha, const u32* beta, const u32* u, const u32* v, void** y_out, void** m_out, u32* final_claim) {
     ZKP_TRY
     tLookupRangeMapping t(low, len, FT(mvals));
-    // a proof of more than one query ends behind the outputs that it was begun on
-    auto p = final_claim && FT(S_in).size > 1 ? t.map_queued(FT(S_in)) : t(FT(S_in));
+    if (final_claim && FT(S_in).size > 1) {          // the proof ends behind the outputs that it was begun on
+        const int k = (int)ceilLog2(FT(S_in).size);
+        auto p = t.map_and_prove_begin(FT(S_in), fr1(r), fr1(alpha), fr1(beta), frs(u, k), frs(v, k));
+        Fr_t f = tLookupRange::prove_end(p.look);
+        memcpy(final_claim, f.val, 32);
+        if (y_out) *y_out = p.y.release();
+        if (m_out) *m_out = p.m.release();
+        return 0;
+    }
+    auto p = t(FT(S_in));
     if (final_claim) {
         const int k = (int)ceilLog2(FT(S_in).size);
         std::vector<Polynomial> proof;

@@ -36,7 +36,9 @@ Rescaling::~Rescaling() {}
 
 // rescaling.cu:41-79.  Challenge order: u, v, (alpha, beta).
 vector<Claim> Rescaling::prove(const FrTensor& X, const FrTensor& X_) {
-    Pending p = prove_begin(X, X_);
+    if (X.size != X_.size) throw std::runtime_error("Error: the size of X and X_ should be the same.");
+    if (!rem_tensor_ptr) throw std::runtime_error("Rescaling::prove called before operator()");
+    Pending p = prove_begin(X, X_, draw(X.size), true);
     prove_end(p);
     return {};
 }
@@ -52,7 +54,7 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_)
     if (!rem_tensor_ptr) throw std::runtime_error("Rescaling::prove called before operator()");
     return prove_begin(X, X_, draw(X.size));
 }
-Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_, const Challenges& ch) {
+Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_, const Challenges& ch, bool at_once) {
     if (X.size != X_.size) throw std::runtime_error("Error: the size of X and X_ should be the same.");
     if (!rem_tensor_ptr) throw std::runtime_error("Rescaling::prove called before operator()");
     const vector<Fr_t>&u = ch.u, &v = ch.v, &rand_temp = ch.rand_temp;
@@ -70,9 +72,9 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_,
         }
         p.rem = padded;
     }
-    p.m.reset(new FrTensor(tl_rem.prep_inside(*p.rem)));          // remainders of a division by the table's length
     // the lookup's job first: its kernels wait for what is queued here so far, and the evaluations below run beside them
-    p.look = tl_rem.prove_begin(*p.rem, *p.m, rand_temp[0], rand_temp[1], u, v);
+    // (inside: remainders of a division by the table's length)
+    p.look = tl_rem.count_and_prove_begin(*p.rem, p.m, true, rand_temp[0], rand_temp[1], u, v, at_once);
     // X_(u) and rem(u) in one pass over the two tensors (the padding of the remainders is zeros: the unpadded tensor has the same
     // extension and the others' length).  X = scaling_factor X_ + rem element by element, so X(u) is that combination of the two
     // values: X itself, 32 bytes an element, is read only with ZKLLM_CHECK_CLAIMS=1, which evaluates it and compares as

@@ -42,7 +42,7 @@ class Rescaling {
     // challenges drawn apart from the proof (same order: u, v, then the lookup's two)
     struct Challenges { vector<Fr_t> u, v, rand_temp; };
     static Challenges draw(uint size);
-    Pending prove_begin(const FrTensor& X, const FrTensor& X_, const Challenges& ch);
+    Pending prove_begin(const FrTensor& X, const FrTensor& X_, const Challenges& ch, bool at_once = false);      // at_once: the caller ends the proof next
     void prove_end(Pending& p);
     ~Rescaling();
     Rescaling(const Rescaling&) = delete;

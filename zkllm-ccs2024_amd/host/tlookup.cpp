@@ -1,6 +1,7 @@
 #include "tlookup.hpp"
 
 #include <cstring>
+#include <iterator>
 
 #include "../../include/zkllm_hip.h"
 #include "../csrc/field.hpp"
@@ -26,12 +27,19 @@ static FrTensor counts_to_m_i32(const void* vals_i32, int low, uint len, uint D,
     ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, nullptr, vals_i32, nullptr, low, len, D, N, 0, nullptr));
     return m;
 }
-// and from the queries themselves, their positions with them where idx is given
-static FrTensor counts_to_m(void* idx, const FrTensor& vals, int low, uint len, uint N, bool inside = false) {
+// and from the queries themselves
+static FrTensor counts_to_m(const FrTensor& vals, int low, uint len, uint N, bool inside = false) {
     const void* h = vals.kept_ints();
     FrTensor m(N);
-    ZKC(zk_lookup_multiplicities(m.gpu_data, idx, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, N, inside, nullptr));
+    ZKC(zk_lookup_multiplicities(m.gpu_data, nullptr, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, N, inside, nullptr));
     return m;
+}
+LookupOpened::~LookupOpened() { if (handle) (void)zk_lookup_open_drop(handle); }
+CountedQueries::~CountedQueries() { if (check) (void)zk_lookup_multiplicities_end(check); }
+void CountedQueries::settle() {
+    void* c = check;
+    check = nullptr;
+    if (c) ZKC(zk_lookup_multiplicities_end(c));
 }
 
 FrTensor tLookup::prep(const uint* indices, const uint D) { return counts_to_m(indices, D, table.size); }
@@ -44,8 +52,8 @@ static FrTensor make_range_table(int low, uint len) {
 tLookupRange::tLookupRange(int low, uint len) : tLookup(make_range_table(low, len)), low(low), len(len) {}
 
 FrTensor tLookupRange::prep(const int* vals, const uint D) { return counts_to_m_i32(vals, low, len, D, table.size); }
-FrTensor tLookupRange::prep(const FrTensor& vals) { return counts_to_m(nullptr, vals, low, len, table.size); }
-FrTensor tLookupRange::prep_inside(const FrTensor& vals) { return counts_to_m(nullptr, vals, low, len, table.size, true); }
+FrTensor tLookupRange::prep(const FrTensor& vals) { return counts_to_m(vals, low, len, table.size); }
+FrTensor tLookupRange::prep_inside(const FrTensor& vals) { return counts_to_m(vals, low, len, table.size, true); }
 
 // mapped values padded by repeating the last one (tlookup.cu:435-444)
 static FrTensor make_mapped(uint len, const FrTensor& mvals) {
@@ -55,7 +63,7 @@ static FrTensor make_mapped(uint len, const FrTensor& mvals) {
     return out;
 }
 tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mvals) : tLookupRange(low, len), mapped_vals(make_mapped(len, mvals)) {
-    mapped_vals.keep_for_folds();          // examined once: outputs of operator() carry an int32 form when these are 32-bit integers
+    mapped_vals.keep_for_folds_queued();          // examined once: outputs of operator() carry an int32 form when these are 32-bit integers
 }
 
 pair<FrTensor, FrTensor> tLookupRangeMapping::operator()(const int* vals, const uint D) {
@@ -74,10 +82,21 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::map(const FrTensor& vals, const Fr
     return p;
 }
 pair<FrTensor, FrTensor> tLookupRangeMapping::map_queued(const FrTensor& vals, const FrTensor* unwritten) {
+    CountedQueries c;
     // queries and mapped values in int32 form: nothing below needs the array of table positions
-    const bool by_queries = mapped_vals.kept_ints() && vals.kept_ints();
-    DevBuf idx(by_queries ? 4 : sizeof(uint) * (size_t)vals.size);
-    FrTensor m = counts_to_m(by_queries ? nullptr : idx.p, vals, low, len, table.size);
+    count(c, vals, !(vals.kept_ints() && mapped_vals.kept_ints()));
+    c.settle();
+    FrTensor y = gather(vals, c, unwritten);
+    return {std::move(y), std::move(*c.m)};
+}
+void tLookupRangeMapping::count(CountedQueries& c, const FrTensor& vals, bool positions) {
+    if (positions) c.idx.reset(new DevBuf(sizeof(uint) * (size_t)vals.size));
+    const void* h = vals.kept_ints();
+    c.m.reset(new FrTensor(table.size));
+    ZKC(zk_lookup_multiplicities_begin(&c.check, c.m->gpu_data, positions ? c.idx->p : nullptr, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, table.size, nullptr));
+}
+// the outputs of counted queries
+FrTensor tLookupRangeMapping::gather(const FrTensor& vals, const CountedQueries& c, const FrTensor* unwritten) {
     const bool ints_only_out = unwritten && unwritten->size == vals.size && mapped_vals.kept_ints() && vals.kept_ints();
     FrTensor y = ints_only_out ? FrTensor::view(*unwritten) : FrTensor(vals.size);
     // mapped values that are 32-bit integers: the outputs get their int32 form with them
@@ -85,9 +104,9 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::map_queued(const FrTensor& vals, c
         // queries with an int32 form: gathered by them, and the outputs' form remembers it (the proof's first round then trusts them)
         y.ints_for_producer();
         ZKC(zk_fr_gather_by_queries_ints(ints_only_out ? nullptr : y.gpu_data, const_cast<void*>(y.kept_ints()), vals.kept_ints(), low, th, vals.size, nullptr));
-    } else if (th) ZKC(zk_fr_gather_ints(y.gpu_data, y.ints_for_producer(), mapped_vals.gpu_data, th, idx.p, vals.size, nullptr));
-    else ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, idx.p, vals.size, nullptr));
-    return {std::move(y), std::move(m)};
+    } else if (th) ZKC(zk_fr_gather_ints(y.gpu_data, y.ints_for_producer(), mapped_vals.gpu_data, th, c.idx->p, vals.size, nullptr));
+    else ZKC(zk_fr_gather(y.gpu_data, mapped_vals.gpu_data, c.idx->p, vals.size, nullptr));
+    return y;
 }
 
 static void drop_lookup_job(void* h, size_t rounds) {
@@ -114,14 +133,14 @@ LookupPending& LookupPending::operator=(LookupPending&& o) noexcept {
 // derives the next claim.
 // S_out / r given: S0 holds the input queries of a mapping table, the combined query S0 + r * S_out is formed on the device
 static LookupPending sumcheck_begin(const FrTensor& S0, const FrTensor& T0, const FrTensor& m0, const Fr_t& alpha0, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
-                                    const FrTensor* hint, int low, const FrTensor* S_out, const Fr_t* r, const void* mapped_ints = nullptr);
+                                    const FrTensor* hint, int low, const FrTensor* S_out, const Fr_t* r, const void* mapped_ints = nullptr, LookupOpened* opened = nullptr, bool queries_ready = false, bool at_once = false);
 LookupPending tLookup_sumcheck_begin(const FrTensor& S0, const FrTensor& T0, const FrTensor& m0, const Fr_t& alpha0, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
                                      const FrTensor* hint, int low) {
     return sumcheck_begin(S0, T0, m0, alpha0, beta, u, v, hint, low, nullptr, nullptr);
 }
 // mapped_ints: the int32 form of the mapping table's (padded) mapped values, when it keeps one
 static LookupPending sumcheck_begin(const FrTensor& S0, const FrTensor& T0, const FrTensor& m0, const Fr_t& alpha0, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
-                                    const FrTensor* hint, int low, const FrTensor* S_out, const Fr_t* r, const void* mapped_ints) {
+                                    const FrTensor* hint, int low, const FrTensor* S_out, const Fr_t* r, const void* mapped_ints, LookupOpened* opened, bool queries_ready, bool at_once) {
     const uint D = S0.size, N = m0.size;
     if (S_out && S_out->size != D) throw std::runtime_error("lookup: input and output queries differ in size");
     if (m0.size != T0.size) throw std::runtime_error("m.size != table.size");
@@ -139,7 +158,11 @@ static LookupPending sumcheck_begin(const FrTensor& S0, const FrTensor& T0, cons
     if (hint && hint->size != D) throw std::runtime_error("lookup hint must have one entry per query");
     // queries that keep an int32 form (the digit planes of a softmax, the outputs of a mapping table) are read from it
     const void *qi = S0.kept_ints(), *oi = S_out ? S_out->kept_ints() : nullptr;
-    if (S_out && qi && oi && mapped_ints)
+    if (opened) {          // hint: the queries, or the mapped queries
+        ZKC(zk_lookup_prove_begin_opened(&p.handle, opened->handle, S0.gpu_data, qi, S_out ? S_out->gpu_data : nullptr, oi, mapped_ints, r ? r->val : nullptr, T0.gpu_data, m0.gpu_data, low,
+                                         beta.val, u[0].val, vs[0].val, D, N, (int)k, queries_ready, at_once, nullptr));
+        opened->handle = nullptr;
+    } else if (S_out && qi && oi && mapped_ints)
         ZKC(zk_lookup_prove_begin_mapped_ints(&p.handle, S0.gpu_data, qi, S_out->gpu_data, oi, mapped_ints, r->val, T0.gpu_data, m0.gpu_data, low, beta.val, u[0].val, vs[0].val,
                                               D, N, (int)k, nullptr));
     else if (S_out && oi && mapped_ints)
@@ -233,6 +256,27 @@ LookupPending tLookupRange::prove_begin(const FrTensor& S, const FrTensor& m, co
     if (m.size != table.size) throw std::runtime_error("m.size != table.size");
     return tLookup_sumcheck_begin(S, table, m, alpha, beta, u, v, &S, low);
 }
+// what a proof over N table entries and D queries has to be for its table to be inverted ahead (anything else goes through prove_begin, which says what is wrong)
+static bool can_open(uint D, uint N, const vector<Fr_t>& u, const vector<Fr_t>& v) {
+    return N >= 2 && N == (1u << ceilLog2(N)) && D == (1u << ceilLog2(D)) && D % N == 0 && u.size() == ceilLog2(D) && v.size() == ceilLog2(D);
+}
+LookupPending tLookupRange::count_and_prove_begin(const FrTensor& S, std::unique_ptr<FrTensor>& m, bool inside, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v, bool at_once) {
+    if (!can_open(S.size, table.size, u, v)) {
+        m.reset(new FrTensor(inside ? prep_inside(S) : prep(S)));
+        return prove_begin(S, *m, alpha, beta, u, v);
+    }
+    const void* h = S.kept_ints();
+    const void* ints = h ? zk_fr_fold_prepared_ints(h) : nullptr;
+    LookupOpened opened;
+    ZKC(zk_lookup_open(&opened.handle, table.gpu_data, beta.val, table.size, nullptr));
+    m.reset(new FrTensor(table.size));
+    CountedQueries c;
+    if (inside) ZKC(zk_lookup_multiplicities(m->gpu_data, nullptr, nullptr, ints, S.gpu_data, low, len, S.size, table.size, 1, nullptr));
+    else ZKC(zk_lookup_multiplicities_begin(&c.check, m->gpu_data, nullptr, nullptr, ints, S.gpu_data, low, len, S.size, table.size, nullptr));
+    LookupPending p = sumcheck_begin(S, table, *m, alpha, beta, u, v, &S, low, nullptr, nullptr, nullptr, &opened, true, at_once);
+    c.settle();
+    return p;
+}
 Fr_t tLookupRange::prove(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v, vector<Polynomial>& proof) {
     LookupPending p = prove_begin(S, m, alpha, beta, u, v);
     return tLookup_sumcheck_end(p);
@@ -240,40 +284,80 @@ Fr_t tLookupRange::prove(const FrTensor& S, const FrTensor& m, const Fr_t& alpha
 
 LookupPending tLookupRangeMapping::prove_begin(const FrTensor& S_in, const FrTensor& S_out, const FrTensor& m, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta,
                                                const vector<Fr_t>& u, const vector<Fr_t>& v) {
+    return prove_begin_on(S_in, S_out, m, r, alpha, beta, u, v, nullptr);
+}
+std::unique_ptr<FrTensor> tLookupRangeMapping::combined(const Fr_t& r) const {
+    std::unique_ptr<FrTensor> T(new FrTensor(table.size));
+    ZKC(zk_fr_add_mul_s(T->gpu_data, table.gpu_data, mapped_vals.gpu_data, r.val, T->size, nullptr));
+    return T;
+}
+tLookupRangeMapping::MappedPending tLookupRangeMapping::map_and_prove_begin(const FrTensor& S_in, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v) {
+    MappedPending p;
+    if (!can_open(1u << ceilLog2(S_in.size), table.size, u, v)) {
+        auto ym = map_queued(S_in);
+        p.y.reset(new FrTensor(std::move(ym.first)));
+        p.m.reset(new FrTensor(std::move(ym.second)));
+        p.look = prove_begin(S_in, *p.y, *p.m, r, alpha, beta, u, v);
+        return p;
+    }
+    const bool positions = !(S_in.kept_ints() && mapped_vals.kept_ints());      // (asked before anything else is queued only where the queries have an int32 form)
+    LookupOpened opened;
+    opened.table = combined(r);
+    ZKC(zk_lookup_open(&opened.handle, opened.table->gpu_data, beta.val, table.size, nullptr));
+    CountedQueries c;
+    count(c, S_in, positions);
+    if (S_in.size != (1u << ceilLog2(S_in.size)) && !S_in.kept_ints()) {          // neither waits for what is asked next
+        opened.queries = padded(opened.keep, S_in, table, false, nullptr);
+        opened.m = padded_m(opened.keep, *c.m, S_in.size);
+    }
+    (void)mapped_vals.kept_ints();          // one wait for this and the range check
+    c.settle();
+    p.y.reset(new FrTensor(gather(S_in, c, nullptr)));
+    p.m = std::move(c.m);
+    p.look = prove_begin_on(S_in, *p.y, *p.m, r, alpha, beta, u, v, &opened);
+    return p;
+}
+// Queries padded to a power of two with the first table entry, which are accounted for in m[0] (tlookup.cu:502-510).  Queries and outputs that
+// keep int32 forms are padded in that form; where the job reads nothing else (zk_lookup_ints_suffice) the padded field elements are not written at all.
+FrTensor* tLookupRangeMapping::padded(std::vector<std::unique_ptr<FrTensor>>& keep, const FrTensor& t, const FrTensor& fill_from, bool ints, const void* fill_ints) const {
+    const uint D = t.size, Dp = 1u << ceilLog2(D);
+    FrTensor* p = new FrTensor(Dp);
+    keep.emplace_back(p);
+    if (!(ints && zk_lookup_ints_suffice(Dp, table.size))) ZKC(zk_fr_pad_from(p->gpu_data, t.gpu_data, D, Dp, fill_from.gpu_data, nullptr));
+    if (ints) ZKC(zk_i32_pad_from(p->ints_for_producer(), zk_fr_fold_prepared_ints(t.kept_ints()), D, Dp, fill_ints, low, nullptr));
+    return p;
+}
+FrTensor* tLookupRangeMapping::padded_m(std::vector<std::unique_ptr<FrTensor>>& keep, const FrTensor& m, uint D) const {
+    keep.emplace_back(new FrTensor(m.size));
+    const Fr_t more{{(1u << ceilLog2(D)) - D, 0, 0, 0, 0, 0, 0, 0}};
+    ZKC(zk_fr_copy_add_first(keep.back()->gpu_data, m.gpu_data, more.val, m.size, nullptr));
+    return keep.back().get();
+}
+LookupPending tLookupRangeMapping::prove_begin_on(const FrTensor& S_in, const FrTensor& S_out, const FrTensor& m, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta,
+                                                  const vector<Fr_t>& u, const vector<Fr_t>& v, LookupOpened* opened) {
     const uint D = S_in.size;
     if (m.size != table.size) throw std::runtime_error("m.size != table.size");
     std::vector<std::unique_ptr<FrTensor>> keep;
     const FrTensor *si = &S_in, *so = &S_out, *mm = &m;
     if (D != (1u << ceilLog2(D))) {
-        // pad the queries with the first table entry and account for them in m[0] (tlookup.cu:502-510)
-        const uint Dp = 1u << ceilLog2(D);
-        // Queries and outputs that keep int32 forms are padded in that form; where the job reads nothing else (zk_lookup_ints_suffice) the
-        // padded field elements are not written at all.
         const bool out_ints = S_out.kept_ints() && mapped_vals.kept_ints(), in_ints = out_ints && S_in.kept_ints();
-        const bool suffice = zk_lookup_ints_suffice(Dp, table.size) != 0;
-        auto padded = [&](const FrTensor& t, const FrTensor& fill_from, bool ints, const void* fill_ints) {
-            FrTensor* p = new FrTensor(Dp);
-            keep.emplace_back(p);
-            if (!(ints && suffice)) ZKC(zk_fr_pad_from(p->gpu_data, t.gpu_data, D, Dp, fill_from.gpu_data, nullptr));
-            if (ints) ZKC(zk_i32_pad_from(p->ints_for_producer(), zk_fr_fold_prepared_ints(t.kept_ints()), D, Dp, fill_ints, low, nullptr));
-            return p;
-        };
-        si = padded(S_in, table, in_ints, nullptr);          // the first table entry is low
-        so = padded(S_out, mapped_vals, out_ints, out_ints ? zk_fr_fold_prepared_ints(mapped_vals.kept_ints()) : nullptr);
-        keep.emplace_back(new FrTensor(m));
-        FrTensor* m_ = keep.back().get();
-        const Fr_t more{{Dp - D, 0, 0, 0, 0, 0, 0, 0}};
-        ZKC(zk_fr_add_s(m_->gpu_data, m_->gpu_data, more.val, 1, nullptr));
-        mm = m_;
+        if (opened && opened->queries) { si = opened->queries; mm = opened->m; }
+        else {
+            si = padded(keep, S_in, table, in_ints, nullptr);          // the first table entry is low
+            mm = padded_m(keep, m, D);
+        }
+        so = padded(keep, S_out, mapped_vals, out_ints, out_ints ? zk_fr_fold_prepared_ints(mapped_vals.kept_ints()) : nullptr);
     }
     const uint N = mm->size;
     if (N != (1u << ceilLog2(N)) || si->size % N != 0) throw std::runtime_error("N is not power of 2, or D is not divisible by N");
     // S_com = S_in + r * S_out (tlookup.cu:517) is formed by the job itself; T_com is small
     if (mapped_vals.size != table.size) throw std::runtime_error("Incompatible dimensions");
-    FrTensor* T_com = new FrTensor(table.size);
-    keep.emplace_back(T_com);
-    ZKC(zk_fr_add_mul_s(T_com->gpu_data, table.gpu_data, mapped_vals.gpu_data, r.val, T_com->size, nullptr));
-    LookupPending p = sumcheck_begin(*si, *T_com, *mm, alpha, beta, u, v, si, low, so, &r, mapped_vals.kept_ints());
+    // (an opened job's table stays with it until the proof has begun: it is being read)
+    std::unique_ptr<FrTensor> own = opened ? nullptr : combined(r);
+    const FrTensor& T_com = opened ? *opened->table : *own;
+    LookupPending p = sumcheck_begin(*si, T_com, *mm, alpha, beta, u, v, si, low, so, &r, mapped_vals.kept_ints(), opened, false, opened != nullptr);
+    keep.emplace_back(opened ? std::move(opened->table) : std::move(own));
+    if (opened) std::move(opened->keep.begin(), opened->keep.end(), std::back_inserter(keep));
     p.keep = std::move(keep);
     return p;
 }

@@ -21,6 +21,28 @@ struct LookupPending {
     vector<Fr_t> u, v;
     uint D = 0, N = 0;
 };
+// A lookup job whose table is being inverted while the caller queues the rest (zk_lookup_open).  One that was never begun is waited for and dropped.
+struct LookupOpened {
+    LookupOpened() = default;
+    LookupOpened(const LookupOpened&) = delete;
+    LookupOpened& operator=(const LookupOpened&) = delete;
+    ~LookupOpened();
+    void* handle = nullptr;
+    std::unique_ptr<FrTensor> table;      // the table it inverts, where that is made for the job
+    std::vector<std::unique_ptr<FrTensor>> keep;      // queries and multiplicities that were padded for it
+    FrTensor *queries = nullptr, *m = nullptr;
+};
+// Multiplicities that are being counted: what the range check found is asked for by settle().
+struct CountedQueries {
+    CountedQueries() = default;
+    CountedQueries(const CountedQueries&) = delete;
+    CountedQueries& operator=(const CountedQueries&) = delete;
+    ~CountedQueries();
+    void settle();                        // waits; throws if a query lies outside the table
+    std::unique_ptr<FrTensor> m;
+    std::unique_ptr<DevBuf> idx;          // the queries' positions, where they are kept
+    void* check = nullptr;
+};
 // hint / low: optionally, where each query is expected in the table (query i == T[hint[i] - low]); never changes a result
 LookupPending tLookup_sumcheck_begin(const FrTensor& S, const FrTensor& T, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
                                      const FrTensor* hint = nullptr, int low = 0);
@@ -55,6 +77,10 @@ class tLookupRange : public tLookup {
     // the queries of a range lookup are their own hints for the table position (value - low)
     Fr_t prove(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v, vector<Polynomial>& proof);
     LookupPending prove_begin(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v);
+    // addition: prep (inside: prep_inside) and prove_begin in one: the table's inverses and the rounds that read no multiplicities run beside the counting.
+    // The multiplicities go to m, which must outlive the proof.  at_once: the caller ends the proof next.
+    LookupPending count_and_prove_begin(const FrTensor& S, std::unique_ptr<FrTensor>& m, bool inside, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
+                                        bool at_once = false);
 };
 
 class tLookupRangeMapping : public tLookupRange {
@@ -78,6 +104,18 @@ class tLookupRangeMapping : public tLookupRange {
                const vector<Fr_t>& v, vector<Polynomial>& proof);
     LookupPending prove_begin(const FrTensor& S_in, const FrTensor& S_out, const FrTensor& m, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u,
                               const vector<Fr_t>& v);
+    // addition: operator() and prove_begin in one, the combined table's inverses beside the counting and the outputs, for a caller that ends the proof next
+    struct MappedPending { std::unique_ptr<FrTensor> y, m; LookupPending look; };
+    MappedPending map_and_prove_begin(const FrTensor& S_in, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v);
+
+   private:
+    void count(CountedQueries& c, const FrTensor& vals, bool positions);
+    FrTensor gather(const FrTensor& vals, const CountedQueries& c, const FrTensor* unwritten);
+    std::unique_ptr<FrTensor> combined(const Fr_t& r) const;      // table + r * mapped values
+    FrTensor* padded(std::vector<std::unique_ptr<FrTensor>>& keep, const FrTensor& t, const FrTensor& fill_from, bool ints, const void* fill_ints) const;
+    FrTensor* padded_m(std::vector<std::unique_ptr<FrTensor>>& keep, const FrTensor& m, uint D) const;
+    LookupPending prove_begin_on(const FrTensor& S_in, const FrTensor& S_out, const FrTensor& m, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
+                                 LookupOpened* opened);
 };
 
 // the sumcheck behind both prove() functions: T is the (possibly combined) table
