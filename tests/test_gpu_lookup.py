@@ -318,6 +318,29 @@ def test_range_lookup_proof_transcript(pv, orc, D, low, length):
     assert t.shape == e_t.shape and (t == e_t).all()
 
 
+# the rounds of a launch on the levels in LDS: one to eight of them, folds by the workgroup or by its first wave, a table that enters in any of them, and
+# (one) an evaluation challenge of one: no round's eq table is then the first one's prefix
+@pytest.mark.parametrize("one", [False, True])
+@pytest.mark.parametrize("D,length", [(2, 2), (8, 8), (8, 2), (64, 16), (128, 128), (256, 4), (512, 512), (1024, 8), (1 << 14, 1 << 14), (1 << 14, 1 << 9), (1 << 16, 2)])
+def test_range_lookup_proof_whose_rounds_share_launches(pv, orc, D, length, one):
+    vals = np.random.default_rng(D + length).integers(-1, length - 1, D)
+    S = fr_array([int(v) % R_MOD for v in vals])
+    k = (D - 1).bit_length()
+    alpha, beta, u, v = ch(1, 1)[0], ch(2, 1)[0], ch(3, k), ch(4, k)
+    if one:
+        u[k // 2] = fr_array([1])[0]
+    orc.orc_transcript_clear()
+    e_fin = np.zeros(8, np.uint32)
+    orc_check(orc.orc_range_prove(S, D, -1, length, alpha, beta, u, v, e_fin))
+    e_t = orc_transcript(orc)
+    pv.transcript_begin()
+    fin = pv.range_prove(pv.from_fr(S), -1, length, alpha, beta, u, v)
+    pv.lib.zkp_transcript_end()
+    assert (fin == e_fin).all()
+    t = pv.transcript()
+    assert t.shape == e_t.shape and (t == e_t).all()
+
+
 @pytest.mark.parametrize("D,low,length", [(6, -2, 4), (64, -8, 16), (1000, -16, 32), (1 << 17, -16, 32)])
 def test_mapping_lookup(pv, orc, D, low, length):
     rng = np.random.default_rng(D)

@@ -104,21 +104,49 @@ struct FinishRounds {
     uint32_t extra_nb, slot;             // slot: where they go, in elements
 };
 struct PartSlice { Fr* p; template <class T> T* as() const { return reinterpret_cast<T*>(p); } };      // a round's share of the partial sums
-__global__ void __launch_bounds__(TPB) k_finish_rounds(Fr* __restrict__ sums, const Fr* __restrict__ part, const FinishRounds fr, uint32_t per_round) {
-    const uint32_t r = blockIdx.y, t = threadIdx.x;
-    const bool behind = r + 1 == gridDim.y;
-    if (behind ? blockIdx.x != 0 : blockIdx.x >= fr.k[r]) return;
+// sum k of round r (behind: what stands behind the rounds' sums), on the first TPB lanes of a workgroup of T; every lane calls it
+template <int T> __device__ __forceinline__ void finish_sum(Fr* __restrict__ sums, const Fr* __restrict__ part, const FinishRounds& fr, uint32_t per_round, uint32_t r, uint32_t k, bool behind, uint32_t t) {
+    if (behind ? k != 0 : k >= fr.k[r]) return;
     if (behind) {
         if (fr.v0 && t < 16) (&sums[fr.slot].v[0])[t] = t < 8 ? fr.v0->v[t] : fr.v1->v[t - 8];
         if (fr.word && t == 0) sums[fr.slot + (fr.v0 ? 2 : 1)].v[0] = *fr.word;
         if (!fr.extra) return;
     }
-    Fr acc[1] = {big_zero<8>()};
-    const uint32_t nb = behind ? fr.extra_nb : fr.nb[r];
-    const Fr* p = behind ? fr.extra : part + fr.off[r] + (size_t)blockIdx.x * nb;
-    for (uint32_t i = t; i < nb; i += TPB) acc[0] = add(acc[0], p[i]);
-    // (block_reduce_store: sum 0 of workgroup blockIdx.x to partials[blockIdx.x])
-    block_reduce_store<1>(acc, sums + (behind ? (size_t)fr.slot : (size_t)r * per_round));
+    constexpr int W = TPB / 64;
+    __shared__ uint32_t red[W][9];
+    if (T == TPB || t < (uint32_t)TPB) {
+        Fr acc = big_zero<8>();
+        const uint32_t nb = behind ? fr.extra_nb : fr.nb[r];
+        const Fr* p = behind ? fr.extra : part + fr.off[r] + (size_t)k * nb;
+        for (uint32_t i = t; i < nb; i += TPB) acc = add(acc, p[i]);
+        const Fr29 x = fr29_repack(acc);
+        uint32_t l[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) l[i] = (uint32_t)x.l[i];
+        fr29_wave_sum(l);
+        if ((t & 63u) == 63u) {
+#pragma unroll
+            for (int i = 0; i < 9; ++i) red[t >> 6][i] = l[i];
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        uint32_t l[9];
+#pragma unroll
+        for (int i = 0; i < 9; ++i) {
+            l[i] = red[0][i];
+#pragma unroll
+            for (int w = 1; w < W; ++w) l[i] += red[w][i];
+        }
+        fr29_carry_u(l);
+        Fr29 x;
+#pragma unroll
+        for (int i = 0; i < 9; ++i) x.l[i] = (int32_t)l[i];
+        sums[behind ? (size_t)fr.slot : (size_t)r * per_round + k] = fr29_canon_pack<5>(fr29_mul(x, fr29_2_261()));      // up to 256 r: as block_reduce_store
+    }
+}
+__global__ void __launch_bounds__(TPB) k_finish_rounds(Fr* __restrict__ sums, const Fr* __restrict__ part, const FinishRounds fr, uint32_t per_round) {
+    finish_sum<TPB>(sums, part, fr, per_round, blockIdx.y, blockIdx.x, blockIdx.y + 1 == gridDim.y, threadIdx.x);
 }
 static inline unsigned reduce_grid(size_t n) {
     size_t b = (n + TPB - 1) / TPB;
@@ -1379,11 +1407,10 @@ template <int K> __device__ __forceinline__ void tail_block_sum(Fr (&acc)[K], Fr
 //   wave 1: E b0 t0 | E b1 t1 | E db dt                               (phase 2)
 //   wave 2: folds of A | S | B | T, and the sums of a0 | a1
 //   wave 3: m0 b0 | m1 b1 | dm db | fold of m                         (phase 2)
-// and the sixteen waves of the workgroup take 64 pairs at a time; a round of fewer leaves the waves of the others out.  The middle
-// coefficients (da s0 + a0 ds and the like) are a1 s1 - a0 s0 - da ds.
-// What binds: instruction issue of the sixteen waves on one compute unit while a round has 64 pairs, the chain of two products
-// below.  These rounds took 17 us each in a workgroup that gave a pair's products to four lanes, 14 us each as launches.
-static constexpr int RM_ROUNDS = 8, RM_P = 1 << RM_ROUNDS, RM_W = 12, RM_ROWS = 16, RM_GROUPS = 4, RM_WIDE_ROUNDS = 3;      // RM_W: words of an element in LDS (rows of sixteen read without conflicts)
+// The middle coefficients (da s0 + a0 ds and the like) are a1 s1 - a0 s0 - da ds.
+// k_sum_rounds: launches of more workgroups than compute units, three rounds of 64 elements in a workgroup of four waves.  What binds is instruction issue (67 %
+// of the slots at 2^17 elements, 41 us; as three launches of k_lookup_round29 and a batch behind them 14 + 38 us).  k_level_rounds: the rest.
+static constexpr int RM_ROUNDS = 8, RM_P = 1 << RM_ROUNDS, RM_W = 12, RM_ROWS = 16, RM_WIDE_P = RM_P / 4, RM_WIDE_ROUNDS = 3;      // RM_W: words of an element in LDS (rows of sixteen read without conflicts)
 static constexpr size_t RM_MAX_N = (size_t)1 << 17;      // elements from which on a sumcheck's rounds run in such launches
 struct RoundsArgs {
     const Fr *A, *S, *B, *T, *m, *E;
@@ -1394,13 +1421,13 @@ struct RoundsArgs {
     uint32_t fold_e, e_span;              // fold_e: E is this round's table alone and is summed down from round to round; e_span: its first round's is E[t] + E[t + e_span]
     uint32_t off[RM_ROUNDS];              // where round r's partial sums start
 };
-template <bool PHASE2, int GROUPS> __global__ void __launch_bounds__(256 * GROUPS)
+template <bool PHASE2> __global__ void __launch_bounds__(256)
 k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
-    constexpr int NT = PHASE2 ? 5 : 2, PM = RM_P / RM_GROUPS * GROUPS, MAXR = GROUPS == RM_GROUPS ? RM_ROUNDS : RM_WIDE_ROUNDS;
+    constexpr int NT = PHASE2 ? 5 : 2, PM = RM_WIDE_P, MAXR = RM_WIDE_ROUNDS;
     __shared__ int32_t X0[NT][PM][RM_W], X1[NT][PM / 2][RM_W], XE[PM / 2][RM_W];
-    __shared__ uint32_t raw[MAXR][GROUPS][RM_ROWS][9];
-    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave & 3u, group = wave >> 2;
-    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u, T = 256u * GROUPS;
+    __shared__ uint32_t raw[MAXR][RM_ROWS][9];
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), kind = wave;
+    const uint32_t row = (threadIdx.x >> 4) & 3u, ln = threadIdx.x & 15u, T = 256u;
     const uint32_t nb = gridDim.x, c = 1u << a.log_c;
     // neighbouring workgroups read neighbouring elements of the same lines: keep them on one die (workgroups go to the eight dies in turn)
     const uint32_t blk = (nb & 7u) == 0 ? (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
@@ -1422,7 +1449,7 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
             if (a.e_span) e = add(e, a.E[g + a.e_span]);
             rm_put(XE[s], fr29_repack(e));
         }
-        for (uint32_t i = threadIdx.x; i < MAXR * GROUPS * RM_ROWS * 9; i += T) (&raw[0][0][0][0])[i] = 0u;
+        for (uint32_t i = threadIdx.x; i < MAXR * RM_ROWS * 9; i += T) (&raw[0][0][0])[i] = 0u;
     }
     __syncthreads();
     for (uint32_t r = 0; r < a.rounds; ++r) {
@@ -1432,11 +1459,11 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
         int32_t* const dst = odd ? &X0[0][0][0] : &X1[0][0][0];
         const uint32_t ss = (odd ? PM / 2 : PM) * RM_W, ds = (odd ? PM : PM / 2) * RM_W;
         auto rd = [&](uint32_t k, uint32_t slot) { return rm_get(src + k * ss + slot * RM_W); };
-        if (group * 16u < half && (phase2 || !(kind & 1u))) {
+        if (phase2 || !(kind & 1u)) {
             uint32_t acc[9];
 #pragma unroll
             for (int l = 0; l < 9; ++l) acc[l] = 0;
-            for (uint32_t t0 = group * 16u; t0 < half; t0 += 16u * GROUPS) {
+            for (uint32_t t0 = 0; t0 < half; t0 += 16u) {
                 const uint32_t t = t0 + ln;
                 const bool live = t < half;
                 const uint32_t ta = live ? t : 0u, tb = ta + half;
@@ -1467,7 +1494,7 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
             fr29_row_sum(acc);
             if (ln == 15) {
 #pragma unroll
-                for (int l = 0; l < 9; ++l) raw[r][group][kind * 4u + row][l] = acc[l];
+                for (int l = 0; l < 9; ++l) raw[r][kind * 4u + row][l] = acc[l];
             }
         }
         __syncthreads();
@@ -1488,11 +1515,7 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
         const uint32_t role = k < 3 ? k : (k < 5 ? 5u + k : (k < 8 ? k - 1u : 4u + k));
         uint32_t l9[9];
 #pragma unroll
-        for (int l = 0; l < 9; ++l) {
-            l9[l] = raw[r][0][role][l];
-#pragma unroll
-            for (int g = 1; g < GROUPS; ++g) l9[l] += raw[r][g][role][l];
-        }
+        for (int l = 0; l < 9; ++l) l9[l] = raw[r][role][l];
         fr29_carry_u(l9);
         Fr29 x;
 #pragma unroll
@@ -1527,6 +1550,176 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
         }
         if (a.fold_e)
             for (uint32_t s = threadIdx.x; s < c; s += T) a.nE[low0 + s] = fr29_pack(rm_get(XE[s]));
+    }
+}
+
+// The same for launches that have a compute unit for each of their workgroups (n <= 2^16): what takes the time there is a round's chain and the issue
+// of one compute unit.  A workgroup has two of the tensors (blockIdx.y: A, S | B, T | m, B, so that three compute units share a block of elements) and keeps
+// every round's level of them in LDS, and the folds run ahead of the sums: the large ones on all lanes with a barrier each, those of at
+// most 32 pairs on the first wave alone, without one, while the others take the sums of the rounds in front.  A fold is one product deep where a round with its sums was two and a
+// barrier.  A unit of work is sixteen pairs of a round: rows of sixteen lanes for x0 y0 | x1 y1 | dx dy (times E), the fourth row for the sums of a0 and a1.
+// The last launch, of one block, also does what k_finish_rounds does for the rounds ahead of it, a workgroup a sum beside its own, and its own sums go straight to
+// where the host reads them.  Seven rounds from 2^14 elements: 17.4 us, from 2^7: 14.6 us (30.6 and 20.6 with all five tensors in one workgroup of sixteen waves and every round's sums ahead of the next round).
+static constexpr int LV_T = 512, LV_UNITS = RM_P / 32 + RM_P / 64 + RM_P / 128 + RM_ROUNDS;      // units: 8, 4, 2, 1, 1, ...
+__device__ __forceinline__ uint32_t lv_units(uint32_t half) { return (half + 15u) / 16u; }
+// sums null: the partial sums go to memory.  rows_from: the first of the workgroups (blockIdx.y) that finish the `before` rounds of fin
+struct FinishHere { FinishRounds fin; Fr* sums; uint32_t per_round, before, rows_from; };
+__global__ void __launch_bounds__(LV_T) k_level_rounds(Fr* __restrict__ partials, const RoundsArgs a, const FinishHere fh) {
+    __shared__ int32_t X[2][2 * RM_P][RM_W], XE[RM_P][RM_W];
+    __shared__ uint32_t raw[LV_UNITS][5][9], res[RM_ROUNDS * 5][8];
+    if (fh.sums && blockIdx.y >= fh.rows_from) {
+        const uint32_t q = blockIdx.y - fh.rows_from, t = threadIdx.x;
+        finish_sum<LV_T>(fh.sums, partials, fh.fin, fh.per_round, q / fh.per_round, q % fh.per_round, q / fh.per_round == fh.before, t);
+        return;
+    }
+    const uint32_t tid = threadIdx.x, wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6)), lane = tid & 63u, row = (tid >> 4) & 3u, ln = tid & 15u;
+    const uint32_t which = blockIdx.y, nb = gridDim.x, c = 1u << a.log_c;
+    const uint32_t blk = (nb & 7u) == 0 ? (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;      // as in k_sum_rounds
+    const uint32_t low0 = blk << a.log_c;
+    const uint32_t r0 = which ? a.phase2_from : 0u, R = a.rounds - r0, P = c << R;      // these tensors' rounds and elements
+    const Fr* const src0 = which == 0 ? a.A : (which == 1 ? a.B : a.m);
+    const Fr* const src1 = which == 0 ? a.S : (which == 1 ? a.T : a.B);
+    auto level = [&](uint32_t r) { return 2u * P - ((2u * P) >> r); };                  // where round r's elements start
+    auto elevel = [&](uint32_t r) { return a.fold_e ? P - (P >> r) : 0u; };             // and its eq weights
+    auto global = [&](uint32_t s) { return (size_t)(s >> a.log_c) * a.nlow + low0 + (s & (c - 1)); };
+    for (uint32_t i = tid; i < 2u * P; i += LV_T) {
+        const uint32_t s = i < P ? i : i - P;
+        rm_put(X[i < P ? 0 : 1][s], fr29_repack((i < P ? src0 : src1)[global(s)]));
+    }
+    if (which < 2) {
+        // E's table of this launch's first round; of a later one it is summed down
+        const uint32_t n_e = a.fold_e ? (c << a.rounds) / 2u : P / 2u;
+        if (!a.fold_e || r0 == 0) {
+            for (uint32_t s = tid; s < n_e; s += LV_T) {
+                const size_t g = global(s);
+                Fr e = a.E[g];
+                if (a.e_span) e = add(e, a.E[g + a.e_span]);
+                rm_put(XE[s], fr29_repack(e));
+            }
+        } else {          // summed down to round r0 by each lane on its own
+            for (uint32_t s = tid; s < P / 2u; s += LV_T) {
+                Fr e = big_zero<8>();
+                for (uint32_t q = 0; q < (1u << r0); ++q) {
+                    const size_t g = global(s + q * (P / 2u));
+                    e = add(e, a.E[g]);
+                    if (a.e_span) e = add(e, a.E[g + a.e_span]);
+                }
+                rm_put(XE[s], fr29_repack(e));
+            }
+        }
+    }
+    __syncthreads();
+    if (a.fold_e && which < 2)
+        for (uint32_t r = 0; r + 1 < R; ++r) {
+            const uint32_t half = P >> (r + 2);
+            for (uint32_t s = tid; s < half; s += LV_T) rm_put(XE[elevel(r + 1) + s], fr29_canon<1>(fr29_add(rm_get(XE[elevel(r) + s]), rm_get(XE[elevel(r) + half + s]))));
+            __syncthreads();
+        }
+    auto fold = [&](uint32_t r, uint32_t k, uint32_t t) {
+        const uint32_t half = P >> (r + 1), at = level(r) + t;
+        const Fr29 x0 = rm_get(X[k][at]), x1 = rm_get(X[k][at + half]);
+        rm_put(X[k][level(r + 1) + t], fr29_canon<2>(fr29_add(x0, fr29_mul(a.v[r0 + r], fr29_sub_plus_r(x1, x0)))));
+    };
+    uint32_t first = 0, done = 0;                           // rounds whose fold the whole workgroup makes; units of the rounds up to there
+    for (; first < R && (P >> (first + 1)) > 32u; ++first) {
+        const uint32_t half = P >> (first + 1);
+        for (uint32_t i = tid; i < 2u * half; i += LV_T) fold(first, i < half ? 0u : 1u, i < half ? i : i - half);
+        __syncthreads();
+    }
+    auto unit = [&](uint32_t u) {                           // the u-th sixteen pairs of all rounds: every lane of a wave
+        uint32_t r = 0, b = u;
+        while (b >= lv_units(P >> (r + 1))) { b -= lv_units(P >> (r + 1)); ++r; }
+        const uint32_t half = P >> (r + 1), t = b * 16u + ln, at = level(r) + (t < half ? t : 0u);
+        const Fr29 x0 = rm_get(X[0][at]), x1 = rm_get(X[0][at + half]), y0 = rm_get(X[1][at]), y1 = rm_get(X[1][at + half]);
+        Fr29 x = fr29_select(row == 0, x0, fr29_select(row == 1, x1, fr29_sub_plus_r(x1, x0)));
+        Fr29 y = fr29_select(row == 0, y0, fr29_select(row == 1, y1, fr29_sub_plus_r(y1, y0)));
+        if (which < 2) y = fr29_select(row < 2, fr29_add(y, a.beta), y);
+        x = fr29_mul(x, y);
+        if (which < 2) x = fr29_mul(rm_get(XE[elevel(r) + (t < half ? t : 0u)]), x);
+        uint32_t acc[9];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) acc[l] = t < half ? (uint32_t)(row == 3 ? x0.l[l] : x.l[l]) : 0u;
+        fr29_row_sum(acc);
+        if (ln == 15) {
+#pragma unroll
+            for (int l = 0; l < 9; ++l) raw[u][row][l] = acc[l];
+        }
+        if (which == 0 && !a.hadamard) {
+#pragma unroll
+            for (int l = 0; l < 9; ++l) acc[l] = t < half ? (uint32_t)x1.l[l] : 0u;
+            fr29_row_sum(acc);
+            if (lane == 63u) {
+#pragma unroll
+                for (int l = 0; l < 9; ++l) raw[u][4][l] = acc[l];
+            }
+        }
+    };
+    uint32_t units = 0;
+    for (uint32_t r = 0; r < R; ++r) {
+        units += lv_units(P >> (r + 1));
+        if (r <= first) done = units;
+    }
+    if (wave == 0) {
+        for (uint32_t r = first; r < R; ++r) {
+            const uint32_t half = P >> (r + 1), k = lane >> 5, t = lane & 31u;
+            if (t < half) fold(r, k, t);
+            // the wave's own LDS operations are in order: only the compiler must keep them so
+            asm volatile("" ::: "memory");
+        }
+    } else {
+        for (uint32_t u = wave - 1u; u < done; u += LV_T / 64 - 1) unit(u);
+    }
+    __syncthreads();
+    for (uint32_t u = done + wave; u < units; u += LV_T / 64) unit(u);
+    __syncthreads();
+    // The sums' residues, with the factors that k_sum_rounds explains
+    const uint32_t per = which == 0 && !a.hadamard ? 5u : 3u;
+    for (uint32_t i = tid; i < per * R; i += LV_T) {
+        const uint32_t r = i / per, k = i % per, rl = k;      // x0 y0, x1 y1 (to be made the middle coefficient), dx dy; a0, a1
+        uint32_t u0 = 0;
+        for (uint32_t q = 0; q < r; ++q) u0 += lv_units(P >> (q + 1));
+        uint32_t l9[9];
+#pragma unroll
+        for (int l = 0; l < 9; ++l) l9[l] = 0;
+        for (uint32_t u = u0; u < u0 + lv_units(P >> (r + 1)); ++u) {
+#pragma unroll
+            for (int l = 0; l < 9; ++l) l9[l] += raw[u][rl][l];
+        }
+        fr29_carry_u(l9);
+        Fr29 x;
+#pragma unroll
+        for (int l = 0; l < 9; ++l) x.l[l] = (int32_t)l9[l];
+        const Fr29 fix = fr29_select(k >= 3, fr29_2_261(), fr29_select(which == 2, fr29_2_266(), fr29_select(a.hadamard != 0, fr29_2_527(), fr29_2_271())));
+        const Fr o = fr29_canon_pack<3>(fr29_mul(x, fix));
+#pragma unroll
+        for (int l = 0; l < 8; ++l) res[i][l] = o.v[l];
+    }
+    __syncthreads();
+    for (uint32_t i = tid; i < per * R; i += LV_T) {
+        const uint32_t r = i / per, k = i % per;
+        auto at = [&](uint32_t q) {
+            Fr x;
+#pragma unroll
+            for (int l = 0; l < 8; ++l) x.v[l] = res[q][l];
+            return x;
+        };
+        Fr o = at(i);
+        if (k == 1) o = sub(sub(o, at(i - 1)), at(i + 1));
+        else if (k == 4) o = sub(o, at(i - 1));
+        const uint32_t at_k = which == 0 ? k : 2u + 3u * which + k;
+        if (fh.sums) fh.sums[(size_t)(fh.before + r0 + r) * fh.per_round + at_k] = o;
+        else partials[(size_t)a.off[r0 + r] + (size_t)at_k * nb + blockIdx.x] = o;
+    }
+    if (a.nA) {
+        Fr* const d0 = which == 0 ? a.nA : (which == 1 ? a.nB : a.nm);
+        Fr* const d1 = which == 0 ? a.nS : (which == 1 ? a.nT : nullptr);
+        for (uint32_t i = tid; i < 2u * c; i += LV_T) {
+            const uint32_t k = i >> a.log_c, s = i & (c - 1);
+            Fr* const d = k ? d1 : d0;
+            if (d) d[low0 + s] = fr29_pack(rm_get(X[k][level(R) + s]));
+        }
+        if (a.fold_e && which == 0)
+            for (uint32_t s = tid; s < c; s += LV_T) a.nE[low0 + s] = fr29_pack(rm_get(XE[elevel(R - 1) + s]));
     }
 }
 
@@ -2804,9 +2997,10 @@ static bool limbs29() { static const bool on = [] { const char* e = getenv("ZKLL
 // A == nullptr with a hint source: 1 / (S + beta) has not been written anywhere; a large first round computes it on
 // the fly, anything else writes it out first.
 // Queues rounds r .. rounds - 1 of a sumcheck over n elements in launches of k_sum_rounds.  hadamard: two tensors A, S; else a lookup whose
-// phase-2 rounds start at round n1.  The rounds' partial sums go behind part_at and are noted in `fin`; eq_prefix: every round reads E's prefix.
+// phase-2 rounds start at round n1.  The rounds' partial sums go behind part_at and are noted in `fin`; finished: the last launch did what k_finish_rounds does.
+// eq_prefix: every round reads E's prefix.
 static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& beta, const uint32_t* v, size_t n, int r,
-                        int rounds, int n1, bool eq_prefix, Fr* part_all, size_t& part_at, FinishRounds& fin) {
+                        int rounds, int n1, bool eq_prefix, Fr* part_all, size_t& part_at, FinishRounds& fin, bool& finished) {
     const uint32_t per1 = hadamard ? 3u : 5u;
     uint32_t e_span = 0;
     while (r < rounds) {
@@ -2814,7 +3008,7 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
         // a full one: three rounds then; all that the workgroup's elements allow, evenly split over the launches, where each has a unit
         // of its own.
         const int left = rounds - r;
-        int R = std::min(RM_WIDE_ROUNDS, left), P = RM_P / RM_GROUPS;
+        int R = std::min(RM_WIDE_ROUNDS, left), P = RM_WIDE_P;
         if (n <= (size_t)256 * RM_P) {
             P = RM_P;
             const int launches = (left + RM_ROUNDS - 1) / RM_ROUNDS;
@@ -2851,11 +3045,22 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
             a.nA = nx.as<Fr>(); a.nS = a.nA + o; a.nB = a.nS + o; a.nT = a.nB + o; a.nm = a.nT + o; a.nE = a.nm + o;
         }
         if (P < RM_P) {
-            if (phase2) hipLaunchKernelGGL((k_sum_rounds<true, 1>), dim3(nb), dim3(256), 0, job.st, part_all, a);
-            else hipLaunchKernelGGL((k_sum_rounds<false, 1>), dim3(nb), dim3(256), 0, job.st, part_all, a);
+            if (phase2) hipLaunchKernelGGL((k_sum_rounds<true>), dim3(nb), dim3(256), 0, job.st, part_all, a);
+            else hipLaunchKernelGGL((k_sum_rounds<false>), dim3(nb), dim3(256), 0, job.st, part_all, a);
         } else {
-            if (phase2) hipLaunchKernelGGL((k_sum_rounds<true, RM_GROUPS>), dim3(nb), dim3(256 * RM_GROUPS), 0, job.st, part_all, a);
-            else hipLaunchKernelGGL((k_sum_rounds<false, RM_GROUPS>), dim3(nb), dim3(256 * RM_GROUPS), 0, job.st, part_all, a);
+            FinishHere fh;
+            memset(&fh, 0, sizeof(fh));
+            uint32_t ny = phase2 ? 3u : 1u;
+            if (r + R == rounds && nb == 1) {
+                fh.fin = fin;
+                fh.sums = job.sums;
+                fh.per_round = (uint32_t)job.per_round;
+                fh.before = (uint32_t)r;
+                fh.rows_from = ny;
+                ny += fh.per_round * (uint32_t)r + 1u;
+                finished = true;
+            }
+            hipLaunchKernelGGL(k_level_rounds, dim3(nb, ny), dim3(LV_T), 0, job.st, part_all, a, fh);
         }
         ZK_LAUNCH_CHECK();
         A = a.nA; S = a.nS;
@@ -2867,7 +3072,7 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
     return 0;
 }
 // partial sums that rounds_queue may need for the rounds of n elements: a workgroup holds 32 pairs of a launch's first round where there are as many
-static size_t rounds_partials(size_t n, int rounds, uint32_t k) { return (size_t)rounds * k * (n / (RM_P / RM_GROUPS) + 1); }
+static size_t rounds_partials(size_t n, int rounds, uint32_t k) { return (size_t)rounds * k * (n / RM_WIDE_P + 1); }
 static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& b, const uint32_t* v, size_t D, size_t N, int rounds,
                         const HintSrc* hs = nullptr) {
     hipStream_t st = job.st;
@@ -2913,6 +3118,7 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
     FinishRounds& fin = job.fin;
     size_t part_at = 0;
     int fin_rounds = 0;              // rounds whose sums come from partials (the rest: the tail kernel's)
+    bool finished = false;
     PartSlice part{nullptr};
     const bool eq_prefix = job.eq_prefix;      // every round reads the first table's prefix
     const Fr *cA = A, *cS = S, *cB = B, *cT = T, *cm = m, *cE = E;
@@ -2923,9 +3129,9 @@ static int lookup_queue(SumJob& job, const Fr* A, const Fr* S, const Fr* B, cons
         const bool phase2 = r >= n1;
         part.p = part_all.as<Fr>() + part_at;
         if (cA && cur <= RM_MAX_N) {
-            int rc = rounds_queue(job, false, cA, cS, cB, cT, cm, cE, b, v, cur, r, rounds, n1, eq_prefix, part_all.as<Fr>(), part_at, fin);
+            int rc = rounds_queue(job, false, cA, cS, cB, cT, cm, cE, b, v, cur, r, rounds, n1, eq_prefix, part_all.as<Fr>(), part_at, fin, finished);
             if (rc) return rc;
-            fin_rounds = rounds;
+            fin_rounds = finished ? 0 : rounds;
             break;
         }
         if (r == 0 && !phase2 && fuse_first && (hs->hint_ints || hs->fr_queries) && limbs29() && two_rounds_on() && n1 >= 2 && rounds >= 2 && (half >> 1) > (size_t)SPLIT_HALF &&
@@ -3091,6 +3297,7 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
     FinishRounds& fin = job.fin;
     size_t part_at = 0;
     int fin_rounds = 0;
+    bool finished = false;
     PartSlice part{nullptr};
     const Fr* cur[4];
     for (int i = 0; i < K; ++i) cur[i] = Xs[i];
@@ -3102,9 +3309,9 @@ static int hadamard_queue(SumJob& job, const Fr* const* Xs, int K, const Fr* E, 
         part.p = part_all.as<Fr>() + part_at;
         // two tensors: all short rounds in a few launches (a first round over int32 forms is a round of its own)
         if (K == 2 && n <= RM_MAX_N && !(r == 0 && ints && ints[0] && ints[1] && half > (size_t)TAIL_HALF)) {
-            int rc = rounds_queue(job, true, cur[0], cur[1], nullptr, nullptr, nullptr, cE, big_zero<8>(), v, n, r, rounds, 0, job.eq_prefix, part_all.as<Fr>(), part_at, fin);
+            int rc = rounds_queue(job, true, cur[0], cur[1], nullptr, nullptr, nullptr, cE, big_zero<8>(), v, n, r, rounds, 0, job.eq_prefix, part_all.as<Fr>(), part_at, fin, finished);
             if (rc) return rc;
-            fin_rounds = rounds;
+            fin_rounds = finished ? 0 : rounds;
             break;
         }
         if (half <= (size_t)TAIL_HALF && rounds - r <= TAIL_ROUNDS) {
