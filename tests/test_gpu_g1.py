@@ -182,6 +182,22 @@ def test_commit_int_tables_of_every_shape_match_the_oracle(pv, orc, m, n, lim):
     assert (norm(orc, pv.commit_int(pv.g1_from_host(gens), pv.from_fr(T)).host()) == norm(orc, exp)).all()
 
 
+@pytest.mark.parametrize("m,n,lim", [(3000, 40, 4000), (4, 2048, 700), (2, 8192, 2 ** 30), (300, 7, 2 ** 20)])
+def test_commit_int_of_generators_of_small_order_matches_the_oracle(pv, orc, m, n, lim):
+    """(0, 2) has order 3: every pair of entries of its windows that k_msm_table_grow adds and subtracts is equal, opposite or holds infinity."""
+    gens = oracle_gens(orc, 70 + n, n)
+    for i, p in ((1, (0, 2)), (3, (0, P_MOD - 2)), (n - 2, (0, 2))):
+        gens[i] = affine_to_jac(p)
+    rng = np.random.default_rng(m + n)
+    t = rng.integers(-lim, lim, (m, n), endpoint=True).astype(np.int64)
+    t[0] = 0
+    t[0, 1], t[1, 1], t[2 % m, 3] = 2, lim, -lim
+    T = fr_array([int(x) % R_MOD for x in t.reshape(-1)])
+    exp = np.zeros((m, 36), np.uint32)
+    orc_check(orc.orc_commit_int(gens, n, T, m * n, exp))
+    assert (norm(orc, pv.commit_int(pv.g1_from_host(gens), pv.from_fr(T)).host()) == norm(orc, exp)).all()
+
+
 @pytest.mark.parametrize("bad", [2 ** 31, R_MOD - 2 ** 31 - 1, 2 ** 32, 2 ** 64, R_MOD - 2 ** 64, 1 << 224, (R_MOD >> 64) << 64, R_MOD - (1 << 224)])
 def test_commit_int_refuses_what_is_no_int32(pv, orc, bad):
     gens = pv.g1_from_host(oracle_gens(orc, 14, 8))

@@ -12,6 +12,7 @@
 // All of it is VALU integer work on 12-limb Fp; results equal the reference's as group elements
 // (a Jacobian triple depends on the order of additions, so bytes are compared after normalising).
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -208,12 +209,23 @@ __device__ __forceinline__ size_t msm_slot(const MsmTable& T, uint32_t w, size_t
     return (size_t)w * T.ngen * T.half + j * (last ? T.top : T.half) + (d - 1);
 }
 __device__ __forceinline__ Fq29 fq29_inverse(const Fq29& v) { return fq29_from_fp(mont_inverse(fq29_to_fp(v))); }
-// The first 2^logs entries of every window (those that it has) out of the normalised bases (window-major), a lane an entry: doublings and additions
-// of the base along the bits of the multiple, and an inversion.  A level of k_msm_table_grow takes what one lane's inversion and
-// its launch take however few its entries are: the first four of 8192 rows took 252 us, so they take 170.
-__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_first(const MsmTable T, const G1Affine* __restrict__ bases, uint32_t logs) {
-    const size_t i = (size_t)blockIdx.x * GT + threadIdx.x, r = i >> logs, rows_full = (size_t)(T.nwin - 1) * T.ngen;
-    const uint32_t d = (uint32_t)(i & ((1u << logs) - 1u)) + 1u;
+// How the entries of a window grow from h to t: entries c + i and c - i out of entry c, the centre, and entry i <= h, which share the slope's denominator
+// x_c - x_i.  With c halfway between h and t <= 3 h that is every entry above h but the centre itself; np: pairs.
+struct GrowSpec { uint32_t h, c, t, np; };
+static constexpr int GROW_MAX = 12;
+struct GrowCentres { uint32_t full_n, top_n; uint16_t full[GROW_MAX], top[GROW_MAX]; };
+// The first entries of every window (those that it has) and the centres of its growth out of the normalised bases (window-major), a lane an entry: doublings and additions
+// of the base along the bits of the multiple, and an inversion.  A step of k_msm_table_grow takes what one lane's inversion and
+// its launch take however few its entries are: the first sixteen of 8192 rows took 330 us in four steps that doubled them, and take 170 here.
+// The centres come first: a wave of them, all of one multiple, takes longest.
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_first(const MsmTable T, const G1Affine* __restrict__ bases, uint32_t first, const GrowCentres gc) {
+    const size_t rows_full = (size_t)(T.nwin - 1) * T.ngen, n_full = rows_full * gc.full_n, n_centres = n_full + T.ngen * gc.top_n;
+    const size_t i = (size_t)blockIdx.x * GT + threadIdx.x;
+    size_t r;
+    uint32_t d;
+    if (i < n_full) { r = i % rows_full; d = gc.full[i / rows_full]; }
+    else if (i < n_centres) { r = rows_full + (i - n_full) % T.ngen; d = gc.top[(i - n_full) / T.ngen]; }
+    else { r = (i - n_centres) / first; d = (uint32_t)((i - n_centres) % first) + 1u; }
     const bool full = r < rows_full;
     if (r >= T.ngen * T.nwin || d > (full ? T.half : T.top)) return;
     const A29 base = a29_from_affine(bases[r]);
@@ -232,60 +244,82 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     (full ? T.tab + r * T.half : T.tab + rows_full * T.half + (r - rows_full) * T.top)[d - 1u] = out;
 }
-// Entries k + 1 .. 2 k of every window that has them, entry k + i = entry i + entry k: affine additions, whose slopes share an inversion
-// among a lane's entries (an inversion costs a lane about 26 products, the rest of an entry seven).  The entry of the
-// same multiple is a doubling; infinity and opposite points are told apart from the coordinates, whatever the generators are.
-// The products before an entry wait in its slot.
-__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_grow(const MsmTable T, uint32_t logk, size_t rows_full, size_t rows, uint32_t per_lane) {
-    const uint32_t k = 1u << logk;
-    const size_t n = rows << logk, base = (size_t)blockIdx.x * GT * per_lane + threadIdx.x;
+// A step of the windows' growth (GrowSpec: of the full windows, and of the highest): a lane's pairs share one inversion (about 26 products), and a pair takes nine products for its two entries
+// and 280 bytes an entry.  Equal and opposite points and infinity are told apart from the coordinates, whatever the generators are.
+// The products before a pair wait in the slot of one of its entries.  Entry by entry, each with a denominator of its own and the windows doubled from launch to launch, 8.4 M entries took 2.0 ms
+// at 56 % of the issue slots (526 bytes an entry); three entries for one
+// from launch to launch this way they take 1.32 ms at 58 % (11008 x 4096 of 13 bits; the whole commitment 10.68 -> 10.18 ms).  Sending for the next pair's points early spills and gains nothing.
+__global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_grow(const MsmTable T, const GrowSpec full, const GrowSpec top, uint32_t n, uint32_t per_lane) {
+    const uint32_t base = blockIdx.x * GT * per_lane + threadIdx.x;
     if (base >= n) return;
-    auto row_of = [&](size_t t) {
-        const size_t r = t >> logk;
-        return r < rows_full ? T.tab + r * T.half : T.tab + rows_full * T.half + (r - rows_full) * T.top;
+    const size_t rows_full = (size_t)(T.nwin - 1) * T.ngen;
+    const uint32_t n_full = (uint32_t)rows_full * full.np;
+    struct At { A29* row; uint32_t i, c, h, t; };
+    auto at = [&](uint32_t q) {
+        if (q < n_full) return At{T.tab + (size_t)(q / full.np) * T.half, q % full.np + 1u, full.c, full.h, full.t};
+        q -= n_full;
+        return At{T.tab + rows_full * T.half + (size_t)(q / top.np) * T.top, q % top.np + 1u, top.c, top.h, top.t};
     };
-    // 0: slope over dx, 1: doubling, 2: a (b is infinity), 3: b, 4: infinity
+    // 0: slopes over dx; 1: equal points (their sum is a doubling, their difference infinity); 2: opposite ones; 3: the centre is infinity; 4: entry i is; 5: both results are infinity
     auto kind_of = [&](const A29& a, const A29& b, Fq29& den) {
         den = fq29_one();
-        if (a29_is_inf(a)) return 3u;
-        if (a29_is_inf(b)) return 2u;
+        if (a29_is_inf(a)) return 4u;
+        if (a29_is_inf(b)) return 3u;
         const Fq29 dx = fq29_sub(a.x, b.x);
         if (!fq29_is_zero_mod_p(dx)) { den = dx; return 0u; }
-        const Fq29 y2 = fq29_dbl(a.y);
-        if (!fq29_is_zero_mod_p(fq29_sub(a.y, b.y)) || fq29_is_zero_mod_p(y2)) return 4u;
+        const Fq29 y2 = fq29_dbl(b.y);
+        if (fq29_is_zero_mod_p(y2)) return 5u;
         den = y2;
-        return 1u;
+        return fq29_is_zero_mod_p(fq29_sub(a.y, b.y)) ? 1u : 2u;
     };
     Fq29 run = fq29_one();
     uint32_t count = 0;
-    for (size_t t = base; count < per_lane && t < n; t += GT, ++count) {
-        A29* row = row_of(t);
+    for (uint32_t q = base; count < per_lane && q < n; q += GT, ++count) {
+        const At p = at(q);
         Fq29 den;
-        (void)kind_of(row[t & (k - 1)], row[k - 1], den);
-        row[k + (t & (k - 1))].x = run;
+        (void)kind_of(p.row[p.i - 1], p.row[p.c - 1], den);
+        p.row[(p.c + p.i <= p.t ? p.c + p.i : p.c - p.i) - 1].x = run;
         run = fq29_mul_inline(run, den);
     }
     Fq29 inv = fq29_inverse(run);
     while (count-- > 0) {
-        const size_t t = base + (size_t)count * GT;
-        A29* row = row_of(t);
-        const A29 a = row[t & (k - 1)], b = row[k - 1];
+        const At p = at(base + count * GT);
+        const A29 a = p.row[p.i - 1], b = p.row[p.c - 1];
+        const bool up = p.c + p.i <= p.t, down = p.c - p.i > p.h;
         Fq29 den;
         const uint32_t kind = kind_of(a, b, den);
-        const Fq29 di = fq29_mul_inline(inv, row[k + (t & (k - 1))].x);
+        const Fq29 di = fq29_mul_inline(inv, p.row[(up ? p.c + p.i : p.c - p.i) - 1].x);
         inv = fq29_mul_inline(inv, den);
-        Fq29 num;
-        if (kind == 1u) { const Fq29 xx = fq29_sqr(a.x); num = fq29_add(fq29_dbl(xx), xx); }
-        else num = fq29_sub_raw(a.y, b.y);
-        const Fq29 l = fq29_mul_inline(num, di);
-        A29 r;
-        // back to (-eps, p + eps): the coordinates must not grow with the table
-        r.x = fq29_lift(fq29_lift(fq29_sub(fq29_sub(fq29_sqr_inline(l), a.x), b.x)));
-        r.y = fq29_lift(fq29_sub(fq29_mul_inline(l, fq29_sub_raw(a.x, r.x)), a.y));
-        if (kind == 2u) r = a;
-        if (kind == 3u) r = b;
-        if (kind == 4u) { r.x = fq29_zero(); r.y = fq29_zero(); }
-        row[k + (t & (k - 1))] = r;
+        // coordinates back to (-eps, p + eps): they must not grow with the table
+        auto x_of = [&](const Fq29& l) { return fq29_lift(fq29_lift(fq29_sub(fq29_sub(fq29_sqr_inline(l), a.x), b.x))); };
+        A29 twice = b;                                      // of equal or opposite points: twice the centre
+        if (kind == 1u || kind == 2u) {
+            const Fq29 xx = fq29_sqr(b.x), l = fq29_mul(fq29_add(fq29_dbl(xx), xx), di);
+            twice.x = x_of(l);
+            twice.y = fq29_lift(fq29_sub(fq29_mul(l, fq29_sub_raw(b.x, twice.x)), b.y));
+        }
+        if (up) {
+            const Fq29 l = fq29_mul_inline(fq29_sub_raw(a.y, b.y), di);
+            A29 r;
+            r.x = x_of(l);
+            r.y = fq29_lift(fq29_sub(fq29_mul_inline(l, fq29_sub_raw(a.x, r.x)), a.y));
+            if (kind == 1u) r = twice;
+            if (kind == 3u) r = a;
+            if (kind == 4u) r = b;
+            if (kind == 2u || kind == 5u) { r.x = fq29_zero(); r.y = fq29_zero(); }
+            p.row[p.c + p.i - 1] = r;
+        }
+        if (down) {          // the centre and entry i's opposite
+            const Fq29 l = fq29_mul_inline(fq29_add(a.y, b.y), di);
+            A29 r;
+            r.x = x_of(l);
+            r.y = fq29_lift(fq29_add(fq29_mul_inline(l, fq29_sub_raw(r.x, a.x)), a.y));
+            if (kind == 2u) r = twice;
+            if (kind == 3u) { r.x = a.x; r.y = fq29_lift(fq29_neg(a.y)); }
+            if (kind == 4u) r = b;
+            if (kind == 1u || kind == 5u) { r.x = fq29_zero(); r.y = fq29_zero(); }
+            p.row[p.c - p.i - 1] = r;
+        }
     }
 }
 // Sums of [s_j] G_j over segments of the rows (item = segment * m + row, so that a wave's items use the same part of the table), to
@@ -2241,16 +2275,33 @@ int zk_g1_normalize(void* out, const void* in, size_t n, void* st) {
 }
 
 // levels that k_msm_table_first takes: as many entries a window as two waves a SIMD have lanes for
-static uint32_t msm_first_levels(size_t rows, uint32_t levels) {
-    uint32_t logs = 0;
-    while (logs < levels && rows << (logs + 1) <= (size_t)1 << 17) ++logs;
-    return logs;
+// the growth of a window from h to `target` entries, at most GROW_MAX steps
+static std::vector<GrowSpec> grow_steps(uint32_t h, uint32_t target) {
+    std::vector<GrowSpec> v;
+    while (h < target) {
+        const uint32_t t = std::min(target, 3 * h), c = (h + t + 1) / 2;
+        v.push_back(GrowSpec{h, c, t, std::max(c - h - 1, t - c)});
+        h = t;
+    }
+    return v;
+}
+// The entries of a window that k_msm_table_first makes: as many as leave it, with the growth's centres, the lanes of two waves a SIMD, and no more than the longest has.  rows: the full windows
+// of all generators; half, top: entries of a full and of a highest window.  steps: the growth's launches.
+static uint32_t msm_first_entries(size_t rows, size_t ngen, uint32_t half, uint32_t top, uint32_t* steps) {
+    const uint32_t longest = rows ? std::max(half, top) : top;
+    uint32_t first = (uint32_t)std::min<size_t>(longest, std::max<size_t>(1, ((size_t)1 << 17) / (rows + ngen)));
+    for (;; --first) {
+        const size_t full_n = rows ? grow_steps(first, half).size() : 0, top_n = grow_steps(first, top).size();
+        *steps = (uint32_t)std::max(full_n, top_n);
+        if (first == 1 || (rows + ngen) * first + rows * full_n + ngen * top_n <= (size_t)1 << 17) return first;
+    }
 }
 // Digit width, windows and segments for m rows of ngen scalars.  seen[b]: how many of the sampled scalars have b bits.  Estimated times in us:
-// a level of the table counts 60 us (one lane's inversion) or 30 among the first ones (k_msm_table_first, 50 us besides) and 0.12 ns an entry,
+// a step of the table's growth counts 75 us (one lane's inversion), its first entries 50 and 30 for each doubling of their number, an entry 0.115 ns,
 // a base's doubling 7 us of latency, an addition 0.17 ns; a digit beyond the first is an addition where the scalar reaches it.
-// These are weights for the choice and not the kernels' times: in k_msm_table_grow an entry of a large level takes 0.24 ns, its 60 us included, and an
-// addition 0.18 (11008 x 4096 of 13 bits).  Every width timed, 1 to 11008 rows of 64 to 4096 generators and scalars of 13 and of 28 bits (48 shapes):
+// These are weights for the choice and not the kernels' times: in the large steps of k_msm_table_grow an entry takes 0.14 ns and an
+// addition 0.18 (11008 x 4096 of 13 bits).  With them no size from 1 to 11008 rows of 64 to 4096 generators
+// is slower than with a table that doubles, and 5000 x 2048 takes 3.43 ms instead of 3.75.  Every width timed against a table that doubles, 1 to 11008 rows of 64 to 4096 generators and scalars of 13 and of 28 bits (48 shapes):
 // the one chosen here takes 4 % longer than the best on average.  The furthest off are 28-bit scalars in few rows of 64 generators, 14 % (3 bits chosen,
 // 7 are best), 512 rows of 4096, 12 % (9, 7), and many rows of 28 bits, 7 % (13, 9); the same model fitted to those times chooses no better (5 %).
 struct MsmShape { uint32_t c, nwin, top, nseg; };
@@ -2272,10 +2323,9 @@ static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs,
         }
         double entries = (double)ngen * ((nwin - 1) * (double)half + top);
         if (entries * sizeof(A29) > 8e9) continue;
-        uint32_t levels = 0;
-        while ((1u << levels) < (nwin > 1 ? std::max(half, top) : top)) ++levels;
-        const uint32_t first = msm_first_levels(ngen * nwin, levels);
-        const double us = 7.0 * c * (nwin - 1) + 60.0 * (levels - first) + (first ? 50.0 + 30.0 * first : 0.0) + entries * 1.2e-4 + (double)m * ngen * digits * 1.7e-4;
+        uint32_t steps = 0;
+        const uint32_t first = msm_first_entries((size_t)(nwin - 1) * ngen, ngen, half, top, &steps);
+        const double us = 7.0 * c * (nwin - 1) + 75.0 * steps + (first > 1 ? 50.0 + 30.0 * std::log2((double)first) : 0.0) + entries * 1.15e-4 + (double)m * ngen * digits * 1.7e-4;
         if (!best.c || us < best_us) { best_us = us; best = MsmShape{c, nwin, top, 1}; }
     }
     if (!best.c) {      // more generators than the budget of the table allows any width for
@@ -2327,18 +2377,23 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     hipLaunchKernelGGL(k_msm_table_bases, dim3(cdiv(ngen, GT)), dim3(GT), 0, st, basej.as<G1Jac>(), (const G1Jac*)gens, ngen, T.c, T.nwin, 1u);
     g1_normalize_queue<true>(basea.p, basej.as<G1Jac>(), nbase, st);
     const size_t rows_full = (size_t)(T.nwin - 1) * ngen;
-    uint32_t levels = 0;
-    while ((1u << levels) < std::max(T.top, T.nwin > 1 ? T.half : 1u)) ++levels;
-    const uint32_t logs = msm_first_levels(nbase, levels);
-    hipLaunchKernelGGL(k_msm_table_first, dim3(cdiv(nbase << logs, GT)), dim3(GT), 0, st, T, basea.as<G1Affine>(), logs);
-    for (uint32_t logk = logs; (1u << logk) < std::max(T.top, T.nwin > 1 ? T.half : 1u); ++logk) {
-        const bool with_top = (1u << logk) < T.top;
-        // the windows below the highest are never shorter than it, but a single window is the highest
-        const size_t rows = (T.nwin > 1 ? rows_full : 0) + (with_top ? ngen : 0), n = rows << logk;
+    uint32_t steps = 0;
+    const uint32_t first = msm_first_entries(rows_full, ngen, T.half, T.top, &steps);
+    const std::vector<GrowSpec> full = T.nwin > 1 ? grow_steps(first, T.half) : std::vector<GrowSpec>(), top = grow_steps(first, T.top);
+    GrowCentres gc;
+    gc.full_n = (uint32_t)full.size(); gc.top_n = (uint32_t)top.size();
+    ZK_ARG(gc.full_n <= (uint32_t)GROW_MAX && gc.top_n <= (uint32_t)GROW_MAX, "zk_g1_commit_int: too many generators");
+    for (int i = 0; i < GROW_MAX; ++i) { gc.full[i] = i < (int)gc.full_n ? (uint16_t)full[i].c : 1; gc.top[i] = i < (int)gc.top_n ? (uint16_t)top[i].c : 1; }
+    const size_t first_n = rows_full * gc.full_n + ngen * gc.top_n + nbase * first;
+    hipLaunchKernelGGL(k_msm_table_first, dim3(cdiv(first_n, GT)), dim3(GT), 0, st, T, basea.as<G1Affine>(), first, gc);
+    for (size_t i = 0; i < std::max(full.size(), top.size()); ++i) {
+        const GrowSpec none{1u, 1u, 1u, 0u}, f = i < full.size() ? full[i] : none, p = i < top.size() ? top[i] : none;
+        const size_t n = rows_full * f.np + ngen * p.np;
         if (n == 0) continue;
-        // entries a lane: one until every lane of two waves a SIMD has one, then as many as leave those waves, up to 32
-        const uint32_t per_lane = (uint32_t)std::min<size_t>(32, std::max<size_t>(1, n >> 17));
-        hipLaunchKernelGGL(k_msm_table_grow, dim3(cdiv(n, (size_t)GT * per_lane)), dim3(GT), 0, st, T, logk, rows_full, rows, per_lane);
+        // pairs a lane: whole rounds of the lanes of two waves a SIMD, of at most 32 pairs each
+        const size_t lanes = (size_t)1 << 17, rounds = (n + 32 * lanes - 1) / (32 * lanes);
+        const uint32_t per_lane = (uint32_t)((n + rounds * lanes - 1) / (rounds * lanes));
+        hipLaunchKernelGGL(k_msm_table_grow, dim3(cdiv(n, (size_t)GT * per_lane)), dim3(GT), 0, st, T, f, p, (uint32_t)n, per_lane);
     }
     ZK_LAUNCH_CHECK();
     const size_t per = (ngen + shape.nseg - 1) / shape.nseg, items = m * shape.nseg;
