@@ -161,6 +161,33 @@ def test_the_two_streams_of_an_opening_are_two_apart(tmp_path):
         assert {x for c, a, b in pairs if c == count for x in (a, b)} == set(range(count))
 
 
+def test_products_in_29_bit_limbs_stay_in_range_and_match_big_integers(tmp_path):
+    """fq29_mul, fq29_sqr and fq29_mul_sub against big integers: limbs all zero, all ones, of either sign, operands of up to 32 p.  A product stands for
+    a b / 2^406 mod p and lies within 2^-14 p of [0, p]: |a b| <= 2^10 p^2 over R' = 2^406 > 2^25 p, the two of mul_sub twice that, and 2^-29 p from the reduction."""
+    src = tmp_path / "fq29.cpp"
+    src.write_text('#include <cstdio>\n#include "fq29.hpp"\nusing namespace zk;\nint main() { Fq29 v[4]; auto rd = [](Fq29& x) { for (int i = 0; i < 14; ++i) if (scanf("%d", &x.l[i]) != 1) return false; return true; };'
+                   ' auto wr = [](const Fq29& x) { for (int i = 0; i < 14; ++i) printf("%d ", x.l[i]); };'
+                   ' while (rd(v[0]) && rd(v[1]) && rd(v[2]) && rd(v[3])) { wr(fq29_mul_inline(v[0], v[1])); wr(fq29_sqr_inline(v[0])); wr(fq29_mul_sub(v[0], v[1], v[2], v[3])); puts(""); } }\n')
+    csrc = os.path.join(ROOT, "zkllm-ccs2024_amd", "csrc")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + csrc, str(src), "-o", str(tmp_path / "fq29")], check=True)
+    m29, rng = (1 << 29) - 1, random.Random(41)
+    norm = lambda x: [(x >> (29 * i)) & m29 for i in range(13)] + [x >> (29 * 13)]
+    value = lambda l: sum(v << (29 * i) for i, v in enumerate(l))
+    normal = [norm(x) for x in (0, 1, -1, P_MOD, -P_MOD, P_MOD - 1, 32 * P_MOD, -32 * P_MOD, (1 << 29) - 1, (1 << 377) - 1, (1 << 384) - 1, -(1 << 384))]
+    normal += [norm(rng.randrange(-32 * P_MOD, 32 * P_MOD)) for _ in range(30)]
+    raw = [[m29] * 13 + [13], [-m29] * 13 + [-13], [m29, -m29] * 6 + [m29, 13], [0] * 13 + [400], [-m29] + [0] * 12 + [-1]]
+    cases = [(a, b, rng.choice(normal), rng.choice(normal)) for a in normal + raw for b in normal + raw]
+    text = "\n".join(" ".join(str(x) for v in c for x in v) for c in cases)
+    out = subprocess.run([str(tmp_path / "fq29")], input=text, check=True, capture_output=True, text=True).stdout.splitlines()
+    rinv, eps = pow(2, -406, P_MOD), P_MOD >> 14
+    assert len(out) == len(cases)
+    for (a, b, c, d), line in zip(cases, out):
+        got = list(map(int, line.split()))
+        for limbs, exact in ((got[:14], value(a) * value(b)), (got[14:28], value(a) ** 2), (got[28:], value(a) * value(b) - value(c) * value(d))):
+            assert all(0 <= x <= m29 for x in limbs[:13])
+            assert -eps <= value(limbs) <= P_MOD + eps and (value(limbs) - exact * rinv) % P_MOD == 0
+
+
 def test_complete_projective_additions_match_the_affine_group_law():
     """p29_add (the bucket reductions' addition: no special cases), run on the CPU, against the affine group law: random points, a point and
     itself, its opposite, infinity on either side and both, and points outside the subgroup of order r, those of order three among them."""
