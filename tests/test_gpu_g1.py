@@ -717,8 +717,9 @@ def test_open_round_whose_lists_are_sorted_a_few_windows_at_a_time():
 
 
 # 4099 x 8 and 33001: the first and the second round on their tables (odd halves); 12300 x 8: the first alone without tables, or on its table;
-# 40000 x 3: three, the third without a table; 2051 x 8: the first on its table and no table for the second
-@pytest.mark.parametrize("n,count,tables", [(4099, 8, 2), (33001, 1, 2), (12300, 8, 0), (12300, 8, 1), (12300, 8, 2), (40000, 3, 2), (2051, 8, 2)])
+# 40000 x 3: three, the third without a table; 2051 x 8: the first on its table and no table for the second; 2049: sums of
+# windows of 128 buckets over all the generators, in a wave a window for two members and with a lane for eight buckets for eight
+@pytest.mark.parametrize("n,count,tables", [(4099, 8, 2), (33001, 1, 2), (12300, 8, 0), (12300, 8, 1), (12300, 8, 2), (40000, 3, 2), (2051, 8, 2), (2049, 2, 0), (2049, 8, 0)])
 def test_open_batches_follow_the_logarithms_of_their_generators(n, count, tables):
     """zk_g1_open_begin_batch over prepared generators of known logarithm, special ones at another place in each member."""
     import ctypes
