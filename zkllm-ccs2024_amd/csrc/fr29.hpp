@@ -23,6 +23,10 @@ ZK_HD constexpr int32_t fr29_p(int i) {                 // r
     constexpr int32_t t[9] = {1, 536870904, 529989567, 457704959, 494949691, 201589968, 354471143, 174404527, 7597479};
     return t[i];
 }
+ZK_HD constexpr int32_t fr29_n(int i) {                 // ((2^29 - 1) r + 1) / 2^29
+    constexpr int32_t t[9] = {9, 6881336, 72284608, 499626180, 293359722, 383989737, 180066615, 166807048, 7597479};
+    return t[i];
+}
 ZK_HD Fr29 fr29_const(const int32_t (&t)[9]) {
     Fr29 r;
 #pragma unroll
@@ -44,8 +48,12 @@ ZK_HD Fr29 fr29_zero() {
 }
 
 // Montgomery reduction interleaved with the columns: col(k), k = 0..17, is the k-th column of the value to reduce (a product:
-// columns 0..16; a Wide29 sum: 18 limbs).  Returns value * 2^-261 mod r as a non-negative integer below value / 2^261 + r.
+// columns 0..16; a Wide29 sum: 18 limbs).  Returns value * 2^-261 mod r as a non-negative integer below value / 2^261 + (1 + 2^-29) r.
+// The first seven limbs go by N = (2^29 - 1) r, which ends in -1: the multiple of N that clears a limb is the limb itself, and what it adds to the columns
+// above is fr29_n, with nothing to negate and nothing to add to the column.  N is 2^29 times r, so the last two limbs go by r: the seven add less than 2^(29 * 7) N = 2^-29 2^261 r.
+// All nine by r: a lookup of 2^22 queries took 491 us instead of 483, an attention head of 2048 tokens 3.16 ms instead of 3.13 (medians of four).
 template <int NCOL, typename Col> ZK_HD Fr29 fr29_redc(Col col) {
+    constexpr int FAST = 7;
     int32_t m[9];
     Fr29 t;
     int64_t carry = 0;
@@ -53,17 +61,23 @@ template <int NCOL, typename Col> ZK_HD Fr29 fr29_redc(Col col) {
     for (int k = 0; k < 9; ++k) {
         int64_t q = carry;
 #pragma unroll
-        for (int i = 0; i < k; ++i) q += (int64_t)m[i] * fr29_p(k - i);
+        for (int i = 0; i < k; ++i) q += (int64_t)m[i] * (i < FAST ? fr29_n(k - i - 1) : fr29_p(k - i));
         q += col(k);
-        m[k] = (int32_t)((0u - (uint32_t)q) & R29M);       // r = 1 mod 2^29: -r^-1 = -1
-        q += (int64_t)m[k];
+        if (k < FAST) m[k] = (int32_t)((uint32_t)q & R29M);
+        else {
+            m[k] = (int32_t)((0u - (uint32_t)q) & R29M);   // r = 1 mod 2^29: -r^-1 = -1
+            q += (int64_t)m[k];
+        }
         carry = q >> 29;
     }
 #pragma unroll
     for (int k = 9; k < 18; ++k) {
         int64_t q = carry;
 #pragma unroll
-        for (int i = k - 8; i < 9; ++i) q += (int64_t)m[i] * fr29_p(k - i);
+        for (int i = k - 9; i < 9; ++i) {
+            if (i < FAST) q += (int64_t)m[i] * fr29_n(k - i - 1);
+            else if (i > k - 9) q += (int64_t)m[i] * fr29_p(k - i);
+        }
         if (k < NCOL) q += col(k);
         if (k < 17) {
             t.l[k - 9] = (int32_t)((uint32_t)q & R29M);
