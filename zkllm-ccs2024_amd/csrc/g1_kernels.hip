@@ -322,19 +322,29 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
     }
 }
+static constexpr int P29_WORDS = 42;
+static_assert(sizeof(P29) == 4 * P29_WORDS, "a point is its coordinates");
+__device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
+    P29 r;
+    const int32_t* src = reinterpret_cast<const int32_t*>(&a);
+    int32_t* dst = reinterpret_cast<int32_t*>(&r);
+#pragma unroll
+    for (int l = 0; l < P29_WORDS; ++l) dst[l] = __shfl(src[l], lane, 64);
+    return r;
+}
 // Sums of [s_j] G_j over segments of the rows (item = segment * m + row, so that a wave's items use the same part of the table), to
-// out[row * nseg + segment].  Sixteen lanes take an item, four items a wave.
+// out[row], or to part[row * nseg + segment] where rows have several.  Sixteen lanes take an item, four items a wave.
 // The scalars' non-zero digits go through a list in LDS, sixteen scalars at a time, and an addition starts when every item of the wave
 // has sixteen: where the second digit of most scalars is zero, lanes that each walked their own scalar's digits would wait for the one
-// in sixty-four that is not.  Sixteen lanes and not the whole wave, because a sum over the lanes of one row is serial: its levels
-// serve four rows at once and are four instead of six.
+// in sixty-four that is not.  Sixteen lanes and not the whole wave, because a sum over the lanes of one row is serial: five additions on four lanes
+// (four levels of Jacobian additions on a lane: 300 rows of 4096 generators 1.67 ms, with k_msm_parts as it is now 1.24).
 // Instruction issue binds it (two waves a SIMD).  11008 rows of 4096 14-bit scalars: 7-bit signed digits of the whole wave's lanes, in
 // Jacobian coordinates, took 17.7 ms; 12-bit digits this way take less than half.
 static constexpr uint32_t MSM_CAP = 256;
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_msm_rows(G1Jac* __restrict__ out, const MsmTable T, const int32_t* __restrict__ scalars, size_t m_rows, uint32_t nseg, uint32_t per) {
+k_msm_rows(G1Jac* __restrict__ out, P29* __restrict__ part, const MsmTable T, const int32_t* __restrict__ scalars, size_t m_rows, uint32_t nseg, uint32_t per) {
     __shared__ uint32_t list[4][MSM_CAP];
-    __shared__ int32_t sums[43][GT];
+    __shared__ int32_t sums[P29_WORDS][GT];
     const uint32_t t = threadIdx.x, grp = t >> 4, ln = t & 15u;
     const size_t item = (size_t)blockIdx.x * 4 + grp;
     const bool valid = item < m_rows * nseg;
@@ -388,29 +398,44 @@ k_msm_rows(G1Jac* __restrict__ out, const MsmTable T, const int32_t* __restrict_
         }
         __syncthreads();
     }
-    J29 v = j29_from_x29(acc);
-    for (uint32_t s = 8; s > 0; s >>= 1) {
-        const int32_t* w = reinterpret_cast<const int32_t*>(&v);
+    P29 r = p29_from_x29(acc);
+    {
+        const int32_t* w = reinterpret_cast<const int32_t*>(&r);
 #pragma unroll
-        for (int l = 0; l < 43; ++l) sums[l][t] = w[l];
-        __syncthreads();
-        J29 o;
-        int32_t* wo = reinterpret_cast<int32_t*>(&o);
-        const uint32_t from = (t & 48u) | ((ln + s) & 15u);
-#pragma unroll
-        for (int l = 0; l < 43; ++l) wo[l] = sums[l][from];
-        v = j29_add(v, o);
-        __syncthreads();
+        for (int l = 0; l < P29_WORDS; ++l) sums[l][t] = w[l];
     }
-    if (valid && ln == 0) out[row * nseg + seg] = j29_to_jac(v);
+    __syncthreads();
+    auto get = [&](uint32_t lane) {
+        P29 o;
+        int32_t* w = reinterpret_cast<int32_t*>(&o);
+#pragma unroll
+        for (int l = 0; l < P29_WORDS; ++l) w[l] = sums[l][lane];
+        return o;
+    };
+    r = get(t & 60u);
+    for (uint32_t step = 0; step < 5; ++step) {             // a quad's other three lanes, then the item's other quads
+        const P29 o = step < 3 ? get((t & 60u) + step + 1) : p29_shfl(r, (int)(t ^ (step == 3 ? 4u : 8u)));
+        p29_quad_add(r, o, t & 3u);
+    }
+    if (valid && ln == 0) {
+        if (nseg > 1) part[row * nseg + seg] = r;
+        else out[row] = p29_to_jac(r);
+    }
 }
-// out[row] = the sum of row's few parts, a lane a row
-__global__ void __launch_bounds__(GT) k_msm_parts(G1Jac* __restrict__ out, const G1Jac* __restrict__ part, size_t m_rows, uint32_t nseg) {
-    const size_t row = (size_t)blockIdx.x * GT + threadIdx.x;
-    if (row >= m_rows) return;
-    J29 s = j29_from_jac(part[row * nseg]);
-    for (uint32_t i = 1; i < nseg; ++i) s = j29_add(s, j29_from_jac(part[row * nseg + i]));
-    out[row] = j29_to_jac(s);
+// out[row] = the sum of row's nseg parts, 2^lg <= nseg groups of four lanes a row.  A chain of additions that nothing else runs beside: one after another
+// on one lane, sixteen parts took 410 us of the 880 that
+// committing 20 rows of 512 generators took; now the whole of it takes 454.
+__global__ void __launch_bounds__(GT) k_msm_parts(G1Jac* __restrict__ out, const P29* __restrict__ part, size_t m_rows, uint32_t nseg, uint32_t lg) {
+    const uint32_t t = threadIdx.x, groups = 1u << lg;
+    const size_t at = (size_t)blockIdx.x * (GT / 4) + (t >> 2), row = at >> lg;
+    const uint32_t g = (uint32_t)at & (groups - 1u), own = nseg >> lg;
+    const P29* __restrict__ P = part + (row < m_rows ? row : 0) * nseg + g;
+    P29 r = P[0];
+    for (uint32_t step = 1; step < own + lg; ++step) {
+        const P29 o = step < own ? P[(size_t)step << lg] : p29_shfl(r, (int)(t ^ (4u << (step - own))));
+        p29_quad_add(r, o, t & 3u);
+    }
+    if (row < m_rows && g == 0 && (t & 3u) == 0) out[row] = p29_to_jac(r);
 }
 // out[i] = [s_i] B for one base point B: additions out of the table of B's multiples d * 2^(8w) B, d = 1..128, w = 0..32
 // (signed 8-bit digits of the 256-bit integer s_i; window 32 only ever holds the last carry).  33 mixed additions at
@@ -710,8 +735,6 @@ __global__ void __launch_bounds__(GT) k_msm_recode(const RecodeBatch rb, size_t 
     msm_recode_store(rb.D[blockIdx.y], n, i, rb.S[blockIdx.y][i], plan);
 }
 
-static constexpr int P29_WORDS = 42;
-static_assert(sizeof(P29) == 4 * P29_WORDS, "a point is its coordinates");
 // The end of a list of points in bucket order that a wave's lanes have divided evenly (lane t the t-th share).  x: the sum of the last part of
 // the lane's share, which belongs to bucket b; begun: the bucket begins in this share (or the share is empty); whole: it ends with this
 // share; lacks: bucket `split`, the first part's, went out already without the shares before this one.  A segmented inclusive scan, as
@@ -1023,14 +1046,6 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
 // instructions; the windows are summed before the walk so that 32 waves and two walks of four lanes do what took 256 walks a sum.
 // The list: sums of one number of windows stand together and begin at a multiple of eight (a wave of k_msm_horner; gaps: out = null), those of few elements last.
 struct PointDesc { P29* buckets; P29* blocks; G1Jac* out; uint32_t few, nwh, hb, pad; };
-__device__ __forceinline__ P29 p29_shfl(const P29& a, int lane) {
-    P29 r;
-    const int32_t* src = reinterpret_cast<const int32_t*>(&a);
-    int32_t* dst = reinterpret_cast<int32_t*>(&r);
-#pragma unroll
-    for (int l = 0; l < P29_WORDS; ++l) dst[l] = __shfl(src[l], lane, 64);
-    return r;
-}
 // win[sum * MW + w]: the windows' sums.  grid: MW workgroups for each of the first `full` sums, then MW / 8 for each from first_few on, of few elements
 // BLOCKS: grid (blocks of a sum, sums), the first of the list; blocks[2 (w * hb / MT + block)]: the two sums of a block
 template <bool BLOCKS> __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_windows(P29* __restrict__ win, const PointDesc* __restrict__ list, uint32_t full, uint32_t first_few) {
@@ -2452,11 +2467,14 @@ int zk_g1_commit_int(void* out, const void* gens, const void* scalars_fr, size_t
     }
     ZK_LAUNCH_CHECK();
     const size_t per = (ngen + shape.nseg - 1) / shape.nseg, items = m * shape.nseg;
-    Scratch part(shape.nseg > 1 ? sizeof(G1Jac) * items : 1, st);
+    Scratch part(shape.nseg > 1 ? sizeof(P29) * items : 1, st);
     if (part.rc) return part.rc;
-    hipLaunchKernelGGL(k_msm_rows, dim3(cdiv(items, 4)), dim3(GT), 0, st, shape.nseg > 1 ? part.as<G1Jac>() : (G1Jac*)out, T, ints.as<int32_t>(), m, shape.nseg, (uint32_t)per);
-    if (shape.nseg > 16) hipLaunchKernelGGL(k_g1_rowsum, dim3((unsigned)m, 1), dim3(GT), 0, st, (G1Jac*)out, part.as<G1Jac>(), (size_t)shape.nseg, 1u);
-    else if (shape.nseg > 1) hipLaunchKernelGGL(k_msm_parts, dim3(cdiv(m, (size_t)GT)), dim3(GT), 0, st, (G1Jac*)out, part.as<G1Jac>(), m, shape.nseg);
+    hipLaunchKernelGGL(k_msm_rows, dim3(cdiv(items, 4)), dim3(GT), 0, st, (G1Jac*)out, part.as<P29>(), T, ints.as<int32_t>(), m, shape.nseg, (uint32_t)per);
+    if (shape.nseg > 1) {           // a power of two: half as many groups as parts are as fast as all
+        uint32_t lg = 0;
+        while (lg < 4 && (4u << lg) <= shape.nseg) ++lg;
+        hipLaunchKernelGGL(k_msm_parts, dim3(cdiv(m << lg, (size_t)GT / 4)), dim3(GT), 0, st, (G1Jac*)out, part.as<P29>(), m, shape.nseg, lg);
+    }
     ZK_LAUNCH_CHECK();
     return 0;
 }
