@@ -1124,7 +1124,7 @@ template <bool BLOCKS> __global__ void __launch_bounds__(GT) __attribute__((amdg
     }
 }
 // The same for windows of 128 buckets of lists that fill the chip: a lane has eight neighbouring buckets and a wave four windows.  An addition takes
-// 2700 instructions on four lanes and 5700 on one, so this takes half of them, but a wave alone 490 us instead of 150: the proof of a small layer, with lists of 66 and 155 sums,
+// 2700 instructions on four lanes and 5700 on one, so this takes half of them, but 340 to 390 us where a wave a window takes 150 alone: the proof of a small layer, with lists of 66 and 155 sums,
 // takes 5.45 ms instead of 5.76 (medians of six).  Blocks of wider windows (2112 and 3016 waves of an opening of 131072 columns) gain nothing by it.
 // grid: (windows of a sum / 4, sums from `first` on)
 static constexpr uint32_t WIN_LANES = 4;                   // windows a wave
