@@ -167,7 +167,7 @@ def test_commit_int_matches_oracle(pv, orc, m, n, lim):
     assert (norm(orc, got) == norm(orc, exp)).all()
 
 
-@pytest.mark.parametrize("m,n,lim", [(40, 100, 1), (5, 64, 7), (3, 520, 9), (2, 8192, 3), (1, 5000, 2 ** 31 - 1), (3, 129, 9), (200, 300, 2 ** 12), (9, 33, 2 ** 20)])
+@pytest.mark.parametrize("m,n,lim", [(40, 100, 1), (5, 64, 7), (3, 520, 9), (2060, 260, 5), (2, 8192, 3), (1, 5000, 2 ** 31 - 1), (3, 129, 9), (200, 300, 2 ** 12), (9, 33, 2 ** 20)])
 def test_commit_int_tables_of_every_shape_match_the_oracle(pv, orc, m, n, lim):
     """Tables whose first entries (k_msm_table_first) are all of a window, none, or as many as two waves a SIMD have lanes for, and rows of
     one to 256 parts; one generator is infinity, two are equal."""

@@ -2404,8 +2404,11 @@ static MsmShape msm_shape(size_t m, size_t ngen, uint32_t bits, uint32_t maxabs,
         for (best.top = 1; best.top < most; best.top <<= 1) {}
     }
     // segments of a row: items (sixteen lanes each) for two waves a SIMD while they keep 32 generators each, and for eight where they keep 512
-    // (a launch of 1.3 times the waves that fit leaves the chip half empty at its end; the sum over an item's lanes costs ten additions)
-    while ((m * best.nseg * 2 <= 8192 && ngen / (best.nseg * 2) >= 32) || (m * best.nseg < 32768 && ngen / (best.nseg * 2) >= 512)) best.nseg *= 2;
+    // (a launch of 1.3 times the waves that fit leaves the chip half empty at its end; the sum over an item's lanes costs five additions on four lanes).
+    // Up to 1536 waves leave most SIMDs one wave or a third of them a second one for all of a launch: twice as many of half the length, where 128 generators are left
+    // for each, take 2100 to 2780 rows of 1024 from 1.66 to 1.40 ms, 5500 of 512 from 1.55 to 1.43; from 8000 items on (4000 rows of 1024, 8000 of 512) they lose 3 %.
+    while ((m * best.nseg * 2 <= 8192 && ngen / (best.nseg * 2) >= 32) || (m * best.nseg < 32768 && ngen / (best.nseg * 2) >= 512)
+           || (m * best.nseg < 6144 && ngen / (best.nseg * 2) >= 128)) best.nseg *= 2;
     return best;
 }
 
