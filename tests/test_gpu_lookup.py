@@ -581,6 +581,45 @@ def test_multi_hadamard_with_evaluation_challenges_of_one_and_zero(pv, orc, spec
     assert (proof == e_proof).all() and (fin == e_fin).all()
 
 
+@pytest.mark.parametrize("k", [6, 13, 18])
+def test_jobs_take_an_evaluation_challenge_of_one_in_any_form(k):
+    """1, r + 1 and 2 r + 1 are one challenge, for which a job writes every round's eq table: begun at once, begun on an opened table, Hadamard."""
+    import ctypes
+    from gpuhelp import Hip, c_void_p, c_size_t, c_int
+    hip = Hip()
+    D, N, low = 1 << k, 32, -16
+    pos = np.random.default_rng(k).integers(0, N, D)
+    T = fr_array([(low + i) % R_MOD for i in range(N)])
+    m = fr_array([int(c) for c in np.bincount(pos, minlength=N)])
+    beta, u, v = ch(43, 1)[0], ch(44, k - 1), ch(45, k)
+    dS, dT, dm, dX = hip.upload(T[pos]), hip.upload(T), hip.upload(m), [hip.upload(ch(46 + i, D)) for i in range(2)]
+    ptrs = (ctypes.c_void_p * 2)(*dX)
+    sizes = (c_size_t(D), c_size_t(N), c_int(k))
+    first = None
+    for one in (1, R_MOD + 1, 2 * R_MOD + 1):
+        u[k // 2] = np.frombuffer(one.to_bytes(32, "little"), np.uint32)
+        out = []
+        for opened in (False, True):
+            h, o = c_void_p(), c_void_p()
+            if opened:
+                hip.call("zk_lookup_open", ctypes.byref(o), c_void_p(dT), beta, c_size_t(N), None)
+                hip.call("zk_lookup_prove_begin_opened", ctypes.byref(h), o, c_void_p(dS), None, None, None, None, None, c_void_p(dT), c_void_p(dm), c_int(low), beta, u, v, *sizes,
+                         c_int(1), c_int(1), None)
+            else:
+                hip.call("zk_lookup_prove_begin_hinted", ctypes.byref(h), c_void_p(dS), c_void_p(dT), c_void_p(dm), c_void_p(dS), c_int(low), beta, u, v, *sizes, None)
+            bm, sums = np.zeros(8, np.uint32), np.zeros((k * 11, 8), np.uint32)
+            hip.call("zk_lookup_prove_end", h, bm, sums)
+            out += [bm, sums]
+        h, coefs = c_void_p(), np.zeros((k * 3, 8), np.uint32)
+        hip.call("zk_hadamard_prove_begin", ctypes.byref(h), ptrs, c_int(2), u, v, c_size_t(D), None)
+        hip.call("zk_hadamard_prove_end", h, coefs)
+        out.append(coefs)
+        first = first or out
+        assert all((a == b).all() for a, b in zip(first, out)), one // R_MOD
+    for p in [dS, dT, dm] + dX:
+        hip.free(p)
+
+
 @pytest.mark.parametrize("n,kept", [(4096, (True, True)), (1 << 17, (True, True)), (1 << 17, (True, False)), (1 << 15, (False, True))])
 def test_multi_hadamard_of_two_tensors_that_keep_an_int32_form(pv, orc, n, kept):
     """Two tensors of 32-bit integers, the extremes included, kept for folds: the job's first round reads their int32 forms

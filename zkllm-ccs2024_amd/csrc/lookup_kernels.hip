@@ -2010,12 +2010,9 @@ static int eq_table_queue(Fr* out, const uint32_t* u, int k, Arena& arena, hipSt
         return 0;
     }
     EqChallenges c;
-    Fr one = big_zero<8>();
-    one.v[0] = 1;
     for (int j = 0; j < 30; ++j) {
-        const Fr uj = j < k ? load_fr(u + 8 * j) : big_zero<8>();
-        c.u[j] = to_mont(uj);
-        c.omu[j] = to_mont(sub(one, uj));
+        c.u[j] = j < k ? to_mont(load_fr(u + 8 * j)) : big_zero<8>();          // reduced here, whatever form the challenge has
+        c.omu[j] = sub(big_one_mont<8>(), c.u[j]);
     }
     const int kl = (k + 1) / 2, kh = k - kl;
     Scratch& half = arena.add(sizeof(Fr) * (((size_t)1 << kl) + ((size_t)1 << kh)));
@@ -2348,12 +2345,9 @@ template <int KF, int KI> __global__ void __launch_bounds__(TPB) k_me_split(Fr* 
 // the tables of k_me_split for k challenges and n elements, queued on the stream (they live in the arena); blocks: its grid
 static int me_split_tabs_queue(MeSplitTabs& tb, unsigned& blocks, const uint32_t* u, int k, size_t n, Arena& arena, hipStream_t st) {
     EqChallenges c;
-    Fr one = big_zero<8>();
-    one.v[0] = 1;
     for (int j = 0; j < 30; ++j) {
-        const Fr uj = j < k ? load_fr(u + 8 * j) : big_zero<8>();
-        c.u[j] = to_mont(uj);
-        c.omu[j] = to_mont(sub(one, uj));
+        c.u[j] = j < k ? to_mont(load_fr(u + 8 * j)) : big_zero<8>();          // reduced here, whatever form the challenge has
+        c.omu[j] = sub(big_one_mont<8>(), c.u[j]);
     }
     const int kl = (k + 1) / 2, kh = k - kl;
     const uint32_t nlo = 1u << kl, nhi_full = 1u << kh;
@@ -2926,10 +2920,9 @@ static int sumjob_need_m(SumJob& job) {
 // whether a job over `rounds` rounds whose table is eq(u_eq, .) of rounds - 1 challenges (index bit j <-> u_eq[j]) can read its prefix throughout: no challenge is 1
 static bool eq_prefix_on() { static const bool on = [] { const char* e = getenv("ZKLLM_EQ_PREFIX"); return !(e && e[0] == '0'); }(); return on; }
 static bool eq_prefix_possible(const uint32_t* u_eq, int rounds) {
-    Fr one = big_zero<8>();
-    one.v[0] = 1u;
+    const Fr one = big_one_mont<8>();
     for (int r = 1; r < rounds; ++r)
-        if (equal(load_fr(u_eq + 8 * (size_t)(r - 1)), one)) return false;
+        if (is_zero(sub(one, to_mont(load_fr(u_eq + 8 * (size_t)(r - 1)))))) return false;      // as residues: a challenge may come unreduced
     return eq_prefix_on();
 }
 // its constants
