@@ -1,0 +1,83 @@
+"""What the class layer asks of the C ABI and in which order, on the CPU: small programs over libzkllm_prover.so that define the
+entry points they reach themselves (a program's own definitions come before the kernel library's).  No GPU needed."""
+import os
+import subprocess
+
+from zkhelp import ROOT
+
+PKG = os.path.join(ROOT, "zkllm-ccs2024_amd")
+
+# device memory is host memory here; `events` holds the calls that a test looks at
+ABI = r"""
+#include <atomic>
+#include <chrono>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <string>
+#include <thread>
+#include <vector>
+#include "tlookup.hpp"
+static std::vector<std::string> events;
+static std::atomic<int> frees{0}, reads{0};
+extern "C" {
+const char* zk_last_error() { return "refused"; }
+int zk_malloc(void** p, size_t n) { *p = calloc(1, n + 64); return 0; }
+int zk_free(void* p) { ++frees; events.push_back("free"); free(p); return 0; }
+int zk_sync(void*) { events.push_back("wait"); return 0; }
+int zk_upload(void* d, const void* s, size_t n, void*) { memcpy(d, s, n); return 0; }
+int zk_memcpy_d2h(void* d, const void* s, size_t n, void*) {
+    ++reads;
+    events.push_back("wait");
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    memcpy(d, s, n);
+    return 0;
+}
+int zk_range_table(void*, int32_t, uint32_t, uint32_t, void*) { return 0; }
+int zk_fr_pad_from(void*, const void*, size_t, size_t, const void*, void*) { return 0; }
+int zk_fr_fold_prepare(void** p, const void*, size_t, void*) { events.push_back("wait"); *p = malloc(4); return 0; }
+int zk_fr_fold_prepare_queue(void** p, void* flag, const void*, size_t, void*) { *p = malloc(4); memset(flag, 0, 4); return 0; }
+int zk_fr_fold_prepared_new(void** p, void** ints, size_t, void*) { *p = malloc(4); *ints = *p; return 0; }
+const void* zk_fr_fold_prepared_ints(const void* p) { return p; }
+int zk_fr_fold_prepared_free(void* p) { events.push_back("free"); free(p); return 0; }
+int zk_fr_add_mul_s(void*, const void*, const void*, const uint32_t*, size_t, void*) { return 0; }
+int zk_fr_copy_add_first(void*, const void*, const uint32_t*, size_t, void*) { return 0; }
+int zk_fr_gather(void*, const void*, const void*, size_t, void*) { return 0; }
+int zk_fr_gather_ints(void*, void*, const void*, const void*, const void*, size_t, void*) { return 0; }
+int zk_i32_pad_from(void*, const void*, size_t, size_t, const void*, int32_t, void*) { return 0; }
+int zk_lookup_ints_suffice(size_t, size_t) { return 0; }
+int zk_lookup_multiplicities_begin(void** c, void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, void*) { *c = malloc(4); return 0; }
+int zk_lookup_multiplicities_end(void* c) { free(c); return 0; }
+int zk_lookup_open(void** o, const void*, const uint32_t*, size_t, void*) { *o = malloc(4); return 0; }
+int zk_lookup_open_drop(void* o) { events.push_back("drop"); free(o); return 0; }
+int zk_lookup_prove_begin_opened(void**, void*, const void*, const void*, const void*, const void*, const void*, const uint32_t*, const void*, const void*, int32_t, const uint32_t*,
+                                 const uint32_t*, const uint32_t*, size_t, size_t, int, int, int, void*) { events.push_back("begin"); return 1; }
+}
+"""
+
+
+def run(tmp_path, name, body):
+    src = tmp_path / (name + ".cpp")
+    src.write_text(ABI + body)
+    exe = str(tmp_path / name)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-rdynamic", "-I" + os.path.join(PKG, "host"), str(src), "-o", exe, "-L" + PKG, "-lzkllm_prover", "-lzkllm_hip",
+                    "-Wl,-rpath," + PKG], check=True)
+    return subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout.split()
+
+
+def test_first_questions_for_an_int32_form_from_two_threads_settle_it_once(tmp_path):
+    """A tensor whose producer has not been asked yet whether every element fits: the flag is read and given back once, and both threads get the form."""
+    out = run(tmp_path, "settle", r"""
+int main() {
+    FrTensor t(8);
+    t.keep_for_folds_queued();
+    const int before = frees;
+    const void* got[2];
+    std::thread a([&] { got[0] = t.kept_ints(); }), b([&] { got[1] = t.kept_ints(); });
+    a.join(); b.join();
+    printf("%d %d %d\n", (int)reads, frees - before, got[0] && got[0] == got[1]);
+    fflush(stdout);
+    _Exit(0);
+}
+""")
+    assert out == ["1", "1", "1"]

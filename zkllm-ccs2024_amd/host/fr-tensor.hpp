@@ -4,6 +4,7 @@
 #include <memory>
 #include <iomanip>
 #include <iostream>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <utility>
@@ -100,11 +101,15 @@ struct FoldCache {
     void* prepared = nullptr;
     bool tried = false;
     // set while nobody has looked yet whether the producer's int32 form holds every element (ints_for_producer_unchecked): 4 bytes
-    // of device memory that the producing kernel raises when one did not fit.  settle() reads it and drops the form if so.
+    // of device memory that the producing kernel raises when one did not fit.  The first question reads it and drops the form if so;
+    // threads may ask together.
     void* unchecked = nullptr;
-    void settle();
+    const void* kept();          // the handle, or null
     void reset();
     ~FoldCache() { reset(); }
+
+   private:
+    std::mutex mu;               // of the first question
 };
 
 class FrTensor {
@@ -191,10 +196,7 @@ class FrTensor {
     // when one does not (the kernel's launch clears it first); it is read at the first question for the form (kept_ints, a
     // fold), so the producer's caller does not wait for the kernel
     void* ints_for_producer_unchecked(void** bad_flag_dev);
-    const void* kept_ints() const {       // the handle, or null
-        if (fold_cache && fold_cache->unchecked) fold_cache->settle();
-        return fold_cache && fold_cache->prepared ? fold_cache->prepared : nullptr;
-    }
+    const void* kept_ints() const { return fold_cache ? fold_cache->kept() : nullptr; }      // the handle, or null
     // additions for stacks of `num` equally shaped matrices stored one after the other: every M x N matrix transposed,
     // and the num products x_i (M x N) * y_i (N x P)
     FrTensor transpose_stack(uint num, uint M, uint N) const;
