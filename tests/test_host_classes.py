@@ -81,3 +81,21 @@ int main() {
 }
 """)
     assert out == ["1", "1", "1"]
+
+
+def test_failed_proof_on_an_opened_table_lets_its_tensors_go_behind_the_job(tmp_path):
+    """zk_lookup_prove_begin_opened may have queued kernels before it fails: what they read is freed only when the opened job has been dropped, which waits for them."""
+    out = run(tmp_path, "order", r"""
+int main() {
+    FrTensor values(4), queries(6);
+    tLookupRangeMapping table(-2, 4, values);
+    const vector<Fr_t> u(3), v(3);
+    events.clear();
+    try { table.map_and_prove_begin(queries, Fr_t{}, Fr_t{}, Fr_t{}, u, v); } catch (const std::exception&) { events.push_back("thrown"); }
+    for (auto& e : events) printf("%s ", e.c_str());
+    fflush(stdout);
+    _Exit(0);
+}
+""")
+    assert out[-1] == "thrown"
+    assert out[out.index("begin") + 1] == "drop", out

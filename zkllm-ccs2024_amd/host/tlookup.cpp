@@ -1,7 +1,6 @@
 #include "tlookup.hpp"
 
 #include <cstring>
-#include <iterator>
 
 #include "../../include/zkllm_hip.h"
 #include "../csrc/field.hpp"
@@ -337,7 +336,9 @@ LookupPending tLookupRangeMapping::prove_begin_on(const FrTensor& S_in, const Fr
                                                   const vector<Fr_t>& u, const vector<Fr_t>& v, LookupOpened* opened) {
     const uint D = S_in.size;
     if (m.size != table.size) throw std::runtime_error("m.size != table.size");
-    std::vector<std::unique_ptr<FrTensor>> keep;
+    // (what is made for an opened job stays with it until the proof has begun: after an error its kernels may still read it, and it is waited for)
+    std::vector<std::unique_ptr<FrTensor>> own_keep;
+    std::vector<std::unique_ptr<FrTensor>>& keep = opened ? opened->keep : own_keep;
     const FrTensor *si = &S_in, *so = &S_out, *mm = &m;
     if (D != (1u << ceilLog2(D))) {
         const bool out_ints = S_out.kept_ints() && mapped_vals.kept_ints(), in_ints = out_ints && S_in.kept_ints();
@@ -352,12 +353,10 @@ LookupPending tLookupRangeMapping::prove_begin_on(const FrTensor& S_in, const Fr
     if (N != (1u << ceilLog2(N)) || si->size % N != 0) throw std::runtime_error("N is not power of 2, or D is not divisible by N");
     // S_com = S_in + r * S_out (tlookup.cu:517) is formed by the job itself; T_com is small
     if (mapped_vals.size != table.size) throw std::runtime_error("Incompatible dimensions");
-    // (an opened job's table stays with it until the proof has begun: it is being read)
-    std::unique_ptr<FrTensor> own = opened ? nullptr : combined(r);
-    const FrTensor& T_com = opened ? *opened->table : *own;
+    std::unique_ptr<FrTensor> own = opened ? std::move(opened->table) : combined(r);
+    const FrTensor& T_com = *own;
+    keep.push_back(std::move(own));
     LookupPending p = sumcheck_begin(*si, T_com, *mm, alpha, beta, u, v, si, low, so, &r, mapped_vals.kept_ints(), opened, false, opened != nullptr);
-    keep.emplace_back(opened ? std::move(opened->table) : std::move(own));
-    if (opened) std::move(opened->keep.begin(), opened->keep.end(), std::back_inserter(keep));
     p.keep = std::move(keep);
     return p;
 }
