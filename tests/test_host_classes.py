@@ -19,11 +19,17 @@ ABI = r"""
 #include <vector>
 #include "tlookup.hpp"
 static std::vector<std::string> events;
+static std::vector<const void*> job;          // what an opened job was given to read
 static std::atomic<int> frees{0}, reads{0};
 extern "C" {
 const char* zk_last_error() { return "refused"; }
 int zk_malloc(void** p, size_t n) { *p = calloc(1, n + 64); return 0; }
-int zk_free(void* p) { ++frees; events.push_back("free"); free(p); return 0; }
+int zk_free(void* p) {
+    ++frees;
+    for (const void* q : job) if (p == q) events.push_back("free of the job's");
+    free(p);
+    return 0;
+}
 int zk_sync(void*) { events.push_back("wait"); return 0; }
 int zk_upload(void* d, const void* s, size_t n, void*) { memcpy(d, s, n); return 0; }
 int zk_memcpy_d2h(void* d, const void* s, size_t n, void*) {
@@ -39,7 +45,7 @@ int zk_fr_fold_prepare(void** p, const void*, size_t, void*) { events.push_back(
 int zk_fr_fold_prepare_queue(void** p, void* flag, const void*, size_t, void*) { *p = malloc(4); memset(flag, 0, 4); return 0; }
 int zk_fr_fold_prepared_new(void** p, void** ints, size_t, void*) { *p = malloc(4); *ints = *p; return 0; }
 const void* zk_fr_fold_prepared_ints(const void* p) { return p; }
-int zk_fr_fold_prepared_free(void* p) { events.push_back("free"); free(p); return 0; }
+int zk_fr_fold_prepared_free(void* p) { return zk_free(p); }
 int zk_fr_add_mul_s(void*, const void*, const void*, const uint32_t*, size_t, void*) { return 0; }
 int zk_fr_copy_add_first(void*, const void*, const uint32_t*, size_t, void*) { return 0; }
 int zk_fr_gather(void*, const void*, const void*, size_t, void*) { return 0; }
@@ -50,8 +56,12 @@ int zk_lookup_multiplicities_begin(void** c, void*, void*, const void*, const vo
 int zk_lookup_multiplicities_end(void* c) { free(c); return 0; }
 int zk_lookup_open(void** o, const void*, const uint32_t*, size_t, void*) { *o = malloc(4); return 0; }
 int zk_lookup_open_drop(void* o) { events.push_back("drop"); free(o); return 0; }
-int zk_lookup_prove_begin_opened(void**, void*, const void*, const void*, const void*, const void*, const void*, const uint32_t*, const void*, const void*, int32_t, const uint32_t*,
-                                 const uint32_t*, const uint32_t*, size_t, size_t, int, int, int, void*) { events.push_back("begin"); return 1; }
+int zk_lookup_prove_begin_opened(void**, void*, const void* S, const void* Si, const void* So, const void* Soi, const void* mi, const uint32_t*, const void* T, const void* m, int32_t,
+                                 const uint32_t*, const uint32_t*, const uint32_t*, size_t, size_t, int, int, int, void*) {
+    for (const void* p : {S, Si, So, Soi, mi, T, m}) if (p) job.push_back(p);
+    events.push_back("begin");
+    return 1;
+}
 }
 """
 
@@ -62,7 +72,7 @@ def run(tmp_path, name, body):
     exe = str(tmp_path / name)
     subprocess.run(["g++", "-O1", "-std=c++17", "-pthread", "-rdynamic", "-I" + os.path.join(PKG, "host"), str(src), "-o", exe, "-L" + PKG, "-lzkllm_prover", "-lzkllm_hip",
                     "-Wl,-rpath," + PKG], check=True)
-    return subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout.split()
+    return subprocess.run([exe], check=True, capture_output=True, text=True, timeout=60).stdout.splitlines()
 
 
 def test_first_questions_for_an_int32_form_from_two_threads_settle_it_once(tmp_path):
@@ -75,7 +85,7 @@ int main() {
     const void* got[2];
     std::thread a([&] { got[0] = t.kept_ints(); }), b([&] { got[1] = t.kept_ints(); });
     a.join(); b.join();
-    printf("%d %d %d\n", (int)reads, frees - before, got[0] && got[0] == got[1]);
+    printf("%d\n%d\n%d\n", (int)reads, frees - before, got[0] && got[0] == got[1]);
     fflush(stdout);
     _Exit(0);
 }
@@ -92,10 +102,10 @@ int main() {
     const vector<Fr_t> u(3), v(3);
     events.clear();
     try { table.map_and_prove_begin(queries, Fr_t{}, Fr_t{}, Fr_t{}, u, v); } catch (const std::exception&) { events.push_back("thrown"); }
-    for (auto& e : events) printf("%s ", e.c_str());
+    for (auto& e : events) puts(e.c_str());
     fflush(stdout);
     _Exit(0);
 }
 """)
-    assert out[-1] == "thrown"
-    assert out[out.index("begin") + 1] == "drop", out
+    assert out[-1] == "thrown" and out[out.index("begin") + 1] == "drop"
+    assert out.count("free of the job's") >= 3          # padded queries and outputs, the combined table
