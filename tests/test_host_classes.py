@@ -109,3 +109,20 @@ int main() {
 """)
     assert out[-1] == "thrown" and out[out.index("begin") + 1] == "drop"
     assert out.count("free of the job's") >= 3          # padded queries and outputs, the combined table
+
+
+def test_constructor_of_a_mapping_table_leaves_nothing_queued_or_unsettled(tmp_path):
+    """A table that a caller has constructed is complete and only read from then on, whatever stream or thread goes on with it; one made with `queued` waits for nothing."""
+    out = run(tmp_path, "made", r"""
+int main() {
+    FrTensor values(4);
+    tLookupRangeMapping table(-2, 4, values);
+    printf("%d\n%d\n", (int)events.size(), table.mapped_vals.fold_cache->unchecked == nullptr);
+    events.clear();
+    tLookupRangeMapping queued(-2, 4, values, tLookupRangeMapping::queued);
+    printf("%d\n", (int)events.size());
+    fflush(stdout);
+    _Exit(0);
+}
+""")
+    assert out == ["1", "1", "0"]

@@ -410,7 +410,7 @@ int zkp_range_prove(void* S, int low, u32 len, const u32* alpha, const u32* beta
 // tLookupRangeMapping: y and m handles are returned through y_out / m_out; prove when final_claim != NULL
 int zkp_mapping(void* S_in, int low, u32 len, void* mvals, const u32* r, const u32* alpha, const u32* beta, const u32* u, const u32* v, void** y_out, void** m_out, u32* final_claim) {
     ZKP_TRY
-    tLookupRangeMapping t(low, len, FT(mvals));
+    tLookupRangeMapping t(low, len, FT(mvals), tLookupRangeMapping::queued);
     if (final_claim && FT(S_in).size > 1) {          // the proof ends behind the outputs that it was begun on
         const int k = (int)ceilLog2(FT(S_in).size);
         auto p = t.map_and_prove_begin(FT(S_in), fr1(r), fr1(alpha), fr1(beta), frs(u, k), frs(v, k));

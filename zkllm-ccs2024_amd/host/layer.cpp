@@ -452,7 +452,7 @@ FrTensor oproj_block(const LayerConfig& c, const Weight& o, const FrTensor& attn
 FfnBlock::FfnBlock(const LayerConfig& c, const Weight& up, const Weight& gate, const Weight& down, const FrTensor& swiglu_values, const FrTensor& input)
     : c(c), up(up), gate(gate), down(down), input(input), up_layer(c.embed_dim, c.hidden_dim, FrTensor::view(up.weight)),
       gate_layer(c.embed_dim, c.hidden_dim, FrTensor::view(gate.weight)), down_layer(c.hidden_dim, c.embed_dim, FrTensor::view(down.weight)), up_rescale(c.sf_linear),
-      gate_rescale(c.sf_gate), hidden_rescale(c.sf_linear), down_rescale(c.sf_linear), swiglu(c.swiglu_low, c.swiglu_len, swiglu_values) {
+      gate_rescale(c.sf_gate), hidden_rescale(c.sf_linear), down_rescale(c.sf_linear), swiglu(c.swiglu_low, c.swiglu_len, swiglu_values, tLookupRangeMapping::queued) {
     up_rescale.lean = gate_rescale.lean = hidden_rescale.lean = down_rescale.lean = true;
     up_rescale.out_ints_lazy = gate_rescale.out_ints_lazy = hidden_rescale.out_ints_lazy = true;      // read by the activation lookup, the product and the down projection's proof
 }

@@ -61,7 +61,10 @@ static FrTensor make_mapped(uint len, const FrTensor& mvals) {
     ZKC(zk_fr_pad_from(out.gpu_data, mvals.gpu_data, mvals.size, out.size, mvals.gpu_data + (mvals.size - 1), nullptr));
     return out;
 }
-tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mvals) : tLookupRange(low, len), mapped_vals(make_mapped(len, mvals)) {
+tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mvals) : tLookupRangeMapping(low, len, mvals, queued) {
+    (void)mapped_vals.kept_ints();          // waits
+}
+tLookupRangeMapping::tLookupRangeMapping(int low, uint len, const FrTensor& mvals, Queued) : tLookupRange(low, len), mapped_vals(make_mapped(len, mvals)) {
     mapped_vals.keep_for_folds_queued();          // examined once: outputs of operator() carry an int32 form when these are 32-bit integers
 }
 

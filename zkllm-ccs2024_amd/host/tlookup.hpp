@@ -87,6 +87,9 @@ class tLookupRangeMapping : public tLookupRange {
    public:
     FrTensor mapped_vals;
     tLookupRangeMapping(int low, uint len, const FrTensor& mapped_vals);
+    // addition: without the wait for the table, for a caller that goes on on the default stream
+    enum Queued { queued };
+    tLookupRangeMapping(int low, uint len, const FrTensor& mapped_vals, Queued);
 
     using tLookupRange::prep;
 

@@ -29,14 +29,14 @@ zkSoftmax::zkSoftmax(const vector<uint>& bs, uint L, uint M, unsigned long scali
         FrTensor mapped_values(bs[i]);
         const double step = static_cast<double>(Bs[i]) / scale;
         ZKC(zk_softmax_table(mapped_values.gpu_data, zkd::log_det(thetas[i - L]), step, bs[i], nullptr));
-        other_segments.emplace_back(0, bs[i], mapped_values);
+        other_segments.emplace_back(0, bs[i], mapped_values, tLookupRangeMapping::queued);
     }
     for (uint i = K - M; i < K; ++i) {
         // indicator of digit 0 (`int mvals[bs[i]] = {1}` in the reference)
         std::vector<int> mvals(bs[i], 0);
         mvals[0] = 1;
         FrTensor mapped_values(bs[i], mvals.data());
-        other_segments.emplace_back(0, bs[i], mapped_values);
+        other_segments.emplace_back(0, bs[i], mapped_values, tLookupRangeMapping::queued);
     }
 }
 
