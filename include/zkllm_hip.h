@@ -232,7 +232,7 @@ int zk_matmul_sumcheck(uint32_t* claim_host, uint32_t* polys_host, uint32_t* fin
 
 /* ---- G1 tensors (g1-tensor.cu) ------------------------------------------------------------------------ */
 /* Points lie on the curve y^2 = x^3 + 4 over F_p or are infinity.  Nothing checks that, as in the reference; for a point that does not, the results are
- * not specified: additions in the openings use the curve's coefficient and that its group has odd order (the reference's use neither). */
+ * not specified: additions in the openings and in zk_g1_commit_int use the curve's coefficient and that its group has odd order (the reference's use neither). */
 int zk_g1_fill(void* out, const uint32_t* point36, size_t n, void* stream);               /* G1Jacobian_assign_broadcast :140 */
 int zk_g1_neg(void* out, const void* a, size_t n, void* stream);                          /* G1_jacobian_elementwise_minus :192 */
 int zk_g1_affine_neg(void* out, const void* a_affine, size_t n, void* stream);            /* G1_affine_elementwise_minus :105 */
