@@ -188,6 +188,34 @@ def test_products_in_29_bit_limbs_stay_in_range_and_match_big_integers(tmp_path)
             assert -eps <= value(limbs) <= P_MOD + eps and (value(limbs) - exact * rinv) % P_MOD == 0
 
 
+def test_reductions_in_29_bit_limbs_stay_in_range_and_match_big_integers(tmp_path):
+    """fr29_mul and wide29_redc against big integers: limbs all zero and all ones, the top limb at its limit (below 2^30, and the product below 2^523), sums as large as the form holds (below 2^522), columns before and after a
+    carry pass.  What is returned is v / 2^261 mod r, limbs normalised, below v / 2^261 + (1 + 2^-29) r: the last two limbs of the reduction add less than r, the seven before them less than 2^-29 r."""
+    src = tmp_path / "fr29.cpp"
+    src.write_text('#include <cstdio>\n#include <initializer_list>\n#include "fr29.hpp"\nusing namespace zk;\nint main() { Fr29 a, b; Wide29 w; unsigned long long c; auto wr = [](const Fr29& x) { for (int i = 0; i < 9; ++i) printf("%d ", x.l[i]); puts(""); };'
+                   ' int kind; while (scanf("%d", &kind) == 1) if (kind == 0) { for (Fr29* x : {&a, &b}) for (int i = 0; i < 9; ++i) if (scanf("%d", &x->l[i]) != 1) return 1; wr(fr29_mul(a, b)); }'
+                   ' else { for (int i = 0; i < 18; ++i) { if (scanf("%llu", &c) != 1) return 1; w.c[i] = c; } wr(wide29_redc(w)); } }\n')
+    csrc = os.path.join(ROOT, "zkllm-ccs2024_amd", "csrc")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + csrc, str(src), "-o", str(tmp_path / "fr29")], check=True)
+    m29, rng = (1 << 29) - 1, random.Random(43)
+    limbs = lambda x, n: [(x >> (29 * i)) & m29 for i in range(n - 1)] + [x >> (29 * (n - 1))]
+    value = lambda l: sum(v << (29 * i) for i, v in enumerate(l))
+    ops = [limbs(x, 9) for x in (0, 1, m29, R_MOD, R_MOD - 1, 2 * R_MOD - 1, (1 << 256) - 1, (1 << 261) - 1, (1 << 232) - 1)] + [[m29] * 8 + [(1 << 30) - 1], [0] * 8 + [(1 << 30) - 1], [m29] + [0] * 8]
+    ops += [limbs(rng.randrange(R_MOD), 9) for _ in range(25)]
+    wide = [limbs(x, 18) for x in (0, 1, m29, R_MOD << 261, (1 << 522) - 1, (1 << 522) - R_MOD, (1 << 261) - 1, (1 << 522) - (1 << 261))]
+    wide += [[36 * m29 * m29] * 16 + [0, 0], [4 * 9 * (1 << 58) + m29] * 9 + [0] * 9, [0] * 16 + [9 * m29 * m29 >> 4, 0]]
+    wide += [limbs(rng.randrange(1 << 522), 18) for _ in range(200)]
+    assert all(value(w) < 1 << 522 for w in wide)
+    cases = [([0] + a + b, value(a) * value(b)) for a in ops for b in ops if value(a) * value(b) < 1 << 523] + [([1] + w, value(w)) for w in wide]
+    out = subprocess.run([str(tmp_path / "fr29")], input="\n".join(" ".join(map(str, c)) for c, _ in cases), check=True, capture_output=True, text=True).stdout.splitlines()
+    rinv = pow(2, -261, R_MOD)
+    assert len(out) == len(cases)
+    for (_, v), line in zip(cases, out):
+        got = list(map(int, line.split()))
+        assert all(0 <= x <= m29 for x in got[:8]) and got[8] >= 0
+        assert (value(got) - v * rinv) % R_MOD == 0 and value(got) << 290 < (v << 29) + (((1 << 29) + 1) * R_MOD << 261)
+
+
 def test_complete_projective_additions_match_the_affine_group_law():
     """p29_add (the bucket reductions' addition: no special cases), run on the CPU, against the affine group law: random points, a point and
     itself, its opposite, infinity on either side and both, and points outside the subgroup of order r, those of order three among them."""

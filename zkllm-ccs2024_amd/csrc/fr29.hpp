@@ -8,7 +8,7 @@
 //
 // Why: with 29-bit limbs a column of the schoolbook product (9 products below 2^58) fits a 64-bit accumulator, so a limb
 // product is ONE v_mad_u64_u32 with no add-with-carry behind it and no carry flag to wait for; r = 1 mod 2^29, so the
-// reduction's multiplier is the negated low limb (no product), and its result needs no conditional subtraction.  About 250
+// reduction's multiplier is the low limb or its negative (no product, fr29_redc), and its result needs no conditional subtraction.  About 220
 // vector instructions per product against 370 in the 32-bit form (field.hpp: 120 multiply-adds, 120 add-with-carry, 130
 // others), and a product that is only summed (Wide29) costs its 81 multiply-adds and a share of a carry pass.
 #pragma once
@@ -88,7 +88,7 @@ template <int NCOL, typename Col> ZK_HD Fr29 fr29_redc(Col col) {
     }
     return t;
 }
-// a b 2^-261 mod r; limbs 0..7 of both below 2^29, limb 8 below 2^30.  Result below a b / 2^261 + r, limbs normalised.
+// a b 2^-261 mod r; limbs 0..7 of both below 2^29, limb 8 below 2^30, a b below 2^523.  Result below a b / 2^261 + (1 + 2^-29) r, limbs normalised.
 ZK_HD Fr29 fr29_mul(const Fr29& a, const Fr29& b) {
     return fr29_redc<17>([&](int k) {
         int64_t s = 0;
@@ -303,7 +303,7 @@ ZK_HD void wide29_carry(Wide29& w) {
         w.c[k] &= (uint64_t)R29M;
     }
 }
-// sum * 2^-261 mod r, below sum / 2^261 + r (the carry pass runs first: every column below 2^29 but the last)
+// sum * 2^-261 mod r, below sum / 2^261 + (1 + 2^-29) r (the carry pass runs first: every column below 2^29 but the last)
 ZK_HD Fr29 wide29_redc(Wide29& w) {
     wide29_carry(w);
     return fr29_redc<18>([&](int k) { return (int64_t)w.c[k]; });
