@@ -249,7 +249,8 @@ def test_open_value_and_g1_transcript(pv, orc, n, m):
     assert (norm(orc, proof) == norm(orc, exp_proof)).all()
 
 
-@pytest.mark.parametrize("n,val", [(300, 70000), (5000, -3), (5000, 0)])
+# up to 256: k_msm_few, with eight windows a wave (up to 64 elements), four (128) or two; 257: sorted lists
+@pytest.mark.parametrize("n,val", [(64, 7), (65, -3), (128, 70000), (129, -3), (200, 2 ** 31 - 1), (256, 70000), (257, 70000), (300, 70000), (5000, -3), (5000, 0)])
 def test_open_with_equal_scalars(pv, orc, n, val):
     """Every scalar in the same bucket of every window (norm weights share their high bytes; here all bytes): the
     bucket sums must not depend on how the elements spread over the buckets."""
@@ -267,10 +268,10 @@ def test_open_with_equal_scalars(pv, orc, n, val):
     assert (norm(orc, proof) == norm(orc, exp_proof)).all()
 
 
-@pytest.mark.parametrize("counts", [[1, 64], [96, 97, 107], [400, 113], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
+@pytest.mark.parametrize("counts", [[1, 64], [32] * 3, [127, 1], [97, 32], [200, 55], [97, 97, 62], [1, 255], [128] * 2, [256, 1], [200, 57], [96, 97, 107], [400, 113], [97, 97, 97, 97, 97, 27], [150, 600, 97, 1200, 98, 255, 96, 400], [97] * 42, [2048, 2048], [128] * 20 + [64] * 16])
 def test_open_with_several_digits_shared_by_many_scalars(pv, orc, counts):
-    """Few scalars (256 at most, a path of its own) and many: buckets about the size from which a workgroup shares them out, whose ends fall inside and at
-    the ends of the lanes' shares."""
+    """Few scalars (256 at most, a path of its own with eight, four or two windows a wave) and many: buckets that span one lane's share to all of them, whose ends fall
+    inside and at the ends of the shares; buckets about the size from which a list is cut into pieces."""
     n = sum(counts)
     gens = oracle_gens(orc, 41 + n, n)
     t = np.repeat(np.arange(1, len(counts) + 1), counts)

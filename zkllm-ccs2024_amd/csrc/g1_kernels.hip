@@ -738,8 +738,8 @@ __global__ void __launch_bounds__(GT) k_msm_recode(const RecodeBatch rb, size_t 
 // The end of a list of points in bucket order that a wave's lanes have divided evenly (lane t the t-th share).  x: the sum of the last part of
 // the lane's share, which belongs to bucket b; begun: the bucket begins in this share (or the share is empty); whole: it ends with this
 // share; lacks: bucket `split`, the first part's, went out already without the shares before this one.  A segmented inclusive scan, as
-// long as a bucket spans further lanes, then the sums to `out` (added to what is there unless fresh).  All lanes call it; pool: 42 x 64 words.
-__device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, P29 x, bool begun, bool whole, uint32_t b, bool lacks, uint32_t split, P29* __restrict__ out, bool fresh, uint32_t t) {
+// long as a bucket spans further lanes, then the sums to `out`.  All lanes call it; pool: 42 x 64 words.
+__device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, P29 x, bool begun, bool whole, uint32_t b, bool lacks, uint32_t split, P29* __restrict__ out, uint32_t t) {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(&x);
     for (uint32_t sd = 1; sd < (uint32_t)MSL && !__all(begun); sd <<= 1) {
         __syncthreads();
@@ -760,10 +760,7 @@ __device__ __forceinline__ void bucket_shares_merge(uint32_t* pool, P29 x, bool 
 #pragma unroll
     for (int l = 0; l < P29_WORDS; ++l) pool[l * MSL + t] = src[l];
     __syncthreads();
-    if (whole) {
-        if (!fresh) x = p29_add<false>(out[b], x);
-        out[b] = x;
-    }
+    if (whole) out[b] = x;
     if (lacks) {
         P29 y;
         uint32_t* py = reinterpret_cast<uint32_t*>(&y);
@@ -965,7 +962,7 @@ __global__ void __launch_bounds__(MSL) k_msm_merge(const SortSpace sp) {
 // Bucket sums of few elements: the 8-bit digits taken as two signed 4-bit digits each, so that a sum has 512 buckets (64 windows
 // of 8) instead of 4096 and the walk over its buckets, which is most of such a sum's work, fits two waves instead of sixteen.  A wave
 // takes nw windows, sorts their elements by bucket in LDS and divides that list evenly over its lanes, whatever the digits are.
-// nw (1, 2, 4 or 8) gives a lane about eight elements, so that the scan behind them costs less than they do.
+// nw (8 up to 64 elements, 4 up to 128, else 2) gives a lane about eight elements, so that the scan behind them costs less than they do.
 // FEW_MAX: an element costs 64 additions here and 32 there, a sum 512 buckets here and 4096 there; an opening of 8 x 512 alone takes
 // 1.00 ms here, 0.93 sorted, one of 4 x 256 0.91 here.
 static constexpr int FEW_MAX = 256, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS = FEW_WINDOWS * FEW_T;
@@ -973,7 +970,7 @@ static constexpr int FEW_MAX = 256, FEW_WINDOWS = 2 * MW, FEW_T = 8, FEW_BUCKETS
 __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_few(P29* __restrict__ buckets, const MsmDesc* __restrict__ descs, uint32_t nw) {
     __shared__ uint32_t cnt[MSL], off[MSL], cursor[MSL];
     __shared__ uint32_t pool[P29_WORDS * MSL];      // the sorted list (u16), then the points of the shares' scan
-    static_assert(FEW_MAX <= 4096 && FEW_MAX * 2 <= P29_WORDS * MSL * 4 && 8 * FEW_T == MSL, "list entries, the pool and a lane for each bucket");
+    static_assert(FEW_MAX <= 4096 && 8 * MSL * 2 <= P29_WORDS * MSL * 4 && 8 * FEW_T == MSL, "list entries, the pool and a lane for each bucket");
     uint16_t* list = reinterpret_cast<uint16_t*>(pool);
     const MsmDesc d = descs[blockIdx.y];
     const A29* __restrict__ A = d.base;
@@ -1034,7 +1031,7 @@ __global__ void __launch_bounds__(MSL) __attribute__((amdgpu_waves_per_eu(2, 2))
         if (en & 0x8000u) pt.y = fq29_neg(pt.y);
         x29_add_mixed(acc29, pt);
     }
-    bucket_shares_merge(pool, p29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, true, t);
+    bucket_shares_merge(pool, p29_from_x29(acc29), start, p1 > p0 && p1 == b_end, b, lacks, split, out, t);
 }
 // The sums of a list from the raw buckets of all their windows, in two launches, three for windows of more than 128 buckets.  k_msm_windows: a wave takes 128 buckets,
 // sum_b (b + 1) B[b]: each four lanes the running sums over eight neighbouring buckets (fourteen additions), then a tree over the sixteen of them in which one
@@ -2074,7 +2071,7 @@ static int bucket_sums_queue(std::vector<MsmDesc> d, const std::vector<G1Jac*>& 
     if (rc) return rc;
     if (plan.digits.nwh == 0) {
         uint32_t nw = 8;
-        while (nw > 1 && nw * count_max > 8 * MSL) nw /= 2;
+        while (nw * count_max > 8 * MSL) nw /= 2;            // 2 at FEW_MAX
         Scratch& buckets = arena.add(sizeof(P29) * (size_t)n_msm * FEW_BUCKETS);
         if (buckets.rc) return buckets.rc;
         rc = join_streams(st, aux, events);
@@ -2344,7 +2341,6 @@ int zk_g1_normalize(void* out, const void* in, size_t n, void* st) {
     return 0;
 }
 
-// levels that k_msm_table_first takes: as many entries a window as two waves a SIMD have lanes for
 // the growth of a window from h to `target` entries, at most GROW_MAX steps
 static std::vector<GrowSpec> grow_steps(uint32_t h, uint32_t target) {
     std::vector<GrowSpec> v;
