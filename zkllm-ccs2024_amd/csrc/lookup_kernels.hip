@@ -1553,13 +1553,14 @@ k_sum_rounds(Fr* __restrict__ partials, const RoundsArgs a) {
     }
 }
 
-// The same for launches that have a compute unit for each of their workgroups (n <= 2^16): what takes the time there is a round's chain and the issue
+// The same for launches over at most 2^16 elements, 256 blocks of them: what takes the time there is a round's chain and the issue
 // of one compute unit.  A workgroup has two of the tensors (blockIdx.y: A, S | B, T | m, B, so that three compute units share a block of elements) and keeps
 // every round's level of them in LDS, and the folds run ahead of the sums: the large ones on all lanes with a barrier each, those of at
 // most 32 pairs on the first wave alone, without one, while the others take the sums of the rounds in front.  A fold is one product deep where a round with its sums was two and a
 // barrier.  A unit of work is sixteen pairs of a round: rows of sixteen lanes for x0 y0 | x1 y1 | dx dy (times E), the fourth row for the sums of a0 and a1.
 // The last launch, of one block, also does what k_finish_rounds does for the rounds ahead of it, a workgroup a sum beside its own, and its own sums go straight to
-// where the host reads them.  Seven rounds from 2^14 elements: 17.4 us, from 2^7: 14.6 us (30.6 and 20.6 with all five tensors in one workgroup of sixteen waves and every round's sums ahead of the next round).
+// where the host reads them.  Seven rounds from 2^14 elements: 17.4 us, from 2^7: 14.6 us alone and 17.7 with the end of all rounds' sums, which took a launch of 7.8 (30.6 and 20.6 with all five tensors in one workgroup
+// of sixteen waves and every round's sums ahead of the next round).
 static constexpr int LV_T = 512, LV_UNITS = RM_P / 32 + RM_P / 64 + RM_P / 128 + RM_ROUNDS;      // units: 8, 4, 2, 1, 1, ...
 __device__ __forceinline__ uint32_t lv_units(uint32_t half) { return (half + 15u) / 16u; }
 // sums null: the partial sums go to memory.  rows_from: the first of the workgroups (blockIdx.y) that finish the `before` rounds of fin
@@ -2989,7 +2990,7 @@ static bool limbs29() { static const bool on = [] { const char* e = getenv("ZKLL
 // all rounds of the lookup sumcheck; sums land in job.sums
 // A == nullptr with a hint source: 1 / (S + beta) has not been written anywhere; a large first round computes it on
 // the fly, anything else writes it out first.
-// Queues rounds r .. rounds - 1 of a sumcheck over n elements in launches of k_sum_rounds.  hadamard: two tensors A, S; else a lookup whose
+// Queues rounds r .. rounds - 1 of a sumcheck over n elements in launches of k_sum_rounds and k_level_rounds.  hadamard: two tensors A, S; else a lookup whose
 // phase-2 rounds start at round n1.  The rounds' partial sums go behind part_at and are noted in `fin`; finished: the last launch did what k_finish_rounds does.
 // eq_prefix: every round reads E's prefix.
 static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, const Fr* B, const Fr* T, const Fr* m, const Fr* E, const Fr& beta, const uint32_t* v, size_t n, int r,
@@ -2997,9 +2998,10 @@ static int rounds_queue(SumJob& job, bool hadamard, const Fr* A, const Fr* S, co
     const uint32_t per1 = hadamard ? 3u : 5u;
     uint32_t e_span = 0;
     while (r < rounds) {
-        // While there are more workgroups than compute units a launch is throughput, and a round of few pairs a workgroup costs as much as
-        // a full one: three rounds then; all that the workgroup's elements allow, evenly split over the launches, where each has a unit
-        // of its own.
+        // While a block of elements has no compute unit of its own a launch is throughput, and a round of few pairs a workgroup costs as much as
+        // a full one: three rounds then (k_sum_rounds); else all that the workgroup's elements allow, evenly split over the launches.
+        // Over a table (phase 2) a block of k_level_rounds is three workgroups, of which a unit holds two: at 2^16 elements they no longer run all at once,
+        // but three rounds of k_sum_rounds first take longer all the same: all rounds from 2^16 on 53 us and 58 with them, from 2^15 39 and 48.
         const int left = rounds - r;
         int R = std::min(RM_WIDE_ROUNDS, left), P = RM_WIDE_P;
         if (n <= (size_t)256 * RM_P) {
