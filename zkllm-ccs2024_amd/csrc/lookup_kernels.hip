@@ -2921,9 +2921,10 @@ static int sumjob_need_m(SumJob& job) {
 // whether a job over `rounds` rounds whose table is eq(u_eq, .) of rounds - 1 challenges (index bit j <-> u_eq[j]) can read its prefix throughout: no challenge is 1
 static bool eq_prefix_on() { static const bool on = [] { const char* e = getenv("ZKLLM_EQ_PREFIX"); return !(e && e[0] == '0'); }(); return on; }
 static bool eq_prefix_possible(const uint32_t* u_eq, int rounds) {
-    const Fr one = big_one_mont<8>();
-    for (int r = 1; r < rounds; ++r)
-        if (is_zero(sub(one, to_mont(load_fr(u_eq + 8 * (size_t)(r - 1)))))) return false;      // as residues: a challenge may come unreduced
+    for (int r = 1; r < rounds; ++r) {          // a challenge may come unreduced: 1, r + 1 or 2 r + 1, whose lowest limbs are 1 to 3
+        const Fr u = load_fr(u_eq + 8 * (size_t)(r - 1));
+        if (u.v[0] <= 3u && equal(to_mont(u), big_one_mont<8>())) return false;
+    }
     return eq_prefix_on();
 }
 // its constants
