@@ -35,12 +35,12 @@ VALU_PEAK_TOPS = 256 * 4 * 16 * 2.4e9 / 1e12
 # WRITE_SIZE on the kernel alone (python3 bench.py --pmc-probe; summary in profiles/k_open_fold29_pmc_traffic.txt), each
 # counter scaled by what it reads for zk_fr_add over 2^24 elements (1 GiB read, 512 MiB written).  It holds for launches of
 # that size; `traffic` of the in-layer entry, whose launches are of every size, is left null and the algorithmic figure given.
-FOLD_TRAFFIC_BYTES_PER_PAIR_AT_262144 = 542.9      # (43895 KiB x 2.000 fetched + 51200 KiB written) / 262144 pairs, profiles/k_open_fold29_pmc_traffic.txt
+FOLD_TRAFFIC_BYTES_PER_PAIR_AT_262144 = 542.4      # (43827 KiB x 2.000 fetched + 51195 KiB written) / 262144 pairs, profiles/k_open_fold29_pmc_traffic.txt
 FOLD_ALGO_BYTES_PER_PAIR = 2 * 112 + 112 + 3 * 32      # two points in, one out (affine, 29-bit limbs: 112 B), two scalars in, one out
 # the same for the table-driven folds, from profiles/fr_mul_fold_msm_pmc.txt (each kernel alone): k_open_fold_comb<1> at 262144 pairs
-# (500607 KiB x 2 fetched + 36864 KiB written) and k_open_fold_jump at 65536 results = 7 x 65536 pairs (821582 KiB x 2 + 9216 KiB)
-COMB_TRAFFIC_BYTES_PER_PAIR = (500607 * 2 + 36864) * 1024 / 262144
-JUMP_TRAFFIC_BYTES_PER_PAIR = (821582 * 2 + 9216) * 1024 / (7 * 65536)
+# (500856 KiB x 2 fetched + 36864 KiB written) and k_open_fold_jump at 65536 results = 7 x 65536 pairs (820898 KiB x 2 + 9216 KiB)
+COMB_TRAFFIC_BYTES_PER_PAIR = (500856 * 2 + 36864) * 1024 / 262144
+JUMP_TRAFFIC_BYTES_PER_PAIR = (820898 * 2 + 9216) * 1024 / (7 * 65536)
 MAD_PER_FP_MUL = 300                                   # 2 * 12^2 + 12 limb products of a 381-bit Montgomery product
 MAD_PER_FR_MUL = 136                                   # 2 * 8^2 + 8
 
@@ -550,7 +550,7 @@ def main():
                     "with each other, with the openings and with the main stream; alone the kernel is bound by instruction issue (4 450 lane instructions per "
                     "quad) and its table gathers, not by these bytes (profiles/layer_c5_seq2048_alone_valu_bytes.txt)"}
     if lr_launches:
-        # ~1750 vector instructions per pair (profiles/fr_mul_fold_msm_pmc.txt: SQ_INSTS_VALU of the kernel alone) of which 855 are limb multiply-adds
+        # ~1700 vector instructions per pair (profiles/fr_mul_fold_msm_pmc.txt: SQ_INSTS_VALU of the kernel alone); 855 limb multiply-adds with a product's reduction counted by r alone (891 as executed)
         lr_tops = lr_pairs * 855.0 / (lr_ms * 1e-3) / 1e12
         out["roofline_lookup_later_rounds"] = {
             "kernel": "k_lookup_round29 (phase-1 rounds of the lookup sumchecks behind the first, one lane per pair, 29-bit limbs; every launch of the timed layers)",
