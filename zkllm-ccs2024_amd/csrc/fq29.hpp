@@ -7,7 +7,7 @@
 // Why: with 29-bit limbs a column of the schoolbook product (at most 28 products of 58 bits) fits a 64-bit
 // accumulator, so a limb product is ONE v_mad_i64_i32 with no carry instruction behind it, the reduction needs no
 // final conditional subtraction (R' is 2^24 times larger than p), and additions / subtractions are limb-wise with a
-// shift-and-mask carry pass -- no carry flags, which on this chip cost wait states.  392 multiply-adds and about 85
+// shift-and-mask carry pass -- no carry flags, which on this chip cost wait states.  395 multiply-adds and 85
 // other instructions per product, against 288 + 288 add-with-carry + about 150 in the 32-bit form (field.hpp).
 //
 // The same formulas as g1.hpp (dbl-2009-l, madd-2007-bl; bls12-381.cu:1361-1464), on points that carry an explicit

@@ -216,7 +216,7 @@ static constexpr int GROW_MAX = 12;
 struct GrowCentres { uint32_t full_n, top_n; uint16_t full[GROW_MAX], top[GROW_MAX]; };
 // The first entries of every window (those that it has) and the centres of its growth out of the normalised bases (window-major), a lane an entry: doublings and additions
 // of the base along the bits of the multiple, and an inversion.  A step of k_msm_table_grow takes what one lane's inversion and
-// its launch take however few its entries are: the first sixteen of 8192 rows took 330 us in four steps that doubled them, and take 170 here.
+// its launch take however few its entries are: the first sixteen of 8192 rows took 330 us in four steps that doubled them, and take 170 here, 200 with the five centres.
 // The centres come first: a wave of them, all of one multiple, takes longest.
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_first(const MsmTable T, const G1Affine* __restrict__ bases, uint32_t first, const GrowCentres gc) {
     const size_t rows_full = (size_t)(T.nwin - 1) * T.ngen, n_full = rows_full * gc.full_n, n_centres = n_full + T.ngen * gc.top_n;
@@ -245,10 +245,10 @@ __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2)))
     (full ? T.tab + r * T.half : T.tab + rows_full * T.half + (r - rows_full) * T.top)[d - 1u] = out;
 }
 // A step of the windows' growth (GrowSpec: of the full windows, and of the highest): a lane's pairs share one inversion (about 26 products), and a pair takes nine products for its two entries
-// and 280 bytes an entry.  Equal and opposite points and infinity are told apart from the coordinates, whatever the generators are.
+// and 320 bytes an entry (1419 MB fetched and 1267 written for 8.4 M).  Equal and opposite points and infinity are told apart from the coordinates, whatever the generators are.
 // The products before a pair wait in the slot of one of its entries.  Entry by entry, each with a denominator of its own and the windows doubled from launch to launch, 8.4 M entries took 2.0 ms
 // at 56 % of the issue slots (526 bytes an entry); three entries for one
-// from launch to launch this way they take 1.32 ms at 58 % (11008 x 4096 of 13 bits; the whole commitment 10.68 -> 10.18 ms).  Sending for the next pair's points early spills and gains nothing.
+// from launch to launch this way they take 1.3 to 1.4 ms, the large launches at 60 to 64 % (11008 x 4096 of 13 bits; the whole commitment 10.68 -> 10.18 ms).  Sending for the next pair's points early spills and gains nothing.
 __global__ void __launch_bounds__(GT) __attribute__((amdgpu_waves_per_eu(2, 2))) k_msm_table_grow(const MsmTable T, const GrowSpec full, const GrowSpec top, uint32_t n, uint32_t per_lane) {
     const uint32_t base = blockIdx.x * GT * per_lane + threadIdx.x;
     if (base >= n) return;
