@@ -2020,7 +2020,9 @@ static int join_streams(hipStream_t st, hipStream_t aux, std::vector<hipEvent_t>
 // them have a scalar other than zero; total: elements of all of them.
 struct SumsPlan { DigitPlan digits{}; uint32_t hb = 0, most = 0, group = 0, state_words = 0; size_t total = 0; uint32_t* state = nullptr; };
 // Windows of a half, and the longest list of one lane: two and a half times the mean of the wide windows' buckets, which cuts outliers alone; buckets a bit narrower have twice the mean,
-// start first and leave the shorter ones to fill up.
+// start first and leave the shorter ones to fill up.  Nothing below 32 is cut, or below 12 where all lists run at once (two waves a SIMD) and the launch takes what its longest list does: opened without a
+// fold of rows, small integers share the few digits that they have, and 512 of them take 1.00 ms where lists of 32 take 1.11 (1.01 as k_msm_few), 2048 1.33 and 1.41; 16 x 1024 0.95 and 1.01.  With 8 some of these
+// are 3 % faster and 1 x 512 4 % slower; from 4096 generators on nothing changes.
 // In instructions of a lane: an element costs an addition of 4700 a window (the first of a list none), a list 1700 and a bucket about 1350 for each step
 // of its wave in k_msm_windows.  The time of these on the whole chip at three quarters of its issue slots, half a list of the last waves, and the launch that
 // windows of more than 128 buckets add.
@@ -2034,7 +2036,7 @@ static uint32_t msm_windows_of_half(size_t terms, uint32_t n, uint32_t* most) {
         const double us = all * 4.0 / 64.0 / (1024.0 * 2400.0) / 0.75 + 6.0 * mean + (hb > 128u ? 80.0 : 0.0);
         if (best == 0 || us < best_us) {
             best = nwh; best_us = us;
-            *most = (uint32_t)std::min(std::max(2.5 * mean, 32.0), (double)MPIECE);
+            *most = (uint32_t)std::min(std::max(2.5 * mean, (double)n * buckets <= 2048.0 * MSL ? 12.0 : 32.0), (double)MPIECE);
         }
     }
     return best;
