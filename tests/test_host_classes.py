@@ -3,6 +3,8 @@ entry points they reach themselves (a program's own definitions come before the 
 import os
 import subprocess
 
+import pytest
+
 from zkhelp import ROOT
 
 PKG = os.path.join(ROOT, "zkllm-ccs2024_amd")
@@ -21,6 +23,7 @@ ABI = r"""
 static std::vector<std::string> events;
 static std::vector<const void*> job;          // what an opened job was given to read
 static std::atomic<int> frees{0}, reads{0};
+static int ready = -1;                       // whether the last opened job's queries were
 extern "C" {
 const char* zk_last_error() { return "refused"; }
 int zk_malloc(void** p, size_t n) { *p = calloc(1, n + 64); return 0; }
@@ -52,12 +55,14 @@ int zk_fr_gather(void*, const void*, const void*, size_t, void*) { return 0; }
 int zk_fr_gather_ints(void*, void*, const void*, const void*, const void*, size_t, void*) { return 0; }
 int zk_i32_pad_from(void*, const void*, size_t, size_t, const void*, int32_t, void*) { return 0; }
 int zk_lookup_ints_suffice(size_t, size_t) { return 0; }
+int zk_lookup_multiplicities(void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, int, void*) { return 0; }
 int zk_lookup_multiplicities_begin(void** c, void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, void*) { *c = malloc(4); return 0; }
 int zk_lookup_multiplicities_end(void* c) { free(c); return 0; }
 int zk_lookup_open(void** o, const void*, const uint32_t*, size_t, void*) { *o = malloc(4); return 0; }
 int zk_lookup_open_drop(void* o) { events.push_back("drop"); free(o); return 0; }
 int zk_lookup_prove_begin_opened(void**, void*, const void* S, const void* Si, const void* So, const void* Soi, const void* mi, const uint32_t*, const void* T, const void* m, int32_t,
-                                 const uint32_t*, const uint32_t*, const uint32_t*, size_t, size_t, int, int, int, void*) {
+                                 const uint32_t*, const uint32_t*, const uint32_t*, size_t, size_t, int, int queries_ready, int, void*) {
+    ready = queries_ready;
     for (const void* p : {S, Si, So, Soi, mi, T, m}) if (p) job.push_back(p);
     events.push_back("begin");
     return 1;
@@ -126,3 +131,20 @@ int main() {
 }
 """)
     assert out == ["1", "1", "0"]
+
+
+@pytest.mark.parametrize("log_queries,log_table,more,ahead", [(23, 16, 1, 1), (24, 15, 1, 1), (24, 16, 1, 0), (24, 20, 1, 0), (25, 16, 1, 0), (24, 16, 0, 1), (10, 4, 1, 1)])
+def test_rounds_of_a_large_job_wait_for_the_counting_where_more_is_queued_behind_it(tmp_path, log_queries, log_table, more, ahead):
+    out = run(tmp_path, "ahead", r"""
+int main() {
+    FrTensor S(1u << %d);
+    tLookupRange table(0, 1u << %d);
+    const vector<Fr_t> u(%d), v(%d);
+    std::unique_ptr<FrTensor> m;
+    try { table.count_and_prove_begin(S, m, true, Fr_t{}, Fr_t{}, u, v, true, %d); } catch (const std::exception&) {}
+    printf("%%d\n", ready);
+    fflush(stdout);
+    _Exit(0);
+}
+""" % (log_queries, log_table, log_queries, log_queries, more))
+    assert out == [str(ahead)]

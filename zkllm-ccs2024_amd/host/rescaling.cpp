@@ -74,7 +74,7 @@ Rescaling::Pending Rescaling::prove_begin(const FrTensor& X, const FrTensor& X_,
     }
     // the lookup's job first: its kernels wait for what is queued here so far, and the evaluations below run beside them
     // (inside: remainders of a division by the table's length)
-    p.look = tl_rem.count_and_prove_begin(*p.rem, p.m, true, rand_temp[0], rand_temp[1], u, v, at_once);
+    p.look = tl_rem.count_and_prove_begin(*p.rem, p.m, true, rand_temp[0], rand_temp[1], u, v, at_once, at_once);
     // X_(u) and rem(u) in one pass over the two tensors (the padding of the remainders is zeros: the unpadded tensor has the same
     // extension and the others' length).  X = scaling_factor X_ + rem element by element, so X(u) is that combination of the two
     // values: X itself, 32 bytes an element, is read only with ZKLLM_CHECK_CLAIMS=1, which evaluates it and compares as

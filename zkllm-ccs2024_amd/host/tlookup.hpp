@@ -78,9 +78,9 @@ class tLookupRange : public tLookup {
     Fr_t prove(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v, vector<Polynomial>& proof);
     LookupPending prove_begin(const FrTensor& S, const FrTensor& m, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v);
     // addition: prep (inside: prep_inside) and prove_begin in one: the table's inverses and the rounds that read no multiplicities run beside the counting.
-    // The multiplicities go to m, which must outlive the proof.  at_once: the caller ends the proof next.
+    // The multiplicities go to m, which must outlive the proof.  at_once: the caller ends the proof next.  more: what it queues behind the counting first is waited for too.
     LookupPending count_and_prove_begin(const FrTensor& S, std::unique_ptr<FrTensor>& m, bool inside, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v,
-                                        bool at_once = false);
+                                        bool at_once = false, bool more = false);
 };
 
 class tLookupRangeMapping : public tLookupRange {
