@@ -55,8 +55,8 @@ int zk_fr_gather(void*, const void*, const void*, size_t, void*) { return 0; }
 int zk_fr_gather_ints(void*, void*, const void*, const void*, const void*, size_t, void*) { return 0; }
 int zk_i32_pad_from(void*, const void*, size_t, size_t, const void*, int32_t, void*) { return 0; }
 int zk_lookup_ints_suffice(size_t, size_t) { return 0; }
-int zk_lookup_multiplicities(void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, int, void*) { return 0; }
-int zk_lookup_multiplicities_begin(void** c, void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, void*) { *c = malloc(4); return 0; }
+int zk_lookup_multiplicities(void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, int, void*) { events.push_back("counted"); return 0; }
+int zk_lookup_multiplicities_begin(void** c, void*, void*, const void*, const void*, const void*, int32_t, uint32_t, size_t, uint32_t, void*) { events.push_back("count begun"); *c = malloc(4); return 0; }
 int zk_lookup_multiplicities_end(void* c) { free(c); return 0; }
 int zk_lookup_open(void** o, const void*, const uint32_t*, size_t, void*) { *o = malloc(4); return 0; }
 int zk_lookup_open_drop(void* o) { events.push_back("drop"); free(o); return 0; }
@@ -131,6 +131,22 @@ int main() {
 }
 """)
     assert out == ["1", "1", "0"]
+
+
+def test_mapping_that_waits_for_its_check_at_once_counts_in_one_call(tmp_path):
+    """An event for a check that is asked for in the next line costs more than the check."""
+    out = run(tmp_path, "counts", r"""
+int main() {
+    FrTensor values(4), queries(6);
+    tLookupRangeMapping table(-2, 4, values);
+    events.clear();
+    (void)table(queries);
+    for (auto& e : events) if (e[0] == 'c') puts(e.c_str());
+    fflush(stdout);
+    _Exit(0);
+}
+""")
+    assert out == ["counted"]
 
 
 @pytest.mark.parametrize("log_queries,log_table,more,ahead", [(23, 16, 1, 1), (24, 15, 1, 1), (24, 16, 1, 0), (24, 20, 1, 0), (25, 16, 1, 0), (24, 16, 0, 1), (10, 4, 1, 1)])

@@ -86,16 +86,19 @@ pair<FrTensor, FrTensor> tLookupRangeMapping::map(const FrTensor& vals, const Fr
 pair<FrTensor, FrTensor> tLookupRangeMapping::map_queued(const FrTensor& vals, const FrTensor* unwritten) {
     CountedQueries c;
     // queries and mapped values in int32 form: nothing below needs the array of table positions
-    count(c, vals, !(vals.kept_ints() && mapped_vals.kept_ints()));
-    c.settle();
+    count(c, vals, !(vals.kept_ints() && mapped_vals.kept_ints()), true);
     FrTensor y = gather(vals, c, unwritten);
     return {std::move(y), std::move(*c.m)};
 }
-void tLookupRangeMapping::count(CountedQueries& c, const FrTensor& vals, bool positions) {
+// wait: the range check is settled here (an attention head of 2 x 128 tokens takes 20 us less so than by settle() in the next line)
+void tLookupRangeMapping::count(CountedQueries& c, const FrTensor& vals, bool positions, bool wait) {
     if (positions) c.idx.reset(new DevBuf(sizeof(uint) * (size_t)vals.size));
     const void* h = vals.kept_ints();
+    const void* ints = h ? zk_fr_fold_prepared_ints(h) : nullptr;
+    void* idx = positions ? c.idx->p : nullptr;
     c.m.reset(new FrTensor(table.size));
-    ZKC(zk_lookup_multiplicities_begin(&c.check, c.m->gpu_data, positions ? c.idx->p : nullptr, nullptr, h ? zk_fr_fold_prepared_ints(h) : nullptr, vals.gpu_data, low, len, vals.size, table.size, nullptr));
+    if (wait) ZKC(zk_lookup_multiplicities(c.m->gpu_data, idx, nullptr, ints, vals.gpu_data, low, len, vals.size, table.size, 0, nullptr));
+    else ZKC(zk_lookup_multiplicities_begin(&c.check, c.m->gpu_data, idx, nullptr, ints, vals.gpu_data, low, len, vals.size, table.size, nullptr));
 }
 // the outputs of counted queries
 FrTensor tLookupRangeMapping::gather(const FrTensor& vals, const CountedQueries& c, const FrTensor* unwritten) {
@@ -312,7 +315,7 @@ tLookupRangeMapping::MappedPending tLookupRangeMapping::map_and_prove_begin(cons
     opened.table = combined(r);
     ZKC(zk_lookup_open(&opened.handle, opened.table->gpu_data, beta.val, table.size, nullptr));
     CountedQueries c;
-    count(c, S_in, positions);
+    count(c, S_in, positions, false);
     if (S_in.size != (1u << ceilLog2(S_in.size)) && !S_in.kept_ints()) {          // neither waits for what is asked next
         opened.queries = padded(opened.keep, S_in, table, false, nullptr);
         opened.m = padded_m(opened.keep, *c.m, S_in.size);

@@ -112,7 +112,7 @@ class tLookupRangeMapping : public tLookupRange {
     MappedPending map_and_prove_begin(const FrTensor& S_in, const Fr_t& r, const Fr_t& alpha, const Fr_t& beta, const vector<Fr_t>& u, const vector<Fr_t>& v);
 
    private:
-    void count(CountedQueries& c, const FrTensor& vals, bool positions);
+    void count(CountedQueries& c, const FrTensor& vals, bool positions, bool wait);
     FrTensor gather(const FrTensor& vals, const CountedQueries& c, const FrTensor* unwritten);
     std::unique_ptr<FrTensor> combined(const Fr_t& r) const;      // table + r * mapped values
     FrTensor* padded(std::vector<std::unique_ptr<FrTensor>>& keep, const FrTensor& t, const FrTensor& fill_from, bool ints, const void* fill_ints) const;
