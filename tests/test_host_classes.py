@@ -19,7 +19,7 @@ ABI = r"""
 #include <string>
 #include <thread>
 #include <vector>
-#include "tlookup.hpp"
+#include "zksoftmax.hpp"
 static std::vector<std::string> events;
 static std::vector<const void*> job;          // what an opened job was given to read
 static std::atomic<int> frees{0}, reads{0};
@@ -43,6 +43,8 @@ int zk_memcpy_d2h(void* d, const void* s, size_t n, void*) {
     return 0;
 }
 int zk_range_table(void*, int32_t, uint32_t, uint32_t, void*) { return 0; }
+int zk_fr_from_i32(void*, const void*, size_t, void*) { return 0; }
+int zk_softmax_table(void*, double, double, uint32_t, void*) { return 0; }
 int zk_fr_pad_from(void*, const void*, size_t, size_t, const void*, void*) { return 0; }
 int zk_fr_fold_prepare(void** p, const void*, size_t, void*) { events.push_back("wait"); *p = malloc(4); return 0; }
 int zk_fr_fold_prepare_queue(void** p, void* flag, const void*, size_t, void*) { *p = malloc(4); memset(flag, 0, 4); return 0; }
@@ -147,6 +149,19 @@ int main() {
 }
 """)
     assert out == ["counted"]
+
+
+def test_constructor_of_a_softmax_leaves_its_tables_settled(tmp_path):
+    out = run(tmp_path, "softmax", r"""
+struct Softmax : zkSoftmax { using zkSoftmax::zkSoftmax; using zkSoftmax::other_segments; };
+int main() {
+    Softmax s({4, 4, 4}, 1, 1, 1, {1.0}, 4, 4, 4, 1);
+    for (auto& t : s.other_segments) printf("%d\n", t.mapped_vals.fold_cache->unchecked == nullptr);
+    fflush(stdout);
+    _Exit(0);
+}
+""")
+    assert out == ["1", "1"]
 
 
 @pytest.mark.parametrize("log_queries,log_table,more,ahead", [(23, 16, 1, 1), (24, 15, 1, 1), (24, 16, 1, 0), (24, 20, 1, 0), (25, 16, 1, 0), (24, 16, 0, 1), (10, 4, 1, 1)])
